@@ -114,6 +114,8 @@ def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
     lib.fl_attn_validate.argtypes = [C.POINTER(FlAttnParams)]
     lib.fl_attn_plan.restype = C.c_int
     lib.fl_attn_plan.argtypes = [C.POINTER(FlAttnParams), C.POINTER(C.c_int64)]
+    lib.fl_attn_rows_plan.restype = C.c_int
+    lib.fl_attn_rows_plan.argtypes = [C.POINTER(FlAttnParams), C.POINTER(C.c_uint64)]
     lib.fl_attn_fwd.restype = C.c_int
     lib.fl_attn_fwd.argtypes = [C.POINTER(FlAttnParams), C.c_void_p]
     lib.fl_static_scratch_bytes.restype = C.c_uint64
@@ -412,6 +414,12 @@ def attn_fwd(
     if validate_only:
         _check(lib.fl_attn_validate(C.byref(p)))
         return out
+    if not p.workspace:
+        scratch = C.c_uint64()
+        if lib.fl_attn_rows_plan(C.byref(p), C.byref(scratch)) and scratch.value:
+            ws = torch.empty(scratch.value, dtype=torch.uint8, device=q.device)
+            p.workspace, p.workspace_bytes = ws.data_ptr(), scratch.value
+            keep.append(ws)
     _launch_on(q.device, lib.fl_attn_fwd, p)
     # tensors in `keep` were last used on the current stream; the caching allocator orders their reuse after it
     del keep

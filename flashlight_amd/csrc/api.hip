@@ -10,6 +10,7 @@
 #include "bwd_instances.h"
 #include "instances.h"
 #include "pairbias_instances.h"
+#include "rows_instances.h"
 
 namespace fl {
 // Builds (min, max) of the document ids of every block of kDocBlock positions.
@@ -260,6 +261,16 @@ void static_scratch_release(hipStream_t s, int dev) {
   } else {
     (void)hipGetLastError();
   }
+}
+
+// Bounds of the element predicate every positional mask reduces to: key < Lk && ((dmin <= key - q <= dmax) || key < pfx)
+void position_bounds(const fl_attn_params* p, int32_t* dmin, int32_t* dmax, int32_t* pfx) {
+  const int kFar = 1 << 29;
+  const bool causal_like = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_SLIDING ||
+                           p->mask_kind == FL_MASK_PREFIX_LM || p->mask_kind == FL_MASK_DOCUMENT_CAUSAL;
+  *dmax = causal_like ? 0 : kFar;
+  *dmin = p->mask_kind == FL_MASK_SLIDING ? -(p->window < kFar ? p->window : kFar) : -kFar;
+  *pfx = p->mask_kind == FL_MASK_PREFIX_LM ? (p->prefix < 0 ? 0 : p->prefix) : 0;
 }
 
 bool is_doc(int kind) { return kind == FL_MASK_DOCUMENT || kind == FL_MASK_DOCUMENT_CAUSAL; }
@@ -593,6 +604,117 @@ bool plan_pairbias(const fl_attn_params* p, fl::PParams* out, int* grid) {
   return true;
 }
 
+// Whether *p (already validated) is a call the few-rows forward (rows_kernel.h) takes.  Fills the kernel's parameters and
+// launch shape.  `scratch`: bytes of p->workspace it would use to cut the keys into chunks; with less the keys of a row
+// tile stay in one workgroup.
+bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves, int* blocks, uint64_t* scratch) {
+  if (p->Dqk != p->Dv || !fl::rows_has_shape(p->Dqk) || is_doc(p->mask_kind) || p->diff || p->gate || p->attended_dump ||
+      p->dropout_threshold || p->score_fn != FL_SCORE_NONE)
+    return false;
+  const bool has_bias = p->bias[0] || p->bias[1];
+  if (has_bias && p->alibi_heads > 0) return false;
+  for (int i = 0; i < 2; ++i)
+    if (p->bias[i] && (p->bias_strides[i][1] != 0 || p->bias_strides[i][2] != 0)) return false;
+  // row offsets inside a tile of 32 keys are 24-bit products
+  if (p->k_strides[2] >= (1 << 22) || p->v_strides[2] >= (1 << 22)) return false;
+  const int64_t units = (int64_t)p->B * p->Hkv, group = p->Hq / p->Hkv, rows = group * p->Lq, tiles = (p->Lk + 31) / 32;
+  if (rows > (1 << 28) || units * rows > (1 << 30)) return false;
+  const int64_t base16 = units * ((rows + 15) / 16), base32 = units * ((rows + 31) / 32);
+  // Decoding (rows <= 32: every key is read once, or twice) belongs here at any size but the shortest: up to 128 keys the
+  // tile kernel's one or two steps are 0.5 us sooner until its padded 128-row workgroups fill the part.
+  // Longer row counts re-read K and V for every 16 rows (32 at head dim 64), from L2: that pays while one workgroup per
+  // compute unit holds all of them, where the tile kernel leaves most of the part idle (head dim 64, 8 heads of 1024
+  // causal rows: 16.8 -> 12.2 us; head dim 128, 4 heads: 21.5 -> 14.5 us), and loses beyond (twice as many rows: 17 -> 18
+  // and 23 -> 30 us).  Up to 64 keys the tile kernel has a single step.
+  int qt = 1;
+  if (rows <= 32) {
+    if (p->Lk <= 128 && (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128) <= 256) return false;
+    if (rows > 16 && p->Dqk == 64 && p->Lk >= 4096) qt = 2;
+  } else if (p->Lk <= 64) {
+    return false;
+  } else if (base16 > 256) {
+    if (p->Dqk != 64 || base32 > 256 || p->Lk <= 256) return false;
+    qt = 2;
+  }
+  const int64_t row_tiles = (rows + 16 * qt - 1) / (16 * qt), base = units * row_tiles;
+  // Waves per workgroup and chunks of the keys.  Eight waves fill a compute unit's registers, so 256 workgroups of eight
+  // or 512 of four are one round.  Enough row tiles: no chunks, and shorter workgroups the more of them there are.  Few:
+  // a chunk has two key tiles per wave at least, and the merge launch behind the chunks costs 4.5 us, about what reading 512
+  // keys in one workgroup costs: up to there they stay together.  Eight waves add up inside the workgroup what four would
+  // send through memory: worth it once a wave has two tiles.
+  int nw = 8;
+  int64_t chunks = 1;
+  if (base >= 1024) {
+    nw = tiles < 16 ? 2 : 4;
+  } else if (base >= 512) {
+    nw = 4;
+  } else if (rows > 32) {
+    nw = tiles > 8 ? 8 : 4;
+  } else if (base < 256 && tiles > 16 && p->mask_kind == FL_MASK_NONE) {
+    if (tiles * base >= 16 * 256) {
+      chunks = 256 / base;
+    } else {
+      nw = 4;
+      chunks = std::max<int64_t>(1, std::min<int64_t>(512 / base, tiles / 8));
+    }
+  }
+  fl::RParams k;
+  std::memset(&k, 0, sizeof(k));
+  *scratch = 0;
+  if (chunks > 1) {
+    const uint64_t n = (uint64_t)base * chunks * 16 * qt;
+    *scratch = n * (p->Dv + 2) * sizeof(float);
+    if (!p->workspace || p->workspace_bytes < *scratch || reinterpret_cast<uintptr_t>(p->workspace) % 16) {
+      chunks = 1;
+    } else {
+      k.part = static_cast<float*>(p->workspace);
+      k.part_ml = k.part + n * p->Dv;
+    }
+  }
+  k.q = static_cast<const fl::bf16_t*>(p->q);
+  k.k = static_cast<const fl::bf16_t*>(p->k);
+  k.v = static_cast<const fl::bf16_t*>(p->v);
+  k.o = static_cast<fl::bf16_t*>(p->o);
+  k.lse = p->lse;
+  for (int i = 0; i < 3; ++i) {
+    k.qs[i] = p->q_strides[i];
+    k.ks[i] = p->k_strides[i];
+    k.vs[i] = p->v_strides[i];
+    k.os[i] = p->o_strides[i];
+  }
+  k.B = p->B;
+  k.Hq = p->Hq;
+  k.Hkv = p->Hkv;
+  k.Lq = p->Lq;
+  k.Lk = p->Lk;
+  k.group = (int)group;
+  k.rows = (int)rows;
+  k.row_tiles = (int)row_tiles;
+  k.chunks = (int)chunks;
+  k.units = (int)units;
+  const float l2e = 1.4426950408889634f;
+  k.scale_log2 = p->scale * l2e;
+  if (p->softcap > 0.f) {
+    k.cap_k1 = p->scale / p->softcap * 2.0f * l2e;
+    k.cap_c = p->softcap * l2e;
+  }
+  position_bounds(p, &k.dmin, &k.dmax, &k.pfx);
+  k.alibi_heads = p->alibi_heads;
+  for (int i = 0; i < 2; ++i) {
+    k.bias[i] = p->bias[i];
+    k.bias_batch[i] = p->bias_strides[i][0];
+    k.bias_key[i] = (int)p->bias_strides[i][3];
+    k.bias_div[i] = p->bias[i] ? p->bias_batch_div[i] : 1;
+    k.bias_f32[i] = p->bias_dtype[i] == FL_F32;
+  }
+  k.by_xcd = units * chunks >= 8 && row_tiles > 1;
+  *grid = (int)(k.by_xcd ? (units * chunks + 7) / 8 * 8 * row_tiles : units * chunks * row_tiles);
+  *waves = nw;
+  *blocks = qt;
+  *out = k;
+  return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -649,6 +771,14 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
   return 0;
 }
 
+int fl_attn_rows_plan(const fl_attn_params* p, uint64_t* scratch_bytes) {
+  if (!p || !scratch_bytes || p->B <= 0 || p->Hkv <= 0 || p->Hq <= 0 || p->Lq <= 0 || p->Lk <= 0) return 0;
+  fl::RParams rp;
+  int grid = 0, waves = 0, blocks = 0;
+  *scratch_bytes = 0;
+  return plan_rows(p, &rp, &grid, &waves, &blocks, scratch_bytes) ? 1 : 0;
+}
+
 int fl_attn_fwd(const fl_attn_params* p, void* stream_) {
   const fl::Instance* in = nullptr;
   int rc = validate(p, &in);
@@ -662,6 +792,17 @@ int fl_attn_fwd(const fl_attn_params* p, void* stream_) {
       const hipError_t e = (p->dtype == FL_F16 ? fl::launch_pairbias_f16 : fl::launch_pairbias_bf16)(
           p->Dqk, p->Lk / 32, p->gate != nullptr, pb.rowb != nullptr, pb, pb_grid, stream);
       if (e != hipSuccess) return fail((int)e, "launch of the shared-bias forward failed: %s", hipGetErrorString(e));
+      return 0;
+    }
+  }
+  {
+    fl::RParams rp;
+    int rows_grid = 0, rows_waves = 0, rows_blocks = 0;
+    uint64_t scratch = 0;
+    if (plan_rows(p, &rp, &rows_grid, &rows_waves, &rows_blocks, &scratch)) {
+      const uint32_t mod = p->bias[0] || p->bias[1] ? fl::F_BIAS : p->alibi_heads > 0 || p->softcap > 0.f ? fl::F_ALIBI | fl::F_SOFTCAP : 0u;
+      const hipError_t e = (p->dtype == FL_F16 ? fl::launch_rows_f16 : fl::launch_rows_bf16)(p->Dqk, rows_blocks, mod, rp, rows_grid, rows_waves, stream);
+      if (e != hipSuccess) return fail((int)e, "launch of the few-rows forward failed: %s", hipGetErrorString(e));
       return 0;
     }
   }
@@ -690,14 +831,7 @@ int fl_attn_fwd(const fl_attn_params* p, void* stream_) {
   kp.mask_kind = p->mask_kind;
   kp.window = p->window;
   kp.prefix = p->prefix;
-  {
-    const int kFar = 1 << 29;
-    const bool causal_like = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_SLIDING ||
-                             p->mask_kind == FL_MASK_PREFIX_LM || p->mask_kind == FL_MASK_DOCUMENT_CAUSAL;
-    kp.dmax = causal_like ? 0 : kFar;
-    kp.dmin = p->mask_kind == FL_MASK_SLIDING ? -(p->window < kFar ? p->window : kFar) : -kFar;
-    kp.pfx = p->mask_kind == FL_MASK_PREFIX_LM ? (p->prefix < 0 ? 0 : p->prefix) : 0;
-  }
+  position_bounds(p, &kp.dmin, &kp.dmax, &kp.pfx);
   kp.doc_ids = p->doc_ids;
   kp.doc_stride = p->doc_stride;
   kp.alibi_heads = p->alibi_heads;
@@ -904,14 +1038,7 @@ int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream_) {
   bp.mask_kind = p->mask_kind;
   bp.window = p->window;
   bp.prefix = p->prefix;
-  {
-    const int kFar = 1 << 29;
-    const bool causal_like = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_SLIDING ||
-                             p->mask_kind == FL_MASK_PREFIX_LM || p->mask_kind == FL_MASK_DOCUMENT_CAUSAL;
-    bp.dmax = causal_like ? 0 : kFar;
-    bp.dmin = p->mask_kind == FL_MASK_SLIDING ? -(p->window < kFar ? p->window : kFar) : -kFar;
-    bp.pfx = p->mask_kind == FL_MASK_PREFIX_LM ? (p->prefix < 0 ? 0 : p->prefix) : 0;
-  }
+  position_bounds(p, &bp.dmin, &bp.dmax, &bp.pfx);
   bp.doc_ids = p->doc_ids;
   bp.doc_stride = p->doc_stride;
   bp.alibi_heads = p->alibi_heads;

@@ -110,11 +110,6 @@ struct BwdTraits {
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
 };
 
-template <bool FIRST, class A>
-__device__ __forceinline__ A& pick(A& a, A& b) {
-  if constexpr (FIRST) return a; else return b;
-}
-
 template <class T>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
 void bwd_kernel(const BParams p) {

@@ -223,6 +223,12 @@ __device__ __forceinline__ bool static_while(F&& f) {
   }
 }
 
+// the first or the second of two objects of one type
+template <bool FIRST, class A>
+__device__ __forceinline__ A& pick(A& a, A& b) {
+  if constexpr (FIRST) return a; else return b;
+}
+
 // ---- mask logic (integer, shared by the tile classifier and the element predicate) -------------------------------
 
 // Class of the key tile [k0, k1) against query rows [q0, q1) for the positional part of the mask.

@@ -101,7 +101,8 @@ typedef struct fl_attn_params {
                   * monkeypatch/fusion/_reduction.py:55-57) */
 
   /* Scratch of document-mask calls (the forward's lists of key tiles per query tile, the backward's table of id
-   * ranges); size from fl_workspace_bytes(), 16-byte aligned; may be NULL otherwise. */
+   * ranges); size from fl_workspace_bytes(), 16-byte aligned.  Optional scratch of calls with few query rows, see
+   * fl_attn_rows_plan().  May be NULL otherwise. */
   void* workspace;
   uint64_t workspace_bytes;
 
@@ -174,6 +175,12 @@ uint64_t fl_workspace_bytes(const fl_attn_params* p);
 /* Bytes of device scratch fl_attn_bwd alone needs in fwd.workspace (0 unless a document mask is used): 16 bytes per 32
  * positions of every batch row.  No counterpart in the reference. */
 uint64_t fl_bwd_workspace_bytes(const fl_attn_params* p);
+
+/* Whether fl_attn_fwd runs *p in the kernel for few query rows per key / value head (decoding steps, short prefills):
+ * 1 or 0.  *scratch_bytes receives what `workspace` may hold then (16-byte aligned, contents undefined before and after)
+ * for the keys to be cut into chunks that run in different workgroups, 0 when that is not wanted; without it the call
+ * is correct and slower.  Host only. */
+int fl_attn_rows_plan(const fl_attn_params* p, uint64_t* scratch_bytes);
 
 /* Runs the fused forward on hipStream_t `stream` (NULL = default stream).
  * Replaces torch.compile(fn)(q, k, v, ...) for the functions of attention_variants/. */

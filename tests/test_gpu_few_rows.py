@@ -1,0 +1,94 @@
+"""The few-rows forward (csrc/rows_kernel.h): decoding steps and short prefills, at the edges of its 16-row tiles, 32-key
+tiles, wave and chunk splits, against the oracle's generic attention; results and row statistics."""
+import ctypes as C
+import math
+
+import pytest
+import torch
+
+from flashlight_amd import _ffi, ops
+from oracle.attention import alibi_slopes
+from tests.conftest import assert_parity
+
+DEV = "cuda"
+
+
+def _taken(B, Hq, Hkv, Lq, Lk, D, **kw):
+    """(whether the call goes to the few-rows kernel, scratch bytes it asks for)"""
+    q, k = torch.empty(B, Hq, Lq, D, dtype=torch.bfloat16), torch.empty(B, Hkv, Lk, D, dtype=torch.bfloat16)
+    a = dict(scale=None, mask_kind=0, window=0, prefix=0, doc_ids=None, alibi_heads=0, softcap=0.0, biases=(), gate=None,
+             diff=False, lambda_full=0.0, attended_dump=None)
+    a.update(kw)
+    lib = _ffi.load_library()
+    p, _ = _ffi._fill_params(lib, q, k, k, q, Hq, Hkv, **a)
+    n = C.c_uint64()
+    return bool(lib.fl_attn_rows_plan(C.byref(p), C.byref(n))), n.value
+
+
+def test_which_calls_the_few_rows_kernel_takes():
+    assert _taken(1, 32, 8, 1, 32768, 128)[0] and _taken(1, 32, 8, 1, 32768, 128)[1] > 0   # decoding, cut into chunks
+    assert _taken(64, 32, 8, 1, 1000, 64) == (True, 0)          # enough workgroups without chunks
+    assert not _taken(1, 8, 8, 1, 128, 64)[0]                   # too short to matter
+    assert _taken(2, 8, 8, 512, 512, 64, mask_kind=_ffi.MASK_CAUSAL) == (True, 0)
+    assert not _taken(4, 16, 16, 4096, 4096, 128)[0]
+
+
+CASES = [  # B, Hq, Hkv, Lq, Lk, D
+    (1, 4, 4, 1, 129, 64), (2, 8, 2, 1, 257, 128), (1, 8, 1, 2, 545, 64), (1, 32, 2, 1, 600, 128), (1, 17, 1, 1, 4097, 64),
+    (3, 8, 8, 1, 2047, 128), (33, 8, 8, 1, 1000, 64), (64, 16, 8, 1, 200, 128), (72, 16, 16, 1, 161, 64),
+    (1, 2, 2, 65, 65, 64), (1, 3, 3, 100, 100, 128), (1, 4, 2, 255, 255, 64), (1, 8, 8, 511, 513, 64), (2, 6, 2, 300, 300, 64),
+    (1, 2, 1, 129, 1000, 128), (1, 16, 16, 257, 257, 64)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp16", [False, True])
+@pytest.mark.parametrize("shape", CASES)
+def test_few_rows_against_the_oracle(shape, fp16):
+    B, Hq, Hkv, Lq, Lk, D = shape
+    dt = torch.float16 if fp16 else torch.bfloat16
+    g = torch.Generator().manual_seed(sum(shape))
+    q = torch.randn(B, Hq, Lq, D, generator=g).to(dt)
+    longer = torch.randn(2, B, Lk + 24, Hkv, D, generator=g).to(dt)   # caches in longer, sequence-major buffers
+    k, v = longer[0, :, 8:8 + Lk].transpose(1, 2), longer[1, :, 16:16 + Lk].transpose(1, 2)
+    dev = longer.cuda()
+    kd, vd = dev[0, :, 8:8 + Lk].transpose(1, 2), dev[1, :, 16:16 + Lk].transpose(1, 2)
+    pos_q, pos_k = torch.arange(Lq)[:, None], torch.arange(Lk)[None]
+    row = torch.randn(B, 1, 1, Lk, generator=g)
+    row[..., 3:Lk // 3] = float("-inf")
+    slopes = alibi_slopes(Hq).view(1, Hq, 1, 1)
+    cases = [("plain", {}, None, None, None),
+             ("causal", dict(mask_kind=_ffi.MASK_CAUSAL), pos_k > pos_q, None, None),
+             ("soft-cap + ALiBi", dict(softcap=4.0, alibi_heads=Hq), None, slopes * (pos_k - pos_q), 4.0),
+             ("row bias", dict(biases=[(row.to(dt).cuda(), 1)]), None, row.to(dt).float(), None),
+             ("fp32 row bias", dict(biases=[(row[:1].contiguous().cuda(), B)]), None, row[:1], None)]
+    if Lq == Lk:
+        cases += [("window", dict(mask_kind=_ffi.MASK_SLIDING, window=33), (pos_k > pos_q) | (pos_q - pos_k > 33), None, None),
+                  ("prefix", dict(mask_kind=_ffi.MASK_PREFIX_LM, prefix=40), (pos_k > pos_q) & (pos_k >= 40), None, None)]
+    G = Hq // Hkv
+    kf, vf = (t.float().repeat_interleave(G, 1) for t in (k, v))
+    for name, kw, masked, bias, cap in cases:
+        lse = torch.empty(B, Hq, Lq, dtype=torch.float32, device=DEV)
+        out = _ffi.attn_fwd(q.cuda(), kd, vd, lse=lse, **kw)
+        s = q.float() @ kf.transpose(-1, -2) / math.sqrt(D)
+        s = cap * torch.tanh(s / cap) if cap else s
+        s = s + bias if bias is not None else s
+        s = s.masked_fill(masked, float("-inf")) if masked is not None else s
+        assert_parity(out, torch.softmax(s, -1).nan_to_num(0.0) @ vf, f"{shape} {name}")
+        want = torch.logsumexp(s, -1) / math.log(2.0)
+        assert (lse.cpu() - want).abs().max().item() < 1e-2, (shape, name)
+        assert_parity(ops.dispatch(q.cuda(), kd, vd, **kw), torch.softmax(s, -1).nan_to_num(0.0) @ vf, f"{shape} {name} (front end)")
+
+
+@pytest.mark.gpu
+def test_rows_without_keys_and_extreme_logits():
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn(2, 8, 1, 128, generator=g).to(torch.bfloat16).cuda()
+    k, v = (torch.randn(2, 2, 3000, 128, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    for fill in (float("-inf"), -1e9):
+        none = torch.full((2, 1, 1, 3000), fill, dtype=torch.bfloat16, device=DEV)
+        lse = torch.zeros(2, 8, 1, dtype=torch.float32, device=DEV)
+        assert torch.count_nonzero(_ffi.attn_fwd(q, k, v, biases=[(none, 1)], lse=lse)) == 0
+        assert torch.isinf(lse).all()
+    k[:, :, 1500:] *= 60.0   # the maximum jumps by hundreds of nats half way through the keys
+    want = torch.nn.functional.scaled_dot_product_attention(q.float().cpu(), k.float().cpu(), v.float().cpu(), enable_gqa=True)
+    assert_parity(ops.dispatch(q, k, v), want, "jump")
