@@ -88,13 +88,14 @@ class FlashlightError(RuntimeError):
 
 
 _lib: Optional[C.CDLL] = None
+_host = None  # the native host path of the front ends (csrc/host.cpp), loaded with the library
 _MAX_DV_DIFF = 128  # widest value slab of a differential-attention kernel instance
 
 
 def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
     """Loads the in-tree shared library once (or the library at `path`, which then serves every later call).  Raises if
     it has not been built (no silent fallback)."""
-    global _lib
+    global _lib, _host
     if _lib is not None and path is None:
         return _lib
     p = Path(path) if path else LIB_PATH
@@ -138,6 +139,13 @@ def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
     if lib.fl_bwd_params_sizeof() != C.sizeof(FlAttnBwdParams):
         raise RuntimeError(f"{p}: fl_attn_bwd_params is {lib.fl_bwd_params_sizeof()} bytes, binding expects "
                            f"{C.sizeof(FlAttnBwdParams)}")
+    try:
+        from . import _host as host_module
+    except ImportError as e:
+        raise ImportError("flashlight_amd/_host.so is missing or does not load: build it with `python -m flashlight_amd.build`") from e
+    _host = host_module
+    _host.bind(*(C.cast(getattr(lib, f), C.c_void_p).value for f in (
+        "fl_attn_fwd", "fl_attn_bwd", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_rows_plan", "fl_last_error")))
     _lib = lib
     return lib
 

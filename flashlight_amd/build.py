@@ -57,7 +57,7 @@ def instance_rows() -> list[tuple[str, str]]:
 
 def _sources_digest() -> str:
     h = hashlib.sha256()
-    for f in sorted(list(CSRC.glob("*.h")) + list(CSRC.glob("*.hip")) + list(CSRC.glob("*.inc")) + list(INCLUDE.glob("*.h"))):
+    for f in sorted(list(CSRC.glob("*.h")) + list(CSRC.glob("*.hip")) + list(CSRC.glob("*.inc")) + list(CSRC.glob("*.cpp")) + list(INCLUDE.glob("*.h"))):
         h.update(f.name.encode())
         h.update(f.read_bytes())
     h.update(" ".join(HIPCC_FLAGS).encode())
@@ -145,9 +145,11 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     if not probe_obj.exists():
         tasks.append(([cc, *HIPCC_FLAGS, "-c", str(CSRC / "probe.hip"), "-o", str(probe_obj)], probe_obj))
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(build_host_module)
         for log in ex.map(_compile, tasks):
             if verbose and log.strip():
                 print(log, file=sys.stderr)
+        host.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     _compile(([cc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-fno-gpu-rdc", *map(str, objs), "-o", str(tmp)], tmp))
     os.replace(tmp, LIB_PATH)
@@ -156,6 +158,29 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     os.replace(tmp, PROBE_LIB_PATH)
     build_c_host()
     return LIB_PATH
+
+
+HOST_SRC = CSRC / "host.cpp"
+HOST_MODULE = PKG_DIR / "_host.so"
+
+
+def build_host_module() -> Path:
+    """The native host path of the front ends (csrc/host.cpp): a Python extension on torch's C++ interface, host code only."""
+    import sysconfig
+
+    import torch
+
+    torch_dir = Path(torch.__file__).parent
+    rocm = Path(hipcc()).resolve().parent.parent
+    tmp = HOST_MODULE.with_suffix(".so.tmp")
+    includes = [INCLUDE, torch_dir / "include", torch_dir / "include/torch/csrc/api/include", rocm / "include",
+                sysconfig.get_paths()["include"]]
+    _compile(([shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1",
+               "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+               *(f"-isystem{i}" for i in includes), str(HOST_SRC), "-o", str(tmp), f"-L{torch_dir / 'lib'}", "-lc10", "-lc10_hip",
+               "-ltorch_cpu", "-ltorch", "-ltorch_python"], tmp))
+    os.replace(tmp, HOST_MODULE)
+    return HOST_MODULE
 
 
 C_HOST_SRC = PKG_DIR.parent / "tests" / "c_host" / "attn_host.c"

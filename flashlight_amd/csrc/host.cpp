@@ -1,0 +1,386 @@
+// Native host path of the front ends: what ops.dispatch does for an ordinary call, without the interpreter.
+//
+// A short call is bound by its host side: through the ctypes binding it spent 12 us on filling the parameter struct field
+// by field, on a differentiable call 100 us in the custom-operator layers, against 5 to 20 us on the GPU.  `forward` here
+// takes the call when it is of the plain kind (dense 16-bit tensors on the current device, compiled head dims, shapes and
+// strides the kernels address as they are, no tracer, transform or dispatch mode at work), allocates the result and
+// launches; with a gradient asked for it hangs a node on the result whose backward launches the gradient kernels.  For
+// anything else, wrong arguments included, it returns None and the Python code does what it always did: the conversions,
+// the compositions, the error messages.  It keeps no state between calls beyond the addresses of the C ABI's functions.
+#define PY_SSIZE_T_CLEAN
+#include <ATen/ATen.h>
+#include <Python.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+
+#include "flashlight_amd.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+struct Api {
+  int (*fwd)(const fl_attn_params*, void*) = nullptr;
+  int (*bwd)(const fl_attn_bwd_params*, void*) = nullptr;
+  uint64_t (*workspace)(const fl_attn_params*) = nullptr;
+  uint64_t (*bwd_workspace)(const fl_attn_params*) = nullptr;
+  int (*rows_plan)(const fl_attn_params*, uint64_t*) = nullptr;
+  const char* (*last_error)(void) = nullptr;
+} g_api;
+
+// One call's arguments.  The tensors are the caller's; `doc`, `bias` and `gate` may be undefined.
+struct Call {
+  Tensor q, k, v, doc, bias[2], gate;
+  int64_t bias_div[2] = {1, 1};
+  double scale = 0;
+  int64_t mask_kind = 0, window = 0, prefix = 0, alibi_heads = 0;
+  double softcap = 0, lambda = 0;
+  bool diff = false, seq_major = false;
+  bool wants_grad = false;
+};
+
+// dense, dim-contiguous rows in 16-byte pieces: what the kernels address as it lies
+bool addressable(const Tensor& t) {
+  if (t.stride(3) != 1 || (reinterpret_cast<uintptr_t>(t.const_data_ptr()) & 15)) return false;
+  for (int i = 0; i < 3; ++i)
+    if (t.stride(i) % 8 || t.stride(i) < 0) return false;
+  return true;
+}
+
+// an ordinary GPU tensor: no transform's wrapper, no lazy conjugate or negation, nothing that dispatches to Python
+bool plain(const Tensor& t) {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet odd({DispatchKey::FuncTorchBatched, DispatchKey::FuncTorchGradWrapper, DispatchKey::BatchedNestedTensor,
+                                        DispatchKey::Python, DispatchKey::PythonTLSSnapshot, DispatchKey::Functionalize,
+                                        DispatchKey::Conjugate, DispatchKey::Negative, DispatchKey::ZeroTensor,
+                                        DispatchKey::FuncTorchVmapMode, DispatchKey::PreDispatch});
+  return t.defined() && t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(odd);
+}
+
+// a dispatch mode, a functional transform or a tracer is at work on this thread
+bool mode_active() {
+  using c10::DispatchKey;
+  static const c10::DispatchKeySet modes({DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::FuncTorchDynamicLayerBackMode,
+                                          DispatchKey::FuncTorchVmapMode, DispatchKey::Python, DispatchKey::Functionalize, DispatchKey::PreDispatch});
+  return c10::impl::TorchDispatchModeTLS::any_modes_set() || c10::impl::tls_local_dispatch_key_set().included_.has_any(modes);
+}
+
+void set_strides(int64_t* to, const Tensor& t) {
+  for (int i = 0; i < 4; ++i) to[i] = t.stride(i);
+}
+
+int element_type(const Tensor& t) {
+  return t.scalar_type() == at::kBFloat16 ? FL_BF16 : t.scalar_type() == at::kHalf ? FL_F16 : -1;
+}
+
+// Fills what the forward and the backward share; false if the call is not of the plain kind.
+bool fill(const Call& c, fl_attn_params& p) {
+  const Tensor &q = c.q, &k = c.k, &v = c.v;
+  const int two = c.diff ? 2 : 1;
+  p.dtype = element_type(q);
+  p.q = q.const_data_ptr();
+  p.k = k.const_data_ptr();
+  p.v = v.const_data_ptr();
+  set_strides(p.q_strides, q);
+  set_strides(p.k_strides, k);
+  set_strides(p.v_strides, v);
+  p.B = (int32_t)q.size(0);
+  p.Hq = (int32_t)(q.size(1) / two);
+  p.Hkv = (int32_t)(k.size(1) / two);
+  p.Lq = (int32_t)q.size(2);
+  p.Lk = (int32_t)k.size(2);
+  p.Dqk = (int32_t)q.size(3);
+  p.Dv = (int32_t)v.size(3);
+  p.scale = (float)c.scale;
+  p.mask_kind = (int32_t)c.mask_kind;
+  p.window = (int32_t)c.window;
+  p.prefix = (int32_t)c.prefix;
+  p.alibi_heads = (int32_t)c.alibi_heads;
+  p.softcap = (float)c.softcap;
+  p.diff = c.diff;
+  p.lambda = (float)c.lambda;
+  if (c.doc.defined()) {
+    p.doc_ids = c.doc.const_data_ptr<int64_t>();
+    p.doc_stride = c.doc.size(0) == p.B && p.B > 1 ? c.doc.stride(0) : 0;
+  }
+  for (int i = 0; i < 2; ++i) {
+    const Tensor& b = c.bias[i];
+    if (!b.defined()) continue;
+    const int64_t want[4] = {p.B / c.bias_div[i], p.Hq, p.Lq, p.Lk};
+    p.bias[i] = b.const_data_ptr();
+    p.bias_dtype[i] = b.scalar_type() == at::kFloat ? FL_F32 : p.dtype;
+    p.bias_batch_div[i] = (int32_t)c.bias_div[i];
+    for (int ax = 0; ax < 4; ++ax) p.bias_strides[i][ax] = b.size(ax) == want[ax] && want[ax] != 1 ? b.stride(ax) : 0;
+  }
+  if (c.gate.defined()) {
+    p.gate = c.gate.const_data_ptr();
+    set_strides(p.gate_strides, c.gate);
+  }
+  return true;
+}
+
+void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+// Launches the forward of `c` into a fresh tensor; an undefined tensor if the C ABI refuses (the Python path then says why).
+// `lse`: when given, receives the row statistics.
+Tensor launch_forward(const Call& c, Tensor* lse) {
+  fl_attn_params p = {};
+  fill(c, p);
+  Tensor q = c.q, out;
+  const auto opt = q.options().requires_grad(false);
+  if (c.seq_major) out = at::empty({p.B, p.Lq, p.Hq, p.Dv}, opt).transpose(1, 2);
+  else out = at::empty({p.B, p.Hq, p.Lq, p.Dv}, opt);
+  p.o = out.data_ptr();
+  set_strides(p.o_strides, out);
+  if (lse) {
+    *lse = at::empty({p.B, p.Hq, p.Lq}, opt.dtype(at::kFloat));
+    p.lse = lse->data_ptr<float>();
+  }
+  uint64_t bytes = 0;
+  Tensor ws;
+  if (c.doc.defined()) {
+    bytes = g_api.workspace(&p);
+  } else if (!g_api.rows_plan(&p, &bytes)) {
+    const bool rows_independent = c.mask_kind == FL_MASK_NONE && !p.gate && !p.diff && !p.alibi_heads && !lse && !c.seq_major &&
+                                  (!p.bias[0] || (p.bias_strides[0][1] == 0 && p.bias_strides[0][2] == 0)) &&
+                                  (!p.bias[1] || (p.bias_strides[1][1] == 0 && p.bias_strides[1][2] == 0));
+    if (rows_independent) {
+      // (without a mask the G query heads of a key / value head may as well be G times as many rows of one head: one
+      // workgroup then reads the keys for all of them)
+      const int64_t group = p.Hq / p.Hkv;
+      int64_t tiles = (int64_t)p.B * p.Hq * ((p.Lq + 127) / 128);
+      if (group > 1 && group * p.Lq <= 128 && q.is_contiguous()) {
+        p.Hq = p.Hkv;
+        p.Lq = (int32_t)(group * p.Lq);
+        p.q_strides[1] = p.Lq * q.stride(2);
+        p.o_strides[1] = p.Lq * out.stride(2);
+        tiles = (int64_t)p.B * p.Hq;
+      }
+      // few workgroups against many keys: the Python path cuts the keys into chunks
+      if (tiles < 256 && p.Lk >= 4096) return Tensor();
+    }
+  }
+  if (bytes) {
+    ws = at::empty({(int64_t)bytes}, opt.dtype(at::kByte));
+    p.workspace = ws.data_ptr();
+    p.workspace_bytes = bytes;
+  }
+  return g_api.fwd(&p, current_stream()) == 0 ? out : Tensor();
+}
+
+struct Refused {};  // the C ABI does not take the call: the Python path then says why
+
+constexpr const char* kOnce = "flashlight_amd: the gradients are not differentiable a second time";
+
+struct Attention : torch::autograd::Function<Attention> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Call& c) {
+    Tensor lse;
+    Tensor out = launch_forward(c, &lse);
+    if (!out.defined()) throw Refused();
+    ctx->save_for_backward({q, k, v, out, lse});
+    ctx->saved_data["i"] = std::vector<int64_t>{c.mask_kind, c.window, c.prefix, c.alibi_heads};
+    ctx->saved_data["f"] = std::vector<double>{c.scale, c.softcap};
+    if (c.doc.defined()) ctx->saved_data["doc"] = c.doc;
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    const auto ints = ctx->saved_data["i"].toIntVector();
+    const auto floats = ctx->saved_data["f"].toDoubleVector();
+    Call c;
+    c.q = saved[0];
+    c.k = saved[1];
+    c.v = saved[2];
+    c.mask_kind = ints[0];
+    c.window = ints[1];
+    c.prefix = ints[2];
+    c.alibi_heads = ints[3];
+    c.scale = floats[0];
+    c.softcap = floats[1];
+    if (ctx->saved_data.count("doc")) c.doc = ctx->saved_data["doc"].toTensor();
+    const Tensor &out = saved[3], &lse = saved[4];
+    variable_list result(4);
+    if (!grads[0].defined()) return result;
+    const bool again = at::GradMode::is_enabled();
+    {
+      at::AutoGradMode off(false);
+      Tensor dout = grads[0].to(c.q.scalar_type());
+      if (!addressable(dout)) dout = dout.contiguous();
+      const auto opt = c.q.options().requires_grad(false);
+      fl_attn_bwd_params b = {};
+      fill(c, b.fwd);
+      b.fwd.o = const_cast<void*>(out.const_data_ptr());
+      set_strides(b.fwd.o_strides, out);
+      b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
+      Tensor dq = at::empty(c.q.sizes(), opt), dk = at::empty(c.k.sizes(), opt), dv = at::empty(c.v.sizes(), opt);
+      Tensor delta = at::empty(lse.sizes(), lse.options()), ws;
+      b.dout = dout.const_data_ptr();
+      b.dq = dq.data_ptr();
+      b.dk = dk.data_ptr();
+      b.dv = dv.data_ptr();
+      b.delta = delta.data_ptr<float>();
+      set_strides(b.dout_strides, dout);
+      set_strides(b.dq_strides, dq);
+      set_strides(b.dk_strides, dk);
+      set_strides(b.dv_strides, dv);
+      if (const uint64_t bytes = g_api.bwd_workspace(&b.fwd)) {
+        ws = at::empty({(int64_t)bytes}, opt.dtype(at::kByte));
+        b.fwd.workspace = ws.data_ptr();
+        b.fwd.workspace_bytes = bytes;
+      }
+      const int rc = g_api.bwd(&b, current_stream());
+      TORCH_CHECK(rc == 0, "flashlight_amd error ", rc, ": ", g_api.last_error());
+      result[0] = dq;
+      result[1] = dk;
+      result[2] = dv;
+    }
+    if (again) {
+      // under create_graph the gradients say that they have none of their own, instead of looking like constants
+      variable_list three(result.begin(), result.begin() + 3);
+      for (auto& t : three) t = t.detach().requires_grad_(true);
+      three = (*std::make_shared<torch::autograd::DelayedError>(kOnce, 3))(std::move(three));
+      std::copy(three.begin(), three.end(), result.begin());
+    }
+    return result;
+  }
+};
+
+// ---- Python boundary -----------------------------------------------------------------------------------------------------
+
+bool take_tensor(PyObject* o, Tensor& t) {
+  if ((PyObject*)Py_TYPE(o) != THPVariableClass) return false;  // (subclasses and Parameters go the Python way)
+  t = THPVariable_Unpack(o);
+  return plain(t);
+}
+
+// forward(q, k, v, scale, mask_kind, window, prefix, doc_ids, alibi_heads, softcap, biases, gate, diff, lambda, seq_major)
+PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 15) {
+    PyErr_SetString(PyExc_TypeError, "forward takes 15 positional arguments");
+    return nullptr;
+  }
+  if (!g_api.fwd) Py_RETURN_NONE;
+  Call c;
+  if (!take_tensor(a[0], c.q) || !take_tensor(a[1], c.k) || !take_tensor(a[2], c.v)) Py_RETURN_NONE;
+  if (mode_active()) Py_RETURN_NONE;
+  const Tensor &q = c.q, &k = c.k, &v = c.v;
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || element_type(q) < 0 || k.scalar_type() != q.scalar_type() ||
+      v.scalar_type() != q.scalar_type())
+    Py_RETURN_NONE;
+  c.diff = a[12] == Py_True;
+  c.seq_major = a[14] == Py_True;
+  const int64_t two = c.diff ? 2 : 1, B = q.size(0), Hq = q.size(1) / two, Hkv = k.size(1) / two, Lq = q.size(2), Lk = k.size(2),
+                D = q.size(3), Dv = v.size(3);
+  if (q.numel() == 0 || k.numel() == 0 || v.numel() == 0 || k.size(0) != B || v.size(0) != B || v.size(2) != Lk || k.size(3) != D ||
+      q.size(1) % two || k.size(1) % two || Hkv == 0 || Hq % Hkv || v.size(1) != Hkv)
+    Py_RETURN_NONE;
+  if (c.diff ? !(D == 64 && Dv == 128) : !(D == Dv && (D == 32 || D == 64 || D == 128))) Py_RETURN_NONE;
+  if (!addressable(q) || !addressable(k) || !addressable(v)) Py_RETURN_NONE;
+  const auto dev = q.device();
+  if (k.device() != dev || v.device() != dev || dev.index() != c10::hip::current_device()) Py_RETURN_NONE;
+  if (a[3] == Py_None) {
+    c.scale = 1.0 / std::sqrt((double)D);
+  } else {
+    c.scale = PyFloat_AsDouble(a[3]);
+  }
+  c.mask_kind = PyLong_AsLongLong(a[4]);
+  c.window = PyLong_AsLongLong(a[5]);
+  c.prefix = PyLong_AsLongLong(a[6]);
+  c.alibi_heads = PyLong_AsLongLong(a[8]);
+  c.softcap = PyFloat_AsDouble(a[9]);
+  c.lambda = PyFloat_AsDouble(a[13]);
+  if (PyErr_Occurred()) {  // (an argument of another type: the Python path converts it or says what is wrong)
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  constexpr int64_t kInt = INT32_MAX;
+  if (std::abs(c.window) > kInt || std::abs(c.prefix) > kInt || B > kInt || Lq > kInt || Lk > kInt) Py_RETURN_NONE;
+  if (a[7] != Py_None) {
+    if (!take_tensor(a[7], c.doc) || c.doc.scalar_type() != at::kLong || c.doc.dim() != 2 || c.doc.size(1) != Lk ||
+        (c.doc.size(0) != B && c.doc.size(0) != 1) || c.doc.stride(1) != 1 || c.doc.device() != dev)
+      Py_RETURN_NONE;
+  }
+  const bool is_doc = c.mask_kind == FL_MASK_DOCUMENT || c.mask_kind == FL_MASK_DOCUMENT_CAUSAL;
+  if (is_doc != c.doc.defined()) Py_RETURN_NONE;
+  PyObject* biases = a[10];
+  if (!PyTuple_Check(biases) && !PyList_Check(biases)) Py_RETURN_NONE;
+  const Py_ssize_t nb = PySequence_Fast_GET_SIZE(biases);
+  if (nb > 2) Py_RETURN_NONE;
+  for (Py_ssize_t i = 0; i < nb; ++i) {
+    PyObject* pair = PySequence_Fast_GET_ITEM(biases, i);
+    if (!PyTuple_Check(pair) || PyTuple_GET_SIZE(pair) != 2 || !PyLong_Check(PyTuple_GET_ITEM(pair, 1))) Py_RETURN_NONE;
+    Tensor& b = c.bias[i];
+    const int64_t div = c.bias_div[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(pair, 1));
+    if (!take_tensor(PyTuple_GET_ITEM(pair, 0), b) || b.dim() != 4 || b.device() != dev || div < 1 || B % div ||
+        (b.scalar_type() != at::kFloat && b.scalar_type() != q.scalar_type()))
+      Py_RETURN_NONE;
+    const int64_t want[4] = {B / div, Hq, Lq, Lk};
+    for (int ax = 0; ax < 4; ++ax)
+      if ((b.size(ax) != want[ax] && b.size(ax) != 1) || b.stride(ax) < 0) Py_RETURN_NONE;
+    if (b.size(3) != 1 && b.stride(3) != 1) Py_RETURN_NONE;
+  }
+  if (a[11] != Py_None) {
+    if (!take_tensor(a[11], c.gate) || c.gate.scalar_type() != q.scalar_type() || c.gate.dim() != 4 || c.gate.device() != dev ||
+        c.gate.size(0) != B || c.gate.size(1) != Hq || c.gate.size(2) != Lq || c.gate.size(3) != Dv || !addressable(c.gate))
+      Py_RETURN_NONE;
+  }
+  c.wants_grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() ||
+                                                (c.gate.defined() && c.gate.requires_grad()) ||
+                                                (c.bias[0].defined() && c.bias[0].requires_grad()) ||
+                                                (c.bias[1].defined() && c.bias[1].requires_grad()));
+  Tensor out;
+  if (c.wants_grad) {
+    if (c.diff || nb || c.gate.defined()) Py_RETURN_NONE;
+    c.seq_major = false;
+    try {
+      out = Attention::apply(q, k, v, c);
+    } catch (const Refused&) {
+      Py_RETURN_NONE;
+    }
+  } else {
+    out = launch_forward(c, nullptr);
+    if (!out.defined()) Py_RETURN_NONE;
+  }
+  return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(addresses): the C ABI's functions in the order of Api, as integers
+PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  void* f[6];
+  if (n != 6) {
+    PyErr_SetString(PyExc_TypeError, "bind takes six addresses");
+    return nullptr;
+  }
+  for (int i = 0; i < 6; ++i) f[i] = PyLong_AsVoidPtr(a[i]);
+  if (PyErr_Occurred()) return nullptr;
+  g_api.fwd = reinterpret_cast<decltype(g_api.fwd)>(f[0]);
+  g_api.bwd = reinterpret_cast<decltype(g_api.bwd)>(f[1]);
+  g_api.workspace = reinterpret_cast<decltype(g_api.workspace)>(f[2]);
+  g_api.bwd_workspace = reinterpret_cast<decltype(g_api.bwd_workspace)>(f[3]);
+  g_api.rows_plan = reinterpret_cast<decltype(g_api.rows_plan)>(f[4]);
+  g_api.last_error = reinterpret_cast<decltype(g_api.last_error)>(f[5]);
+  Py_RETURN_NONE;
+}
+
+PyMethodDef kMethods[] = {
+    {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_forward)), METH_FASTCALL, "Result of the call, or None when it is not of the plain kind."},
+    {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_bind)), METH_FASTCALL, "Takes the addresses of the C ABI's functions."},
+    {nullptr, nullptr, 0, nullptr}};
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "Native host path of the attention front ends.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+extern "C" __attribute__((visibility("default"))) PyObject* PyInit__host(void) { return PyModule_Create(&kModule); }

@@ -352,6 +352,13 @@ def dispatch(q, k, v, *, scale=None, mask_kind=_ffi.MASK_NONE, window=0, prefix=
     generator, so `torch.manual_seed` reproduces a run; the same seed gives the same decisions in forward and backward.
     `doc_workspace` (an `_ffi.DocWorkspace`) is used by the plain forward call only; traced and differentiable calls run
     their pre-pass every time.  `score_fn` = (kind, four constants), see `_ffi.attn_fwd`: forward only."""
+    if not dropout_p and score_fn is None and doc_workspace is None and not torch.compiler.is_compiling() and \
+            _ffi._host is not None:
+        # an ordinary call, differentiable or not, is launched by native code; None: it is not of that kind
+        out = _ffi._host.forward(q, k, v, scale, mask_kind, window, prefix, doc_ids, alibi_heads, softcap, biases, gate, diff,
+                            lambda_full, seq_major_out)
+        if out is not None:
+            return out
     dropout_p = float(dropout_p)
     _ffi.dropout_threshold(dropout_p)  # range check
     if q.dim() == 4 and k.dim() == 4 and v.dim() == 4 and q.is_cuda and (q.numel() == 0 or k.size(2) == 0):
