@@ -145,7 +145,8 @@ def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
         raise ImportError("flashlight_amd/_host.so is missing or does not load: build it with `python -m flashlight_amd.build`") from e
     _host = host_module
     _host.bind(*(C.cast(getattr(lib, f), C.c_void_p).value for f in (
-        "fl_attn_fwd", "fl_attn_bwd", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_rows_plan", "fl_last_error")))
+        "fl_attn_fwd", "fl_attn_bwd", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_rows_plan",
+        "fl_attn_shared_bias_bwd_bytes", "fl_attn_shared_bias_bwd", "fl_last_error")))
     _lib = lib
     return lib
 

@@ -127,12 +127,13 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
         objs.append(o)
         if not o.exists():
             tasks.append(([cc, *HIPCC_FLAGS, f"-DFL_INST_F16={f16}", "-c", str(CSRC / "pairbias_unit.hip"), "-o", str(o)], o))
-    # the few-rows forward: one unit per element type
-    for f16 in (0, 1):
-        o = objdir / f"rows{'_f16' if f16 else ''}.o"
-        objs.append(o)
-        if not o.exists():
-            tasks.append(([cc, *HIPCC_FLAGS, f"-DFL_INST_F16={f16}", "-c", str(CSRC / "rows_unit.hip"), "-o", str(o)], o))
+    # the few-rows forward and the shared-bias backward: one unit each per element type
+    for unit in ("rows", "pairbias_bwd"):
+        for f16 in (0, 1):
+            o = objdir / f"{unit}{'_f16' if f16 else ''}.o"
+            objs.append(o)
+            if not o.exists():
+                tasks.append(([cc, *HIPCC_FLAGS, f"-DFL_INST_F16={f16}", "-c", str(CSRC / f"{unit}_unit.hip"), "-o", str(o)], o))
     # the instance tables are host data only: compiling them for the device would reference the host launchers
     for src, extra in (("instances_table.hip", ["--cuda-host-only"]), ("bwd_table.hip", ["--cuda-host-only"]),
                        ("api.hip", []), ("ipa_pack.hip", []), ("merge_chunks.hip", [])):

@@ -9,6 +9,7 @@
 #include "flashlight_amd.h"
 #include "bwd_instances.h"
 #include "instances.h"
+#include "pairbias_bwd_instances.h"
 #include "pairbias_instances.h"
 #include "rows_instances.h"
 
@@ -715,6 +716,54 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   return true;
 }
 
+
+// Layout of the shared-bias backward's scratch, in bytes from its start (parts aligned to 256).
+struct SBScratch {
+  int dense = -1, row = -1;  // which operand is the shared one, which the row per batch entry
+  int chunks = 1, chunk_len = 1;
+  uint64_t delta = 0, rowb = 0, dgated = 0, part = 0, total = 0;
+};
+// Whether the forward call *p is one whose gradients the shared-bias backward computes.
+bool plan_shared_bias_bwd(const fl_attn_params* p, SBScratch* out) {
+  if (p->Dqk != p->Dv || (p->Dqk != 32 && p->Dqk != 64) || p->Hq != p->Hkv || p->Lq != p->Lk || p->Lk > 512 || p->Lk <= 0 || p->B <= 0 ||
+      p->Hq <= 0 || p->mask_kind != FL_MASK_NONE || p->alibi_heads > 0 || p->softcap > 0.f || p->diff || p->attended_dump ||
+      p->dropout_threshold || p->score_fn != FL_SCORE_NONE)
+    return false;
+  SBScratch x;
+  for (int i = 0; i < 2; ++i) {
+    if (!p->bias[i]) continue;
+    const int64_t* st = p->bias_strides[i];
+    if (p->bias_batch_div[i] <= 0 || p->B % p->bias_batch_div[i]) return false;
+    if (st[1] == 0 && st[2] == 0 && x.row < 0 && (p->Hq > 1 || p->Lq > 1)) x.row = i;
+    else if ((st[1] != 0 || p->Hq == 1) && (st[2] != 0 || p->Lq == 1) && (st[3] == 1 || p->Lk == 1) && x.dense < 0) x.dense = i;
+    else return false;
+  }
+  if (x.dense < 0) return false;
+  // per-lane byte offsets inside one (batch entry, head) are 32-bit
+  for (const int64_t* st : {p->q_strides, p->k_strides, p->v_strides, p->o_strides})
+    if (st[2] < 0 || st[2] >= (1 << 20)) return false;
+  const int64_t S = p->Lk, H = p->Hq, div = p->bias_batch_div[x.dense], groups = p->B / div, tiles = (S + 31) / 32;
+  // entries per workgroup: as many as leave one round of workgroups
+  const int per_cu = fl::pairbias_bwd_shape(p->Dqk, (int)S).lds_bytes <= 80 * 1024 ? 2 : 1;
+  int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(div, 256 * per_cu / (groups * H * tiles)));
+  const int64_t len = (div + chunks - 1) / chunks;
+  chunks = (div + len - 1) / len;
+  if (groups * chunks * H * tiles > (1 << 28)) return false;
+  x.chunks = (int)chunks;
+  x.chunk_len = (int)len;
+  auto add = [&](uint64_t bytes) {
+    const uint64_t at = x.total;
+    x.total += (bytes + 255) / 256 * 256;
+    return at;
+  };
+  x.delta = add((uint64_t)p->B * H * S * 4);
+  x.rowb = add(x.row >= 0 ? (uint64_t)p->B * S * 4 : 0);
+  x.dgated = add(p->gate ? (uint64_t)p->B * H * S * p->Dv * 2 : 0);
+  x.part = add((uint64_t)groups * chunks * H * S * ((S + 3) / 4 * 4) * 4);
+  *out = x;
+  return true;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1071,6 +1120,119 @@ int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream_) {
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dQ kernel failed: %s", hipGetErrorString(e));
   e = in->launch_dkv(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dK/dV kernel failed: %s", hipGetErrorString(e));
+  return 0;
+}
+
+uint64_t fl_attn_shared_bias_bwd_bytes(const fl_attn_params* p) {
+  SBScratch x;
+  return p && plan_shared_bias_bwd(p, &x) ? x.total : 0;
+}
+
+int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* stream_) {
+  if (!b) return fail(FL_ERR_NULL, "params is null");
+  const fl_attn_params* p = &b->fwd;
+  int rc = validate(p, nullptr);
+  if (rc) return rc;
+  SBScratch x;
+  if (!plan_shared_bias_bwd(p, &x)) return fail(FL_ERR_UNSUPPORTED, "fl_attn_shared_bias_bwd does not take this call");
+  if ((rc = check_ptr("dout", b->dout, 16)) || (rc = check_ptr("dq", b->dq, 8)) || (rc = check_ptr("dk", b->dk, 8)) ||
+      (rc = check_ptr("dv", b->dv, 8)) || (rc = check_ptr("fwd.lse", p->lse, 4)) || (rc = check_ptr("fwd.o", p->o, 16)) ||
+      (rc = check_strides("o", p->o_strides, 8)) || (rc = check_strides("dout", b->dout_strides, 8)) ||
+      (rc = check_strides("dq", b->dq_strides, 4)) || (rc = check_strides("dk", b->dk_strides, 4)) ||
+      (rc = check_strides("dv", b->dv_strides, 4)))
+    return rc;
+  for (const int64_t* st : {b->dout_strides, b->dq_strides, b->dk_strides, b->dv_strides})
+    if (st[2] >= (1 << 20)) return fail(FL_ERR_STRIDE, "sequence stride of a gradient too large (%lld elements)", (long long)st[2]);
+  if (p->gate && ((rc = check_ptr("gate", p->gate, 16)) || (rc = check_strides("gate", p->gate_strides, 8)) ||
+                  (rc = check_ptr("dgate", b->dgate, 16)) || (rc = check_strides("dgate", b->dgate_strides, 8))))
+    return rc;
+  if ((rc = check_ptr("workspace", b->workspace, 256))) return rc;
+  if (b->workspace_bytes < x.total)
+    return fail(FL_ERR_WORKSPACE, "workspace of %llu bytes needed, got %llu", (unsigned long long)x.total, (unsigned long long)b->workspace_bytes);
+  const bool f32 = p->bias_dtype[x.dense] == FL_F32;
+  if (b->dbias && reinterpret_cast<uintptr_t>(b->dbias) % (f32 ? 4 : 2)) return fail(FL_ERR_ALIGN, "dbias is not aligned");
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  unsigned char* ws = static_cast<unsigned char*>(b->workspace);
+  const bool f16 = p->dtype == FL_F16, gate = p->gate != nullptr;
+
+  fl::SBPrepParams pp;
+  std::memset(&pp, 0, sizeof(pp));
+  pp.out = static_cast<const fl::bf16_t*>(p->o);
+  pp.dout = static_cast<const fl::bf16_t*>(b->dout);
+  pp.gate = static_cast<const fl::bf16_t*>(p->gate);
+  pp.dgated = reinterpret_cast<fl::bf16_t*>(ws + x.dgated);
+  pp.dgate = static_cast<fl::bf16_t*>(b->dgate);
+  pp.delta = reinterpret_cast<float*>(ws + x.delta);
+  pp.row_div = 1;
+  if (x.row >= 0) {
+    pp.row = p->bias[x.row];
+    pp.rowb = reinterpret_cast<float*>(ws + x.rowb);
+    pp.row_batch = p->bias_strides[x.row][0];
+    pp.row_key = (int)p->bias_strides[x.row][3];
+    pp.row_div = p->bias_batch_div[x.row];
+    pp.row_f32 = p->bias_dtype[x.row] == FL_F32;
+  }
+  pp.B = p->B;
+  pp.H = p->Hq;
+  pp.S = p->Lq;
+  const int64_t row = (int64_t)p->Hq * p->Dv, dgs[3] = {row * p->Lq, p->Dv, row};  // gated dO: [batch][position][head][dim]
+  for (int i = 0; i < 3; ++i) {
+    pp.os[i] = p->o_strides[i];
+    pp.dos[i] = b->dout_strides[i];
+    pp.gs[i] = p->gate_strides[i];
+    pp.dgs[i] = b->dgate_strides[i];
+    pp.dgds[i] = dgs[i];
+  }
+  hipError_t e = (f16 ? fl::launch_pairbias_bwd_prep_f16 : fl::launch_pairbias_bwd_prep_bf16)(p->Dqk, gate, pp, stream);
+  if (e != hipSuccess) return fail((int)e, "shared-bias backward: launch of the row-sum kernel failed: %s", hipGetErrorString(e));
+
+  fl::SBParams sp;
+  std::memset(&sp, 0, sizeof(sp));
+  sp.q = static_cast<const fl::bf16_t*>(p->q);
+  sp.k = static_cast<const fl::bf16_t*>(p->k);
+  sp.v = static_cast<const fl::bf16_t*>(p->v);
+  sp.dout = gate ? pp.dgated : pp.dout;
+  sp.lse = p->lse;
+  sp.delta = pp.delta;
+  sp.rowb = pp.rowb;
+  sp.dq = static_cast<fl::bf16_t*>(b->dq);
+  sp.dk = static_cast<fl::bf16_t*>(b->dk);
+  sp.dv = static_cast<fl::bf16_t*>(b->dv);
+  for (int i = 0; i < 3; ++i) {
+    sp.qs[i] = p->q_strides[i];
+    sp.ks[i] = p->k_strides[i];
+    sp.vs[i] = p->v_strides[i];
+    sp.dos[i] = gate ? dgs[i] : b->dout_strides[i];
+    sp.dqs[i] = b->dq_strides[i];
+    sp.dks[i] = b->dk_strides[i];
+    sp.dvs[i] = b->dv_strides[i];
+    sp.bs[i] = p->bias_strides[x.dense][i];
+  }
+  sp.bias = p->bias[x.dense];
+  sp.bias_f32 = f32;
+  sp.bias_vec = p->Lk % 4 == 0 && sp.bs[0] % 4 == 0 && sp.bs[1] % 4 == 0 && sp.bs[2] % 4 == 0 &&
+                reinterpret_cast<uintptr_t>(sp.bias) % (f32 ? 16 : 8) == 0;
+  sp.B = p->B;
+  sp.H = p->Hq;
+  sp.S = p->Lk;
+  sp.div = p->bias_batch_div[x.dense];
+  sp.groups = sp.B / sp.div;
+  sp.chunks = x.chunks;
+  sp.chunk_len = x.chunk_len;
+  sp.tiles = (sp.S + 31) / 32;
+  sp.s_pad = (sp.S + 3) / 4 * 4;
+  sp.scale = p->scale;
+  sp.scale_log2 = p->scale * 1.4426950408889634f;
+  sp.dbias_part = b->dbias ? reinterpret_cast<float*>(ws + x.part) : nullptr;
+  const fl::SBShape shape = fl::pairbias_bwd_shape(p->Dqk, sp.S);
+  sp.slots = shape.slots;
+  e = (f16 ? fl::launch_pairbias_bwd_f16 : fl::launch_pairbias_bwd_bf16)(p->Dqk, shape, sp, stream);
+  if (e != hipSuccess) return fail((int)e, "shared-bias backward: launch failed: %s", hipGetErrorString(e));
+  if (b->dbias) {
+    e = (f16 ? fl::launch_pairbias_bwd_reduce_f16 : fl::launch_pairbias_bwd_reduce_bf16)(f32, sp, b->dbias, stream);
+    if (e != hipSuccess) return fail((int)e, "shared-bias backward: launch of the reduction failed: %s", hipGetErrorString(e));
+  }
+  g_err[0] = 0;
   return 0;
 }
 

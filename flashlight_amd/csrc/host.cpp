@@ -35,8 +35,11 @@ struct Api {
   uint64_t (*workspace)(const fl_attn_params*) = nullptr;
   uint64_t (*bwd_workspace)(const fl_attn_params*) = nullptr;
   int (*rows_plan)(const fl_attn_params*, uint64_t*) = nullptr;
+  uint64_t (*shared_bias_bwd_bytes)(const fl_attn_params*) = nullptr;
+  int (*shared_bias_bwd)(const fl_attn_shared_bias_bwd_params*, void*) = nullptr;
   const char* (*last_error)(void) = nullptr;
 } g_api;
+constexpr int kApiFunctions = 8;
 
 // One call's arguments.  The tensors are the caller's; `doc`, `bias` and `gate` may be undefined.
 struct Call {
@@ -83,8 +86,8 @@ int element_type(const Tensor& t) {
   return t.scalar_type() == at::kBFloat16 ? FL_BF16 : t.scalar_type() == at::kHalf ? FL_F16 : -1;
 }
 
-// Fills what the forward and the backward share; false if the call is not of the plain kind.
-bool fill(const Call& c, fl_attn_params& p) {
+// Fills what the forward and the backward share.
+void fill(const Call& c, fl_attn_params& p) {
   const Tensor &q = c.q, &k = c.k, &v = c.v;
   const int two = c.diff ? 2 : 1;
   p.dtype = element_type(q);
@@ -126,7 +129,6 @@ bool fill(const Call& c, fl_attn_params& p) {
     p.gate = c.gate.const_data_ptr();
     set_strides(p.gate_strides, c.gate);
   }
-  return true;
 }
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
@@ -138,7 +140,8 @@ Tensor launch_forward(const Call& c, Tensor* lse) {
   fill(c, p);
   Tensor q = c.q, out;
   const auto opt = q.options().requires_grad(false);
-  if (c.seq_major) out = at::empty({p.B, p.Lq, p.Hq, p.Dv}, opt).transpose(1, 2);
+  const int64_t row = (int64_t)p.Hq * p.Dv;  // (seq_major: memory order [batch, position, head, dim])
+  if (c.seq_major) out = at::empty_strided({p.B, p.Hq, p.Lq, p.Dv}, {row * p.Lq, p.Dv, row, 1}, opt);
   else out = at::empty({p.B, p.Hq, p.Lq, p.Dv}, opt);
   p.o = out.data_ptr();
   set_strides(p.o_strides, out);
@@ -180,7 +183,47 @@ Tensor launch_forward(const Call& c, Tensor* lse) {
 
 struct Refused {};  // the C ABI does not take the call: the Python path then says why
 
-constexpr const char* kOnce = "flashlight_amd: the gradients are not differentiable a second time";
+// Fresh memory in the operand's own order where that is dense, contiguous otherwise.
+Tensor empty_for_gradient(const Tensor& t) {
+  const auto opt = t.options().requires_grad(false);
+  return t.is_non_overlapping_and_dense() ? at::empty_strided(t.sizes(), t.strides(), opt) : at::empty(t.sizes(), opt);
+}
+
+// The call's scalars, kept with the node between forward and backward.
+void keep_scalars(AutogradContext* ctx, const Call& c) {
+  ctx->saved_data["i"] = std::vector<int64_t>{c.mask_kind, c.window, c.prefix, c.alibi_heads, c.bias_div[0], c.bias_div[1]};
+  ctx->saved_data["f"] = std::vector<double>{c.scale, c.softcap};
+}
+void take_scalars(AutogradContext* ctx, Call& c) {
+  const auto ints = ctx->saved_data["i"].toIntVector();
+  const auto floats = ctx->saved_data["f"].toDoubleVector();
+  c.mask_kind = ints[0];
+  c.window = ints[1];
+  c.prefix = ints[2];
+  c.alibi_heads = ints[3];
+  c.bias_div[0] = ints[4];
+  c.bias_div[1] = ints[5];
+  c.scale = floats[0];
+  c.softcap = floats[1];
+}
+
+// Under create_graph the gradients say that they have none of their own, instead of looking like constants.
+void once_differentiable(variable_list& grads, bool grad_mode) {
+  if (!grad_mode) return;
+  variable_list some;
+  for (auto& t : grads)
+    if (t.defined()) some.push_back(t.detach().requires_grad_(true));
+  some = (*std::make_shared<torch::autograd::DelayedError>("flashlight_amd: the gradients are not differentiable a second time",
+                                                           (int64_t)some.size()))(std::move(some));
+  size_t i = 0;
+  for (auto& t : grads)
+    if (t.defined()) t = some[i++];
+}
+
+Tensor prepare_dout(const Tensor& grad, const Tensor& like) {
+  Tensor d = grad.to(like.scalar_type());
+  return addressable(d) ? d : d.contiguous();
+}
 
 struct Attention : torch::autograd::Function<Attention> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Call& c) {
@@ -188,42 +231,32 @@ struct Attention : torch::autograd::Function<Attention> {
     Tensor out = launch_forward(c, &lse);
     if (!out.defined()) throw Refused();
     ctx->save_for_backward({q, k, v, out, lse});
-    ctx->saved_data["i"] = std::vector<int64_t>{c.mask_kind, c.window, c.prefix, c.alibi_heads};
-    ctx->saved_data["f"] = std::vector<double>{c.scale, c.softcap};
+    keep_scalars(ctx, c);
     if (c.doc.defined()) ctx->saved_data["doc"] = c.doc;
     return out;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    const auto ints = ctx->saved_data["i"].toIntVector();
-    const auto floats = ctx->saved_data["f"].toDoubleVector();
     Call c;
     c.q = saved[0];
     c.k = saved[1];
     c.v = saved[2];
-    c.mask_kind = ints[0];
-    c.window = ints[1];
-    c.prefix = ints[2];
-    c.alibi_heads = ints[3];
-    c.scale = floats[0];
-    c.softcap = floats[1];
+    take_scalars(ctx, c);
     if (ctx->saved_data.count("doc")) c.doc = ctx->saved_data["doc"].toTensor();
     const Tensor &out = saved[3], &lse = saved[4];
     variable_list result(4);
     if (!grads[0].defined()) return result;
-    const bool again = at::GradMode::is_enabled();
+    const bool grad_mode = at::GradMode::is_enabled();
     {
       at::AutoGradMode off(false);
-      Tensor dout = grads[0].to(c.q.scalar_type());
-      if (!addressable(dout)) dout = dout.contiguous();
-      const auto opt = c.q.options().requires_grad(false);
+      const Tensor dout = prepare_dout(grads[0], c.q);
       fl_attn_bwd_params b = {};
       fill(c, b.fwd);
       b.fwd.o = const_cast<void*>(out.const_data_ptr());
       set_strides(b.fwd.o_strides, out);
       b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
-      Tensor dq = at::empty(c.q.sizes(), opt), dk = at::empty(c.k.sizes(), opt), dv = at::empty(c.v.sizes(), opt);
+      Tensor dq = empty_for_gradient(c.q), dk = empty_for_gradient(c.k), dv = empty_for_gradient(c.v);
       Tensor delta = at::empty(lse.sizes(), lse.options()), ws;
       b.dout = dout.const_data_ptr();
       b.dq = dq.data_ptr();
@@ -235,7 +268,7 @@ struct Attention : torch::autograd::Function<Attention> {
       set_strides(b.dk_strides, dk);
       set_strides(b.dv_strides, dv);
       if (const uint64_t bytes = g_api.bwd_workspace(&b.fwd)) {
-        ws = at::empty({(int64_t)bytes}, opt.dtype(at::kByte));
+        ws = at::empty({(int64_t)bytes}, delta.options().dtype(at::kByte));
         b.fwd.workspace = ws.data_ptr();
         b.fwd.workspace_bytes = bytes;
       }
@@ -245,16 +278,83 @@ struct Attention : torch::autograd::Function<Attention> {
       result[1] = dk;
       result[2] = dv;
     }
-    if (again) {
-      // under create_graph the gradients say that they have none of their own, instead of looking like constants
-      variable_list three(result.begin(), result.begin() + 3);
-      for (auto& t : three) t = t.detach().requires_grad_(true);
-      three = (*std::make_shared<torch::autograd::DelayedError>(kOnce, 3))(std::move(three));
-      std::copy(three.begin(), three.end(), result.begin());
-    }
+    once_differentiable(result, grad_mode);
     return result;
   }
 };
+
+// Calls with a bias shared by batch entries, and optionally the gate (fl_attn_shared_bias_bwd).  bias[0] is the shared
+// operand here, bias[1] the row per batch entry, which takes no gradient.
+struct SharedBias : torch::autograd::Function<SharedBias> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& bias,
+                        const std::optional<Tensor>& row, const std::optional<Tensor>& gate, const Call& c) {
+    Tensor lse;
+    Tensor out = launch_forward(c, &lse);
+    if (!out.defined()) throw Refused();
+    ctx->save_for_backward({q, k, v, bias, row.value_or(Tensor()), gate.value_or(Tensor()), out, lse});
+    keep_scalars(ctx, c);
+    return out;
+  }
+
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const auto saved = ctx->get_saved_variables();
+    Call c;
+    c.q = saved[0];
+    c.k = saved[1];
+    c.v = saved[2];
+    c.bias[0] = saved[3];
+    c.bias[1] = saved[4];
+    c.gate = saved[5];
+    take_scalars(ctx, c);
+    const Tensor &out = saved[6], &lse = saved[7];
+    variable_list result(7);
+    if (!grads[0].defined()) return result;
+    const bool grad_mode = at::GradMode::is_enabled();
+    {
+      at::AutoGradMode off(false);
+      const Tensor dout = prepare_dout(grads[0], c.q);
+      fl_attn_shared_bias_bwd_params b = {};
+      fill(c, b.fwd);
+      b.fwd.o = const_cast<void*>(out.const_data_ptr());
+      set_strides(b.fwd.o_strides, out);
+      b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
+      Tensor dq = empty_for_gradient(c.q), dk = empty_for_gradient(c.k), dv = empty_for_gradient(c.v);
+      b.dout = dout.const_data_ptr();
+      b.dq = dq.data_ptr();
+      b.dk = dk.data_ptr();
+      b.dv = dv.data_ptr();
+      set_strides(b.dout_strides, dout);
+      set_strides(b.dq_strides, dq);
+      set_strides(b.dk_strides, dk);
+      set_strides(b.dv_strides, dv);
+      Tensor dgate, dbias;
+      if (c.gate.defined()) {
+        dgate = empty_for_gradient(c.gate);
+        b.dgate = dgate.data_ptr();
+        set_strides(b.dgate_strides, dgate);
+      }
+      if (ctx->needs_input_grad(3)) {
+        dbias = at::empty(c.bias[0].sizes(), c.bias[0].options().requires_grad(false));
+        b.dbias = dbias.data_ptr();
+      }
+      const uint64_t bytes = g_api.shared_bias_bwd_bytes(&b.fwd);
+      Tensor ws = at::empty({(int64_t)bytes}, lse.options().dtype(at::kByte));
+      b.workspace = ws.data_ptr();
+      b.workspace_bytes = bytes;
+      const int rc = g_api.shared_bias_bwd(&b, current_stream());
+      TORCH_CHECK(rc == 0, "flashlight_amd error ", rc, ": ", g_api.last_error());
+      result[0] = dq;
+      result[1] = dk;
+      result[2] = dv;
+      result[3] = dbias;
+      result[5] = dgate;
+    }
+    once_differentiable(result, grad_mode);
+    return result;
+  }
+};
+
+std::optional<Tensor> given(const Tensor& t) { return t.defined() ? std::optional<Tensor>(t) : std::nullopt; }
 
 // ---- Python boundary -----------------------------------------------------------------------------------------------------
 
@@ -342,10 +442,23 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                                 (c.bias[1].defined() && c.bias[1].requires_grad()));
   Tensor out;
   if (c.wants_grad) {
-    if (c.diff || nb || c.gate.defined()) Py_RETURN_NONE;
-    c.seq_major = false;
+    if (c.diff) Py_RETURN_NONE;
+    if (nb || c.gate.defined()) {
+      if (c.bias[1].defined() && c.bias[1].size(1) == Hq && c.bias[1].size(2) == Lq && Hq * Lq > 1) {  // the shared operand first
+        std::swap(c.bias[0], c.bias[1]);
+        std::swap(c.bias_div[0], c.bias_div[1]);
+      }
+      fl_attn_params p = {};
+      fill(c, p);
+      if (!c.bias[0].defined() || c.bias[0].size(1) != Hq || c.bias[0].size(2) != Lq || c.bias[0].size(3) != Lk ||
+          (c.bias[1].defined() && (c.bias[1].requires_grad() || c.bias[1].size(1) != 1 || c.bias[1].size(2) != 1)) ||
+          !g_api.shared_bias_bwd_bytes(&p))
+        Py_RETURN_NONE;
+    } else {
+      c.seq_major = false;
+    }
     try {
-      out = Attention::apply(q, k, v, c);
+      out = nb ? SharedBias::apply(q, k, v, c.bias[0], given(c.bias[1]), given(c.gate), c) : Attention::apply(q, k, v, c);
     } catch (const Refused&) {
       Py_RETURN_NONE;
     }
@@ -359,19 +472,21 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // bind(addresses): the C ABI's functions in the order of Api, as integers
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  void* f[6];
-  if (n != 6) {
-    PyErr_SetString(PyExc_TypeError, "bind takes six addresses");
+  void* f[kApiFunctions];
+  if (n != kApiFunctions) {
+    PyErr_SetString(PyExc_TypeError, "bind takes the addresses of eight functions");
     return nullptr;
   }
-  for (int i = 0; i < 6; ++i) f[i] = PyLong_AsVoidPtr(a[i]);
+  for (int i = 0; i < kApiFunctions; ++i) f[i] = PyLong_AsVoidPtr(a[i]);
   if (PyErr_Occurred()) return nullptr;
   g_api.fwd = reinterpret_cast<decltype(g_api.fwd)>(f[0]);
   g_api.bwd = reinterpret_cast<decltype(g_api.bwd)>(f[1]);
   g_api.workspace = reinterpret_cast<decltype(g_api.workspace)>(f[2]);
   g_api.bwd_workspace = reinterpret_cast<decltype(g_api.bwd_workspace)>(f[3]);
   g_api.rows_plan = reinterpret_cast<decltype(g_api.rows_plan)>(f[4]);
-  g_api.last_error = reinterpret_cast<decltype(g_api.last_error)>(f[5]);
+  g_api.shared_bias_bwd_bytes = reinterpret_cast<decltype(g_api.shared_bias_bwd_bytes)>(f[5]);
+  g_api.shared_bias_bwd = reinterpret_cast<decltype(g_api.shared_bias_bwd)>(f[6]);
+  g_api.last_error = reinterpret_cast<decltype(g_api.last_error)>(f[7]);
   Py_RETURN_NONE;
 }
 

@@ -1,0 +1,462 @@
+// Backward of attention with one dense bias shared by several consecutive batch entries (the Evoformer's row attention:
+// a pair bias over all rows of an alignment), with an optional bias row per batch entry and an optional sigmoid gate.
+//
+// What bounded it in the general backward (bwd_kernel.h, F_BIAS) were the bias's two ends: a 2-byte global load per score
+// in both roles, and the bias gradient as a dense fp32 array of every batch entry's score gradients (4 bytes per score
+// cleared, written, and read back by a reduction; 268 MB each for 128 x 8 x 256 x 256).  Here a workgroup stays with one
+// 32-row stripe of one head's score matrix and walks over the batch entries: the bias of the stripe is read once into
+// registers, and in the role that produces dQ the score gradients of all its entries add up in registers too, so that
+// the bias gradient leaves as one fp32 tile per workgroup, summed over the few workgroups that share a stripe by
+// pairbias_bwd_reduce_kernel in a fixed order (no atomics).
+//
+// Two roles, as in the general backward, every product with the streamed tile as the MFMA A operand:
+//   ROLE_DQ   owns 32 queries, streams all keys:     S^T = K.Q^T, dP^T = V.dO^T, dQ^T += K^T.dS^T, dBias += dS^T
+//   ROLE_DKV  owns 32 keys, streams all queries:     S = Q.K^T,   dP = dO.V^T,   dK^T += Q^T.dS,   dV^T += dO^T.P
+// The waves of a workgroup split the streamed rows (NB blocks of 32 each), fetch their own rows into their own part of LDS
+// (no barrier for them), and add up their partial dQ / dK, dV through LDS once per batch entry.  The next entry's rows are
+// on their way while one is worked on.  The sequence has at most 512 positions.
+//
+// Measured, 128 x 8 x 256 x 256, head dim 32, mask row and gate, bf16, whole step: 852 -> 177 us (ROLE_DQ 325 -> 46, ROLE_DKV
+// 232 -> 55, row sums and gate 150 -> 20, clearing and summing the bias gradient 97 -> 4).  Per score seven vector
+// instructions are left, and no global load, conversion or store; what bounds the roles now is the chain an entry goes
+// through (tiles, two products, weights, products, sums over the waves: 2.1 and 2.7 us) with two waves per SIMD to cover it:
+// the vector unit issues in 35 % of the cycles.  Two blocks per wave in four waves beat one in eight (67 and 93 us: the sums
+// over the waves cost more than the occupancy gains).
+#pragma once
+#include "fwd_kernel.h"
+
+namespace fl {
+
+struct SBParams {
+  const bf16_t *q, *k, *v, *dout;  // dout: already multiplied by the gate
+  const float *lse, *delta;        // [B, H, S]; delta: minus rowsum(dO o O)
+  const float* rowb;               // [B, S] in log2 units, or null
+  bf16_t *dq, *dk, *dv;
+  int64_t qs[3], ks[3], vs[3], dos[3], dqs[3], dks[3], dvs[3];  // element strides: batch, head, seq
+  const void* bias;
+  int64_t bs[3];                   // group, head, query (key stride 1)
+  int32_t bias_f32;
+  int32_t bias_vec;                // rows of the bias may be read four keys at a time
+  int32_t B, H, S;
+  int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
+  int32_t tiles;                   // 32-row stripes
+  int32_t slots;                   // tiles of batch entries resident in LDS: 2, or 1 where two do not fit
+  int32_t s_pad;                   // row length of the partial bias gradient (S rounded up to 4)
+  float scale, scale_log2;
+  float* dbias_part;               // [groups][chunks][H][S][s_pad], or null: no gradient of the bias wanted
+};
+
+// rows of an operand that are not in the sequence repeat the last one; their weights are 0 (their bias is -inf)
+template <int D_, int ROLE_, int NB_, bool ROWB_, class Elem_>
+struct SBTraits {
+  using Elem = Elem_;
+  static constexpr int D = D_, ROLE = ROLE_, NB = NB_;
+  static constexpr bool ROWB = ROWB_, DQ = ROLE_ == 0;
+  static constexpr int KS = D / 16, DB = D / 32;
+  static constexpr int T_BYTES = NB * 32 * D * 2;        // one streamed operand of one wave
+  static constexpr int O_BYTES = 32 * D * 2;             // one owned operand
+  static constexpr int PARK = 32 * D * 4;                // partial sums of one accumulator set of one wave
+  // per wave and slot: both streamed operands, and the fp32 values per streamed row (LSE and Delta in ROLE_DKV, the bias
+  // row in ROLE_DQ): two areas of 64 floats
+  static constexpr int W_BYTES = 2 * T_BYTES + 2 * 256;
+  static constexpr int S_OWN = 2 * O_BYTES + 2 * 256;    // per slot: owned operands and their values per row
+  static constexpr int TPW = T_BYTES / 1024;             // 1 KiB transfers per streamed operand
+  // the partial sums go where the consumed tiles were: both sets at once when a wave's two tiles have room for them
+  static constexpr bool ONE_PASS = DQ || 2 * T_BYTES >= 2 * PARK;
+};
+
+template <class T>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+void pairbias_bwd_kernel(const SBParams p) {
+  constexpr int D = T::D, NB = T::NB, KS = T::KS, DB = T::DB;
+  constexpr bool kDQ = T::DQ, kRowB = T::ROWB;
+  constexpr float kLog2e = 1.4426950408889634f;
+  using E = typename T::Elem;
+  typedef E ex8 __attribute__((ext_vector_type(8)));
+  typedef E ex4 __attribute__((ext_vector_type(4)));
+  using L = TileLayout<D>;
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+
+  const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+  const int NW = blockDim.x / 64, NT = blockDim.x;
+  const int r = lane % 32, h = lane / 32;
+
+  // ---- workgroup -> (group, chunk of batch entries, head, stripe): the stripes of one (chunk, head) read the same
+  // tensors and stay on one XCD
+  int tile, uc;
+  {
+    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
+    tile = i % p.tiles;
+    uc = i / p.tiles * 8 + x;
+    if (uc >= p.groups * p.chunks * p.H) return;  // (before any barrier)
+  }
+  const int head = uc % p.H, gc = uc / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
+  const int n0 = group * p.div + chunk * p.chunk_len, n1 = min(group * p.div + p.div, n0 + p.chunk_len);
+  const int o0 = tile * 32, S = p.S;
+  const int own = o0 + r;                 // this lane's query (ROLE_DQ) or key
+  const int w0 = wave * NB * 32;          // first streamed row of this wave
+
+  // ---- the stripe's bias in log2 units, -inf outside the score matrix: register (b, i) is streamed row
+  // w0 + 32 b + 8 (i / 4) + 4 h + i % 4 against this lane's owned row
+  float bias[NB][16];
+  {
+    const int64_t base = (int64_t)group * p.bs[0] + (int64_t)head * p.bs[1];
+    // (one loop per element type, and the loads before anything looks at them: 16 NB loads in flight together)
+    auto fetch = [&](auto* src) FL_INLINE {
+      using X = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;
+      typedef X x4 __attribute__((ext_vector_type(4)));
+      X x[NB][16];
+      if (kDQ && p.bias_vec) {  // four consecutive keys of the lane's query in one load (5 -> 1 us for NB = 2)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const x4 v = *reinterpret_cast<const x4*>(src + base + (int64_t)min(own, S - 1) * p.bs[2] + min(w0 + 32 * b + 8 * g + 4 * h, S - 4));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[b][4 * g + e] = v[e];
+          }
+      } else {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const int st = w0 + 32 * b + 8 * (i / 4) + 4 * h + i % 4;
+            x[b][i] = src[base + (int64_t)min(kDQ ? own : st, S - 1) * p.bs[2] + min(kDQ ? st : own, S - 1)];
+          }
+      }
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int st = w0 + 32 * b + 8 * (i / 4) + 4 * h + i % 4;
+          bias[b][i] = (st < S && own < S) ? (float)x[b][i] * kLog2e : -INFINITY;
+        }
+    };
+    if (p.bias_f32) fetch(static_cast<const float*>(p.bias));
+    else fetch(static_cast<const E*>(p.bias));
+  }
+  float db[kDQ ? NB : 1][16];
+  if constexpr (kDQ) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) db[b][i] = 0.f;
+  }
+
+  // ---- transfers of a batch entry into ring slot `slot`.  The per-lane offsets do not change from entry to entry and the
+  // scalar base addresses advance by one batch stride: per entry a transfer costs its issue and nothing else.
+  const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem);
+  const unsigned w_bytes = T::W_BYTES * NW, slot_bytes = w_bytes + T::S_OWN;
+  constexpr int RPT = 512 / D;  // rows per 1 KiB transfer
+  // byte offset of this lane's 16 bytes of transfer `it` of rows row0 .., rows past the end repeating the last one
+  auto lane_offset = [&](int row0, int it, int64_t stride) FL_INLINE -> unsigned {
+    const int row = it * RPT + lane / L::CPR;
+    return (uint32_t)min(row0 + row, S - 1) * ((uint32_t)stride * 2u) + (uint32_t)(L::swz_kv(row, lane % L::CPR) * 16);
+  };
+  struct Operand {
+    uint64_t at;   // address of the next entry's [S][D] rows of this head
+    uint64_t step;
+  };
+  auto operand = [&](const void* base, const int64_t (&st)[3]) FL_INLINE -> Operand {
+    return {uniform_ptr(static_cast<const bf16_t*>(base) + (int64_t)n0 * st[0] + (int64_t)head * st[1]), (uint64_t)uniform_i64(st[0] * 2)};
+  };
+  Operand st1 = operand(kDQ ? p.k : p.q, kDQ ? p.ks : p.qs), st2 = operand(kDQ ? p.v : p.dout, kDQ ? p.vs : p.dos);
+  Operand ow1 = operand(kDQ ? p.q : p.k, kDQ ? p.qs : p.ks), ow2 = operand(kDQ ? p.dout : p.v, kDQ ? p.dos : p.vs);
+  unsigned off1[T::TPW], off2[T::TPW];
+#pragma unroll
+  for (int it = 0; it < T::TPW; ++it) {
+    off1[it] = lane_offset(w0, it, kDQ ? p.ks[2] : p.qs[2]);
+    off2[it] = lane_offset(w0, it, kDQ ? p.vs[2] : p.dos[2]);
+  }
+  // the owned rows: 2 OT transfers shared out over the waves (one wave takes several where there are fewer waves)
+  constexpr int OT = T::O_BYTES / 1024;
+  // per-row fp32 values: LSE and Delta rows of this head, the bias row of the entry
+  uint64_t lse_at = uniform_ptr(p.lse + ((int64_t)n0 * p.H + head) * S), del_at = uniform_ptr(p.delta + ((int64_t)n0 * p.H + head) * S);
+  uint64_t row_at = kRowB ? uniform_ptr(p.rowb + (int64_t)n0 * S) : 0;
+  const uint64_t stat_step = (uint64_t)p.H * S * 4u, row_step = (uint64_t)S * 4u;
+  const unsigned st_row = (uint32_t)min(w0 + lane, S - 1) * 4u, ow_row = (uint32_t)min(o0 + lane, S - 1) * 4u;
+  auto load_entry = [&](int slot) FL_INLINE {
+    const unsigned s0 = lds0 + slot * slot_bytes, mine = s0 + wave * T::W_BYTES, own_at = s0 + w_bytes;
+#pragma unroll
+    for (int it = 0; it < T::TPW; ++it) {
+      dma16(st1.at, off1[it], mine + it * 1024);
+      dma16(st2.at, off2[it], mine + T::T_BYTES + it * 1024);
+    }
+    if constexpr (kDQ) {
+      if constexpr (kRowB) dma4(row_at, st_row, mine + 2 * T::T_BYTES);
+    } else {
+      dma4(lse_at, st_row, mine + 2 * T::T_BYTES);
+      dma4(del_at, st_row, mine + 2 * T::T_BYTES + 256);
+    }
+    for (int x = wave; x < 2 * OT; x += NW) {
+      if (x < OT) dma16(ow1.at, lane_offset(o0, x, kDQ ? p.qs[2] : p.ks[2]), own_at + x * 1024);
+      else dma16(ow2.at, lane_offset(o0, x - OT, kDQ ? p.dos[2] : p.vs[2]), own_at + x * 1024);
+    }
+    if (wave == NW - 1) {
+      if constexpr (kDQ) {
+        dma4(lse_at, ow_row, own_at + 2 * T::O_BYTES);
+        dma4(del_at, ow_row, own_at + 2 * T::O_BYTES + 256);
+      } else if constexpr (kRowB) {
+        dma4(row_at, ow_row, own_at + 2 * T::O_BYTES);
+      }
+    }
+    st1.at += st1.step;
+    st2.at += st2.step;
+    ow1.at += ow1.step;
+    ow2.at += ow2.step;
+    lse_at += stat_step;
+    del_at += stat_step;
+    if constexpr (kRowB) row_at += row_step;
+  };
+
+  // ---- LDS operand reads, as in bwd_kernel.h
+  auto frag_row = [&](const unsigned char* t, int row, int ks) FL_INLINE -> ex8 {
+    return *reinterpret_cast<const ex8*>(t + row * (D * 2) + L::swz_kv(row, 2 * ks + h) * 16);
+  };
+  auto frag_tr = [&](const unsigned char* t, int c, int dbk) FL_INLINE -> ex8 {
+    ex8 f;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int i16 = lane % 16, g = (lane / 16) % 2;
+      const int row = 16 * c + 8 * j + 4 * h + i16 / 4, col = dbk * 32 + g * 16 + 4 * (i16 % 4);
+      const unsigned char* ap = t + row * (D * 2) + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
+      typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
+      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ap)));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
+    }
+    return f;
+  };
+  // partial sums of one set: [owned row][D] floats, 16-byte chunks XOR-swizzled with the row
+  constexpr int PC = D / 4;
+  auto park_at = [&](int row, int c) FL_INLINE { return row * (D * 4) + ((c ^ row) & (PC - 1)) * 16; };
+
+  if (n0 < n1) load_entry(0);
+  for (int n = n0; n < n1; ++n) {
+    const int slot = p.slots == 2 ? (n - n0) & 1 : 0;
+    dma_wait<0>();
+    __syncthreads();  // the owned rows are visible; everyone is done with the other slot
+    if (p.slots == 2 && n + 1 < n1) load_entry(slot ^ 1);
+
+    unsigned char* s0 = smem + slot * slot_bytes;
+    unsigned char* mine = s0 + wave * T::W_BYTES;
+    const unsigned char* own_at = s0 + w_bytes;
+    ex8 o1[KS], o2[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      o1[ks] = frag_row(own_at, r, ks);
+      o2[ks] = frag_row(own_at + T::O_BYTES, r, ks);
+    }
+    const float* own_f = reinterpret_cast<const float*>(own_at + 2 * T::O_BYTES);
+    const float* st_f = reinterpret_cast<const float*>(mine + 2 * T::T_BYTES);
+    const float own_a = kDQ ? own_f[r] : (kRowB ? own_f[r] : 0.f);  // LSE of the query, or the bias row at the key
+    f32x16 x2_init;
+    if constexpr (kDQ) {
+      const float nd = own_f[64 + r];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x2_init[i] = nd;
+    }
+    f32x16 acc1[DB], acc2[kDQ ? 1 : DB];
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        acc1[d][i] = 0.f;
+        if constexpr (!kDQ) acc2[d][i] = 0.f;
+      }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      f32x16 x1, x2;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x1[i] = 0.f;
+      float st_a[16];  // per streamed row: the bias row (ROLE_DQ) or the LSE
+      if constexpr (!kDQ || kRowB) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(st_f + 32 * b + 8 * g + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) st_a[4 * g + e] = a[e];
+        }
+      }
+      if constexpr (kDQ) {
+        x2 = x2_init;
+      } else {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x4 a = *reinterpret_cast<const f32x4*>(st_f + 64 + 32 * b + 8 * g + 4 * h);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x2[4 * g + e] = a[e];
+        }
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        x1 = mfma32(frag_row(mine, 32 * b + r, ks), o1[ks], x1);
+        x2 = mfma32(frag_row(mine + T::T_BYTES, 32 * b + r, ks), o2[ks], x2);
+      }
+      ex8 pf[2], dsf[2];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        // logit in log2 units minus the row's LSE
+        float c = bias[b][i];
+        if constexpr (kDQ) {
+          c -= own_a;
+          if constexpr (kRowB) c += st_a[i];
+        } else {
+          c -= st_a[i];
+          if constexpr (kRowB) c += own_a;
+        }
+        const float w = fast_exp2(__builtin_fmaf(x1[i], p.scale_log2, c));
+        const float ds = w * x2[i];
+        if constexpr (kDQ) db[b][i] += ds;
+        else pf[i / 8][i % 8] = (E)w;
+        dsf[i / 8][i % 8] = (E)ds;
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int d = 0; d < DB; ++d) {
+          acc1[d] = mfma32(frag_tr(mine, 2 * b + c, d), dsf[c], acc1[d]);
+          if constexpr (!kDQ) acc2[d] = mfma32(frag_tr(mine + T::T_BYTES, 2 * b + c, d), pf[c], acc2[d]);
+        }
+    }
+
+    // ---- the waves add up: accumulator register i of block d is column 32 d + 8 (i / 4) + 4 h + i % 4 of owned row r
+    auto park = [&](const f32x16 (&acc)[DB], unsigned char* at) FL_INLINE {
+#pragma unroll
+      for (int d = 0; d < DB; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<f32x4*>(at + park_at(r, 8 * d + 2 * g + h)) = f32x4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
+    };
+    auto gather = [&](unsigned offset, bf16_t* out, const int64_t (&st)[3], float scale) FL_INLINE {
+      for (int x = tid; x < 32 * PC; x += NT) {
+        const int row = x / PC, c = x % PC;
+        const unsigned char* at = s0 + offset + park_at(row, c);
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+        // (the usual wave counts with all their reads in flight)
+        if (NW == 4) {
+#pragma unroll
+          for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
+        } else if (NW == 8) {
+#pragma unroll
+          for (int w = 0; w < 8; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
+        } else {
+          for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
+        }
+        if (o0 + row < S) {
+          ex4 o4;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o4[e] = (E)(sum[e] * scale);
+          // (32-bit offsets inside one (batch entry, head): S rows of at most 2^20 elements)
+          *reinterpret_cast<ex4*>(reinterpret_cast<unsigned char*>(out + (int64_t)n * st[0] + (int64_t)head * st[1]) +
+                                  (uint32_t)((o0 + row) * (int)st[2] + 4 * c) * 2u) = o4;
+        }
+      }
+    };
+    // (a wave parks over its own tiles only, which it alone has read)
+    park(acc1, mine);
+    if constexpr (!kDQ && T::ONE_PASS) park(acc2, mine + T::PARK);
+    __syncthreads();
+    gather(0, kDQ ? p.dq : p.dk, kDQ ? p.dqs : p.dks, p.scale);
+    if constexpr (!kDQ && T::ONE_PASS) gather(T::PARK, p.dv, p.dvs, 1.0f);
+    if constexpr (!kDQ && !T::ONE_PASS) {
+      __syncthreads();
+      park(acc2, mine);
+      __syncthreads();
+      gather(0, p.dv, p.dvs, 1.0f);
+    }
+    if (p.slots == 1 && n + 1 < n1) {
+      __syncthreads();  // the sums have been read
+      load_entry(0);
+    }
+  }
+
+  if constexpr (kDQ) {
+    if (p.dbias_part != nullptr && own < S) {
+      float* out = p.dbias_part + ((((int64_t)group * p.chunks + chunk) * p.H + head) * S + own) * p.s_pad;
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int st = w0 + 32 * b + 8 * g + 4 * h;
+          if (st < p.s_pad) *reinterpret_cast<f32x4*>(out + st) = f32x4{db[b][4 * g], db[b][4 * g + 1], db[b][4 * g + 2], db[b][4 * g + 3]};
+        }
+    }
+  }
+}
+
+// Sums the chunks' partial bias gradients (in chunk order) into [groups, H, S, S] of the bias's type.
+template <class OUT>
+__global__ __launch_bounds__(256) void pairbias_bwd_reduce_kernel(const float* part, OUT* out, int chunks, int64_t rows_per_group,
+                                                                  int S, int s_pad, int64_t total4) {
+  const int64_t x = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (x >= total4) return;
+  const int q4 = s_pad / 4;
+  const int64_t row = x / q4, grp = row / rows_per_group, in_grp = row % rows_per_group;  // row: [group][head][query]
+  const int c = (int)(x % q4) * 4;
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int ch = 0; ch < chunks; ++ch)
+    s += *reinterpret_cast<const f32x4*>(part + ((grp * chunks + ch) * rows_per_group + in_grp) * s_pad + c);
+  OUT* o = out + row * S + c;
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (c + e < S) o[e] = (OUT)s[e];
+}
+
+struct SBPrepParams {
+  const bf16_t *out, *dout, *gate;
+  bf16_t *dgated, *dgate;  // dout * sigmoid(gate); gradient of the gate's logits
+  float* delta;            // [B, H, S], minus the row sums
+  const void* row;         // bias row per batch entry (or null), and where it goes in log2 units: [B, S]
+  float* rowb;
+  int64_t row_batch;
+  int32_t row_key, row_div, row_f32;
+  int64_t os[3], dos[3], gs[3], dgds[3], dgs[3];
+  int32_t B, H, S;
+};
+
+// What the two roles need per row, in one pass over dO and the result.  With the gate g and the result out = sigmoid(g) o O
+// the general formulas need only out: Delta = rowsum(dO sigmoid(g) o O) = rowsum(dO o out), and the gradient of the
+// logits dO o O sigmoid(g) (1 - sigmoid(g)) = dO o out (1 - sigmoid(g)).
+template <int D, bool GATE, class E>
+__global__ __launch_bounds__(256) void pairbias_bwd_prep_kernel(const SBPrepParams p) {
+  typedef E ex8 __attribute__((ext_vector_type(8)));
+  constexpr int LPR = D / 8;
+  const int64_t rows = (int64_t)p.B * p.S * p.H, x = ((int64_t)blockIdx.x * 256 + threadIdx.x) / LPR;
+  const int c = threadIdx.x % LPR * 8;
+  // rows in (batch, position, head) order: the Evoformer's memory order
+  const int64_t row = x < rows ? x : rows - 1;
+  const int hd = (int)(row % p.H), s = (int)(row / p.H % p.S), b = (int)(row / ((int64_t)p.H * p.S));
+  const ex8 d8 = *reinterpret_cast<const ex8*>(p.dout + b * p.dos[0] + hd * p.dos[1] + s * p.dos[2] + c);
+  const ex8 o8 = *reinterpret_cast<const ex8*>(p.out + b * p.os[0] + hd * p.os[1] + s * p.os[2] + c);
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum += (float)d8[e] * (float)o8[e];
+#pragma unroll
+  for (int d = 1; d < LPR; d *= 2) sum += __shfl_xor(sum, d);
+  if constexpr (GATE) {
+    const ex8 g8 = *reinterpret_cast<const ex8*>(p.gate + b * p.gs[0] + hd * p.gs[1] + s * p.gs[2] + c);
+    ex8 a8, b8;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float sg = fast_rcp(1.0f + fast_exp2(-1.4426950408889634f * (float)g8[e]));
+      a8[e] = (E)((float)d8[e] * sg);
+      b8[e] = (E)((float)d8[e] * (float)o8[e] * (1.0f - sg));
+    }
+    if (x < rows) {
+      *reinterpret_cast<ex8*>(p.dgated + b * p.dgds[0] + hd * p.dgds[1] + s * p.dgds[2] + c) = a8;
+      *reinterpret_cast<ex8*>(p.dgate + b * p.dgs[0] + hd * p.dgs[1] + s * p.dgs[2] + c) = b8;
+    }
+  }
+  if (x < rows && c == 0) {
+    p.delta[((int64_t)b * p.H + hd) * p.S + s] = -sum;
+    if (p.row != nullptr && hd == 0) {
+      const int64_t off = (int64_t)(b / p.row_div) * p.row_batch + (int64_t)s * p.row_key;
+      p.rowb[(int64_t)b * p.S + s] =
+          1.4426950408889634f * (p.row_f32 ? static_cast<const float*>(p.row)[off] : (float)static_cast<const E*>(p.row)[off]);
+    }
+  }
+}
+
+}  // namespace fl

@@ -252,6 +252,29 @@ int fl_attn_bwd_static(const fl_attn_bwd_params* p, void* stream);
 /* FL_STATIC_SCRATCH_BYTES of the loaded library. */
 uint64_t fl_static_scratch_bytes(void);
 
+/* Gradients of a forward call with one dense bias operand shared by consecutive batch entries, optionally a second operand
+ * that is one row of keys per batch entry, and optionally the sigmoid gate: the Evoformer's row attention
+ * (evoformer.py:8-36).  No counterpart in the reference, which is forward-only.  Unmasked, no score modification, no
+ * dropout; Lq == Lk <= 512, Hq == Hkv, Dqk == Dv in {32, 64}; the dense operand has its own row for every head and query.
+ * fwd, dout, dq, dk, dv as in fl_attn_bwd_params, with fwd.o the (gated) result, and fwd.gate as in the forward.
+ * dbias (optional): gradient of the dense operand, [B / bias_batch_div, Hq, Lq, Lk] contiguous, in the operand's type.
+ * dgate (with fwd.gate): gradient of the gate's logits, addressed with dgate_strides.
+ * workspace: fl_attn_shared_bias_bwd_bytes() bytes, 256-byte aligned, contents undefined.
+ * Four launches (row sums and gate; dQ and the bias's partial sums; dK and dV; the sum), no atomics. */
+typedef struct fl_attn_shared_bias_bwd_params {
+  fl_attn_params fwd;
+  const void* dout;
+  int64_t dout_strides[4];
+  void *dq, *dk, *dv, *dgate, *dbias;
+  int64_t dq_strides[4], dk_strides[4], dv_strides[4], dgate_strides[4];
+  void* workspace;
+  uint64_t workspace_bytes;
+} fl_attn_shared_bias_bwd_params;
+/* Bytes of workspace for the gradients of the forward call *p, or 0 when fl_attn_shared_bias_bwd does not take it (the
+ * pointers of *p need not be set, apart from which of bias[0], bias[1] and gate are present).  Host only. */
+uint64_t fl_attn_shared_bias_bwd_bytes(const fl_attn_params* p);
+int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* p, void* stream);
+
 /* Operand packing for invariant point attention (tests/test_ipa.py:57-125, a test-only function of the reference):
  * builds the concatenated operands with which the function becomes one fl_attn_fwd call.  All tensors are bf16,
  * contiguous, `rows` = batch * heads * residues rows each:

@@ -1,0 +1,93 @@
+"""The backward of attention with a bias shared by several batch entries (csrc/pairbias_bwd_kernel.h): the Evoformer's
+row attention in training, at the edges of its 32-row stripes, wave splits and resident-entry counts, against autograd
+through the fp32 oracle."""
+import ctypes as C
+
+import pytest
+import torch
+
+import flashlight_amd.attention_variants as A
+import oracle as O
+from flashlight_amd import _ffi
+from tests.test_abi import good_params
+
+DEV = "cuda"
+
+
+def test_which_calls_the_shared_bias_backward_takes():
+    lib = _ffi.load_library()
+    lib.fl_attn_shared_bias_bwd_bytes.restype = C.c_uint64
+
+    def params(S=256, D=32, H=4, **kw):
+        p = good_params(D=D)
+        p.B, p.Hq, p.Hkv, p.Lq, p.Lk = 12, H, H, S, S
+        p.q_strides[:] = p.k_strides[:] = p.v_strides[:] = p.o_strides[:] = (S * H * D, D, H * D, 1)
+        p.bias[0], p.bias_batch_div[0] = 0x60000, 6
+        p.bias_strides[0][:] = (H * S * S, S * S, S, 1)
+        for n, v in kw.items():
+            setattr(p, n, v)
+        return p
+
+    takes = lambda p: lib.fl_attn_shared_bias_bwd_bytes(C.byref(p)) > 0  # noqa: E731
+    assert takes(params()) and takes(params(S=512, D=64)) and takes(params(S=1))
+    assert not takes(params(S=513)) and not takes(params(D=128)) and not takes(params(softcap=3.0))
+    assert not takes(params(mask_kind=_ffi.MASK_CAUSAL)) and not takes(params(Hkv=2)) and not takes(params(Lq=128))
+    p = params()
+    p.bias_strides[0][1] = 0  # one bias for all heads: another sum
+    assert not takes(p)
+    p = params()
+    p.bias[1], p.bias_batch_div[1] = 0x70000, 1
+    p.bias_strides[1][:] = (256, 0, 0, 1)
+    assert takes(p)
+
+
+CASES = [  # B, N, S, H, D
+    (1, 3, 32, 2, 32), (2, 5, 64, 3, 32), (1, 9, 100, 4, 64), (2, 17, 129, 2, 32), (1, 4, 256, 4, 64), (1, 40, 256, 8, 32),
+    (1, 7, 257, 2, 64), (1, 6, 384, 2, 32), (1, 3, 511, 2, 64), (1, 3, 512, 1, 32), (3, 2, 33, 1, 64), (1, 1, 77, 2, 32)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("gate", [False, True])
+@pytest.mark.parametrize("shape", CASES)
+def test_gradients_against_the_oracle(shape, gate):
+    B, N, S, H, D = shape
+    g = torch.Generator().manual_seed(sum(shape))
+    for dt, mask, f32 in ((torch.bfloat16, False, False), (torch.float16, True, False), (torch.bfloat16, True, True)):
+        mk = lambda *s: torch.randn(*s, generator=g).to(dt)  # noqa: E731
+        q, k, v, dout = (mk(B, N, S, H, D) for _ in range(4))
+        pair = torch.randn(B, 1, H, S, S, generator=g).to(torch.float32 if f32 else dt)
+        gl = mk(B, N, S, H, D) if gate else None
+        row = None
+        if mask:
+            row = torch.where(torch.rand(B, N, 1, 1, S, generator=g) < 0.2, float("-inf"), 0.0).to(dt)
+            row[..., 0] = 0
+        leaves = [t for t in (q, k, v, pair, gl) if t is not None]
+        dev = [t.to(DEV).requires_grad_(True) for t in leaves]
+        kw = {"gate": dev[4]} if gate else {}
+        out = A.attention_reference(dev[0], dev[1], dev[2], ([row.to(DEV)] if mask else []) + [dev[3]], **kw)
+        grads = torch.autograd.grad(out, dev, dout.to(DEV))
+        ref = [t.float().requires_grad_(True) for t in leaves]
+        want = O.attention_evoformer(ref[0], ref[1], ref[2], ([row.float()] if mask else []) + [ref[3]], **({"gate": ref[4]} if gate else {}))
+        wgrads = torch.autograd.grad(want, ref, dout.float())
+        for name, a, b in zip(("out", "dq", "dk", "dv", "dbias", "dgate"), (out, *grads), (want, *wgrads)):
+            rel = ((a.float().cpu() - b).norm() / b.norm()).item()
+            assert a.dtype == (torch.float32 if f32 and name == "dbias" else dt) and a.shape == b.shape
+            assert rel < (1e-2 if dt == torch.bfloat16 else 3e-3), (shape, gate, mask, f32, name, rel)
+
+
+@pytest.mark.gpu
+def test_layouts_partial_gradients_and_repetition():
+    """Heads-first operands, gradients of the bias alone or not at all, the same bits twice, and a second derivative that
+    is refused instead of missing."""
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn(1, 6, 2, 96, 32, generator=g).to(torch.bfloat16).to(DEV).transpose(-2, -3) for _ in range(3))
+    pair = torch.randn(1, 1, 2, 96, 96, generator=g).to(torch.bfloat16).to(DEV).requires_grad_(True)
+    a, = torch.autograd.grad(A.attention_reference(q, k, v, [pair]).float().square().sum(), [pair])
+    q.requires_grad_(True)
+    b = torch.autograd.grad(A.attention_reference(q, k, v, [pair]).float().square().sum(), [pair, q])
+    c = torch.autograd.grad(A.attention_reference(q, k, v, [pair.detach()]).float().square().sum(), [q])
+    assert torch.equal(a, b[0]) and torch.equal(b[1], c[0])
+    out = A.attention_reference(q, k, v, [pair])
+    dq, = torch.autograd.grad(out.float().sum(), [q], create_graph=True)
+    with pytest.raises(RuntimeError, match="not differentiable a second time"):
+        dq.float().sum().backward()
