@@ -125,6 +125,10 @@ def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
     lib.fl_attn_bwd_validate.argtypes = [C.POINTER(FlAttnBwdParams)]
     lib.fl_attn_bwd.restype = C.c_int
     lib.fl_attn_bwd.argtypes = [C.POINTER(FlAttnBwdParams), C.c_void_p]
+    lib.fl_attn_bwd_split_bytes.restype = C.c_uint64
+    lib.fl_attn_bwd_split_bytes.argtypes = [C.POINTER(FlAttnParams)]
+    lib.fl_attn_bwd_split.restype = C.c_int
+    lib.fl_attn_bwd_split.argtypes = [C.POINTER(FlAttnBwdParams), C.c_void_p, C.c_uint64, C.c_void_p]
     lib.fl_attn_bwd_static.restype = C.c_int
     lib.fl_attn_bwd_static.argtypes = [C.POINTER(FlAttnBwdParams), C.c_void_p]
     lib.fl_attn_merge_chunks.restype = C.c_int
@@ -145,7 +149,7 @@ def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
         raise ImportError("flashlight_amd/_host.so is missing or does not load: build it with `python -m flashlight_amd.build`") from e
     _host = host_module
     _host.bind(*(C.cast(getattr(lib, f), C.c_void_p).value for f in (
-        "fl_attn_fwd", "fl_attn_bwd", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_rows_plan",
+        "fl_attn_fwd", "fl_attn_bwd_split", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_bwd_split_bytes", "fl_attn_rows_plan",
         "fl_attn_shared_bias_bwd_bytes", "fl_attn_shared_bias_bwd", "fl_last_error")))
     _lib = lib
     return lib
@@ -440,7 +444,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
              doc_ids: Optional[torch.Tensor] = None, alibi_heads: int = 0, softcap: float = 0.0,
              validate_only: bool = False, dropout_p: float = 0.0, dropout_seed: int = 0, static_scratch: bool = False,
              grads: Optional[Sequence[torch.Tensor]] = None, biases: Sequence[tuple[torch.Tensor, int]] = (),
-             dscores: Optional[torch.Tensor] = None):
+             dscores: Optional[torch.Tensor] = None, split: bool = False):
     """Gradients (dq, dk, dv) of `attn_fwd` called with the same arguments (dropout rate and seed included); `out` and `lse` are what that call
     returned and filled, `dout` [B, Hq, Lq, Dv] the gradient of its result.  Three launches on the current stream.
     `grads` = (dq, dk, dv) receives the results when given.  `static_scratch` goes through `fl_attn_bwd_static`: nothing
@@ -448,7 +452,8 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
     overlap on one GPU must not both use it).
     `biases` are the forward's bias operands; `dscores`, a zero-filled contiguous float32 [B, Hq, Lq, Lk] tensor, then
     receives the gradient with respect to the scores, from which the caller sums the gradient of each operand over the
-    axes it broadcasts over (not under a soft-cap)."""
+    axes it broadcasts over (not under a soft-cap).  `split` lets several workgroups share a tile where tiles alone would
+    leave the GPU idle (`fl_attn_bwd_split`: sums in another order)."""
     lib = load_library()
     for name, t in (("query", q), ("key", k), ("value", v), ("out", out), ("dout", dout)):
         _require_gpu_half(name, t, q if isinstance(q, torch.Tensor) and q.dtype in _HALF_TYPES else None)
@@ -491,7 +496,12 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
     if validate_only:
         _check(lib.fl_attn_bwd_validate(C.byref(b)))
         return dq, dk, dv
-    _launch_on(q.device, lib.fl_attn_bwd_static if use_static else lib.fl_attn_bwd, b)
+    split_bytes = lib.fl_attn_bwd_split_bytes(C.byref(b.fwd)) if split and not use_static else 0
+    if split_bytes:
+        scratch = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
+        _launch_on(q.device, lambda params, stream: lib.fl_attn_bwd_split(params, scratch.data_ptr(), split_bytes, stream), b)
+    else:
+        _launch_on(q.device, lib.fl_attn_bwd_static if use_static else lib.fl_attn_bwd, b)
     del keep, delta
     return dq, dk, dv
 

@@ -1048,10 +1048,53 @@ static int validate_bwd(const fl_attn_bwd_params* b, const fl::BwdInstance** out
 
 int fl_attn_bwd_validate(const fl_attn_bwd_params* b) { return validate_bwd(b, nullptr); }
 
-int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream_) {
+// Workgroups per owner tile of the two backward kernels, and the scratch their partial sums take (the second launch reuses
+// the first one's).  A tile of 128 query rows or keys is one workgroup, and while the grid leaves compute units idle, or
+// with one wave per SIMD, its walk over the streamed steps is a chain of latencies: 1.9 us per step of the dK/dV kernel
+// at head dim 64 with one wave per SIMD, next to nothing more with two.  So the steps of a tile are cut until one round of
+// workgroups fills the part: 512 of four waves, 256 of eight (dK/dV at head dim 128); two rounds where the mask makes tiles
+// of unequal length, whose shorter ones then fill up behind the longer ones (8192 causal rows of 8 heads over 1, head dim
+// 64: 494 us with one round, 353 with two, 360 with four; 1024 unmasked rows of 2 x 16 over 2, head dim 128: 109, 132, 132).
+// A split costs the writing and reading of its partial sums and its own prologue, and the summing launch 4 us: it keeps at
+// least eight steps, counted over the longest tile (4 x 300 causal rows, 8 heads over 1: 38 us with eight, 63 with sixteen).
+// Whole gradients, bf16, before -> after: 3 x 16 heads over 4 x 1000 prefix rows, head dim 64: 186 -> 86 us; 8 over 1 x 2048
+// causal, 128: 640 -> 94; 32 over 4 x 4096 causal, 128: 1354 -> 575; 8 x 4096 causal, 128: 287 -> 202.
+namespace {
+struct BwdSplits {
+  int dq = 1, dkv = 1;
+  uint64_t bytes = 0;
+};
+BwdSplits plan_bwd_splits(const fl_attn_params* p) {
+  BwdSplits x;
+  const int64_t D = p->Dqk, q_tiles = (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128), k_tiles = (int64_t)p->B * p->Hkv * ((p->Lk + 127) / 128);
+  int64_t q_steps = (p->Lk + (D <= 64 ? 63 : 31)) / (D <= 64 ? 64 : 32), k_steps = (p->Lq + 63) / 64;
+  if (p->mask_kind == FL_MASK_SLIDING) {
+    q_steps = std::min<int64_t>(q_steps, ((int64_t)p->window + 128) / (D <= 64 ? 64 : 32) + 1);
+    k_steps = std::min<int64_t>(k_steps, ((int64_t)p->window + 128) / 64 + 1);
+  }
+  k_steps *= p->Hq / p->Hkv;
+  const int64_t rounds = p->mask_kind == FL_MASK_NONE || p->mask_kind == FL_MASK_SLIDING ? 1 : 2;
+  const auto splits = [&](int64_t slots, int64_t tiles, int64_t steps) { return (int)std::max<int64_t>(1, std::min(rounds * slots / tiles, steps / 8)); };
+  x.dq = splits(512, q_tiles, q_steps);
+  x.dkv = splits(D <= 64 ? 512 : 256, k_tiles, k_steps);
+  if (x.dq > 1) x.bytes = (uint64_t)x.dq * q_tiles * 128 * D * sizeof(float);
+  if (x.dkv > 1) x.bytes = std::max(x.bytes, (uint64_t)x.dkv * k_tiles * 128 * D * 2 * sizeof(float));
+  return x;
+}
+}  // namespace
+
+uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p) {
+  if (!p || p->B <= 0 || p->Hkv <= 0 || p->Hq < p->Hkv || p->Lq <= 0 || p->Lk <= 0 || p->Dqk <= 0) return 0;
+  return plan_bwd_splits(p).bytes;
+}
+
+int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream) { return fl_attn_bwd_split(b, nullptr, 0, stream); }
+
+int fl_attn_bwd_split(const fl_attn_bwd_params* b, void* scratch, uint64_t scratch_bytes, void* stream_) {
   const fl::BwdInstance* in = nullptr;
   int rc = validate_bwd(b, &in);
   if (rc) return rc;
+  if (scratch && reinterpret_cast<uintptr_t>(scratch) % 16) return fail(FL_ERR_ALIGN, "scratch must be 16-byte aligned");
   const fl_attn_params* p = &b->fwd;
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   fl::BParams bp;
@@ -1114,10 +1157,18 @@ int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream_) {
     bp.doc_table = table;
     bp.doc_blocks = blocks;
   }
+  BwdSplits splits;
+  if (scratch) {
+    splits = plan_bwd_splits(p);
+    if (splits.bytes > scratch_bytes) splits = BwdSplits();
+  }
+  bp.part = static_cast<float*>(scratch);
   hipError_t e = in->launch_delta(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the row-sum kernel failed: %s", hipGetErrorString(e));
+  bp.splits = splits.dq;
   e = in->launch_dq(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dQ kernel failed: %s", hipGetErrorString(e));
+  bp.splits = splits.dkv;
   e = in->launch_dkv(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dK/dV kernel failed: %s", hipGetErrorString(e));
   return 0;

@@ -19,14 +19,23 @@ struct BwdInstance {
 extern const BwdInstance kBwdInstances[];
 extern const int kNumBwdInstances;
 
-template <class T>
-hipError_t launch_bwd(const BParams& bp, hipStream_t stream) {
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_kernel<T>),
+template <class T, bool SPLIT>
+hipError_t launch_bwd_tiles(const BParams& bp, int64_t tiles, hipStream_t stream) {
+  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_kernel<T, SPLIT>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
   if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((bwd_kernel<T, SPLIT>), dim3((unsigned)(tiles * bp.splits)), dim3(T::NT), T::LDS_BYTES, stream, bp);
+  return hipGetLastError();
+}
+
+template <class T>
+hipError_t launch_bwd(const BParams& bp, hipStream_t stream) {
   const int len = T::ROLE == ROLE_DQ ? bp.Lq : bp.Lk, heads = T::ROLE == ROLE_DQ ? bp.Hq : bp.Hkv;
-  const int64_t grid = (int64_t)bp.B * heads * ((len + T::OWN - 1) / T::OWN);
-  hipLaunchKernelGGL(bwd_kernel<T>, dim3((unsigned)grid), dim3(T::NT), T::LDS_BYTES, stream, bp);
+  const int64_t tiles = (int64_t)bp.B * heads * ((len + T::OWN - 1) / T::OWN);
+  if (bp.splits == 1) return launch_bwd_tiles<T, false>(bp, tiles, stream);
+  const hipError_t e = launch_bwd_tiles<T, true>(bp, tiles, stream);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(bwd_split_sum_kernel<T>, dim3((unsigned)(tiles * 4), T::ROLE == ROLE_DQ ? 1 : 2), dim3(256), 0, stream, bp);
   return hipGetLastError();
 }
 

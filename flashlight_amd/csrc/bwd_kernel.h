@@ -56,6 +56,11 @@ struct BParams {
   int32_t bdiv[2];
   int32_t bias_f32[2];
   float* dscores;  // optional [B, Hq, Lq, Lk]: d(loss) / d(score), written by the dQ kernel for the tiles it visits
+  // Workgroups per owner tile, each with its share of the streamed steps.  With more than one they leave their
+  // fp32 sums in `part`, which bwd_split_sum_kernel adds up:
+  // [split][owner tile][wave block of 32 positions][dQ, or dK then dV][register / 4][lane][4]
+  float* part;
+  int32_t splits;
 };
 
 // delta[b, h, q] = -sum_d dO[b, h, q, d] * O[b, h, q, d]; one row per group of DV / 8 lanes.
@@ -110,7 +115,9 @@ struct BwdTraits {
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
 };
 
-template <class T>
+// SPLIT: several workgroups per owner tile.  A kernel of its own: with the second epilogue in it the dK/dV kernel at head
+// dim 128 is 4 % slower (another register allocation throughout).
+template <class T, bool SPLIT>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
 void bwd_kernel(const BParams p) {
   constexpr int D = T::D, ROLE = T::ROLE, TB = T::TB, BT = T::BT, KS = T::KS, DB = T::DB, NT = T::NT;
@@ -138,14 +145,19 @@ void bwd_kernel(const BParams p) {
   // (ROLE_DKV): heads are taken four at a time and their tiles dealt longest first, so the grid drains on short ones.
   const int n_own = kDQ ? (p.Lq + T::OWN - 1) / T::OWN : (p.Lk + T::OWN - 1) / T::OWN;
   const int oh = kDQ ? p.Hq : p.Hkv;
-  int ot, bh;
+  // The splits of a tile (p.splits > 1) are dealt next to each other.
+  const int nbh = p.B * oh;
+  int ot, bh, split = 0;
   {
-    const int nbh = p.B * oh;
     int i = blockIdx.x, run = nbh, base = 0;
     if (nbh % 8 == 0) {
       run = nbh / 8;
       base = (i % 8) * run;
       i /= 8;
+    }
+    if constexpr (SPLIT) {
+      split = i % p.splits;
+      i /= p.splits;
     }
     const int G = (p.mask_kind == MASK_CAUSAL || p.mask_kind == MASK_PREFIX || p.mask_kind == MASK_DOC_CAUSAL) ? 4 : 1;
     const int g = i / (G * n_own), rem = i % (G * n_own);
@@ -178,7 +190,9 @@ void bwd_kernel(const BParams p) {
   }
   const int n_tiles = t_hi >= t_lo ? t_hi - t_lo + 1 : 0;
   const int n_heads = kDQ ? 1 : p.group;   // ROLE_DKV walks the query heads of its group
-  const int n_steps = n_tiles * n_heads;
+  const int all_steps = n_tiles * n_heads;
+  const int s_first = SPLIT ? (int)((int64_t)all_steps * split / p.splits) : 0;
+  const int n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / p.splits) : all_steps;  // this workgroup's steps: [s_first, n_steps)
 
   // ---- per-lane constants ---------------------------------------------------------------------------------------------
   float cap_k1 = 0.f, cap_c = 0.f;
@@ -292,7 +306,7 @@ void bwd_kernel(const BParams p) {
       for (int i = 0; i < 16; ++i) acc2[db][i] = 0.f;
   }
 
-  if (n_steps > 0) {
+  if (n_steps > s_first) {
     if constexpr (!kDQ) {
       const int valid = o1 - o0;
       load_tile(kptr + (int64_t)o0 * p.ks[2], p.ks[2], valid, T::O1_OFF, T::O_PER_T);
@@ -557,7 +571,7 @@ void bwd_kernel(const BParams p) {
       return s;
     };
     bool full = false, doc_uniform = false;
-    int s = next_live(0, full, doc_uniform);
+    int s = next_live(s_first, full, doc_uniform);
     if (s < n_steps) load_step(s, 0);
     dma_wait<0>();
     for (int slot = 0; s < n_steps; slot ^= 1) {
@@ -573,9 +587,9 @@ void bwd_kernel(const BParams p) {
     }
   } else {
     // positional masks: every step of [t_lo, t_hi] is visited (a dead one only occurs under a prefix-LM mask)
-    if (n_steps > 0) load_step(0, 0);
+    if (n_steps > s_first) load_step(s_first, s_first & 1);
     dma_wait<0>();
-    for (int s = 0; s < n_steps; ++s) {
+    for (int s = s_first; s < n_steps; ++s) {
       const int slot = s & 1;
       __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
       if (s + 1 < n_steps) load_step(s + 1, slot ^ 1);
@@ -611,6 +625,25 @@ void bwd_kernel(const BParams p) {
     }
   }
 
+  if constexpr (SPLIT) {
+    if (qh == 0) {
+      constexpr int SETS = kDQ ? 1 : 2;
+      float* to = p.part + ((((int64_t)split * nbh * n_own + (int64_t)bh * n_own + ot) * 4 + ow) * SETS * DB * 16 * 64) + lane * 4;
+#pragma unroll
+      for (int set = 0; set < SETS; ++set)
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            f32x4 x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = set == 0 ? acc1[db][4 * g + e] : acc2[kDQ ? 0 : db][4 * g + e];
+            *reinterpret_cast<f32x4*>(to + (set * DB * 4 + db * 4 + g) * 256) = x;
+          }
+    }
+    return;
+  }
+
   // ---- epilogue: register i of block db is column 32 db + 8 (i / 4) + 4 h + i % 4 of this lane's owner row ---------------
   if (opos < olen && qh == 0) {
     bf16_t* out1 = kDQ ? p.dq + (int64_t)batch * p.dqs[0] + (int64_t)ohead * p.dqs[1] + (int64_t)opos * p.dqs[2]
@@ -636,6 +669,41 @@ void bwd_kernel(const BParams p) {
           *reinterpret_cast<ex4*>(out2 + 32 * db + 8 * g + 4 * h) = o4;
         }
     }
+  }
+}
+
+// Adds up the splits of one owner tile's block of 32 positions and writes its rows of dQ, or of dK (blockIdx.y 0) and dV
+// (1).  Reads in the order the sums were left (1 KiB per wave and load); a workgroup's stores fill whole rows.
+template <class T>
+__global__ __launch_bounds__(256) void bwd_split_sum_kernel(const BParams p) {
+  constexpr int DB = T::DB, SETS = T::ROLE == ROLE_DQ ? 1 : 2;
+  constexpr bool kDQ = T::ROLE == ROLE_DQ;
+  using E = typename T::Elem;
+  typedef E ex4 __attribute__((ext_vector_type(4)));
+  const int olen = kDQ ? p.Lq : p.Lk, oh = kDQ ? p.Hq : p.Hkv, n_own = (olen + T::OWN - 1) / T::OWN;
+  const int tile = blockIdx.x / 4, bh = tile / n_own, head = bh % oh, batch = bh / oh, set = blockIdx.y;
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int pos = tile % n_own * T::OWN + blockIdx.x % 4 * 32 + lane % 32;
+  if (pos >= olen) return;
+  const int64_t split_stride = (int64_t)gridDim.x * SETS * DB * 16 * 64;
+  const float* from = p.part + ((int64_t)blockIdx.x * SETS + set) * DB * 16 * 64 + lane * 4;
+  const float factor = set == 0 ? p.scale : (T::FEAT & F_DROPOUT) ? p.drop_rescale : 1.0f;
+  bf16_t* out = kDQ ? p.dq + (int64_t)batch * p.dqs[0] + (int64_t)head * p.dqs[1] + (int64_t)pos * p.dqs[2]
+                : set == 0 ? p.dk + (int64_t)batch * p.dks[0] + (int64_t)head * p.dks[1] + (int64_t)pos * p.dks[2]
+                           : p.dv + (int64_t)batch * p.dvs[0] + (int64_t)head * p.dvs[1] + (int64_t)pos * p.dvs[2];
+  f32x4 x[DB];  // wave w takes the register groups w, w + 4, ...: DB of the block's 4 DB
+#pragma unroll
+  for (int j = 0; j < DB; ++j) x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+  for (int s = 0; s < p.splits; ++s)
+#pragma unroll
+    for (int j = 0; j < DB; ++j) x[j] += *reinterpret_cast<const f32x4*>(from + s * split_stride + (4 * j + wave) * 256);
+#pragma unroll
+  for (int j = 0; j < DB; ++j) {  // register group 4 j + w: columns 32 j + 8 w + 4 h ...
+    ex4 o4;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o4[e] = (E)(x[j][e] * factor);
+    *reinterpret_cast<ex4*>(out + 32 * j + 8 * wave + 4 * (lane / 32)) = o4;
   }
 }
 

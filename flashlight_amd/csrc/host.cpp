@@ -31,15 +31,16 @@ using torch::autograd::variable_list;
 
 struct Api {
   int (*fwd)(const fl_attn_params*, void*) = nullptr;
-  int (*bwd)(const fl_attn_bwd_params*, void*) = nullptr;
+  int (*bwd)(const fl_attn_bwd_params*, void*, uint64_t, void*) = nullptr;
   uint64_t (*workspace)(const fl_attn_params*) = nullptr;
   uint64_t (*bwd_workspace)(const fl_attn_params*) = nullptr;
+  uint64_t (*bwd_split_bytes)(const fl_attn_params*) = nullptr;
   int (*rows_plan)(const fl_attn_params*, uint64_t*) = nullptr;
   uint64_t (*shared_bias_bwd_bytes)(const fl_attn_params*) = nullptr;
   int (*shared_bias_bwd)(const fl_attn_shared_bias_bwd_params*, void*) = nullptr;
   const char* (*last_error)(void) = nullptr;
 } g_api;
-constexpr int kApiFunctions = 8;
+constexpr int kApiFunctions = 9;
 
 // One call's arguments.  The tensors are the caller's; `doc`, `bias` and `gate` may be undefined.
 struct Call {
@@ -257,7 +258,7 @@ struct Attention : torch::autograd::Function<Attention> {
       set_strides(b.fwd.o_strides, out);
       b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
       Tensor dq = empty_for_gradient(c.q), dk = empty_for_gradient(c.k), dv = empty_for_gradient(c.v);
-      Tensor delta = at::empty(lse.sizes(), lse.options()), ws;
+      Tensor delta = at::empty(lse.sizes(), lse.options()), ws, split;
       b.dout = dout.const_data_ptr();
       b.dq = dq.data_ptr();
       b.dk = dk.data_ptr();
@@ -272,7 +273,9 @@ struct Attention : torch::autograd::Function<Attention> {
         b.fwd.workspace = ws.data_ptr();
         b.fwd.workspace_bytes = bytes;
       }
-      const int rc = g_api.bwd(&b, current_stream());
+      const uint64_t split_bytes = g_api.bwd_split_bytes(&b.fwd);
+      if (split_bytes) split = at::empty({(int64_t)split_bytes}, delta.options().dtype(at::kByte));
+      const int rc = g_api.bwd(&b, split_bytes ? split.data_ptr() : nullptr, split_bytes, current_stream());
       TORCH_CHECK(rc == 0, "flashlight_amd error ", rc, ": ", g_api.last_error());
       result[0] = dq;
       result[1] = dk;
@@ -474,7 +477,7 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* f[kApiFunctions];
   if (n != kApiFunctions) {
-    PyErr_SetString(PyExc_TypeError, "bind takes the addresses of eight functions");
+    PyErr_SetString(PyExc_TypeError, "bind takes the addresses of nine functions");
     return nullptr;
   }
   for (int i = 0; i < kApiFunctions; ++i) f[i] = PyLong_AsVoidPtr(a[i]);
@@ -483,10 +486,11 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   g_api.bwd = reinterpret_cast<decltype(g_api.bwd)>(f[1]);
   g_api.workspace = reinterpret_cast<decltype(g_api.workspace)>(f[2]);
   g_api.bwd_workspace = reinterpret_cast<decltype(g_api.bwd_workspace)>(f[3]);
-  g_api.rows_plan = reinterpret_cast<decltype(g_api.rows_plan)>(f[4]);
-  g_api.shared_bias_bwd_bytes = reinterpret_cast<decltype(g_api.shared_bias_bwd_bytes)>(f[5]);
-  g_api.shared_bias_bwd = reinterpret_cast<decltype(g_api.shared_bias_bwd)>(f[6]);
-  g_api.last_error = reinterpret_cast<decltype(g_api.last_error)>(f[7]);
+  g_api.bwd_split_bytes = reinterpret_cast<decltype(g_api.bwd_split_bytes)>(f[4]);
+  g_api.rows_plan = reinterpret_cast<decltype(g_api.rows_plan)>(f[5]);
+  g_api.shared_bias_bwd_bytes = reinterpret_cast<decltype(g_api.shared_bias_bwd_bytes)>(f[6]);
+  g_api.shared_bias_bwd = reinterpret_cast<decltype(g_api.shared_bias_bwd)>(f[7]);
+  g_api.last_error = reinterpret_cast<decltype(g_api.last_error)>(f[8]);
   Py_RETURN_NONE;
 }
 

@@ -88,7 +88,7 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
     """(dq, dk, dv) of `attn_fwd_lse` for the output gradient `dout`."""
     return _ffi.attn_bwd(q, k, v, out, lse, dout, scale=scale if scale > 0 else None, mask_kind=mask_kind, window=window,
                          prefix=prefix, doc_ids=doc_ids, alibi_heads=alibi_heads, softcap=softcap, dropout_p=dropout_p,
-                         dropout_seed=dropout_seed)
+                         dropout_seed=dropout_seed, split=True)
 
 
 @attn_bwd.register_fake
@@ -158,7 +158,7 @@ def attn_bwd_bias(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.
     dq, dk, dv = _ffi.attn_bwd(q, k, v, out, lse, dout, scale=scale if scale > 0 else None, mask_kind=mask_kind,
                                window=window, prefix=prefix, biases=biases, dscores=dscores if want_dscores else None,
                                dropout_p=dropout_p, dropout_seed=dropout_seed, doc_ids=doc_ids, alibi_heads=alibi_heads,
-                               softcap=softcap)
+                               softcap=softcap, split=True)
     return dq, dk, dv, dscores
 
 

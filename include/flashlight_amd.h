@@ -234,6 +234,13 @@ int fl_attn_bwd_validate(const fl_attn_bwd_params* p);
 /* Launches the three backward kernels (row sums of dO o O, then dQ, then dK and dV) on `stream`. */
 int fl_attn_bwd(const fl_attn_bwd_params* p, void* stream);
 
+/* fl_attn_bwd with scratch of its own (16-byte aligned, contents undefined before and after) in which workgroups that
+ * share a tile leave partial sums: for calls whose tiles alone would leave most of the GPU idle.  Up to two more
+ * launches.  With less than fl_attn_bwd_split_bytes(), or NULL, the call is fl_attn_bwd. */
+int fl_attn_bwd_split(const fl_attn_bwd_params* p, void* scratch, uint64_t scratch_bytes, void* stream);
+/* Bytes of scratch fl_attn_bwd_split can use for the gradients of the forward call *p; 0: none.  Host only. */
+uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p);
+
 /* fl_attn_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight training loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and results as fl_attn_bwd,
  * except that p->delta and p->fwd.workspace / workspace_bytes are ignored: the row sums and the document table live in

@@ -1,0 +1,84 @@
+"""Backward tiles cut into several workgroups (fl_attn_bwd_split) against the same call with whole tiles, which the other
+backward tests hold against the oracle; which calls are cut, and that the partial sums stay inside the scratch."""
+import ctypes as C
+
+import pytest
+import torch
+
+from flashlight_amd import _ffi
+from tests.test_abi import good_params
+
+DEV = "cuda"
+
+
+def _split_bytes(B, Hq, Hkv, Lq, Lk, D, mask=_ffi.MASK_NONE, window=0):
+    p = good_params(D=D)
+    p.B, p.Hq, p.Hkv, p.Lq, p.Lk, p.mask_kind, p.window = B, Hq, Hkv, Lq, Lk, mask, window
+    return _ffi.load_library().fl_attn_bwd_split_bytes(C.byref(p))
+
+
+def test_which_backwards_are_cut():
+    assert _split_bytes(4, 16, 16, 4096, 4096, 128, _ffi.MASK_CAUSAL) == 0      # enough tiles
+    assert _split_bytes(1, 8, 8, 256, 256, 64) == 0                             # too few steps
+    # 3 x 16 heads over 4, 1000 rows: 96 tiles of keys, two rounds of 512 workgroups, dK and dV of 128 x 64 floats each
+    assert _split_bytes(3, 16, 4, 1000, 1000, 64, _ffi.MASK_PREFIX_LM) == 8 * 96 * 128 * 64 * 2 * 4
+    # a window of 100: few steps per tile whatever the length
+    assert _split_bytes(1, 2, 2, 8192, 8192, 64, _ffi.MASK_SLIDING, 100) == 0
+    assert _ffi.load_library().fl_attn_bwd_split_bytes(None) == 0
+
+
+CASES = [  # B, Hq, Hkv, Lq, Lk, D, mask, extra
+    (3, 16, 4, 1000, 1000, 64, _ffi.MASK_PREFIX_LM, dict(prefix=200)),
+    (1, 8, 1, 513, 513, 128, _ffi.MASK_CAUSAL, {}),
+    (1, 3, 3, 2047, 2047, 32, _ffi.MASK_NONE, {}),
+    (1, 1, 1, 100, 3001, 64, _ffi.MASK_NONE, {}),
+    (1, 8, 2, 1025, 77, 128, _ffi.MASK_NONE, dict(softcap=3.0)),
+    (2, 4, 1, 1500, 1500, 128, _ffi.MASK_SLIDING, dict(window=700)),
+    (1, 4, 4, 1111, 1111, 64, _ffi.MASK_DOCUMENT_CAUSAL, {}),
+    (1, 8, 2, 900, 900, 64, _ffi.MASK_CAUSAL, dict(dropout_p=0.25, dropout_seed=11)),
+    (1, 5, 5, 1300, 1300, 128, _ffi.MASK_CAUSAL, dict(alibi_heads=5)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("case", CASES)
+def test_cut_tiles_give_the_gradients_of_whole_tiles(case, dtype, monkeypatch):
+    B, Hq, Hkv, Lq, Lk, D, mask, extra = case
+    g = torch.Generator().manual_seed(Lq + Lk)
+    mk = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)  # noqa: E731
+    q, k, v, dout = mk(B, Hq, Lq, D), mk(B, Hkv, Lk, D), mk(B, Hkv, Lk, D), mk(B, Hq, Lq, D)
+    kw = dict(mask_kind=mask, **extra)
+    if mask == _ffi.MASK_DOCUMENT_CAUSAL:
+        kw["doc_ids"] = torch.sort(torch.randint(0, 4, (B, Lk), generator=g), dim=1).values.to(DEV)
+    lse = torch.empty(B, Hq, Lq, dtype=torch.float32, device=DEV)
+    out = _ffi.attn_fwd(q, k, v, lse=lse, **kw)
+    lib = _ffi.load_library()
+    calls = []
+
+    class Recorded:  # the library with its split entry given a scratch of exactly the asked size, NaN inside and out
+        def __getattr__(self, name):
+            if name != "fl_attn_bwd_split":
+                return getattr(lib, name)
+
+            def entry(params, _scratch, n, stream):
+                buf = torch.full((n // 4 + 1024,), float("nan"), device=DEV)
+                rc = lib.fl_attn_bwd_split(params, buf.data_ptr(), n, stream)
+                calls.append((buf, n))
+                return rc
+            return entry
+
+    monkeypatch.setattr(_ffi, "load_library", lambda *a: Recorded())
+    cut = _ffi.attn_bwd(q, k, v, out, lse, dout, split=True, **kw)
+    whole = _ffi.attn_bwd(q, k, v, out, lse, dout, **kw)
+    torch.cuda.synchronize()
+    (buf, n), = calls
+    assert torch.isnan(buf[n // 4:]).all()
+    # the same 16-bit weights and score gradients, added up in another order in fp32 (relative error of a sum of n terms
+    # below n * 2^-24 of their magnitudes): results may differ where they round to the other neighbour
+    ulp = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for name, a, b in zip(("dq", "dk", "dv"), cut, whole):
+        assert torch.isfinite(a).all(), name
+        d, ref = (a.double() - b.double()), b.double()
+        assert (d.norm() / ref.norm()).item() < ulp / 4, name
+        assert (d.abs() <= 2 * ulp * ref.abs() + 2e-5 * ref.abs().max()).all(), name
