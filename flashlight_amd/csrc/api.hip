@@ -1048,44 +1048,52 @@ static int validate_bwd(const fl_attn_bwd_params* b, const fl::BwdInstance** out
 
 int fl_attn_bwd_validate(const fl_attn_bwd_params* b) { return validate_bwd(b, nullptr); }
 
-// Workgroups per owner tile of the two backward kernels, and the scratch their partial sums take (the second launch reuses
-// the first one's).  A tile of 128 query rows or keys is one workgroup, and while the grid leaves compute units idle, or
-// with one wave per SIMD, its walk over the streamed steps is a chain of latencies: 1.9 us per step of the dK/dV kernel
-// at head dim 64 with one wave per SIMD, next to nothing more with two.  So the steps of a tile are cut until one round of
-// workgroups fills the part: 512 of four waves, 256 of eight (dK/dV at head dim 128); two rounds where the mask makes tiles
-// of unequal length, whose shorter ones then fill up behind the longer ones (8192 causal rows of 8 heads over 1, head dim
-// 64: 494 us with one round, 353 with two, 360 with four; 1024 unmasked rows of 2 x 16 over 2, head dim 128: 109, 132, 132).
-// A split costs the writing and reading of its partial sums and its own prologue, and the summing launch 4 us: it keeps at
-// least eight steps, counted over the longest tile (4 x 300 causal rows, 8 heads over 1: 38 us with eight, 63 with sixteen).
-// Whole gradients, bf16, before -> after: 3 x 16 heads over 4 x 1000 prefix rows, head dim 64: 186 -> 86 us; 8 over 1 x 2048
-// causal, 128: 640 -> 94; 32 over 4 x 4096 causal, 128: 1354 -> 575; 8 x 4096 causal, 128: 287 -> 202.
+// How the gradient kernels are launched.  A tile of 128 query rows or keys is one workgroup, and a launch that leaves compute
+// units idle, or one wave per SIMD, is a chain of latencies: 1.9 us per step of the dK/dV kernel at head dim 64 with one
+// wave per SIMD, next to nothing more with two.  So while the tiles of one role alone do not fill the part about twice
+// (512 workgroups of four waves, 256 of eight at head dim 128), both roles run in one launch, and tiles whose walk over the
+// streamed steps is longer than an even share of all steps (half of them under masks of growing length) are cut into
+// splits of about that share.  A split costs the writing and reading of its partial sums and its own prologue, and the
+// sums a launch of 5 to 9 us: no split has fewer than eight steps, and a tile of up to one and a half shares stays whole.
+// Beyond, a launch per role is the better one (4 x 16 x 2048, head dim 64, causal: 177 us against 188; 2 x 16 x 2048, head
+// dim 128, unmasked: 271 against 300).
+// Gradients, bf16, a launch per role with whole tiles -> this rule: 3 x 16 heads over 4 x 1000 prefix rows, head dim 64:
+// 157 -> 77 us; 8 x 512 causal, 64: 36 -> 25; 8 over 1 x 8192 causal, 64: 1980 -> 342; 8 x 512 causal, 128: 47 -> 29; 8 over
+// 1 x 2048 causal, 128: 568 -> 73; 32 over 4 x 4096 causal, 128: 1214 -> 611; 2 x 16 x 2048 causal, 64: 131 -> 107.
 namespace {
-struct BwdSplits {
-  int dq = 1, dkv = 1;
-  uint64_t bytes = 0;
+struct BwdPlan {
+  bool both = false;    // one launch
+  int dq = 1, dkv = 1;  // splits per tile
+  uint64_t dq_bytes = 0, bytes = 0;  // scratch: dQ's partial sums, then dK's and dV's
 };
-BwdSplits plan_bwd_splits(const fl_attn_params* p) {
-  BwdSplits x;
+BwdPlan plan_bwd(const fl_attn_params* p) {
+  BwdPlan x;
   const int64_t D = p->Dqk, q_tiles = (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128), k_tiles = (int64_t)p->B * p->Hkv * ((p->Lk + 127) / 128);
-  int64_t q_steps = (p->Lk + (D <= 64 ? 63 : 31)) / (D <= 64 ? 64 : 32), k_steps = (p->Lq + 63) / 64;
+  const int64_t least = std::min(q_tiles, k_tiles);
+  x.both = D <= 64 ? least <= 512 : least < 512;
+  if (!x.both) return x;
+  int64_t q_steps = (p->Lk + 63) / 64, k_steps = (p->Lq + 63) / 64;
   if (p->mask_kind == FL_MASK_SLIDING) {
-    q_steps = std::min<int64_t>(q_steps, ((int64_t)p->window + 128) / (D <= 64 ? 64 : 32) + 1);
-    k_steps = std::min<int64_t>(k_steps, ((int64_t)p->window + 128) / 64 + 1);
+    const int64_t band = ((int64_t)p->window + 128) / 64 + 1;
+    q_steps = std::min(q_steps, band);
+    k_steps = std::min(k_steps, band);
   }
   k_steps *= p->Hq / p->Hkv;
-  const int64_t rounds = p->mask_kind == FL_MASK_NONE || p->mask_kind == FL_MASK_SLIDING ? 1 : 2;
-  const auto splits = [&](int64_t slots, int64_t tiles, int64_t steps) { return (int)std::max<int64_t>(1, std::min(rounds * slots / tiles, steps / 8)); };
-  x.dq = splits(512, q_tiles, q_steps);
-  x.dkv = splits(D <= 64 ? 512 : 256, k_tiles, k_steps);
-  if (x.dq > 1) x.bytes = (uint64_t)x.dq * q_tiles * 128 * D * sizeof(float);
-  if (x.dkv > 1) x.bytes = std::max(x.bytes, (uint64_t)x.dkv * k_tiles * 128 * D * 2 * sizeof(float));
+  const bool growing = p->mask_kind != FL_MASK_NONE && p->mask_kind != FL_MASK_SLIDING;
+  const int64_t total = (q_tiles * q_steps + k_tiles * k_steps) / (growing ? 2 : 1);
+  const int64_t share = std::max<int64_t>(8, total / (D <= 64 ? 512 : 256));
+  const auto splits = [&](int64_t steps) { return (int)(2 * steps <= 3 * share ? 1 : (steps + share - 1) / share); };
+  x.dq = splits(q_steps);
+  x.dkv = splits(k_steps);
+  x.dq_bytes = x.dq > 1 ? (uint64_t)x.dq * q_tiles * 128 * D * sizeof(float) : 0;
+  x.bytes = x.dq_bytes + (x.dkv > 1 ? (uint64_t)x.dkv * k_tiles * 128 * D * 2 * sizeof(float) : 0);
   return x;
 }
 }  // namespace
 
 uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p) {
   if (!p || p->B <= 0 || p->Hkv <= 0 || p->Hq < p->Hkv || p->Lq <= 0 || p->Lk <= 0 || p->Dqk <= 0) return 0;
-  return plan_bwd_splits(p).bytes;
+  return plan_bwd(p).bytes;
 }
 
 int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream) { return fl_attn_bwd_split(b, nullptr, 0, stream); }
@@ -1157,18 +1165,21 @@ int fl_attn_bwd_split(const fl_attn_bwd_params* b, void* scratch, uint64_t scrat
     bp.doc_table = table;
     bp.doc_blocks = blocks;
   }
-  BwdSplits splits;
-  if (scratch) {
-    splits = plan_bwd_splits(p);
-    if (splits.bytes > scratch_bytes) splits = BwdSplits();
-  }
-  bp.part = static_cast<float*>(scratch);
+  BwdPlan plan = plan_bwd(p);
+  if (!scratch || plan.bytes > scratch_bytes) plan.dq = plan.dkv = 1;
+  bp.part_dq = static_cast<float*>(scratch);
+  if (plan.dkv > 1) bp.part = bp.part_dq + plan.dq_bytes / sizeof(float);
+  bp.splits_dq = plan.dq;
+  bp.splits = plan.dkv;
   hipError_t e = in->launch_delta(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the row-sum kernel failed: %s", hipGetErrorString(e));
-  bp.splits = splits.dq;
+  if (plan.both) {
+    e = in->launch_both(bp, stream);
+    if (e != hipSuccess) return fail((int)e, "backward: launch of the gradient kernel failed: %s", hipGetErrorString(e));
+    return 0;
+  }
   e = in->launch_dq(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dQ kernel failed: %s", hipGetErrorString(e));
-  bp.splits = splits.dkv;
   e = in->launch_dkv(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dK/dV kernel failed: %s", hipGetErrorString(e));
   return 0;

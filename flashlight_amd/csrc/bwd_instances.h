@@ -13,29 +13,43 @@ struct BwdInstance {
   int dtype;  // element type of q, k, v, o, dout and the gradients: FL_BF16 (0) or FL_F16 (2)
   hipError_t (*launch_dq)(const BParams&, hipStream_t);
   hipError_t (*launch_dkv)(const BParams&, hipStream_t);
+  hipError_t (*launch_both)(const BParams&, hipStream_t);
   hipError_t (*launch_delta)(const BParams&, hipStream_t);
 };
 
 extern const BwdInstance kBwdInstances[];
 extern const int kNumBwdInstances;
 
-template <class T, bool SPLIT>
-hipError_t launch_bwd_tiles(const BParams& bp, int64_t tiles, hipStream_t stream) {
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&bwd_kernel<T, SPLIT>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
-  if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((bwd_kernel<T, SPLIT>), dim3((unsigned)(tiles * bp.splits)), dim3(T::NT), T::LDS_BYTES, stream, bp);
-  return hipGetLastError();
+template <class K>
+hipError_t allow_lds(K kernel) {
+  return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
 }
 
 template <class T>
-hipError_t launch_bwd(const BParams& bp, hipStream_t stream) {
-  const int len = T::ROLE == ROLE_DQ ? bp.Lq : bp.Lk, heads = T::ROLE == ROLE_DQ ? bp.Hq : bp.Hkv;
-  const int64_t tiles = (int64_t)bp.B * heads * ((len + T::OWN - 1) / T::OWN);
-  if (bp.splits == 1) return launch_bwd_tiles<T, false>(bp, tiles, stream);
-  const hipError_t e = launch_bwd_tiles<T, true>(bp, tiles, stream);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(bwd_split_sum_kernel<T>, dim3((unsigned)(tiles * 4), T::ROLE == ROLE_DQ ? 1 : 2), dim3(256), 0, stream, bp);
+hipError_t launch_bwd_role(const BParams& bp, int64_t tiles, hipStream_t stream) {
+  static const hipError_t attr = allow_lds(&bwd_kernel<T>);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL(bwd_kernel<T>, dim3((unsigned)tiles), dim3(T::NT), T::LDS_BYTES, stream, bp);
+  return hipGetLastError();
+}
+
+inline int64_t bwd_q_tiles(const BParams& bp) { return (int64_t)bp.B * bp.Hq * ((bp.Lq + 127) / 128); }
+inline int64_t bwd_k_tiles(const BParams& bp) { return (int64_t)bp.B * bp.Hkv * ((bp.Lk + 127) / 128); }
+
+// dQ, dK and dV in one launch, and the sums of the tiles that were split.
+template <int D, uint32_t FEAT, class E>
+hipError_t launch_bwd_both(const BParams& bp, hipStream_t stream) {
+  using TQ = BwdTraits<D, ROLE_DQ, FEAT, E, true>;
+  using TKV = BwdTraits<D, ROLE_DKV, FEAT, E, true>;
+  constexpr int lds = TQ::LDS_BYTES > TKV::LDS_BYTES ? TQ::LDS_BYTES : TKV::LDS_BYTES;
+  static const hipError_t attr = allow_lds(&bwd_both_kernel<TQ, TKV>);
+  if (attr != hipSuccess) return attr;
+  const int64_t q_tiles = bwd_q_tiles(bp), k_tiles = bwd_k_tiles(bp);
+  hipLaunchKernelGGL((bwd_both_kernel<TQ, TKV>), dim3((unsigned)(q_tiles * bp.splits_dq + k_tiles * bp.splits)), dim3(TQ::NT), lds, stream, bp);
+  const hipError_t e = hipGetLastError();
+  const int64_t blocks = (bp.splits > 1 ? 8 * k_tiles : 0) + (bp.splits_dq > 1 ? 4 * q_tiles : 0);
+  if (e != hipSuccess || blocks == 0) return e;
+  hipLaunchKernelGGL((bwd_split_sum_kernel<TQ, TKV>), dim3((unsigned)blocks), dim3(256), 0, stream, bp);
   return hipGetLastError();
 }
 
@@ -61,19 +75,22 @@ hipError_t launch_delta(const BParams& bp, hipStream_t stream) {
   namespace fl {                                                              \
   hipError_t launch_bwd_dq_##D##_##FEAT##SFX(const BParams&, hipStream_t);    \
   hipError_t launch_bwd_dkv_##D##_##FEAT##SFX(const BParams&, hipStream_t);   \
+  hipError_t launch_bwd_both_##D##_##FEAT##SFX(const BParams&, hipStream_t);  \
   hipError_t launch_bwd_delta_##D##_##FEAT##SFX(const BParams&, hipStream_t); \
   }
 #define FL_BWD_DECL(D, FEAT) FL_BWD_DECL_(D, FEAT, _bf16) FL_BWD_DECL_(D, FEAT, _f16)
 #define FL_BWD_DEF(D, FEAT, SFX, ELEM)                                                                              \
   namespace fl {                                                                                                    \
   hipError_t launch_bwd_dq_##D##_##FEAT##SFX(const BParams& bp, hipStream_t s) {                                    \
-    return launch_bwd<BwdTraits<D, ROLE_DQ, FEAT, ELEM>>(bp, s);                                                    \
+    return launch_bwd_role<BwdTraits<D, ROLE_DQ, FEAT, ELEM>>(bp, bwd_q_tiles(bp), s);                              \
   }                                                                                                                 \
   hipError_t launch_bwd_dkv_##D##_##FEAT##SFX(const BParams& bp, hipStream_t s) {                                   \
-    return launch_bwd<BwdTraits<D, ROLE_DKV, FEAT, ELEM>>(bp, s);                                                   \
+    return launch_bwd_role<BwdTraits<D, ROLE_DKV, FEAT, ELEM>>(bp, bwd_k_tiles(bp), s);                             \
   }                                                                                                                 \
+  hipError_t launch_bwd_both_##D##_##FEAT##SFX(const BParams& bp, hipStream_t s) { return launch_bwd_both<D, FEAT, ELEM>(bp, s); } \
   hipError_t launch_bwd_delta_##D##_##FEAT##SFX(const BParams& bp, hipStream_t s) { return launch_delta<D, ELEM>(bp, s); } \
   }
 #define FL_BWD_ROW_(D, FEAT, SFX, DT) \
-  {D, FEAT, DT, &fl::launch_bwd_dq_##D##_##FEAT##SFX, &fl::launch_bwd_dkv_##D##_##FEAT##SFX, &fl::launch_bwd_delta_##D##_##FEAT##SFX},
+  {D, FEAT, DT, &fl::launch_bwd_dq_##D##_##FEAT##SFX, &fl::launch_bwd_dkv_##D##_##FEAT##SFX, \
+   &fl::launch_bwd_both_##D##_##FEAT##SFX, &fl::launch_bwd_delta_##D##_##FEAT##SFX},
 #define FL_BWD_ROW(D, FEAT) FL_BWD_ROW_(D, FEAT, _bf16, 0) FL_BWD_ROW_(D, FEAT, _f16, 2)

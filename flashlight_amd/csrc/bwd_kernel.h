@@ -61,6 +61,9 @@ struct BParams {
   // [split][owner tile][wave block of 32 positions][dQ, or dK then dV][register / 4][lane][4]
   float* part;
   int32_t splits;
+  // bwd_both_kernel: `part` and `splits` are the dK/dV role's, these the dQ role's
+  float* part_dq;
+  int32_t splits_dq;
 };
 
 // delta[b, h, q] = -sum_d dO[b, h, q, d] * O[b, h, q, d]; one row per group of DV / 8 lanes.
@@ -84,7 +87,8 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const BParams p) {
   if (row < rows && c == 0) p.delta[row] = -s;  // stored negated: the consumers add it (or start dP's accumulators from it)
 }
 
-template <int D_, int ROLE_, uint32_t FEAT_, class Elem_ = bf16_t>
+// SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size
+template <int D_, int ROLE_, uint32_t FEAT_, class Elem_ = bf16_t, bool SHARED_ = false>
 struct BwdTraits {
   using Elem = Elem_;  // element type of q, k, v, o, dout and the gradients: bf16_t or f16_t
   static constexpr int D = D_, ROLE = ROLE_;
@@ -93,7 +97,7 @@ struct BwdTraits {
   // ROLE_DKV at D = 128 holds 128 accumulator registers per lane; to still run two waves per SIMD its workgroup has
   // 8 waves, two per owner block, which take the two halves of every streamed tile and add up their partial sums
   // through LDS at the end (one workgroup per CU, 128 KB of LDS).
-  static constexpr int QH = (ROLE == ROLE_DKV && D_ > 64) ? 2 : 1;   // waves per owner block
+  static constexpr int QH = ((ROLE == ROLE_DKV || SHARED_) && D_ > 64) ? 2 : 1;   // waves per owner block
   static constexpr int NW = 4 * QH, NT = 64 * NW;
   static constexpr int TB = (D_ <= 64) ? 2 : 1;  // 32-position blocks per wave and step (register budget)
   static constexpr int BT = 32 * TB * QH;                  // streamed positions per step
@@ -115,11 +119,11 @@ struct BwdTraits {
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
 };
 
-// SPLIT: several workgroups per owner tile.  A kernel of its own: with the second epilogue in it the dK/dV kernel at head
-// dim 128 is 4 % slower (another register allocation throughout).
+// One workgroup's share of the work of a role: workgroup `block` of tiles * splits.  SPLIT: several workgroups per owner tile
+// (one at run time is fine), compiled apart: with the second epilogue in it the dK/dV kernel at head dim 128 is 4 %
+// slower (another register allocation throughout).
 template <class T, bool SPLIT>
-__global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
-void bwd_kernel(const BParams p) {
+__device__ __forceinline__ void bwd_tile(const BParams& p, const int block, const int splits, float* const part_sums) {
   constexpr int D = T::D, ROLE = T::ROLE, TB = T::TB, BT = T::BT, KS = T::KS, DB = T::DB, NT = T::NT;
   constexpr uint32_t FEAT = T::FEAT;
   constexpr bool kAlibi = FEAT & F_ALIBI, kSoftcap = FEAT & F_SOFTCAP, kDoc = FEAT & F_DOC, kBias = FEAT & F_BIAS;
@@ -145,19 +149,19 @@ void bwd_kernel(const BParams p) {
   // (ROLE_DKV): heads are taken four at a time and their tiles dealt longest first, so the grid drains on short ones.
   const int n_own = kDQ ? (p.Lq + T::OWN - 1) / T::OWN : (p.Lk + T::OWN - 1) / T::OWN;
   const int oh = kDQ ? p.Hq : p.Hkv;
-  // The splits of a tile (p.splits > 1) are dealt next to each other.
+  // The splits of a tile are dealt next to each other.
   const int nbh = p.B * oh;
   int ot, bh, split = 0;
   {
-    int i = blockIdx.x, run = nbh, base = 0;
+    int i = block, run = nbh, base = 0;
     if (nbh % 8 == 0) {
       run = nbh / 8;
       base = (i % 8) * run;
       i /= 8;
     }
     if constexpr (SPLIT) {
-      split = i % p.splits;
-      i /= p.splits;
+      split = i % splits;
+      i /= splits;
     }
     const int G = (p.mask_kind == MASK_CAUSAL || p.mask_kind == MASK_PREFIX || p.mask_kind == MASK_DOC_CAUSAL) ? 4 : 1;
     const int g = i / (G * n_own), rem = i % (G * n_own);
@@ -191,8 +195,8 @@ void bwd_kernel(const BParams p) {
   const int n_tiles = t_hi >= t_lo ? t_hi - t_lo + 1 : 0;
   const int n_heads = kDQ ? 1 : p.group;   // ROLE_DKV walks the query heads of its group
   const int all_steps = n_tiles * n_heads;
-  const int s_first = SPLIT ? (int)((int64_t)all_steps * split / p.splits) : 0;
-  const int n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / p.splits) : all_steps;  // this workgroup's steps: [s_first, n_steps)
+  const int s_first = SPLIT ? (int)((int64_t)all_steps * split / splits) : 0;
+  const int n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / splits) : all_steps;  // this workgroup's steps: [s_first, n_steps)
 
   // ---- per-lane constants ---------------------------------------------------------------------------------------------
   float cap_k1 = 0.f, cap_c = 0.f;
@@ -604,13 +608,13 @@ void bwd_kernel(const BParams p) {
   if constexpr (T::QH == 2) {
     float* park = reinterpret_cast<float*>(smem);
 #pragma unroll
-    for (int set = 0; set < 2; ++set) {
+    for (int set = 0; set < (kDQ ? 1 : 2); ++set) {
       __syncthreads();  // the tiles (set 0) or the previous set's sums (set 1) have been read
       if (qh == 1) {
 #pragma unroll
         for (int db = 0; db < DB; ++db)
 #pragma unroll
-          for (int i = 0; i < 16; ++i) park[((ow * 64 + db * 16 + i) * 64) + lane] = set == 0 ? acc1[db][i] : acc2[db][i];
+          for (int i = 0; i < 16; ++i) park[((ow * 64 + db * 16 + i) * 64) + lane] = set == 0 ? acc1[db][i] : acc2[kDQ ? 0 : db][i];
       }
       __syncthreads();
       if (qh == 0) {
@@ -619,16 +623,16 @@ void bwd_kernel(const BParams p) {
 #pragma unroll
           for (int i = 0; i < 16; ++i) {
             const float x = park[((ow * 64 + db * 16 + i) * 64) + lane];
-            if (set == 0) acc1[db][i] += x; else acc2[db][i] += x;
+            if (set == 0) acc1[db][i] += x; else acc2[kDQ ? 0 : db][i] += x;
           }
       }
     }
   }
 
-  if constexpr (SPLIT) {
+  if (SPLIT && splits > 1) {
     if (qh == 0) {
       constexpr int SETS = kDQ ? 1 : 2;
-      float* to = p.part + ((((int64_t)split * nbh * n_own + (int64_t)bh * n_own + ot) * 4 + ow) * SETS * DB * 16 * 64) + lane * 4;
+      float* to = part_sums + ((((int64_t)split * nbh * n_own + (int64_t)bh * n_own + ot) * 4 + ow) * SETS * DB * 16 * 64) + lane * 4;
 #pragma unroll
       for (int set = 0; set < SETS; ++set)
 #pragma unroll
@@ -672,21 +676,37 @@ void bwd_kernel(const BParams p) {
   }
 }
 
-// Adds up the splits of one owner tile's block of 32 positions and writes its rows of dQ, or of dK (blockIdx.y 0) and dV
-// (1).  Reads in the order the sums were left (1 KiB per wave and load); a workgroup's stores fill whole rows.
 template <class T>
-__global__ __launch_bounds__(256) void bwd_split_sum_kernel(const BParams p) {
+__global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
+void bwd_kernel(const BParams p) {
+  bwd_tile<T, false>(p, blockIdx.x, 1, nullptr);
+}
+
+// Both roles in one launch, dK/dV first: neither needs the other, and a small call's tails and gaps cost as much as its work.
+template <class TQ, class TKV>
+__global__ __launch_bounds__(TQ::NT) __attribute__((amdgpu_waves_per_eu(TQ::WAVES_PER_EU, TQ::WAVES_PER_EU)))
+void bwd_both_kernel(const BParams p) {
+  static_assert(TQ::NT == TKV::NT, "one workgroup size");
+  const int n_kv = p.B * p.Hkv * ((p.Lk + TKV::OWN - 1) / TKV::OWN) * p.splits;
+  if ((int)blockIdx.x < n_kv) bwd_tile<TKV, true>(p, blockIdx.x, p.splits, p.part);
+  else bwd_tile<TQ, true>(p, blockIdx.x - n_kv, p.splits_dq, p.part_dq);
+}
+
+// Adds up the splits of one owner tile's block of 32 positions and writes its rows of dQ, of dK (set 0) or of dV (set 1).
+// Reads in the order the sums were left (1 KiB per wave and load); a workgroup's stores fill whole rows.
+template <class T>
+__device__ __forceinline__ void bwd_sum_block(const BParams& p, const int block, const int set, const int splits, const float* const part) {
   constexpr int DB = T::DB, SETS = T::ROLE == ROLE_DQ ? 1 : 2;
   constexpr bool kDQ = T::ROLE == ROLE_DQ;
   using E = typename T::Elem;
   typedef E ex4 __attribute__((ext_vector_type(4)));
   const int olen = kDQ ? p.Lq : p.Lk, oh = kDQ ? p.Hq : p.Hkv, n_own = (olen + T::OWN - 1) / T::OWN;
-  const int tile = blockIdx.x / 4, bh = tile / n_own, head = bh % oh, batch = bh / oh, set = blockIdx.y;
+  const int tile = block / 4, bh = tile / n_own, head = bh % oh, batch = bh / oh;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int pos = tile % n_own * T::OWN + blockIdx.x % 4 * 32 + lane % 32;
+  const int pos = tile % n_own * T::OWN + block % 4 * 32 + lane % 32;
   if (pos >= olen) return;
-  const int64_t split_stride = (int64_t)gridDim.x * SETS * DB * 16 * 64;
-  const float* from = p.part + ((int64_t)blockIdx.x * SETS + set) * DB * 16 * 64 + lane * 4;
+  const int64_t split_stride = (int64_t)p.B * oh * n_own * 4 * SETS * DB * 16 * 64;
+  const float* from = part + ((int64_t)block * SETS + set) * DB * 16 * 64 + lane * 4;
   const float factor = set == 0 ? p.scale : (T::FEAT & F_DROPOUT) ? p.drop_rescale : 1.0f;
   bf16_t* out = kDQ ? p.dq + (int64_t)batch * p.dqs[0] + (int64_t)head * p.dqs[1] + (int64_t)pos * p.dqs[2]
                 : set == 0 ? p.dk + (int64_t)batch * p.dks[0] + (int64_t)head * p.dks[1] + (int64_t)pos * p.dks[2]
@@ -694,8 +714,8 @@ __global__ __launch_bounds__(256) void bwd_split_sum_kernel(const BParams p) {
   f32x4 x[DB];  // wave w takes the register groups w, w + 4, ...: DB of the block's 4 DB
 #pragma unroll
   for (int j = 0; j < DB; ++j) x[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int s = 0; s < p.splits; ++s)
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s)
 #pragma unroll
     for (int j = 0; j < DB; ++j) x[j] += *reinterpret_cast<const f32x4*>(from + s * split_stride + (4 * j + wave) * 256);
 #pragma unroll
@@ -705,6 +725,18 @@ __global__ __launch_bounds__(256) void bwd_split_sum_kernel(const BParams p) {
     for (int e = 0; e < 4; ++e) o4[e] = (E)(x[j][e] * factor);
     *reinterpret_cast<ex4*>(out + 32 * j + 8 * wave + 4 * (lane / 32)) = o4;
   }
+}
+
+// Workgroups [0, 8 tiles) dK and dV of every block of 32 keys when that role was split, the others dQ.
+template <class TQ, class TKV>
+__global__ __launch_bounds__(256) void bwd_split_sum_kernel(const BParams p) {
+  int block = blockIdx.x;
+  if (p.splits > 1) {
+    const int n_kv = p.B * p.Hkv * ((p.Lk + TKV::OWN - 1) / TKV::OWN) * 8;
+    if (block < n_kv) return bwd_sum_block<TKV>(p, block / 2, block % 2, p.splits, p.part);
+    block -= n_kv;
+  }
+  bwd_sum_block<TQ>(p, block, 0, p.splits_dq, p.part_dq);
 }
 
 }  // namespace fl

@@ -20,8 +20,10 @@ def _split_bytes(B, Hq, Hkv, Lq, Lk, D, mask=_ffi.MASK_NONE, window=0):
 def test_which_backwards_are_cut():
     assert _split_bytes(4, 16, 16, 4096, 4096, 128, _ffi.MASK_CAUSAL) == 0      # enough tiles
     assert _split_bytes(1, 8, 8, 256, 256, 64) == 0                             # too few steps
-    # 3 x 16 heads over 4, 1000 rows: 96 tiles of keys, two rounds of 512 workgroups, dK and dV of 128 x 64 floats each
-    assert _split_bytes(3, 16, 4, 1000, 1000, 64, _ffi.MASK_PREFIX_LM) == 8 * 96 * 128 * 64 * 2 * 4
+    # 3 x 16 heads over 4, 1000 rows: 384 tiles of 16 steps and 96 of 64, half of them attended: a share is 12 steps
+    assert _split_bytes(3, 16, 4, 1000, 1000, 64, _ffi.MASK_PREFIX_LM) == 6 * 96 * 128 * 64 * 2 * 4
+    # 8 heads over 1, 2048 rows: 128 tiles of 32 steps, 16 of 256
+    assert _split_bytes(1, 8, 1, 2048, 2048, 128, _ffi.MASK_CAUSAL) == (2 * 128 + 16 * 16 * 2) * 128 * 128 * 4
     # a window of 100: few steps per tile whatever the length
     assert _split_bytes(1, 2, 2, 8192, 8192, 64, _ffi.MASK_SLIDING, 100) == 0
     assert _ffi.load_library().fl_attn_bwd_split_bytes(None) == 0
