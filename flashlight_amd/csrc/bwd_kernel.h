@@ -114,6 +114,8 @@ struct BwdTraits {
                        S1_OFF = O2_OFF + OBYTES, S2_OFF = S1_OFF + 2 * SBYTES;
   static constexpr int LDS_BYTES = S2_OFF + 2 * SBYTES;
   static_assert(QH == 1 || LDS_BYTES >= 4 * 64 * 64 * 4, "the partial sums of one accumulator set must fit in LDS");
+  // two steps per turn of the loop, see there (the dK/dV kernel, 1 to 4 % slower with it, and bias operands have no registers for it)
+  static constexpr bool UNROLL2 = ROLE == ROLE_DQ && !(FEAT_ & F_BIAS);
   static constexpr int WAVES_PER_EU = 2;
   static constexpr bool WIDE_X2 = D_ > 64;                      // dP's fp32 tile declared next to S's
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
@@ -371,6 +373,30 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       auto rows4 = [&](unsigned staged_off, int q4) FL_INLINE -> f32x4 {
         return *reinterpret_cast<const f32x4*>(smem + staged_off + slot * T::SBYTES + (q4 - t0) * 4);
       };
+      // element predicate as an interval of the register offset `off` (8 (i / 4) + i % 4): lo <= off <= hi
+      auto bounds = [&](int sbase, int& lo, int& hi) FL_INLINE {
+        if constexpr (kDQ) {
+          // streamed = key, owner = query: key < Lk && (dmin <= key - q <= dmax || key < pfx)
+          const int rel = sbase - opos;
+          hi = min(p.Lk - sbase - 1, max(p.dmax - rel, p.pfx - sbase - 1));
+          lo = p.dmin - rel;
+        } else {
+          // streamed = query, owner = key: q < Lq && (dmin <= key - q <= dmax || key < pfx), key = opos
+          const int rel = opos - sbase;  // key - q at off = 0; key - q = rel - off
+          hi = min(p.Lq - sbase - 1, opos < p.pfx ? (1 << 29) : rel - p.dmin);
+          lo = opos < p.pfx ? -(1 << 29) : rel - p.dmax;
+          if (opos >= p.Lk) hi = -(1 << 29);
+        }
+      };
+      auto attended = [&](int sbase, int off, int lo, int hi) FL_INLINE -> bool {
+        bool ok = (off <= hi) & (off >= lo);
+        if constexpr (kDoc) {
+          if (!doc_uniform) ok = ok & (p.doc_ids[(int64_t)batch * p.doc_stride + min(sbase + off, slen - 1)] == odoc);
+        }
+        return ok;
+      };
+      // (document ids beside bias operands: the mask goes with each weight, sixteen ids in flight do not fit in the registers)
+      constexpr bool kMaskApart = !(kDoc && kBias);
       // X2 = T2 . O2^T (dP).  At D = 128 its fp32 tile is declared out here, next to X1's, and (ROLE_DQ) its MFMAs are issued
       // right after X1's, before the weights' vector work; at D = 64 it lives in the block that consumes it.  Both choices
       // are measured: the first is 15 % faster at D = 128 and 1-2 % slower at D = 64.
@@ -409,6 +435,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         const uint32_t s0 = drop_head_seed(p.drop_seed[0], p.drop_seed[1], (uint32_t)(batch * p.Hq + shead));
         drop_o = s0 + (kDQ ? (uint32_t)opos * kDropQ : (uint32_t)(opos >> 1) * kDropK);
       }
+      float pv[TB][16];
       {
         f32x16 x1[TB];
 #pragma unroll
@@ -428,24 +455,11 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 #pragma unroll
         for (int sb = 0; sb < TB; ++sb) {
           const int sbase = t0 + 32 * (qh * TB + sb) + 4 * h;  // streamed position of register 0
-          // element predicate as an interval of the register offset `off` (8 (i / 4) + i % 4): lo <= off <= hi
-          int lo, hi;
-          if constexpr (kDQ) {
-            // streamed = key, owner = query: key < Lk && (dmin <= key - q <= dmax || key < pfx)
-            const int rel = sbase - opos;
-            hi = min(p.Lk - sbase - 1, max(p.dmax - rel, p.pfx - sbase - 1));
-            lo = p.dmin - rel;
-          } else {
-            // streamed = query, owner = key: q < Lq && (dmin <= key - q <= dmax || key < pfx), key = opos
-            const int rel = opos - sbase;  // key - q at off = 0; key - q = rel - off
-            hi = min(p.Lq - sbase - 1, opos < p.pfx ? (1 << 29) : rel - p.dmin);
-            lo = opos < p.pfx ? -(1 << 29) : rel - p.dmax;
-            if (opos >= p.Lk) hi = -(1 << 29);
-          }
-          float pv[16];
           // what does not depend on the register goes into one addend: minus the row's LSE, and the ALiBi term at
           // off = 0 (key - q = rel0 + off in ROLE_DQ, rel0 - off in ROLE_DKV), which leaves slope * off as one
           // multiply-add with a literal per score
+          int lo = 0, hi = 0;
+          if constexpr (!kMaskApart) bounds(sbase, lo, hi);
           const float alibi0 = kAlibi ? slope_l2 * (float)(kDQ ? sbase - opos : opos - sbase) : 0.f;
           const float slope_off = kDQ ? slope_l2 : -slope_l2;
 #pragma unroll
@@ -472,18 +486,33 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
                 const int sp = min(sbase + off, slen - 1), op = min(opos, olen - 1);
                 s2 = __builtin_fmaf(bias_at(kDQ ? op : sp, kDQ ? sp : op, shead), kLog2e, s2);
               }
-              float pw = fast_exp2(s2);
-              if (!full) {  // workgroup-uniform
-                bool ok = (off <= hi) & (off >= lo);
-                if constexpr (kDoc) {
-                  if (!doc_uniform) ok = ok & (p.doc_ids[(int64_t)batch * p.doc_stride + min(sbase + off, slen - 1)] == odoc);
-                }
-                pw = ok ? pw : 0.f;
-              }
-              pv[i] = pw;
-              pd[sb][i] = kSoftcap ? pw * dfac : pw;
+              pv[sb][i] = fast_exp2(s2);
+              if (!kMaskApart && !full && !attended(sbase, off, lo, hi)) pv[sb][i] = 0.f;
+              pd[sb][i] = kSoftcap ? dfac : 1.0f;
             }
           }
+        }
+      }
+      if constexpr (T::WIDE_X2 && !T::EARLY_X2) second_product(x2_wide);
+      {
+#pragma unroll
+        for (int sb = 0; sb < TB; ++sb) {
+          const int sbase = t0 + 32 * (qh * TB + sb) + 4 * h;
+          if (kMaskApart && !full) {  // workgroup-uniform
+            // (the asm keeps this a branch: as selects it was three vector and two scalar instructions per score on every step,
+            // full ones included, beside the four that make a weight and its gradient.  It stands behind the products that
+            // do not need it, which the compiler can then interleave.  Gradients of 4 x 16 x 4096, this and the unrolled
+            // dQ loop: head dim 128 unmasked 2.00 -> 1.85 ms, causal 1.10 -> 1.01; head dim 64 1.135 -> 0.985, 0.62 -> 0.545)
+            int lo, hi;
+            bounds(sbase, lo, hi);
+            asm volatile("" : "+v"(lo), "+v"(hi));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              if (!attended(sbase, 8 * (i / 4) + i % 4, lo, hi)) pv[sb][i] = 0.f;
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < 16; ++i) pd[sb][i] = kSoftcap ? pv[sb][i] * pd[sb][i] : pv[sb][i];
           if constexpr (kDrop) {
             // ROLE_DQ: registers (i, i + 1), i even, are the key pair (sbase + off) / 2 of this lane's query: one hash.
             // ROLE_DKV: register i is query sbase + off against this lane's key: its own hash, the key's half of it.
@@ -493,14 +522,14 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
               if constexpr (kDQ) {
                 const uint32_t x = drop_pair_hash(drop_o + (uint32_t)((sbase + off) >> 1) * kDropK);
                 const bool keep0 = (x & 0xFFFFu) >= p.drop_thr, keep1 = (x >> 16) >= p.drop_thr;
-                pv[i] = keep0 ? pv[i] : 0.f;
-                pv[i + 1] = keep1 ? pv[i + 1] : 0.f;
+                pv[sb][i] = keep0 ? pv[sb][i] : 0.f;
+                pv[sb][i + 1] = keep1 ? pv[sb][i + 1] : 0.f;
                 pd[sb][i] = keep0 ? pd[sb][i] : -pd[sb][i];
                 pd[sb][i + 1] = keep1 ? pd[sb][i + 1] : -pd[sb][i + 1];
               } else {
                 const uint32_t x = drop_pair_hash(drop_o + (uint32_t)(sbase + off) * kDropQ);
                 const bool keep = ((x >> (16 * (opos & 1))) & 0xFFFFu) >= p.drop_thr;
-                pv[i] = keep ? pv[i] : 0.f;
+                pv[sb][i] = keep ? pv[sb][i] : 0.f;
                 pd[sb][i] = keep ? pd[sb][i] : -pd[sb][i];
               }
             }
@@ -508,7 +537,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 #pragma unroll
           for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) pf[2 * sb + j][e] = (E)pv[8 * j + e];
+            for (int e = 0; e < 8; ++e) pf[2 * sb + j][e] = (E)pv[sb][8 * j + e];
         }
       }
       {
@@ -524,8 +553,6 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
             for (int sb = 0; sb < TB; ++sb)
               x2[sb] = mfma32(frag_row(t2, (qh * TB + sb) * 32 + r, ks), b2, x2[sb]);
           }
-        } else if constexpr (!T::EARLY_X2) {
-          second_product(x2);
         }
 #pragma unroll
         for (int sb = 0; sb < TB; ++sb) {
@@ -591,15 +618,36 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
   } else {
     // positional masks: every step of [t_lo, t_hi] is visited (a dead one only occurs under a prefix-LM mask)
-    if (n_steps > s_first) load_step(s_first, s_first & 1);
-    dma_wait<0>();
-    for (int s = s_first; s < n_steps; ++s) {
-      const int slot = s & 1;
-      __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
-      if (s + 1 < n_steps) load_step(s + 1, slot ^ 1);
-      bool full, doc_uniform;
-      if (!classify_step(s, full, doc_uniform)) run_step(s, slot, full, doc_uniform);
+    if constexpr (T::UNROLL2) {
+      // (two steps per turn of the loop: the ring slot is then a constant, part of the LDS instructions' offsets instead of 20
+      // address additions per step)
+      auto step_at = [&](int s, auto slot_tag) FL_INLINE {
+        constexpr int slot = decltype(slot_tag)::value;
+        __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
+        if (s + 1 < n_steps) load_step(s + 1, slot ^ 1);
+        bool full, doc_uniform;
+        if (!classify_step(s, full, doc_uniform)) run_step(s, slot, full, doc_uniform);
+        dma_wait<0>();
+      };
+      if (n_steps > s_first) load_step(s_first, 0);
       dma_wait<0>();
+      int s = s_first;
+      for (; s + 1 < n_steps; s += 2) {
+        step_at(s, std::integral_constant<int, 0>{});
+        step_at(s + 1, std::integral_constant<int, 1>{});
+      }
+      if (s < n_steps) step_at(s, std::integral_constant<int, 0>{});
+    } else {
+      if (n_steps > s_first) load_step(s_first, s_first & 1);
+      dma_wait<0>();
+      for (int s = s_first; s < n_steps; ++s) {
+        const int slot = s & 1;
+        __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
+        if (s + 1 < n_steps) load_step(s + 1, slot ^ 1);
+        bool full, doc_uniform;
+        if (!classify_step(s, full, doc_uniform)) run_step(s, slot, full, doc_uniform);
+        dma_wait<0>();
+      }
     }
   }
 
