@@ -496,10 +496,11 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
     if validate_only:
         _check(lib.fl_attn_bwd_validate(C.byref(b)))
         return dq, dk, dv
-    split_bytes = lib.fl_attn_bwd_split_bytes(C.byref(b.fwd)) if split and not use_static else 0
-    if split_bytes:
-        scratch = torch.empty(split_bytes, dtype=torch.uint8, device=q.device)
-        _launch_on(q.device, lambda params, stream: lib.fl_attn_bwd_split(params, scratch.data_ptr(), split_bytes, stream), b)
+    if split and not use_static:
+        split_bytes = lib.fl_attn_bwd_split_bytes(C.byref(b.fwd))
+        scratch = torch.empty(split_bytes, dtype=torch.uint8, device=q.device) if split_bytes else None
+        _launch_on(q.device, lambda params, stream: lib.fl_attn_bwd_split(
+            params, scratch.data_ptr() if split_bytes else None, split_bytes, stream), b)
     else:
         _launch_on(q.device, lib.fl_attn_bwd_static if use_static else lib.fl_attn_bwd, b)
     del keep, delta

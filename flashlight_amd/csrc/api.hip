@@ -1096,9 +1096,8 @@ uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p) {
   return plan_bwd(p).bytes;
 }
 
-int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream) { return fl_attn_bwd_split(b, nullptr, 0, stream); }
-
-int fl_attn_bwd_split(const fl_attn_bwd_params* b, void* scratch, uint64_t scratch_bytes, void* stream_) {
+// `planned`: sums may be taken in another order than one workgroup per tile and role takes them in, whatever else the call holds
+static int launch_gradients(const fl_attn_bwd_params* b, bool planned, void* scratch, uint64_t scratch_bytes, void* stream_) {
   const fl::BwdInstance* in = nullptr;
   int rc = validate_bwd(b, &in);
   if (rc) return rc;
@@ -1166,7 +1165,11 @@ int fl_attn_bwd_split(const fl_attn_bwd_params* b, void* scratch, uint64_t scrat
     bp.doc_blocks = blocks;
   }
   BwdPlan plan = plan_bwd(p);
-  if (!scratch || plan.bytes > scratch_bytes) plan.dq = plan.dkv = 1;
+  if (plan.bytes && (!scratch || plan.bytes > scratch_bytes)) planned = false;
+  if (!planned) {
+    plan.dq = plan.dkv = 1;
+    plan.both = plan.both && p->Dqk <= 64;  // (at head dim 128 the shared launch halves every dQ step between two waves)
+  }
   bp.part_dq = static_cast<float*>(scratch);
   if (plan.dkv > 1) bp.part = bp.part_dq + plan.dq_bytes / sizeof(float);
   bp.splits_dq = plan.dq;
@@ -1183,6 +1186,12 @@ int fl_attn_bwd_split(const fl_attn_bwd_params* b, void* scratch, uint64_t scrat
   e = in->launch_dkv(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the dK/dV kernel failed: %s", hipGetErrorString(e));
   return 0;
+}
+
+int fl_attn_bwd(const fl_attn_bwd_params* b, void* stream) { return launch_gradients(b, false, nullptr, 0, stream); }
+
+int fl_attn_bwd_split(const fl_attn_bwd_params* b, void* scratch, uint64_t scratch_bytes, void* stream) {
+  return launch_gradients(b, true, scratch, scratch_bytes, stream);
 }
 
 uint64_t fl_attn_shared_bias_bwd_bytes(const fl_attn_params* p) {

@@ -234,9 +234,10 @@ int fl_attn_bwd_validate(const fl_attn_bwd_params* p);
 /* Launches the backward kernels (row sums of dO o O; then dQ, dK and dV, in one launch or two) on `stream`. */
 int fl_attn_bwd(const fl_attn_bwd_params* p, void* stream);
 
-/* fl_attn_bwd with scratch of its own (16-byte aligned, contents undefined before and after) in which workgroups that
- * share a tile leave partial sums: for calls whose tiles alone would leave most of the GPU idle.  One more launch
- * adds them up.  With less than fl_attn_bwd_split_bytes(), or NULL, the call is fl_attn_bwd. */
+/* fl_attn_bwd for calls whose tiles alone would leave most of the GPU idle: sums may be taken in an order that depends on
+ * the size of the call (the same for the same call).  scratch (16-byte aligned, contents undefined before and after):
+ * workgroups that share a tile leave partial sums in it and one more launch adds them up.  With less than
+ * fl_attn_bwd_split_bytes(), the call is fl_attn_bwd. */
 int fl_attn_bwd_split(const fl_attn_bwd_params* p, void* scratch, uint64_t scratch_bytes, void* stream);
 /* Bytes of scratch fl_attn_bwd_split can use for the gradients of the forward call *p; 0: none.  Host only. */
 uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p);
