@@ -470,7 +470,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
             for (int e = 0; e < 4; ++e) {
               const int i = 4 * g + e, off = 8 * g + e;
               const float x = x1[sb][i];
-              const float c0 = alibi0 - (kDQ ? lse_o : lse4[e]);
+              const float lse = kDQ ? lse_o : lse4[e];
+              const float c0 = kAlibi ? alibi0 - lse : -lse;  // (0 - lse would be an instruction of its own)
               float s2, dfac = 1.0f;  // logit in log2 units minus the LSE; d(score) / d(qk * scale)
               if constexpr (kSoftcap) {
                 const float ex = fast_exp2(x * cap_k1);
