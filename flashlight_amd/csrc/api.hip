@@ -1057,9 +1057,10 @@ int fl_attn_bwd_validate(const fl_attn_bwd_params* b) { return validate_bwd(b, n
 // sums a launch of 5 to 9 us: no split has fewer than eight steps, and a tile of up to one and a half shares stays whole.
 // Beyond, a launch per role is the better one (4 x 16 x 2048, head dim 64, causal: 177 us against 188; 2 x 16 x 2048, head
 // dim 128, unmasked: 271 against 300).
-// Gradients, bf16, a launch per role with whole tiles -> this rule: 3 x 16 heads over 4 x 1000 prefix rows, head dim 64:
-// 157 -> 77 us; 8 x 512 causal, 64: 36 -> 25; 8 over 1 x 8192 causal, 64: 1980 -> 342; 8 x 512 causal, 128: 47 -> 29; 8 over
-// 1 x 2048 causal, 128: 568 -> 73; 32 over 4 x 4096 causal, 128: 1214 -> 611; 2 x 16 x 2048 causal, 64: 131 -> 107.
+// Gradients, bf16, a launch per role with whole tiles -> this rule (both with the mask as selects, see bwd_kernel.h), now in
+// brackets: 3 x 16 heads over 4 x 1000 prefix rows, head dim 64: 157 -> 77 us (72); 8 x 512 causal, 64: 36 -> 25 (20); 8 over
+// 1 x 8192 causal, 64: 1980 -> 342 (284); 8 x 512 causal, 128: 47 -> 29 (27); 8 over 1 x 2048 causal, 128: 568 -> 73 (72);
+// 32 over 4 x 4096 causal, 128: 1214 -> 611 (565); 2 x 16 x 2048 causal, 64: 131 -> 107 (94).
 namespace {
 struct BwdPlan {
   bool both = false;    // one launch
