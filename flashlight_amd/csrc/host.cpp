@@ -337,6 +337,8 @@ struct SharedBias : torch::autograd::Function<SharedBias> {
         set_strides(b.dgate_strides, dgate);
       }
       if (ctx->needs_input_grad(3)) {
+        TORCH_CHECK(c.bias[0].size(0) == b.fwd.B / c.bias_div[0], "one gradient per ", c.bias_div[0], " batch entries, ",
+                    c.bias[0].size(0), " operands");
         dbias = at::empty(c.bias[0].sizes(), c.bias[0].options().requires_grad(false));
         b.dbias = dbias.data_ptr();
       }
@@ -451,6 +453,9 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
         std::swap(c.bias[0], c.bias[1]);
         std::swap(c.bias_div[0], c.bias_div[1]);
       }
+      // a batch axis of 1 says that all batch entries share the operand: the gradient kernels write one [Hq, Lq, Lk] per
+      // B / divisor, and there is room for one
+      if (c.bias[0].defined() && c.bias[0].size(0) == 1) c.bias_div[0] = B;
       fl_attn_params p = {};
       fill(c, p);
       if (!c.bias[0].defined() || c.bias[0].size(1) != Hq || c.bias[0].size(2) != Lq || c.bias[0].size(3) != Lk ||

@@ -265,7 +265,8 @@ uint64_t fl_static_scratch_bytes(void);
  * (evoformer.py:8-36).  No counterpart in the reference, which is forward-only.  Unmasked, no score modification, no
  * dropout; Lq == Lk <= 512, Hq == Hkv, Dqk == Dv in {32, 64}; the dense operand has its own row for every head and query.
  * fwd, dout, dq, dk, dv as in fl_attn_bwd_params, with fwd.o the (gated) result, and fwd.gate as in the forward.
- * dbias (optional): gradient of the dense operand, [B / bias_batch_div, Hq, Lq, Lk] contiguous, in the operand's type.
+ * dbias (optional): gradient of the dense operand, [B / bias_batch_div, Hq, Lq, Lk] contiguous, in the operand's type; also
+ * with a batch stride of 0, where the caller adds up the B / bias_batch_div gradients (or says bias_batch_div = B).
  * dgate (with fwd.gate): gradient of the gate's logits, addressed with dgate_strides.
  * workspace: fl_attn_shared_bias_bwd_bytes() bytes, 256-byte aligned, contents undefined.
  * Four launches (row sums and gate; dQ and the bias's partial sums; dK and dV; the sum), no atomics. */

@@ -8,7 +8,7 @@ import torch
 
 import flashlight_amd.attention_variants as A
 import oracle as O
-from flashlight_amd import _ffi
+from flashlight_amd import _ffi, ops
 from tests.test_abi import good_params
 
 DEV = "cuda"
@@ -73,6 +73,32 @@ def test_gradients_against_the_oracle(shape, gate):
             rel = ((a.float().cpu() - b).norm() / b.norm()).item()
             assert a.dtype == (torch.float32 if f32 and name == "dbias" else dt) and a.shape == b.shape
             assert rel < (1e-2 if dt == torch.bfloat16 else 3e-3), (shape, gate, mask, f32, name, rel)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(8, 2, 33, 32), (5, 1, 64, 64), (3, 2, 96, 32)])  # B, H, S, D
+@pytest.mark.parametrize("bias_dtype", [torch.bfloat16, torch.float32])
+def test_one_bias_for_the_whole_batch(shape, bias_dtype):
+    """A bias with a batch axis of 1 and the divisor left at 1: its gradient is the sum over the batch, and nothing is
+    written beside it (the freed slot between tensors of the gradient's size is where the allocator puts it)."""
+    B, H, S, D = shape
+    g = torch.Generator().manual_seed(sum(shape))
+    q, k, v, dout = (torch.randn(B, H, S, D, generator=g).to(torch.bfloat16) for _ in range(4))
+    pair = torch.randn(1, H, S, S, generator=g).to(bias_dtype)
+    row = torch.randn(B, 1, 1, S, generator=g).to(torch.bfloat16)
+    for biases in ([pair], [pair, row], [row, pair]):
+        dev = [t.to(DEV).requires_grad_(True) for t in (q, k, v, pair)]
+        out = ops.dispatch(*dev[:3], biases=[(dev[3] if b is pair else b.to(DEV), 1) for b in biases])
+        around = [torch.full((1, H, S, S), 7.0, dtype=bias_dtype, device=DEV) for _ in range(4 * B)]
+        del around[2 * B]
+        grads = torch.autograd.grad(out, dev, dout.to(DEV))
+        assert all((t == 7.0).all() for t in around)
+        ref = [t.float().requires_grad_(True) for t in (q, k, v, pair)]
+        s = ref[0] @ ref[1].transpose(-1, -2) / D ** 0.5 + sum(ref[3] if b is pair else b.float() for b in biases)
+        want = torch.autograd.grad(torch.softmax(s, -1) @ ref[2], ref, dout.float())
+        for name, a, b in zip(("dq", "dk", "dv", "dbias"), grads, want):
+            assert a.shape == b.shape
+            assert ((a.float().cpu() - b).norm() / b.norm()).item() < 1e-2, (shape, name)
 
 
 @pytest.mark.gpu
