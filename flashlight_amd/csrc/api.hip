@@ -742,6 +742,7 @@ bool plan_shared_bias_bwd(const fl_attn_params* p, SBScratch* out) {
   // per-lane byte offsets inside one (batch entry, head) are 32-bit
   for (const int64_t* st : {p->q_strides, p->k_strides, p->v_strides, p->o_strides})
     if (st[2] < 0 || st[2] >= (1 << 20)) return false;
+  if ((int64_t)p->Hq * p->Dv >= (1 << 20)) return false;  // (of a result, and of the gated output gradient, in sequence-major order)
   const int64_t S = p->Lk, H = p->Hq, div = p->bias_batch_div[x.dense], groups = p->B / div, tiles = (S + 31) / 32;
   // entries per workgroup: as many as leave one round of workgroups
   const int per_cu = fl::pairbias_bwd_shape(p->Dqk, (int)S).lds_bytes <= 80 * 1024 ? 2 : 1;

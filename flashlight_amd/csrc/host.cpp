@@ -315,7 +315,8 @@ struct SharedBias : torch::autograd::Function<SharedBias> {
     const bool grad_mode = at::GradMode::is_enabled();
     {
       at::AutoGradMode off(false);
-      const Tensor dout = prepare_dout(grads[0], c.q);
+      Tensor dout = prepare_dout(grads[0], c.q);
+      if (dout.stride(2) >= 1 << 20) dout = dout.contiguous();  // (the kernels' offsets inside one (batch entry, head))
       fl_attn_shared_bias_bwd_params b = {};
       fill(c, b.fwd);
       b.fwd.o = const_cast<void*>(out.const_data_ptr());

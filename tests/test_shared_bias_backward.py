@@ -32,6 +32,7 @@ def test_which_calls_the_shared_bias_backward_takes():
     assert takes(params()) and takes(params(S=512, D=64)) and takes(params(S=1))
     assert not takes(params(S=513)) and not takes(params(D=128)) and not takes(params(softcap=3.0))
     assert not takes(params(mask_kind=_ffi.MASK_CAUSAL)) and not takes(params(Hkv=2)) and not takes(params(Lq=128))
+    assert not takes(params(H=1 << 15)) and takes(params(H=(1 << 15) - 1))  # rows of [position][head][dim] results: 2^20 elements
     p = params()
     p.bias_strides[0][1] = 0  # one bias for all heads: another sum
     assert not takes(p)
@@ -99,6 +100,21 @@ def test_one_bias_for_the_whole_batch(shape, bias_dtype):
         for name, a, b in zip(("dq", "dk", "dv", "dbias"), grads, want):
             assert a.shape == b.shape
             assert ((a.float().cpu() - b).norm() / b.norm()).item() < 1e-2, (shape, name)
+
+
+@pytest.mark.gpu
+def test_output_gradient_with_rows_far_apart():
+    """An output gradient whose positions lie 2^20 elements apart, beyond the kernels' offsets, is copied."""
+    g = torch.Generator().manual_seed(2)
+    q, k, v, gate, dout = (torch.randn(1, 2, 33, 2, 32, generator=g).to(torch.bfloat16).to(DEV).requires_grad_(True) for _ in range(5))
+    pair = torch.randn(1, 1, 2, 33, 33, generator=g).to(torch.bfloat16).to(DEV).requires_grad_(True)
+    far = torch.empty(33 << 20, dtype=torch.bfloat16, device=DEV).as_strided(dout.shape, (128, 64, 1 << 20, 32, 1))
+    far.copy_(dout.detach())
+    for kw in ({}, {"gate": gate}):
+        leaves = [q, k, v, pair, *kw.values()]
+        out = A.attention_reference(q, k, v, [pair], **kw)
+        near = torch.autograd.grad(out, leaves, dout.detach(), retain_graph=True)
+        assert all(torch.equal(a, b) for a, b in zip(torch.autograd.grad(out, leaves, far), near))
 
 
 @pytest.mark.gpu
