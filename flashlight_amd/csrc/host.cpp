@@ -370,6 +370,25 @@ bool take_tensor(PyObject* o, Tensor& t) {
   return plain(t);
 }
 
+// Other Python threads run while this one allocates and launches (the allocator may go to the driver, the launch queue may
+// be full).
+struct WithoutGil {
+  PyThreadState* state = PyEval_SaveThread();
+  ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
+// The call itself; an undefined tensor if the C ABI does not take it.
+Tensor attend(const Call& c) {
+  const WithoutGil no_gil;
+  if (!c.wants_grad) return launch_forward(c, nullptr);
+  try {
+    return c.bias[0].defined() ? SharedBias::apply(c.q, c.k, c.v, c.bias[0], given(c.bias[1]), given(c.gate), c)
+                               : Attention::apply(c.q, c.k, c.v, c);
+  } catch (const Refused&) {
+    return Tensor();
+  }
+}
+
 // forward(q, k, v, scale, mask_kind, window, prefix, doc_ids, alibi_heads, softcap, biases, gate, diff, lambda, seq_major)
 PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -446,7 +465,6 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
                                                 (c.gate.defined() && c.gate.requires_grad()) ||
                                                 (c.bias[0].defined() && c.bias[0].requires_grad()) ||
                                                 (c.bias[1].defined() && c.bias[1].requires_grad()));
-  Tensor out;
   if (c.wants_grad) {
     if (c.diff) Py_RETURN_NONE;
     if (nb || c.gate.defined()) {
@@ -466,15 +484,9 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     } else {
       c.seq_major = false;
     }
-    try {
-      out = nb ? SharedBias::apply(q, k, v, c.bias[0], given(c.bias[1]), given(c.gate), c) : Attention::apply(q, k, v, c);
-    } catch (const Refused&) {
-      Py_RETURN_NONE;
-    }
-  } else {
-    out = launch_forward(c, nullptr);
-    if (!out.defined()) Py_RETURN_NONE;
   }
+  Tensor out = attend(c);
+  if (!out.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }

@@ -1,0 +1,40 @@
+"""The native host path of the front ends (csrc/host.cpp): what it takes, and that it behaves as the Python path does."""
+import ctypes as C
+
+import pytest
+import torch
+
+from flashlight_amd import _ffi, ops
+
+DEV = "cuda"
+_BOUND = ("fl_attn_fwd", "fl_attn_bwd_split", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_bwd_split_bytes", "fl_attn_rows_plan",
+          "fl_attn_shared_bias_bwd_bytes", "fl_attn_shared_bias_bwd", "fl_last_error")
+
+
+def _operands(*shape, dtype=torch.bfloat16, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return [torch.randn(*shape, generator=g).to(dtype).to(DEV) for _ in range(3)]
+
+
+@pytest.mark.gpu
+def test_other_threads_run_while_a_call_is_launched():
+    """The library's entries replaced by CPython's own question whether this thread holds the interpreter: it returns 1,
+    which the host path reads as a refusal, or 0, a launch."""
+    lib = _ffi.load_library()
+    address = {f: C.cast(getattr(lib, f), C.c_void_p).value for f in _BOUND}
+    asked = C.cast(C.pythonapi.PyGILState_Check, C.c_void_p).value
+    q, k, v = _operands(1, 2, 64, 64)
+    pair = torch.zeros(1, 2, 64, 64, dtype=torch.bfloat16, device=DEV)
+    args = (None, 0, 0, 0, None, 0, 0.0)
+    try:
+        _ffi._host.bind(*(asked if f in ("fl_attn_fwd", "fl_attn_bwd_split", "fl_attn_shared_bias_bwd") else a for f, a in address.items()))
+        assert _ffi._host.forward(q, k, v, *args, (), None, False, 0.0, False) is not None
+        q.requires_grad_(True)
+        for biases in ((), ((pair, 1),)):
+            out = _ffi._host.forward(q, k, v, *args, biases, None, False, 0.0, False)
+            assert out is not None
+            torch.autograd.grad(out, [q], torch.zeros_like(out))
+    finally:
+        _ffi._host.bind(*address.values())
+    q.requires_grad_(False)
+    assert torch.isfinite(ops.dispatch(q, k, v)).all()
