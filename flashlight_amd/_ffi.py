@@ -89,6 +89,9 @@ class FlashlightError(RuntimeError):
 
 _lib: Optional[C.CDLL] = None
 _host = None  # the native host path of the front ends (csrc/host.cpp), loaded with the library
+_HOST_ENTRIES = ("fl_attn_fwd", "fl_attn_bwd_split", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_bwd_split_bytes",
+                 "fl_attn_rows_plan", "fl_attn_shared_bias_bwd_bytes", "fl_attn_shared_bias_bwd", "fl_last_error",
+                 "fl_attn_fwd_ungated")  # what it calls, in the order it expects
 _MAX_DV_DIFF = 128  # widest value slab of a differential-attention kernel instance
 
 
@@ -148,9 +151,7 @@ def load_library(path: os.PathLike | str | None = None) -> C.CDLL:
     except ImportError as e:
         raise ImportError("flashlight_amd/_host.so is missing or does not load: build it with `python -m flashlight_amd.build`") from e
     _host = host_module
-    _host.bind(*(C.cast(getattr(lib, f), C.c_void_p).value for f in (
-        "fl_attn_fwd", "fl_attn_bwd_split", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_bwd_split_bytes", "fl_attn_rows_plan",
-        "fl_attn_shared_bias_bwd_bytes", "fl_attn_shared_bias_bwd", "fl_last_error")))
+    _host.bind(*(C.cast(getattr(lib, f), C.c_void_p).value for f in _HOST_ENTRIES))
     _lib = lib
     return lib
 
@@ -233,7 +234,7 @@ class DocWorkspace:
         self.ids = None
 
 
-FLAG_DOC_PREPARED = 1
+FLAG_DOC_PREPARED, FLAG_UNGATED = 1, 2  # fl_attn_params.flags
 SCORE_NONE, SCORE_SIGMOID, SCORE_CLAMP, SCORE_POLY = 0, 1, 2, 3  # fl_attn_params.score_fn
 
 

@@ -392,7 +392,7 @@ int check_ptr(const char* what, const void* ptr, int align) {
   return 0;
 }
 
-int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = false) {
+int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = false, uint32_t flags = FL_FLAG_DOC_PREPARED) {
   if (!p) return fail(FL_ERR_NULL, "params is null");
   int rc;
   if ((rc = check_ptr("q", p->q, 16)) || (rc = check_ptr("k", p->k, 16)) || (rc = check_ptr("v", p->v, 16)) ||
@@ -410,7 +410,7 @@ int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = f
   if ((rc = check_strides("q", p->q_strides, 8)) || (rc = check_strides("k", p->k_strides, 8)) ||
       (rc = check_strides("v", p->v_strides, 8)) || (rc = check_strides("o", p->o_strides, 4)))
     return rc;
-  if (p->flags & ~(uint32_t)FL_FLAG_DOC_PREPARED) return fail(FL_ERR_ARG, "unknown bits in flags: 0x%x", p->flags);
+  if (p->flags & ~flags) return fail(FL_ERR_ARG, "unknown bits in flags: 0x%x", p->flags);
   if ((p->flags & FL_FLAG_DOC_PREPARED) && !is_doc(p->mask_kind))
     return fail(FL_ERR_ARG, "FL_FLAG_DOC_PREPARED goes with a document mask only");
   if (p->dropout_threshold) {
@@ -829,13 +829,13 @@ int fl_attn_rows_plan(const fl_attn_params* p, uint64_t* scratch_bytes) {
   return plan_rows(p, &rp, &grid, &waves, &blocks, scratch_bytes) ? 1 : 0;
 }
 
-int fl_attn_fwd(const fl_attn_params* p, void* stream_) {
+static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_) {
   const fl::Instance* in = nullptr;
   int rc = validate(p, &in);
   if (rc) return rc;
   hipStream_t stream = static_cast<hipStream_t>(stream_);
 
-  {
+  if (!ungated) {
     fl::PParams pb;
     int pb_grid = 0;
     if (plan_pairbias(p, &pb, &pb_grid)) {
@@ -941,6 +941,7 @@ int fl_attn_fwd(const fl_attn_params* p, void* stream_) {
     else if (kp.bias_lds < 0) kp.bias_lds = nb;
   }
   kp.gate = static_cast<const fl::bf16_t*>(p->gate);
+  kp.ungated = static_cast<fl::bf16_t*>(ungated);
   kp.lambda = p->lambda;
   if (p->diff) {
     // heads [0, H) are branch 0, heads [H, 2H) branch 1 (query: H = Hq, key: H = Hkv)
@@ -993,6 +994,15 @@ int fl_attn_fwd(const fl_attn_params* p, void* stream_) {
   hipError_t e = in->launch(kp, grid, (int)lds_bytes_for(in, p), stream);
   if (e != hipSuccess) return fail((int)e, "launch of %s failed: %s", in->name, hipGetErrorString(e));
   return 0;
+}
+
+int fl_attn_fwd(const fl_attn_params* p, void* stream) { return launch_forward(p, nullptr, stream); }
+
+int fl_attn_fwd_ungated(const fl_attn_params* p, void* ungated, void* stream) {
+  if (!p) return fail(FL_ERR_NULL, "params is null");
+  if (!p->gate) return fail(FL_ERR_ARG, "a result before the gate needs a gate");
+  const int rc = check_ptr("ungated", ungated, 16);
+  return rc ? rc : launch_forward(p, ungated, stream);
 }
 
 uint64_t fl_static_scratch_bytes(void) { return kStaticScratchBytes; }
@@ -1204,7 +1214,7 @@ uint64_t fl_attn_shared_bias_bwd_bytes(const fl_attn_params* p) {
 int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* stream_) {
   if (!b) return fail(FL_ERR_NULL, "params is null");
   const fl_attn_params* p = &b->fwd;
-  int rc = validate(p, nullptr);
+  int rc = validate(p, nullptr, false, FL_FLAG_DOC_PREPARED | FL_FLAG_UNGATED);
   if (rc) return rc;
   SBScratch x;
   if (!plan_shared_bias_bwd(p, &x)) return fail(FL_ERR_UNSUPPORTED, "fl_attn_shared_bias_bwd does not take this call");
@@ -1233,6 +1243,7 @@ int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* strea
   pp.out = static_cast<const fl::bf16_t*>(p->o);
   pp.dout = static_cast<const fl::bf16_t*>(b->dout);
   pp.gate = static_cast<const fl::bf16_t*>(p->gate);
+  pp.ungated = (p->flags & FL_FLAG_UNGATED) != 0;
   pp.dgated = reinterpret_cast<fl::bf16_t*>(ws + x.dgated);
   pp.dgate = static_cast<fl::bf16_t*>(b->dgate);
   pp.delta = reinterpret_cast<float*>(ws + x.delta);

@@ -99,6 +99,7 @@ struct KParams {
   float score_k[4];
   int32_t n_qtiles;  // ceil(Lq / BM)
   int32_t n_ktiles;  // ceil(Lk / BN)
+  bf16_t* ungated;   // with a gate, optional: the result before the gate as well, addressed like o (for the gradients)
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -1424,7 +1425,27 @@ void fwd_kernel(const KParams p) {
   // ---- epilogue: O^T register i of block (dvb, qb) is out[q = qrow[qb]][dv = 32*dvb + 8*(i/4) + 4h + i%4] ----------
   bf16_t* optr = p.o + (int64_t)batch * p.os[0] + (int64_t)head * p.os[1];
   const bf16_t* gptr = (kGate && p.gate) ? p.gate + (int64_t)batch * p.gs[0] + (int64_t)head * p.gs[1] : nullptr;
+  bf16_t* uptr = (kGate && p.ungated) ? p.ungated + (int64_t)batch * p.os[0] + (int64_t)head * p.os[1] : nullptr;
   const bool wide = __builtin_amdgcn_readfirstlane(p.o_wide) != 0;
+  auto store_block = [&](const ex4 (&quad)[4], bf16_t* to, int qb, int dvb) FL_INLINE {
+    if (wide) {
+      // the two lanes of a query trade halves of two groups of 4 columns, after which the first holds columns
+      // 16 j .. + 8 of the block and the second the next 8: 16-byte stores, half as many partial lines per store
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const u32x2 qa = __builtin_bit_cast(u32x2, quad[2 * j]), qb_ = __builtin_bit_cast(u32x2, quad[2 * j + 1]);
+        uint32_t a0 = qa[0], a1 = qa[1], b0 = qb_[0], b1 = qb_[1];
+        swap_halves(a0, b0);
+        swap_halves(a1, b1);
+        const u32x4 w = {a0, a1, b0, b1};
+        if (qrow[qb] < p.Lq) *reinterpret_cast<u32x4*>(to + (int64_t)qrow[qb] * p.os[2] + 32 * dvb + 16 * j + 8 * h) = w;
+      }
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<ex4*>(to + (int64_t)qrow[qb] * p.os[2] + 32 * dvb + 8 * g + 4 * h) = quad[g];
+    }
+  };
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     // (the wide path trades register halves between the two lanes of a query: rows past Lq go along and store nothing)
@@ -1451,22 +1472,15 @@ void fwd_kernel(const KParams p) {
         }
         quad[g] = o4;
       }
-      if (wide) {
-        // the two lanes of a query trade halves of two groups of 4 columns, after which the first holds columns
-        // 16 j .. + 8 of the block and the second the next 8: 16-byte stores, half as many partial lines per store
+      store_block(quad, optr, qb, dvb);
+      if constexpr (kGate) {
+        if (uptr) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          const u32x2 qa = __builtin_bit_cast(u32x2, quad[2 * j]), qb_ = __builtin_bit_cast(u32x2, quad[2 * j + 1]);
-          uint32_t a0 = qa[0], a1 = qa[1], b0 = qb_[0], b1 = qb_[1];
-          swap_halves(a0, b0);
-          swap_halves(a1, b1);
-          const u32x4 w = {a0, a1, b0, b1};
-          if (qrow[qb] < p.Lq) *reinterpret_cast<u32x4*>(optr + (int64_t)qrow[qb] * p.os[2] + 32 * dvb + 16 * j + 8 * h) = w;
+          for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) quad[g][e] = (E)oacc[dvb][qb][4 * g + e];
+          store_block(quad, uptr, qb, dvb);
         }
-      } else {
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<ex4*>(optr + (int64_t)qrow[qb] * p.os[2] + 32 * dvb + 8 * g + 4 * h) = quad[g];
       }
     }
   }

@@ -39,8 +39,9 @@ struct Api {
   uint64_t (*shared_bias_bwd_bytes)(const fl_attn_params*) = nullptr;
   int (*shared_bias_bwd)(const fl_attn_shared_bias_bwd_params*, void*) = nullptr;
   const char* (*last_error)(void) = nullptr;
+  int (*fwd_ungated)(const fl_attn_params*, void*, void*) = nullptr;
 } g_api;
-constexpr int kApiFunctions = 9;
+constexpr int kApiFunctions = 10;
 
 // One call's arguments.  The tensors are the caller's; `doc`, `bias` and `gate` may be undefined.
 struct Call {
@@ -135,8 +136,8 @@ void fill(const Call& c, fl_attn_params& p) {
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 // Launches the forward of `c` into a fresh tensor; an undefined tensor if the C ABI refuses (the Python path then says why).
-// `lse`: when given, receives the row statistics.
-Tensor launch_forward(const Call& c, Tensor* lse) {
+// `lse`: when given, receives the row statistics; `ungated` the result before the gate.
+Tensor launch_forward(const Call& c, Tensor* lse, Tensor* ungated = nullptr) {
   fl_attn_params p = {};
   fill(c, p);
   Tensor q = c.q, out;
@@ -149,6 +150,10 @@ Tensor launch_forward(const Call& c, Tensor* lse) {
   if (lse) {
     *lse = at::empty({p.B, p.Hq, p.Lq}, opt.dtype(at::kFloat));
     p.lse = lse->data_ptr<float>();
+  }
+  if (ungated) {
+    *ungated = at::empty_strided(out.sizes(), out.strides(), opt);
+    return g_api.fwd_ungated(&p, ungated->data_ptr(), current_stream()) == 0 ? out : Tensor();
   }
   uint64_t bytes = 0;
   Tensor ws;
@@ -291,10 +296,11 @@ struct Attention : torch::autograd::Function<Attention> {
 struct SharedBias : torch::autograd::Function<SharedBias> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& bias,
                         const std::optional<Tensor>& row, const std::optional<Tensor>& gate, const Call& c) {
-    Tensor lse;
-    Tensor out = launch_forward(c, &lse);
+    Tensor lse, ungated;
+    Tensor out = launch_forward(c, &lse, gate ? &ungated : nullptr);
     if (!out.defined()) throw Refused();
-    ctx->save_for_backward({q, k, v, bias, row.value_or(Tensor()), gate.value_or(Tensor()), out, lse});
+    // (the gradients are formed from the attention's own result: a nearly closed gate leaves the gated one few bits)
+    ctx->save_for_backward({q, k, v, bias, row.value_or(Tensor()), gate.value_or(Tensor()), gate ? ungated : out, lse});
     keep_scalars(ctx, c);
     return out;
   }
@@ -322,6 +328,7 @@ struct SharedBias : torch::autograd::Function<SharedBias> {
       b.fwd.o = const_cast<void*>(out.const_data_ptr());
       set_strides(b.fwd.o_strides, out);
       b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
+      if (c.gate.defined()) b.fwd.flags = FL_FLAG_UNGATED;
       Tensor dq = empty_for_gradient(c.q), dk = empty_for_gradient(c.k), dv = empty_for_gradient(c.v);
       b.dout = dout.const_data_ptr();
       b.dq = dq.data_ptr();
@@ -495,7 +502,7 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* f[kApiFunctions];
   if (n != kApiFunctions) {
-    PyErr_SetString(PyExc_TypeError, "bind takes the addresses of nine functions");
+    PyErr_SetString(PyExc_TypeError, "bind takes the addresses of ten functions");
     return nullptr;
   }
   for (int i = 0; i < kApiFunctions; ++i) f[i] = PyLong_AsVoidPtr(a[i]);
@@ -509,6 +516,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   g_api.shared_bias_bwd_bytes = reinterpret_cast<decltype(g_api.shared_bias_bwd_bytes)>(f[6]);
   g_api.shared_bias_bwd = reinterpret_cast<decltype(g_api.shared_bias_bwd)>(f[7]);
   g_api.last_error = reinterpret_cast<decltype(g_api.last_error)>(f[8]);
+  g_api.fwd_ungated = reinterpret_cast<decltype(g_api.fwd_ungated)>(f[9]);
   Py_RETURN_NONE;
 }
 

@@ -412,13 +412,16 @@ struct SBPrepParams {
   float* rowb;
   int64_t row_batch;
   int32_t row_key, row_div, row_f32;
+  int32_t ungated;         // `out` is the result before the gate
   int64_t os[3], dos[3], gs[3], dgds[3], dgs[3];
   int32_t B, H, S;
 };
 
-// What the two roles need per row, in one pass over dO and the result.  With the gate g and the result out = sigmoid(g) o O
-// the general formulas need only out: Delta = rowsum(dO sigmoid(g) o O) = rowsum(dO o out), and the gradient of the
-// logits dO o O sigmoid(g) (1 - sigmoid(g)) = dO o out (1 - sigmoid(g)).
+// What the two roles need per row, in one pass over dO and the result.  With the gate's weights sg and the result before
+// the gate O: the output gradient of the attention dA = dO o sg, as rounded for the roles' products; Delta = rowsum(dA o O);
+// and the gradient of the logits dO o O o sg (1 - sg).  A caller that kept only the gated result out = sg o O gets
+// Delta = rowsum(dO o out) and dO o out (1 - sg): another rounding than dA's in Delta, and nothing of O where a nearly
+// closed gate leaves a 16-bit out few bits (fp16, logits around -12: 1e-2 instead of 3e-4 in the logits' gradient).
 template <int D, bool GATE, class E>
 __global__ __launch_bounds__(256) void pairbias_bwd_prep_kernel(const SBPrepParams p) {
   typedef E ex8 __attribute__((ext_vector_type(8)));
@@ -430,25 +433,28 @@ __global__ __launch_bounds__(256) void pairbias_bwd_prep_kernel(const SBPrepPara
   const int hd = (int)(row % p.H), s = (int)(row / p.H % p.S), b = (int)(row / ((int64_t)p.H * p.S));
   const ex8 d8 = *reinterpret_cast<const ex8*>(p.dout + b * p.dos[0] + hd * p.dos[1] + s * p.dos[2] + c);
   const ex8 o8 = *reinterpret_cast<const ex8*>(p.out + b * p.os[0] + hd * p.os[1] + s * p.os[2] + c);
-  float sum = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) sum += (float)d8[e] * (float)o8[e];
-#pragma unroll
-  for (int d = 1; d < LPR; d *= 2) sum += __shfl_xor(sum, d);
+  ex8 s8 = d8;  // what Delta sums against the result
   if constexpr (GATE) {
     const ex8 g8 = *reinterpret_cast<const ex8*>(p.gate + b * p.gs[0] + hd * p.gs[1] + s * p.gs[2] + c);
     ex8 a8, b8;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float sg = fast_rcp(1.0f + fast_exp2(-1.4426950408889634f * (float)g8[e]));
-      a8[e] = (E)((float)d8[e] * sg);
-      b8[e] = (E)((float)d8[e] * (float)o8[e] * (1.0f - sg));
+      const float da = (float)d8[e] * sg;
+      a8[e] = (E)da;
+      b8[e] = (E)((p.ungated ? da : (float)d8[e]) * (float)o8[e] * (1.0f - sg));
     }
+    if (p.ungated) s8 = a8;
     if (x < rows) {
       *reinterpret_cast<ex8*>(p.dgated + b * p.dgds[0] + hd * p.dgds[1] + s * p.dgds[2] + c) = a8;
       *reinterpret_cast<ex8*>(p.dgate + b * p.dgs[0] + hd * p.dgs[1] + s * p.dgs[2] + c) = b8;
     }
   }
+  float sum = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) sum += (float)s8[e] * (float)o8[e];
+#pragma unroll
+  for (int d = 1; d < LPR; d *= 2) sum += __shfl_xor(sum, d);
   if (x < rows && c == 0) {
     p.delta[((int64_t)b * p.H + hd) * p.S + s] = -sum;
     if (p.row != nullptr && hd == 0) {

@@ -155,6 +155,9 @@ typedef struct fl_attn_params {
  * are still read by the kernel itself; passing other ids than the workspace was prepared for gives wrong results. */
 #define FL_FLAG_DOC_PREPARED 1u
 
+/* fl_attn_shared_bias_bwd, with a gate: fwd.o is the result before the gate (fl_attn_fwd_ungated). */
+#define FL_FLAG_UNGATED 2u
+
 /* ABI version of the loaded library (FL_ABI_VERSION it was built with). */
 int fl_version(void);
 
@@ -185,6 +188,10 @@ int fl_attn_rows_plan(const fl_attn_params* p, uint64_t* scratch_bytes);
 /* Runs the fused forward on hipStream_t `stream` (NULL = default stream).
  * Replaces torch.compile(fn)(q, k, v, ...) for the functions of attention_variants/. */
 int fl_attn_fwd(const fl_attn_params* p, void* stream);
+
+/* fl_attn_fwd for calls with a gate whose gradients will be wanted: the result before the gate is written besides, to
+ * `ungated`, addressed like `o` (o_strides; 16-byte aligned). */
+int fl_attn_fwd_ungated(const fl_attn_params* p, void* ungated, void* stream);
 
 /* Describes the kernel instance fl_attn_fwd would pick for *p: tile sizes and launch shape.
  * out[0]=rows per workgroup, out[1]=keys per tile, out[2]=threads, out[3]=workgroups, out[4]=LDS bytes,
@@ -264,7 +271,9 @@ uint64_t fl_static_scratch_bytes(void);
  * that is one row of keys per batch entry, and optionally the sigmoid gate: the Evoformer's row attention
  * (evoformer.py:8-36).  No counterpart in the reference, which is forward-only.  Unmasked, no score modification, no
  * dropout; Lq == Lk <= 512, Hq == Hkv, Dqk == Dv in {32, 64}; the dense operand has its own row for every head and query.
- * fwd, dout, dq, dk, dv as in fl_attn_bwd_params, with fwd.o the (gated) result, and fwd.gate as in the forward.
+ * fwd, dout, dq, dk, dv as in fl_attn_bwd_params, with fwd.gate as in the forward.  Under a gate fwd.o is the result
+ * before it, with FL_FLAG_UNGATED in fwd.flags; without the flag fwd.o is the gated result, from which the gradients of a
+ * nearly closed gate come out coarser (fp16: once the gated values are no longer normal numbers).
  * dbias (optional): gradient of the dense operand, [B / bias_batch_div, Hq, Lq, Lk] contiguous, in the operand's type; also
  * with a batch stride of 0, where the caller adds up the B / bias_batch_div gradients (or says bias_batch_div = B).
  * dgate (with fwd.gate): gradient of the gate's logits, addressed with dgate_strides.

@@ -7,8 +7,6 @@ import torch
 from flashlight_amd import _ffi, ops
 
 DEV = "cuda"
-_BOUND = ("fl_attn_fwd", "fl_attn_bwd_split", "fl_workspace_bytes", "fl_bwd_workspace_bytes", "fl_attn_bwd_split_bytes", "fl_attn_rows_plan",
-          "fl_attn_shared_bias_bwd_bytes", "fl_attn_shared_bias_bwd", "fl_last_error")
 
 
 def _operands(*shape, dtype=torch.bfloat16, seed=0):
@@ -21,7 +19,7 @@ def test_other_threads_run_while_a_call_is_launched():
     """The library's entries replaced by CPython's own question whether this thread holds the interpreter: it returns 1,
     which the host path reads as a refusal, or 0, a launch."""
     lib = _ffi.load_library()
-    address = {f: C.cast(getattr(lib, f), C.c_void_p).value for f in _BOUND}
+    address = {f: C.cast(getattr(lib, f), C.c_void_p).value for f in _ffi._HOST_ENTRIES}
     asked = C.cast(C.pythonapi.PyGILState_Check, C.c_void_p).value
     q, k, v = _operands(1, 2, 64, 64)
     pair = torch.zeros(1, 2, 64, 64, dtype=torch.bfloat16, device=DEV)

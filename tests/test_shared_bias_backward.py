@@ -40,6 +40,10 @@ def test_which_calls_the_shared_bias_backward_takes():
     p.bias[1], p.bias_batch_div[1] = 0x70000, 1
     p.bias_strides[1][:] = (256, 0, 0, 1)
     assert takes(p)
+    # a result before the gate goes with a gate, and is named as such in the backward alone
+    assert lib.fl_attn_fwd_ungated(C.byref(params()), C.c_void_p(0x90000), None) == -5
+    assert lib.fl_attn_fwd_ungated(C.byref(params(gate=0x80000)), C.c_void_p(0x90008), None) == -7
+    assert lib.fl_attn_validate(C.byref(params(flags=_ffi.FLAG_UNGATED))) == -5
 
 
 CASES = [  # B, N, S, H, D
@@ -100,6 +104,28 @@ def test_one_bias_for_the_whole_batch(shape, bias_dtype):
         for name, a, b in zip(("dq", "dk", "dv", "dbias"), grads, want):
             assert a.shape == b.shape
             assert ((a.float().cpu() - b).norm() / b.norm()).item() < 1e-2, (shape, name)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 6, 64, 2, 32), (1, 4, 129, 2, 64)])  # B, N, S, H, D
+def test_nearly_closed_gates(shape):
+    """fp16, gate logits around -12 under a loss scale: the gated result is mostly below the normal numbers, the gradients
+    are not and keep the type's precision.  (Each is a product of a few factors rounded to 11 bits, rms error 2^-11 / sqrt 3
+    = 2.8e-4 each; formed from the gated result the gate's gradient is off by 1e-2, dq by 2e-3.)"""
+    B, N, S, H, D = shape
+    g = torch.Generator().manual_seed(sum(shape))
+    q, k, v, dout, gate = (torch.randn(B, N, S, H, D, generator=g) for _ in range(5))
+    pair = torch.randn(B, 1, H, S, S, generator=g).half()
+    leaves = [q.half(), k.half(), v.half(), pair, (gate - 12.0).half()]
+    dout = (1024.0 * dout).half()
+    dev = [t.to(DEV).requires_grad_(True) for t in leaves]
+    out = A.attention_reference(*dev[:3], [dev[3]], gate=dev[4])
+    ref = [t.double().requires_grad_(True) for t in leaves]
+    want = O.attention_evoformer(*ref[:3], [ref[3]], gate=ref[4])
+    assert ((out.double().cpu() - want).abs() <= 2.0 ** -24 + 2.0 ** -10 * want.abs()).all()  # half a subnormal step, two roundings
+    for name, a, b in zip(("dq", "dk", "dv", "dbias", "dgate"), torch.autograd.grad(out, dev, dout.to(DEV)),
+                          torch.autograd.grad(want, ref, dout.double())):
+        assert ((a.double().cpu() - b).norm() / b.norm()).item() < 1e-3, (shape, name)
 
 
 @pytest.mark.gpu
