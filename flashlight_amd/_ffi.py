@@ -234,7 +234,7 @@ class DocWorkspace:
         self.ids = None
 
 
-FLAG_DOC_PREPARED, FLAG_UNGATED = 1, 2  # fl_attn_params.flags
+FLAG_DOC_PREPARED, FLAG_UNGATED, FLAG_SCRATCH = 1, 2, 8  # fl_attn_params.flags
 SCORE_NONE, SCORE_SIGMOID, SCORE_CLAMP, SCORE_POLY = 0, 1, 2, 3  # fl_attn_params.score_fn
 
 
@@ -433,6 +433,7 @@ def attn_fwd(
         if lib.fl_attn_rows_plan(C.byref(p), C.byref(scratch)) and scratch.value:
             ws = torch.empty(scratch.value, dtype=torch.uint8, device=q.device)
             p.workspace, p.workspace_bytes = ws.data_ptr(), scratch.value
+            p.flags |= FLAG_SCRATCH
             keep.append(ws)
     _launch_on(q.device, lib.fl_attn_fwd, p)
     # tensors in `keep` were last used on the current stream; the caching allocator orders their reuse after it

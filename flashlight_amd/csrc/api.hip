@@ -392,7 +392,7 @@ int check_ptr(const char* what, const void* ptr, int align) {
   return 0;
 }
 
-int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = false, uint32_t flags = FL_FLAG_DOC_PREPARED) {
+int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = false, uint32_t flags = FL_FLAG_DOC_PREPARED | FL_FLAG_SCRATCH) {
   if (!p) return fail(FL_ERR_NULL, "params is null");
   int rc;
   if ((rc = check_ptr("q", p->q, 16)) || (rc = check_ptr("k", p->k, 16)) || (rc = check_ptr("v", p->v, 16)) ||
@@ -606,8 +606,8 @@ bool plan_pairbias(const fl_attn_params* p, fl::PParams* out, int* grid) {
 }
 
 // Whether *p (already validated) is a call the few-rows forward (rows_kernel.h) takes.  Fills the kernel's parameters and
-// launch shape.  `scratch`: bytes of p->workspace it would use to cut the keys into chunks; with less the keys of a row
-// tile stay in one workgroup.
+// launch shape.  `scratch`: bytes of p->workspace it would use to cut the keys into chunks; with less, or without the caller's
+// word that the workspace is scratch, the keys of a row tile stay in one workgroup.
 bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves, int* blocks, uint64_t* scratch) {
   if (p->Dqk != p->Dv || !fl::rows_has_shape(p->Dqk) || is_doc(p->mask_kind) || p->diff || p->gate || p->attended_dump ||
       p->dropout_threshold || p->score_fn != FL_SCORE_NONE)
@@ -665,7 +665,7 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   if (chunks > 1) {
     const uint64_t n = (uint64_t)base * chunks * 16 * qt;
     *scratch = n * (p->Dv + 2) * sizeof(float);
-    if (!p->workspace || p->workspace_bytes < *scratch || reinterpret_cast<uintptr_t>(p->workspace) % 16) {
+    if (!(p->flags & FL_FLAG_SCRATCH) || !p->workspace || p->workspace_bytes < *scratch || reinterpret_cast<uintptr_t>(p->workspace) % 16) {
       chunks = 1;
     } else {
       k.part = static_cast<float*>(p->workspace);
@@ -1214,7 +1214,7 @@ uint64_t fl_attn_shared_bias_bwd_bytes(const fl_attn_params* p) {
 int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* stream_) {
   if (!b) return fail(FL_ERR_NULL, "params is null");
   const fl_attn_params* p = &b->fwd;
-  int rc = validate(p, nullptr, false, FL_FLAG_DOC_PREPARED | FL_FLAG_UNGATED);
+  int rc = validate(p, nullptr, false, FL_FLAG_UNGATED);
   if (rc) return rc;
   SBScratch x;
   if (!plan_shared_bias_bwd(p, &x)) return fail(FL_ERR_UNSUPPORTED, "fl_attn_shared_bias_bwd does not take this call");

@@ -183,6 +183,7 @@ Tensor launch_forward(const Call& c, Tensor* lse, Tensor* ungated = nullptr) {
     ws = at::empty({(int64_t)bytes}, opt.dtype(at::kByte));
     p.workspace = ws.data_ptr();
     p.workspace_bytes = bytes;
+    if (!c.doc.defined()) p.flags = FL_FLAG_SCRATCH;
   }
   return g_api.fwd(&p, current_stream()) == 0 ? out : Tensor();
 }

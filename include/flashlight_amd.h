@@ -101,8 +101,8 @@ typedef struct fl_attn_params {
                   * monkeypatch/fusion/_reduction.py:55-57) */
 
   /* Scratch of document-mask calls (the forward's lists of key tiles per query tile, the backward's table of id
-   * ranges); size from fl_workspace_bytes(), 16-byte aligned.  Optional scratch of calls with few query rows, see
-   * fl_attn_rows_plan().  May be NULL otherwise. */
+   * ranges); size from fl_workspace_bytes(), 16-byte aligned.  With FL_FLAG_SCRATCH, optional scratch of calls with few
+   * query rows, see fl_attn_rows_plan().  Neither read nor written otherwise, and may be NULL. */
   void* workspace;
   uint64_t workspace_bytes;
 
@@ -158,6 +158,11 @@ typedef struct fl_attn_params {
 /* fl_attn_shared_bias_bwd, with a gate: fwd.o is the result before the gate (fl_attn_fwd_ungated). */
 #define FL_FLAG_UNGATED 2u
 
+/* fl_attn_fwd: `workspace` holds nothing the caller wants kept, and a call that has a use for scratch may write to it
+ * (fl_attn_rows_plan).  Without it only document-mask calls touch the workspace: a host that keeps one parameter struct
+ * for calls with and without a document mask keeps its prepared lists. */
+#define FL_FLAG_SCRATCH 8u
+
 /* ABI version of the loaded library (FL_ABI_VERSION it was built with). */
 int fl_version(void);
 
@@ -180,9 +185,9 @@ uint64_t fl_workspace_bytes(const fl_attn_params* p);
 uint64_t fl_bwd_workspace_bytes(const fl_attn_params* p);
 
 /* Whether fl_attn_fwd runs *p in the kernel for few query rows per key / value head (decoding steps, short prefills):
- * 1 or 0.  *scratch_bytes receives what `workspace` may hold then (16-byte aligned, contents undefined before and after)
- * for the keys to be cut into chunks that run in different workgroups, 0 when that is not wanted; without it the call
- * is correct and slower.  Host only. */
+ * 1 or 0.  *scratch_bytes receives what `workspace` may hold then (16-byte aligned, contents undefined before and after,
+ * with FL_FLAG_SCRATCH in flags) for the keys to be cut into chunks that run in different workgroups, 0 when that is not
+ * wanted; without it the call is correct and slower.  Host only. */
 int fl_attn_rows_plan(const fl_attn_params* p, uint64_t* scratch_bytes);
 
 /* Runs the fused forward on hipStream_t `stream` (NULL = default stream).

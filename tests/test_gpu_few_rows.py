@@ -92,3 +92,23 @@ def test_rows_without_keys_and_extreme_logits():
     k[:, :, 1500:] *= 60.0   # the maximum jumps by hundreds of nats half way through the keys
     want = torch.nn.functional.scaled_dot_product_attention(q.float().cpu(), k.float().cpu(), v.float().cpu(), enable_gqa=True)
     assert_parity(ops.dispatch(q, k, v), want, "jump")
+
+
+@pytest.mark.gpu
+def test_the_workspace_is_scratch_only_when_the_caller_says_so():
+    """A parameter struct with a workspace that holds something (a document call's prepared lists), used for a decoding
+    step that would cut its keys into chunks: the workspace keeps its bytes unless FL_FLAG_SCRATCH gives it away."""
+    g = torch.Generator().manual_seed(6)
+    q = torch.randn(1, 8, 1, 64, generator=g).to(torch.bfloat16).cuda()
+    k, v = (torch.randn(1, 2, 9000, 64, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+    want = torch.nn.functional.scaled_dot_product_attention(q.float().cpu(), k.float().cpu(), v.float().cpu(), enable_gqa=True)
+    lib, out, n = _ffi.load_library(), torch.empty_like(q), C.c_uint64()
+    p, _ = _ffi._fill_params(lib, q, k, v, out, 8, 2, None, 0, 0, 0, None, 0, 0.0, (), None, False, 0.0, None)
+    assert lib.fl_attn_rows_plan(C.byref(p), C.byref(n)) and n.value
+    ws = torch.full((n.value,), 0x5A, dtype=torch.uint8, device=DEV)
+    p.workspace, p.workspace_bytes = ws.data_ptr(), n.value
+    for flags in (0, _ffi.FLAG_SCRATCH):
+        p.flags = flags
+        _ffi._launch_on(q.device, lib.fl_attn_fwd, p)
+        assert_parity(out, want, f"flags {flags}")
+        assert bool((ws == 0x5A).all()) == (not flags)
