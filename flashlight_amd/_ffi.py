@@ -234,7 +234,8 @@ class DocWorkspace:
         self.ids = None
 
 
-FLAG_DOC_PREPARED, FLAG_UNGATED, FLAG_SCRATCH = 1, 2, 8  # fl_attn_params.flags
+FLAG_DOC_PREPARED, FLAG_UNGATED, FLAG_SCRATCH, FLAG_F32_RESULT = 1, 2, 8, 16  # fl_attn_params.flags
+PARTS_F32 = 256  # fl_attn_merge_chunks
 SCORE_NONE, SCORE_SIGMOID, SCORE_CLAMP, SCORE_POLY = 0, 1, 2, 3  # fl_attn_params.score_fn
 
 
@@ -362,6 +363,7 @@ def attn_fwd(
     `biases` holds up to two (tensor, batch_div) pairs; each tensor is 4-D, bf16 or fp32, broadcastable to
     [B/batch_div, Hq, Lq, Lk] (size-1 axes broadcast).  q, k, v (and gate, 16-bit biases) are all bf16 or all fp16.  Returns `out` [B, Hq, Lq, Dv]
     in that type, written on the current stream.
+    `out` may be float32: a result over a part of the keys, to be merged (`merge_chunks`); no gate, no diff.
     `lse` (float32 [B, Hq, Lq]) receives the row statistics that `attn_bwd` needs.
     `dropout_p` > 0 drops softmax weights (torch.nn.functional.dropout semantics) by a hash of (`dropout_seed`, batch,
     head, query, key); positional masks and GQA only.
@@ -391,7 +393,7 @@ def attn_fwd(
         raise ValueError(f"value has {Hv} heads, expected {Hkv}")
     if out is None:
         out = torch.empty((B, Hq, Lq, Dv), dtype=q.dtype, device=q.device)
-    elif tuple(out.shape) != (B, Hq, Lq, Dv) or out.dtype != q.dtype or out.device != q.device:
+    elif tuple(out.shape) != (B, Hq, Lq, Dv) or out.dtype not in (q.dtype, torch.float32) or out.device != q.device:
         raise ValueError("out has the wrong shape, dtype or device")
     if Dv > _MAX_DV_DIFF and Dv % _MAX_DV_DIFF == 0 and attended_dump is None and (diff or Dqk >= 128):
         # Value columns are independent of one another, so wide values go in slabs of _MAX_DV_DIFF columns, one launch
@@ -415,6 +417,8 @@ def attn_fwd(
     p, keep = _fill_params(lib, q, k, v, out, Hq, Hkv, scale, mask_kind, window, prefix, doc_ids, alibi_heads, softcap,
                            biases, gate, diff, lambda_full, attended_dump, dropout_p, dropout_seed,
                            doc_workspace=doc_workspace)
+    if out.dtype == torch.float32:
+        p.flags |= FLAG_F32_RESULT
     if score_fn is not None:
         kind, consts = score_fn
         if len(consts) != 4:
@@ -624,16 +628,20 @@ def probe_coissue(mfma_rows: int, valu_kind: str, valu_per_mfma: int, waves_per_
     return {"slowest_wave": float(c.max()) / per, "mean_wave": float(c.mean()) / per}
 
 
-def merge_chunks(part: torch.Tensor, lse: torch.Tensor) -> torch.Tensor:
-    """`fl_attn_merge_chunks`: part [outer, chunks, inner, dv] (bf16 / fp16) and lse [outer, chunks, inner] (fp32) of one
-    launch over key chunks -> [outer, inner, dv], the attention over all the keys.  One launch on the current stream."""
-    _require_gpu_half("part", part, None)
+def merge_chunks(part: torch.Tensor, lse: torch.Tensor, dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+    """`fl_attn_merge_chunks`: part [outer, chunks, inner, dv] (bf16 / fp16, or fp32 for a result of `dtype`) and lse
+    [outer, chunks, inner] (fp32) of one launch over key chunks -> [outer, inner, dv], the attention over all the keys.
+    One launch on the current stream."""
+    f32 = dtype in _HALF_TYPES and isinstance(part, torch.Tensor) and part.is_cuda and part.dtype == torch.float32
+    if not f32:
+        _require_gpu_half("part", part, None)
+        dtype = part.dtype
     outer, chunks, inner, dv = part.shape
     if lse.dtype != torch.float32 or tuple(lse.shape) != (outer, chunks, inner) or not (part.is_contiguous() and lse.is_contiguous()):
         raise ValueError("merge_chunks: lse must be float32 [outer, chunks, inner], both operands contiguous")
-    out = torch.empty((outer, inner, dv), dtype=part.dtype, device=part.device)
+    out = torch.empty((outer, inner, dv), dtype=dtype, device=part.device)
     rc = load_library().fl_attn_merge_chunks(C.c_void_p(part.data_ptr()), C.c_void_p(lse.data_ptr()), C.c_void_p(out.data_ptr()),
-                                             outer, chunks, inner, dv, _HALF_TYPES[part.dtype],
+                                             outer, chunks, inner, dv, _HALF_TYPES[dtype] + (PARTS_F32 if f32 else 0),
                                              C.c_void_p(torch.cuda.current_stream().cuda_stream))
     if rc != 0:
         raise FlashlightError(rc, "fl_attn_merge_chunks rejected its arguments or could not launch")

@@ -392,7 +392,7 @@ int check_ptr(const char* what, const void* ptr, int align) {
   return 0;
 }
 
-int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = false, uint32_t flags = FL_FLAG_DOC_PREPARED | FL_FLAG_SCRATCH) {
+int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = false, uint32_t flags = FL_FLAG_DOC_PREPARED | FL_FLAG_SCRATCH | FL_FLAG_F32_RESULT) {
   if (!p) return fail(FL_ERR_NULL, "params is null");
   int rc;
   if ((rc = check_ptr("q", p->q, 16)) || (rc = check_ptr("k", p->k, 16)) || (rc = check_ptr("v", p->v, 16)) ||
@@ -411,6 +411,10 @@ int validate(const fl_attn_params* p, const fl::Instance** out, bool for_bwd = f
       (rc = check_strides("v", p->v_strides, 8)) || (rc = check_strides("o", p->o_strides, 4)))
     return rc;
   if (p->flags & ~flags) return fail(FL_ERR_ARG, "unknown bits in flags: 0x%x", p->flags);
+  if (p->flags & FL_FLAG_F32_RESULT) {
+    if (for_bwd || p->gate || p->diff) return fail(FL_ERR_UNSUPPORTED, "a result in fp32 goes with forward calls without gate and differential attention");
+    if (reinterpret_cast<uintptr_t>(p->o) % 16) return fail(FL_ERR_ALIGN, "o pointer must be 16-byte aligned");
+  }
   if ((p->flags & FL_FLAG_DOC_PREPARED) && !is_doc(p->mask_kind))
     return fail(FL_ERR_ARG, "FL_FLAG_DOC_PREPARED goes with a document mask only");
   if (p->dropout_threshold) {
@@ -518,7 +522,7 @@ bool plan_pairbias(const fl_attn_params* p, fl::PParams* out, int* grid) {
   static const bool disabled = std::getenv("FL_NO_PAIRBIAS") != nullptr;  // A/B knob: the general kernel instead
   if (disabled) return false;
   if (p->Dqk != p->Dv || p->mask_kind != FL_MASK_NONE || p->alibi_heads > 0 || p->softcap > 0.f ||
-      p->diff || p->attended_dump || p->dropout_threshold || p->lse || p->score_fn != FL_SCORE_NONE)
+      p->diff || p->attended_dump || p->dropout_threshold || p->lse || p->score_fn != FL_SCORE_NONE || (p->flags & FL_FLAG_F32_RESULT))
     return false;
   // one operand that several consecutive batch entries share (dense over heads, queries and keys), and optionally one
   // that is a row of keys per batch entry, the same for every head and query; in either order
@@ -626,7 +630,9 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   // Longer row counts re-read K and V for every 16 rows (32 at head dim 64), from L2: that pays while one workgroup per
   // compute unit holds all of them, where the tile kernel leaves most of the part idle (head dim 64, 8 heads of 1024
   // causal rows: 16.8 -> 12.2 us; head dim 128, 4 heads: 21.5 -> 14.5 us), and loses beyond (twice as many rows: 17 -> 18
-  // and 23 -> 30 us).  Up to 64 keys the tile kernel has a single step.
+  // and 23 -> 30 us).  Up to 64 keys the tile kernel has a single step.  Against a long cache the front end has the tile
+  // kernel over chunks of the keys besides, and takes it where that is sooner (chunks_beat_rows_kernel in host.cpp); a
+  // single launch of the tile kernel is the slower one at any length (8 heads, 40 queries of 5000 keys: 81 us, here 17).
   int qt = 1;
   if (rows <= 32) {
     if (p->Lk <= 128 && (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128) <= 256) return false;
@@ -641,15 +647,16 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   // Waves per workgroup and chunks of the keys.  Eight waves fill a compute unit's registers, so 256 workgroups of eight
   // or 512 of four are one round.  Enough row tiles: no chunks, and shorter workgroups the more of them there are.  Few:
   // a chunk has two key tiles per wave at least, and the merge launch behind the chunks costs 4.5 us, about what reading 512
-  // keys in one workgroup costs: up to there they stay together.  Eight waves add up inside the workgroup what four would
-  // send through memory: worth it once a wave has two tiles.
+  // keys in one workgroup costs (1024 where more than two row tiles read them): up to there they stay together.  Eight waves
+  // add up inside the workgroup what four would send through memory: worth it once a wave has two tiles.  (8 heads, head dim
+  // 128, rows of one workgroup each -> chunks: 128 queries of 2048 keys 23.6 -> 14.8 us, 48 of 3000 keys 31.6 -> 15.3.)
   int nw = 8;
   int64_t chunks = 1;
   if (base >= 1024) {
     nw = tiles < 16 ? 2 : 4;
   } else if (base >= 512) {
     nw = 4;
-  } else if (rows > 32) {
+  } else if (rows > 32 && (p->mask_kind != FL_MASK_NONE || tiles <= 32)) {
     nw = tiles > 8 ? 8 : 4;
   } else if (base < 256 && tiles > 16 && p->mask_kind == FL_MASK_NONE) {
     if (tiles * base >= 16 * 256) {
@@ -658,6 +665,10 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
       nw = 4;
       chunks = std::max<int64_t>(1, std::min<int64_t>(512 / base, tiles / 8));
     }
+    // the row tiles of one (unit, chunk) stay on one XCD (by_xcd below): no XCD gets more of them than it runs at once (2 heads,
+    // 48 queries, 32768 keys: 42 chunks 28.9 us, 40 chunks 18.8)
+    if (row_tiles > 2 && units * chunks >= 8)
+      chunks = std::max<int64_t>(1, std::min<int64_t>(chunks, 8 * ((nw == 8 ? 32 : 64) / row_tiles) / units));
   }
   fl::RParams k;
   std::memset(&k, 0, sizeof(k));
@@ -708,6 +719,7 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
     k.bias_div[i] = p->bias[i] ? p->bias_batch_div[i] : 1;
     k.bias_f32[i] = p->bias_dtype[i] == FL_F32;
   }
+  k.o_f32 = (p->flags & FL_FLAG_F32_RESULT) != 0;
   k.by_xcd = units * chunks >= 8 && row_tiles > 1;
   *grid = (int)(k.by_xcd ? (units * chunks + 7) / 8 * 8 * row_tiles : units * chunks * row_tiles);
   *waves = nw;
@@ -942,6 +954,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   }
   kp.gate = static_cast<const fl::bf16_t*>(p->gate);
   kp.ungated = static_cast<fl::bf16_t*>(ungated);
+  kp.o_f32 = (p->flags & FL_FLAG_F32_RESULT) != 0;
   kp.lambda = p->lambda;
   if (p->diff) {
     // heads [0, H) are branch 0, heads [H, 2H) branch 1 (query: H = Hq, key: H = Hkv)

@@ -100,6 +100,7 @@ struct KParams {
   int32_t n_qtiles;  // ceil(Lq / BM)
   int32_t n_ktiles;  // ceil(Lk / BN)
   bf16_t* ungated;   // with a gate, optional: the result before the gate as well, addressed like o (for the gradients)
+  int32_t o_f32;     // o holds fp32 elements (partial results over a part of the keys; no gate, not with diff)
 };
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -1423,6 +1424,22 @@ void fwd_kernel(const KParams p) {
   }
 
   // ---- epilogue: O^T register i of block (dvb, qb) is out[q = qrow[qb]][dv = 32*dvb + 8*(i/4) + 4h + i%4] ----------
+  if constexpr (!kDiff) {
+    if (p.o_f32) {
+      float* fptr = reinterpret_cast<float*>(p.o) + (int64_t)batch * p.os[0] + (int64_t)head * p.os[1];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        if (qrow[qb] >= p.Lq) continue;
+#pragma unroll
+        for (int dvb = 0; dvb < DVB; ++dvb)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(fptr + (int64_t)qrow[qb] * p.os[2] + 32 * dvb + 8 * g + 4 * h) =
+                f32x4{oacc[dvb][qb][4 * g], oacc[dvb][qb][4 * g + 1], oacc[dvb][qb][4 * g + 2], oacc[dvb][qb][4 * g + 3]};
+      }
+      return;
+    }
+  }
   bf16_t* optr = p.o + (int64_t)batch * p.os[0] + (int64_t)head * p.os[1];
   const bf16_t* gptr = (kGate && p.gate) ? p.gate + (int64_t)batch * p.gs[0] + (int64_t)head * p.gs[1] : nullptr;
   bf16_t* uptr = (kGate && p.ungated) ? p.ungated + (int64_t)batch * p.os[0] + (int64_t)head * p.os[1] : nullptr;

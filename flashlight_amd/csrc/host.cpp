@@ -19,6 +19,7 @@
 #include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "flashlight_amd.h"
@@ -135,6 +136,42 @@ void fill(const Call& c, fl_attn_params& p) {
 
 void* current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
+// Into how many chunks the front end cuts the keys of an unmasked call whose rows are independent (ops._split_over_keys: the
+// chunks run as heads or batch entries of one launch of the tile kernel, with results in fp32, and a second launch merges
+// them); 0: it does not.  `groups` counts the tile kernel's workgroups without chunks.
+int64_t key_chunks(const fl_attn_params& p, const Tensor& k, const Tensor& v, int64_t groups) {
+  if (groups >= 256 || p.Lk < 4096) return 0;
+  // one batch entry with dense rows: chunks of a multiple of 8 keys as batch entries, the rest is one more; otherwise the
+  // caches have to be one block, and the chunks divide them into heads
+  const bool one = p.B == 1 && p.k_strides[2] == p.Dqk && p.v_strides[2] == p.Dv;
+  if (!one && !(k.is_contiguous() && v.is_contiguous())) return 0;
+  // One round of workgroups, two per compute unit; where half as many chunks would leave an eighth of that idle, up to two
+  // rounds.  (More only make partial results: 8 heads, 256 queries, 65536 keys, head dim 128: 107 us with 2048 workgroups,
+  // 106 with 1024, 87 with 512; 128 heads' tiles of 8192 keys 125, 96, 89; 192 of 16384 keys 238, 227, 240.)
+  for (int64_t c = 64; c > 1; c /= 2)
+    if ((groups * c <= 512 || (groups * c <= 1024 && groups * c / 2 < 448)) &&
+        (one ? p.Lk / c / 8 * 8 >= 512 : p.Lk % (8 * c) == 0 && p.Lk / c >= 512))
+      return c;
+  return 0;
+}
+
+// Whether those chunks are the better way where the few-rows kernel would take the call (fl_attn_rows_plan).  It reads K and V
+// for every 16 rows, from L2: 256 workgroups together 150 keys per microsecond each at head dim 64, 100 at 128, and 8 us for a
+// start and a merge where they work on chunks.  The tile kernel reads them once for 128 rows: 64 and 50 keys per microsecond in
+// a workgroup of its own compute unit, 28 and 25 with two on each, and 9 us.  Estimates in microseconds, from 50 shapes of 33 to
+// 4096 rows over 4096 to 131072 keys; with up to 32 rows the keys are read once there, too.
+// (few-rows kernel without chunks -> this rule: 32 heads over 8, 16 queries, 32768 keys, head dim 128: 284 -> 38 us; 8 heads, 64
+// queries, 65536 keys: 563 -> 57; 2 heads, 48 queries, 32768 keys: 285 -> 19; 8 heads, 128 queries, 4096 keys, 64: 26 -> 15.)
+bool chunks_beat_rows_kernel(const fl_attn_params& p, int64_t groups, int64_t chunks) {
+  const int64_t units = (int64_t)p.B * p.Hkv, rows = (int64_t)(p.Hq / p.Hkv) * p.Lq;
+  if (rows <= 32) return false;
+  const int64_t base = std::min<int64_t>(256, units * ((rows + 15) / 16)), own = 256 / base;
+  const bool narrow = p.Dqk <= 64;
+  const double by_rows = (double)p.Lk / own / (narrow ? 150 : 100) + (own > 1 ? 8 : 0);
+  const double by_chunks = 9 + std::max((double)p.Lk / chunks / (narrow ? 64 : 50), (double)groups * p.Lk / 512 / (narrow ? 28 : 25));
+  return by_chunks < by_rows;
+}
+
 // Launches the forward of `c` into a fresh tensor; an undefined tensor if the C ABI refuses (the Python path then says why).
 // `lse`: when given, receives the row statistics; `ungated` the result before the gate.
 Tensor launch_forward(const Call& c, Tensor* lse, Tensor* ungated = nullptr) {
@@ -159,7 +196,8 @@ Tensor launch_forward(const Call& c, Tensor* lse, Tensor* ungated = nullptr) {
   Tensor ws;
   if (c.doc.defined()) {
     bytes = g_api.workspace(&p);
-  } else if (!g_api.rows_plan(&p, &bytes)) {
+  } else {
+    const bool rows_kernel = g_api.rows_plan(&p, &bytes);
     const bool rows_independent = c.mask_kind == FL_MASK_NONE && !p.gate && !p.diff && !p.alibi_heads && !lse && !c.seq_major &&
                                   (!p.bias[0] || (p.bias_strides[0][1] == 0 && p.bias_strides[0][2] == 0)) &&
                                   (!p.bias[1] || (p.bias_strides[1][1] == 0 && p.bias_strides[1][2] == 0));
@@ -167,16 +205,20 @@ Tensor launch_forward(const Call& c, Tensor* lse, Tensor* ungated = nullptr) {
       // (without a mask the G query heads of a key / value head may as well be G times as many rows of one head: one
       // workgroup then reads the keys for all of them)
       const int64_t group = p.Hq / p.Hkv;
-      int64_t tiles = (int64_t)p.B * p.Hq * ((p.Lq + 127) / 128);
-      if (group > 1 && group * p.Lq <= 128 && q.is_contiguous()) {
+      const bool pack = group > 1 && group * p.Lq <= 128 && q.is_contiguous();
+      const int64_t groups = pack ? (int64_t)p.B * p.Hkv : (int64_t)p.B * p.Hq * ((p.Lq + 127) / 128);
+      // few workgroups against many keys: the Python path cuts the keys into chunks
+      const auto whole_row = [&](const Tensor& b) { return !b.defined() || (b.is_contiguous() && b.size(3) == p.Lk); };
+      if (whole_row(c.bias[0]) && whole_row(c.bias[1])) {
+        const int64_t chunks = key_chunks(p, c.k, c.v, groups);
+        if (chunks && (!rows_kernel || chunks_beat_rows_kernel(p, groups, chunks))) return Tensor();
+      }
+      if (pack && !rows_kernel) {
         p.Hq = p.Hkv;
         p.Lq = (int32_t)(group * p.Lq);
         p.q_strides[1] = p.Lq * q.stride(2);
         p.o_strides[1] = p.Lq * out.stride(2);
-        tiles = (int64_t)p.B * p.Hq;
       }
-      // few workgroups against many keys: the Python path cuts the keys into chunks
-      if (tiles < 256 && p.Lk >= 4096) return Tensor();
     }
   }
   if (bytes) {
@@ -499,6 +541,34 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// key_chunks(q, k, v): into how many chunks ops._split_over_keys cuts the keys (0: it does not, operands it cannot judge
+// included), and whether the front end should let it
+PyObject* py_key_chunks(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 3) {
+    PyErr_SetString(PyExc_TypeError, "key_chunks takes three tensors");
+    return nullptr;
+  }
+  Call c;
+  int64_t chunks = 0;
+  bool better = false;
+  if (g_api.fwd && THPVariable_Check(a[0]) && THPVariable_Check(a[1]) && THPVariable_Check(a[2])) {
+    const Tensor &q = c.q = THPVariable_Unpack(a[0]), &k = c.k = THPVariable_Unpack(a[1]), &v = c.v = THPVariable_Unpack(a[2]);
+    if (element_type(q) >= 0 && q.dim() == 4 && k.dim() == 4 && v.dim() == 4 &&
+        q.numel() > 0 && k.numel() > 0 && v.numel() > 0 && k.size(0) == q.size(0) && v.size(0) == q.size(0) && k.size(3) == q.size(3) &&
+        v.size(1) == k.size(1) && v.size(2) == k.size(2) && q.size(1) % k.size(1) == 0 && k.stride(3) == 1 && v.stride(3) == 1) {
+      fl_attn_params p = {};
+      uint64_t bytes;
+      fill(c, p);
+      const int64_t groups = (int64_t)p.B * p.Hq * ((p.Lq + 127) / 128);
+      chunks = key_chunks(p, k, v, groups);
+      better = chunks && (!g_api.rows_plan(&p, &bytes) || chunks_beat_rows_kernel(p, groups, chunks));
+    }
+  }
+  return Py_BuildValue("LN", (long long)chunks, PyBool_FromLong(better));
+  END_HANDLE_TH_ERRORS
+}
+
 // bind(addresses): the C ABI's functions in the order of Api, as integers
 PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* f[kApiFunctions];
@@ -523,6 +593,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 PyMethodDef kMethods[] = {
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_forward)), METH_FASTCALL, "Result of the call, or None when it is not of the plain kind."},
+    {"key_chunks", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_key_chunks)), METH_FASTCALL, "Chunks the keys may be cut into, and whether they should be."},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_bind)), METH_FASTCALL, "Takes the addresses of the C ABI's functions."},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", "Native host path of the attention front ends.", -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -274,31 +274,26 @@ def _pad_head_dims(q, k, v, gate, diff, bias_only=True, min_dim=32):
 def _split_over_keys(q, k, v, scale, softcap, biases=()):
     """Few queries against many keys (a decoding step over a long cache): B * Hq workgroups cannot fill 256 CUs, so the
     keys are cut into C chunks that run as C times as many heads of one launch, each leaving a normalised partial result
-    and its row statistic, and a second small launch merges the partial results with the weights 2^(lse_c - max).  Returns None when the
-    call is not of that shape (enough workgroups already, short or indivisible key length, key / value tensors whose
-    heads are not contiguous in memory when there is more than one batch entry), and the caller launches as usual."""
+    (fp32) and its row statistic, and a second small launch merges the partial results with the weights 2^(lse_c - max).
+    Returns None when the call is not of that shape (enough workgroups already, short or indivisible key length, key /
+    value tensors whose heads are not contiguous in memory when there is more than one batch entry), and the caller
+    launches as usual."""
+    _ffi.load_library()
+    chunks, _ = _ffi._host.key_chunks(q, k, v)   # (one rule for this path and the native one, csrc/host.cpp)
+    if not chunks:
+        return None
     B, Hq, Lq, D = q.shape
     Hkv, Lk, Dv = k.size(1), k.size(2), v.size(3)
-    groups = B * Hq * ((Lq + 127) // 128)
-    # (a workgroup walks about 64 keys per microsecond; the copy of q, the row statistics and the merge launch cost
-    # about 20: worth it from 4096 keys on)
-    if groups >= 256 or Lk < 4096 or Hq % Hkv:
-        return None
-    whole = k.is_contiguous() and v.is_contiguous()
-    # a cache that is a slice of a longer buffer (dense rows, heads further apart): with one batch entry the chunks can
-    # be the batch entries of the launch instead of heads
-    rows_dense = B == 1 and k.stride(3) == 1 and v.stride(3) == 1 and k.stride(2) == D and v.stride(2) == Dv
-    if not (whole or rows_dense):
-        return None
     if scale is None:
         scale = 1.0 / math.sqrt(D)
-    if rows_dense:
-        # one batch entry (also when the cache is one block): the chunks are the batch entries of the launch, which reads
-        # the queries with batch stride 0 (no copy).  Chunks of a multiple of 8 keys; what is left over at the end of a key
-        # length that does not divide is one more, shorter chunk from a launch of its own
-        chunks = next((c for c in (64, 32, 16, 8, 4, 2) if (Lk // c) // 8 * 8 >= 512 and groups * c <= 2048), 0)
-        if not chunks:
-            return None
+    # (partial results in 16 bits add their rounding to the result's: rms error of 4096 to 131072 keys 2.9e-3 instead of 2.3e-3
+    # in bf16; fp32 costs 5 % at head dim 256, whose values go in two launches, and is left out there)
+    part_type = torch.float32 if Dv <= 128 else q.dtype
+    if B == 1 and k.stride(2) == D and v.stride(2) == Dv:
+        # one batch entry (a cache that is one block, or a slice of a longer buffer: dense rows, heads further apart): the
+        # chunks are the batch entries of the launch, which reads the queries with batch stride 0 (no copy).  Chunks of a
+        # multiple of 8 keys; what is left over at the end of a key length that does not divide is one more, shorter chunk
+        # from a launch of its own
         Lc = (Lk // chunks) // 8 * 8
         main = chunks * Lc
         kc = k.as_strided((chunks, Hkv, Lc, D), (Lc * D, k.stride(1), D, 1), k.storage_offset())
@@ -306,20 +301,13 @@ def _split_over_keys(q, k, v, scale, softcap, biases=()):
         bc = [(b[..., :main].reshape(chunks, 1, 1, Lc), 1) for b, _ in biases]   # ([1, 1, 1, Lk] rows: chunk c is entry c)
         total = chunks + (1 if main < Lk else 0)   # (both launches write into one pair of buffers)
         lse = torch.empty(total, Hq, Lq, dtype=torch.float32, device=q.device)
-        part = torch.empty(total, Hq, Lq, Dv, dtype=q.dtype, device=q.device)
+        part = torch.empty(total, Hq, Lq, Dv, dtype=part_type, device=q.device)
         _ffi.attn_fwd(q.expand(chunks, Hq, Lq, D), kc, vc, scale=scale, softcap=softcap, lse=lse[:chunks], biases=bc,
                       out=part[:chunks])
         if main < Lk:
             _ffi.attn_fwd(q, k[:, :, main:], v[:, :, main:], scale=scale, softcap=softcap, lse=lse[chunks:],
                           biases=[(b[..., main:], 1) for b, _ in biases], out=part[chunks:])
-        return _ffi.merge_chunks(part.view(1, total, Hq * Lq, Dv), lse.view(1, total, Hq * Lq)).view(1, Hq, Lq, Dv)
-    chunks = 0
-    for c in (64, 32, 16, 8, 4, 2):
-        if Lk % c == 0 and Lk // c >= 512 and (Lk // c) % 8 == 0 and groups * c <= 2048:
-            chunks = c
-            break
-    if not chunks:
-        return None
+        return _ffi.merge_chunks(part.view(1, total, Hq * Lq, Dv), lse.view(1, total, Hq * Lq), q.dtype).view(1, Hq, Lq, Dv)
     G, Lc = Hq // Hkv, Lk // chunks
     # chunk c of key / value head h becomes head h * C + c; its G query heads are copies of the G of head h
     qc = q.reshape(B, Hkv, 1, G, Lq, D).expand(B, Hkv, chunks, G, Lq, D).reshape(B, Hkv * chunks * G, Lq, D)
@@ -328,9 +316,10 @@ def _split_over_keys(q, k, v, scale, softcap, biases=()):
     bc = [(b.view(b.size(0), 1, chunks, 1, Lc).expand(b.size(0), Hkv, chunks, G, Lc).reshape(b.size(0), Hkv * chunks * G, 1, Lc), d)
           for b, d in biases]
     lse = torch.empty(B, Hkv * chunks * G, Lq, dtype=torch.float32, device=q.device)
-    part = _ffi.attn_fwd(qc, kc, vc, scale=scale, softcap=softcap, lse=lse, biases=bc)
+    part = torch.empty(B, Hkv * chunks * G, Lq, Dv, dtype=part_type, device=q.device)
+    _ffi.attn_fwd(qc, kc, vc, scale=scale, softcap=softcap, lse=lse, biases=bc, out=part)
     # one small launch: weights 2^(lse_c - max) over the chunks of a row; a chunk, or a row, without keys counts as zeros
-    merged = _ffi.merge_chunks(part.view(B * Hkv, chunks, G * Lq, Dv), lse.view(B * Hkv, chunks, G * Lq))
+    merged = _ffi.merge_chunks(part.view(B * Hkv, chunks, G * Lq, Dv), lse.view(B * Hkv, chunks, G * Lq), q.dtype)
     return merged.view(B, Hq, Lq, Dv)
 
 
@@ -424,9 +413,9 @@ def dispatch(q, k, v, *, scale=None, mask_kind=_ffi.MASK_NONE, window=0, prefix=
                         doc_ids, int(alibi_heads), float(softcap), bl[0][0], int(bl[0][1]), bl[1][0], int(bl[1][1]), gate,
                         bool(diff), float(lambda_full), bool(seq_major_out), fn_kind, fn_c[0], fn_c[1], fn_c[2], fn_c[3])
     if rows_independent:
-        split = _split_over_keys(q, k, v, scale, softcap, biases) if all(b.is_contiguous() for b, _ in biases) else None
-        if split is not None:
-            return split
+        _ffi.load_library()
+        if all(b.is_contiguous() and b.size(3) == k.size(2) for b, _ in biases) and _ffi._host.key_chunks(q, k, v)[1]:
+            return _split_over_keys(q, k, v, scale, softcap, biases)
     out = _alloc_out(q, v, diff, seq_major_out) if seq_major_out else None
     return _ffi.attn_fwd(q, k, v, scale=scale, mask_kind=mask_kind, window=window, prefix=prefix, doc_ids=doc_ids,
                          alibi_heads=alibi_heads, softcap=softcap, biases=biases, gate=gate, diff=diff,

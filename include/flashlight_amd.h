@@ -163,6 +163,10 @@ typedef struct fl_attn_params {
  * for calls with and without a document mask keeps its prepared lists. */
 #define FL_FLAG_SCRATCH 8u
 
+/* fl_attn_fwd: `o` holds fp32 elements (o_strides in those, multiples of 4; 16-byte aligned).  For results over a part of
+ * the keys that fl_attn_merge_chunks will put together.  Not with a gate or differential attention. */
+#define FL_FLAG_F32_RESULT 16u
+
 /* ABI version of the loaded library (FL_ABI_VERSION it was built with). */
 int fl_version(void);
 
@@ -321,10 +325,12 @@ int fl_ipa_pack(const fl_ipa_pack_params* p, void* stream);
 /* Merges partial results of one attention over `chunks` disjoint chunks of its keys (no counterpart in the reference,
  * whose kernel walks all keys of a row in one program, monkeypatch/fusion/reduction_kernel_fusion.py:1102; used by the
  * front end for decoding steps, where a few query rows meet a long key sequence and the chunks run as extra heads of
- * one fl_attn_fwd launch).  part [outer, chunks, inner, dv] (element type `dtype`, contiguous) holds the chunks' results
+ * one fl_attn_fwd launch).  part [outer, chunks, inner, dv] (element type `dtype`, or fp32 with FL_PARTS_F32 added to
+ * `dtype`; contiguous) holds the chunks' results
  * as fl_attn_fwd wrote them, lse [outer, chunks, inner] the row statistics of the same launch (fl_attn_params.lse: +inf
  * for a row that attends nothing in a chunk); out [outer, inner, dv] receives sum_c w_c part_c / sum_c w_c with
  * w_c = 2^(lse_c - max_c lse_c), zeros for a row that attends nothing at all.  dv even. */
+#define FL_PARTS_F32 256
 int fl_attn_merge_chunks(const void* part, const float* lse, void* out, int64_t outer, int32_t chunks, int64_t inner,
                          int32_t dv, int32_t dtype, void* stream);
 

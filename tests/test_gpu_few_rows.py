@@ -31,13 +31,39 @@ def test_which_calls_the_few_rows_kernel_takes():
     assert not _taken(1, 8, 8, 1, 128, 64)[0]                   # too short to matter
     assert _taken(2, 8, 8, 512, 512, 64, mask_kind=_ffi.MASK_CAUSAL) == (True, 0)
     assert not _taken(4, 16, 16, 4096, 4096, 128)[0]
+    # more than 32 rows against many keys: few workgroups without chunks
+    for shape in ((1, 32, 8, 9, 32768, 128), (1, 8, 8, 64, 65536, 128), (1, 8, 8, 128, 65536, 64), (2, 8, 2, 40, 5000, 128)):
+        assert _taken(*shape)[0] and _taken(*shape)[1] > 0, shape
+    assert _taken(1, 8, 8, 64, 1024, 64) == (True, 0) and _taken(1, 1, 1, 4096, 4096, 64, mask_kind=_ffi.MASK_CAUSAL) == (True, 0)
+
+
+def test_which_calls_the_front_end_cuts_into_chunks():
+    """The tile kernel over chunks of the keys, or the few-rows kernel: the estimate of host.cpp at shapes where the two
+    measured far apart, and the forms that cannot be cut."""
+    _ffi.load_library()
+
+    def chunks(B, Hq, Hkv, Lq, Lk, D, longer=0):
+        q, k = torch.empty(B, Hq, Lq, D, dtype=torch.bfloat16), torch.empty(B, Hkv, Lk + longer, D, dtype=torch.bfloat16)[:, :, :Lk]
+        return _ffi._host.key_chunks(q, k, k)
+
+    for shape, n in (((1, 8, 8, 64, 32768, 128), 64), ((1, 8, 8, 64, 65536, 128), 64), ((1, 8, 8, 512, 65536, 128), 16),
+                     ((1, 1, 1, 4096, 65536, 128), 16), ((4, 8, 8, 64, 8192, 64), 16), ((1, 24, 24, 1000, 16384, 128), 4),
+                     ((1, 16, 16, 200, 16384, 32), 16), ((1, 4, 4, 128, 16384, 256), 32)):
+        assert chunks(*shape) == (n, True), shape
+    for shape in ((1, 32, 8, 1, 32768, 128), (1, 8, 8, 64, 4096, 128), (1, 2, 2, 48, 32768, 128), (5, 16, 16, 40, 4096, 64)):
+        assert chunks(*shape)[0] > 1 and not chunks(*shape)[1], shape          # the few-rows kernel is the sooner one
+    assert chunks(1, 8, 8, 64, 4095, 128)[0] == 0 and chunks(2, 8, 8, 64, 8200, 128)[0] == 0     # short; no divisor
+    assert chunks(1, 8, 8, 64, 65536, 128, longer=8) == (64, True) and chunks(2, 8, 8, 64, 65536, 128, longer=8)[0] == 0
+    assert chunks(4, 16, 16, 4096, 4096, 128)[0] == 0
 
 
 CASES = [  # B, Hq, Hkv, Lq, Lk, D
     (1, 4, 4, 1, 129, 64), (2, 8, 2, 1, 257, 128), (1, 8, 1, 2, 545, 64), (1, 32, 2, 1, 600, 128), (1, 17, 1, 1, 4097, 64),
     (3, 8, 8, 1, 2047, 128), (33, 8, 8, 1, 1000, 64), (64, 16, 8, 1, 200, 128), (72, 16, 16, 1, 161, 64),
     (1, 2, 2, 65, 65, 64), (1, 3, 3, 100, 100, 128), (1, 4, 2, 255, 255, 64), (1, 8, 8, 511, 513, 64), (2, 6, 2, 300, 300, 64),
-    (1, 2, 1, 129, 1000, 128), (1, 16, 16, 257, 257, 64)]
+    (1, 2, 1, 129, 1000, 128), (1, 16, 16, 257, 257, 64),
+    (1, 8, 2, 24, 4500, 128), (2, 4, 2, 33, 4099, 128), (1, 3, 3, 70, 4200, 64), (1, 2, 2, 300, 4096, 64), (1, 16, 4, 16, 8200, 128),
+    (1, 1, 1, 520, 4111, 128), (2, 8, 8, 40, 1041, 64)]
 
 
 @pytest.mark.gpu
@@ -112,3 +138,19 @@ def test_the_workspace_is_scratch_only_when_the_caller_says_so():
         _ffi._launch_on(q.device, lib.fl_attn_fwd, p)
         assert_parity(out, want, f"flags {flags}")
         assert bool((ws == 0x5A).all()) == (not flags)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(2, 8, 2, 1, 600, 64), (1, 8, 8, 3, 9000, 128), (2, 4, 4, 300, 300, 128), (1, 4, 2, 700, 333, 64),
+                                   (3, 2, 2, 130, 77, 32), (1, 4, 4, 200, 500, 256)])
+def test_results_in_fp32_are_what_the_16_bit_results_round(shape):
+    """FL_FLAG_F32_RESULT, for partial results that are merged: the same numbers before their rounding, from either kernel."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    g = torch.Generator().manual_seed(sum(shape))
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(torch.bfloat16).cuda() for h, n in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    row = torch.randn(B, 1, 1, Lk, generator=g).cuda()
+    for kw in ({}, dict(softcap=5.0), dict(mask_kind=_ffi.MASK_CAUSAL), dict(biases=[(row, 1)])):
+        wide = torch.full((B, Hq, Lq, D), float("nan"), dtype=torch.float32, device=DEV)
+        assert torch.equal(_ffi.attn_fwd(q, k, v, out=wide, **kw).to(torch.bfloat16), _ffi.attn_fwd(q, k, v, **kw)), kw
+    with pytest.raises(_ffi.FlashlightError, match="fp32"):
+        _ffi.attn_fwd(q, k, v, out=wide, gate=torch.zeros(B, Hq, Lq, D, dtype=torch.bfloat16, device=DEV))
