@@ -834,7 +834,8 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
 }
 
 int fl_attn_rows_plan(const fl_attn_params* p, uint64_t* scratch_bytes) {
-  if (!p || !scratch_bytes || p->B <= 0 || p->Hkv <= 0 || p->Hq <= 0 || p->Lq <= 0 || p->Lk <= 0) return 0;
+  // (asked before fl_attn_fwd has checked the call)
+  if (!p || !scratch_bytes || p->B <= 0 || p->Hkv <= 0 || p->Hq < p->Hkv || p->Hq % p->Hkv || p->Lq <= 0 || p->Lk <= 0) return 0;
   fl::RParams rp;
   int grid = 0, waves = 0, blocks = 0;
   *scratch_bytes = 0;

@@ -31,6 +31,7 @@ def test_which_calls_the_few_rows_kernel_takes():
     assert not _taken(1, 8, 8, 1, 128, 64)[0]                   # too short to matter
     assert _taken(2, 8, 8, 512, 512, 64, mask_kind=_ffi.MASK_CAUSAL) == (True, 0)
     assert not _taken(4, 16, 16, 4096, 4096, 128)[0]
+    assert not _taken(1, 1, 2, 1, 1000, 64)[0] and not _taken(1, 3, 2, 1, 1000, 64)[0]   # (asked before the call is refused)
     # more than 32 rows against many keys: few workgroups without chunks
     for shape in ((1, 32, 8, 9, 32768, 128), (1, 8, 8, 64, 65536, 128), (1, 8, 8, 128, 65536, 64), (2, 8, 2, 40, 5000, 128)):
         assert _taken(*shape)[0] and _taken(*shape)[1] > 0, shape
