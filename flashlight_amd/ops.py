@@ -342,8 +342,9 @@ def dispatch(q, k, v, *, scale=None, mask_kind=_ffi.MASK_NONE, window=0, prefix=
     `doc_workspace` (an `_ffi.DocWorkspace`) is used by the plain forward call only; traced and differentiable calls run
     their pre-pass every time.  `score_fn` = (kind, four constants), see `_ffi.attn_fwd`: forward only."""
     if not dropout_p and score_fn is None and doc_workspace is None and not torch.compiler.is_compiling() and \
-            _ffi._host is not None:
-        # an ordinary call, differentiable or not, is launched by native code; None: it is not of that kind
+            (_ffi._host is not None or (q.is_cuda and _ffi.load_library())):
+        # an ordinary call, the first one included, differentiable or not, is launched by native code; None: it is not of
+        # that kind
         out = _ffi._host.forward(q, k, v, scale, mask_kind, window, prefix, doc_ids, alibi_heads, softcap, biases, gate, diff,
                             lambda_full, seq_major_out)
         if out is not None:

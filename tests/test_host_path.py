@@ -36,3 +36,18 @@ def test_other_threads_run_while_a_call_is_launched():
         _ffi._host.bind(*address.values())
     q.requires_grad_(False)
     assert torch.isfinite(ops.dispatch(q, k, v)).all()
+
+
+@pytest.mark.gpu
+def test_the_first_call_goes_the_way_of_the_others(monkeypatch):
+    """The library is loaded by the first call, which takes the native path like every later one (a differentiable gated
+    call rounds its result once there, twice in the Python path's composition)."""
+    q, k, v = _operands(4, 2, 64, 32)
+    gate, = _operands(4, 2, 64, 32, seed=1)[:1]
+    pair = torch.randn(1, 2, 64, 64, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).to(DEV)
+    q.requires_grad_(True)
+    call = lambda: ops.dispatch(q, k, v, biases=[(pair, 4)], gate=gate)  # noqa: E731
+    later = call()
+    monkeypatch.setattr(_ffi, "_lib", None)
+    monkeypatch.setattr(_ffi, "_host", None)
+    assert torch.equal(call(), later)
