@@ -614,7 +614,7 @@ bool plan_pairbias(const fl_attn_params* p, fl::PParams* out, int* grid) {
 // word that the workspace is scratch, the keys of a row tile stay in one workgroup.
 bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves, int* blocks, uint64_t* scratch) {
   if (p->Dqk != p->Dv || !fl::rows_has_shape(p->Dqk) || is_doc(p->mask_kind) || p->diff || p->gate || p->attended_dump ||
-      p->dropout_threshold || p->score_fn != FL_SCORE_NONE)
+      p->dropout_threshold || p->score_fn != FL_SCORE_NONE || (p->flags & FL_FLAG_F32_RESULT))
     return false;
   const bool has_bias = p->bias[0] || p->bias[1];
   if (has_bias && p->alibi_heads > 0) return false;
@@ -719,7 +719,6 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
     k.bias_div[i] = p->bias[i] ? p->bias_batch_div[i] : 1;
     k.bias_f32[i] = p->bias_dtype[i] == FL_F32;
   }
-  k.o_f32 = (p->flags & FL_FLAG_F32_RESULT) != 0;
   k.by_xcd = units * chunks >= 8 && row_tiles > 1;
   *grid = (int)(k.by_xcd ? (units * chunks + 7) / 8 * 8 * row_tiles : units * chunks * row_tiles);
   *waves = nw;

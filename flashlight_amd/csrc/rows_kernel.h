@@ -38,7 +38,6 @@ struct RParams {
   int32_t B, Hq, Hkv, Lq, Lk, group;
   int32_t rows;                              // group * Lq: packed rows per key / value head
   int32_t row_tiles, chunks, units;          // units = B * Hkv
-  int32_t o_f32;                             // o holds fp32 elements, as in KParams
   int32_t by_xcd;                            // row tiles of one (unit, chunk) on one XCD (units * chunks >= 8)
   float scale_log2, cap_k1, cap_c;           // as in fwd_kernel; cap_c = 0: no soft-cap
   int32_t dmin, dmax, pfx;                   // attend iff key < Lk && ((dmin <= key - q <= dmax) || key < pfx)
@@ -70,13 +69,6 @@ __device__ __forceinline__ int wave_min(int x) {
 #pragma unroll
   for (int d = 1; d < 64; d *= 2) x = min(x, __shfl_xor(x, d, 64));
   return x;
-}
-// four columns of a result at element `at`
-template <class E>
-__device__ __forceinline__ void store_result(const RParams& p, int64_t at, f32x4 o) {
-  typedef E ex4 __attribute__((ext_vector_type(4)));
-  if (p.o_f32) *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(p.o) + at) = o;
-  else *reinterpret_cast<ex4*>(p.o + at) = ex4{(E)o[0], (E)o[1], (E)o[2], (E)o[3]};
 }
 // MOD: 0 plain, F_ALIBI | F_SOFTCAP (either may be off at run time), F_BIAS (row biases, and the soft-cap at run time)
 // QT: 16-row blocks per wave (1 or 2)
@@ -361,7 +353,11 @@ void rows_kernel(const RParams p) {
     if (p.chunks == 1) {
       const int pr = rt * RB + r, hd = pr / p.Lq, pos = pr - hd * p.Lq, oh = kvh * p.group + hd;
       const float inv = L > 0.f ? 1.0f / L : 0.f;  // a row that attends nothing yields zeros
-      store_result<E>(p, (int64_t)batch * p.os[0] + (int64_t)oh * p.os[1] + (int64_t)pos * p.os[2] + c, o * inv);
+      typedef E ex4 __attribute__((ext_vector_type(4)));
+      ex4 w;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w[e] = (E)(o[e] * inv);
+      *reinterpret_cast<ex4*>(p.o + (int64_t)batch * p.os[0] + (int64_t)oh * p.os[1] + (int64_t)pos * p.os[2] + c) = w;
       if (p.lse != nullptr && c == 0)
         p.lse[((int64_t)batch * p.Hq + oh) * p.Lq + pos] = L > 0.f ? ref + __builtin_log2f(L) : INFINITY;
     } else {
@@ -416,7 +412,11 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
   }
   const int batch = unit / p.Hkv, kvh = unit % p.Hkv, hd = row / p.Lq, pos = row - hd * p.Lq, oh = kvh * p.group + hd;
   const float inv = Lt > 0.f ? 1.0f / Lt : 0.f;
-  store_result<E>(p, (int64_t)batch * p.os[0] + (int64_t)oh * p.os[1] + (int64_t)pos * p.os[2] + c, ot * inv);
+  typedef E ex4 __attribute__((ext_vector_type(4)));
+  ex4 w;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w[e] = (E)(ot[e] * inv);
+  *reinterpret_cast<ex4*>(p.o + (int64_t)batch * p.os[0] + (int64_t)oh * p.os[1] + (int64_t)pos * p.os[2] + c) = w;
   if (p.lse != nullptr && c == 0)
     p.lse[((int64_t)batch * p.Hq + oh) * p.Lq + pos] = Lt > 0.f ? reft + __builtin_log2f(Lt) : INFINITY;
 }

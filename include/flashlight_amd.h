@@ -164,7 +164,8 @@ typedef struct fl_attn_params {
 #define FL_FLAG_SCRATCH 8u
 
 /* fl_attn_fwd: `o` holds fp32 elements (o_strides in those, multiples of 4; 16-byte aligned).  For results over a part of
- * the keys that fl_attn_merge_chunks will put together.  Not with a gate or differential attention. */
+ * the keys that fl_attn_merge_chunks will put together; such calls never run in the kernel for few query rows.  Not with a
+ * gate or differential attention. */
 #define FL_FLAG_F32_RESULT 16u
 
 /* ABI version of the loaded library (FL_ABI_VERSION it was built with). */
