@@ -156,3 +156,31 @@ def test_results_in_fp32_are_what_the_16_bit_results_round(shape):
         assert torch.equal(_ffi.attn_fwd(q, k, v, out=wide, **kw).to(torch.bfloat16), _ffi.attn_fwd(q, k, v, **kw)), kw
     with pytest.raises(_ffi.FlashlightError, match="fp32"):
         _ffi.attn_fwd(q, k, v, out=wide, gate=torch.zeros(B, Hq, Lq, D, dtype=torch.bfloat16, device=DEV))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 8, 8, 64, 16384, 128), (1, 8, 8, 48, 9003, 128), (2, 8, 8, 130, 8192, 64), (1, 8, 2, 24, 4500, 64)])
+def test_chunks_of_the_keys_replay_from_a_graph(shape):
+    """More than 32 rows against many keys, by either way of cutting the keys, captured and replayed on new operands."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    g = torch.Generator(device=DEV).manual_seed(Lk)
+    q, k, v = (torch.randn(B, h, n, D, generator=g, device=DEV).to(torch.bfloat16) for h, n in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        ops.dispatch(q, k, v)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.dispatch(q, k, v)
+    for _ in range(3):
+        q.copy_(torch.randn(q.shape, generator=g, device=DEV))
+        v.mul_(-0.5)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = ops.dispatch(q, k, v)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+    G = Hq // Hkv
+    kf, vf = (t.float().cpu().repeat_interleave(G, 1) for t in (k, v))
+    assert_parity(eager, torch.softmax(q.float().cpu() @ kf.transpose(-1, -2) / math.sqrt(D), -1) @ vf, str(shape))
