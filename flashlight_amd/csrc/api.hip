@@ -954,7 +954,6 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   }
   kp.gate = static_cast<const fl::bf16_t*>(p->gate);
   kp.ungated = static_cast<fl::bf16_t*>(ungated);
-  kp.o_f32 = (p->flags & FL_FLAG_F32_RESULT) != 0;
   kp.lambda = p->lambda;
   if (p->diff) {
     // heads [0, H) are branch 0, heads [H, 2H) branch 1 (query: H = Hq, key: H = Hkv)
@@ -980,6 +979,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   }
   kp.o_wide = reinterpret_cast<uintptr_t>(p->o) % 16 == 0 && p->o_strides[0] % 8 == 0 && p->o_strides[1] % 8 == 0 &&
               p->o_strides[2] % 8 == 0;
+  if (p->flags & FL_FLAG_F32_RESULT) kp.o_wide = 2;
   const int grid = p->B * p->Hq * kp.n_qtiles;
 
   if (is_doc(p->mask_kind)) {
