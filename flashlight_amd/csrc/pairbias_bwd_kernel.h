@@ -16,12 +16,13 @@
 // (no barrier for them), and add up their partial dQ / dK, dV through LDS once per batch entry.  The next entry's rows are
 // on their way while one is worked on.  The sequence has at most 512 positions.
 //
-// Measured, 128 x 8 x 256 x 256, head dim 32, mask row and gate, bf16, whole step: 852 -> 177 us (ROLE_DQ 325 -> 46, ROLE_DKV
-// 232 -> 55, row sums and gate 150 -> 20, clearing and summing the bias gradient 97 -> 4).  Per score seven vector
-// instructions are left, and no global load, conversion or store; what bounds the roles now is the chain an entry goes
-// through (tiles, two products, weights, products, sums over the waves: 2.1 and 2.7 us) with two waves per SIMD to cover it:
-// the vector unit issues in 35 % of the cycles.  Two blocks per wave in four waves beat one in eight (67 and 93 us: the sums
-// over the waves cost more than the occupancy gains).
+// Measured, 128 x 8 x 256 x 256, head dim 32, mask row and gate, bf16, whole step: 852 -> 168 us (ROLE_DQ 325 -> 46, ROLE_DKV
+// 232 -> 56, row sums and gate 150 -> 16, clearing and summing the bias gradient 97 -> 4).  Per score ten vector
+// instructions are left (27 and 21 per MFMA; seven make the weight and its gradient, the rest operands and the sums over the
+// waves), and no global load, conversion or store; what bounds the roles now is the chain an entry goes through (tiles, two
+// products, weights, products, sums over the waves: 2.1 and 2.7 us) with two waves per SIMD to cover it: the vector unit takes
+// an instruction in 40 and 36 % of the cycles (SQ_ACTIVE_INST_VALU).  Two blocks per wave in four waves beat one in eight (67
+// and 93 us: the sums over the waves cost more than the occupancy gains).
 #pragma once
 #include "fwd_kernel.h"
 
