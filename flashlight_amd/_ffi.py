@@ -640,9 +640,10 @@ def merge_chunks(part: torch.Tensor, lse: torch.Tensor, dtype: Optional[torch.dt
     if lse.dtype != torch.float32 or tuple(lse.shape) != (outer, chunks, inner) or not (part.is_contiguous() and lse.is_contiguous()):
         raise ValueError("merge_chunks: lse must be float32 [outer, chunks, inner], both operands contiguous")
     out = torch.empty((outer, inner, dv), dtype=dtype, device=part.device)
-    rc = load_library().fl_attn_merge_chunks(C.c_void_p(part.data_ptr()), C.c_void_p(lse.data_ptr()), C.c_void_p(out.data_ptr()),
-                                             outer, chunks, inner, dv, _HALF_TYPES[dtype] + (PARTS_F32 if f32 else 0),
-                                             C.c_void_p(torch.cuda.current_stream().cuda_stream))
+    with torch.cuda.device(part.device):
+        rc = load_library().fl_attn_merge_chunks(C.c_void_p(part.data_ptr()), C.c_void_p(lse.data_ptr()), C.c_void_p(out.data_ptr()),
+                                                 outer, chunks, inner, dv, _HALF_TYPES[dtype] + (PARTS_F32 if f32 else 0),
+                                                 C.c_void_p(torch.cuda.current_stream().cuda_stream))
     if rc != 0:
         raise FlashlightError(rc, "fl_attn_merge_chunks rejected its arguments or could not launch")
     return out

@@ -1227,7 +1227,7 @@ uint64_t fl_attn_shared_bias_bwd_bytes(const fl_attn_params* p) {
 int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* stream_) {
   if (!b) return fail(FL_ERR_NULL, "params is null");
   const fl_attn_params* p = &b->fwd;
-  int rc = validate(p, nullptr, false, FL_FLAG_UNGATED);
+  int rc = validate(p, nullptr, false, FL_FLAG_UNGATED | FL_FLAG_SCRATCH);
   if (rc) return rc;
   SBScratch x;
   if (!plan_shared_bias_bwd(p, &x)) return fail(FL_ERR_UNSUPPORTED, "fl_attn_shared_bias_bwd does not take this call");

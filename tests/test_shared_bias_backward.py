@@ -45,6 +45,12 @@ def test_which_calls_the_shared_bias_backward_takes():
     assert lib.fl_attn_fwd_ungated(C.byref(params(gate=0x80000)), C.c_void_p(0x90008), None) == -7
     assert lib.fl_attn_validate(C.byref(params(flags=_ffi.FLAG_UNGATED))) == -5
 
+    class Bwd(C.Structure):  # fl_attn_shared_bias_bwd_params, as far as a refusal looks: its forward's flags come first
+        _fields_ = [("fwd", _ffi.FlAttnParams), ("rest", C.c_uint64 * 40)]
+
+    for flags, rc in ((_ffi.FLAG_UNGATED | _ffi.FLAG_SCRATCH, -1), (_ffi.FLAG_F32_RESULT, -5), (4, -5)):   # (-1: no dout)
+        assert lib.fl_attn_shared_bias_bwd(C.byref(Bwd(fwd=params(flags=flags))), None) == rc
+
 
 CASES = [  # B, N, S, H, D
     (1, 3, 32, 2, 32), (2, 5, 64, 3, 32), (1, 9, 100, 4, 64), (2, 17, 129, 2, 32), (1, 4, 256, 4, 64), (1, 40, 256, 8, 32),
