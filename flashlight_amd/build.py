@@ -127,8 +127,8 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
         objs.append(o)
         if not o.exists():
             tasks.append(([cc, *HIPCC_FLAGS, f"-DFL_INST_F16={f16}", "-c", str(CSRC / "pairbias_unit.hip"), "-o", str(o)], o))
-    # the few-rows forward and the shared-bias backward: one unit each per element type
-    for unit in ("rows", "pairbias_bwd"):
+    # the few-rows forward, the shared-bias backward and the shared-bias stripe forward: one unit each per element type
+    for unit in ("rows", "pairbias_bwd", "stripe"):
         for f16 in (0, 1):
             o = objdir / f"{unit}{'_f16' if f16 else ''}.o"
             objs.append(o)

@@ -12,6 +12,7 @@
 #include "pairbias_bwd_instances.h"
 #include "pairbias_instances.h"
 #include "rows_instances.h"
+#include "stripe_instances.h"
 
 namespace fl {
 // Builds (min, max) of the document ids of every block of kDocBlock positions.
@@ -609,6 +610,98 @@ bool plan_pairbias(const fl_attn_params* p, fl::PParams* out, int* grid) {
   return true;
 }
 
+// Whether bias operand `nb` can travel through LDS with the general forward's K/V tiles: rows addressable in 16-byte pieces, and
+// per-lane byte offsets inside one (batch, head) slice in 32 bits.
+bool bias_stageable(const fl_attn_params* p, int nb) {
+  const int64_t* st = p->bias_strides[nb];
+  return p->bias[nb] && st[3] == 1 && reinterpret_cast<uintptr_t>(p->bias[nb]) % 16 == 0 && p->Lk % 8 == 0 && st[0] % 8 == 0 &&
+         st[1] % 8 == 0 && st[2] % 8 == 0 && ((int64_t)p->Lq * st[2] + p->Lk) * 4 < ((int64_t)1 << 31);
+}
+
+// Whether *p (already validated) is a call the shared-bias stripe forward (stripe_kernel.h) takes.  Fills the kernel's parameters,
+// its wave count, and the number of workgroups and their LDS bytes.
+bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, int* waves, int64_t (&launch)[2]) {
+  if (p->Dqk != p->Dv || (p->Dqk != 32 && p->Dqk != 64) || p->Hq != p->Hkv || p->Lq > 512 || p->Lk > 512 || p->Lk < 4 ||
+      p->mask_kind != FL_MASK_NONE || p->alibi_heads > 0 || p->softcap > 0.f || p->diff || p->attended_dump || p->dropout_threshold ||
+      p->score_fn != FL_SCORE_NONE || (p->flags & FL_FLAG_F32_RESULT))
+    return false;
+  // one operand that several consecutive batch entries share, dense over heads and queries, and optionally one that is a row of keys
+  // per batch entry, the same for every head and query; in either order
+  int pi = -1, ri = -1;
+  for (int i = 0; i < 2; ++i) {
+    if (!p->bias[i]) continue;
+    const int64_t* st = p->bias_strides[i];
+    if (p->bias_batch_div[i] >= 2 && (st[1] != 0 || p->Hq == 1) && (st[2] != 0 || p->Lq == 1) && (st[3] == 1 || p->Lk == 1) && pi < 0) pi = i;
+    else if (st[1] == 0 && st[2] == 0 && st[3] <= 0x7fffffff && ri < 0) ri = i;
+    else return false;
+  }
+  if (pi < 0) return false;
+  // Where the general kernel has to read the bias two bytes at a time (odd lengths, fp32), this one is three to five times sooner
+  // (bf16, us: 414 x 4 x 494 x 494, head dim 32: 806 -> 201; 34 x 4 x 235 x 235, head dim 64: 43 -> 17; 28 x 4 x 106 x 106: 14 -> 6).  Where
+  // that kernel can stage the bias beside its tiles, this one is ahead at head dim 32 with three or four waves, which fill the
+  // compute unit twice over (128 x 8 x 160 / 192 / 256 keys: 39.8 -> 34.7, 38.2 -> 34.4, 44 -> 37) and behind at other lengths (128
+  // keys: 18.6 against 21.4; 320: 73 against 87; 512 a tie) and at head dim 64 (256 keys: 60 against 99: one block of queries per
+  // workgroup).
+  if (p->bias_dtype[pi] != FL_F32 && bias_stageable(p, pi) && !(p->Dqk == 32 && p->Lk > 128 && p->Lk <= 256)) return false;
+  // per-lane byte offsets inside one (batch entry, head) are 32-bit; results leave and gate logits arrive 16 bytes at a time
+  for (const int64_t* st : {p->q_strides, p->k_strides, p->v_strides, p->o_strides})
+    if (st[2] >= (1 << 20)) return false;
+  if (reinterpret_cast<uintptr_t>(p->o) % 16 || p->o_strides[0] % 8 || p->o_strides[1] % 8 || p->o_strides[2] % 8) return false;
+  if (p->gate && (reinterpret_cast<uintptr_t>(p->gate) % 16 || p->gate_strides[0] % 8 || p->gate_strides[1] % 8 || p->gate_strides[2] % 8))
+    return false;
+  fl::StripeParams k;
+  std::memset(&k, 0, sizeof(k));
+  k.q = static_cast<const fl::bf16_t*>(p->q);
+  k.k = static_cast<const fl::bf16_t*>(p->k);
+  k.v = static_cast<const fl::bf16_t*>(p->v);
+  k.o = static_cast<fl::bf16_t*>(p->o);
+  for (int i = 0; i < 3; ++i) {
+    k.qs[i] = p->q_strides[i];
+    k.ks[i] = p->k_strides[i];
+    k.vs[i] = p->v_strides[i];
+    k.os[i] = p->o_strides[i];
+    k.gs[i] = p->gate_strides[i];
+    k.bs[i] = p->bias_strides[pi][i];
+  }
+  k.bias = p->bias[pi];
+  k.bias_f32 = p->bias_dtype[pi] == FL_F32;
+  k.row_div = 1;
+  if (ri >= 0) {
+    k.row = p->bias[ri];
+    k.row_batch = p->bias_strides[ri][0];
+    k.row_key = (int)p->bias_strides[ri][3];
+    k.row_div = p->bias_batch_div[ri];
+    k.row_f32 = p->bias_dtype[ri] == FL_F32;
+  }
+  k.gate = static_cast<const fl::bf16_t*>(p->gate);
+  k.ungated = static_cast<fl::bf16_t*>(ungated);
+  k.lse = p->lse;
+  k.B = p->B;
+  k.H = p->Hq;
+  k.Lq = p->Lq;
+  k.Lk = p->Lk;
+  k.div = p->bias_batch_div[pi];
+  k.groups = p->B / k.div;
+  k.scale = p->scale;
+  k.scale_log2 = p->scale * 1.4426950408889634f;
+  const fl::StripeShape shape = fl::stripe_shape(p->Dqk, p->Lk, ri >= 0);
+  // (the general kernel forms the weights of a last tile of fewer than 64 keys against its maximum, which makes the largest
+  // weight exact; here the whole row's maximum, at 6 to 20 % of the time)
+  k.by_maximum = p->Lk % 64 != 0;
+  k.tiles = (p->Lq + 32 * shape.qb - 1) / (32 * shape.qb);
+  // entries per workgroup: as many as leave one round of workgroups
+  const int64_t units = (int64_t)k.groups * k.H * k.tiles;
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(k.div, 256 * shape.per_cu / units));
+  k.chunk_len = (int)((k.div + most - 1) / most);
+  k.chunks = (k.div + k.chunk_len - 1) / k.chunk_len;
+  if (units * k.chunks > (1 << 28)) return false;
+  *out = k;
+  *waves = shape.waves;
+  launch[0] = ((int64_t)k.groups * k.chunks * k.H + 7) / 8 * 8 * k.tiles;
+  launch[1] = shape.lds_bytes;
+  return true;
+}
+
 // Whether *p (already validated) is a call the few-rows forward (rows_kernel.h) takes.  Fills the kernel's parameters and
 // launch shape.  `scratch`: bytes of p->workspace it would use to cut the keys into chunks; with less, or without the caller's
 // word that the workspace is scratch, the keys of a row tile stay in one workgroup.
@@ -826,6 +919,18 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
       out[3] = pb_grid;
       out[4] = 2 * (p->Dqk == 32 ? 6 : 4) * 64 * p->Dqk * 2 + (pb.rowb ? 4 * 2 * 1024 : 0);
       out[6] = 1;
+      return 0;
+    }
+    fl::StripeParams sp;
+    int waves = 0;
+    int64_t launch[2];
+    if (plan_stripe(p, nullptr, &sp, &waves, launch)) {
+      out[0] = p->Dqk == 32 ? 64 : 32;
+      out[1] = 64 * waves;
+      out[2] = 64 * waves;
+      out[3] = launch[0];
+      out[4] = launch[1];
+      out[6] = 2;
     }
   }
   out[7] = 0;
@@ -854,6 +959,16 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
       const hipError_t e = (p->dtype == FL_F16 ? fl::launch_pairbias_f16 : fl::launch_pairbias_bf16)(
           p->Dqk, p->Lk / 32, p->gate != nullptr, pb.rowb != nullptr, pb, pb_grid, stream);
       if (e != hipSuccess) return fail((int)e, "launch of the shared-bias forward failed: %s", hipGetErrorString(e));
+      return 0;
+    }
+  }
+  {
+    fl::StripeParams sp;
+    int waves = 0;
+    int64_t plan[2];
+    if (plan_stripe(p, ungated, &sp, &waves, plan)) {
+      const hipError_t e = (p->dtype == FL_F16 ? fl::launch_stripe_f16 : fl::launch_stripe_bf16)(p->Dqk, waves, sp, stream);
+      if (e != hipSuccess) return fail((int)e, "launch of the shared-bias stripe forward failed: %s", hipGetErrorString(e));
       return 0;
     }
   }
@@ -939,16 +1054,10 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   kp.bias_lds = -1;
   kp.bias_row = -1;
   for (int nb = 0; nb < 2; ++nb) {
-    if (!p->bias[nb] || p->bias_strides[nb][3] != 1 || reinterpret_cast<uintptr_t>(p->bias[nb]) % 16 != 0) continue;
-    if (p->Lk % 8 != 0) continue;
+    if (!bias_stageable(p, nb)) continue;
     // fp32: staged only as the row-broadcast operand (the [rows][keys] tiles hold 16-bit elements, so a second fp32 row
     // operand takes the direct path)
     if (kp.bias_f32[nb] && (p->bias_strides[nb][2] != 0 || kp.bias_row >= 0)) continue;
-    bool ok = true;
-    for (int i = 0; i < 3; ++i) ok = ok && p->bias_strides[nb][i] % 8 == 0;
-    // per-lane byte offsets inside one (batch, head) slice are 32-bit
-    ok = ok && ((int64_t)p->Lq * p->bias_strides[nb][2] + p->Lk) * 4 < ((int64_t)1 << 31);
-    if (!ok) continue;
     if (p->bias_strides[nb][2] == 0 && kp.bias_row < 0) kp.bias_row = nb;
     else if (kp.bias_lds < 0) kp.bias_lds = nb;
   }
