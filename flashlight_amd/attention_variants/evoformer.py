@@ -46,6 +46,11 @@ def attention_reference(q_input: torch.Tensor, k_input: torch.Tensor, v_input: t
     `gate=` (not in the reference): bf16 logits shaped like the result; the result is multiplied by sigmoid(gate)
     in the kernel's epilogue."""
     gate = kwargs.get("gate")
+    if not torch.compiler.is_compiling() and (_ffi._host is not None or (q_input.is_cuda and _ffi.load_library())):
+        # an ordinary call is native code's from here on; None: it is not of that kind
+        out = _ffi._host.evoformer(q_input, k_input, v_input, biases, sm_scale, gate)
+        if out is not None:
+            return out
     if q_input.dim() < 4:
         raise ValueError("expected inputs of shape [*, S, H, D]")
     lead = tuple(q_input.shape[:-3])

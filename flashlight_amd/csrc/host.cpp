@@ -9,6 +9,8 @@
 // the compositions, the error messages.  It keeps no state between calls beyond the addresses of the C ABI's functions.
 #define PY_SSIZE_T_CLEAN
 #include <ATen/ATen.h>
+#include <ATen/TensorUtils.h>
+#include <ATen/core/LegacyTypeDispatch.h>
 #include <Python.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
@@ -53,7 +55,46 @@ struct Call {
   double softcap = 0, lambda = 0;
   bool diff = false, seq_major = false;
   bool wants_grad = false;
+  // Calls of the Evoformer front end: the leading axes of its [*, S, H, D] operands, of which q, k, v and gate here are the
+  // [prod(*), H, S, D] views and the biases the kernels' 4-D form.  Its gradients hang on the operands as the caller passed them,
+  // in one node (as views of their own the operands and the result cost a dozen nodes, 80 of 110 us of a short backward pass).
+  std::vector<int64_t> lead;
+  Tensor given_q, given_k, given_v, given_bias[2], given_gate;  // with `lead`: the operands as the caller passed them
 };
+
+// [*, S, H, D] -> its [prod(*), H, S, D] view; undefined where the leading axes do not merge.
+Tensor heads_first(const Tensor& t, size_t lead) {
+  const auto sizes = t.sizes();
+  int64_t rows = 1;
+  for (size_t i = 0; i < lead; ++i) rows *= sizes[i];
+  const int64_t merged[4] = {rows, sizes[lead], sizes[lead + 1], sizes[lead + 2]};
+  const auto st = at::detail::computeStride(sizes, t.strides(), at::IntArrayRef(merged, 4));
+  if (!st) return Tensor();
+  const at::AutoDispatchBelowADInplaceOrView plainly;  // (a view for the kernels' use, which autograd does not see)
+  const int64_t size4[4] = {rows, merged[2], merged[1], merged[3]}, stride4[4] = {(*st)[0], (*st)[2], (*st)[1], (*st)[3]};
+  return t.as_strided(at::IntArrayRef(size4, 4), at::IntArrayRef(stride4, 4));
+}
+
+// A bias broadcastable to [*, H, S, S] in the kernels' form, [Bb, H or 1, S or 1, S] with batch entry b reading Bb index
+// b / div: as evoformer._as_kernel_bias, undefined where that would copy.
+Tensor kernel_bias(const Tensor& b, const std::vector<int64_t>& lead, int64_t H, int64_t S, int64_t& div) {
+  const int64_t nl = (int64_t)lead.size(), missing = nl + 3 - b.dim();
+  if (missing < 0 || b.dim() == 0) return Tensor();
+  const auto size = [&](int64_t i) { return i < missing ? 1 : b.size(i - missing); };
+  if ((size(nl) != H && size(nl) != 1) || (size(nl + 1) != S && size(nl + 1) != 1) || size(nl + 2) != S) return Tensor();
+  int64_t split = nl, nb = 1;
+  while (split > 0 && size(split - 1) == 1) --split;
+  for (int64_t i = 0; i < split; ++i) {
+    if (size(i) != lead[i]) return Tensor();
+    nb *= lead[i];
+  }
+  div = 1;
+  for (int64_t i = split; i < nl; ++i) div *= lead[i];
+  const int64_t shape[4] = {nb, size(nl), size(nl + 1), S};
+  const auto st = at::detail::computeStride(b.sizes(), b.strides(), at::IntArrayRef(shape, 4));
+  const at::AutoDispatchBelowADInplaceOrView plainly;
+  return st ? b.as_strided(at::IntArrayRef(shape, 4), *st) : Tensor();
+}
 
 // dense, dim-contiguous rows in 16-byte pieces: what the kernels address as it lies
 bool addressable(const Tensor& t) {
@@ -306,24 +347,25 @@ struct Attention : torch::autograd::Function<Attention> {
       set_strides(b.fwd.o_strides, out);
       b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
       Tensor dq = empty_for_gradient(c.q), dk = empty_for_gradient(c.k), dv = empty_for_gradient(c.v);
-      Tensor delta = at::empty(lse.sizes(), lse.options()), ws, split;
       b.dout = dout.const_data_ptr();
       b.dq = dq.data_ptr();
       b.dk = dk.data_ptr();
       b.dv = dv.data_ptr();
-      b.delta = delta.data_ptr<float>();
       set_strides(b.dout_strides, dout);
       set_strides(b.dq_strides, dq);
       set_strides(b.dk_strides, dk);
       set_strides(b.dv_strides, dv);
-      if (const uint64_t bytes = g_api.bwd_workspace(&b.fwd)) {
-        ws = at::empty({(int64_t)bytes}, delta.options().dtype(at::kByte));
-        b.fwd.workspace = ws.data_ptr();
-        b.fwd.workspace_bytes = bytes;
+      // scratch in one block: the row sums, the document table, partial sums
+      const auto up = [](uint64_t bytes) { return (bytes + 255) / 256 * 256; };
+      const uint64_t table = g_api.bwd_workspace(&b.fwd), split = g_api.bwd_split_bytes(&b.fwd), sums = up(4 * (uint64_t)lse.numel());
+      Tensor scratch = at::empty({(int64_t)(sums + up(table) + split)}, lse.options().dtype(at::kByte));
+      unsigned char* const at = scratch.data_ptr<unsigned char>();
+      b.delta = reinterpret_cast<float*>(at);
+      if (table) {
+        b.fwd.workspace = at + sums;
+        b.fwd.workspace_bytes = table;
       }
-      const uint64_t split_bytes = g_api.bwd_split_bytes(&b.fwd);
-      if (split_bytes) split = at::empty({(int64_t)split_bytes}, delta.options().dtype(at::kByte));
-      const int rc = g_api.bwd(&b, split_bytes ? split.data_ptr() : nullptr, split_bytes, current_stream());
+      const int rc = g_api.bwd(&b, split ? at + sums + up(table) : nullptr, split, current_stream());
       TORCH_CHECK(rc == 0, "flashlight_amd error ", rc, ": ", g_api.last_error());
       result[0] = dq;
       result[1] = dk;
@@ -334,64 +376,87 @@ struct Attention : torch::autograd::Function<Attention> {
   }
 };
 
+// The result of an Evoformer call as its caller sees it, [*, S, H, D], from the kernels' sequence-major 4-D one.
+Tensor with_lead(const Tensor& out, const std::vector<int64_t>& lead) {
+  std::vector<int64_t> sizes(lead);
+  sizes.insert(sizes.end(), {out.size(2), out.size(1), out.size(3)});
+  std::vector<int64_t> strides(sizes.size());
+  int64_t s = 1;
+  for (size_t i = sizes.size(); i-- > 0; s *= sizes[i]) strides[i] = s;
+  const at::AutoDispatchBelowADInplaceOrView plainly;  // (the caller's tensor, not a view of one it never sees)
+  return out.as_strided(sizes, strides);
+}
+
 // Calls with a bias shared by batch entries, and optionally the gate (fl_attn_shared_bias_bwd).  bias[0] is the shared
-// operand here, bias[1] the row per batch entry, which takes no gradient.
+// operand here, bias[1] the row per batch entry, which takes no gradient.  The tensors are the caller's, `c` holds the kernels'
+// views of them.
 struct SharedBias : torch::autograd::Function<SharedBias> {
   static Tensor forward(AutogradContext* ctx, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& bias,
                         const std::optional<Tensor>& row, const std::optional<Tensor>& gate, const Call& c) {
     Tensor lse, ungated;
     Tensor out = launch_forward(c, &lse, gate ? &ungated : nullptr);
     if (!out.defined()) throw Refused();
+    if (!c.lead.empty()) out = with_lead(out, c.lead);
     // (the gradients are formed from the attention's own result: a nearly closed gate leaves the gated one few bits)
     ctx->save_for_backward({q, k, v, bias, row.value_or(Tensor()), gate.value_or(Tensor()), gate ? ungated : out, lse});
     keep_scalars(ctx, c);
+    ctx->saved_data["lead"] = c.lead;
     return out;
   }
 
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     const auto saved = ctx->get_saved_variables();
-    Call c;
-    c.q = saved[0];
-    c.k = saved[1];
-    c.v = saved[2];
-    c.bias[0] = saved[3];
-    c.bias[1] = saved[4];
-    c.gate = saved[5];
-    take_scalars(ctx, c);
-    const Tensor &out = saved[6], &lse = saved[7];
     variable_list result(7);
     if (!grads[0].defined()) return result;
     const bool grad_mode = at::GradMode::is_enabled();
     {
-      at::AutoGradMode off(false);
-      Tensor dout = prepare_dout(grads[0], c.q);
-      if (dout.stride(2) >= 1 << 20) dout = dout.contiguous();  // (the kernels' offsets inside one (batch entry, head))
+      at::AutoDispatchBelowAutograd below;
+      Call c;
+      take_scalars(ctx, c);
+      c.lead = ctx->saved_data["lead"].toIntVector();
+      const size_t nl = c.lead.size();
+      const auto view = [&](const Tensor& t) {
+        if (!nl || !t.defined()) return t;
+        const Tensor x = heads_first(t, nl);
+        return x.defined() ? x : heads_first(t.contiguous(), nl);
+      };
+      c.q = view(saved[0]);
+      c.k = view(saved[1]);
+      c.v = view(saved[2]);
+      c.gate = view(saved[5]);
+      for (int i = 0; i < 2; ++i) {
+        int64_t div;
+        c.bias[i] = nl && saved[3 + i].defined() ? kernel_bias(saved[3 + i], c.lead, c.q.size(1), c.q.size(2), div) : saved[3 + i];
+      }
+      const Tensor out = c.gate.defined() ? saved[6] : view(saved[6]);
+      const Tensor& lse = saved[7];
+      Tensor dout = view(grads[0].to(c.q.scalar_type()));
+      if (!addressable(dout) || dout.stride(2) >= 1 << 20) {  // (the kernels' offsets inside one (batch entry, head))
+        dout = nl ? dout.transpose(1, 2).contiguous().transpose(1, 2) : dout.contiguous();
+      }
       fl_attn_shared_bias_bwd_params b = {};
       fill(c, b.fwd);
       b.fwd.o = const_cast<void*>(out.const_data_ptr());
       set_strides(b.fwd.o_strides, out);
       b.fwd.lse = const_cast<float*>(lse.const_data_ptr<float>());
       if (c.gate.defined()) b.fwd.flags = FL_FLAG_UNGATED;
-      Tensor dq = empty_for_gradient(c.q), dk = empty_for_gradient(c.k), dv = empty_for_gradient(c.v);
+      // the gradients lie as the caller's operands do
+      const auto gradient = [&](Tensor& to, const Tensor& like, int64_t* strides) -> void* {
+        to = empty_for_gradient(like);
+        set_strides(strides, view(to));
+        return to.data_ptr();
+      };
       b.dout = dout.const_data_ptr();
-      b.dq = dq.data_ptr();
-      b.dk = dk.data_ptr();
-      b.dv = dv.data_ptr();
       set_strides(b.dout_strides, dout);
-      set_strides(b.dq_strides, dq);
-      set_strides(b.dk_strides, dk);
-      set_strides(b.dv_strides, dv);
-      Tensor dgate, dbias;
-      if (c.gate.defined()) {
-        dgate = empty_for_gradient(c.gate);
-        b.dgate = dgate.data_ptr();
-        set_strides(b.dgate_strides, dgate);
-      }
+      b.dq = gradient(result[0], saved[0], b.dq_strides);
+      b.dk = gradient(result[1], saved[1], b.dk_strides);
+      b.dv = gradient(result[2], saved[2], b.dv_strides);
+      if (c.gate.defined()) b.dgate = gradient(result[5], saved[5], b.dgate_strides);
       if (ctx->needs_input_grad(3)) {
         TORCH_CHECK(c.bias[0].size(0) == b.fwd.B / c.bias_div[0], "one gradient per ", c.bias_div[0], " batch entries, ",
                     c.bias[0].size(0), " operands");
-        dbias = at::empty(c.bias[0].sizes(), c.bias[0].options().requires_grad(false));
-        b.dbias = dbias.data_ptr();
+        result[3] = at::empty(saved[3].sizes(), saved[3].options());
+        b.dbias = result[3].data_ptr();
       }
       const uint64_t bytes = g_api.shared_bias_bwd_bytes(&b.fwd);
       Tensor ws = at::empty({(int64_t)bytes}, lse.options().dtype(at::kByte));
@@ -399,11 +464,6 @@ struct SharedBias : torch::autograd::Function<SharedBias> {
       b.workspace_bytes = bytes;
       const int rc = g_api.shared_bias_bwd(&b, current_stream());
       TORCH_CHECK(rc == 0, "flashlight_amd error ", rc, ": ", g_api.last_error());
-      result[0] = dq;
-      result[1] = dk;
-      result[2] = dv;
-      result[3] = dbias;
-      result[5] = dgate;
     }
     once_differentiable(result, grad_mode);
     return result;
@@ -432,11 +492,67 @@ Tensor attend(const Call& c) {
   const WithoutGil no_gil;
   if (!c.wants_grad) return launch_forward(c, nullptr);
   try {
+    if (!c.lead.empty())
+      return SharedBias::apply(c.given_q, c.given_k, c.given_v, c.given_bias[0], given(c.given_bias[1]), given(c.given_gate), c);
     return c.bias[0].defined() ? SharedBias::apply(c.q, c.k, c.v, c.bias[0], given(c.bias[1]), given(c.gate), c)
                                : Attention::apply(c.q, c.k, c.v, c);
   } catch (const Refused&) {
     return Tensor();
   }
+}
+
+// ---- what the native path takes ------------------------------------------------------------------------------------------
+
+bool operands_fit(const Call& c) {
+  const Tensor &q = c.q, &k = c.k, &v = c.v;
+  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || element_type(q) < 0 || k.scalar_type() != q.scalar_type() ||
+      v.scalar_type() != q.scalar_type())
+    return false;
+  const int64_t two = c.diff ? 2 : 1, B = q.size(0), Hq = q.size(1) / two, Hkv = k.size(1) / two, Lk = k.size(2), D = q.size(3),
+                Dv = v.size(3);
+  if (q.numel() == 0 || k.numel() == 0 || v.numel() == 0 || k.size(0) != B || v.size(0) != B || v.size(2) != Lk || k.size(3) != D ||
+      q.size(1) % two || k.size(1) % two || Hkv == 0 || Hq % Hkv || v.size(1) != Hkv)
+    return false;
+  if (c.diff ? !(D == 64 && Dv == 128) : !(D == Dv && (D == 32 || D == 64 || D == 128))) return false;
+  if (!addressable(q) || !addressable(k) || !addressable(v)) return false;
+  const auto dev = q.device();
+  return k.device() == dev && v.device() == dev && dev.index() == c10::hip::current_device();
+}
+
+bool bias_fits(const Call& c, int i) {
+  const Tensor& b = c.bias[i];
+  const int64_t div = c.bias_div[i], B = c.q.size(0), Hq = c.q.size(1) / (c.diff ? 2 : 1);
+  if (b.dim() != 4 || b.device() != c.q.device() || div < 1 || B % div || (b.scalar_type() != at::kFloat && b.scalar_type() != c.q.scalar_type()))
+    return false;
+  const int64_t want[4] = {B / div, Hq, c.q.size(2), c.k.size(2)};
+  for (int ax = 0; ax < 4; ++ax)
+    if ((b.size(ax) != want[ax] && b.size(ax) != 1) || b.stride(ax) < 0) return false;
+  return b.size(3) == 1 || b.stride(3) == 1;
+}
+
+bool gate_fits(const Call& c) {
+  const Tensor& g = c.gate;
+  return g.scalar_type() == c.q.scalar_type() && g.dim() == 4 && g.device() == c.q.device() && g.size(0) == c.q.size(0) &&
+         g.size(1) == c.q.size(1) / (c.diff ? 2 : 1) && g.size(2) == c.q.size(2) && g.size(3) == c.v.size(3) && addressable(g);
+}
+
+// Whether the shared-bias gradient kernels take a differentiable call with bias operands, a gate or both; puts the shared operand
+// first.  `given`: the operands as the caller passed them (c.bias, or c.given_bias).
+bool shared_bias_gradients(Call& c, Tensor* given) {
+  const int64_t Hq = c.q.size(1), Lq = c.q.size(2), Lk = c.k.size(2), B = c.q.size(0);
+  if (c.bias[1].defined() && c.bias[1].size(1) == Hq && c.bias[1].size(2) == Lq && Hq * Lq > 1) {
+    std::swap(c.bias[0], c.bias[1]);
+    std::swap(c.bias_div[0], c.bias_div[1]);
+    if (given != c.bias) std::swap(given[0], given[1]);
+  }
+  // a batch axis of 1 says that all batch entries share the operand: the gradient kernels write one [Hq, Lq, Lk] per
+  // B / divisor, and there is room for one
+  if (c.bias[0].defined() && c.bias[0].size(0) == 1) c.bias_div[0] = B;
+  fl_attn_params p = {};
+  fill(c, p);
+  return c.bias[0].defined() && c.bias[0].size(1) == Hq && c.bias[0].size(2) == Lq && c.bias[0].size(3) == Lk &&
+         !(c.bias[1].defined() && (given[1].requires_grad() || c.bias[1].size(1) != 1 || c.bias[1].size(2) != 1)) &&
+         g_api.shared_bias_bwd_bytes(&p) > 0;
 }
 
 // forward(q, k, v, scale, mask_kind, window, prefix, doc_ids, alibi_heads, softcap, biases, gate, diff, lambda, seq_major)
@@ -450,23 +566,14 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Call c;
   if (!take_tensor(a[0], c.q) || !take_tensor(a[1], c.k) || !take_tensor(a[2], c.v)) Py_RETURN_NONE;
   if (mode_active()) Py_RETURN_NONE;
-  const Tensor &q = c.q, &k = c.k, &v = c.v;
-  if (q.dim() != 4 || k.dim() != 4 || v.dim() != 4 || element_type(q) < 0 || k.scalar_type() != q.scalar_type() ||
-      v.scalar_type() != q.scalar_type())
-    Py_RETURN_NONE;
   c.diff = a[12] == Py_True;
   c.seq_major = a[14] == Py_True;
-  const int64_t two = c.diff ? 2 : 1, B = q.size(0), Hq = q.size(1) / two, Hkv = k.size(1) / two, Lq = q.size(2), Lk = k.size(2),
-                D = q.size(3), Dv = v.size(3);
-  if (q.numel() == 0 || k.numel() == 0 || v.numel() == 0 || k.size(0) != B || v.size(0) != B || v.size(2) != Lk || k.size(3) != D ||
-      q.size(1) % two || k.size(1) % two || Hkv == 0 || Hq % Hkv || v.size(1) != Hkv)
-    Py_RETURN_NONE;
-  if (c.diff ? !(D == 64 && Dv == 128) : !(D == Dv && (D == 32 || D == 64 || D == 128))) Py_RETURN_NONE;
-  if (!addressable(q) || !addressable(k) || !addressable(v)) Py_RETURN_NONE;
+  if (!operands_fit(c)) Py_RETURN_NONE;
+  const Tensor &q = c.q, &k = c.k, &v = c.v;
+  const int64_t B = q.size(0), Lq = q.size(2), Lk = k.size(2);
   const auto dev = q.device();
-  if (k.device() != dev || v.device() != dev || dev.index() != c10::hip::current_device()) Py_RETURN_NONE;
   if (a[3] == Py_None) {
-    c.scale = 1.0 / std::sqrt((double)D);
+    c.scale = 1.0 / std::sqrt((double)q.size(3));
   } else {
     c.scale = PyFloat_AsDouble(a[3]);
   }
@@ -496,21 +603,10 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   for (Py_ssize_t i = 0; i < nb; ++i) {
     PyObject* pair = PySequence_Fast_GET_ITEM(biases, i);
     if (!PyTuple_Check(pair) || PyTuple_GET_SIZE(pair) != 2 || !PyLong_Check(PyTuple_GET_ITEM(pair, 1))) Py_RETURN_NONE;
-    Tensor& b = c.bias[i];
-    const int64_t div = c.bias_div[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(pair, 1));
-    if (!take_tensor(PyTuple_GET_ITEM(pair, 0), b) || b.dim() != 4 || b.device() != dev || div < 1 || B % div ||
-        (b.scalar_type() != at::kFloat && b.scalar_type() != q.scalar_type()))
-      Py_RETURN_NONE;
-    const int64_t want[4] = {B / div, Hq, Lq, Lk};
-    for (int ax = 0; ax < 4; ++ax)
-      if ((b.size(ax) != want[ax] && b.size(ax) != 1) || b.stride(ax) < 0) Py_RETURN_NONE;
-    if (b.size(3) != 1 && b.stride(3) != 1) Py_RETURN_NONE;
+    c.bias_div[i] = PyLong_AsLongLong(PyTuple_GET_ITEM(pair, 1));
+    if (!take_tensor(PyTuple_GET_ITEM(pair, 0), c.bias[i]) || !bias_fits(c, i)) Py_RETURN_NONE;
   }
-  if (a[11] != Py_None) {
-    if (!take_tensor(a[11], c.gate) || c.gate.scalar_type() != q.scalar_type() || c.gate.dim() != 4 || c.gate.device() != dev ||
-        c.gate.size(0) != B || c.gate.size(1) != Hq || c.gate.size(2) != Lq || c.gate.size(3) != Dv || !addressable(c.gate))
-      Py_RETURN_NONE;
-  }
+  if (a[11] != Py_None && (!take_tensor(a[11], c.gate) || !gate_fits(c))) Py_RETURN_NONE;
   c.wants_grad = at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad() ||
                                                 (c.gate.defined() && c.gate.requires_grad()) ||
                                                 (c.bias[0].defined() && c.bias[0].requires_grad()) ||
@@ -518,19 +614,7 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (c.wants_grad) {
     if (c.diff) Py_RETURN_NONE;
     if (nb || c.gate.defined()) {
-      if (c.bias[1].defined() && c.bias[1].size(1) == Hq && c.bias[1].size(2) == Lq && Hq * Lq > 1) {  // the shared operand first
-        std::swap(c.bias[0], c.bias[1]);
-        std::swap(c.bias_div[0], c.bias_div[1]);
-      }
-      // a batch axis of 1 says that all batch entries share the operand: the gradient kernels write one [Hq, Lq, Lk] per
-      // B / divisor, and there is room for one
-      if (c.bias[0].defined() && c.bias[0].size(0) == 1) c.bias_div[0] = B;
-      fl_attn_params p = {};
-      fill(c, p);
-      if (!c.bias[0].defined() || c.bias[0].size(1) != Hq || c.bias[0].size(2) != Lq || c.bias[0].size(3) != Lk ||
-          (c.bias[1].defined() && (c.bias[1].requires_grad() || c.bias[1].size(1) != 1 || c.bias[1].size(2) != 1)) ||
-          !g_api.shared_bias_bwd_bytes(&p))
-        Py_RETURN_NONE;
+      if (!shared_bias_gradients(c, c.bias)) Py_RETURN_NONE;
     } else {
       c.seq_major = false;
     }
@@ -538,6 +622,58 @@ PyObject* py_forward(PyObject*, PyObject* const* a, Py_ssize_t n) {
   Tensor out = attend(c);
   if (!out.defined()) Py_RETURN_NONE;
   return THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
+// evoformer(q, k, v, biases, scale, gate): attention over the rows of [*, S, H, D] operands with biases broadcastable to
+// [*, H, S, S], as attention_variants.evoformer.attention_reference; None when the call is not of the plain kind.
+PyObject* py_evoformer(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  if (n != 6) {
+    PyErr_SetString(PyExc_TypeError, "evoformer takes 6 positional arguments");
+    return nullptr;
+  }
+  if (!g_api.fwd) Py_RETURN_NONE;
+  Call c;
+  if (!take_tensor(a[0], c.given_q) || !take_tensor(a[1], c.given_k) || !take_tensor(a[2], c.given_v) || mode_active()) Py_RETURN_NONE;
+  const Tensor &q = c.given_q, &k = c.given_k, &v = c.given_v;
+  if (q.dim() < 4 || k.sizes() != q.sizes() || v.sizes() != q.sizes()) Py_RETURN_NONE;
+  const size_t nl = (size_t)q.dim() - 3;
+  c.lead.assign(q.sizes().begin(), q.sizes().begin() + nl);
+  c.q = heads_first(q, nl);
+  c.k = heads_first(k, nl);
+  c.v = heads_first(v, nl);
+  c.seq_major = true;
+  if (!c.q.defined() || !c.k.defined() || !c.v.defined() || !operands_fit(c)) Py_RETURN_NONE;
+  c.scale = a[4] == Py_None ? 1.0 / std::sqrt((double)c.q.size(3)) : PyFloat_AsDouble(a[4]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  constexpr int64_t kInt = INT32_MAX;
+  if (c.q.size(0) > kInt || c.q.size(2) > kInt) Py_RETURN_NONE;
+  c.mask_kind = FL_MASK_NONE;
+  PyObject* biases = a[3];
+  if (!PyTuple_Check(biases) && !PyList_Check(biases)) Py_RETURN_NONE;
+  const Py_ssize_t nb = PySequence_Fast_GET_SIZE(biases);
+  if (nb > 2) Py_RETURN_NONE;
+  for (Py_ssize_t i = 0; i < nb; ++i) {
+    if (!take_tensor(PySequence_Fast_GET_ITEM(biases, i), c.given_bias[i])) Py_RETURN_NONE;
+    c.bias[i] = kernel_bias(c.given_bias[i], c.lead, c.q.size(1), c.q.size(2), c.bias_div[i]);
+    if (!c.bias[i].defined() || !bias_fits(c, (int)i)) Py_RETURN_NONE;
+  }
+  if (a[5] != Py_None) {
+    if (!take_tensor(a[5], c.given_gate) || c.given_gate.sizes() != v.sizes()) Py_RETURN_NONE;
+    c.gate = heads_first(c.given_gate, nl);
+    if (!c.gate.defined() || !gate_fits(c)) Py_RETURN_NONE;
+  }
+  const auto wants = [](const Tensor& t) { return t.defined() && t.requires_grad(); };
+  c.wants_grad = at::GradMode::is_enabled() && (wants(q) || wants(k) || wants(v) || wants(c.given_gate) || wants(c.given_bias[0]) ||
+                                                wants(c.given_bias[1]));
+  if (c.wants_grad && !shared_bias_gradients(c, c.given_bias)) Py_RETURN_NONE;
+  Tensor out = attend(c);
+  if (!out.defined()) Py_RETURN_NONE;
+  return THPVariable_Wrap(c.wants_grad ? std::move(out) : with_lead(out, c.lead));
   END_HANDLE_TH_ERRORS
 }
 
@@ -593,6 +729,7 @@ PyObject* py_bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 PyMethodDef kMethods[] = {
     {"forward", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_forward)), METH_FASTCALL, "Result of the call, or None when it is not of the plain kind."},
+    {"evoformer", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_evoformer)), METH_FASTCALL, "Result of an Evoformer call, or None when it is not of the plain kind."},
     {"key_chunks", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_key_chunks)), METH_FASTCALL, "Chunks the keys may be cut into, and whether they should be."},
     {"bind", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)(void)>(&py_bind)), METH_FASTCALL, "Takes the addresses of the C ABI's functions."},
     {nullptr, nullptr, 0, nullptr}};
