@@ -112,7 +112,11 @@ struct BwdTraits {
   static constexpr int SBYTES = (ROLE == ROLE_DKV) ? 1024 : 0;
   static constexpr int T1_OFF = 0, T2_OFF = 2 * TBYTES, O1_OFF = 4 * TBYTES, O2_OFF = O1_OFF + OBYTES,
                        S1_OFF = O2_OFF + OBYTES, S2_OFF = S1_OFF + 2 * SBYTES;
-  static constexpr int LDS_BYTES = S2_OFF + 2 * SBYTES;
+  // Document masks: the list of live tiles (up to LIST of them at a time, with one count per wave behind it) and, per slot, the ids
+  // of the streamed positions
+  static constexpr bool DOC = FEAT_ & F_DOC;
+  static constexpr int LIST = 1024, LIST_OFF = S2_OFF + 2 * SBYTES, IDS_OFF = LIST_OFF + (DOC ? LIST * 4 + 64 : 0);
+  static constexpr int LDS_BYTES = IDS_OFF + (DOC ? 2 * BT * 8 : 0);
   static_assert(QH == 1 || LDS_BYTES >= 4 * 64 * 64 * 4, "the partial sums of one accumulator set must fit in LDS");
   // two steps per turn of the loop, see there (the dK/dV kernel, 1 to 4 % slower with it, and bias operands have no registers for it)
   static constexpr bool UNROLL2 = ROLE == ROLE_DQ && !(FEAT_ & F_BIAS);
@@ -196,9 +200,13 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   }
   const int n_tiles = t_hi >= t_lo ? t_hi - t_lo + 1 : 0;
   const int n_heads = kDQ ? 1 : p.group;   // ROLE_DKV walks the query heads of its group
-  const int all_steps = n_tiles * n_heads;
-  const int s_first = SPLIT ? (int)((int64_t)all_steps * split / splits) : 0;
-  const int n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / splits) : all_steps;  // this workgroup's steps: [s_first, n_steps)
+  // this workgroup's steps: [s_first, n_steps) of all (under a document mask: of the live tiles of every query head, see below)
+  int s_first = 0, n_steps = n_tiles * n_heads;
+  const auto take_share = [&](int all_steps) FL_INLINE {
+    s_first = SPLIT ? (int)((int64_t)all_steps * split / splits) : 0;
+    n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / splits) : all_steps;
+  };
+  take_share(n_steps);
 
   // ---- per-lane constants ---------------------------------------------------------------------------------------------
   float cap_k1 = 0.f, cap_c = 0.f;
@@ -251,13 +259,12 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // needs would also wait for the tile transfers that are in flight for the next step.
   auto step_head = [&](int s) FL_INLINE { return kDQ ? ohead : kvh * p.group + s / n_tiles; };
   auto step_tile = [&](int s) FL_INLINE { return t_lo + (kDQ ? s : s % n_tiles); };
-  auto load_step = [&](int s, int slot) FL_INLINE {
-    const int t0 = step_tile(s) * BT, valid = min(BT, slen - t0);
+  auto load_tiles = [&](int tile, int hd, int slot) FL_INLINE {
+    const int t0 = tile * BT, valid = min(BT, slen - t0);
     if constexpr (kDQ) {
       load_tile(kptr + (int64_t)t0 * p.ks[2], p.ks[2], valid, T::T1_OFF + slot * T::TBYTES, T::T_PER_T);
       load_tile(vptr + (int64_t)t0 * p.vs[2], p.vs[2], valid, T::T2_OFF + slot * T::TBYTES, T::T_PER_T);
     } else {
-      const int hd = step_head(s);
       load_tile(p.q + (int64_t)batch * p.qs[0] + (int64_t)hd * p.qs[1] + (int64_t)t0 * p.qs[2], p.qs[2], valid,
                 T::T1_OFF + slot * T::TBYTES, T::T_PER_T);
       load_tile(p.dout + (int64_t)batch * p.dos[0] + (int64_t)hd * p.dos[1] + (int64_t)t0 * p.dos[2], p.dos[2], valid,
@@ -272,6 +279,18 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         dma4(uniform_ptr(p.lse + row0), off, (unsigned)(uintptr_t)smem + T::S1_OFF + slot * T::SBYTES);
         dma4(uniform_ptr(p.delta + row0), off, (unsigned)(uintptr_t)smem + T::S2_OFF + slot * T::SBYTES);
       }
+    }
+  };
+  auto load_step = [&](int s, int slot) FL_INLINE { load_tiles(step_tile(s), step_head(s), slot); };
+  // the ids of the streamed positions, for a step that compares them (positions past the end repeat the last one)
+  auto load_ids = [&](int tile, int slot) FL_INLINE {
+    const int t0 = tile * BT;
+    if (wave != T::NW - 1) return;
+#pragma unroll
+    for (int j = 0; j < BT / 32; ++j) {
+      const int word = 64 * j + lane;  // of the tile's ids, two words each
+      const unsigned off = (unsigned)(min(word / 2, slen - 1 - t0) * 8 + word % 2 * 4);
+      dma4(uniform_ptr(p.doc_ids + (int64_t)batch * p.doc_stride + t0), off, (unsigned)(uintptr_t)smem + T::IDS_OFF + slot * BT * 8 + j * 256);
     }
   };
 
@@ -312,7 +331,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       for (int i = 0; i < 16; ++i) acc2[db][i] = 0.f;
   }
 
-  if (n_steps > s_first) {
+  if (kDoc ? n_tiles > 0 : n_steps > s_first) {
     if constexpr (!kDQ) {
       const int valid = o1 - o0;
       load_tile(kptr + (int64_t)o0 * p.ks[2], p.ks[2], valid, T::O1_OFF, T::O_PER_T);
@@ -320,13 +339,11 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
   }
 
-  // Workgroup-level class of a step: nothing of its tile is attended by the workgroup's owner range (`skip`: document
+  // Workgroup-level class of a streamed tile: nothing of it is attended by the workgroup's owner range (returns true: document
   // ranges apart; positional emptiness inside [t_lo, t_hi] only occurs for a prefix-LM mask), everything is (`full`),
   // or every position of the tile and of the owner range carries one and the same document id (`doc_uniform`).
-  // Steps that are skipped are never transferred: the loop goes from one live step to the next (under a document mask
-  // most steps of the range are dead).
-  auto classify_step = [&](int s, bool& full, bool& doc_uniform) FL_INLINE -> bool {
-    const int t0 = step_tile(s) * BT;
+  auto classify_tile = [&](int tile, bool& full, bool& doc_uniform) FL_INLINE -> bool {
+    const int t0 = tile * BT;
     const int s1 = min(t0 + BT, slen);
     const int qa = kDQ ? o0 : t0, qb_ = kDQ ? o1 : s1, ka = kDQ ? t0 : o0, kb_ = kDQ ? s1 : o1;
     const int cls = classify_positional(p.mask_kind, qa, qb_, ka, kb_, p.window, p.prefix);
@@ -343,6 +360,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     return skip;
   };
+  auto classify_step = [&](int s, bool& full, bool& doc_uniform) FL_INLINE -> bool { return classify_tile(step_tile(s), full, doc_uniform); };
   // Sum of the bias operands at (query, key) of head `hd` (positions inside the sequences)
   auto bias_at = [&](int qpos, int kpos, int hd) FL_INLINE -> float {
     float b = 0.f;
@@ -358,9 +376,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     return b;
   };
   // One step: the tile in ring slot `slot` against the owner operands.
-  auto run_step = [&](int s, int slot, bool full, bool doc_uniform) FL_INLINE {
-    const int t0 = step_tile(s) * BT;
-    const int shead = step_head(s);  // the query head of this step
+  auto run_tile = [&](int tile, const int shead, int slot, bool full, bool doc_uniform) FL_INLINE {
+    const int t0 = tile * BT;
     {
       const unsigned t1 = T::T1_OFF + slot * T::TBYTES, t2 = T::T2_OFF + slot * T::TBYTES;
       // ---- X1 = T1 . O1^T, then the weights; X2 = T2 . O2^T, then dS (one after the other: the two fp32 tiles are
@@ -391,7 +408,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       auto attended = [&](int sbase, int off, int lo, int hi) FL_INLINE -> bool {
         bool ok = (off <= hi) & (off >= lo);
         if constexpr (kDoc) {
-          if (!doc_uniform) ok = ok & (p.doc_ids[(int64_t)batch * p.doc_stride + min(sbase + off, slen - 1)] == odoc);
+          if (!doc_uniform) ok = ok & (*reinterpret_cast<const int64_t*>(smem + T::IDS_OFF + slot * BT * 8 + (sbase - t0 + off) * 8) == odoc);
         }
         return ok;
       };
@@ -596,26 +613,69 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         }
     }
   };
+  auto run_step = [&](int s, int slot, bool full, bool doc_uniform) FL_INLINE { run_tile(step_tile(s), step_head(s), slot, full, doc_uniform); };
   if constexpr (kDoc) {
-    // (the class of a step is worked out before its transfers are issued: the table reads must not wait on them)
-    auto next_live = [&](int s, bool& full, bool& doc_uniform) FL_INLINE -> int {
-      while (s < n_steps && classify_step(s, full, doc_uniform)) ++s;
-      return s;
-    };
-    bool full = false, doc_uniform = false;
-    int s = next_live(s_first, full, doc_uniform);
-    if (s < n_steps) load_step(s, 0);
-    dma_wait<0>();
-    for (int slot = 0; s < n_steps; slot ^= 1) {
-      __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
-      bool full_next = false, doc_uniform_next = false;
-      const int s_next = next_live(s + 1, full_next, doc_uniform_next);
-      if (s_next < n_steps) load_step(s_next, slot ^ 1);
-      run_step(s, slot, full, doc_uniform);
+    // Most tiles of the range are dead: documents apart.  The live ones are listed first, a wave per LIST / NW tiles with their
+    // table reads in flight together; every head of the group then walks the list, and splits share out what is on it.  (Read one after
+    // the other as the loop got there, with two dependent table reads each, the dead tiles were most of the time: 2 x 32 over 8
+    // heads of 8037 positions in documents of up to 4000, head dim 64: 672 and 1503 us for the two roles, now 495 and 992.)
+    uint32_t* const list = reinterpret_cast<uint32_t*>(smem + T::LIST_OFF);
+    int* const counts = reinterpret_cast<int*>(smem + T::LIST_OFF + T::LIST * 4);
+    for (int w0 = t_lo; w0 <= t_hi; w0 += T::LIST) {
+      constexpr int PER = T::LIST / T::NW / 64;  // tiles per lane
+      const int mine = w0 + wave * (T::LIST / T::NW);
+      uint32_t entry[PER];
+      uint64_t live[PER];
+      int count = 0;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const int tile = mine + 64 * j + lane;
+        bool full = false, doc_uniform = false;
+        const bool skip = tile > t_hi || classify_tile(min(tile, t_hi), full, doc_uniform);
+        entry[j] = (uint32_t)tile << 2 | (full ? 1u : 0u) | (doc_uniform ? 2u : 0u);
+        live[j] = __builtin_amdgcn_ballot_w64(!skip);
+        count += __builtin_popcountll(live[j]);
+      }
+      __syncthreads();  // (the previous list has been walked)
+      if (lane == 0) counts[wave] = count;
+      __syncthreads();
+      int n_live = 0, at = 0;
+#pragma unroll
+      for (int w = 0; w < T::NW; ++w) {
+        const int c = __builtin_amdgcn_readfirstlane(counts[w]);
+        at += w < wave ? c : 0;
+        n_live += c;
+      }
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        if ((live[j] >> lane) & 1) list[at + __builtin_popcountll(live[j] & ((1ull << lane) - 1))] = entry[j];
+        at += __builtin_popcountll(live[j]);
+      }
+      __syncthreads();
+      take_share(n_live * n_heads);
+      if (s_first >= n_steps) continue;
+      int head = kDQ ? ohead : kvh * p.group + s_first / n_live, i = s_first % n_live;
+      auto at_list = [&](int i) FL_INLINE { return (uint32_t)__builtin_amdgcn_readfirstlane((int)list[i]); };
+      uint32_t e = at_list(i);
+      load_tiles((int)(e >> 2), head, 0);
+      if (!(e & 2)) load_ids((int)(e >> 2), 0);
       dma_wait<0>();
-      s = s_next;
-      full = full_next;
-      doc_uniform = doc_uniform_next;
+      for (int s = s_first, slot = 0; s < n_steps; ++s, slot ^= 1) {
+        __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
+        const uint32_t now = e;
+        const int head_now = head;
+        if (s + 1 < n_steps) {
+          if (++i == n_live) {
+            i = 0;
+            ++head;
+          }
+          e = at_list(i);
+          load_tiles((int)(e >> 2), head, slot ^ 1);
+          if (!(e & 2)) load_ids((int)(e >> 2), slot ^ 1);
+        }
+        run_tile((int)(now >> 2), head_now, slot, now & 1, now & 2);
+        dma_wait<0>();
+      }
     }
   } else {
     // positional masks: every step of [t_lo, t_hi] is visited (a dead one only occurs under a prefix-LM mask)
