@@ -118,12 +118,56 @@ struct BwdTraits {
   static constexpr int LIST = 1024, LIST_OFF = S2_OFF + 2 * SBYTES, IDS_OFF = LIST_OFF + (DOC ? LIST * 4 + 64 : 0);
   static constexpr int LDS_BYTES = IDS_OFF + (DOC ? 2 * BT * 8 : 0);
   static_assert(QH == 1 || LDS_BYTES >= 4 * 64 * 64 * 4, "the partial sums of one accumulator set must fit in LDS");
-  // two steps per turn of the loop, see there (the dK/dV kernel, 1 to 4 % slower with it, and bias operands have no registers for it)
-  static constexpr bool UNROLL2 = ROLE == ROLE_DQ && !(FEAT_ & F_BIAS);
+  // Calls without score modifications: the LDS addresses of the operand reads stay in registers (24 at head dim 128; worked out
+  // where they are used they were a third of the vector instructions), and the order of reads, products and vector work is
+  // prescribed (sched_scores, sched_gradients).  4 x 16 x 4096, unmasked / causal, us: head dim 128, dQ 744 / 398 -> 695 / 380, dK and
+  // dV 1187 / 644 -> 1095 / 630; head dim 64, dQ 435 / 235 -> 385 / 204; dK and dV there are the slower for it (581 / 311 -> 626 / 332:
+  // two blocks per step leave less room).
+  static constexpr bool TUNED = (FEAT_ == 0 && D_ > 64) || ((FEAT_ & ~F_DOC) == 0 && D_ == 64 && ROLE_ == ROLE_DQ);
+  // ROLE_DQ: dP's accumulators start from a tile of -Delta that stays in registers, where there is room for it
+  static constexpr bool DELTA_TILE = ROLE_ == ROLE_DQ && (TUNED || (D_ <= 64 && !(FEAT_ & (F_BIAS | F_DROPOUT))));
+  // two steps per turn of the loop, see there (without addresses in registers the dK/dV kernel is 1 to 4 % slower with it; bias
+  // operands have no registers for it)
+  static constexpr bool UNROLL2 = (ROLE == ROLE_DQ || TUNED) && !(FEAT_ & F_BIAS);
   static constexpr int WAVES_PER_EU = 2;
   static constexpr bool WIDE_X2 = D_ > 64;                      // dP's fp32 tile declared next to S's
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
 };
+
+// The order of a step's instructions (T::TUNED): N times M products, each followed by R LDS reads and V vector instructions.
+template <int N, int M, int R, int V>
+__device__ __forceinline__ void sched_run() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(SG_MFMA, M, 0);
+    if constexpr (R > 0) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, R, 0);
+    if constexpr (V > 0) __builtin_amdgcn_sched_group_barrier(SG_VALU | SG_TRANS, V, 0);
+  }
+}
+// X1's products, their operands read two k-steps ahead (left to itself the compiler waits for the two reads in front of every one)
+template <int KS, int TB, bool DQ>
+__device__ __forceinline__ void sched_scores() {
+  constexpr int R = TB + (DQ ? 0 : 1), A = 2;
+  __builtin_amdgcn_sched_group_barrier(SG_DS_READ, A * R, 0);
+  sched_run<KS - A, TB, R, 0>();
+  sched_run<A, TB, 0, 0>();
+}
+// X2's products with the weights' vector work under them, then (ROLE_DKV) dV's with dS's, then those of dS
+template <int KS, int TB, int DB, bool DQ>
+__device__ __forceinline__ void sched_gradients() {
+  constexpr int R = TB + (DQ ? 0 : 1), A = 2, NA = 2 * TB * DB, PA = 2;
+  __builtin_amdgcn_sched_group_barrier(SG_DS_READ, (DQ ? 0 : 8 * TB) + A * R, 0);
+  sched_run<KS - A, TB, R, 32 * TB / KS>();
+  sched_run<A, TB, 2 * PA / A, 32 * TB / KS>();
+  if constexpr (DQ) {
+    __builtin_amdgcn_sched_group_barrier(SG_VALU, 24 * TB, 0);
+  } else {
+    __builtin_amdgcn_sched_group_barrier(SG_VALU, 8 * TB, 0);
+    sched_run<NA, 1, 2, 12 / DB>();
+  }
+  sched_run<NA - PA, 1, 2, 0>();
+  sched_run<PA, 1, 0, 0>();
+}
 
 // One workgroup's share of the work of a role: workgroup `block` of tiles * splits.  SPLIT: several workgroups per owner tile
 // (one at run time is fine), compiled apart: with the second epilogue in it the dK/dV kernel at head dim 128 is 4 %
@@ -200,13 +244,9 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   }
   const int n_tiles = t_hi >= t_lo ? t_hi - t_lo + 1 : 0;
   const int n_heads = kDQ ? 1 : p.group;   // ROLE_DKV walks the query heads of its group
-  // this workgroup's steps: [s_first, n_steps) of all (under a document mask: of the live tiles of every query head, see below)
-  int s_first = 0, n_steps = n_tiles * n_heads;
-  const auto take_share = [&](int all_steps) FL_INLINE {
-    s_first = SPLIT ? (int)((int64_t)all_steps * split / splits) : 0;
-    n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / splits) : all_steps;
-  };
-  take_share(n_steps);
+  const int all_steps = n_tiles * n_heads;
+  const int s_first = SPLIT ? (int)((int64_t)all_steps * split / splits) : 0;
+  const int n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / splits) : all_steps;  // this workgroup's steps: [s_first, n_steps)
 
   // ---- per-lane constants ---------------------------------------------------------------------------------------------
   float cap_k1 = 0.f, cap_c = 0.f;
@@ -295,23 +335,60 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   };
 
   // ---- LDS operand reads --------------------------------------------------------------------------------------------------
-  // row-wise: 8 consecutive elements [row][16 ks + 8 h, +8) (A operand of X1/X2 from a streamed tile, or B operand from
-  // an owner tile)
-  auto frag_row = [&](unsigned tile_off, int row, int ks) FL_INLINE -> ex8 {
-    return *reinterpret_cast<const ex8*>(smem + tile_off + row * (D * 2) + L::swz_kv(row, 2 * ks + h) * 16);
+  // The addresses of the k-steps (and of the column blocks) differ in swizzled bits, those of tiles, slots and blocks of rows by
+  // constants.  TUNED: held in registers (the empty asm keeps the compiler from working them out again at every read).
+  constexpr int RB = D * 2;  // bytes per row
+  unsigned a_row[KS], a_own[KS], a_tr[2][DB];
+  if constexpr (T::TUNED) {
+    const unsigned lds0 = (unsigned)(uintptr_t)smem;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      a_row[ks] = lds0 + (qh * TB * 32 + r) * RB + L::swz_kv(r, 2 * ks + h) * 16;
+      asm volatile("" : "+v"(a_row[ks]));
+      if constexpr (!kDQ) {
+        a_own[ks] = lds0 + T::O1_OFF + (ow * 32 + r) * RB + L::swz_kv(r, 2 * ks + h) * 16;
+        asm volatile("" : "+v"(a_own[ks]));
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int db = 0; db < DB; ++db) {
+        const int i16 = lane % 16, row = 8 * j + 4 * h + i16 / 4, col = db * 32 + (lane / 16) % 2 * 16 + 4 * (i16 % 4);
+        a_tr[j][db] = lds0 + (qh * TB * 32 + row) * RB + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
+        asm volatile("" : "+v"(a_tr[j][db]));
+      }
+  }
+  typedef __attribute__((address_space(3))) const ex8* lds_ex8_ptr;
+  typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
+  // row-wise: 8 consecutive elements [row][16 ks + 8 h, +8), row = 32 (qh TB + sb) + r of a streamed tile (A operand of X1/X2) or this
+  // lane's row of an owner tile (B operand)
+  auto frag_row = [&](unsigned tile_off, int sb, int ks) FL_INLINE -> ex8 {
+    if constexpr (T::TUNED) return *(lds_ex8_ptr)(a_row[ks] + tile_off + sb * 32 * RB);
+    const int row = (qh * TB + sb) * 32 + r;
+    return *reinterpret_cast<const ex8*>(smem + tile_off + row * RB + L::swz_kv(row, 2 * ks + h) * 16);
   };
-  // transposing: A operand of the accumulating products for 16-position chunk c and column block db; slot j of lane
+  auto frag_own = [&](unsigned tile_off, int ks) FL_INLINE -> ex8 {
+    if constexpr (T::TUNED) return *(lds_ex8_ptr)(a_own[ks] + (tile_off - T::O1_OFF));
+    const int row = ow * 32 + r;
+    return *reinterpret_cast<const ex8*>(smem + tile_off + row * RB + L::swz_kv(row, 2 * ks + h) * 16);
+  };
+  // transposing: A operand of the accumulating products for 16-position chunk c (of this wave's) and column block db; slot j of lane
   // (r, h) is streamed position 16 c + 8 (j / 4) + 4 h + j % 4, the order in which the weights are packed
   auto frag_tr = [&](unsigned tile_off, int c, int db) FL_INLINE -> ex8 {
     ex8 f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const int i16 = lane % 16, g = (lane / 16) % 2;
-      const int row = 16 * c + 8 * j + 4 * h + i16 / 4;
-      const int col = db * 32 + g * 16 + 4 * (i16 % 4);
-      const unsigned char* ap = smem + tile_off + row * (D * 2) + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
-      typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
-      const s16x4 t4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ap));
+      s16x4 t4;
+      if constexpr (T::TUNED) {
+        t4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j][db] + tile_off + c * 16 * RB));
+      } else {
+        const int i16 = lane % 16, g = (lane / 16) % 2;
+        const int row = 16 * (2 * TB * qh + c) + 8 * j + 4 * h + i16 / 4;
+        const int col = db * 32 + g * 16 + 4 * (i16 % 4);
+        const unsigned char* ap = smem + tile_off + row * RB + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
+        t4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ap));
+      }
       const ex4 b4 = __builtin_bit_cast(ex4, t4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
@@ -319,6 +396,14 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     return f;
   };
 
+  // -Delta of this lane's row, as the tile that dP's accumulators start from (the asm keeps it in registers: copied into the
+  // accumulators on every step it would cost what it saves)
+  f32x16 delta_tile;
+  if constexpr (T::DELTA_TILE) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) delta_tile[i] = delta_o;
+    asm volatile("" : "+v"(delta_tile));
+  }
   f32x16 acc1[DB], acc2[kDQ ? 1 : DB];
 #pragma unroll
   for (int db = 0; db < DB; ++db)
@@ -414,16 +499,22 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       };
       // (document ids beside bias operands: the mask goes with each weight, sixteen ids in flight do not fit in the registers)
       constexpr bool kMaskApart = !(kDoc && kBias);
+      constexpr bool kMaskScores = FEAT == 0 || (FEAT == F_DOC && D <= 64);
+      constexpr bool kSched = T::TUNED;
       // X2 = T2 . O2^T (dP).  At D = 128 its fp32 tile is declared out here, next to X1's, and (ROLE_DQ) its MFMAs are issued
       // right after X1's, before the weights' vector work; at D = 64 it lives in the block that consumes it.  Both choices
       // are measured: the first is 15 % faster at D = 128 and 1-2 % slower at D = 64.
       f32x16 x2_wide[TB];
-      // dP's accumulators start from zero, or (ROLE_DKV without dropout) from the staged -Delta of their rows, which saves
-      // the subtraction per score later
-      constexpr bool kDeltaInit = !kDQ && !kDrop;
+      // dP's accumulators start from zero, or (without dropout) from the -Delta of their rows, staged or (ROLE_DQ) this lane's, which
+      // saves the subtraction per score later
+      constexpr bool kDeltaInit = !kDrop && (!kDQ || T::DELTA_TILE);
       auto init_x2 = [&](f32x16 (&x2)[TB]) FL_INLINE {
 #pragma unroll
-        for (int sb = 0; sb < TB; ++sb)
+        for (int sb = 0; sb < TB; ++sb) {
+          if constexpr (T::DELTA_TILE) {
+            x2[sb] = delta_tile;
+            continue;
+          }
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
             f32x4 nd = {0.f, 0.f, 0.f, 0.f};
@@ -431,16 +522,17 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 #pragma unroll
             for (int e = 0; e < 4; ++e) x2[sb][4 * g + e] = nd[e];
           }
+        }
       };
       auto second_product = [&](f32x16 (&x2)[TB]) FL_INLINE {
         init_x2(x2);
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           ex8 b2;
-          if constexpr (kDQ) b2 = o2f[ks]; else b2 = frag_row(T::O2_OFF, ow * 32 + r, ks);
+          if constexpr (kDQ) b2 = o2f[ks]; else b2 = frag_own(T::O2_OFF, ks);
 #pragma unroll
           for (int sb = 0; sb < TB; ++sb)
-            x2[sb] = mfma32(frag_row(t2, (qh * TB + sb) * 32 + r, ks), b2, x2[sb]);
+            x2[sb] = mfma32(frag_row(t2, sb, ks), b2, x2[sb]);
         }
       };
       ex8 pf[2 * TB], dsf[2 * TB];
@@ -462,10 +554,26 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           ex8 b1;
-          if constexpr (kDQ) b1 = o1f[ks]; else b1 = frag_row(T::O1_OFF, ow * 32 + r, ks);
+          if constexpr (kDQ) b1 = o1f[ks]; else b1 = frag_own(T::O1_OFF, ks);
 #pragma unroll
           for (int sb = 0; sb < TB; ++sb)
-            x1[sb] = mfma32(frag_row(t1, (qh * TB + sb) * 32 + r, ks), b1, x1[sb]);
+            x1[sb] = mfma32(frag_row(t1, sb, ks), b1, x1[sb]);
+        }
+        if constexpr (kSched) sched_scores<KS, TB, kDQ>();
+        if constexpr (kMaskScores) {
+          if (!full) {  // workgroup-uniform; here, so that everything from the weights on is one block to be ordered
+#pragma unroll
+            for (int sb = 0; sb < TB; ++sb) {
+              const int sbase = t0 + 32 * (qh * TB + sb) + 4 * h;
+              int lo, hi;
+              bounds(sbase, lo, hi);
+              asm volatile("" : "+v"(lo), "+v"(hi));
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                if (!attended(sbase, 8 * (i / 4) + i % 4, lo, hi)) x1[sb][i] = -INFINITY;
+              }
+            }
+          }
         }
         // where the registers allow and it pays (measured), dP's MFMAs are issued before the weights' vector work
         if constexpr (T::EARLY_X2) second_product(x2_wide);
@@ -516,8 +624,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 #pragma unroll
         for (int sb = 0; sb < TB; ++sb) {
           const int sbase = t0 + 32 * (qh * TB + sb) + 4 * h;
-          if (kMaskApart && !full) {  // workgroup-uniform
-            // (the asm keeps this a branch: as selects it was three vector and two scalar instructions per score on every step,
+          if (kMaskApart && !kMaskScores && !full) {  // workgroup-uniform
+            // (where -inf would not do as a score: under the soft-cap.  The asm keeps this a branch: as selects it was three vector and two scalar instructions per score on every step,
             // full ones included, beside the four that make a weight and its gradient.  It stands behind the products that
             // do not need it, which the compiler can then interleave.  Gradients of 4 x 16 x 4096, this and the unrolled
             // dQ loop: head dim 128 unmasked 2.00 -> 1.85 ms, causal 1.10 -> 1.01; head dim 64 1.135 -> 0.985, 0.62 -> 0.545)
@@ -566,10 +674,10 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 #pragma unroll
           for (int ks = 0; ks < KS; ++ks) {
             ex8 b2;
-            if constexpr (kDQ) b2 = o2f[ks]; else b2 = frag_row(T::O2_OFF, ow * 32 + r, ks);
+            if constexpr (kDQ) b2 = o2f[ks]; else b2 = frag_own(T::O2_OFF, ks);
 #pragma unroll
             for (int sb = 0; sb < TB; ++sb)
-              x2[sb] = mfma32(frag_row(t2, (qh * TB + sb) * 32 + r, ks), b2, x2[sb]);
+              x2[sb] = mfma32(frag_row(t2, sb, ks), b2, x2[sb]);
           }
         }
 #pragma unroll
@@ -603,14 +711,20 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         }
       }
       // ---- acc1 += T1^T . dS,  acc2 += T2^T . P -------------------------------------------------------------------------------
+      if constexpr (!kDQ && kMaskScores) {  // (dV first: its products cover the vector work that forms dS)
+#pragma unroll
+        for (int c = 0; c < 2 * TB; ++c)
+#pragma unroll
+          for (int db = 0; db < DB; ++db) acc2[db] = mfma32(frag_tr(t2, c, db), pf[c], acc2[db]);
+      }
 #pragma unroll
       for (int c = 0; c < 2 * TB; ++c)
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
-          acc1[db] = mfma32(frag_tr(t1, 2 * TB * qh + c, db), dsf[c], acc1[db]);
-          if constexpr (!kDQ)
-            acc2[db] = mfma32(frag_tr(t2, 2 * TB * qh + c, db), pf[c], acc2[db]);
+          acc1[db] = mfma32(frag_tr(t1, c, db), dsf[c], acc1[db]);
+          if constexpr (!kDQ && !kMaskScores) acc2[db] = mfma32(frag_tr(t2, c, db), pf[c], acc2[db]);
         }
+      if constexpr (kSched) sched_gradients<KS, TB, DB, kDQ>();
     }
   };
   auto run_step = [&](int s, int slot, bool full, bool doc_uniform) FL_INLINE { run_tile(step_tile(s), step_head(s), slot, full, doc_uniform); };
@@ -652,7 +766,9 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         at += __builtin_popcountll(live[j]);
       }
       __syncthreads();
-      take_share(n_live * n_heads);
+      const int all_live = n_live * n_heads;
+      const int s_first = SPLIT ? (int)((int64_t)all_live * split / splits) : 0;
+      const int n_steps = SPLIT ? (int)((int64_t)all_live * (split + 1) / splits) : all_live;
       if (s_first >= n_steps) continue;
       int head = kDQ ? ohead : kvh * p.group + s_first / n_live, i = s_first % n_live;
       auto at_list = [&](int i) FL_INLINE { return (uint32_t)__builtin_amdgcn_readfirstlane((int)list[i]); };
