@@ -191,18 +191,24 @@ __device__ __forceinline__ int64_t uniform_i64(int64_t x) {
   return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)x) |
                    ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)x >> 32)) << 32));
 }
+// NOPS: idle cycles between the write of m0 and the transfer, less one.  The transfer reads gbase_uniform five wait states or more
+// after a vector instruction that wrote it (v_readfirstlane, or the v_readlane that brings back a spilled scalar register); the compiler
+// keeps that distance for instructions it knows, not for an asm.  3 keeps it whatever comes before; with 0 it is up to the kernel,
+// whose addresses are then made by scalar instructions or far ahead.
+template <int NOPS = 0>
 __device__ __forceinline__ void dma16(uint64_t gbase_uniform, unsigned voff, unsigned lds_base) {
   const unsigned lds_base_uniform = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_base);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(gbase_uniform), "v"(voff),
-               "s"(lds_base_uniform)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop %3\n\tglobal_load_lds_dwordx4 %1, %0" ::"s"(gbase_uniform), "v"(voff),
+               "s"(lds_base_uniform), "n"(NOPS)
                : "m0");
 }
 
 // The same with 4 bytes per lane (lane l writes LDS bytes [4 l, 4 l + 4)): for fp32 rows whose start is only 4-byte aligned.
+template <int NOPS = 0>
 __device__ __forceinline__ void dma4(uint64_t gbase_uniform, unsigned voff, unsigned lds_base) {
   const unsigned lds_base_uniform = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_base);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" ::"s"(gbase_uniform), "v"(voff),
-               "s"(lds_base_uniform)
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop %3\n\tglobal_load_lds_dword %1, %0" ::"s"(gbase_uniform), "v"(voff),
+               "s"(lds_base_uniform), "n"(NOPS)
                : "m0");
 }
 
@@ -747,16 +753,16 @@ void fwd_kernel(const KParams p) {
           const int last_chunk = (min(p.Lk - t * BN, BN)) / 8 - 1;
           if (row_f32) {
             const int last4 = (min(p.Lk - t * BN, BN)) / 4 - 1;
-            dma16(uniform_ptr(rptr + (int64_t)t * BN * 2), (unsigned)min(lane % (BN / 4), last4) * 16u, lds_r + slot * T::RBYTES);
+            dma16<3>(uniform_ptr(rptr + (int64_t)t * BN * 2), (unsigned)min(lane % (BN / 4), last4) * 16u, lds_r + slot * T::RBYTES);
           } else {
-            dma16(uniform_ptr(rptr + (int64_t)t * BN), (unsigned)min(lane % LB::CPR, last_chunk) * 16u, lds_r + slot * T::RBYTES);
+            dma16<3>(uniform_ptr(rptr + (int64_t)t * BN), (unsigned)min(lane % LB::CPR, last_chunk) * 16u, lds_r + slot * T::RBYTES);
           }
         }
         if (!stage_bias) return;
         const uint64_t base = uniform_ptr(bptr + (int64_t)t * BN);
         if (t * BN + BN <= p.Lk) {
 #pragma unroll
-          for (int it = 0; it < T::B_PER_T; ++it) dma16(base, boff[it], lds_b + slot * T::BBYTES + it * 1024);
+          for (int it = 0; it < T::B_PER_T; ++it) dma16<3>(base, boff[it], lds_b + slot * T::BBYTES + it * 1024);
         } else {
           const int last_chunk = (p.Lk - t * BN) / 8 - 1;  // Lk % 8 == 0 whenever a bias is staged
 #pragma unroll
@@ -764,7 +770,7 @@ void fwd_kernel(const KParams p) {
             const int id = it * 64 + lane, row = id / LB::CPR, pc = id % LB::CPR;
             const unsigned off =
                 (unsigned)(min(qw0 + row, p.Lq - 1) * (int)p.bs[nbl][2] + min(LB::swz(row, pc), last_chunk) * 8) * 2u;
-            dma16(base, off, lds_b + slot * T::BBYTES + it * 1024);
+            dma16<3>(base, off, lds_b + slot * T::BBYTES + it * 1024);
           }
         }
       }

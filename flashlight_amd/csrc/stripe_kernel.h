@@ -69,12 +69,13 @@ struct StripeTraits {
   static constexpr int PER_CU = 8 / NW < 160 * 1024 / LDS_BYTES ? 8 / NW : 160 * 1024 / LDS_BYTES;
 };
 
-// stores that the waits count (see pairbias_kernel.h: the idle cycles are part of a 16-byte store written as asm)
+// stores that the waits count.  As asm they bring the distances that the compiler keeps for its own: five wait states behind a vector
+// instruction that wrote the scalar address (see dma16), and two behind a store of more than 8 bytes, which still reads its data
 __device__ __forceinline__ void stripe_store16(uint64_t sbase, unsigned voff, u32x4 data) {
-  asm volatile("global_store_dwordx4 %0, %1, %2\n\ts_nop 1" ::"v"(voff), "v"(data), "s"(sbase) : "memory");
+  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2\n\ts_nop 1" ::"v"(voff), "v"(data), "s"(sbase) : "memory");
 }
 __device__ __forceinline__ void stripe_store4(uint64_t sbase, unsigned voff, float data) {
-  asm volatile("global_store_dword %0, %1, %2" ::"v"(voff), "v"(data), "s"(sbase) : "memory");
+  asm volatile("s_nop 4\n\tglobal_store_dword %0, %1, %2" ::"v"(voff), "v"(data), "s"(sbase) : "memory");
 }
 
 template <class T>
@@ -130,9 +131,9 @@ void stripe_kernel(const StripeParams p) {
   auto load_keys = [&](uint64_t ka, uint64_t va, int slot) FL_INLINE {
     const unsigned mine = lds0 + slot * slot_bytes + wave * T::W_BYTES;
 #pragma unroll
-    for (int it = 0; it < T::TPW; ++it) dma16(ka, koff[it], mine + it * 1024);
+    for (int it = 0; it < T::TPW; ++it) dma16<3>(ka, koff[it], mine + it * 1024);
 #pragma unroll
-    for (int it = 0; it < T::TPW; ++it) dma16(va, voff[it], mine + T::T_BYTES + it * 1024);
+    for (int it = 0; it < T::TPW; ++it) dma16<3>(va, voff[it], mine + T::T_BYTES + it * 1024);
   };
   constexpr int QPW = (T::QT + NW - 1) / NW;  // of the stripe's queries, shared out over the waves
   unsigned qoff[QPW];
@@ -142,7 +143,7 @@ void stripe_kernel(const StripeParams p) {
     const unsigned q_at = lds0 + slot * slot_bytes + w_bytes;
 #pragma unroll
     for (int j = 0; j < QPW; ++j)
-      if ((j + 1) * NW <= T::QT || j * NW + wave < T::QT) dma16(qa, qoff[j], q_at + (j * NW + wave) * 1024);
+      if ((j + 1) * NW <= T::QT || j * NW + wave < T::QT) dma16<3>(qa, qoff[j], q_at + (j * NW + wave) * 1024);
     load_keys(ka, va, slot);
     qa += qstep;
     ka += kstep;
