@@ -618,6 +618,25 @@ bool bias_stageable(const fl_attn_params* p, int nb) {
          st[1] % 8 == 0 && st[2] % 8 == 0 && ((int64_t)p->Lq * st[2] + p->Lk) * 4 < ((int64_t)1 << 31);
 }
 
+// Into how many chunks the `div` batch entries that share a bias are cut.  A chunk of one head and one group of entries is `tiles`
+// workgroups, which stay on one of the 8 XCDs; `per_cu` of them run at once on each of its 32 compute units.  Taken is the number with
+// the fewest rounds times what a round takes: the entries of a chunk, and a start worth two and a half of them.  (Gradients, both
+// roles, us: 128 x 8 x 256 x 256, head dim 32: 4 chunks in one round 83, 8 in two 92; 65 x 4 x 384 x 384, 64: 2 chunks in one round
+// 125, 5 in three 156, 10 in four 125; 256 x 8 x 384 x 384, 32: 1 chunk 707, 2 chunks 670, 5 chunks 550.)
+int64_t chunks_of_entries(int64_t heads_and_groups, int64_t tiles, int per_cu, int64_t div) {
+  int64_t best = 1;
+  double least = 0;
+  for (int64_t c = 1; c <= div && (c == 1 || c * heads_and_groups * tiles <= 4 * 256 * per_cu); ++c) {
+    const int64_t rounds = ((heads_and_groups * c + 7) / 8 * tiles + 32 * per_cu - 1) / (32 * per_cu);
+    const double t = (double)rounds * ((double)((div + c - 1) / c) + 2.5);
+    if (c == 1 || t < least) {
+      least = t;
+      best = c;
+    }
+  }
+  return best;
+}
+
 // Whether *p (already validated) is a call the shared-bias stripe forward (stripe_kernel.h) takes.  Fills the kernel's parameters,
 // its wave count, and the number of workgroups and their LDS bytes.
 bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, int* waves, int64_t (&launch)[2]) {
@@ -689,9 +708,7 @@ bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, 
   // weight exact; here the whole row's maximum, at 6 to 20 % of the time)
   k.by_maximum = p->Lk % 64 != 0;
   k.tiles = (p->Lq + 32 * shape.qb - 1) / (32 * shape.qb);
-  // entries per workgroup: as many as leave one round of workgroups
-  const int64_t units = (int64_t)k.groups * k.H * k.tiles;
-  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(k.div, 256 * shape.per_cu / units));
+  const int64_t units = (int64_t)k.groups * k.H * k.tiles, most = chunks_of_entries((int64_t)k.groups * k.H, k.tiles, shape.per_cu, k.div);
   k.chunk_len = (int)((k.div + most - 1) / most);
   k.chunks = (k.div + k.chunk_len - 1) / k.chunk_len;
   if (units * k.chunks > (1 << 28)) return false;
@@ -848,9 +865,9 @@ bool plan_shared_bias_bwd(const fl_attn_params* p, SBScratch* out) {
     if (st[2] < 0 || st[2] >= (1 << 20)) return false;
   if ((int64_t)p->Hq * p->Dv >= (1 << 20)) return false;  // (of a result, and of the gated output gradient, in sequence-major order)
   const int64_t S = p->Lk, H = p->Hq, div = p->bias_batch_div[x.dense], groups = p->B / div, tiles = (S + 31) / 32;
-  // entries per workgroup: as many as leave one round of workgroups
+  // (both roles run in one launch)
   const int per_cu = fl::pairbias_bwd_shape(p->Dqk, (int)S).lds_bytes <= 80 * 1024 ? 2 : 1;
-  int64_t chunks = std::max<int64_t>(1, std::min<int64_t>(div, 256 * per_cu / (groups * H * tiles)));
+  int64_t chunks = chunks_of_entries(groups * H, 2 * tiles, per_cu, div);
   const int64_t len = (div + chunks - 1) / chunks;
   chunks = (div + len - 1) / len;
   if (groups * chunks * H * tiles > (1 << 28)) return false;
@@ -1431,7 +1448,6 @@ int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* strea
   sp.scale_log2 = p->scale * 1.4426950408889634f;
   sp.dbias_part = b->dbias ? reinterpret_cast<float*>(ws + x.part) : nullptr;
   const fl::SBShape shape = fl::pairbias_bwd_shape(p->Dqk, sp.S);
-  sp.slots = shape.slots;
   e = (f16 ? fl::launch_pairbias_bwd_f16 : fl::launch_pairbias_bwd_bf16)(p->Dqk, shape, sp, stream);
   if (e != hipSuccess) return fail((int)e, "shared-bias backward: launch failed: %s", hipGetErrorString(e));
   if (b->dbias) {

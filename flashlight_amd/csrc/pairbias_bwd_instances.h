@@ -6,19 +6,18 @@
 
 namespace fl {
 struct SBShape {
-  int nb, waves, slots, lds_bytes;  // 32-row blocks per wave, waves, resident batch entries
+  int nb, waves, lds_bytes;  // 32-row blocks per wave, waves
 };
 // Eight waves fill a compute unit's registers.  Up to 256 positions of head dim 32 two workgroups of four waves share it
 // (two resident entries each, 79 KB); head dim 64 takes one workgroup of up to eight; longer sequences two blocks per wave.
 // Two entries stay resident where they fit.
-inline SBShape pairbias_bwd_shape(int d, int s) {
+constexpr SBShape pairbias_bwd_shape(int d, int s) {
   const int blocks = (s + 31) / 32;
-  SBShape x;
+  SBShape x{};
   x.nb = blocks <= 4 ? 1 : blocks <= 8 ? (d == 32 ? 2 : 1) : 2;
   x.waves = (blocks + x.nb - 1) / x.nb;
   const int slot = x.waves * (x.nb * 128 * d + 512) + 128 * d + 512;
-  x.slots = 2 * slot <= 160 * 1024 ? 2 : 1;
-  x.lds_bytes = x.slots * slot;
+  x.lds_bytes = (2 * slot <= 160 * 1024 ? 2 : 1) * slot;
   return x;
 }
 hipError_t launch_pairbias_bwd_bf16(int d, const SBShape& shape, const SBParams& p, hipStream_t stream);

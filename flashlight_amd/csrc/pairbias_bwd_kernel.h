@@ -17,12 +17,13 @@
 // on their way while one is worked on.  The sequence has at most 512 positions.
 //
 // Measured, 128 x 8 x 256 x 256, head dim 32, mask row and gate, bf16, whole step: 852 -> 168 us (ROLE_DQ 325 -> 46, ROLE_DKV
-// 232 -> 56, row sums and gate 150 -> 16, clearing and summing the bias gradient 97 -> 4).  Per score ten vector
-// instructions are left (27 and 21 per MFMA; seven make the weight and its gradient, the rest operands and the sums over the
-// waves), and no global load, conversion or store; what bounds the roles now is the chain an entry goes through (tiles, two
-// products, weights, products, sums over the waves: 2.1 and 2.7 us) with two waves per SIMD to cover it: the vector unit takes
-// an instruction in 40 and 36 % of the cycles (SQ_ACTIVE_INST_VALU).  Two blocks per wave in four waves beat one in eight (67
-// and 93 us: the sums over the waves cost more than the occupancy gains).
+// 232 -> 56, row sums and gate 150 -> 16, clearing and summing the bias gradient 97 -> 4), then both roles in one launch, wave counts
+// compiled in (the sums over a run-time count were loops) and waits that leave the stores outstanding: 103 -> 83; 2 x 230 x 4 x 192 x
+// 192: 139 -> 107; 65 x 4 x 384 x 384, head dim 64: 244 -> 119; 256 x 8 x 384 x 384: 811 -> 545.  Per score ten vector
+// instructions are left (seven make the weight and its gradient, the rest operands and the sums over the waves), and no global
+// load, conversion or store; what bounds the roles is the chain an entry goes through (tiles, two products, weights, products, sums
+// over the waves) with two waves per SIMD to cover it.  Two blocks per wave in four waves beat one in eight (67 and 93 us for the two
+// roles against 46 and 56: the sums over the waves cost more than the occupancy gains).
 #pragma once
 #include "fwd_kernel.h"
 
@@ -41,17 +42,16 @@ struct SBParams {
   int32_t B, H, S;
   int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
   int32_t tiles;                   // 32-row stripes
-  int32_t slots;                   // tiles of batch entries resident in LDS: 2, or 1 where two do not fit
   int32_t s_pad;                   // row length of the partial bias gradient (S rounded up to 4)
   float scale, scale_log2;
   float* dbias_part;               // [groups][chunks][H][S][s_pad], or null: no gradient of the bias wanted
 };
 
 // rows of an operand that are not in the sequence repeat the last one; their weights are 0 (their bias is -inf)
-template <int D_, int ROLE_, int NB_, bool ROWB_, class Elem_>
+template <int D_, int ROLE_, int NB_, int NW_, bool ROWB_, class Elem_>
 struct SBTraits {
   using Elem = Elem_;
-  static constexpr int D = D_, ROLE = ROLE_, NB = NB_;
+  static constexpr int D = D_, ROLE = ROLE_, NB = NB_, NW = NW_;
   static constexpr bool ROWB = ROWB_, DQ = ROLE_ == 0;
   static constexpr int KS = D / 16, DB = D / 32;
   static constexpr int T_BYTES = NB * 32 * D * 2;        // one streamed operand of one wave
@@ -62,14 +62,23 @@ struct SBTraits {
   static constexpr int W_BYTES = 2 * T_BYTES + 2 * 256;
   static constexpr int S_OWN = 2 * O_BYTES + 2 * 256;    // per slot: owned operands and their values per row
   static constexpr int TPW = T_BYTES / 1024;             // 1 KiB transfers per streamed operand
+  static constexpr int SLOT_BYTES = NW * W_BYTES + S_OWN;  // one batch entry
+  // tiles of batch entries resident in LDS
+  static constexpr int SLOTS = 2 * SLOT_BYTES <= 160 * 1024 ? 2 : 1;
+  static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES;
   // the partial sums go where the consumed tiles were: both sets at once when a wave's two tiles have room for them
   static constexpr bool ONE_PASS = DQ || 2 * T_BYTES >= 2 * PARK;
 };
 
+// a store that the waits count; the idle cycles keep it five wait states behind a vector instruction that wrote the address (see dma16)
+__device__ __forceinline__ void sb_store8(uint64_t sbase, unsigned voff, u32x2 data) {
+  asm volatile("s_nop 4\n\tglobal_store_dwordx2 %0, %1, %2" ::"v"(voff), "v"(data), "s"(sbase) : "memory");
+}
+
+// One workgroup's share of a role: workgroup `block` of the role's.
 template <class T>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
-void pairbias_bwd_kernel(const SBParams p) {
-  constexpr int D = T::D, NB = T::NB, KS = T::KS, DB = T::DB;
+__device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int block) {
+  constexpr int D = T::D, NB = T::NB, KS = T::KS, DB = T::DB, NW = T::NW;
   constexpr bool kDQ = T::DQ, kRowB = T::ROWB;
   constexpr float kLog2e = 1.4426950408889634f;
   using E = typename T::Elem;
@@ -79,14 +88,13 @@ void pairbias_bwd_kernel(const SBParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
-  const int NW = blockDim.x / 64, NT = blockDim.x;
   const int r = lane % 32, h = lane / 32;
 
   // ---- workgroup -> (group, chunk of batch entries, head, stripe): the stripes of one (chunk, head) read the same
   // tensors and stay on one XCD
   int tile, uc;
   {
-    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
+    const int x = block % 8, i = block / 8;
     tile = i % p.tiles;
     uc = i / p.tiles * 8 + x;
     if (uc >= p.groups * p.chunks * p.H) return;  // (before any barrier)
@@ -147,7 +155,7 @@ void pairbias_bwd_kernel(const SBParams p) {
   // ---- transfers of a batch entry into ring slot `slot`.  The per-lane offsets do not change from entry to entry and the
   // scalar base addresses advance by one batch stride: per entry a transfer costs its issue and nothing else.
   const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem);
-  const unsigned w_bytes = T::W_BYTES * NW, slot_bytes = w_bytes + T::S_OWN;
+  constexpr unsigned w_bytes = T::W_BYTES * NW, slot_bytes = T::SLOT_BYTES;
   constexpr int RPT = 512 / D;  // rows per 1 KiB transfer
   // byte offset of this lane's 16 bytes of transfer `it` of rows row0 .., rows past the end repeating the last one
   auto lane_offset = [&](int row0, int it, int64_t stride) FL_INLINE -> unsigned {
@@ -170,7 +178,13 @@ void pairbias_bwd_kernel(const SBParams p) {
     off2[it] = lane_offset(w0, it, kDQ ? p.vs[2] : p.dos[2]);
   }
   // the owned rows: 2 OT transfers shared out over the waves (one wave takes several where there are fewer waves)
-  constexpr int OT = T::O_BYTES / 1024;
+  constexpr int OT = T::O_BYTES / 1024, OPW = (2 * OT + NW - 1) / NW;
+  unsigned ooff[OPW];
+#pragma unroll
+  for (int j = 0; j < OPW; ++j) {
+    const int x = j * NW + wave;
+    ooff[j] = x < OT ? lane_offset(o0, x, kDQ ? p.qs[2] : p.ks[2]) : lane_offset(o0, x - OT, kDQ ? p.dos[2] : p.vs[2]);
+  }
   // per-row fp32 values: LSE and Delta rows of this head, the bias row of the entry
   uint64_t lse_at = uniform_ptr(p.lse + ((int64_t)n0 * p.H + head) * S), del_at = uniform_ptr(p.delta + ((int64_t)n0 * p.H + head) * S);
   uint64_t row_at = kRowB ? uniform_ptr(p.rowb + (int64_t)n0 * S) : 0;
@@ -180,25 +194,26 @@ void pairbias_bwd_kernel(const SBParams p) {
     const unsigned s0 = lds0 + slot * slot_bytes, mine = s0 + wave * T::W_BYTES, own_at = s0 + w_bytes;
 #pragma unroll
     for (int it = 0; it < T::TPW; ++it) {
-      dma16(st1.at, off1[it], mine + it * 1024);
-      dma16(st2.at, off2[it], mine + T::T_BYTES + it * 1024);
+      dma16<3>(st1.at, off1[it], mine + it * 1024);
+      dma16<3>(st2.at, off2[it], mine + T::T_BYTES + it * 1024);
     }
     if constexpr (kDQ) {
-      if constexpr (kRowB) dma4(row_at, st_row, mine + 2 * T::T_BYTES);
+      if constexpr (kRowB) dma4<3>(row_at, st_row, mine + 2 * T::T_BYTES);
     } else {
-      dma4(lse_at, st_row, mine + 2 * T::T_BYTES);
-      dma4(del_at, st_row, mine + 2 * T::T_BYTES + 256);
+      dma4<3>(lse_at, st_row, mine + 2 * T::T_BYTES);
+      dma4<3>(del_at, st_row, mine + 2 * T::T_BYTES + 256);
     }
-    for (int x = wave; x < 2 * OT; x += NW) {
-      if (x < OT) dma16(ow1.at, lane_offset(o0, x, kDQ ? p.qs[2] : p.ks[2]), own_at + x * 1024);
-      else dma16(ow2.at, lane_offset(o0, x - OT, kDQ ? p.dos[2] : p.vs[2]), own_at + x * 1024);
+#pragma unroll
+    for (int j = 0; j < OPW; ++j) {
+      const int x = j * NW + wave;
+      if ((j + 1) * NW <= 2 * OT || x < 2 * OT) dma16<3>(x < OT ? ow1.at : ow2.at, ooff[j], own_at + x * 1024);
     }
     if (wave == NW - 1) {
       if constexpr (kDQ) {
-        dma4(lse_at, ow_row, own_at + 2 * T::O_BYTES);
-        dma4(del_at, ow_row, own_at + 2 * T::O_BYTES + 256);
+        dma4<3>(lse_at, ow_row, own_at + 2 * T::O_BYTES);
+        dma4<3>(del_at, ow_row, own_at + 2 * T::O_BYTES + 256);
       } else if constexpr (kRowB) {
-        dma4(row_at, ow_row, own_at + 2 * T::O_BYTES);
+        dma4<3>(row_at, ow_row, own_at + 2 * T::O_BYTES);
       }
     }
     st1.at += st1.step;
@@ -232,12 +247,22 @@ void pairbias_bwd_kernel(const SBParams p) {
   constexpr int PC = D / 4;
   auto park_at = [&](int row, int c) FL_INLINE { return row * (D * 4) + ((c ^ row) & (PC - 1)) * 16; };
 
+  // where this entry's sums go; pieces of 64 lanes with 4 columns each, which the waves take in turn
+  const int rows = min(32, S - o0);
+  uint64_t out1 = uniform_ptr((kDQ ? p.dq : p.dk) + (int64_t)n0 * (kDQ ? p.dqs[0] : p.dks[0]) + (int64_t)head * (kDQ ? p.dqs[1] : p.dks[1]));
+  uint64_t out2 = kDQ ? 0 : uniform_ptr(p.dv + (int64_t)n0 * p.dvs[0] + (int64_t)head * p.dvs[1]);
+  const uint64_t step1 = (uint64_t)uniform_i64((kDQ ? p.dqs[0] : p.dks[0]) * 2), step2 = (uint64_t)uniform_i64(p.dvs[0] * 2);
+  constexpr int RPP = 256 / D, PIECES = 32 / RPP, PPW = (PIECES + NW - 1) / NW;
+  const int pieces = (rows + RPP - 1) / RPP, my_pieces = (pieces - wave + NW - 1) / NW;
+
   if (n0 < n1) load_entry(0);
   for (int n = n0; n < n1; ++n) {
-    const int slot = p.slots == 2 ? (n - n0) & 1 : 0;
-    dma_wait<0>();
+    const int slot = T::SLOTS == 2 ? (n - n0) & 1 : 0;
+    // everything this wave has asked for has landed, except the stores that were issued since
+    if (T::SLOTS == 1 || n == n0 || my_pieces < PPW) dma_wait<0>();
+    else dma_wait<(kDQ ? 1 : 2) * PPW>();
     __syncthreads();  // the owned rows are visible; everyone is done with the other slot
-    if (p.slots == 2 && n + 1 < n1) load_entry(slot ^ 1);
+    if (T::SLOTS == 2 && n + 1 < n1) load_entry(slot ^ 1);
 
     unsigned char* s0 = smem + slot * slot_bytes;
     unsigned char* mine = s0 + wave * T::W_BYTES;
@@ -329,44 +354,39 @@ void pairbias_bwd_kernel(const SBParams p) {
         for (int g = 0; g < 4; ++g)
           *reinterpret_cast<f32x4*>(at + park_at(r, 8 * d + 2 * g + h)) = f32x4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
     };
-    auto gather = [&](unsigned offset, bf16_t* out, const int64_t (&st)[3], float scale) FL_INLINE {
-      for (int x = tid; x < 32 * PC; x += NT) {
-        const int row = x / PC, c = x % PC;
+    auto gather = [&](unsigned offset, uint64_t out, int64_t row_stride, float scale) FL_INLINE {
+#pragma unroll
+      for (int j = 0; j < PPW; ++j) {
+        const int piece = j * NW + wave;
+        if (piece >= pieces) break;
+        // (rows past the end repeat the last one: every wave's stores are counted)
+        const int row = min(piece * RPP + lane / PC, rows - 1), c = lane % PC;
         const unsigned char* at = s0 + offset + park_at(row, c);
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
-        // (the usual wave counts with all their reads in flight)
-        if (NW == 4) {
 #pragma unroll
-          for (int w = 0; w < 4; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
-        } else if (NW == 8) {
+        for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
+        ex4 o4;
 #pragma unroll
-          for (int w = 0; w < 8; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
-        } else {
-          for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);
-        }
-        if (o0 + row < S) {
-          ex4 o4;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) o4[e] = (E)(sum[e] * scale);
-          // (32-bit offsets inside one (batch entry, head): S rows of at most 2^20 elements)
-          *reinterpret_cast<ex4*>(reinterpret_cast<unsigned char*>(out + (int64_t)n * st[0] + (int64_t)head * st[1]) +
-                                  (uint32_t)((o0 + row) * (int)st[2] + 4 * c) * 2u) = o4;
-        }
+        for (int e = 0; e < 4; ++e) o4[e] = (E)(sum[e] * scale);
+        // (32-bit offsets inside one (batch entry, head): S rows of at most 2^20 elements)
+        sb_store8(out, (uint32_t)((o0 + row) * (int)row_stride + 4 * c) * 2u, __builtin_bit_cast(u32x2, o4));
       }
     };
     // (a wave parks over its own tiles only, which it alone has read)
     park(acc1, mine);
     if constexpr (!kDQ && T::ONE_PASS) park(acc2, mine + T::PARK);
     __syncthreads();
-    gather(0, kDQ ? p.dq : p.dk, kDQ ? p.dqs : p.dks, p.scale);
-    if constexpr (!kDQ && T::ONE_PASS) gather(T::PARK, p.dv, p.dvs, 1.0f);
+    gather(0, out1, kDQ ? p.dqs[2] : p.dks[2], p.scale);
+    if constexpr (!kDQ && T::ONE_PASS) gather(T::PARK, out2, p.dvs[2], 1.0f);
     if constexpr (!kDQ && !T::ONE_PASS) {
       __syncthreads();
       park(acc2, mine);
       __syncthreads();
-      gather(0, p.dv, p.dvs, 1.0f);
+      gather(0, out2, p.dvs[2], 1.0f);
     }
-    if (p.slots == 1 && n + 1 < n1) {
+    out1 += step1;
+    out2 += step2;
+    if (T::SLOTS == 1 && n + 1 < n1) {
       __syncthreads();  // the sums have been read
       load_entry(0);
     }
@@ -384,6 +404,17 @@ void pairbias_bwd_kernel(const SBParams p) {
         }
     }
   }
+}
+
+// Both roles in one launch, the longer one first: neither needs the other, and the start of a workgroup (the stripe's bias) and the end
+// of a launch are latency that the other workgroup of the compute unit covers.
+template <class TQ, class TKV>
+__global__ __launch_bounds__(64 * TQ::NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void pairbias_bwd_kernel(const SBParams p) {
+  static_assert(TQ::NW == TKV::NW && TQ::LDS_BYTES == TKV::LDS_BYTES, "one workgroup shape");
+  const int half = gridDim.x / 2;
+  if ((int)blockIdx.x < half) pairbias_bwd_stripe<TKV>(p, blockIdx.x);
+  else pairbias_bwd_stripe<TQ>(p, blockIdx.x - half);
 }
 
 // Sums the chunks' partial bias gradients (in chunk order) into [groups, H, S, S] of the bias's type.

@@ -4,29 +4,34 @@
 
 namespace fl {
 namespace {
-template <class T>
-hipError_t launch_role(const SBShape& shape, const SBParams& p, hipStream_t stream) {
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pairbias_bwd_kernel<T>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+template <int D, int NB, int NW, bool ROWB, class E>
+hipError_t launch_one(const SBParams& p, hipStream_t stream) {
+  using TQ = SBTraits<D, 0, NB, NW, ROWB, E>;
+  using TKV = SBTraits<D, 1, NB, NW, ROWB, E>;
+  static_assert(TQ::LDS_BYTES == pairbias_bwd_shape(D, 32 * NB * NW).lds_bytes, "one rule");
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pairbias_bwd_kernel<TQ, TKV>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
   if (attr != hipSuccess) return attr;
   const int64_t units = (int64_t)p.groups * p.chunks * p.H;
-  const int64_t grid = (units + 7) / 8 * 8 * p.tiles;
-  hipLaunchKernelGGL((pairbias_bwd_kernel<T>), dim3((unsigned)grid), dim3(64 * shape.waves), shape.lds_bytes, stream, p);
+  const int64_t grid = 2 * ((units + 7) / 8 * 8 * p.tiles);
+  hipLaunchKernelGGL((pairbias_bwd_kernel<TQ, TKV>), dim3((unsigned)grid), dim3(64 * NW), TQ::LDS_BYTES, stream, p);
   return hipGetLastError();
 }
-template <int D, int NB, bool ROWB, class E>
-hipError_t launch_both(const SBShape& shape, const SBParams& p, hipStream_t stream) {
-  const hipError_t e = launch_role<SBTraits<D, 0, NB, ROWB, E>>(shape, p, stream);
-  return e != hipSuccess ? e : launch_role<SBTraits<D, 1, NB, ROWB, E>>(shape, p, stream);
-}
-template <int D, class E>
-hipError_t launch_d(const SBShape& shape, const SBParams& p, hipStream_t stream) {
-  if (shape.nb == 1) return p.rowb ? launch_both<D, 1, true, E>(shape, p, stream) : launch_both<D, 1, false, E>(shape, p, stream);
-  return p.rowb ? launch_both<D, 2, true, E>(shape, p, stream) : launch_both<D, 2, false, E>(shape, p, stream);
+// the shapes that pairbias_bwd_shape names
+template <int D, bool ROWB, class E, int BLOCKS = 16>
+hipError_t launch_shape(const SBShape& shape, const SBParams& p, hipStream_t stream) {
+  if constexpr (BLOCKS > 0) {
+    constexpr SBShape x = pairbias_bwd_shape(D, 32 * BLOCKS);
+    if (shape.nb == x.nb && shape.waves == x.waves) return launch_one<D, x.nb, x.waves, ROWB, E>(p, stream);
+    return launch_shape<D, ROWB, E, BLOCKS - 1>(shape, p, stream);
+  }
+  return hipErrorInvalidValue;
 }
 template <class E>
 hipError_t launch_any(int d, const SBShape& shape, const SBParams& p, hipStream_t stream) {
-  return d == 32 ? launch_d<32, E>(shape, p, stream) : d == 64 ? launch_d<64, E>(shape, p, stream) : hipErrorInvalidValue;
+  if (d == 32) return p.rowb ? launch_shape<32, true, E>(shape, p, stream) : launch_shape<32, false, E>(shape, p, stream);
+  if (d == 64) return p.rowb ? launch_shape<64, true, E>(shape, p, stream) : launch_shape<64, false, E>(shape, p, stream);
+  return hipErrorInvalidValue;
 }
 template <int D, bool GATE, class E>
 hipError_t launch_prep_one(const SBPrepParams& p, hipStream_t stream) {
