@@ -12,6 +12,9 @@
 // front end): 32 query heads over 8, one row, 32768 keys, head dim 128: 42.2 -> 31.2 us (27.4 for this kernel = 4.9 TB/s,
 // launch included, 4.5 for the merge); 8 sequences of 3001 keys in longer buffers: 51.6 -> 21.9 us; 32 x 2048 keys 5.5 TB/s;
 // causal prefill 2 x 8 heads x 512, head dim 64: 10.9 -> 9.2 us.
+// What such a call spends beside its reads is a chain: with the sums over the waves unrolled (a run-time count was one LDS wait after the
+// other), no division where one head has all rows, and the merge's loads in flight together, 9.20 -> 8.86, decoding 31.2 -> 30.1, 22.1 ->
+// 21.7 and, 2 x 8 heads of 282 rows, 7.8 -> 7.5.
 //
 // Rows are packed: row x of key / value head n is position x % Lq of query head n * G + x / Lq, so the G query heads that
 // share a key / value head are rows of one tile and the keys are read once for all of them.
@@ -120,7 +123,9 @@ void rows_kernel(const RParams p) {
   int any_lo = 1 << 30, any_hi = -1, all_lo = 0, all_hi = 1 << 30;  // keys some row / every row of the tile attends
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
-    const int crow = min(rt * RB + u * 16 + n16, p.rows - 1), gh = crow / p.Lq;
+    // (a division costs thirty dependent instructions at the start of a kernel that takes a few microseconds: none where one head
+    // has all rows, or every head one)
+    const int crow = min(rt * RB + u * 16 + n16, p.rows - 1), gh = p.group == 1 ? 0 : p.Lq == 1 ? crow : crow / p.Lq;
     qpos[u] = crow - gh * p.Lq;
     head[u] = kvh * p.group + gh;
     khi[u] = min(p.Lk - 1, max(p.dmax + qpos[u], p.pfx - 1));
@@ -137,8 +142,16 @@ void rows_kernel(const RParams p) {
   int t_end, t;
   {
     const int t0 = any_lo / 32, n = any_hi >= any_lo ? any_hi / 32 + 1 - t0 : 0;
-    t = t0 + (int)((int64_t)n * chunk / p.chunks) + wave;
-    t_end = t0 + (int)((int64_t)n * (chunk + 1) / p.chunks);
+    // chunk c takes n / chunks tiles, the first n % chunks of them one more
+    int first = 0, share = n;
+    if (p.chunks > 1) {
+      share = n / p.chunks;
+      const int more = n - share * p.chunks;
+      first = share * chunk + min(chunk, more);
+      share += chunk < more ? 1 : 0;
+    }
+    t = t0 + first + wave;
+    t_end = t0 + first + share;
   }
 
   ex8 qf[QT][KS];
@@ -338,34 +351,50 @@ void rows_kernel(const RParams p) {
   }
   __syncthreads();
   const int n_valid = min(RB, p.rows - rt * RB);
-  for (int x = threadIdx.x; x < n_valid * (D / 4); x += NW * 64) {
-    const int r = x / (D / 4), c = x % (D / 4) * 4;
-    float M = -INFINITY;
-    for (int w = 0; w < NW; ++w) M = __builtin_fmaxf(M, xml[(w * RB + r) * 2]);
-    const float ref = M == -INFINITY ? 0.f : M;
-    float L = 0.f;
-    f32x4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int w = 0; w < NW; ++w) {
-      const float a = fast_exp2(xml[(w * RB + r) * 2] - ref);
-      L += a * xml[(w * RB + r) * 2 + 1];
-      o += a * *reinterpret_cast<const f32x4*>(xo + (w * RB + r) * T::ROW_F + c);
-    }
-    if (p.chunks == 1) {
-      const int pr = rt * RB + r, hd = pr / p.Lq, pos = pr - hd * p.Lq, oh = kvh * p.group + hd;
-      const float inv = L > 0.f ? 1.0f / L : 0.f;  // a row that attends nothing yields zeros
-      typedef E ex4 __attribute__((ext_vector_type(4)));
-      ex4 w;
+  // (the wave count as a constant: all reads of the exchange in flight together instead of one wait after the other)
+  auto add_up = [&](auto nw_tag) FL_INLINE {
+    constexpr int N = decltype(nw_tag)::value;
+    for (int x = threadIdx.x; x < n_valid * (D / 4); x += N * 64) {
+      const int r = x / (D / 4), c = x % (D / 4) * 4;
+      f32x2 ml[N];
+      f32x4 ow[N];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = (E)(o[e] * inv);
-      *reinterpret_cast<ex4*>(p.o + (int64_t)batch * p.os[0] + (int64_t)oh * p.os[1] + (int64_t)pos * p.os[2] + c) = w;
-      if (p.lse != nullptr && c == 0)
-        p.lse[((int64_t)batch * p.Hq + oh) * p.Lq + pos] = L > 0.f ? ref + __builtin_log2f(L) : INFINITY;
-    } else {
-      const int64_t slot = (((int64_t)unit * p.row_tiles + rt) * p.chunks + chunk) * RB + r;
-      *reinterpret_cast<f32x4*>(p.part + slot * D + c) = o;
-      if (c == 0) *reinterpret_cast<f32x2*>(p.part_ml + slot * 2) = f32x2{M, L};
+      for (int w = 0; w < N; ++w) {
+        ml[w] = *reinterpret_cast<const f32x2*>(xml + (w * RB + r) * 2);
+        ow[w] = *reinterpret_cast<const f32x4*>(xo + (w * RB + r) * T::ROW_F + c);
+      }
+      float M = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < N; ++w) M = __builtin_fmaxf(M, ml[w][0]);
+      const float ref = M == -INFINITY ? 0.f : M;
+      float L = 0.f;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < N; ++w) {
+        const float a = fast_exp2(ml[w][0] - ref);
+        L += a * ml[w][1];
+        o += a * ow[w];
+      }
+      if (p.chunks == 1) {
+        const int pr = rt * RB + r, hd = p.group == 1 ? 0 : p.Lq == 1 ? pr : pr / p.Lq, pos = pr - hd * p.Lq, oh = kvh * p.group + hd;
+        const float inv = L > 0.f ? 1.0f / L : 0.f;  // a row that attends nothing yields zeros
+        typedef E ex4 __attribute__((ext_vector_type(4)));
+        ex4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = (E)(o[e] * inv);
+        *reinterpret_cast<ex4*>(p.o + (int64_t)batch * p.os[0] + (int64_t)oh * p.os[1] + (int64_t)pos * p.os[2] + c) = w;
+        if (p.lse != nullptr && c == 0)
+          p.lse[((int64_t)batch * p.Hq + oh) * p.Lq + pos] = L > 0.f ? ref + __builtin_log2f(L) : INFINITY;
+      } else {
+        const int64_t slot = (((int64_t)unit * p.row_tiles + rt) * p.chunks + chunk) * RB + r;
+        *reinterpret_cast<f32x4*>(p.part + slot * D + c) = o;
+        if (c == 0) *reinterpret_cast<f32x2*>(p.part_ml + slot * 2) = f32x2{M, L};
+      }
     }
-  }
+  };
+  if (NW == 8) add_up(std::integral_constant<int, 8>{});
+  else if (NW == 4) add_up(std::integral_constant<int, 4>{});
+  else add_up(std::integral_constant<int, 2>{});
 }
 
 // Adds up the chunks of a row: one workgroup of 256 threads per (unit, row); D / 4 threads take four columns each, and
@@ -380,16 +409,31 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
   __shared__ float xml[NG][2];
   float M = -INFINITY, L = 0.f;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
-  // (maxima first: the pairs are small and every group reads its own)
-  for (int ch = grp; ch < p.chunks; ch += NG) M = __builtin_fmaxf(M, p.part_ml[(slot0 + (int64_t)ch * RB) * 2]);
-  const float ref = M == -INFINITY ? 0.f : M;
-#pragma unroll 4
-  for (int ch = grp; ch < p.chunks; ch += NG) {
-    const int64_t s = slot0 + (int64_t)ch * RB;
-    const f32x2 ml = *reinterpret_cast<const f32x2*>(p.part_ml + s * 2);
-    const float a = fast_exp2(ml[0] - ref);
-    L += a * ml[1];
-    o += a * *reinterpret_cast<const f32x4*>(p.part + s * D + c);
+  // four chunks at a time, pairs and results asked for together (the pairs first and then the results, one after the other, was five
+  // trips to memory for 32 chunks: 4.5 us of a decoding step's 31)
+  for (int base = grp; base < p.chunks; base += 4 * NG) {
+    f32x2 ml[4];
+    f32x4 part[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int64_t s = slot0 + (int64_t)min(base + j * NG, p.chunks - 1) * RB;
+      ml[j] = *reinterpret_cast<const f32x2*>(p.part_ml + s * 2);
+      part[j] = *reinterpret_cast<const f32x4*>(p.part + s * D + c);
+    }
+    float M_new = M;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) M_new = base + j * NG < p.chunks ? __builtin_fmaxf(M_new, ml[j][0]) : M_new;
+    const float ref = M_new == -INFINITY ? 0.f : M_new;
+    const float keep = fast_exp2(M - ref);  // (0 before the first chunk with a key)
+    M = M_new;
+    L *= keep;
+    o *= keep;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float a = base + j * NG < p.chunks ? fast_exp2(ml[j][0] - ref) : 0.f;
+      L += a * ml[j][1];
+      o += a * part[j];
+    }
   }
   *reinterpret_cast<f32x4*>(&xo[grp][c]) = o;
   if (c == 0) {
