@@ -1205,8 +1205,19 @@ int fl_attn_bwd_validate(const fl_attn_bwd_params* b) { return validate_bwd(b, n
 // streamed steps is longer than an even share of all steps (half of them under masks of growing length) are cut into
 // splits of about that share.  A split costs the writing and reading of its partial sums and its own prologue, and the
 // sums a launch of 5 to 9 us: no split has fewer than eight steps, and a tile of up to one and a half shares stays whole.
-// Beyond, a launch per role is the better one (4 x 16 x 2048, head dim 64, causal: 177 us against 188; 2 x 16 x 2048, head
-// dim 128, unmasked: 271 against 300).
+// Beyond, a launch per role is the better one (dQ alone has room for more workgroups: 4 x 16 x 4096, head dim 64, causal: 533 us
+// against 565; 2 x 16 x 2048, head dim 128, unmasked: 271 against 300), unless the dK/dV launch ends on a second round that is
+// far from full (up to 896 tiles at head dim 64) or on the tiles of long documents (up to 2048): dQ's workgroups then fill what the
+// two launches leave idle.  Two launches -> one, us, head dim 64: 32 over 10 x 8 heads of 1139, unmasked 497 -> 457, window 300 238 -> 214;
+// 16 over 10 x 4 of 2000 with a prefix 505 -> 424; documents: 32 over 2 x 8 of 8037 1475 -> 1063, 16 of 16384 742 -> 647.  Full
+// rounds lose (1024 tiles, unmasked: 262 -> 270), and so does head dim 128 (7 x 16 of 1000: 298 -> 302; 6 x 32 over 8 of 2000: 1389 -> 1417).
+// A whole dK/dV tile is also too long a walk where it is near a share itself: the compute units that have two of them run late.
+// Measured at 0.9 shares and two dozen steps, with a step of this role at five quarters of one of dQ's (head dim 64; us, whole ->
+// cut in two): 8 over 12 heads of 3000 (288 tiles of 376 steps) 963 -> 853, over 14: 987 -> 974, over 16: 1088 -> 1095; 32 over 5 x 4 of 1139
+// 311 -> 246; head dim 128, 8 over 11 of 1000: 247 -> 199.  For the same reason not a few more splits than compute units at head dim 64
+// (8 over 3 of 3730, 90 tiles: 270 splits 423, 360 splits 359).  Under documents the steps that count are fewer than the
+// positions tell, and at head dim 128, with one workgroup per compute unit, the longest tile is what the others wait for: three
+// quarters of a share there (8 over 2 x 2 of 6000: 553 -> 312, 8 over 5 of 3266 with four draws of documents 345, 263, 363, 254 -> 307, 268, 334, 261).
 // Gradients, bf16, a launch per role with whole tiles -> this rule (both with the mask as selects, see bwd_kernel.h), now in
 // brackets: 3 x 16 heads over 4 x 1000 prefix rows, head dim 64: 157 -> 77 us (72); 8 x 512 causal, 64: 36 -> 25 (20); 8 over
 // 1 x 8192 causal, 64: 1980 -> 342 (284); 8 x 512 causal, 128: 47 -> 29 (27); 8 over 1 x 2048 causal, 128: 568 -> 73 (72);
@@ -1221,8 +1232,12 @@ BwdPlan plan_bwd(const fl_attn_params* p) {
   BwdPlan x;
   const int64_t D = p->Dqk, q_tiles = (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128), k_tiles = (int64_t)p->B * p->Hkv * ((p->Lk + 127) / 128);
   const int64_t least = std::min(q_tiles, k_tiles);
-  x.both = D <= 64 ? least <= 512 : least < 512;
-  if (!x.both) return x;
+  const bool small = D <= 64, doc = is_doc(p->mask_kind);
+  x.both = small ? least <= 512 : least < 512;
+  if (!x.both) {
+    x.both = small && k_tiles <= (doc ? 2048 : 896);
+    return x;
+  }
   int64_t q_steps = (p->Lk + 63) / 64, k_steps = (p->Lq + 63) / 64;
   if (p->mask_kind == FL_MASK_SLIDING) {
     const int64_t band = ((int64_t)p->window + 128) / 64 + 1;
@@ -1231,11 +1246,16 @@ BwdPlan plan_bwd(const fl_attn_params* p) {
   }
   k_steps *= p->Hq / p->Hkv;
   const bool growing = p->mask_kind != FL_MASK_NONE && p->mask_kind != FL_MASK_SLIDING;
-  const int64_t total = (q_tiles * q_steps + k_tiles * k_steps) / (growing ? 2 : 1);
-  const int64_t share = std::max<int64_t>(8, total / (D <= 64 ? 512 : 256));
-  const auto splits = [&](int64_t steps) { return (int)(2 * steps <= 3 * share ? 1 : (steps + share - 1) / share); };
-  x.dq = splits(q_steps);
-  x.dkv = splits(k_steps);
+  const int64_t dq_work = q_tiles * q_steps / (growing ? 2 : 1), dkv_work = k_tiles * k_steps / (growing ? 2 : 1);
+  const int64_t slots = small ? 512 : 256;
+  const int64_t share = std::max<int64_t>(8, (dq_work + dkv_work) / slots);
+  const int64_t dkv_share = small ? (4 * dq_work + 5 * dkv_work) / (5 * slots) : share;
+  const auto splits = [](int64_t steps, int64_t share) { return (int)((steps + share - 1) / share); };
+  if (2 * q_steps > 3 * share) x.dq = splits(q_steps, share);
+  if (2 * k_steps > 3 * share || 10 * k_steps > 9 * dkv_share + 240) {
+    x.dkv = std::max(2, splits(k_steps, doc && !small ? std::max<int64_t>(8, share * 3 / 4) : share));
+    if (small && k_tiles * x.dkv > 256 && k_tiles * x.dkv <= 320 && k_steps >= 16 * x.dkv) ++x.dkv;
+  }
   x.dq_bytes = x.dq > 1 ? (uint64_t)x.dq * q_tiles * 128 * D * sizeof(float) : 0;
   x.bytes = x.dq_bytes + (x.dkv > 1 ? (uint64_t)x.dkv * k_tiles * 128 * D * 2 * sizeof(float) : 0);
   return x;

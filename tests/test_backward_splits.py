@@ -84,3 +84,43 @@ def test_cut_tiles_give_the_gradients_of_whole_tiles(case, dtype, monkeypatch):
         d, ref = (a.double() - b.double()), b.double()
         assert (d.norm() / ref.norm()).item() < ulp / 4, name
         assert (d.abs() <= 2 * ulp * ref.abs() + 2e-5 * ref.abs().max()).all(), name
+
+
+LONG_WALKS = [  # cut though no tile is longer than one and a half shares; more splits than the share asks for; documents' shares
+    (44, 16, 2, 512, 100, 128, _ffi.MASK_NONE, {}),
+    (90, 8, 1, 2000, 100, 32, _ffi.MASK_NONE, {}),
+    (6, 8, 2, 1900, 1900, 128, _ffi.MASK_DOCUMENT_CAUSAL, {}),
+]
+
+
+def test_which_long_walks_are_cut():
+    sums = lambda splits, tiles, D: splits * tiles * 128 * D * 2 * 4  # noqa: E731
+    assert [_split_bytes(*c[:7]) for c in LONG_WALKS] == [sums(2, 88, 128), sums(4, 90, 32), sums(2, 180, 128)]
+    assert _split_bytes(12, 8, 1, 3000, 3000, 64) == sums(2, 288, 64)
+    assert _split_bytes(16, 8, 1, 3000, 3000, 64) == 0   # a walk of 0.75 shares
+    assert _split_bytes(10, 16, 4, 2000, 2000, 64) == 0  # one launch, whole tiles
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", LONG_WALKS)
+def test_long_walks_give_the_gradients_of_whole_tiles(case, monkeypatch):
+    test_cut_tiles_give_the_gradients_of_whole_tiles(case, torch.bfloat16, monkeypatch)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("mask", [_ffi.MASK_NONE, _ffi.MASK_CAUSAL, _ffi.MASK_DOCUMENT_CAUSAL])
+def test_both_roles_in_one_launch_beyond_a_round(mask, D):
+    """528 tiles of keys: the same bits as the two halves, which have 256 and 272."""
+    g = torch.Generator().manual_seed(D)
+    q, k, v, dout = (torch.randn(33, h, 70, D, generator=g).to(torch.bfloat16).to(DEV) for h in (32, 16, 16, 32))
+    ids = torch.sort(torch.randint(0, 3, (33, 70), generator=g), dim=1).values.to(DEV)
+
+    def gradients(part):
+        kw = dict(mask_kind=mask, **(dict(doc_ids=ids[part]) if mask == _ffi.MASK_DOCUMENT_CAUSAL else {}))
+        lse = torch.empty(*q[part].shape[:3], dtype=torch.float32, device=DEV)
+        out = _ffi.attn_fwd(q[part], k[part], v[part], lse=lse, **kw)
+        return _ffi.attn_bwd(q[part], k[part], v[part], out, lse, dout[part], split=True, **kw)
+
+    for whole, a, b in zip(gradients(slice(None)), gradients(slice(0, 16)), gradients(slice(16, 33))):
+        assert torch.equal(whole, torch.cat([a, b]))
