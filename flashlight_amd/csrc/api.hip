@@ -294,6 +294,44 @@ uint32_t wanted_features(const fl_attn_params* p) {
 // Features a kernel may be compiled with yet leave unused at run time (null pointer / zero slope).
 constexpr uint32_t kOptionalFeatures = fl::F_ALIBI | fl::F_BIAS | fl::F_GATE;
 
+// Calls of few workgroups: a workgroup of 128 rows walks its key tiles one after the other, 0.8 us each with one wave per
+// SIMD, and ends when the longest walk does.  Smaller workgroups (64 rows: `waves` = 2) and groups of waves that share the rows and
+// take a part of the tiles each (fwd_kernel.h) fill what idles.  Tiles of 128 rows up to one per compute unit: always; up to two under
+// masks of growing length, whose longest walk is twice the average, while they belong to few heads (many short heads end together).
+// us, 128 rows -> this rule, bf16: head dim 64, causal: 2 x 8 heads of 2048 29.3 -> 19.8, 8 of 4096 52.6 -> 33.6, 16 of 3000 (384 tiles)
+// 40.1 -> 31.4, 4 of 4096 in four groups 52.0 -> 26.2 (in two 30.9); ALiBi and soft-cap, 16 of 2048: 41.9 -> 27.4; head dim 128, causal:
+// 8 of 4096 69.5 -> 58.3, 16 of 3000 with 128 rows in two groups 58.0 -> 48.5; unmasked, 8 of 4096: 53.5 -> 43.9; documents: 8 heads of 6000,
+// head dim 128, 119 -> 85.  Beyond, the second group's prologue and the adding up cost more: causal, 5 x 16 of 1184 (800 tiles) 33.9 -> 36.0,
+// 8 x 16 of 512 15.9 -> 17.4, 2 x 32 of 700 under a prefix of 600 16.1 -> 18.7.
+struct FewPlan {
+  int waves = 0;   // preferred waves per group (0: no preference)
+  int groups = 1;  // preferred groups
+};
+FewPlan plan_few(const fl_attn_params* p, uint32_t want) {
+  FewPlan x;
+  if (p->Dqk != p->Dv || (p->Dqk != 64 && p->Dqk != 128) || (want & ~(fl::F_ALIBI | fl::F_SOFTCAP | fl::F_DOC | fl::F_DUMP))) return x;
+  const int64_t heads = (int64_t)p->B * p->Hq, tiles = heads * ((p->Lq + 127) / 128);
+  // Walks of few tiles: the second group's prologue and the adding up cost more than the tiles it takes.  us: head dim 64, causal, 5 x 16
+  // of 320 8.8 -> 9.4, 2 x 16 of 400 9.9 -> 8.4; unmasked, 4 x 8 of 512 10.7 -> 11.0, of 800 15.6 -> 14.6; documents, 6 x 16 of 64
+  // 12.9 -> 13.8, of 200 18.6 -> 16.9; head dim 128, causal, 2 x 16 of 192 8.4 -> 8.7, of 256 10.6 -> 9.7; unmasked, 4 x 8 of 640 16.7 -> 17.4.
+  const int64_t walk = p->mask_kind == FL_MASK_SLIDING ? std::min<int64_t>(p->Lk, (int64_t)p->window + 128) : p->Lk;
+  const bool narrow = p->Dqk == 64;
+  if (walk < ((want & fl::F_DOC) ? 192 : p->mask_kind == FL_MASK_NONE ? (narrow ? 640 : 1024) : narrow ? 384 : 256)) return x;
+  if (heads == 1) return x;  // (one head by itself is what slices of large calls are compared with: it keeps their order of sums)
+  if (p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM) {
+    if (narrow ? tiles > 256 && (tiles > 512 || heads > 48) : tiles > 512 || heads > 48) return x;
+    x.waves = narrow || tiles <= 256 ? 2 : 4;
+    x.groups = narrow && tiles <= 128 && p->Lk >= 1024 ? 4 : 2;
+  } else if (tiles <= 256) {
+    x.groups = 2;
+  } else if (want & fl::F_DOC) {
+    // (the walks are as long as the documents, which only the device knows: 1 x 16 x 4768, documents of 512 to 2384: 77 -> 55, but
+    // 1 x 16 x 4096 in documents of 512 each: 23.5 -> 28.9; from 32 heads on it is even or loses whatever the documents)
+    x.groups = tiles <= 1024 && heads <= 16 && p->Lk >= 4000 ? 2 : 1;
+  }
+  return x;
+}
+
 const fl::Instance* select_instance(const fl_attn_params* p) {
   const uint32_t want = wanted_features(p);
   const fl::Instance* best = nullptr;
@@ -312,14 +350,15 @@ const fl::Instance* select_instance(const fl_attn_params* p) {
   // keys one workgroup of 128 query rows visits: the window plus its own rows for a sliding window, else up to Lk
   const int64_t visited = p->mask_kind == FL_MASK_SLIDING ? std::min<int64_t>(p->Lk, (int64_t)p->window + 128) : p->Lk;
   // (measured: from a window of 256 on the 4-wave tile ties or wins on warm operands and wins by 4 % on cold ones)
-  const bool short_loop = p->mask_kind == FL_MASK_SLIDING && visited < 384;
+  const bool short_loop = p->mask_kind == FL_MASK_SLIDING && visited < 384 && p->Dqk == 128 && !(want & (fl::F_ALIBI | fl::F_SOFTCAP));
   // Unmasked calls at head dim 128 whose grid still fills the part twice over with 256-row workgroups take the
   // 8-wave tile: one workgroup per compute unit brings every K/V tile in once for 256 rows instead of twice, which on
   // ordinary data is worth more than the second workgroup's independence (2.4 % on N(0,1) operands; at head dim 64,
   // under masks and on all-zero operands it is not).
   const bool wide_group = p->mask_kind == FL_MASK_NONE && want == 0 && p->Dqk == 128 && p->Dv == 128 &&
                           (int64_t)p->B * p->Hq * ((p->Lq + 255) / 256) >= 512;
-  const int preferred_nw = short_loop ? 2 : (wide_group ? 8 : 4);
+  const FewPlan few = plan_few(p, want);
+  const int preferred_nw = few.waves ? few.waves : short_loop ? 2 : (wide_group ? 8 : 4);
   for (int i = 0; i < fl::kNumInstances; ++i) {
     const fl::Instance& in = fl::kInstances[i];
     if (in.dqk != p->Dqk || in.dv != p->Dv || in.dtype != p->dtype) continue;
@@ -367,6 +406,11 @@ int64_t lds_bytes_for(const fl::Instance* in, const fl_attn_params* p) {
 }
 // Dynamic LDS bytes of the document-mask pre-pass (doc_lists_kernel): 20 per key tile; it has 128 static bytes besides
 int64_t prepass_lds_bytes(int64_t n_ktiles) { return n_ktiles * 20; }
+// Groups of waves a call is launched with, and the LDS of all of them
+int groups_for(const fl::Instance* in, const fl_attn_params* p) {
+  const int groups = std::min(plan_few(p, wanted_features(p)).groups, in->max_groups);
+  return lds_bytes_for(in, p) + (int64_t)(groups - 1) * in->lds_fixed_bytes <= fl::kMaxLdsBytes ? groups : 1;
+}
 int64_t max_keys_for(const fl::Instance* in) {
   int64_t tiles = fl::kMaxKeyTiles;
   if (in->feat & fl::F_DOC) {
@@ -925,6 +969,7 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
   out[4] = lds_bytes_for(in, p);
   out[5] = in->feat;
   out[6] = 0;
+  out[7] = groups_for(in, p);
   {
     // calls the shared-bias streaming forward takes: its fixed shape, and out[6] = 1
     fl::PParams pb;
@@ -936,6 +981,7 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
       out[3] = pb_grid;
       out[4] = 2 * (p->Dqk == 32 ? 6 : 4) * 64 * p->Dqk * 2 + (pb.rowb ? 4 * 2 * 1024 : 0);
       out[6] = 1;
+      out[7] = 1;
       return 0;
     }
     fl::StripeParams sp;
@@ -948,9 +994,9 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
       out[3] = launch[0];
       out[4] = launch[1];
       out[6] = 2;
+      out[7] = 1;
     }
   }
-  out[7] = 0;
   return 0;
 }
 
@@ -1130,7 +1176,8 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
     kp.doc_list_stride = (int)d.list_stride;
     kp.doc_order = order;
   }
-  hipError_t e = in->launch(kp, grid, (int)lds_bytes_for(in, p), stream);
+  const int groups = groups_for(in, p);
+  hipError_t e = in->launch(kp, groups, grid, (int)lds_bytes_for(in, p) + (groups - 1) * in->lds_fixed_bytes, stream);
   if (e != hipSuccess) return fail((int)e, "launch of %s failed: %s", in->name, hipGetErrorString(e));
   return 0;
 }

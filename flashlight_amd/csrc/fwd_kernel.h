@@ -26,6 +26,7 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // Feature bits selected at compile time; everything else is a runtime field.
@@ -357,14 +358,15 @@ __device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) { return __
 __device__ __forceinline__ float dot2acc(bf16x2 a, bf16x2 b, float c) { return __builtin_amdgcn_fdot2_f32_bf16(a, b, c, false); }
 __device__ __forceinline__ float dot2acc(f16x2 a, f16x2 b, float c) { return __builtin_amdgcn_fdot2(a, b, c, false); }
 
-template <int DQK_, int DV_, int RW_, int BN_, int NW_, uint32_t FEAT_, int NS_ = 4, class Elem_ = bf16_t>
+template <int DQK_, int DV_, int RW_, int BN_, int NW_, uint32_t FEAT_, int NS_ = 4, class Elem_ = bf16_t, int KG_ = 1>
 struct FwdTraits {
   using Elem = Elem_;
   static constexpr int DQK = DQK_, DV = DV_, RW = RW_, BN = BN_, NW = NW_;
   static constexpr int NS = NS_;  // K/V tiles resident in LDS (ring); transfers run NS - 1 tiles ahead of their use
   static_assert(NS >= 2 && NS <= 8 && NS % 2 == 0, "ring depth (even: the two score buffers alternate with the slots)");
   static constexpr uint32_t FEAT = FEAT_;
-  static constexpr int NT = NW * 64;
+  static constexpr int KG = KG_;      // groups of NW waves that share the rows and take a part of the key tiles each
+  static constexpr int NT = NW * 64;  // threads of a group
   static constexpr int BM = NW * RW;
   static constexpr int QB = RW / 32;   // 32-row query blocks per wave
   static constexpr int KB = BN / 32;   // 32-key blocks per tile
@@ -400,7 +402,8 @@ struct FwdTraits {
   static_assert(!(FEAT & F_DOC) || (BN * 8) % 256 == 0, "whole transfers of 64 dwords");
   static constexpr int K_OFF = 0, V_OFF = NS * KBYTES, B_OFF = NS * (KBYTES + VBYTES), R_OFF = B_OFF + NS * BBYTES,
                        I_OFF = R_OFF + NS * RBYTES, LIST_OFF = I_OFF + NS * IBYTES;
-  static constexpr int LDS_FIXED_BYTES = LIST_OFF;
+  static constexpr int LDS_FIXED_BYTES = KG * LIST_OFF;
+  static_assert(KG == 1 || (KG - 1) * NW * 64 * QB * (16 * DVB + 2) * 4 <= LDS_FIXED_BYTES, "the groups' results must fit in LDS");
 };
 
 // The main loop is software-pipelined over key tiles so that one wave keeps both the matrix pipe and the vector
@@ -410,8 +413,11 @@ struct FwdTraits {
 //     rare       element mask of S(tb) on partial tiles; rescale of O, l when the maximum grew
 // while the global -> LDS transfers of K(tc) and V(tb), issued at the top of the iteration into the buffers that
 // iteration i-1 freed, are in flight; the barrier that ends the iteration publishes them.
+//
+// KG > 1, for calls of few workgroups: one wave per SIMD takes 0.8 us per tile and two take 1.35, so KG groups of waves with a ring each
+// walk consecutive parts of the list of tiles and the first adds up what they leave in LDS.  Registers allow two waves per SIMD.
 template <class T>
-__global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
+__global__ __launch_bounds__(T::KG * T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
 void fwd_kernel(const KParams p) {
   constexpr int DQK = T::DQK, DV = T::DV, RW = T::RW, BN = T::BN, NW = T::NW, NT = T::NT, BM = T::BM;
   constexpr int QB = T::QB, KB = T::KB, KS = T::KS, DVB = T::DVB;
@@ -430,12 +436,17 @@ void fwd_kernel(const KParams p) {
   using LK = TileLayout<DQK>;
   using LV = TileLayout<DV>;
 
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  constexpr int KG = T::KG;
+  static_assert(KG == 1 || !(kDiff || kBias || kDump), "groups of waves: kernels without a second branch, bias operands or the dump");
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
   // tile list (document masks): word 0 = number of entries, then one entry per key tile that is not empty for the
   // whole workgroup, in key order: bits 0-15 tile index, bits 16.. two class bits per wave
-  const uint32_t* tlist = reinterpret_cast<const uint32_t*>(smem + T::LIST_OFF) + 1;
+  const uint32_t* tlist = reinterpret_cast<const uint32_t*>(smem_all + KG * T::LIST_OFF) + 1;
 
-  const int tid = threadIdx.x;
+  // each group of waves has its own K/V ring
+  const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  unsigned char* const smem = KG > 1 ? smem_all + group * T::LIST_OFF : smem_all;
+  const int tid = KG > 1 ? threadIdx.x % NT : threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   const int r = lane % 32, h = lane / 32;
 
@@ -481,7 +492,7 @@ void fwd_kernel(const KParams p) {
     // before the key loop, so that the query loads below run under its latency
     const int n_chunks = p.doc_list_stride / 4;
     const uint64_t lbase = uniform_ptr(p.doc_lists + ((int64_t)batch * p.n_qtiles + qt) * p.doc_list_stride);
-    const unsigned lds_l = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem + T::LIST_OFF);
+    const unsigned lds_l = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem_all + KG * T::LIST_OFF);
     for (int c0 = wave * 64; c0 < n_chunks; c0 += NW * 64)
       dma16(lbase, (unsigned)min(c0 + lane, n_chunks - 1) * 16u, lds_l + c0 * 16);
   } else {
@@ -492,6 +503,18 @@ void fwd_kernel(const KParams p) {
     if (p.mask_kind == MASK_SLIDING) lo_key = max(0, q0 - p.window);
     t_lo = lo_key / BN;
     n_list = hi_key >= lo_key ? hi_key / BN - t_lo + 1 : 0;
+  }
+  // The groups take consecutive parts of the list; all of them make n_list steps, the last ones idle where a part is shorter.
+  int n_own = 0, first = 0;  // this group's part: list positions [first, first + n_own)
+  auto take_part = [&]() FL_INLINE {
+    const int all = n_list;
+    n_list = (all + KG - 1) / KG;
+    n_own = max(0, min(n_list, all - group * n_list));
+    first = n_own > 0 ? group * n_list : 0;
+  };
+  if constexpr (KG > 1 && !kDoc) {
+    take_part();
+    t_lo += first;
   }
   // This wave's tile classes for a positional mask, as index ranges: tiles outside [e_lo, e_hi] are EMPTY for its
   // rows [a, b), tiles inside [f_lo, f_hi] FULL, the rest PARTIAL (the same closed forms as classify_positional,
@@ -521,13 +544,14 @@ void fwd_kernel(const KParams p) {
   // tile-list entry of list position i (the last entry again past the end): bits 0-15 tile index, two class bits per
   // wave from bit 16 on (only this wave's are filled in when the entry is computed rather than read)
   auto list_entry = [&](int i) FL_INLINE -> uint32_t {
+    const int last_own = KG > 1 ? max(n_own, 1) - 1 : n_list - 1;
     if constexpr (kDoc) {
-      return tlist[min(i, n_list - 1)];
+      return tlist[first + min(i, last_own)];
     } else {
       // ALiBi adds a term that grows with the key position: visiting the tiles from the last one down makes every
       // later tile's scores fall away from the running reference instead of climbing above it, so the reference set by
       // the first tile visited holds and the accumulators are never rescaled
-      const int t = (FEAT & F_ALIBI) ? t_lo + n_list - 1 - min(i, n_list - 1) : t_lo + min(i, n_list - 1);
+      const int t = (FEAT & F_ALIBI) ? t_lo + last_own - min(i, last_own) : t_lo + min(i, last_own);
       const int cw = (t < e_lo || t > e_hi) ? TILE_EMPTY : ((t >= f_lo && t <= f_hi) ? TILE_FULL : TILE_PARTIAL);
       return ((uint32_t)cw << (16 + 2 * wave)) | (uint32_t)t;
     }
@@ -1212,16 +1236,19 @@ void fwd_kernel(const KParams p) {
     // (the previous branch is done with the LDS buffers; every wave's share of the tile list is visible to all)
     if (br > 0 || kDoc) __syncthreads();
     if constexpr (kDoc) n_list = __builtin_amdgcn_readfirstlane((int)tlist[-1]);
+    if constexpr (KG > 1 && kDoc) take_part();
     // whether the weights of a tile-list entry's tile are formed without looking at its row maxima first
     auto reference_free = [&](uint32_t e) FL_INLINE { return kFastRef && (kLazyMasked || entry_class(e) == TILE_FULL); };
     // Head of a step, vector work only: element mask of the current tile if it is not FULL for this wave, its row
-    // maxima, and the (rare) rescale.
-    auto settle = [&](f32x16 (&sc)[KB][QB], uint32_t e, int vslot) FL_INLINE {
+    // maxima, and the (rare) rescale.  own_max: the first tile of a group of waves, whose row maxima then are the group's reference (the
+    // rounding of 16-bit weights is least where the largest is 1: without it the error against fp64 of 3 x 8 heads of 967 causal rows
+    // is that of the whole walk, 2.06e-3 of the result's norm, with it 2.01e-3; 0.1 us).
+    auto settle = [&](f32x16 (&sc)[KB][QB], uint32_t e, int vslot, bool own_max) FL_INLINE {
       const int t = entry_tile(e);
       const bool full = entry_class(e) == TILE_FULL;
       if constexpr (kLazyMasked) {
         if (!full) apply_mask(sc, t, vslot);
-      } else if (!full || !kFastRef) {
+      } else if (!full || !kFastRef || own_max) {
         if (!full) apply_mask(sc, t, vslot);
         float mx[QB];
         row_max(sc, mx);
@@ -1236,13 +1263,14 @@ void fwd_kernel(const KParams p) {
     // below are unrolled over the two ring slots and entered at slot 0): an EMPTY tile ahead of it is taken into the run
     // and computed and masked like any other.
     auto live_run = [&](int& a_live, int& b_live) FL_INLINE {
+      const int n = KG > 1 ? n_own : n_list;
       a_live = 0;
-      b_live = n_list;
+      b_live = n;
       if constexpr (kDoc) {
-        int a = n_list, b = 0;
-        for (int base = 0; base < n_list; base += 64) {
+        int a = n, b = 0;
+        for (int base = 0; base < n; base += 64) {
           const int i = base + lane;
-          const bool live = i < n_list && ((tlist[min(i, n_list - 1)] >> (16 + 2 * wave)) & 3u) != (unsigned)TILE_EMPTY;
+          const bool live = i < n && ((tlist[first + min(i, n - 1)] >> (16 + 2 * wave)) & 3u) != (unsigned)TILE_EMPTY;
           const uint64_t m = __builtin_amdgcn_ballot_w64(live);
           if (m != 0) {
             a = min(a, base + (int)__builtin_ctzll(m));
@@ -1252,11 +1280,11 @@ void fwd_kernel(const KParams p) {
         a_live = __builtin_amdgcn_readfirstlane(a);
         b_live = __builtin_amdgcn_readfirstlane(b);
       } else if constexpr (FEAT & F_ALIBI) {  // positions run from the last tile down
-        a_live = max(0, t_lo + n_list - 1 - e_hi);
-        b_live = min(n_list, t_lo + n_list - e_lo);
+        a_live = max(0, t_lo + n - 1 - e_hi);
+        b_live = min(n, t_lo + n - e_lo);
       } else {
         a_live = max(0, e_lo - t_lo);
-        b_live = min(n_list, e_hi - t_lo + 1);
+        b_live = min(n, e_hi - t_lo + 1);
       }
       if (a_live >= b_live) a_live = b_live = n_list;  // nothing for this wave
       else a_live -= a_live % T::NS;
@@ -1322,7 +1350,7 @@ void fwd_kernel(const KParams p) {
         // K slot `slot` held this tile's K and V slot `slot - 1` the previous tile's V: both were last read before the
         // barrier that ended the previous step
         const bool steady = issue_loads(slot);
-        settle(sc, ent[0], slot);
+        settle(sc, ent[0], slot, KG > 1 && pos == a_live);
         ex8 pf[QB][2 * KB];
         // Raised issue priority while this wave has matrix work: of the two waves sharing a SIMD, the one that is in
         // its MFMA phase wins the issue port, which drives the pair into opposite phases (one on the matrix pipe while
@@ -1377,10 +1405,10 @@ void fwd_kernel(const KParams p) {
         ex8 pf[QB][2 * KB];
         ex8 vfirst[DVB];
         if constexpr (slot % 2 == 0) {
-          settle(s_a, ent[0], slot);
+          settle(s_a, ent[0], slot, KG > 1 && pos == a_live);
           weights_checked(s_a, pf, reference_free(ent[0]), std::false_type{}, vfirst, slot, entry_tile(ent[0]), std::false_type{});
         } else {
-          settle(s_b, ent[0], slot);
+          settle(s_b, ent[0], slot, KG > 1 && pos == a_live);
           weights_checked(s_b, pf, reference_free(ent[0]), std::false_type{}, vfirst, slot, entry_tile(ent[0]), std::false_type{});
         }
         pv_mma(pf, slot, vfirst, std::false_type{});
@@ -1392,6 +1420,64 @@ void fwd_kernel(const KParams p) {
       while (pos + 1 < n_list) {
         const bool steady = issue_loads(pos % NS);
         end_step(steady);
+      }
+    }
+
+    // ---- the groups' sums, each relative to the reference its group ended with, are added up by the first group --------------
+    if constexpr (KG > 1) {
+      constexpr int W = QB * (16 * DVB + 2);  // floats per lane
+      float* const sums = reinterpret_cast<float*>(smem_all) + wave * (W * 64) + 4 * lane;
+      constexpr int kGroup = NW * W * 64;
+      float ref[QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) ref[qb] = xhalf_sum(l_run[qb]) == 0.f ? -INFINITY : ref_now(qb);
+      __syncthreads();  // (every wave is done with the tiles)
+      if (group > 0) {
+        float* const to = sums + (group - 1) * kGroup;
+#pragma unroll
+        for (int qb = 0; qb < QB; ++qb) {
+#pragma unroll
+          for (int dvb = 0; dvb < DVB; ++dvb)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+              *reinterpret_cast<f32x4*>(to + ((qb * DVB + dvb) * 4 + g) * 256) =
+                  f32x4{oacc[dvb][qb][4 * g], oacc[dvb][qb][4 * g + 1], oacc[dvb][qb][4 * g + 2], oacc[dvb][qb][4 * g + 3]};
+          *reinterpret_cast<f32x2*>(to + QB * DVB * 1024 + qb * 128 - 2 * lane) = f32x2{ref[qb], l_run[qb]};
+        }
+      }
+      __syncthreads();
+      if (group > 0) return;
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb) {
+        f32x2 other[KG - 1];
+        float m = ref[qb];
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g) {
+          other[g] = *reinterpret_cast<const f32x2*>(sums + g * kGroup + QB * DVB * 1024 + qb * 128 - 2 * lane);
+          m = __builtin_fmaxf(m, other[g][0]);
+        }
+        const float m_use = m == -INFINITY ? 0.f : m;
+        const float alpha = fast_exp2((ref[qb] - m_use) * c2);
+        m_run[qb] = m;
+        l_run[qb] *= alpha;
+#pragma unroll
+        for (int dvb = 0; dvb < DVB; ++dvb)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) oacc[dvb][qb][i] *= alpha;
+#pragma unroll
+        for (int g = 0; g < KG - 1; ++g) {
+          __builtin_amdgcn_sched_barrier(0);  // one group's sums in flight at a time
+          const float beta = fast_exp2((other[g][0] - m_use) * c2);
+          l_run[qb] = __builtin_fmaf(other[g][1], beta, l_run[qb]);
+#pragma unroll
+          for (int dvb = 0; dvb < DVB; ++dvb)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const f32x4 x = *reinterpret_cast<const f32x4*>(sums + g * kGroup + ((qb * DVB + dvb) * 4 + j) * 256);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) oacc[dvb][qb][4 * j + e] = __builtin_fmaf(x[e], beta, oacc[dvb][qb][4 * j + e]);
+            }
+        }
       }
     }
 

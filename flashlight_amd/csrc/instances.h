@@ -13,7 +13,8 @@ struct Instance {
   int rw, bn, nw, ns;  // rows per wave, keys per tile, waves per workgroup, K/V tiles resident in LDS
   uint32_t feat;
   int lds_fixed_bytes;  // LDS without the tile list (4 more bytes per key tile)
-  hipError_t (*launch)(const KParams&, int grid, int lds_bytes, hipStream_t);
+  int max_groups;  // groups of nw waves a workgroup can be launched with (1, 2 or 4), each with lds_fixed_bytes
+  hipError_t (*launch)(const KParams&, int groups, int grid, int lds_bytes, hipStream_t);
 };
 
 // Defined by instances_table.cpp from the per-file launchers.
@@ -27,8 +28,26 @@ hipError_t launch_fwd(const KParams& kp, int grid, int lds_bytes, hipStream_t st
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<T>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(fwd_kernel<T>, dim3(grid), dim3(T::NT), lds_bytes, stream, kp);
+  hipLaunchKernelGGL(fwd_kernel<T>, dim3(grid), dim3(T::KG * T::NT), lds_bytes, stream, kp);
   return hipGetLastError();
+}
+
+// Groups of waves the shape can be launched with (plan_few in api.hip): every instance compiled for them is that many kernels, so
+// only the default tiles have them.  Eight waves are two per SIMD, all the registers hold (four groups of four spill).
+constexpr int max_groups(int dqk, int dv, int rw, int bn, int nw, int ns, uint32_t feat) {
+  if (dqk != dv || (dqk != 64 && dqk != 128) || rw != 32 || ns != 2 || (feat & ~(F_ALIBI | F_SOFTCAP | F_DOC))) return 1;
+  if (nw == 2) return dqk == 64 ? 4 : 2;
+  return nw == 4 && bn == (dqk == 128 && (feat & F_DOC) ? 32 : 64) ? 2 : 1;
+}
+
+template <int DQK, int DV, int RW, int BN, int NW, int NS, uint32_t FEAT, class E>
+hipError_t launch_fwd_groups(const KParams& kp, int groups, int grid, int lds_bytes, hipStream_t stream) {
+  constexpr int MAX = max_groups(DQK, DV, RW, BN, NW, NS, FEAT);
+  if constexpr (MAX >= 4)
+    if (groups == 4) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E, 4>>(kp, grid, lds_bytes, stream);
+  if constexpr (MAX >= 2)
+    if (groups == 2) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E, 2>>(kp, grid, lds_bytes, stream);
+  return groups == 1 ? launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E>>(kp, grid, lds_bytes, stream) : hipErrorInvalidValue;
 }
 
 }  // namespace fl
@@ -36,17 +55,18 @@ hipError_t launch_fwd(const KParams& kp, int grid, int lds_bytes, hipStream_t st
 // Declares (FL_INSTANCE_DECL) or defines (FL_INSTANCE_DEF) the launcher of one instance for one element type
 // (SFX = _bf16 / _f16, ELEM = fl::bf16_t / fl::f16_t), and its row of the table (DT = FL_BF16 / FL_F16).
 #define FL_INSTANCE_DECL_(NAME, SFX) \
-  namespace fl { hipError_t launch_##NAME##SFX(const KParams&, int, int, hipStream_t); }
+  namespace fl { hipError_t launch_##NAME##SFX(const KParams&, int, int, int, hipStream_t); }
 #define FL_INSTANCE_DECL(NAME, DQK, DV, RW, BN, NW, NS, FEAT) \
   FL_INSTANCE_DECL_(NAME, _bf16) FL_INSTANCE_DECL_(NAME, _f16)
 #define FL_INSTANCE_DEF_(NAME, SFX, ELEM, DQK, DV, RW, BN, NW, NS, FEAT)                          \
   namespace fl {                                                                                  \
-  hipError_t launch_##NAME##SFX(const KParams& kp, int grid, int lds, hipStream_t s) {            \
-    return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, (FEAT), NS, ELEM>>(kp, grid, lds, s);        \
+  hipError_t launch_##NAME##SFX(const KParams& kp, int groups, int grid, int lds, hipStream_t s) { \
+    return launch_fwd_groups<DQK, DV, RW, BN, NW, NS, (FEAT), ELEM>(kp, groups, grid, lds, s);     \
   }                                                                                               \
   }
 #define FL_INSTANCE_DEF(NAME, SFX, ELEM, ...) FL_INSTANCE_DEF_(NAME, SFX, ELEM, __VA_ARGS__)
 #define FL_INSTANCE_ROW_(NAME, SFX, DT, DQK, DV, RW, BN, NW, NS, FEAT) \
-  {#NAME, DT, DQK, DV, RW, BN, NW, NS, (FEAT), fl::FwdTraits<DQK, DV, RW, BN, NW, (FEAT), NS>::LDS_FIXED_BYTES, &fl::launch_##NAME##SFX},
+  {#NAME, DT, DQK, DV, RW, BN, NW, NS, (FEAT), fl::FwdTraits<DQK, DV, RW, BN, NW, (FEAT), NS>::LDS_FIXED_BYTES, \
+   fl::max_groups(DQK, DV, RW, BN, NW, NS, (FEAT)), &fl::launch_##NAME##SFX},
 #define FL_INSTANCE_ROW(NAME, ...) \
   FL_INSTANCE_ROW_(NAME, _bf16, 0, __VA_ARGS__) FL_INSTANCE_ROW_(NAME, _f16, 2, __VA_ARGS__)

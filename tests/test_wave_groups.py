@@ -1,0 +1,107 @@
+"""Forward calls of few workgroups: 64-row workgroups and groups of waves that share the rows and take a part of the key tiles each
+(plan_few in csrc/api.hip), against the same rows in a call of many workgroups, whose waves walk all tiles in order."""
+import ctypes as C
+
+import pytest
+import torch
+
+from flashlight_amd import _ffi
+from tests.test_abi import good_params
+
+DEV = "cuda"
+NONE, CAUSAL, SLIDING, PREFIX, DOC, DOC_CAUSAL = (_ffi.MASK_NONE, _ffi.MASK_CAUSAL, _ffi.MASK_SLIDING, _ffi.MASK_PREFIX_LM,
+                                                  _ffi.MASK_DOCUMENT, _ffi.MASK_DOCUMENT_CAUSAL)
+
+
+def _shape(B, H, S, D, mask, **kw):
+    """(rows per workgroup, groups of waves) the library plans."""
+    p = good_params(B=B, Hq=H, Hkv=H, L=S, D=D)
+    p.mask_kind, p.window, p.prefix = mask, 300, 100
+    if mask in (DOC, DOC_CAUSAL):
+        p.doc_ids, p.workspace, p.workspace_bytes = 0x50000, 0x80000, 1 << 30
+    for n, v in kw.items():
+        setattr(p, n, v)
+    out = (C.c_int64 * 8)()
+    assert _ffi.load_library().fl_attn_plan(C.byref(p), out) == 0, _ffi.last_error()
+    return out[0], out[7]
+
+
+def test_which_calls_take_groups():
+    for mask in (CAUSAL, PREFIX):
+        assert _shape(2, 8, 2048, 64, mask) == (64, 2)                   # one workgroup of 128 rows per compute unit
+        assert _shape(1, 8, 2048, 64, mask) == (64, 4)                   # half of that, long walks
+        assert _shape(1, 16, 3000, 64, mask) == (64, 2)                  # up to two per compute unit, few heads
+        assert _shape(8, 16, 512, 64, mask) == (128, 1)                  # many heads
+        assert _shape(4, 16, 4096, 64, mask) == (128, 1)
+        assert _shape(1, 8, 4096, 128, mask) == (64, 2) and _shape(1, 16, 3000, 128, mask) == (128, 2)
+        assert _shape(4, 16, 512, 128, mask) == (128, 1) and _shape(2, 4, 700, 32, mask) == (128, 1)
+    assert _shape(1, 8, 4096, 64, NONE) == (128, 2) and _shape(1, 16, 4096, 64, NONE) == (128, 1)
+    assert _shape(1, 8, 4096, 128, SLIDING) == (128, 2) and _shape(2, 16, 2100, 128, SLIDING) == (128, 1)
+    # the shape of the lists does not depend on the heads
+    assert _shape(2, 16, 1000, 64, DOC) == (128, 2) and _shape(4, 16, 1000, 64, DOC) == (128, 1)
+    assert _shape(1, 16, 5000, 64, DOC_CAUSAL) == (128, 2) and _shape(1, 32, 5000, 64, DOC_CAUSAL) == (128, 1)
+    assert _shape(2, 8, 1000, 128, CAUSAL, alibi_heads=8, softcap=3.0) == (64, 2)
+    assert _shape(2, 8, 1000, 128, CAUSAL, dropout_threshold=1000) == (128, 1)
+    assert _shape(1, 1, 4096, 64, CAUSAL) == (128, 1) and _shape(6, 16, 250, 64, CAUSAL) == (128, 1)   # one head; walks of few tiles
+    assert _shape(6, 16, 512, 64, NONE)[1] == 1 and _shape(6, 16, 128, 64, DOC)[1] == 1 and _shape(6, 16, 200, 64, DOC)[1] == 2
+
+
+SIZES = {  # (batch, heads, rows, keys): parts of one tile and none, odd parts, ragged last tiles, four groups
+    CAUSAL: [(2, 16, 257, 257), (2, 18, 384, 384), (2, 16, 385, 385), (5, 8, 513, 513), (6, 2, 1025, 1025), (2, 5, 1983, 1983),
+             (6, 8, 40, 390), (6, 8, 500, 390)],
+    PREFIX: [(2, 18, 385, 385), (2, 16, 449, 449), (3, 4, 1100, 1100)],
+    SLIDING: [(8, 6, 385, 385), (3, 10, 700, 700), (2, 10, 900, 900)],
+    NONE: [(12, 8, 129, 641), (3, 10, 700, 700), (2, 8, 200, 1025)],
+    DOC: [(2, 6, 193, 193), (2, 6, 255, 255), (2, 6, 1000, 1000)],
+    DOC_CAUSAL: [(2, 6, 193, 193), (1, 6, 300, 300), (2, 6, 777, 777)],
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mask,mods", [(m, False) for m in SIZES] + [(CAUSAL, True), (NONE, True)])
+def test_groups_give_the_rows_of_a_large_call(mask, mods, D, dtype):
+    for B, H, Lq, Lk in SIZES[mask]:
+        g = torch.Generator().manual_seed(Lq + Lk + D)
+        mk = lambda *s: torch.randn(*s, generator=g).to(dtype).to(DEV)  # noqa: E731
+        q, k, v = mk(B, H, Lq, D), mk(B, H // (2 if H % 2 == 0 else 1), Lk, D), mk(B, H // (2 if H % 2 == 0 else 1), Lk, D)
+        kw = dict(mask_kind=mask)
+        if mask == SLIDING:
+            kw["window"] = 260
+        if mask == PREFIX:
+            kw["prefix"] = 100
+        if mask in (DOC, DOC_CAUSAL):
+            ids = torch.randint(0, 5, (B, Lk), generator=g)
+            kw["doc_ids"] = (ids if Lk == 1000 else ids.sort(dim=1).values).to(DEV)
+        if mods:
+            kw.update(alibi_heads=H, softcap=8.0)
+        times = -(-1100 // (B * H * -(-Lq // 128)))
+        many = {n: t.repeat(times, 1) if n == "doc_ids" else t for n, t in kw.items()}
+        r = lambda t: t.repeat(times, 1, 1, 1)  # noqa: E731
+        lse, lse_many = (torch.empty(n, H, Lq, dtype=torch.float32, device=DEV) for n in (B, B * times))
+        out = _ffi.attn_fwd(q, k, v, lse=lse, **kw)
+        ref = _ffi.attn_fwd(r(q), r(k), r(v), lse=lse_many, **many)[:B].double()
+        mean_abs = _ffi.attn_fwd(r(q), r(k), r(v.abs()), **many)[:B].double()  # sum of weight * |value|
+        # Weights are rounded to 16 bits relative to another reference (u of their size; fp16 weights far below it are subnormal, together
+        # less than 2^-15 of the row's sum), numerator and row sum alike; the result is rounded once more: both sides may be off by
+        # u (mean_abs + |o|) + u |o|.  Row statistics: u of the sum.  (a quarter more with a soft-cap, whose exponential is approximate)
+        u = (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11) * (1.25 if mods else 1.0)
+        bound = 2 * (u * (mean_abs + 2 * ref.abs()) + 2.0 ** -15 * v.abs().max().item())
+        case = f"B={B} H={H} Lq={Lq} Lk={Lk}"
+        assert torch.isfinite(out).all(), case
+        assert ((out.double() - ref).abs() <= bound).all(), case
+        assert ((lse - lse_many[:B]).abs() <= 2 * 1.4427 * u + 1e-4).all(), case
+
+
+@pytest.mark.gpu
+def test_groups_keep_infinities_and_empty_parts_apart():
+    """A part all of whose weights vanish beside the others' maximum, one that attends nothing, and a NaN that stays in its rows."""
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(1, 8, 1100, 64, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3))
+    k[:, :, 700:] *= 300  # logits of thousands in the last part only
+    q[:, :, 500, 0] = float("nan")
+    ref = _ffi.attn_fwd(*(t.repeat(16, 1, 1, 1) for t in (q, k, v)), mask_kind=CAUSAL)[:1]
+    out = _ffi.attn_fwd(q, k, v, mask_kind=CAUSAL)
+    assert torch.equal(out.isnan(), ref.isnan()) and out[:, :, 500].isnan().all() and out.isnan().sum().item() == 8 * 64
+    assert (out.nan_to_num().float() - ref.nan_to_num().float()).abs().max().item() <= 2.0 ** -5  # (values of 1 to 4: two roundings)
