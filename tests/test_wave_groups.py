@@ -31,7 +31,7 @@ def test_which_calls_take_groups():
         assert _shape(2, 8, 2048, 64, mask) == (64, 2)                   # one workgroup of 128 rows per compute unit
         assert _shape(1, 8, 2048, 64, mask) == (64, 4)                   # half of that, long walks
         assert _shape(1, 16, 3000, 64, mask) == (64, 2)                  # up to two per compute unit, few heads
-        assert _shape(8, 16, 512, 64, mask) == (128, 1)                  # many heads
+        assert _shape(8, 16, 1100, 64, mask) == (128, 1)                 # many heads
         assert _shape(4, 16, 4096, 64, mask) == (128, 1)
         assert _shape(1, 8, 4096, 128, mask) == (64, 2) and _shape(1, 16, 3000, 128, mask) == (128, 2)
         assert _shape(4, 16, 512, 128, mask) == (128, 1) and _shape(2, 4, 700, 32, mask) == (128, 1)
@@ -42,7 +42,7 @@ def test_which_calls_take_groups():
     assert _shape(1, 16, 5000, 64, DOC_CAUSAL) == (128, 2) and _shape(1, 32, 5000, 64, DOC_CAUSAL) == (128, 1)
     assert _shape(2, 8, 1000, 128, CAUSAL, alibi_heads=8, softcap=3.0) == (64, 2)
     assert _shape(2, 8, 1000, 128, CAUSAL, dropout_threshold=1000) == (128, 1)
-    assert _shape(1, 1, 4096, 64, CAUSAL) == (128, 1) and _shape(6, 16, 250, 64, CAUSAL) == (128, 1)   # one head; walks of few tiles
+    assert _shape(1, 1, 4096, 64, CAUSAL) == (128, 1) and _shape(6, 16, 250, 64, CAUSAL) == (64, 1)    # one head; walks of few tiles
     assert _shape(6, 16, 512, 64, NONE)[1] == 1 and _shape(6, 16, 128, 64, DOC)[1] == 1 and _shape(6, 16, 200, 64, DOC)[1] == 2
 
 
@@ -105,3 +105,27 @@ def test_groups_keep_infinities_and_empty_parts_apart():
     out = _ffi.attn_fwd(q, k, v, mask_kind=CAUSAL)
     assert torch.equal(out.isnan(), ref.isnan()) and out[:, :, 500].isnan().all() and out.isnan().sum().item() == 8 * 64
     assert (out.nan_to_num().float() - ref.nan_to_num().float()).abs().max().item() <= 2.0 ** -5  # (values of 1 to 4: two roundings)
+
+
+def test_which_calls_take_64_row_workgroups():
+    assert _shape(16, 16, 700, 64, CAUSAL) == (64, 1) and _shape(16, 16, 1024, 64, CAUSAL) == (128, 1)
+    assert _shape(16, 16, 128, 64, CAUSAL) == (128, 1) and _shape(16, 16, 700, 128, CAUSAL) == (128, 1)
+    assert _shape(16, 16, 700, 64, PREFIX, prefix=350) == (64, 1) and _shape(16, 16, 700, 64, PREFIX, prefix=351) == (128, 1)
+    assert _shape(4, 16, 4096, 64, SLIDING, window=895) == (64, 1) and _shape(4, 16, 4096, 64, SLIDING, window=896) == (128, 1)
+    assert _shape(4, 16, 4096, 64, NONE) == (128, 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,kw", [(CAUSAL, {}), (PREFIX, dict(prefix=60)), (SLIDING, dict(window=70)), (SLIDING, dict(window=300))])
+@pytest.mark.parametrize("S", [129, 191, 192, 193, 500])
+def test_64_row_workgroups_against_fp64(mask, kw, S):
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (torch.randn(8, 66, S, 64, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3))
+    out = _ffi.attn_fwd(q, k, v, mask_kind=mask, **kw)[7].double()
+    i = torch.arange(S, device=DEV)
+    d = i[:, None] - i[None, :]
+    live = (d >= 0) & (d <= kw.get("window", S)) | (i[None, :] < kw.get("prefix", 0))
+    w = torch.softmax((torch.matmul(q[7].double(), k[7].double().transpose(1, 2).contiguous()) / 8).masked_fill(~live, -torch.inf), -1)
+    ref, mean_abs = torch.matmul(w, v[7].double()), torch.matmul(w, v[7].double().abs())
+    # weights rounded to u = 2^-8 of their size, numerator and row sum alike, and the result once more
+    assert ((out - ref).abs() <= 2.0 ** -8 * (mean_abs + 2 * ref.abs()) + 1e-5).all()
