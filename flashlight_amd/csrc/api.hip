@@ -37,24 +37,6 @@ static __global__ void doc_table_kernel(const int64_t* ids, int64_t ids_stride, 
   table[2 * (int64_t)i + 1] = mx;
 }
 
-// (min, max) over a wave of one int64 per lane, wave-uniform.  Nearly every 32- or 64-position run lies inside one
-// document, so "all equal to the first lane's" is tested with one ballot before the reduction.
-static __device__ __forceinline__ void wave_id_range(int64_t x, int64_t& mn, int64_t& mx) {
-  const int64_t first = uniform_i64(x);
-  mn = mx = first;
-  if (__builtin_amdgcn_ballot_w64(x != first) != 0) {
-    int64_t a = x, b = x;
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) {
-      const int64_t a2 = __shfl_xor(a, d, 64), b2 = __shfl_xor(b, d, 64);
-      a = a2 < a ? a2 : a;
-      b = b2 > b ? b2 : b;
-    }
-    mn = uniform_i64(a);
-    mx = uniform_i64(b);
-  }
-}
-
 // Forward pre-pass for document masks, one workgroup of 1024 threads per (batch, query tile of `bm` rows), straight from
 // the ids: lists the key tiles (of `bn` keys) that some row of the query tile attends, with the class of each for every
 // wave of the forward (`rw` rows per wave): EMPTY when the id ranges of the tile's keys and the wave's rows do not meet,
@@ -1161,11 +1143,22 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   if (p->flags & FL_FLAG_F32_RESULT) kp.o_wide = 2;
   const int grid = p->B * p->Hq * kp.n_qtiles;
 
+  const int groups = groups_for(in, p);
+  int lds = (int)lds_bytes_for(in, p) + (groups - 1) * in->lds_fixed_bytes;
+
   if (is_doc(p->mask_kind)) {
     const DocScratch d = doc_scratch(p->B, p->Lk, bm, in->bn);
     uint32_t* lists = reinterpret_cast<uint32_t*>(static_cast<unsigned char*>(p->workspace) + d.table_bytes);
     int32_t* order = reinterpret_cast<int32_t*>(static_cast<unsigned char*>(p->workspace) + d.table_bytes + d.lists_bytes);
-    if (!(p->flags & FL_FLAG_DOC_PREPARED)) {
+    // Few key tiles and workgroups: each workgroup lists its own tiles (fwd_kernel.h) and the pre-pass is not launched.  Up to two rounds:
+    // beyond, every workgroup's own list and the order that is missing cost more than the launches (us, launches -> own: 4 x 32 heads
+    // of 837 ids, head dim 64, 896 workgroups 39.7 -> 36.3; 2 x 32 of 2500, 1280: 59.8 -> 60.9; 16 x 16 of 1500, 3072: 86 -> 92).
+    const bool own = !(p->flags & FL_FLAG_DOC_PREPARED) && kp.n_ktiles <= fl::kOwnListTiles && grid <= 1024 &&
+                     lds + fl::kOwnListBytes <= fl::kMaxLdsBytes;
+    if (own) {
+      kp.doc_own = 1;
+      lds += fl::kOwnListBytes;
+    } else if (!(p->flags & FL_FLAG_DOC_PREPARED)) {
       static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fl::doc_lists_kernel),
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, fl::kMaxLdsBytes - 128);
       if (attr != hipSuccess) return fail((int)attr, "doc_lists_kernel: %s", hipGetErrorString(attr));
@@ -1183,8 +1176,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
     kp.doc_list_stride = (int)d.list_stride;
     kp.doc_order = order;
   }
-  const int groups = groups_for(in, p);
-  hipError_t e = in->launch(kp, groups, grid, (int)lds_bytes_for(in, p) + (groups - 1) * in->lds_fixed_bytes, stream);
+  hipError_t e = in->launch(kp, groups, grid, lds, stream);
   if (e != hipSuccess) return fail((int)e, "launch of %s failed: %s", in->name, hipGetErrorString(e));
   return 0;
 }

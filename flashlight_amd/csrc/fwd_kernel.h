@@ -48,6 +48,7 @@ enum : int { TILE_EMPTY = 0, TILE_PARTIAL = 1, TILE_FULL = 2 };
 // Key tiles are numbered in 16 bits inside the LDS tile list.
 constexpr int kMaxKeyTiles = 65535;
 // Granularity (positions) of the document-id min/max table built by doc_table_kernel.
+constexpr int kOwnListTiles = 64, kOwnListBytes = 2 * 64 * 8 + 2 * 8 * 8;  // (behind the list: (min, max) id of 64 key tiles and 8 waves' rows)
 constexpr int kDocBlock = 32;
 
 struct KParams {
@@ -68,11 +69,14 @@ struct KParams {
   // Document masks: the key tiles each query tile visits, listed by doc_lists_kernel before the launch (the lists are
   // the same for every head): per (batch, query tile) doc_list_stride words, word 0 = number of entries, then the
   // entries in key order (bits 0-15 tile index, two class bits per wave from bit 16 on).
-  const uint32_t* doc_lists;
+  uint32_t* doc_lists;
   int32_t doc_list_stride;  // words per (batch, query tile): a multiple of 4, at least n_ktiles + 1
   // per batch row the query tiles ordered by falling list length (doc_order_kernel): workgroups are dealt in that order,
   // so that the ones still running when the grid drains are the short ones whatever the document layout
-  const int32_t* doc_order;
+  int32_t* doc_order;
+  // The lists have not been made by a launch of their own (at most kOwnListTiles key tiles): every workgroup lists its tiles itself, and
+  // those of a batch row's first head leave the lists in doc_lists for later calls.  doc_order then says that there is no order (-1).
+  int32_t doc_own;
   int32_t alibi_heads;
   float softcap;
   const bf16_t* bias[2];
@@ -238,6 +242,10 @@ __device__ __forceinline__ A& pick(A& a, A& b) {
   if constexpr (FIRST) return a; else return b;
 }
 
+// Every lambda of the kernel must be inlined: an outlined one would take its captures (the accumulators) by address
+// through scratch memory.
+#define FL_INLINE __attribute__((always_inline))
+
 // ---- mask logic (integer, shared by the tile classifier and the element predicate) -------------------------------
 
 // Class of the key tile [k0, k1) against query rows [q0, q1) for the positional part of the mask.
@@ -267,6 +275,40 @@ __device__ __forceinline__ void doc_range(const int64_t* table, int p0, int p1, 
     int64_t a = table[2 * b], c = table[2 * b + 1];
     mn = a < mn ? a : mn;
     mx = c > mx ? c : mx;
+  }
+}
+
+// (min, max) over a wave of one int64 per lane, wave-uniform.  Nearly every 32- or 64-position run lies inside one
+// document, so "all equal to the first lane's" is tested with one ballot before the reduction.  The reduction exchanges lanes in
+// registers (quads, halves and whole rows of 16; the four rows' results in scalars): six trips through LDS are what a short call waits for.
+template <int CTRL>
+__device__ __forceinline__ int64_t dpp_i64(int64_t x) {
+  const int lo = (int)(uint32_t)(uint64_t)x, hi = (int)(uint32_t)((uint64_t)x >> 32);
+  return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, true) |
+                   ((uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, true) << 32));
+}
+__device__ __forceinline__ void wave_id_range(int64_t x, int64_t& mn, int64_t& mx) {
+  const int64_t first = uniform_i64(x);
+  mn = mx = first;
+  if (__builtin_amdgcn_ballot_w64(x != first) != 0) {
+    int64_t a = x, b = x;
+    auto fold = [&](int64_t a2, int64_t b2) FL_INLINE {
+      a = a2 < a ? a2 : a;
+      b = b2 > b ? b2 : b;
+    };
+    fold(dpp_i64<0xB1>(a), dpp_i64<0xB1>(b));    // quad_perm 1 0 3 2
+    fold(dpp_i64<0x4E>(a), dpp_i64<0x4E>(b));    // quad_perm 2 3 0 1
+    fold(dpp_i64<0x141>(a), dpp_i64<0x141>(b));  // row_half_mirror
+    fold(dpp_i64<0x140>(a), dpp_i64<0x140>(b));  // row_mirror: a row of 16 agrees
+    auto row = [&](int64_t v, int lane) FL_INLINE {
+      return (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(uint64_t)v, lane) |
+                       ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), lane) << 32));
+    };
+    const int64_t a0 = row(a, 0), a1 = row(a, 16), a2 = row(a, 32), a3 = row(a, 48);
+    const int64_t b0 = row(b, 0), b1 = row(b, 16), b2 = row(b, 32), b3 = row(b, 48);
+    const int64_t a01 = a0 < a1 ? a0 : a1, a23 = a2 < a3 ? a2 : a3, b01 = b0 > b1 ? b0 : b1, b23 = b2 > b3 ? b2 : b3;
+    mn = a01 < a23 ? a01 : a23;
+    mx = b01 > b23 ? b01 : b23;
   }
 }
 
@@ -311,9 +353,6 @@ struct BiasLayout {
 // Scheduling pipeline for the straight-line tile step (see fwd_kernel): instruction classes of
 // __builtin_amdgcn_sched_group_barrier.
 enum : int { SG_VALU = 0x2, SG_MFMA = 0x8, SG_DS_READ = 0x100, SG_TRANS = 0x400 };
-// Every lambda of the kernel must be inlined: an outlined one would take its captures (the accumulators) by address
-// through scratch memory.
-#define FL_INLINE __attribute__((always_inline))
 
 #ifndef FL_SCHED
 #define FL_SCHED 1
@@ -472,7 +511,12 @@ void fwd_kernel(const KParams p) {
     qt = nq - 1 - rem / gg;
     bh = base + G * g + rem % gg;
     // document masks: the work of a query tile is the length of its tile list, known from the pre-pass
-    if constexpr (kDoc) qt = p.doc_order[(bh / p.Hq) * nq + rem / gg];
+    if constexpr (kDoc) {
+      if (!p.doc_own) {
+        const int32_t* order = p.doc_order + (bh / p.Hq) * nq;
+        if (order[0] >= 0) qt = order[rem / gg];
+      }
+    }
   }
   const int head = bh % p.Hq, batch = bh / p.Hq;
   const int kvh = head / p.group;
@@ -490,7 +534,7 @@ void fwd_kernel(const KParams p) {
     // the list of this (batch, query tile) goes global -> LDS in whole wave transfers (64 chunks of 16 bytes each; chunks
     // past the end repeat the last one); it is awaited, together with the first K/V transfers' predecessors, right
     // before the key loop, so that the query loads below run under its latency
-    const int n_chunks = p.doc_list_stride / 4;
+    const int n_chunks = p.doc_own ? 0 : p.doc_list_stride / 4;
     const uint64_t lbase = uniform_ptr(p.doc_lists + ((int64_t)batch * p.n_qtiles + qt) * p.doc_list_stride);
     const unsigned lds_l = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem_all + KG * T::LIST_OFF);
     for (int c0 = wave * 64; c0 < n_chunks; c0 += NW * 64)
@@ -1232,6 +1276,70 @@ void fwd_kernel(const KParams p) {
         }
     };
 
+    // Documents of few key tiles, whose pre-pass was not launched (doc_own): the list is made here, by the steps of doc_lists_kernel.  A
+    // wave per key tile leaves its ids' (min, max) in LDS; every wave then classifies all tiles, one per lane, for all waves, and writes
+    // the same list.  The two launches ahead of this one were 6 to 7 us; here it is a round trip to memory and some 150 instructions
+    // (8 heads of 837 ids, head dim 64: 21.5 -> 15.7 us; 16 x 16 of 100: 16.0 -> 10.6).
+    if constexpr (kDoc) {
+      if (p.doc_own) {
+        constexpr int WAVES = KG * NW, PER = kOwnListTiles / WAVES;
+        static_assert(kOwnListTiles % WAVES == 0 && (BN == 32 || BN == 64) && RW == 32, "ids of a tile in one load");
+        uint32_t* const list = reinterpret_cast<uint32_t*>(smem_all + KG * T::LIST_OFF);
+        int64_t* const krange = reinterpret_cast<int64_t*>(smem_all + KG * T::LIST_OFF + 1024);
+        int64_t* const qrange = krange + 2 * kOwnListTiles;
+        const int64_t* ids = p.doc_ids + (int64_t)batch * p.doc_stride;
+        const int t_end = p.mask_kind == MASK_DOC_CAUSAL ? min(nk, (min(q0 + BM, p.Lk) - 1) / BN + 1) : nk;
+        const int w0 = group * NW + wave;
+        int64_t kid[PER];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) kid[u] = ids[min(min(w0 + WAVES * u, t_end - 1) * BN + lane % BN, p.Lk - 1)];
+        int64_t mn, mx;
+        wave_id_range(ids[min(qw0 + lane % RW, p.Lk - 1)], mn, mx);
+        if (lane == 0) {
+          qrange[2 * wave] = mn;
+          qrange[2 * wave + 1] = mx;
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+          const int t = w0 + WAVES * u;
+          if (t >= t_end) break;
+          wave_id_range(kid[u], mn, mx);
+          if (lane == 0) {
+            krange[2 * t] = mn;
+            krange[2 * t + 1] = mx;
+          }
+        }
+        __syncthreads();
+        const int t = min(lane, t_end - 1), k0 = t * BN, k1 = min(k0 + BN, p.Lk);
+        const int64_t kmn = krange[2 * t], kmx = krange[2 * t + 1];
+        uint32_t classes = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+          const int a = q0 + w * RW, e = min(a + RW, p.Lk);
+          const int64_t qmn = qrange[2 * w], qmx = qrange[2 * w + 1];
+          int cw = TILE_EMPTY;
+          if (a < e && !(kmx < qmn || kmn > qmx)) {
+            cw = classify_positional(p.mask_kind, a, e, k0, k1, 0, 0);
+            if (cw == TILE_FULL && (!(kmn == kmx && qmn == qmx && kmn == qmn) || k0 + BN > p.Lk)) cw = TILE_PARTIAL;
+          }
+          classes |= (uint32_t)cw << (2 * w);
+        }
+        const bool keep = lane < t_end && classes != 0;
+        const uint64_t live = __builtin_amdgcn_ballot_w64(keep);
+        const int at = __builtin_popcountll(live & ((1ull << lane) - 1)), count = __builtin_popcountll(live);
+        const uint32_t entry = classes << 16 | (uint32_t)t;
+        if (keep) list[1 + at] = entry;
+        if (lane == 0) list[0] = (uint32_t)count;
+        if (head == 0 && w0 == 0) {
+          uint32_t* out = p.doc_lists + ((int64_t)batch * p.n_qtiles + qt) * p.doc_list_stride;
+          if (keep) out[1 + at] = entry;
+          if (lane == 0) {
+            out[0] = (uint32_t)count;
+            if (qt == 0) p.doc_order[batch * p.n_qtiles] = -1;
+          }
+        }
+      }
+    }
     if constexpr (kDoc) dma_wait<0>();  // the tile list (issued first thing) has landed
     // (the previous branch is done with the LDS buffers; every wave's share of the tile list is visible to all)
     if (br > 0 || kDoc) __syncthreads();

@@ -1,0 +1,55 @@
+"""Document-mask forwards whose workgroups list their key tiles themselves (doc_own in csrc/fwd_kernel.h): the lists of the launch they
+stand in for, at the edges of 64 tiles, for ids of any order and size; workspaces they prepared, read by calls of any size."""
+import pytest
+import torch
+
+from flashlight_amd import _ffi
+
+DEV = "cuda"
+KINDS = ("sorted", "unsorted", "huge", "one", "pairs")
+
+
+def _ids(kind, B, S, g):
+    if kind == "one":
+        return torch.full((B, S), -7, dtype=torch.int64)
+    if kind == "pairs":
+        return torch.arange(S).repeat(B, 1) // 2
+    ids = torch.randint(-3, 4, (B, S), generator=g)
+    return ids.sort(dim=1).values if kind == "sorted" else ids * 2 ** 40 + (1 << 33) if kind == "huge" else ids
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask", [_ffi.MASK_DOCUMENT, _ffi.MASK_DOCUMENT_CAUSAL])
+@pytest.mark.parametrize("kind", KINDS)
+@pytest.mark.parametrize("S", [1, 31, 33, 64, 129, 700, 4096, 4097])
+def test_own_lists_are_those_of_the_launch(S, kind, mask):
+    """Head dim 32 has one form of the kernel: a call of many workgroups, whose lists are made by a launch, gives the same bits."""
+    g = torch.Generator().manual_seed(S)
+    ids = _ids(kind, 2, S, g).to(DEV)
+    q, k, v = (torch.randn(2, 2, S, 32, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3))
+    out = _ffi.attn_fwd(q, k, v, mask_kind=mask, doc_ids=ids)
+    times = 1024 // (2 * -(-S // 128)) + 1
+    many = _ffi.attn_fwd(*(t.repeat(1, times, 1, 1) for t in (q, k, v)), mask_kind=mask, doc_ids=ids)
+    assert torch.equal(out, many[:, :2]) and torch.equal(out, many[:, -2:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,S", [(64, 600), (128, 2048), (128, 2049), (64, 1)])
+def test_prepared_workspaces_serve_calls_of_other_heads(D, S):
+    """What a call of few workgroups leaves in the workspace has lists but no order of the query tiles; calls of many workgroups read
+    it all the same, and the other way round."""
+    g = torch.Generator().manual_seed(D + S)
+    ids = torch.randint(0, 5, (2, S), generator=g).sort(dim=1).values.to(DEV)
+    few, many = 2, 600 // -(-S // 128) + 1
+    operands = {H: tuple(torch.randn(2, H, S, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3)) for H in (few, many)}
+    plain = {H: _ffi.attn_fwd(*x, mask_kind=_ffi.MASK_DOCUMENT_CAUSAL, doc_ids=ids) for H, x in operands.items()}
+    for first, then in ((few, many), (many, few), (few, few)):
+        ws = _ffi.DocWorkspace()
+        for H in (first, then):
+            if ws.key is not None:  # the C interface does not ask for the same heads; the Python handle does
+                ws.key = ws.key[:5] + (H, H) + ws.key[7:]
+            q, k, v = operands[H]
+            ready = ws.buffer
+            out = _ffi.attn_fwd(q, k, v, mask_kind=_ffi.MASK_DOCUMENT_CAUSAL, doc_ids=ids, doc_workspace=ws)
+            assert ready is None or ws.buffer is ready  # (not prepared anew)
+            assert torch.equal(out, plain[H]), (first, then, H)
