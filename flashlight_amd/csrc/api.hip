@@ -306,6 +306,12 @@ FewPlan plan_few(const fl_attn_params* p, uint32_t want) {
     x.groups = narrow && tiles <= 128 && p->Lk >= 1024 ? 4 : 2;
   } else if (tiles <= 256) {
     x.groups = 2;
+    // (walks of one length, half as many tiles as compute units: 64 rows as well, head dim 64 in four groups: 8 of 2048 24.4 -> 17.2, with
+    // ALiBi and soft-cap 35.9 -> 23.7, 2 of 8192 77.5 -> 49.2; head dim 128, 8 of 2048 33.8 -> 30.8 and 43.2 -> 34.6)
+    if (!(want & fl::F_DOC) && tiles <= 128 && walk >= 1024) {
+      x.waves = 2;
+      x.groups = narrow ? 4 : 2;
+    }
   } else if (want & fl::F_DOC) {
     // (the walks are as long as the documents, which only the device knows: 1 x 16 x 4768, documents of 512 to 2384: 77 -> 55, but
     // 1 x 16 x 4096 in documents of 512 each: 23.5 -> 28.9; from 32 heads on it is even or loses whatever the documents)

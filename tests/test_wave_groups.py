@@ -36,6 +36,7 @@ def test_which_calls_take_groups():
         assert _shape(1, 8, 4096, 128, mask) == (64, 2) and _shape(1, 16, 3000, 128, mask) == (128, 2)
         assert _shape(4, 16, 512, 128, mask) == (128, 1) and _shape(2, 4, 700, 32, mask) == (128, 1)
     assert _shape(1, 8, 4096, 64, NONE) == (128, 2) and _shape(1, 16, 4096, 64, NONE) == (128, 1)
+    assert _shape(1, 4, 4096, 64, NONE) == (64, 4) and _shape(1, 4, 4096, 128, SLIDING, window=1000) == (64, 2)
     assert _shape(1, 8, 4096, 128, SLIDING) == (128, 2) and _shape(2, 16, 2100, 128, SLIDING) == (128, 1)
     # the shape of the lists does not depend on the heads
     assert _shape(2, 16, 1000, 64, DOC) == (128, 2) and _shape(4, 16, 1000, 64, DOC) == (128, 1)
@@ -50,8 +51,8 @@ SIZES = {  # (batch, heads, rows, keys): parts of one tile and none, odd parts, 
     CAUSAL: [(2, 16, 257, 257), (2, 18, 384, 384), (2, 16, 385, 385), (5, 8, 513, 513), (6, 2, 1025, 1025), (2, 5, 1983, 1983),
              (6, 8, 40, 390), (6, 8, 500, 390)],
     PREFIX: [(2, 18, 385, 385), (2, 16, 449, 449), (3, 4, 1100, 1100)],
-    SLIDING: [(8, 6, 385, 385), (3, 10, 700, 700), (2, 10, 900, 900)],
-    NONE: [(12, 8, 129, 641), (3, 10, 700, 700), (2, 8, 200, 1025)],
+    SLIDING: [(8, 6, 385, 385), (3, 10, 700, 700), (2, 10, 900, 900), (2, 4, 1500, 1500)],
+    NONE: [(12, 8, 129, 641), (3, 10, 700, 700), (2, 8, 200, 1025), (3, 3, 1100, 1100), (4, 16, 300, 1500)],
     DOC: [(2, 6, 193, 193), (2, 6, 255, 255), (2, 6, 1000, 1000)],
     DOC_CAUSAL: [(2, 6, 193, 193), (1, 6, 300, 300), (2, 6, 777, 777)],
 }
@@ -68,7 +69,7 @@ def test_groups_give_the_rows_of_a_large_call(mask, mods, D, dtype):
         q, k, v = mk(B, H, Lq, D), mk(B, H // (2 if H % 2 == 0 else 1), Lk, D), mk(B, H // (2 if H % 2 == 0 else 1), Lk, D)
         kw = dict(mask_kind=mask)
         if mask == SLIDING:
-            kw["window"] = 260
+            kw["window"] = 260 if Lk < 1000 else 1100
         if mask == PREFIX:
             kw["prefix"] = 100
         if mask in (DOC, DOC_CAUSAL):
