@@ -1158,7 +1158,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
     int32_t* order = reinterpret_cast<int32_t*>(static_cast<unsigned char*>(p->workspace) + d.table_bytes + d.lists_bytes);
     // Few key tiles and workgroups: each workgroup lists its own tiles (fwd_kernel.h) and the pre-pass is not launched.  Up to two rounds:
     // beyond, every workgroup's own list and the order that is missing cost more than the launches (us, launches -> own: 4 x 32 heads
-    // of 837 ids, head dim 64, 896 workgroups 39.7 -> 36.3; 2 x 32 of 2500, 1280: 59.8 -> 60.9; 16 x 16 of 1500, 3072: 86 -> 92).
+    // of 837 ids, head dim 64, 896 workgroups 39.3 -> 37.3; 2 x 32 of 2500, 1280: 59.8 -> 60.9; 16 x 16 of 1500, 3072: 86 -> 92).
     const bool own = !(p->flags & FL_FLAG_DOC_PREPARED) && kp.n_ktiles <= fl::kOwnListTiles && grid <= 1024 &&
                      lds + fl::kOwnListBytes <= fl::kMaxLdsBytes;
     if (own) {

@@ -514,7 +514,8 @@ void fwd_kernel(const KParams p) {
     if constexpr (kDoc) {
       if (!p.doc_own) {
         const int32_t* order = p.doc_order + (bh / p.Hq) * nq;
-        if (order[0] >= 0) qt = order[rem / gg];
+        const int head_of_order = order[0], mine = order[rem / gg];  // (both in flight together)
+        qt = head_of_order >= 0 ? mine : qt;
       }
     }
   }
@@ -1279,9 +1280,9 @@ void fwd_kernel(const KParams p) {
     // Documents of few key tiles, whose pre-pass was not launched (doc_own): the list is made here, by the steps of doc_lists_kernel.  A
     // wave per key tile leaves its ids' (min, max) in LDS; every wave then classifies all tiles, one per lane, for all waves, and writes
     // the same list.  The two launches ahead of this one were 6 to 7 us; here it is a round trip to memory and some 150 instructions
-    // (8 heads of 837 ids, head dim 64: 21.5 -> 15.7 us; 16 x 16 of 100: 16.0 -> 10.6).
+    // (8 heads of 837 ids, head dim 64: 21.5 -> 16.3 us; 16 x 16 of 100: 16.0 -> 11.5).
     if constexpr (kDoc) {
-      if (p.doc_own) {
+      if (__builtin_expect(p.doc_own, 0)) {
         constexpr int WAVES = KG * NW, PER = kOwnListTiles / WAVES;
         static_assert(kOwnListTiles % WAVES == 0 && (BN == 32 || BN == 64) && RW == 32, "ids of a tile in one load");
         uint32_t* const list = reinterpret_cast<uint32_t*>(smem_all + KG * T::LIST_OFF);
@@ -1299,11 +1300,23 @@ void fwd_kernel(const KParams p) {
           qrange[2 * wave] = mn;
           qrange[2 * wave + 1] = mx;
         }
+        // (a loop over the few tiles with a boundary in them: the reduction PER times over is 10 KB of instructions, which every
+        // workgroup of a large call, that has its lists from the launch, fetched past: 0.5 %)
+        uint32_t mixed = 0;
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
+          const int64_t first = uniform_i64(kid[u]);
           const int t = w0 + WAVES * u;
-          if (t >= t_end) break;
-          wave_id_range(kid[u], mn, mx);
+          if (t < t_end && __builtin_amdgcn_ballot_w64(kid[u] != first) != 0) mixed |= 1u << u;
+          if (lane == 0 && t < t_end) krange[2 * t] = krange[2 * t + 1] = first;
+        }
+#pragma unroll 1
+        for (; mixed != 0; mixed &= mixed - 1) {
+          const int which = (int)__builtin_ctz(mixed), t = w0 + WAVES * which;
+          int64_t x = kid[0];
+#pragma unroll
+          for (int u = 1; u < PER; ++u) x = which == u ? kid[u] : x;
+          wave_id_range(x, mn, mx);
           if (lane == 0) {
             krange[2 * t] = mn;
             krange[2 * t + 1] = mx;
