@@ -339,13 +339,15 @@ const fl::Instance* select_instance(const fl_attn_params* p) {
   // workgroups of 64 rows: less of each tile lies outside the mask, and more independent workgroups overlap their first loads.
   // Head dim 64, us, 128 rows -> 64: window, 4 x 16 heads of 4096: 64 keys 38.6 -> 34.2, 256 50.7 -> 45.0, 700 78.2 -> 75.5, 1200 105.6 ->
   // 107.2; causal, 20 x 32 of 138 19.3 -> 15.2, 30 x 16 of 700 69.7 -> 62.5, 16 x 16 of 1000 61.6 -> 60.0, 4 x 32 of 1500 even; a prefix
-  // of 200 in 700 48.9 -> 44.5, of 600 57.8 -> 60.3; two key tiles at most (16 x 16 of 128 under a window of 64): 7.3 -> 8.1.
+  // of 200 in 700 48.9 -> 44.5, of 600 57.8 -> 60.3; two key tiles at most (16 x 16 of 128 under a window of 64): 7.3 -> 8.1,
+  // and whole short walks while 128-row workgroups all run at once: causal, 15 x 8 of 151 7.2 -> 8.0, 6 x 16 of 300 9.3 -> 10.1, of 370 even.
   // Head dim 128, whose tile then has 32 keys: from a window of 256 on the 4-wave tile ties or wins on warm operands and wins by 4 % on
   // cold ones; ALiBi and soft-cap under a window of 100, 4 x 32 of 2000: 69.0 -> 59.0.
   const int64_t visited = p->mask_kind == FL_MASK_SLIDING ? std::min<int64_t>(p->Lk, (int64_t)p->window + 128) : p->Lk;
   const bool thin = p->mask_kind == FL_MASK_SLIDING ||
                     (p->Dqk == 64 && (p->mask_kind == FL_MASK_CAUSAL || (p->mask_kind == FL_MASK_PREFIX_LM && p->prefix <= p->Lk / 2)));
-  const bool short_loop = thin && (p->Dqk == 64 ? visited > 128 && visited < 1024 : visited < 384);
+  const bool many = (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128) > 512;
+  const bool short_loop = thin && (p->Dqk == 64 ? visited >= (many || visited < p->Lk ? 129 : 384) && visited < 1024 : visited < 384);
   // Unmasked calls at head dim 128 whose grid still fills the part twice over with 256-row workgroups take the
   // 8-wave tile: one workgroup per compute unit brings every K/V tile in once for 256 rows instead of twice, which on
   // ordinary data is worth more than the second workgroup's independence (2.4 % on N(0,1) operands; at head dim 64,

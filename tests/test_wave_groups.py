@@ -43,7 +43,7 @@ def test_which_calls_take_groups():
     assert _shape(1, 16, 5000, 64, DOC_CAUSAL) == (128, 2) and _shape(1, 32, 5000, 64, DOC_CAUSAL) == (128, 1)
     assert _shape(2, 8, 1000, 128, CAUSAL, alibi_heads=8, softcap=3.0) == (64, 2)
     assert _shape(2, 8, 1000, 128, CAUSAL, dropout_threshold=1000) == (128, 1)
-    assert _shape(1, 1, 4096, 64, CAUSAL) == (128, 1) and _shape(6, 16, 250, 64, CAUSAL) == (64, 1)    # one head; walks of few tiles
+    assert _shape(1, 1, 4096, 64, CAUSAL) == (128, 1) and _shape(6, 16, 250, 64, CAUSAL) == (128, 1)    # one head; walks of few tiles
     assert _shape(6, 16, 512, 64, NONE)[1] == 1 and _shape(6, 16, 128, 64, DOC)[1] == 1 and _shape(6, 16, 200, 64, DOC)[1] == 2
 
 
@@ -110,6 +110,7 @@ def test_groups_keep_infinities_and_empty_parts_apart():
 
 def test_which_calls_take_64_row_workgroups():
     assert _shape(16, 16, 700, 64, CAUSAL) == (64, 1) and _shape(16, 16, 1024, 64, CAUSAL) == (128, 1)
+    assert _shape(15, 8, 151, 64, CAUSAL) == (128, 1) and _shape(30, 16, 151, 64, CAUSAL) == (64, 1)
     assert _shape(16, 16, 128, 64, CAUSAL) == (128, 1) and _shape(16, 16, 700, 128, CAUSAL) == (128, 1)
     assert _shape(16, 16, 700, 64, PREFIX, prefix=350) == (64, 1) and _shape(16, 16, 700, 64, PREFIX, prefix=351) == (128, 1)
     assert _shape(4, 16, 4096, 64, SLIDING, window=895) == (64, 1) and _shape(4, 16, 4096, 64, SLIDING, window=896) == (128, 1)
