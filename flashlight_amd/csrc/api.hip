@@ -696,6 +696,7 @@ bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, 
     else return false;
   }
   if (pi < 0) return false;
+  if (p->B % p->bias_batch_div[pi] != 0) return false;  // (workgroups walk whole groups of entries; the general kernel divides per entry)
   // Where the general kernel has to read the bias two bytes at a time (odd lengths, fp32), this one is three to five times sooner
   // (bf16, us: 414 x 4 x 494 x 494, head dim 32: 806 -> 201; 34 x 4 x 235 x 235, head dim 64: 43 -> 17; 28 x 4 x 106 x 106: 14 -> 6).  Where
   // that kernel can stage the bias beside its tiles, this one is ahead at head dim 32 with three or four waves, which fill the

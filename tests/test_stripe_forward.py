@@ -1,5 +1,6 @@
 """The shared-bias stripe forward (csrc/stripe_kernel.h): lengths at the edges of its 64-key waves and 32-row blocks, against the
 fp32 oracle; fp32 operands; rows that attend nothing or whose logits are large; which calls take it."""
+import ctypes as C
 import math
 
 import pytest
@@ -95,3 +96,37 @@ def test_rows_that_attend_nothing_and_large_logits(S, fill):
     assert (out[1] == 0).all() and (lse[1] == float("inf")).all()
     for n in (0, 2, 3, 4):
         assert ((out[n] - ref[n]).norm() / ref[n].norm()).item() < 3e-3, n
+
+
+UNEVEN = [(6, 4, 250), (5, 8, 250), (7, 6, 256), (3, 2, 63)]  # batch, divisor that leaves a remainder (or is larger), length
+
+
+@pytest.mark.parametrize("B,div,S", UNEVEN)
+def test_a_batch_that_the_divisor_does_not_divide_goes_elsewhere(B, div, S):
+    """Entry n takes bias n / divisor whatever the batch size; the stripe kernel's workgroups walk whole groups of entries."""
+    p = params(S=S, lse=0x90000, B=B)
+    p.bias_batch_div[0] = div
+    plan = _ffi.plan(p)
+    assert plan["streaming"] == 0 and plan["workgroups"] == B * p.Hq * -(-S // plan["rows_per_workgroup"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,div,S", UNEVEN)
+def test_a_batch_that_the_divisor_does_not_divide(B, div, S):
+    g = torch.Generator().manual_seed(B * S)
+    H, D, groups = 2, 32, -(-B // div)
+    q, k, v = (torch.randn(B, H, S, D, generator=g).to(torch.bfloat16) for _ in range(3))
+    pair = torch.randn(groups, H, S, S, generator=g).to(torch.bfloat16)
+    lib, dev = _ffi.load_library(), [t.to(DEV) for t in (q, k, v, pair)]
+    out = torch.full((B, H, S, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    lse = torch.full((B, H, S), float("nan"), device=DEV)
+    p, keep = _ffi._fill_params(lib, *dev[:3], out, H, H, None, 0, 0, 0, None, 0, 0.0, [(dev[3][:1], B)], None, False, 0.0, None)
+    p.bias_strides[0][0], p.bias_batch_div[0], p.lse = H * S * S, div, lse.data_ptr()   # (the Python entries refuse such divisors)
+    assert lib.fl_attn_fwd(C.byref(p), torch.cuda.current_stream().cuda_stream) == 0, _ffi.last_error()
+    s = q.double() @ k.double().transpose(-1, -2) / D ** 0.5 + pair.double()[torch.arange(B) // div]
+    ref = torch.softmax(s, -1) @ v.double()
+    # weights and results rounded to bf16, as above
+    assert ((out.cpu().double() - ref).norm() / ref.norm()).item() < 3e-3
+    # every rounded weight is off by at most 2^-9 of its size, and so is their sum: 2^-9 / ln 2 in log2 units (1e-4: the exponential)
+    assert (lse.cpu().double() - torch.logsumexp(s, -1) / math.log(2.0)).abs().max().item() < 2.0 ** -9 / math.log(2.0) + 1e-4
+    del keep
