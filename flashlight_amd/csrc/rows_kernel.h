@@ -420,9 +420,16 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
       ml[j] = *reinterpret_cast<const f32x2*>(p.part_ml + s * 2);
       part[j] = *reinterpret_cast<const f32x4*>(p.part + s * D + c);
     }
+    // (past the last chunk: no key and zeros, not the last chunk times a weight of 0, which is NaN where a value was infinite)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (base + j * NG < p.chunks) continue;
+      ml[j] = f32x2{-INFINITY, 0.f};
+      part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     float M_new = M;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) M_new = base + j * NG < p.chunks ? __builtin_fmaxf(M_new, ml[j][0]) : M_new;
+    for (int j = 0; j < 4; ++j) M_new = __builtin_fmaxf(M_new, ml[j][0]);
     const float ref = M_new == -INFINITY ? 0.f : M_new;
     const float keep = fast_exp2(M - ref);  // (0 before the first chunk with a key)
     M = M_new;
@@ -430,7 +437,7 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
     o *= keep;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float a = base + j * NG < p.chunks ? fast_exp2(ml[j][0] - ref) : 0.f;
+      const float a = fast_exp2(ml[j][0] - ref);
       L += a * ml[j][1];
       o += a * part[j];
     }

@@ -184,3 +184,22 @@ def test_chunks_of_the_keys_replay_from_a_graph(shape):
     G = Hq // Hkv
     kf, vf = (t.float().cpu().repeat_interleave(G, 1) for t in (k, v))
     assert_parity(eager, torch.softmax(q.float().cpu() @ kf.transpose(-1, -2) / math.sqrt(D), -1) @ vf, str(shape))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 8, 8, 1, 1024, 128), (1, 32, 8, 1, 2048, 128), (1, 2, 2, 1, 4096, 64), (1, 8, 8, 48, 4096, 128),
+                                   (1, 32, 8, 1, 32768, 128)])
+def test_infinite_values_stay_in_their_columns(shape):
+    """An infinite value anywhere in the cache makes its column infinite and nothing else, whichever chunk of the keys holds it and
+    however many chunks the merge has."""
+    B, Hq, Hkv, Lq, Lk, D = shape
+    g = torch.Generator().manual_seed(sum(shape))
+    q, k, v = (torch.randn(B, h, n, D, generator=g).to(torch.bfloat16) for h, n in ((Hq, Lq), (Hkv, Lk), (Hkv, Lk)))
+    assert _taken(*shape)[0] and _taken(*shape)[1] > 0   # cut into chunks
+    w = torch.softmax(q.float() @ k.float().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2) / math.sqrt(D), -1)
+    assert w.min() > 1e-30                               # (no weight is zero in any of the types it goes through)
+    v[:, :, 0, 0], v[:, :, Lk // 2 + 5, 1], v[:, :, Lk - 1, 2], v[:, :, Lk - 1, D - 1] = (math.inf, -math.inf, math.inf, -math.inf)
+    want = w @ v.float().repeat_interleave(Hq // Hkv, 1)
+    out = ops.dispatch(q.cuda(), k.cuda(), v.cuda()).float().cpu()
+    assert torch.equal(out.isinf(), want.isinf()) and torch.equal(out[want.isinf()], want[want.isinf()])
+    assert_parity(out.masked_fill(out.isinf(), 0).to(torch.bfloat16), want.masked_fill(want.isinf(), 0), str(shape))
