@@ -793,6 +793,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         dma_wait<0>();
       }
     }
+    dma_wait<0>();  // (a workgroup that found nothing to do has asked for its owner rows all the same)
   } else {
     // positional masks: every step of [t_lo, t_hi] is visited (a dead one only occurs under a prefix-LM mask)
     if constexpr (T::UNROLL2) {

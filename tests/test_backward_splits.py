@@ -124,3 +124,24 @@ def test_both_roles_in_one_launch_beyond_a_round(mask, D):
 
     for whole, a, b in zip(gradients(slice(None)), gradients(slice(0, 16)), gradients(slice(16, 33))):
         assert torch.equal(whole, torch.cat([a, b]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("run", [1, 3, 64])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 2000, 64), (1, 2, 1, 2000, 128), (1, 1, 1, 3000, 128)])
+def test_splits_that_find_no_live_tile(shape, run):
+    """Documents so short that a tile of keys has fewer live tiles of queries than it has splits (four and more)."""
+    B, Hq, Hkv, S, D = shape
+    assert _split_bytes(B, Hq, Hkv, S, S, D, _ffi.MASK_DOCUMENT_CAUSAL) >= 4 * Hkv * -(-S // 128) * 128 * D * 2 * 4
+    g = torch.Generator().manual_seed(S + run)
+    q, k, v, dout = (torch.randn(B, h, S, D, generator=g).to(torch.bfloat16).to(DEV) for h in (Hq, Hkv, Hkv, Hq))
+    kw = dict(mask_kind=_ffi.MASK_DOCUMENT_CAUSAL, doc_ids=(torch.arange(S) // run * 5 - 9)[None].to(DEV))
+    lse = torch.empty(B, Hq, S, dtype=torch.float32, device=DEV)
+    out = _ffi.attn_fwd(q, k, v, lse=lse, **kw)
+    cut = _ffi.attn_bwd(q, k, v, out, lse, dout, split=True, **kw)
+    for a, b in zip(cut, _ffi.attn_bwd(q, k, v, out, lse, dout, **kw)):
+        # the same 16-bit weights and score gradients, added up in another order: as above
+        assert torch.isfinite(a).all() and ((a.double() - b.double()).abs() <= 2.0 ** -7 * b.double().abs() + 2e-5 * v.abs().max()).all()
+    if run == 1:  # one key per query: the weights are 1
+        want = dout.double().view(B, Hkv, Hq // Hkv, S, D).sum(2)
+        assert ((cut[2].double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -9 * dout.abs().max()).all()
