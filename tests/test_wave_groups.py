@@ -131,3 +131,75 @@ def test_64_row_workgroups_against_fp64(mask, kw, S):
     ref, mean_abs = torch.matmul(w, v[7].double()), torch.matmul(w, v[7].double().abs())
     # weights rounded to u = 2^-8 of their size, numerator and row sum alike, and the result once more
     assert ((out - ref).abs() <= 2.0 ** -8 * (mean_abs + 2 * ref.abs()) + 1e-5).all()
+
+
+ATTENDED = [  # mask, options, (batch, heads, length, head dim), (rows per workgroup, groups of waves)
+    (CAUSAL, {}, (2, 8, 2048, 64), (64, 2)), (CAUSAL, {}, (1, 8, 2047, 64), (64, 4)), (CAUSAL, {}, (1, 16, 3000, 128), (128, 2)),
+    (CAUSAL, {}, (2, 18, 385, 64), (64, 2)), (CAUSAL, {}, (1, 8, 1025, 128), (64, 2)),
+    (PREFIX, dict(prefix=333), (2, 8, 1100, 64), (64, 2)), (PREFIX, dict(prefix=1000), (1, 8, 1500, 64), (64, 4)),
+    (PREFIX, dict(prefix=70), (1, 8, 900, 128), (64, 2)),
+    (SLIDING, dict(window=300), (1, 8, 4000, 128), (128, 2)), (SLIDING, dict(window=1000), (1, 4, 2500, 128), (64, 2)),
+    (SLIDING, dict(window=1300), (1, 4, 2500, 64), (64, 4)),
+    (NONE, {}, (1, 8, 2100, 128), (128, 2)), (NONE, {}, (1, 4, 3001, 64), (64, 4)), (NONE, {}, (1, 8, 4096, 64), (128, 2)),
+    (DOC, {}, (2, 16, 1000, 64), (128, 2)), (DOC, {}, (1, 16, 1500, 128), (128, 2)), (DOC_CAUSAL, {}, (1, 16, 5000, 64), (128, 2)),
+    (DOC_CAUSAL, {}, (2, 8, 777, 128), (128, 2)),
+]
+
+
+def _attended(mask, kw, S, g):
+    """Which key each row attends, and the options of the call."""
+    i = torch.arange(S, device=DEV)
+    d = i[:, None] - i[None, :]
+    live = torch.ones(S, S, dtype=torch.bool, device=DEV) if mask in (NONE, DOC) else d >= 0
+    call = dict(kw, mask_kind=mask)
+    if mask == SLIDING:
+        live &= d <= kw["window"]
+    if mask == PREFIX:
+        live |= (i < kw["prefix"])[None, :]
+    if mask in (DOC, DOC_CAUSAL):
+        ids = torch.randint(0, 6, (S,), generator=g).sort().values.to(DEV)
+        ids[S // 3] = 5  # (a document that comes back)
+        live &= ids[:, None] == ids[None, :]
+        call["doc_ids"] = ids[None]
+    return live, call
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,kw,shape,plan", ATTENDED)
+def test_which_keys_the_groups_attend(mask, kw, shape, plan):
+    """Read off the results, as the dump of attended pairs runs without groups: equal logits, and values that are the unit vectors,
+    a block of D keys per (batch, head).  Row q then holds 1 / n at each of the n keys it attends, and 0 at every other."""
+    B, H, S, D = shape
+    assert _shape(B, H, S, D, mask, **kw) == plan
+    g = torch.Generator().manual_seed(S)
+    live, call = _attended(mask, kw, S, g)
+    q = torch.zeros(B, H, S, D, dtype=torch.bfloat16, device=DEV)
+    k = torch.randn(B, H, S, D, generator=g).to(torch.bfloat16).to(DEV)
+    found = torch.empty(S, -(-S // D) * D, device=DEV)
+    for first in range(0, -(-S // D), B * H):
+        v = torch.zeros(B * H, S, D, dtype=torch.bfloat16, device=DEV)
+        for bh in range(B * H):
+            at = (first + bh) * D
+            n = max(0, min(D, S - at))
+            v[bh, at:at + n] = torch.eye(D, dtype=torch.bfloat16, device=DEV)[:n]
+        out = _ffi.attn_fwd(q, k, v.view(B, H, S, D), **call).float().view(B * H, S, D)
+        for bh in range(min(B * H, -(-S // D) - first)):
+            found[:, (first + bh) * D:(first + bh + 1) * D] = out[bh]
+    want = live / live.sum(1, keepdim=True)
+    assert torch.equal(found[:, :S] != 0, live)
+    # equal logits: every weight is 1 and the sums are exact, or off together; one rounding of the result
+    assert ((found[:, :S] - want).abs() <= 2.0 ** -8 * want).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mask,kw,shape,plan", [c for c in ATTENDED if c[2][2] <= 2100])
+def test_groups_against_fp64(mask, kw, shape, plan):
+    B, H, S, D = shape
+    g = torch.Generator().manual_seed(S + 1)
+    q, k, v = (torch.randn(B, H, S, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3))
+    live, call = _attended(mask, kw, S, g)
+    out = _ffi.attn_fwd(q, k, v, **call)[-1].double()
+    w = torch.softmax((torch.matmul(q[-1].double(), k[-1].double().transpose(1, 2).contiguous()) / D ** 0.5).masked_fill(~live, -torch.inf), -1)
+    ref, mean_abs = torch.matmul(w, v[-1].double()), torch.matmul(w, v[-1].double().abs())
+    # weights rounded to u = 2^-8 of their size, numerator and row sum alike, and the result once more
+    assert ((out - ref).abs() <= 2.0 ** -8 * (mean_abs + 2 * ref.abs()) + 1e-5).all()
