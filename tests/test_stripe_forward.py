@@ -127,6 +127,6 @@ def test_a_batch_that_the_divisor_does_not_divide(B, div, S):
     ref = torch.softmax(s, -1) @ v.double()
     # weights and results rounded to bf16, as above
     assert ((out.cpu().double() - ref).norm() / ref.norm()).item() < 3e-3
-    # every rounded weight is off by at most 2^-9 of its size, and so is their sum: 2^-9 / ln 2 in log2 units (1e-4: the exponential)
-    assert (lse.cpu().double() - torch.logsumexp(s, -1) / math.log(2.0)).abs().max().item() < 2.0 ** -9 / math.log(2.0) + 1e-4
+    # every rounded weight is off by at most 2^-8 of its size, and so is their sum: 2^-8 / ln 2 in log2 units (1e-4: the exponential)
+    assert (lse.cpu().double() - torch.logsumexp(s, -1) / math.log(2.0)).abs().max().item() < 2.0 ** -8 / math.log(2.0) + 1e-4
     del keep
