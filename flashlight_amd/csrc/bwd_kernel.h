@@ -18,7 +18,7 @@
 // P, dS never leave registers.  T1/T2 are staged in LDS by global_load_lds transfers, two slots, one barrier per tile;
 // T^T operands come from the same tiles through the transposing LDS read.
 #pragma once
-#include "fwd_kernel.h"
+#include "tile_operands.h"
 
 namespace fl {
 
@@ -184,6 +184,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   constexpr bool kDrop = FEAT & F_DROPOUT;
   constexpr float kLog2e = 1.4426950408889634f;
   using L = TileLayout<D>;
+  using Ops = TileOperands<D, E>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x;
@@ -365,31 +366,19 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // lane's row of an owner tile (B operand)
   auto frag_row = [&](unsigned tile_off, int sb, int ks) FL_INLINE -> ex8 {
     if constexpr (T::TUNED) return *(lds_ex8_ptr)(a_row[ks] + tile_off + sb * 32 * RB);
-    const int row = (qh * TB + sb) * 32 + r;
-    return *reinterpret_cast<const ex8*>(smem + tile_off + row * RB + L::swz_kv(row, 2 * ks + h) * 16);
+    return Ops::rows(smem + tile_off, (qh * TB + sb) * 32 + r, ks, h);
   };
   auto frag_own = [&](unsigned tile_off, int ks) FL_INLINE -> ex8 {
     if constexpr (T::TUNED) return *(lds_ex8_ptr)(a_own[ks] + (tile_off - T::O1_OFF));
-    const int row = ow * 32 + r;
-    return *reinterpret_cast<const ex8*>(smem + tile_off + row * RB + L::swz_kv(row, 2 * ks + h) * 16);
+    return Ops::rows(smem + tile_off, ow * 32 + r, ks, h);
   };
-  // transposing: A operand of the accumulating products for 16-position chunk c (of this wave's) and column block db; slot j of lane
-  // (r, h) is streamed position 16 c + 8 (j / 4) + 4 h + j % 4, the order in which the weights are packed
+  // transposing: A operand of the accumulating products for 16-position chunk c (of this wave's) and column block db
   auto frag_tr = [&](unsigned tile_off, int c, int db) FL_INLINE -> ex8 {
+    if constexpr (!T::TUNED) return Ops::columns(smem + tile_off, 2 * TB * qh + c, db, lane, h);
     ex8 f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      s16x4 t4;
-      if constexpr (T::TUNED) {
-        t4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j][db] + tile_off + c * 16 * RB));
-      } else {
-        const int i16 = lane % 16, g = (lane / 16) % 2;
-        const int row = 16 * (2 * TB * qh + c) + 8 * j + 4 * h + i16 / 4;
-        const int col = db * 32 + g * 16 + 4 * (i16 % 4);
-        const unsigned char* ap = smem + tile_off + row * RB + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
-        t4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ap));
-      }
-      const ex4 b4 = __builtin_bit_cast(ex4, t4);
+      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j][db] + tile_off + c * 16 * RB)));
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
     }

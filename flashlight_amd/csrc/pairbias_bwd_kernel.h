@@ -25,7 +25,7 @@
 // over the waves) with two waves per SIMD to cover it.  Two blocks per wave in four waves beat one in eight (67 and 93 us for the two
 // roles against 46 and 56: the sums over the waves cost more than the occupancy gains).
 #pragma once
-#include "fwd_kernel.h"
+#include "tile_operands.h"
 
 namespace fl {
 
@@ -84,22 +84,15 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
   using E = typename T::Elem;
   typedef E ex8 __attribute__((ext_vector_type(8)));
   typedef E ex4 __attribute__((ext_vector_type(4)));
-  using L = TileLayout<D>;
+  using Ops = TileOperands<D, E>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r = lane % 32, h = lane / 32;
 
-  // ---- workgroup -> (group, chunk of batch entries, head, stripe): the stripes of one (chunk, head) read the same
-  // tensors and stay on one XCD
-  int tile, uc;
-  {
-    const int x = block % 8, i = block / 8;
-    tile = i % p.tiles;
-    uc = i / p.tiles * 8 + x;
-    if (uc >= p.groups * p.chunks * p.H) return;  // (before any barrier)
-  }
-  const int head = uc % p.H, gc = uc / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
+  const StripePlace place(p, block);
+  if (place.none(p)) return;  // (before any barrier)
+  const int tile = place.tile, head = place.unit % p.H, gc = place.unit / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
   const int n0 = group * p.div + chunk * p.chunk_len, n1 = min(group * p.div + p.div, n0 + p.chunk_len);
   const int o0 = tile * 32, S = p.S;
   const int own = o0 + r;                 // this lane's query (ROLE_DQ) or key
@@ -156,12 +149,6 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
   // scalar base addresses advance by one batch stride: per entry a transfer costs its issue and nothing else.
   const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem);
   constexpr unsigned w_bytes = T::W_BYTES * NW, slot_bytes = T::SLOT_BYTES;
-  constexpr int RPT = 512 / D;  // rows per 1 KiB transfer
-  // byte offset of this lane's 16 bytes of transfer `it` of rows row0 .., rows past the end repeating the last one
-  auto lane_offset = [&](int row0, int it, int64_t stride) FL_INLINE -> unsigned {
-    const int row = it * RPT + lane / L::CPR;
-    return (uint32_t)min(row0 + row, S - 1) * ((uint32_t)stride * 2u) + (uint32_t)(L::swz_kv(row, lane % L::CPR) * 16);
-  };
   struct Operand {
     uint64_t at;   // address of the next entry's [S][D] rows of this head
     uint64_t step;
@@ -174,8 +161,8 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
   unsigned off1[T::TPW], off2[T::TPW];
 #pragma unroll
   for (int it = 0; it < T::TPW; ++it) {
-    off1[it] = lane_offset(w0, it, kDQ ? p.ks[2] : p.qs[2]);
-    off2[it] = lane_offset(w0, it, kDQ ? p.vs[2] : p.dos[2]);
+    off1[it] = Ops::transfer_offset(w0, S, it, kDQ ? p.ks[2] : p.qs[2], lane);
+    off2[it] = Ops::transfer_offset(w0, S, it, kDQ ? p.vs[2] : p.dos[2], lane);
   }
   // the owned rows: 2 OT transfers shared out over the waves (one wave takes several where there are fewer waves)
   constexpr int OT = T::O_BYTES / 1024, OPW = (2 * OT + NW - 1) / NW;
@@ -183,7 +170,7 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
 #pragma unroll
   for (int j = 0; j < OPW; ++j) {
     const int x = j * NW + wave;
-    ooff[j] = x < OT ? lane_offset(o0, x, kDQ ? p.qs[2] : p.ks[2]) : lane_offset(o0, x - OT, kDQ ? p.dos[2] : p.vs[2]);
+    ooff[j] = x < OT ? Ops::transfer_offset(o0, S, x, kDQ ? p.qs[2] : p.ks[2], lane) : Ops::transfer_offset(o0, S, x - OT, kDQ ? p.dos[2] : p.vs[2], lane);
   }
   // per-row fp32 values: LSE and Delta rows of this head, the bias row of the entry
   uint64_t lse_at = uniform_ptr(p.lse + ((int64_t)n0 * p.H + head) * S), del_at = uniform_ptr(p.delta + ((int64_t)n0 * p.H + head) * S);
@@ -225,28 +212,7 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
     if constexpr (kRowB) row_at += row_step;
   };
 
-  // ---- LDS operand reads, as in bwd_kernel.h
-  auto frag_row = [&](const unsigned char* t, int row, int ks) FL_INLINE -> ex8 {
-    return *reinterpret_cast<const ex8*>(t + row * (D * 2) + L::swz_kv(row, 2 * ks + h) * 16);
-  };
-  auto frag_tr = [&](const unsigned char* t, int c, int dbk) FL_INLINE -> ex8 {
-    ex8 f;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int i16 = lane % 16, g = (lane / 16) % 2;
-      const int row = 16 * c + 8 * j + 4 * h + i16 / 4, col = dbk * 32 + g * 16 + 4 * (i16 % 4);
-      const unsigned char* ap = t + row * (D * 2) + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
-      typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
-      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ap)));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
-    }
-    return f;
-  };
-  // partial sums of one set: [owned row][D] floats, 16-byte chunks XOR-swizzled with the row
-  constexpr int PC = D / 4;
-  auto park_at = [&](int row, int c) FL_INLINE { return row * (D * 4) + ((c ^ row) & (PC - 1)) * 16; };
-
+  constexpr int PC = D / 4;  // 16-byte chunks per row of partial sums
   // where this entry's sums go; pieces of 64 lanes with 4 columns each, which the waves take in turn
   const int rows = min(32, S - o0);
   uint64_t out1 = uniform_ptr((kDQ ? p.dq : p.dk) + (int64_t)n0 * (kDQ ? p.dqs[0] : p.dks[0]) + (int64_t)head * (kDQ ? p.dqs[1] : p.dks[1]));
@@ -270,8 +236,8 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
     ex8 o1[KS], o2[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      o1[ks] = frag_row(own_at, r, ks);
-      o2[ks] = frag_row(own_at + T::O_BYTES, r, ks);
+      o1[ks] = Ops::rows(own_at, r, ks, h);
+      o2[ks] = Ops::rows(own_at + T::O_BYTES, r, ks, h);
     }
     const float* own_f = reinterpret_cast<const float*>(own_at + 2 * T::O_BYTES);
     const float* st_f = reinterpret_cast<const float*>(mine + 2 * T::T_BYTES);
@@ -316,8 +282,8 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
       }
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        x1 = mfma32(frag_row(mine, 32 * b + r, ks), o1[ks], x1);
-        x2 = mfma32(frag_row(mine + T::T_BYTES, 32 * b + r, ks), o2[ks], x2);
+        x1 = mfma32(Ops::rows(mine, 32 * b + r, ks, h), o1[ks], x1);
+        x2 = mfma32(Ops::rows(mine + T::T_BYTES, 32 * b + r, ks, h), o2[ks], x2);
       }
       ex8 pf[2], dsf[2];
 #pragma unroll
@@ -341,8 +307,8 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int d = 0; d < DB; ++d) {
-          acc1[d] = mfma32(frag_tr(mine, 2 * b + c, d), dsf[c], acc1[d]);
-          if constexpr (!kDQ) acc2[d] = mfma32(frag_tr(mine + T::T_BYTES, 2 * b + c, d), pf[c], acc2[d]);
+          acc1[d] = mfma32(Ops::columns(mine, 2 * b + c, d, lane, h), dsf[c], acc1[d]);
+          if constexpr (!kDQ) acc2[d] = mfma32(Ops::columns(mine + T::T_BYTES, 2 * b + c, d, lane, h), pf[c], acc2[d]);
         }
     }
 
@@ -352,7 +318,7 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
       for (int d = 0; d < DB; ++d)
 #pragma unroll
         for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<f32x4*>(at + park_at(r, 8 * d + 2 * g + h)) = f32x4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
+          *reinterpret_cast<f32x4*>(at + Ops::park_at(r, 8 * d + 2 * g + h)) = f32x4{acc[d][4 * g], acc[d][4 * g + 1], acc[d][4 * g + 2], acc[d][4 * g + 3]};
     };
     auto gather = [&](unsigned offset, uint64_t out, int64_t row_stride, float scale) FL_INLINE {
 #pragma unroll
@@ -361,7 +327,7 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
         if (piece >= pieces) break;
         // (rows past the end repeat the last one: every wave's stores are counted)
         const int row = min(piece * RPP + lane / PC, rows - 1), c = lane % PC;
-        const unsigned char* at = s0 + offset + park_at(row, c);
+        const unsigned char* at = s0 + offset + Ops::park_at(row, c);
         f32x4 sum = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int w = 0; w < NW; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * T::W_BYTES);

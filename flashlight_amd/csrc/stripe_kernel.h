@@ -21,7 +21,7 @@
 // bf16, general kernel -> here: 128 x 8 x 256 x 256, head dim 32, gate, row and statistics: 48 -> 39 us; 2 x 207 x 4 x 494 x 494, head
 // dim 32: 806 -> 201; 2 x 17 x 4 x 235 x 235, head dim 64, gate and row: 43 -> 17; 28 x 4 x 106 x 106, head dim 32, gate: 14 -> 6.
 #pragma once
-#include "fwd_kernel.h"
+#include "tile_operands.h"
 
 namespace fl {
 
@@ -86,24 +86,17 @@ void stripe_kernel(const StripeParams p) {
   constexpr float kLog2e = 1.4426950408889634f;
   using E = typename T::Elem;
   typedef E ex8 __attribute__((ext_vector_type(8)));
-  typedef E ex4 __attribute__((ext_vector_type(4)));
   typedef E ex2 __attribute__((ext_vector_type(2)));
   using L = TileLayout<D>;
+  using Ops = TileOperands<D, E>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r = lane % 32, h = lane / 32;
 
-  // ---- workgroup -> (group, chunk of batch entries, head, stripe): the stripes of one (chunk, head) read the same K and V and
-  // stay on one XCD
-  int tile, uc;
-  {
-    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
-    tile = i % p.tiles;
-    uc = i / p.tiles * 8 + x;
-    if (uc >= p.groups * p.chunks * p.H) return;  // (before any barrier)
-  }
-  const int head = uc % p.H, gc = uc / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
+  const StripePlace place(p, blockIdx.x);
+  if (place.none(p)) return;  // (before any barrier)
+  const int tile = place.tile, head = place.unit % p.H, gc = place.unit / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
   const int n0 = group * p.div + chunk * p.chunk_len, n1 = min(group * p.div + p.div, n0 + p.chunk_len);
   const int o0 = tile * QB * 32, Lk = p.Lk;
   const int rows = min(QB * 32, p.Lq - o0);  // of this stripe
@@ -112,17 +105,11 @@ void stripe_kernel(const StripeParams p) {
   // ---- addresses.  Per-lane offsets do not change from entry to entry; the scalar bases advance by one batch stride.
   const unsigned lds0 = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem);
   constexpr unsigned w_bytes = T::W_BYTES * NW, slot_bytes = T::SLOT_BYTES;
-  constexpr int RPT = 512 / D;  // rows per 1 KiB transfer
-  // byte offset of this lane's 16 bytes of transfer `it` of rows row0 .., rows past the end repeating the last one
-  auto lane_offset = [&](int row0, int len, int it, int64_t stride) FL_INLINE -> unsigned {
-    const int row = it * RPT + lane / L::CPR;
-    return (uint32_t)min(row0 + row, len - 1) * ((uint32_t)stride * 2u) + (uint32_t)(L::swz_kv(row, lane % L::CPR) * 16);
-  };
   unsigned koff[T::TPW], voff[T::TPW];
 #pragma unroll
   for (int it = 0; it < T::TPW; ++it) {
-    koff[it] = lane_offset(w0, Lk, it, p.ks[2]);
-    voff[it] = lane_offset(w0, Lk, it, p.vs[2]);
+    koff[it] = Ops::transfer_offset(w0, Lk, it, p.ks[2], lane);
+    voff[it] = Ops::transfer_offset(w0, Lk, it, p.vs[2], lane);
   }
   uint64_t ka = uniform_ptr(p.k + (int64_t)n0 * p.ks[0] + (int64_t)head * p.ks[1]);  // of the entry to be fetched next
   uint64_t va = uniform_ptr(p.v + (int64_t)n0 * p.vs[0] + (int64_t)head * p.vs[1]);
@@ -138,7 +125,7 @@ void stripe_kernel(const StripeParams p) {
   constexpr int QPW = (T::QT + NW - 1) / NW;  // of the stripe's queries, shared out over the waves
   unsigned qoff[QPW];
 #pragma unroll
-  for (int j = 0; j < QPW; ++j) qoff[j] = lane_offset(o0, p.Lq, j * NW + wave, p.qs[2]);
+  for (int j = 0; j < QPW; ++j) qoff[j] = Ops::transfer_offset(o0, p.Lq, j * NW + wave, p.qs[2], lane);
   auto load_entry = [&](int slot) FL_INLINE {
     const unsigned q_at = lds0 + slot * slot_bytes + w_bytes;
 #pragma unroll
@@ -211,28 +198,6 @@ void stripe_kernel(const StripeParams p) {
     else fetch(static_cast<const E*>(p.bias));
   }
 
-  // ---- LDS operand reads, as in bwd_kernel.h
-  auto frag_row = [&](const unsigned char* t, int row, int ks) FL_INLINE -> ex8 {
-    return *reinterpret_cast<const ex8*>(t + row * (D * 2) + L::swz_kv(row, 2 * ks + h) * 16);
-  };
-  auto frag_tr = [&](const unsigned char* t, int c, int dbk) FL_INLINE -> ex8 {
-    ex8 f;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int i16 = lane % 16, g = (lane / 16) % 2;
-      const int row = 16 * c + 8 * j + 4 * h + i16 / 4, col = dbk * 32 + g * 16 + 4 * (i16 % 4);
-      const unsigned char* ap = t + row * (D * 2) + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
-      typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
-      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(ap)));
-#pragma unroll
-      for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
-    }
-    return f;
-  };
-  // partial results of one wave: [row of the stripe][D] floats, 16-byte chunks XOR-swizzled with the row
-  constexpr int PC = D / 4;
-  auto park_at = [&](int row, int c) FL_INLINE { return row * (D * 4) + ((c ^ row) & (PC - 1)) * 16; };
-
   uint64_t oa = uniform_ptr(p.o + (int64_t)n0 * p.os[0] + (int64_t)head * p.os[1]);
   uint64_t ua = uniform_ptr(p.ungated + (int64_t)n0 * p.os[0] + (int64_t)head * p.os[1]);
   uint64_t la = uniform_ptr(p.lse + ((int64_t)n0 * p.H + head) * p.Lq);
@@ -267,7 +232,7 @@ void stripe_kernel(const StripeParams p) {
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = frag_row(s0 + w_bytes, 32 * qb + r, ks);
+      for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = Ops::rows(s0 + w_bytes, 32 * qb + r, ks, h);
 
     f32x16 acc[QB][DB];
     float l[QB];
@@ -284,7 +249,7 @@ void stripe_kernel(const StripeParams p) {
       for (int qb = 0; qb < QB; ++qb) x[qb] = init;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const ex8 kf = frag_row(mine, 32 * b + r, ks);
+        const ex8 kf = Ops::rows(mine, 32 * b + r, ks, h);
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) x[qb] = mfma32(kf, qf[qb][ks], x[qb]);
       }
@@ -310,7 +275,7 @@ void stripe_kernel(const StripeParams p) {
       for (int c = 0; c < 2; ++c)
 #pragma unroll
         for (int d = 0; d < DB; ++d) {
-          const ex8 vf = frag_tr(mine + T::T_BYTES, 2 * b + c, d);
+          const ex8 vf = Ops::columns(mine + T::T_BYTES, 2 * b + c, d, lane, h);
 #pragma unroll
           for (int qb = 0; qb < QB; ++qb) acc[qb][d] = mfma32(vf, pf[qb][c], acc[qb][d]);
         }
@@ -380,7 +345,7 @@ void stripe_kernel(const StripeParams p) {
         for (int d = 0; d < DB; ++d)
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<f32x4*>(mine + park_at(32 * qb + r, 8 * d + 2 * g + h)) =
+            *reinterpret_cast<f32x4*>(mine + Ops::park_at(32 * qb + r, 8 * d + 2 * g + h)) =
                 f32x4{acc[qb][d][4 * g], acc[qb][d][4 * g + 1], acc[qb][d][4 * g + 2], acc[qb][d][4 * g + 3]};
         l[qb] = xhalf_sum(l[qb]);
         if (h == 0) sums[(wave * QB + qb) * 32 + r] = l[qb];
@@ -427,8 +392,8 @@ void stripe_kernel(const StripeParams p) {
       }
       t = __shfl(t, row % 32);
       f32x4 a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
-      const unsigned char* at0 = s0 + park_at(row, 2 * pcol);
-      const unsigned char* at1 = s0 + park_at(row, 2 * pcol + 1);
+      const unsigned char* at0 = s0 + Ops::park_at(row, 2 * pcol);
+      const unsigned char* at1 = s0 + Ops::park_at(row, 2 * pcol + 1);
       auto add = [&](int w) FL_INLINE {
         a += *reinterpret_cast<const f32x4*>(at0 + w * T::W_BYTES);
         b += *reinterpret_cast<const f32x4*>(at1 + w * T::W_BYTES);
