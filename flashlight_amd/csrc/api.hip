@@ -299,7 +299,10 @@ FewPlan plan_few(const fl_attn_params* p, uint32_t want) {
   const int64_t walk = p->mask_kind == FL_MASK_SLIDING ? std::min<int64_t>(p->Lk, (int64_t)p->window + 128) : p->Lk;
   const bool narrow = p->Dqk == 64;
   if (walk < ((want & fl::F_DOC) ? 192 : p->mask_kind == FL_MASK_NONE ? (narrow ? 640 : 1024) : narrow ? 384 : 256)) return x;
-  if (heads == 1) return x;  // (one head by itself is what slices of large calls are compared with: it keeps their order of sums)
+  // One head by itself keeps the order of sums it has inside a large call: slices of operands beyond 2^31 elements are compared with it bit
+  // by bit.  That costs such a call (us, as is / by the lines below): unmasked, 8192 rows, head dim 128, 131 / 102; 16384 rows, 257 / 199,
+  // head dim 64, 194 / 95; up to 8192 rows at head dim 64 the few-rows kernel has them.
+  if (heads == 1) return x;
   if (p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM) {
     if (narrow ? tiles > 256 && (tiles > 512 || heads > 48) : tiles > 512 || heads > 48) return x;
     x.waves = narrow || tiles <= 256 ? 2 : 4;
@@ -798,7 +801,7 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   const int64_t row_tiles = (rows + 16 * qt - 1) / (16 * qt), base = units * row_tiles;
   // Waves per workgroup and chunks of the keys.  Eight waves fill a compute unit's registers, so 256 workgroups of eight
   // or 512 of four are one round.  Enough row tiles: no chunks, and shorter workgroups the more of them there are.  Few:
-  // a chunk has two key tiles per wave at least, and the merge launch behind the chunks costs 4.5 us, about what reading 512
+  // a chunk has two key tiles per wave at least, and the merge launch behind the chunks costs 4 us, about what reading 512
   // keys in one workgroup costs (1024 where more than two row tiles read them): up to there they stay together.  Eight waves
   // add up inside the workgroup what four would send through memory: worth it once a wave has two tiles.  (8 heads, head dim
   // 128, rows of one workgroup each -> chunks: 128 queries of 2048 keys 23.6 -> 14.8 us, 48 of 3000 keys 31.6 -> 15.3.)

@@ -10,7 +10,7 @@
 // while it works on the current one: eight waves on a compute unit have 128 KiB outstanding.
 // Measured (MI355X, bf16, operands larger than the memory-side cache; before: the tile kernel over key chunks made by the
 // front end): 32 query heads over 8, one row, 32768 keys, head dim 128: 42.2 -> 31.2 us (27.4 for this kernel = 4.9 TB/s,
-// launch included, 4.5 for the merge); 8 sequences of 3001 keys in longer buffers: 51.6 -> 21.9 us; 32 x 2048 keys 5.5 TB/s;
+// launch included, 4.5 for the merge, now 4); 8 sequences of 3001 keys in longer buffers: 51.6 -> 21.9 us; 32 x 2048 keys 5.5 TB/s;
 // causal prefill 2 x 8 heads x 512, head dim 64: 10.9 -> 9.2 us.
 // What such a call spends beside its reads is a chain: with the sums over the waves unrolled (a run-time count was one LDS wait after the
 // other), no division where one head has all rows, and the merge's loads in flight together, 9.20 -> 8.86, decoding 31.2 -> 30.1, 22.1 ->

@@ -17,7 +17,8 @@
 // products, exponentials, sums over the waves, stores: about 600 instructions per wave, 350 of them for its four blocks of
 // 32 x 32) with two waves per SIMD to cover it.  Two blocks of queries per wave share the K and V operands, and halve what is
 // exchanged per score against one (128 x 8 x 256 x 256, head dim 32, gate and row: 61 us with one; head dim 64 has no registers
-// for two).  Wave counts are compiled in: sums over a run-time count wait for one LDS read after the other (55 us against 39).
+// for two).  Head dim 32 is at the limit of the 256 registers that two waves per SIMD leave: with three waves, or two and a bias row, one
+// value goes to scratch and comes back once per batch entry, with one wave and a row nine do; the other shapes fit.  Wave counts are compiled in: sums over a run-time count wait for one LDS read after the other (55 us against 39).
 // bf16, general kernel -> here: 128 x 8 x 256 x 256, head dim 32, gate, row and statistics: 48 -> 39 us; 2 x 207 x 4 x 494 x 494, head
 // dim 32: 806 -> 201; 2 x 17 x 4 x 235 x 235, head dim 64, gate and row: 43 -> 17; 28 x 4 x 106 x 106, head dim 32, gate: 14 -> 6.
 #pragma once

@@ -291,7 +291,7 @@ uint64_t fl_static_scratch_bytes(void);
  * with a batch stride of 0, where the caller adds up the B / bias_batch_div gradients (or says bias_batch_div = B).
  * dgate (with fwd.gate): gradient of the gate's logits, addressed with dgate_strides.
  * workspace: fl_attn_shared_bias_bwd_bytes() bytes, 256-byte aligned, contents undefined.
- * Four launches (row sums and gate; dQ and the bias's partial sums; dK and dV; the sum), no atomics. */
+ * Three launches (row sums and gate; dQ, the bias's partial sums, dK and dV; the sum), no atomics. */
 typedef struct fl_attn_shared_bias_bwd_params {
   fl_attn_params fwd;
   const void* dout;
