@@ -1136,7 +1136,10 @@ void fwd_kernel(const KParams p) {
           // (a row that is fully masked so far takes the floor as its reference too: whatever comes next is above it).
           // Only bias operands bring such numbers: the other kernels keep the plain maximum.
           float m_new = __builtin_fmaxf(floor_, mx[qb]);
-          if constexpr (kBias) m_new = __builtin_fmaxf(m_new, ref_floor);
+          // Kernels whose scores are formed relative to the reference (kFoldRef) take none from a tile that holds nothing but such masks, or
+          // nothing attended: relative to -2^15 the scores of the row's first real tile would be rounded to 2^-8 (the row statistic of
+          // a single key was off by 5e-3; fp16 results of windows under a soft-cap by three times their rounding).
+          if constexpr (kBias) m_new = kFoldRef && m_new < 2.0f * ref_floor ? -INFINITY : __builtin_fmaxf(m_new, ref_floor);
           const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // row fully masked so far
           // (the clamp keeps 0 * inf out of accumulators whose contents have underflowed to nothing)
           const float m_old = fresh ? 0.f : m_run[qb];

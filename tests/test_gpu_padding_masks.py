@@ -78,3 +78,31 @@ def test_additive_padding_mask(seed):
         assert torch.isfinite(out).all(), c
     d = ((out - ref).abs() * rows).nan_to_num(0.0)
     assert d.max().item() <= 2e-2 * c["amp"] and d.mean().item() <= 2e-3 * c["amp"], (c, d.max().item(), d.mean().item())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("softcap", [0.0, 4.0])
+def test_one_key_behind_masked_tiles(softcap, D, dtype):
+    """Rows that attend a single key, behind tiles of which they attend nothing: by a window of 0, or by a row of -inf, the type's lowest
+    value or -1e9 everywhere else.  The result is that key's value, and the row statistic its score, which no weight rounds: fp32
+    operations on numbers below 16, 2^-20 each, and an exponential and a reciprocal of about as much under the soft-cap."""
+    g = torch.Generator().manual_seed(D)
+    B, H, S = 2, 3, 300
+    q, k, v = (torch.randn(B, H, S, D, generator=g).to(dtype) for _ in range(3))
+    bias = torch.randn(1, H, S, S, generator=g)
+    s = q.double() @ k.double().transpose(-1, -2) / math.sqrt(D)
+    s = softcap * torch.tanh(s / softcap) if softcap else s
+    dev = [t.to(DEV) for t in (q, k, v)]
+    lse = torch.empty(B, H, S, device=DEV)
+    out = _ffi.attn_fwd(*dev, mask_kind=_ffi.MASK_SLIDING, window=0, softcap=softcap, biases=[(bias.to(DEV), B)], lse=lse)
+    want = (s + bias.double()).diagonal(dim1=-2, dim2=-1) / math.log(2.0)
+    assert torch.equal(out.cpu(), v) and (lse.cpu().double() - want).abs().max().item() < 2e-5
+    for fill in (float("-inf"), torch.finfo(dtype).min, -1e9):
+        for key in (0, 63, 64, 200, 299):
+            row = torch.full((1, 1, 1, S), fill)
+            row[..., key] = 0.5
+            out = _ffi.attn_fwd(*dev, softcap=softcap, biases=[(bias.to(DEV), B), (row.to(DEV), B)], lse=lse)
+            want = (s[..., key] + bias[..., key].double() + 0.5) / math.log(2.0)
+            assert torch.equal(out.cpu(), v[:, :, key:key + 1].expand_as(v)), (fill, key)
+            assert (lse.cpu().double() - want).abs().max().item() < 2e-5, (fill, key)
