@@ -410,26 +410,28 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
   float M = -INFINITY, L = 0.f;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
   // four chunks at a time, pairs and results asked for together (the pairs first and then the results, one after the other, was five
-  // trips to memory for 32 chunks: 4.5 us of a decoding step's 31)
+  // trips to memory for 32 chunks: 4.5 us of a decoding step's 31).  The buffers end with the row's last chunk: what lies past it reads as
+  // zeros (the last chunk once more, with a weight of 0, is NaN where a value was infinite).  As selects behind the loads that was 0.1 us,
+  // as branches around them 0.2; fetching instructions counts in a kernel of 4 us.  (at most 512 chunks of 32 rows: 8 MiB)
+  constexpr int kRaw = 0x00027000;  // untyped, range-checked by the byte
+  const int last = (p.chunks - 1) * RB;
+  const __amdgpu_buffer_rsrc_t parts = __builtin_amdgcn_make_buffer_rsrc(p.part + slot0 * D, 0, (last + 1) * D * 4, kRaw);
+  const __amdgpu_buffer_rsrc_t pairs = __builtin_amdgcn_make_buffer_rsrc(p.part_ml + slot0 * 2, 0, (last + 1) * 8, kRaw);
   for (int base = grp; base < p.chunks; base += 4 * NG) {
     f32x2 ml[4];
     f32x4 part[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int64_t s = slot0 + (int64_t)min(base + j * NG, p.chunks - 1) * RB;
-      ml[j] = *reinterpret_cast<const f32x2*>(p.part_ml + s * 2);
-      part[j] = *reinterpret_cast<const f32x4*>(p.part + s * D + c);
-    }
-    // (past the last chunk: no key and zeros, not the last chunk times a weight of 0, which is NaN where a value was infinite)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (base + j * NG < p.chunks) continue;
-      ml[j] = f32x2{-INFINITY, 0.f};
-      part[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const int s = (base + j * NG) * RB;
+      ml[j] = __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(pairs, s * 8, 0, 0));
+      part[j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(parts, (s * D + c) * 4, 0, 0));
     }
     float M_new = M;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) M_new = __builtin_fmaxf(M_new, ml[j][0]);
+    for (int j = 0; j < 4; ++j) {
+      ml[j][0] = base + j * NG < p.chunks ? ml[j][0] : -INFINITY;
+      M_new = __builtin_fmaxf(M_new, ml[j][0]);
+    }
     const float ref = M_new == -INFINITY ? 0.f : M_new;
     const float keep = fast_exp2(M - ref);  // (0 before the first chunk with a key)
     M = M_new;
