@@ -859,6 +859,11 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   k.row_tiles = (int)row_tiles;
   k.chunks = (int)chunks;
   k.units = (int)units;
+  k.by_rows = fl::Div::by((uint32_t)rows);
+  k.by_row_tiles = fl::Div::by((uint32_t)row_tiles);
+  k.by_chunks = fl::Div::by((uint32_t)chunks);
+  k.by_Hkv = fl::Div::by((uint32_t)p->Hkv);
+  k.by_Lq = fl::Div::by((uint32_t)p->Lq);
   const float l2e = 1.4426950408889634f;
   k.scale_log2 = p->scale * l2e;
   if (p->softcap > 0.f) {

@@ -51,6 +51,26 @@ constexpr int kMaxKeyTiles = 65535;
 constexpr int kOwnListTiles = 64, kOwnListBytes = 2 * 64 * 8 + 2 * 8 * 8;  // (behind the list: (min, max) id of 64 key tiles and 8 waves' rows)
 constexpr int kDocBlock = 32;
 
+// Division of 0 .. 2^31 - 1 by a number that the host knows: a multiplication, an addition and a shift.  A division by a run-time number
+// is some thirty dependent instructions, and a workgroup has several ahead of its first load.
+// 2^32 + mul is 2^(32 + s) / d rounded up, s = ceil(log2 d), which is exact for numerators below 2^31.
+struct Div {
+  uint32_t mul, shift;
+  __host__ static constexpr Div by(uint32_t d) {
+    uint32_t s = 0;
+    while ((uint64_t{1} << s) < d) ++s;
+    return {(uint32_t)((((uint64_t{1} << s) - d) << 32) / d + 1), s};
+  }
+  __host__ __device__ __forceinline__ constexpr uint32_t of(uint32_t n) const { return ((uint32_t)(((uint64_t)n * mul) >> 32) + n) >> shift; }
+};
+constexpr bool div_holds(uint32_t d) {
+  const Div x = Div::by(d);
+  const uint32_t top = 0x7fffffffu, m = top / d * d;  // the largest multiple: the quotient steps there
+  return x.of(0) == 0 && x.of(d - 1) == 0 && x.of(d) == 1 && x.of(top) == top / d && x.of(m) == m / d && x.of(m - 1) == (m - 1) / d;
+}
+static_assert(div_holds(1) && div_holds(2) && div_holds(3) && div_holds(5) && div_holds(7) && div_holds(641) && div_holds(1000) &&
+              div_holds(65535) && div_holds(65537) && div_holds(0x3fffffffu) && div_holds(0x40000001u) && div_holds(0x7fffffffu));
+
 struct KParams {
   const bf16_t* q;
   const bf16_t* k;

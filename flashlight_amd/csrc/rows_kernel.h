@@ -14,7 +14,8 @@
 // causal prefill 2 x 8 heads x 512, head dim 64: 10.9 -> 9.2 us.
 // What such a call spends beside its reads is a chain: with the sums over the waves unrolled (a run-time count was one LDS wait after the
 // other), no division where one head has all rows, and the merge's loads in flight together, 9.20 -> 8.86, decoding 31.2 -> 30.1, 22.1 ->
-// 21.7 and, 2 x 8 heads of 282 rows, 7.8 -> 7.5.
+// 21.7 and, 2 x 8 heads of 282 rows, 7.8 -> 7.5.  With nothing ahead of the first load that goes through LDS (the tile's bounds) and no
+// division at all (Div), 8.87 -> 8.19, decoding 30.0 -> 29.3 and 21.6 -> 20.6.
 //
 // Rows are packed: row x of key / value head n is position x % Lq of query head n * G + x / Lq, so the G query heads that
 // share a key / value head are rows of one tile and the keys are read once for all of them.
@@ -41,6 +42,7 @@ struct RParams {
   int32_t B, Hq, Hkv, Lq, Lk, group;
   int32_t rows;                              // group * Lq: packed rows per key / value head
   int32_t row_tiles, chunks, units;          // units = B * Hkv
+  Div by_rows, by_row_tiles, by_chunks, by_Hkv, by_Lq;
   int32_t by_xcd;                            // row tiles of one (unit, chunk) on one XCD (units * chunks >= 8)
   float scale_log2, cap_k1, cap_c;           // as in fwd_kernel; cap_c = 0: no soft-cap
   int32_t dmin, dmax, pfx;                   // attend iff key < Lk && ((dmin <= key - q <= dmax) || key < pfx)
@@ -67,11 +69,6 @@ __device__ __forceinline__ float groups_max(float x) {
 __device__ __forceinline__ float groups_sum(float x) {
   x += __shfl_xor(x, 16, 64);
   return x + __shfl_xor(x, 32, 64);
-}
-__device__ __forceinline__ int wave_min(int x) {
-#pragma unroll
-  for (int d = 1; d < 64; d *= 2) x = min(x, __shfl_xor(x, d, 64));
-  return x;
 }
 // MOD: 0 plain, F_ALIBI | F_SOFTCAP (either may be off at run time), F_BIAS (row biases, and the soft-cap at run time)
 // QT: 16-row blocks per wave (1 or 2)
@@ -106,46 +103,46 @@ void rows_kernel(const RParams p) {
   // ---- workgroup -> (unit, chunk, row tile); the row tiles of one (unit, chunk) read the same keys
   int rt, uc;
   if (p.by_xcd) {
-    const int x = blockIdx.x % 8, i = blockIdx.x / 8;
-    rt = i % p.row_tiles;
-    uc = i / p.row_tiles * 8 + x;
+    const int x = blockIdx.x % 8, i = blockIdx.x / 8, o = p.by_row_tiles.of(i);
+    rt = i - o * p.row_tiles;
+    uc = o * 8 + x;
     if (uc >= p.units * p.chunks) return;
   } else {
-    rt = blockIdx.x % p.row_tiles;
-    uc = blockIdx.x / p.row_tiles;
+    uc = p.by_row_tiles.of(blockIdx.x);
+    rt = blockIdx.x - uc * p.row_tiles;
   }
   rt = p.row_tiles - 1 - rt;  // under a causal mask the last rows have the most keys: dealt first
-  const int unit = uc / p.chunks, chunk = uc % p.chunks;
-  const int batch = unit / p.Hkv, kvh = unit % p.Hkv;
+  const int unit = p.by_chunks.of(uc), chunk = uc - unit * p.chunks;
+  const int batch = p.by_Hkv.of(unit), kvh = unit - batch * p.Hkv;
 
   // ---- this lane's rows (rows past the end repeat the last one and are not stored) and the interval of keys each attends
   int qpos[QT], head[QT], khi[QT], klo[QT];
-  int any_lo = 1 << 30, any_hi = -1, all_lo = 0, all_hi = 1 << 30;  // keys some row / every row of the tile attends
+  auto first_key = [&](int q) FL_INLINE { return max(0, q + p.dmin); };
+  auto last_key = [&](int q) FL_INLINE { return min(p.Lk - 1, max(p.dmax + q, p.pfx - 1)); };
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
-    // (a division costs thirty dependent instructions at the start of a kernel that takes a few microseconds: none where one head
-    // has all rows, or every head one)
-    const int crow = min(rt * RB + u * 16 + n16, p.rows - 1), gh = p.group == 1 ? 0 : p.Lq == 1 ? crow : crow / p.Lq;
+    const int crow = min(rt * RB + u * 16 + n16, p.rows - 1), gh = p.by_Lq.of(crow);
     qpos[u] = crow - gh * p.Lq;
-    head[u] = kvh * p.group + gh;
-    khi[u] = min(p.Lk - 1, max(p.dmax + qpos[u], p.pfx - 1));
-    klo[u] = max(0, qpos[u] + p.dmin);
-    any_lo = min(any_lo, klo[u]);
-    any_hi = max(any_hi, khi[u]);
-    all_lo = max(all_lo, klo[u]);
-    all_hi = min(all_hi, khi[u]);
+    head[u] = gh;
+    khi[u] = last_key(qpos[u]);
+    klo[u] = first_key(qpos[u]);
   }
-  any_lo = __builtin_amdgcn_readfirstlane(wave_min(any_lo));
-  any_hi = -__builtin_amdgcn_readfirstlane(wave_min(-any_hi));
-  all_lo = -__builtin_amdgcn_readfirstlane(wave_min(-all_lo));
-  all_hi = __builtin_amdgcn_readfirstlane(wave_min(all_hi));
+  // Keys that some row and that every row of the tile attends: both bounds grow with the position, so the smallest and the largest one
+  // say it, which are the first and the last row's, or 0 and Lq - 1 where the rows run on into another head.  (Taken over the wave
+  // by exchanges through LDS this was 24 of them ahead of the first load.)
+  const bool one_head = __builtin_amdgcn_readlane(head[0], 0) == __builtin_amdgcn_readlane(head[QT - 1], 15);
+  const int q_min = one_head ? __builtin_amdgcn_readlane(qpos[0], 0) : 0;
+  const int q_max = one_head ? __builtin_amdgcn_readlane(qpos[QT - 1], 15) : p.Lq - 1;
+  const int any_lo = first_key(q_min), any_hi = last_key(q_max), all_lo = first_key(q_max), all_hi = last_key(q_min);
+#pragma unroll
+  for (int u = 0; u < QT; ++u) head[u] += kvh * p.group;
   int t_end, t;
   {
     const int t0 = any_lo / 32, n = any_hi >= any_lo ? any_hi / 32 + 1 - t0 : 0;
     // chunk c takes n / chunks tiles, the first n % chunks of them one more
     int first = 0, share = n;
     if (p.chunks > 1) {
-      share = n / p.chunks;
+      share = p.by_chunks.of(n);
       const int more = n - share * p.chunks;
       first = share * chunk + min(chunk, more);
       share += chunk < more ? 1 : 0;
@@ -376,7 +373,7 @@ void rows_kernel(const RParams p) {
         o += a * ow[w];
       }
       if (p.chunks == 1) {
-        const int pr = rt * RB + r, hd = p.group == 1 ? 0 : p.Lq == 1 ? pr : pr / p.Lq, pos = pr - hd * p.Lq, oh = kvh * p.group + hd;
+        const int pr = rt * RB + r, hd = p.by_Lq.of(pr), pos = pr - hd * p.Lq, oh = kvh * p.group + hd;
         const float inv = L > 0.f ? 1.0f / L : 0.f;  // a row that attends nothing yields zeros
         typedef E ex4 __attribute__((ext_vector_type(4)));
         ex4 w;
@@ -402,7 +399,7 @@ void rows_kernel(const RParams p) {
 template <int D, int RB, class E>
 __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
   constexpr int TPR = D / 4, NG = 256 / TPR;
-  const int unit = blockIdx.x / p.rows, row = blockIdx.x % p.rows;
+  const int unit = p.by_rows.of(blockIdx.x), row = blockIdx.x - unit * p.rows;
   const int c = threadIdx.x % TPR * 4, grp = threadIdx.x / TPR;
   const int64_t slot0 = (((int64_t)unit * p.row_tiles + row / RB) * p.chunks) * RB + row % RB;
   __shared__ float xo[NG][D];
@@ -463,7 +460,7 @@ __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
     Lt += a * xml[w][1];
     ot += a * *reinterpret_cast<const f32x4*>(&xo[w][c]);
   }
-  const int batch = unit / p.Hkv, kvh = unit % p.Hkv, hd = row / p.Lq, pos = row - hd * p.Lq, oh = kvh * p.group + hd;
+  const int batch = p.by_Hkv.of(unit), kvh = unit - batch * p.Hkv, hd = p.by_Lq.of(row), pos = row - hd * p.Lq, oh = kvh * p.group + hd;
   const float inv = Lt > 0.f ? 1.0f / Lt : 0.f;
   typedef E ex4 __attribute__((ext_vector_type(4)));
   ex4 w;
