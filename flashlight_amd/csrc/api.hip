@@ -859,6 +859,7 @@ bool plan_rows(const fl_attn_params* p, fl::RParams* out, int* grid, int* waves,
   k.row_tiles = (int)row_tiles;
   k.chunks = (int)chunks;
   k.units = (int)units;
+  k.waves = nw;
   k.by_rows = fl::Div::by((uint32_t)rows);
   k.by_row_tiles = fl::Div::by((uint32_t)row_tiles);
   k.by_chunks = fl::Div::by((uint32_t)chunks);

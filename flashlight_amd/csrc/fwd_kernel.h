@@ -71,6 +71,21 @@ constexpr bool div_holds(uint32_t d) {
 static_assert(div_holds(1) && div_holds(2) && div_holds(3) && div_holds(5) && div_holds(7) && div_holds(641) && div_holds(1000) &&
               div_holds(65535) && div_holds(65537) && div_holds(0x3fffffffu) && div_holds(0x40000001u) && div_holds(0x7fffffffu));
 
+// Asks for every 64-byte line of a kernel's parameters at once.  Left to themselves the loads follow the branches that use them, and
+// half a dozen lines are misses one after the other ahead of a workgroup's first transfer.
+template <class P>
+__device__ __forceinline__ void fetch_params() {
+  constexpr int last = ((int)sizeof(P) - 1) / 64;
+  static_assert(last < 12, "a line per operand below");
+  const auto* const at = (const __attribute__((address_space(4))) uint32_t*)__builtin_amdgcn_kernarg_segment_ptr();
+  const uint32_t x[12] = {at[0], at[16 * (1 < last ? 1 : last)], at[16 * (2 < last ? 2 : last)], at[16 * (3 < last ? 3 : last)],
+                          at[16 * (4 < last ? 4 : last)], at[16 * (5 < last ? 5 : last)], at[16 * (6 < last ? 6 : last)],
+                          at[16 * (7 < last ? 7 : last)], at[16 * (8 < last ? 8 : last)], at[16 * (9 < last ? 9 : last)],
+                          at[16 * (10 < last ? 10 : last)], at[16 * last]};
+  asm volatile("" ::"s"(x[0]), "s"(x[1]), "s"(x[2]), "s"(x[3]), "s"(x[4]), "s"(x[5]), "s"(x[6]), "s"(x[7]), "s"(x[8]), "s"(x[9]),
+               "s"(x[10]), "s"(x[11]));
+}
+
 struct KParams {
   const bf16_t* q;
   const bf16_t* k;

@@ -15,7 +15,8 @@
 // What such a call spends beside its reads is a chain: with the sums over the waves unrolled (a run-time count was one LDS wait after the
 // other), no division where one head has all rows, and the merge's loads in flight together, 9.20 -> 8.86, decoding 31.2 -> 30.1, 22.1 ->
 // 21.7 and, 2 x 8 heads of 282 rows, 7.8 -> 7.5.  With nothing ahead of the first load that goes through LDS (the tile's bounds) and no
-// division at all (Div), 8.87 -> 8.19, decoding 30.0 -> 29.3 and 21.6 -> 20.6.
+// division at all (Div), 8.87 -> 8.19, decoding 30.0 -> 29.3 and 21.6 -> 20.6; with the parameters' lines asked for together
+// (fetch_params) 7.97, 28.5 and 20.1.
 //
 // Rows are packed: row x of key / value head n is position x % Lq of query head n * G + x / Lq, so the G query heads that
 // share a key / value head are rows of one tile and the keys are read once for all of them.
@@ -41,7 +42,7 @@ struct RParams {
   int64_t qs[3], ks[3], vs[3], os[3];        // element strides: batch, head, seq
   int32_t B, Hq, Hkv, Lq, Lk, group;
   int32_t rows;                              // group * Lq: packed rows per key / value head
-  int32_t row_tiles, chunks, units;          // units = B * Hkv
+  int32_t row_tiles, chunks, units, waves;   // units = B * Hkv; waves per workgroup
   Div by_rows, by_row_tiles, by_chunks, by_Hkv, by_Lq;
   int32_t by_xcd;                            // row tiles of one (unit, chunk) on one XCD (units * chunks >= 8)
   float scale_log2, cap_k1, cap_c;           // as in fwd_kernel; cap_c = 0: no soft-cap
@@ -96,8 +97,9 @@ void rows_kernel(const RParams p) {
   typedef E ex2 __attribute__((ext_vector_type(2)));
   typedef uint32_t vreg __attribute__((ext_vector_type(W / 2)));  // W elements of 16 bits
 
+  fetch_params<RParams>();
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int NW = blockDim.x / 64;
+  const int NW = p.waves;
   const int n16 = lane % 16, g = lane / 16;
 
   // ---- workgroup -> (unit, chunk, row tile); the row tiles of one (unit, chunk) read the same keys
@@ -398,6 +400,7 @@ void rows_kernel(const RParams p) {
 // the 1024 / D groups of them take every (1024 / D)-th chunk, so that a row's loads are in flight together.
 template <int D, int RB, class E>
 __global__ __launch_bounds__(256) void rows_merge_kernel(const RParams p) {
+  fetch_params<RParams>();
   constexpr int TPR = D / 4, NG = 256 / TPR;
   const int unit = p.by_rows.of(blockIdx.x), row = blockIdx.x - unit * p.rows;
   const int c = threadIdx.x % TPR * 4, grp = threadIdx.x / TPR;
