@@ -1155,6 +1155,12 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
     const bool growing = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM || is_doc(p->mask_kind);
     static const int knob = std::getenv("FL_HEAD_GROUP") ? std::atoi(std::getenv("FL_HEAD_GROUP")) : 0;  // tuning knob
     kp.head_group = !growing ? 1 : (knob > 0 ? knob : 4);
+    const uint32_t pairs = (uint32_t)p->B * p->Hq, per_xcd = pairs % 8 ? pairs : pairs / 8, rest = per_xcd % kp.head_group;
+    kp.by_heads = fl::Div::by((uint32_t)kp.head_group * kp.n_qtiles);
+    kp.by_head_group = fl::Div::by(kp.head_group);
+    kp.by_rest = fl::Div::by(rest ? rest : 1);
+    kp.by_Hq = fl::Div::by(p->Hq);
+    kp.by_group = fl::Div::by(kp.group);
   }
   kp.o_wide = reinterpret_cast<uintptr_t>(p->o) % 16 == 0 && p->o_strides[0] % 8 == 0 && p->o_strides[1] % 8 == 0 &&
               p->o_strides[2] % 8 == 0;

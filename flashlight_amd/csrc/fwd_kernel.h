@@ -72,7 +72,9 @@ static_assert(div_holds(1) && div_holds(2) && div_holds(3) && div_holds(5) && di
               div_holds(65535) && div_holds(65537) && div_holds(0x3fffffffu) && div_holds(0x40000001u) && div_holds(0x7fffffffu));
 
 // Asks for every 64-byte line of a kernel's parameters at once.  Left to themselves the loads follow the branches that use them, and
-// half a dozen lines are misses one after the other ahead of a workgroup's first transfer.
+// half a dozen lines are misses one after the other ahead of a workgroup's first transfer.  (This and Div in fwd_kernel, us: windows, 8 heads
+// of 1124, head dim 128, 9.86 -> 9.52, 2 x 16 of 322 10.01 -> 9.54; 42 x 8 of 448 with a shared bias, head dim 64, 47.6 -> 46.3; calls of
+// several workgroups per place, 0 to 1 %: another workgroup covers the start there.)
 template <class P>
 __device__ __forceinline__ void fetch_params() {
   constexpr int last = ((int)sizeof(P) - 1) / 64;
@@ -139,6 +141,9 @@ struct KParams {
   // 3: ((k3 x + k2) x + k1) x + k0
   int32_t score_fn;
   float score_k[4];
+  Div by_heads;      // head_group * n_qtiles
+  Div by_head_group, by_rest;  // head_group, and what the (batch, head) pairs of an XCD leave over
+  Div by_Hq, by_group;
   int32_t n_qtiles;  // ceil(Lq / BM)
   int32_t n_ktiles;  // ceil(Lk / BN)
 };
@@ -510,6 +515,7 @@ void fwd_kernel(const KParams p) {
   using LK = TileLayout<DQK>;
   using LV = TileLayout<DV>;
 
+  fetch_params<KParams>();
   constexpr int KG = T::KG;
   static_assert(KG == 1 || !(kDiff || kBias || kDump), "groups of waves: kernels without a second branch, bias operands or the dump");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
@@ -541,21 +547,21 @@ void fwd_kernel(const KParams p) {
       i /= 8;
     }
     const int G = p.head_group;
-    const int g = i / (G * nq), rem = i % (G * nq);
-    const int gg = min(G, run - G * g);
-    qt = nq - 1 - rem / gg;
-    bh = base + G * g + rem % gg;
+    const int g = p.by_heads.of(i), rem = i - g * (G * nq);
+    const int gg = min(G, run - G * g), rank = (gg == G ? p.by_head_group : p.by_rest).of(rem);
+    qt = nq - 1 - rank;
+    bh = base + G * g + rem - rank * gg;
     // document masks: the work of a query tile is the length of its tile list, known from the pre-pass
     if constexpr (kDoc) {
       if (!p.doc_own) {
-        const int32_t* order = p.doc_order + (bh / p.Hq) * nq;
-        const int head_of_order = order[0], mine = order[rem / gg];  // (both in flight together)
+        const int32_t* order = p.doc_order + p.by_Hq.of(bh) * nq;
+        const int head_of_order = order[0], mine = order[rank];  // (both in flight together)
         qt = head_of_order >= 0 ? mine : qt;
       }
     }
   }
-  const int head = bh % p.Hq, batch = bh / p.Hq;
-  const int kvh = head / p.group;
+  const int batch = p.by_Hq.of(bh), head = bh - batch * p.Hq;
+  const int kvh = p.by_group.of(head);
 
   const int q0 = qt * BM;             // first query row of the workgroup
   const int qw0 = q0 + wave * RW;     // first query row of this wave
