@@ -1415,6 +1415,19 @@ static int launch_gradients(const fl_attn_bwd_params* b, bool planned, void* scr
   if (plan.dkv > 1) bp.part = bp.part_dq + plan.dq_bytes / sizeof(float);
   bp.splits_dq = plan.dq;
   bp.splits = plan.dkv;
+  bp.head_group = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM || p->mask_kind == FL_MASK_DOCUMENT_CAUSAL ? 4 : 1;
+  bp.by_head_group = fl::Div::by(bp.head_group);
+  bp.by_group = fl::Div::by(bp.group);
+  bp.by_Hq = fl::Div::by(p->Hq);
+  for (int r = 0; r < 2; ++r) {
+    const uint32_t heads = r ? p->Hkv : p->Hq, tiles = ((r ? p->Lk : p->Lq) + 127) / 128, pairs = p->B * heads;
+    const uint32_t rest = (pairs % 8 ? pairs : pairs / 8) % bp.head_group;
+    bp.role[r].by_heads = fl::Div::by(bp.head_group * tiles);
+    bp.role[r].by_rest = fl::Div::by(rest ? rest : 1);
+    bp.role[r].by_oh = fl::Div::by(heads);
+    bp.role[r].by_splits = fl::Div::by(r ? plan.dkv : plan.dq);
+    bp.role[r].by_tiles = fl::Div::by(tiles);
+  }
   hipError_t e = in->launch_delta(bp, stream);
   if (e != hipSuccess) return fail((int)e, "backward: launch of the row-sum kernel failed: %s", hipGetErrorString(e));
   if (plan.both) {

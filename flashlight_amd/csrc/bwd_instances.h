@@ -55,10 +55,10 @@ hipError_t launch_bwd_both(const BParams& bp, hipStream_t stream) {
 
 template <int DV, class E>
 hipError_t launch_delta(const BParams& bp, hipStream_t stream) {
-  const int64_t rows = (int64_t)bp.B * bp.Hq * bp.Lq;
-  const int rows_per_block = 256 / (DV / 8);
-  hipLaunchKernelGGL((bwd_delta_kernel<DV, E>), dim3((unsigned)((rows + rows_per_block - 1) / rows_per_block)), dim3(256), 0,
-                     stream, bp);
+  const int rows_per_block = 256 / (DV / 8), blocks = (bp.Lq + rows_per_block - 1) / rows_per_block;
+  BParams p = bp;
+  p.by_delta_blocks = Div::by(blocks);
+  hipLaunchKernelGGL((bwd_delta_kernel<DV, E>), dim3((unsigned)((int64_t)bp.B * bp.Hq * blocks)), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 

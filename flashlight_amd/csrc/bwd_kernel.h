@@ -64,19 +64,25 @@ struct BParams {
   // bwd_both_kernel: `part` and `splits` are the dK/dV role's, these the dQ role's
   float* part_dq;
   int32_t splits_dq;
+  // Divisors, per role (0: dQ, 1: dK/dV).  (batch, head) pairs are dealt head_group at a time
+  int32_t head_group;
+  Div by_head_group, by_group, by_Hq, by_delta_blocks;
+  struct {
+    Div by_heads, by_rest, by_oh, by_splits, by_tiles;  // head_group * owner tiles; pairs an XCD leaves over; owner heads; splits; tiles
+  } role[2];
 };
 
-// delta[b, h, q] = -sum_d dO[b, h, q, d] * O[b, h, q, d]; one row per group of DV / 8 lanes.
+// delta[b, h, q] = -sum_d dO[b, h, q, d] * O[b, h, q, d]; one row per group of DV / 8 lanes, delta_blocks workgroups per (batch, head):
+// bound by reading both (6.4 TB/s at 4 x 16 x 4096, head dim 128).
 template <int DV, class E>
 __global__ __launch_bounds__(256) void bwd_delta_kernel(const BParams p) {
+  fetch_params<BParams>();
   typedef E ex8 __attribute__((ext_vector_type(8)));
-  constexpr int LPR = DV / 8;  // lanes per row, 16 bytes each
-  const int64_t rows = (int64_t)p.B * p.Hq * p.Lq;
-  const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
-  const int c = threadIdx.x % LPR;
+  constexpr int LPR = DV / 8, RPB = 256 / LPR;  // lanes per row, 16 bytes each; rows per workgroup
+  const int bh = p.by_delta_blocks.of(blockIdx.x), first = (blockIdx.x - bh * ((p.Lq + RPB - 1) / RPB)) * RPB;
+  const int b = p.by_Hq.of(bh), h = bh - b * p.Hq, q = first + threadIdx.x / LPR, c = threadIdx.x % LPR;
   float s = 0.f;
-  if (row < rows) {
-    const int q = (int)(row % p.Lq), h = (int)((row / p.Lq) % p.Hq), b = (int)(row / ((int64_t)p.Lq * p.Hq));
+  if (q < p.Lq) {
     const ex8 a = *reinterpret_cast<const ex8*>(p.dout + b * p.dos[0] + h * p.dos[1] + q * p.dos[2] + 8 * c);
     const ex8 o = *reinterpret_cast<const ex8*>(p.o + b * p.os[0] + h * p.os[1] + q * p.os[2] + 8 * c);
 #pragma unroll
@@ -84,7 +90,7 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const BParams p) {
   }
 #pragma unroll
   for (int d = 1; d < LPR; d *= 2) s += __shfl_xor(s, d);
-  if (row < rows && c == 0) p.delta[row] = -s;  // stored negated: the consumers add it (or start dP's accumulators from it)
+  if (q < p.Lq && c == 0) p.delta[(int64_t)bh * p.Lq + q] = -s;  // stored negated: the consumers add it (or start dP's accumulators from it)
 }
 
 // SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size
@@ -198,6 +204,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // different XCDs, hence ids are regrouped to give every XCD a contiguous run of (batch, head) pairs, head by head.
   // Under causal-like masks the work of a tile grows with the query position (ROLE_DQ) or shrinks with the key position
   // (ROLE_DKV): heads are taken four at a time and their tiles dealt longest first, so the grid drains on short ones.
+  const auto& divs = p.role[kDQ ? 0 : 1];
   const int n_own = kDQ ? (p.Lq + T::OWN - 1) / T::OWN : (p.Lk + T::OWN - 1) / T::OWN;
   const int oh = kDQ ? p.Hq : p.Hkv;
   // The splits of a tile are dealt next to each other.
@@ -211,23 +218,24 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       i /= 8;
     }
     if constexpr (SPLIT) {
-      split = i % splits;
-      i /= splits;
+      const int tile = divs.by_splits.of(i);
+      split = i - tile * splits;
+      i = tile;
     }
-    const int G = (p.mask_kind == MASK_CAUSAL || p.mask_kind == MASK_PREFIX || p.mask_kind == MASK_DOC_CAUSAL) ? 4 : 1;
-    const int g = i / (G * n_own), rem = i % (G * n_own);
+    const int G = p.head_group;
+    const int g = divs.by_heads.of(i), rem = i - g * (G * n_own);
     const int gg = min(G, run - G * g);
-    const int rank = rem / gg;  // 0 = longest under a causal-like mask
-    bh = base + G * g + rem % gg;
+    const int rank = (gg == G ? p.by_head_group : divs.by_rest).of(rem);  // 0 = longest under a causal-like mask
+    bh = base + G * g + rem - rank * gg;
     ot = kDQ ? n_own - 1 - rank : rank;
   }
-  const int ohead = bh % oh, batch = bh / oh;
+  const int batch = divs.by_oh.of(bh), ohead = bh - batch * oh;
   const int o0 = ot * T::OWN;               // first owner position of the workgroup
   const int o1 = min(o0 + T::OWN, kDQ ? p.Lq : p.Lk);
   const int opos = o0 + ow * 32 + r;        // this lane's owner position (a query row or a key)
   const int olen = kDQ ? p.Lq : p.Lk;
   const int slen = kDQ ? p.Lk : p.Lq;       // streamed sequence length
-  const int kvh = kDQ ? ohead / p.group : ohead;
+  const int kvh = kDQ ? (int)p.by_group.of(ohead) : ohead;
 
   // ---- streamed tile range [t_lo, t_hi] for the workgroup's owner range [o0, o1) under the positional mask ----------
   int t_lo = 0, t_hi = (slen + BT - 1) / BT - 1;
@@ -246,8 +254,13 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   const int n_tiles = t_hi >= t_lo ? t_hi - t_lo + 1 : 0;
   const int n_heads = kDQ ? 1 : p.group;   // ROLE_DKV walks the query heads of its group
   const int all_steps = n_tiles * n_heads;
-  const int s_first = SPLIT ? (int)((int64_t)all_steps * split / splits) : 0;
-  const int n_steps = SPLIT ? (int)((int64_t)all_steps * (split + 1) / splits) : all_steps;  // this workgroup's steps: [s_first, n_steps)
+  // first step of a split: all * split / splits, rounded down
+  auto split_start = [&](int all, int split) FL_INLINE -> int {
+    const int whole = divs.by_splits.of(all);
+    return whole * split + divs.by_splits.of((all - whole * splits) * split);
+  };
+  const int s_first = SPLIT ? split_start(all_steps, split) : 0;
+  const int n_steps = SPLIT ? split_start(all_steps, split + 1) : all_steps;  // this workgroup's steps: [s_first, n_steps)
 
   // ---- per-lane constants ---------------------------------------------------------------------------------------------
   float cap_k1 = 0.f, cap_c = 0.f;
@@ -286,8 +299,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // ---- global -> LDS transfers of a [rows][D] tile into its swizzled image ---------------------------------------------------
   // lane l of a 1 KiB transfer writes LDS bytes [16 l, 16 l + 16); it fetches the logical chunk that the swizzle maps
   // there.  Rows past `valid` repeat the last valid row (their contributions are masked).
-  auto load_tile = [&](const bf16_t* row0, int64_t stride, int valid, unsigned lds_off, int n_per_t) FL_INLINE {
-    const uint64_t base = uniform_ptr(row0);
+  auto load_tile = [&](uint64_t base, int64_t stride, int valid, unsigned lds_off, int n_per_t) FL_INLINE {
     const unsigned lds0 = (unsigned)(uintptr_t)smem + lds_off + wave * 1024;
     for (int it = 0; it < n_per_t; ++it) {
       const int id = it * NT + tid, row = id / L::CPR, pc = id % L::CPR;
@@ -295,34 +307,60 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       dma16(base, off, lds0 + it * NT * 16);
     }
   };
-  // streamed step s -> (query head of the group, tile).  ROLE_DKV: the statistics of the streamed rows (LSE, Delta) ride
-  // the tile transfers into LDS, 4 bytes per lane, so that the loop holds no ordinary global load: the wait such a load
-  // needs would also wait for the tile transfers that are in flight for the next step.
-  auto step_head = [&](int s) FL_INLINE { return kDQ ? ohead : kvh * p.group + s / n_tiles; };
-  auto step_tile = [&](int s) FL_INLINE { return t_lo + (kDQ ? s : s % n_tiles); };
+  // The streamed operands: whole tiles are fetched at one per-lane offset that does not change from tile to tile (the rows of a
+  // thread's transfers lie a multiple of the swizzle's period apart), from scalar addresses that advance by a tile per step; the last,
+  // ragged one works its offsets out.  (Worked out at every transfer, with a step's head and tile as quotient and rest of its number, this was
+  // a third of the instructions of the shared launch's loops; us for a training step: 4 x 16 x 4096 causal, head dim 128, 1260 -> 1237, 64, 677 ->
+  // 668; 16 over 3 x 4 of 1000 with a prefix 86.8 -> 84.9; 32 over 7 x 8 of 306, head dim 128, 104.9 -> 100.8.)  ROLE_DKV: the statistics of the streamed rows (LSE, Delta) ride the tile transfers into LDS, 4 bytes
+  // per lane, so that the loop holds no ordinary global load: the wait such a load needs would also wait for the tile transfers that are
+  // in flight for the next step.
+  constexpr int ROWS_PER_T = NT / L::CPR;
+  static_assert(NT % L::CPR == 0 && ROWS_PER_T % (L::RPW * (L::CPR >= 16 ? 16 : L::CPR >= 8 ? 8 : 4)) == 0, "one offset for all transfers of a thread");
+  struct Operand {
+    uint64_t base;       // of the batch entry's (or, ROLE_DQ, of the head's) first row
+    int64_t head_bytes;  // ROLE_DKV: from one query head to the next
+    uint32_t tile_bytes, row_bytes;
+    unsigned off;
+  };
+  auto operand = [&](const bf16_t* ptr, const int64_t (&st)[3]) FL_INLINE -> Operand {
+    const uint32_t row_bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)st[2] * 2u));
+    return {uniform_ptr(ptr), uniform_i64(st[1] * 2), row_bytes * BT, row_bytes,
+            (unsigned)(tid / L::CPR) * row_bytes + L::swz_kv(tid / L::CPR, tid % L::CPR) * 16u};
+  };
+  const Operand s1 = operand(kDQ ? kptr : p.q + (int64_t)batch * p.qs[0], kDQ ? p.ks : p.qs);
+  const Operand s2 = operand(kDQ ? vptr : p.dout + (int64_t)batch * p.dos[0], kDQ ? p.vs : p.dos);
+  const uint64_t lse_at = uniform_ptr(p.lse), delta_at = uniform_ptr(p.delta);
   auto load_tiles = [&](int tile, int hd, int slot) FL_INLINE {
-    const int t0 = tile * BT, valid = min(BT, slen - t0);
-    if constexpr (kDQ) {
-      load_tile(kptr + (int64_t)t0 * p.ks[2], p.ks[2], valid, T::T1_OFF + slot * T::TBYTES, T::T_PER_T);
-      load_tile(vptr + (int64_t)t0 * p.vs[2], p.vs[2], valid, T::T2_OFF + slot * T::TBYTES, T::T_PER_T);
+    const int valid = slen - tile * BT;
+    auto at = [&](const Operand& s) FL_INLINE -> uint64_t {
+      uint64_t a = s.base + (uint64_t)(uint32_t)tile * s.tile_bytes;
+      if constexpr (!kDQ) a += (uint64_t)(s.head_bytes * hd);
+      return a;
+    };
+    const uint64_t a1 = at(s1), a2 = at(s2);
+    if (valid >= BT) {
+      const unsigned lds0 = (unsigned)(uintptr_t)smem + slot * T::TBYTES + wave * 1024;
+#pragma unroll
+      for (int it = 0; it < T::T_PER_T; ++it) dma16(a1 + (uint64_t)(it * ROWS_PER_T * s1.row_bytes), s1.off, lds0 + T::T1_OFF + it * NT * 16);
+#pragma unroll
+      for (int it = 0; it < T::T_PER_T; ++it) dma16(a2 + (uint64_t)(it * ROWS_PER_T * s2.row_bytes), s2.off, lds0 + T::T2_OFF + it * NT * 16);
     } else {
-      load_tile(p.q + (int64_t)batch * p.qs[0] + (int64_t)hd * p.qs[1] + (int64_t)t0 * p.qs[2], p.qs[2], valid,
-                T::T1_OFF + slot * T::TBYTES, T::T_PER_T);
-      load_tile(p.dout + (int64_t)batch * p.dos[0] + (int64_t)hd * p.dos[1] + (int64_t)t0 * p.dos[2], p.dos[2], valid,
-                T::T2_OFF + slot * T::TBYTES, T::T_PER_T);
+      load_tile(a1, kDQ ? p.ks[2] : p.qs[2], valid, T::T1_OFF + slot * T::TBYTES, T::T_PER_T);
+      load_tile(a2, kDQ ? p.vs[2] : p.dos[2], valid, T::T2_OFF + slot * T::TBYTES, T::T_PER_T);
+    }
+    if constexpr (!kDQ) {
       if (wave == 0) {
         // one wave brings both arrays (every wave waits for all of its own transfers before the barrier, so the counts
         // need not match).  Lane l fetches row t0 + l; lanes past the end of the tile or of the sequence repeat the last
         // valid row (those rows are masked).
         static_assert(BT <= 64, "one lane per streamed row");
-        const int64_t row0 = ((int64_t)batch * p.Hq + hd) * p.Lq + t0;
-        const unsigned off = (unsigned)min(lane, valid - 1) * 4u;
-        dma4(uniform_ptr(p.lse + row0), off, (unsigned)(uintptr_t)smem + T::S1_OFF + slot * T::SBYTES);
-        dma4(uniform_ptr(p.delta + row0), off, (unsigned)(uintptr_t)smem + T::S2_OFF + slot * T::SBYTES);
+        const uint64_t row0 = (uint64_t)(((int64_t)batch * p.Hq + hd) * p.Lq + tile * BT) * 4u;
+        const unsigned off = (unsigned)min(lane, min(BT, valid) - 1) * 4u;
+        dma4(lse_at + row0, off, (unsigned)(uintptr_t)smem + T::S1_OFF + slot * T::SBYTES);
+        dma4(delta_at + row0, off, (unsigned)(uintptr_t)smem + T::S2_OFF + slot * T::SBYTES);
       }
     }
   };
-  auto load_step = [&](int s, int slot) FL_INLINE { load_tiles(step_tile(s), step_head(s), slot); };
   // the ids of the streamed positions, for a step that compares them (positions past the end repeat the last one)
   auto load_ids = [&](int tile, int slot) FL_INLINE {
     const int t0 = tile * BT;
@@ -408,8 +446,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   if (kDoc ? n_tiles > 0 : n_steps > s_first) {
     if constexpr (!kDQ) {
       const int valid = o1 - o0;
-      load_tile(kptr + (int64_t)o0 * p.ks[2], p.ks[2], valid, T::O1_OFF, T::O_PER_T);
-      load_tile(vptr + (int64_t)o0 * p.vs[2], p.vs[2], valid, T::O2_OFF, T::O_PER_T);
+      load_tile(uniform_ptr(kptr + (int64_t)o0 * p.ks[2]), p.ks[2], valid, T::O1_OFF, T::O_PER_T);
+      load_tile(uniform_ptr(vptr + (int64_t)o0 * p.vs[2]), p.vs[2], valid, T::O2_OFF, T::O_PER_T);
     }
   }
 
@@ -434,7 +472,6 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     return skip;
   };
-  auto classify_step = [&](int s, bool& full, bool& doc_uniform) FL_INLINE -> bool { return classify_tile(step_tile(s), full, doc_uniform); };
   // Sum of the bias operands at (query, key) of head `hd` (positions inside the sequences)
   auto bias_at = [&](int qpos, int kpos, int hd) FL_INLINE -> float {
     float b = 0.f;
@@ -449,6 +486,9 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     return b;
   };
+  // ALiBi slope of the streamed head in log2 units, worked out where the head changes
+  int slope_head = -1;
+  float slope_l2 = 0.f;
   // One step: the tile in ring slot `slot` against the owner operands.
   auto run_tile = [&](int tile, const int shead, int slot, bool full, bool doc_uniform) FL_INLINE {
     const int t0 = tile * BT;
@@ -457,9 +497,12 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       // ---- X1 = T1 . O1^T, then the weights; X2 = T2 . O2^T, then dS (one after the other: the two fp32 tiles are
       // never live together, which is what lets 128 accumulator registers fit) ----------------------------------------------
       // register i of block sb is streamed position t0 + 32 (qh TB + sb) + 8 (i / 4) + 4 h + i % 4
-      float slope_l2 = 0.f;
-      if constexpr (kAlibi)
-        slope_l2 = p.alibi_heads > 0 ? exp2f(-8.0f * (float)(shead + 1) / (float)p.alibi_heads) * kLog2e : 0.f;
+      if constexpr (kAlibi) {
+        if (shead != slope_head) {
+          slope_head = shead;
+          slope_l2 = p.alibi_heads > 0 ? exp2f(-8.0f * (float)(shead + 1) / (float)p.alibi_heads) * kLog2e : 0.f;
+        }
+      }
       // 4 consecutive streamed rows of a staged per-row fp32 array
       auto rows4 = [&](unsigned staged_off, int q4) FL_INLINE -> f32x4 {
         return *reinterpret_cast<const f32x4*>(smem + staged_off + slot * T::SBYTES + (q4 - t0) * 4);
@@ -716,7 +759,6 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       if constexpr (kSched) sched_gradients<KS, TB, DB, kDQ>();
     }
   };
-  auto run_step = [&](int s, int slot, bool full, bool doc_uniform) FL_INLINE { run_tile(step_tile(s), step_head(s), slot, full, doc_uniform); };
   if constexpr (kDoc) {
     // Most tiles of the range are dead: documents apart.  The live ones are listed first, a wave per LIST / NW tiles with their
     // table reads in flight together; every head of the group then walks the list, and splits share out what is on it.  (Read one after
@@ -756,8 +798,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       }
       __syncthreads();
       const int all_live = n_live * n_heads;
-      const int s_first = SPLIT ? (int)((int64_t)all_live * split / splits) : 0;
-      const int n_steps = SPLIT ? (int)((int64_t)all_live * (split + 1) / splits) : all_live;
+      const int s_first = SPLIT ? split_start(all_live, split) : 0;
+      const int n_steps = SPLIT ? split_start(all_live, split + 1) : all_live;
       if (s_first >= n_steps) continue;
       int head = kDQ ? ohead : kvh * p.group + s_first / n_live, i = s_first % n_live;
       auto at_list = [&](int i) FL_INLINE { return (uint32_t)__builtin_amdgcn_readfirstlane((int)list[i]); };
@@ -784,37 +826,49 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     dma_wait<0>();  // (a workgroup that found nothing to do has asked for its owner rows all the same)
   } else {
-    // positional masks: every step of [t_lo, t_hi] is visited (a dead one only occurs under a prefix-LM mask)
+    // positional masks: every step of [t_lo, t_hi] is visited (a dead one only occurs under a prefix-LM mask); ROLE_DKV walks them for
+    // every query head of the group.  The step to be fetched next is (tile, head); its place goes from step to step (worked out from
+    // the step's number it was two divisions per step).
+    int tile = t_lo + s_first, head = kDQ ? ohead : kvh * p.group;
+    if (!kDQ && SPLIT && s_first >= n_tiles && n_tiles > 0) {
+      const int skipped = s_first / n_tiles;
+      head += skipped;
+      tile -= skipped * n_tiles;
+    }
+    int tile_now = tile, head_now = head;
+    auto fetch_next = [&](int slot) FL_INLINE {
+      load_tiles(tile, head, slot);
+      ++tile;
+      if (!kDQ && tile > t_hi) {
+        tile = t_lo;
+        ++head;
+      }
+    };
+    auto step_at = [&](int s, const int slot) FL_INLINE {
+      __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
+      const int t = tile_now, hd = head_now;
+      tile_now = tile;
+      head_now = head;
+      if (s + 1 < n_steps) fetch_next(slot ^ 1);
+      bool full, doc_uniform;
+      if (!classify_tile(t, full, doc_uniform)) run_tile(t, hd, slot, full, doc_uniform);
+      dma_wait<0>();
+    };
     if constexpr (T::UNROLL2) {
       // (two steps per turn of the loop: the ring slot is then a constant, part of the LDS instructions' offsets instead of 20
       // address additions per step)
-      auto step_at = [&](int s, auto slot_tag) FL_INLINE {
-        constexpr int slot = decltype(slot_tag)::value;
-        __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
-        if (s + 1 < n_steps) load_step(s + 1, slot ^ 1);
-        bool full, doc_uniform;
-        if (!classify_step(s, full, doc_uniform)) run_step(s, slot, full, doc_uniform);
-        dma_wait<0>();
-      };
-      if (n_steps > s_first) load_step(s_first, 0);
+      if (n_steps > s_first) fetch_next(0);
       dma_wait<0>();
       int s = s_first;
       for (; s + 1 < n_steps; s += 2) {
-        step_at(s, std::integral_constant<int, 0>{});
-        step_at(s + 1, std::integral_constant<int, 1>{});
+        step_at(s, 0);
+        step_at(s + 1, 1);
       }
-      if (s < n_steps) step_at(s, std::integral_constant<int, 0>{});
+      if (s < n_steps) step_at(s, 0);
     } else {
-      if (n_steps > s_first) load_step(s_first, s_first & 1);
+      if (n_steps > s_first) fetch_next(0);
       dma_wait<0>();
-      for (int s = s_first; s < n_steps; ++s) {
-        const int slot = s & 1;
-        __syncthreads();  // publishes slot `slot` (every wave waited for its own transfers) and frees the other slot
-        if (s + 1 < n_steps) load_step(s + 1, slot ^ 1);
-        bool full, doc_uniform;
-        if (!classify_step(s, full, doc_uniform)) run_step(s, slot, full, doc_uniform);
-        dma_wait<0>();
-      }
+      for (int s = s_first; s < n_steps; ++s) step_at(s, (s - s_first) & 1);
     }
   }
 
@@ -894,6 +948,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 template <class T>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
 void bwd_kernel(const BParams p) {
+  fetch_params<BParams>();
   bwd_tile<T, false>(p, blockIdx.x, 1, nullptr);
 }
 
@@ -902,6 +957,7 @@ template <class TQ, class TKV>
 __global__ __launch_bounds__(TQ::NT) __attribute__((amdgpu_waves_per_eu(TQ::WAVES_PER_EU, TQ::WAVES_PER_EU)))
 void bwd_both_kernel(const BParams p) {
   static_assert(TQ::NT == TKV::NT, "one workgroup size");
+  fetch_params<BParams>();
   const int n_kv = p.B * p.Hkv * ((p.Lk + TKV::OWN - 1) / TKV::OWN) * p.splits;
   if ((int)blockIdx.x < n_kv) bwd_tile<TKV, true>(p, blockIdx.x, p.splits, p.part);
   else bwd_tile<TQ, true>(p, blockIdx.x - n_kv, p.splits_dq, p.part_dq);
@@ -916,9 +972,10 @@ __device__ __forceinline__ void bwd_sum_block(const BParams& p, const int block,
   using E = typename T::Elem;
   typedef E ex4 __attribute__((ext_vector_type(4)));
   const int olen = kDQ ? p.Lq : p.Lk, oh = kDQ ? p.Hq : p.Hkv, n_own = (olen + T::OWN - 1) / T::OWN;
-  const int tile = block / 4, bh = tile / n_own, head = bh % oh, batch = bh / oh;
+  const auto& divs = p.role[kDQ ? 0 : 1];
+  const int tile = block / 4, bh = divs.by_tiles.of(tile), batch = divs.by_oh.of(bh), head = bh - batch * oh;
   const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int pos = tile % n_own * T::OWN + block % 4 * 32 + lane % 32;
+  const int pos = (tile - bh * n_own) * T::OWN + block % 4 * 32 + lane % 32;
   if (pos >= olen) return;
   const int64_t split_stride = (int64_t)p.B * oh * n_own * 4 * SETS * DB * 16 * 64;
   const float* from = part + ((int64_t)block * SETS + set) * DB * 16 * 64 + lane * 4;
@@ -945,6 +1002,7 @@ __device__ __forceinline__ void bwd_sum_block(const BParams& p, const int block,
 // Workgroups [0, 8 tiles) dK and dV of every block of 32 keys when that role was split, the others dQ.
 template <class TQ, class TKV>
 __global__ __launch_bounds__(256) void bwd_split_sum_kernel(const BParams p) {
+  fetch_params<BParams>();
   int block = blockIdx.x;
   if (p.splits > 1) {
     const int n_kv = p.B * p.Hkv * ((p.Lk + TKV::OWN - 1) / TKV::OWN) * 8;
