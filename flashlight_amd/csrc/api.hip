@@ -323,6 +323,42 @@ FewPlan plan_few(const fl_attn_params* p, uint32_t want) {
   return x;
 }
 
+// Differential attention.  A group of waves per softmax branch: each holds one result, which leaves the registers room for 64-key tiles,
+// both walk the same V tiles, and a call of few workgroups takes half as long.  One after the other in the same waves, the branches
+// need 32-key tiles.  us, one after the other -> this rule: head dim 64, causal: 2 x 16 heads of 4096 238 -> 225, 8 of 16384 853 -> 798,
+// 4 x 16 of 512 29.1 -> 17.4, 8 of 1024 47.1 -> 20.5, 4 x 8 of 2048 90.8 -> 62.1; head dim 128, 4 x 8 of 1024 114 -> 67, 2 x 16 of 4096 589 -> 554.
+struct DiffPlan {
+  int waves = 0;   // preferred waves per branch (0: no preference)
+  int keys = 0;    // preferred keys per tile
+  int groups = 1;  // 1: the branches one after the other
+};
+DiffPlan plan_diff(const fl_attn_params* p) {
+  DiffPlan x;
+  if (!p->diff || p->attended_dump) return x;
+  const bool narrow = p->Dqk == 64, window = p->mask_kind == FL_MASK_SLIDING, growing = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM;
+  const int64_t tiles = (int64_t)p->B * p->Hq * ((p->Lq + 127) / 128);
+  const int64_t visited = window ? std::min<int64_t>(p->Lk, (int64_t)p->window + 128) : p->Lk;
+  x.waves = 4;
+  x.keys = 32;
+  // Short walks whose workgroups of 128 rows fill rounds of two per compute unit: one start and one store for both branches.  us, one after
+  // the other / a group each: head dim 64, unmasked, 16 x 16 of 160 14.7 / 17.2, of 256 22.4 / 23.5, of 450 61.0 / 65.7, of 512 65.0 / 65.7, but of
+  // 300 (768 tiles) 39.1 / 34.4; causal of 200 20.9 / 19.4; head dim 128, causal of 256 57.9 / 60.6, of 512 145 / 134, unmasked of 512 170 / 174.
+  // Windows, 4 x 16 of 4096, head dim 128: of 256 150 / 171, of 1100 336 / 325 (at head dim 64 with 64 rows: of 256 123 / 96, of 1500 322 / 283).
+  const bool full_rounds = tiles > 256 && (tiles % 512 == 0 || tiles % 512 > 384);
+  if (window ? !narrow && visited <= 1024 : full_rounds && visited <= (!growing ? 512 : narrow ? 0 : 256)) return x;
+  x.groups = 2;
+  // Up to 16 tiles of 128 rows keep 32 keys, the shape that the dump of attended pairs has and is compared in at every edge (2 heads of 256:
+  // 18.3 -> 13.9, where 64 rows and keys take 8.5).
+  if (narrow && tiles <= 16) return x;
+  x.keys = 64;
+  // 64 rows per workgroup, two of which share a compute unit, where 128 would leave a round far from full or the walks are short (head
+  // dim 128 spills so).  us, head dim 64, 128 rows -> 64: causal, 8 heads of 1024 27.7 -> 20.5, 3 x 8 of 2048 52.0 -> 49.8, 6 x 8 of 2048 110 -> 100,
+  // 8 x 32 of 300 36.4 -> 27.0, of 1024 152 -> 140; unmasked, 6 of 8192 362 -> 329; causal, 4 x 8 of 2048 62.1 -> 64.1, 2 x 16 of 4096 220 ->
+  // 223, 8 of 16384 798 -> 818; unmasked, 8 of 8192 393 -> 414.
+  if (narrow && (tiles <= 448 || visited < 2048 || (growing && tiles > 512 && tiles < 1024))) x.waves = 2;
+  return x;
+}
+
 const fl::Instance* select_instance(const fl_attn_params* p) {
   const uint32_t want = wanted_features(p);
   const fl::Instance* best = nullptr;
@@ -358,7 +394,8 @@ const fl::Instance* select_instance(const fl_attn_params* p) {
   const bool wide_group = p->mask_kind == FL_MASK_NONE && want == 0 && p->Dqk == 128 && p->Dv == 128 &&
                           (int64_t)p->B * p->Hq * ((p->Lq + 255) / 256) >= 512;
   const FewPlan few = plan_few(p, want);
-  const int preferred_nw = few.waves ? few.waves : short_loop ? 2 : (wide_group ? 8 : 4);
+  const DiffPlan diff = plan_diff(p);
+  const int preferred_nw = diff.waves ? diff.waves : few.waves ? few.waves : short_loop ? 2 : (wide_group ? 8 : 4);
   for (int i = 0; i < fl::kNumInstances; ++i) {
     const fl::Instance& in = fl::kInstances[i];
     if (in.dqk != p->Dqk || in.dv != p->Dv || in.dtype != p->dtype) continue;
@@ -366,8 +403,8 @@ const fl::Instance* select_instance(const fl_attn_params* p) {
     const uint32_t extra = in.feat & ~want;
     if (extra & ~kOptionalFeatures) continue;
     if (want_rw && (in.rw != want_rw || in.bn != want_bn || in.nw != want_nw || (want_ns && in.ns != want_ns))) continue;
-    // fewer unused features first; among equals the preferred workgroup size, then the listed order
-    const int n = 2 * __builtin_popcount(extra) + (in.nw == preferred_nw ? 0 : 1);
+    // fewer unused features first; among equals the preferred workgroup size, the preferred tile, then the listed order
+    const int n = 4 * __builtin_popcount(extra) + (in.nw == preferred_nw ? 0 : 2) + (!diff.keys || in.bn == diff.keys ? 0 : 1);
     if (n < best_extra) {
       best = &in;
       best_extra = n;
@@ -408,6 +445,7 @@ int64_t lds_bytes_for(const fl::Instance* in, const fl_attn_params* p) {
 int64_t prepass_lds_bytes(int64_t n_ktiles) { return n_ktiles * 20; }
 // Groups of waves a call is launched with, and the LDS of all of them
 int groups_for(const fl::Instance* in, const fl_attn_params* p) {
+  if (p->diff) return std::min(plan_diff(p).groups, in->max_groups);
   const int groups = std::min(plan_few(p, wanted_features(p)).groups, in->max_groups);
   return lds_bytes_for(in, p) + (int64_t)(groups - 1) * in->lds_fixed_bytes <= fl::kMaxLdsBytes ? groups : 1;
 }
@@ -973,10 +1011,10 @@ int fl_attn_plan(const fl_attn_params* p, int64_t out[8]) {
   out[1] = in->bn;
   out[2] = in->nw * 64;
   out[3] = (int64_t)p->B * p->Hq * ((p->Lq + bm - 1) / bm);
-  out[4] = lds_bytes_for(in, p);
   out[5] = in->feat;
   out[6] = 0;
   out[7] = groups_for(in, p);
+  out[4] = p->diff && out[7] == 2 ? in->branches_lds_bytes : lds_bytes_for(in, p);
   {
     // calls the shared-bias streaming forward takes: its fixed shape, and out[6] = 1
     fl::PParams pb;
@@ -1168,7 +1206,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   const int grid = p->B * p->Hq * kp.n_qtiles;
 
   const int groups = groups_for(in, p);
-  int lds = (int)lds_bytes_for(in, p) + (groups - 1) * in->lds_fixed_bytes;
+  int lds = p->diff && groups == 2 ? in->branches_lds_bytes : (int)lds_bytes_for(in, p) + (groups - 1) * in->lds_fixed_bytes;
 
   if (is_doc(p->mask_kind)) {
     const DocScratch d = doc_scratch(p->B, p->Lk, bm, in->bn);

@@ -444,8 +444,12 @@ struct FwdTraits {
   static constexpr int NS = NS_;  // K/V tiles resident in LDS (ring); transfers run NS - 1 tiles ahead of their use
   static_assert(NS >= 2 && NS <= 8 && NS % 2 == 0, "ring depth (even: the two score buffers alternate with the slots)");
   static constexpr uint32_t FEAT = FEAT_;
-  static constexpr int KG = KG_;      // groups of NW waves that share the rows and take a part of the key tiles each
+  // groups of NW waves that share the rows and take a part of the key tiles each or, in differential attention, a softmax branch each
+  // (one group there walks the branches one after the other)
+  static constexpr int KG = KG_;
+  static constexpr bool BRANCHES = (FEAT_ & F_DIFF) && KG == 2;
   static constexpr int NT = NW * 64;  // threads of a group
+  static constexpr int NTV = BRANCHES ? KG * NT : NT;  // threads that bring in a V tile (the branches share it)
   static constexpr int BM = NW * RW;
   static constexpr int QB = RW / 32;   // 32-row query blocks per wave
   static constexpr int KB = BN / 32;   // 32-key blocks per tile
@@ -453,8 +457,8 @@ struct FwdTraits {
   static constexpr int DVB = DV / 32;  // 32-wide blocks of the value dimension
   static constexpr int KBYTES = BN * DQK * 2, VBYTES = BN * DV * 2;
   static constexpr int K_CHUNKS = BN * DQK / 8, V_CHUNKS = BN * DV / 8;
-  static constexpr int K_PER_T = K_CHUNKS / NT, V_PER_T = V_CHUNKS / NT;
-  static_assert(K_CHUNKS % NT == 0 && V_CHUNKS % NT == 0, "tile must divide evenly over the threads");
+  static constexpr int K_PER_T = K_CHUNKS / NT, V_PER_T = V_CHUNKS / NTV;
+  static_assert(K_CHUNKS % NT == 0 && V_CHUNKS % NTV == 0, "tile must divide evenly over the threads");
   static_assert(RW % 32 == 0 && BN % 32 == 0 && DQK % 16 == 0 && DV % 32 == 0, "MFMA 32x32x16 blocking");
   static_assert(NW <= 8, "tile classes are packed two bits per wave into 16 bits");
   // waves per SIMD the register budget is sized for
@@ -481,8 +485,11 @@ struct FwdTraits {
   static_assert(!(FEAT & F_DOC) || (BN * 8) % 256 == 0, "whole transfers of 64 dwords");
   static constexpr int K_OFF = 0, V_OFF = NS * KBYTES, B_OFF = NS * (KBYTES + VBYTES), R_OFF = B_OFF + NS * BBYTES,
                        I_OFF = R_OFF + NS * RBYTES, LIST_OFF = I_OFF + NS * IBYTES;
-  static constexpr int LDS_FIXED_BYTES = KG * LIST_OFF;
-  static_assert(KG == 1 || (KG - 1) * NW * 64 * QB * (16 * DVB + 2) * 4 <= LDS_FIXED_BYTES, "the groups' results must fit in LDS");
+  // (differential attention: a K ring per branch, then the V ring of both; at the end each branch leaves half of its columns there)
+  static constexpr int RING_BYTES = BRANCHES ? NS * (KG * KBYTES + VBYTES) : KG * LIST_OFF, HALVES_BYTES = BRANCHES ? NW * 64 * QB * 16 * DVB * 4 : 0;
+  static constexpr int LDS_FIXED_BYTES = RING_BYTES > HALVES_BYTES ? RING_BYTES : HALVES_BYTES;
+  static_assert(KG == 1 || BRANCHES || (KG - 1) * NW * 64 * QB * (16 * DVB + 2) * 4 <= LDS_FIXED_BYTES, "the groups' results must fit in LDS");
+  static_assert(!(FEAT_ & F_DIFF) || (KG <= 2 && DVB % 2 == 0 && !(FEAT_ & (F_BIAS | F_DOC | F_GATE))), "differential attention");
 };
 
 // The main loop is software-pipelined over key tiles so that one wave keeps both the matrix pipe and the vector
@@ -517,15 +524,19 @@ void fwd_kernel(const KParams p) {
 
   fetch_params<KParams>();
   constexpr int KG = T::KG;
-  static_assert(KG == 1 || !(kDiff || kBias || kDump), "groups of waves: kernels without a second branch, bias operands or the dump");
+  constexpr bool kBranches = T::BRANCHES;         // the groups take a softmax branch each
+  constexpr bool kSplit = KG > 1 && !kBranches;  // the groups take parts of the tiles
+  constexpr bool kSequential = kDiff && !kBranches;
+  static_assert(!kSplit || !(kBias || kDump), "groups of waves: kernels without bias operands or the dump");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];
   // tile list (document masks): word 0 = number of entries, then one entry per key tile that is not empty for the
   // whole workgroup, in key order: bits 0-15 tile index, bits 16.. two class bits per wave
   const uint32_t* tlist = reinterpret_cast<const uint32_t*>(smem_all + KG * T::LIST_OFF) + 1;
 
-  // each group of waves has its own K/V ring
+  // each group of waves has its own K/V ring (the branches of differential attention a K ring each and one V ring)
   const int group = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
-  unsigned char* const smem = KG > 1 ? smem_all + group * T::LIST_OFF : smem_all;
+  unsigned char* const smem = KG > 1 ? smem_all + group * (kBranches ? T::V_OFF : T::LIST_OFF) : smem_all;
+  unsigned char* const smem_v = kBranches ? smem_all + KG * T::V_OFF : smem + T::V_OFF;
   const int tid = KG > 1 ? threadIdx.x % NT : threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   const int r = lane % 32, h = lane / 32;
@@ -598,7 +609,7 @@ void fwd_kernel(const KParams p) {
     n_own = max(0, min(n_list, all - group * n_list));
     first = n_own > 0 ? group * n_list : 0;
   };
-  if constexpr (KG > 1 && !kDoc) {
+  if constexpr (kSplit && !kDoc) {
     take_part();
     t_lo += first;
   }
@@ -630,7 +641,7 @@ void fwd_kernel(const KParams p) {
   // tile-list entry of list position i (the last entry again past the end): bits 0-15 tile index, two class bits per
   // wave from bit 16 on (only this wave's are filled in when the entry is computed rather than read)
   auto list_entry = [&](int i) FL_INLINE -> uint32_t {
-    const int last_own = KG > 1 ? max(n_own, 1) - 1 : n_list - 1;
+    const int last_own = kSplit ? max(n_own, 1) - 1 : n_list - 1;
     if constexpr (kDoc) {
       return tlist[first + min(i, last_own)];
     } else {
@@ -710,13 +721,14 @@ void fwd_kernel(const KParams p) {
     }
   }
 
-  f32x16 ofin[kDiff ? DVB : 1][kDiff ? QB : 1];  // branch-0 result kept while branch 1 runs (diff only)
+  f32x16 ofin[kSequential ? DVB : 1][kSequential ? QB : 1];  // branch-0 result kept while branch 1 runs
   f32x16 oacc[DVB][QB];
   float m_run[QB], l_run[QB];
   auto ref_now = [&](int qb) FL_INLINE { return (m_run[qb] == -INFINITY) ? 0.f : m_run[qb]; };
 
 #pragma unroll
-  for (int br = 0; br < (kDiff ? 2 : 1); ++br) {
+  for (int turn = 0; turn < (kSequential ? 2 : 1); ++turn) {
+    const int br = kBranches ? group : turn;  // softmax branch
     const bf16_t* qptr = p.q + (int64_t)batch * p.qs[0] + (int64_t)head * p.qs[1] + (int64_t)br * p.q_branch_stride;
     const bf16_t* kptr = p.k + (int64_t)batch * p.ks[0] + (int64_t)kvh * p.ks[1] + (int64_t)br * p.k_branch_stride;
     const bf16_t* vptr = p.v + (int64_t)batch * p.vs[0] + (int64_t)kvh * p.vs[1];
@@ -749,14 +761,15 @@ void fwd_kernel(const KParams p) {
     // keys are masked, p = 0).
     // LDS byte addresses this wave's transfers of slot 0, first transfer, land at
     const unsigned lds_k = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem + T::K_OFF + wave * 1024);
-    const unsigned lds_v = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem + T::V_OFF + wave * 1024);
+    const unsigned lds_v = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem_v + (kBranches ? group * NW + wave : wave) * 1024);
     const unsigned lds_i = __builtin_amdgcn_readfirstlane((unsigned)(uintptr_t)smem + T::I_OFF + wave * (BN * 8));
     // The rows of a thread's transfer `it` lie it * (NT / CPR) below those of its transfer 0.  When that step is a multiple
     // of the swizzle's period in rows, the chunk a lane fetches is the same for every transfer, and one per-lane offset
     // serves them all: the row step goes into the scalar base address instead of into a register per transfer.
-    constexpr int K_ROWS_PER_T = NT / LK::CPR, V_ROWS_PER_T = NT / LV::CPR;
+    constexpr int K_ROWS_PER_T = NT / LK::CPR, V_ROWS_PER_T = T::NTV / LV::CPR;
     constexpr bool kOneKoff = NT % LK::CPR == 0 && K_ROWS_PER_T % (LK::RPW * (LK::CPR >= 16 ? 16 : LK::CPR)) == 0;
-    constexpr bool kOneVoff = NT % LV::CPR == 0 && V_ROWS_PER_T % (LV::RPW * (LV::CPR >= 16 ? 16 : LV::CPR)) == 0;
+    constexpr bool kOneVoff = T::NTV % LV::CPR == 0 && V_ROWS_PER_T % (LV::RPW * (LV::CPR >= 16 ? 16 : LV::CPR)) == 0;
+    const int tid_v = kBranches ? group * NT + tid : tid;
     unsigned koff[kOneKoff ? 1 : T::K_PER_T], voff[kOneVoff ? 1 : T::V_PER_T];
 #pragma unroll
     for (int it = 0; it < (kOneKoff ? 1 : T::K_PER_T); ++it) {
@@ -765,7 +778,7 @@ void fwd_kernel(const KParams p) {
     }
 #pragma unroll
     for (int it = 0; it < (kOneVoff ? 1 : T::V_PER_T); ++it) {
-      const int id = it * NT + tid, row = id / LV::CPR, pc = id % LV::CPR;
+      const int id = it * T::NTV + tid_v, row = id / LV::CPR, pc = id % LV::CPR;
       voff[it] = (unsigned)(row * (int)p.vs[2] + LV::swz_v(row, pc) * 8) * 2u;
     }
     const uint32_t k_step_bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)(K_ROWS_PER_T * (uint32_t)p.ks[2] * 2u));
@@ -810,15 +823,15 @@ void fwd_kernel(const KParams p) {
       if (t * BN + BN <= p.Lk) {
 #pragma unroll
         for (int it = 0; it < T::V_PER_T; ++it) {
-          if constexpr (kOneVoff) dma16(base + (uint64_t)((uint32_t)it * v_step_bytes), voff[0], lds_v + slot * T::VBYTES + it * NT * 16);
-          else dma16(base, voff[it], lds_v + slot * T::VBYTES + it * NT * 16);
+          if constexpr (kOneVoff) dma16(base + (uint64_t)((uint32_t)it * v_step_bytes), voff[0], lds_v + slot * T::VBYTES + it * T::NTV * 16);
+          else dma16(base, voff[it], lds_v + slot * T::VBYTES + it * T::NTV * 16);
         }
       } else {
 #pragma unroll
         for (int it = 0; it < T::V_PER_T; ++it) {
-          const int id = it * NT + tid, row = id / LV::CPR, pc = id % LV::CPR;
+          const int id = it * T::NTV + tid_v, row = id / LV::CPR, pc = id % LV::CPR;
           const unsigned off = (unsigned)(min(row, p.Lk - 1 - t * BN) * (int)p.vs[2] + LV::swz_v(row, pc) * 8) * 2u;
-          dma16(base, off, lds_v + slot * T::VBYTES + it * NT * 16);
+          dma16(base, off, lds_v + slot * T::VBYTES + it * T::NTV * 16);
         }
       }
     };
@@ -1122,7 +1135,7 @@ void fwd_kernel(const KParams p) {
     // ---- A operand of O^T += V^T . P^T for 16-key chunk c and value block dvb, through the transposing LDS read.
     // Slot j of lane (r, h) is key 16c + 8*(j/4) + 4h + j%4, the key order of the packed weights.
     auto v_frag = [&](int buf, int c, int dvb) FL_INLINE -> ex8 {
-      const unsigned char* vb_ = smem + T::V_OFF + buf * T::VBYTES;
+      const unsigned char* vb_ = smem_v + buf * T::VBYTES;
       ex8 vf;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
@@ -1399,9 +1412,9 @@ void fwd_kernel(const KParams p) {
     }
     if constexpr (kDoc) dma_wait<0>();  // the tile list (issued first thing) has landed
     // (the previous branch is done with the LDS buffers; every wave's share of the tile list is visible to all)
-    if (br > 0 || kDoc) __syncthreads();
+    if (turn > 0 || kDoc) __syncthreads();
     if constexpr (kDoc) n_list = __builtin_amdgcn_readfirstlane((int)tlist[-1]);
-    if constexpr (KG > 1 && kDoc) take_part();
+    if constexpr (kSplit && kDoc) take_part();
     // whether the weights of a tile-list entry's tile are formed without looking at its row maxima first
     auto reference_free = [&](uint32_t e) FL_INLINE { return kFastRef && (kLazyMasked || entry_class(e) == TILE_FULL); };
     // Head of a step, vector work only: element mask of the current tile if it is not FULL for this wave, its row
@@ -1428,7 +1441,7 @@ void fwd_kernel(const KParams p) {
     // below are unrolled over the two ring slots and entered at slot 0): an EMPTY tile ahead of it is taken into the run
     // and computed and masked like any other.
     auto live_run = [&](int& a_live, int& b_live) FL_INLINE {
-      const int n = KG > 1 ? n_own : n_list;
+      const int n = kSplit ? n_own : n_list;
       a_live = 0;
       b_live = n;
       if constexpr (kDoc) {
@@ -1515,7 +1528,7 @@ void fwd_kernel(const KParams p) {
         // K slot `slot` held this tile's K and V slot `slot - 1` the previous tile's V: both were last read before the
         // barrier that ended the previous step
         const bool steady = issue_loads(slot);
-        settle(sc, ent[0], slot, KG > 1 && pos == a_live);
+        settle(sc, ent[0], slot, kSplit && pos == a_live);
         ex8 pf[QB][2 * KB];
         // Raised issue priority while this wave has matrix work: of the two waves sharing a SIMD, the one that is in
         // its MFMA phase wins the issue port, which drives the pair into opposite phases (one on the matrix pipe while
@@ -1570,10 +1583,10 @@ void fwd_kernel(const KParams p) {
         ex8 pf[QB][2 * KB];
         ex8 vfirst[DVB];
         if constexpr (slot % 2 == 0) {
-          settle(s_a, ent[0], slot, KG > 1 && pos == a_live);
+          settle(s_a, ent[0], slot, kSplit && pos == a_live);
           weights_checked(s_a, pf, reference_free(ent[0]), std::false_type{}, vfirst, slot, entry_tile(ent[0]), std::false_type{});
         } else {
-          settle(s_b, ent[0], slot, KG > 1 && pos == a_live);
+          settle(s_b, ent[0], slot, kSplit && pos == a_live);
           weights_checked(s_b, pf, reference_free(ent[0]), std::false_type{}, vfirst, slot, entry_tile(ent[0]), std::false_type{});
         }
         pv_mma(pf, slot, vfirst, std::false_type{});
@@ -1589,7 +1602,7 @@ void fwd_kernel(const KParams p) {
     }
 
     // ---- the groups' sums, each relative to the reference its group ended with, are added up by the first group --------------
-    if constexpr (KG > 1) {
+    if constexpr (kSplit) {
       constexpr int W = QB * (16 * DVB + 2);  // floats per lane
       float* const sums = reinterpret_cast<float*>(smem_all) + wave * (W * 64) + 4 * lane;
       constexpr int kGroup = NW * W * 64;
@@ -1659,18 +1672,14 @@ void fwd_kernel(const KParams p) {
           p.lse[((int64_t)batch * p.Hq + head) * p.Lq + qrow[qb]] = l > 0.f ? mc + __builtin_log2f(l) : INFINITY;
         }
       }
-      if constexpr (kDiff) {
-        if (br == 0) {
+      if constexpr (kSequential) {
 #pragma unroll
-          for (int dvb = 0; dvb < DVB; ++dvb)
+        for (int dvb = 0; dvb < DVB; ++dvb)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) ofin[dvb][qb][i] = oacc[dvb][qb][i] * inv;
-        } else {
-#pragma unroll
-          for (int dvb = 0; dvb < DVB; ++dvb)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) oacc[dvb][qb][i] = ofin[dvb][qb][i] - p.lambda * (oacc[dvb][qb][i] * inv);
-        }
+          for (int i = 0; i < 16; ++i) {
+            const float x = oacc[dvb][qb][i] * inv;
+            if (turn == 0) ofin[dvb][qb][i] = x; else oacc[dvb][qb][i] = ofin[dvb][qb][i] - p.lambda * x;
+          }
       } else {
 #pragma unroll
         for (int dvb = 0; dvb < DVB; ++dvb)
@@ -1678,6 +1687,39 @@ void fwd_kernel(const KParams p) {
           for (int i = 0; i < 16; ++i) oacc[dvb][qb][i] *= inv;
       }
     }
+  }
+
+  // ---- differential attention: the branches trade halves of their columns through LDS, and each finishes and stores one half --------
+  auto mine = [&](int dvb) FL_INLINE { return !kBranches || dvb / (DVB / 2 > 0 ? DVB / 2 : 1) == group; };
+  if constexpr (kBranches) {
+    float* const halves = reinterpret_cast<float*>(smem_all) + wave * (QB * DVB * 1024) + 4 * lane;
+    __syncthreads();  // (every wave is done with the tiles)
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int dvb = 0; dvb < DVB; ++dvb)
+        if (!mine(dvb)) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<f32x4*>(halves + ((qb * DVB + dvb) * 4 + g) * 256) =
+                f32x4{oacc[dvb][qb][4 * g], oacc[dvb][qb][4 * g + 1], oacc[dvb][qb][4 * g + 2], oacc[dvb][qb][4 * g + 3]};
+        }
+    __syncthreads();
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int dvb = 0; dvb < DVB; ++dvb)
+        if (mine(dvb)) {
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(halves + ((qb * DVB + dvb) * 4 + g) * 256);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float own = oacc[dvb][qb][4 * g + e];
+              oacc[dvb][qb][4 * g + e] = group == 0 ? own - p.lambda * x[e] : x[e] - p.lambda * own;
+            }
+          }
+        }
   }
 
   // ---- epilogue: O^T register i of block (dvb, qb) is out[q = qrow[qb]][dv = 32*dvb + 8*(i/4) + 4h + i%4] ----------
@@ -1717,6 +1759,7 @@ void fwd_kernel(const KParams p) {
     if (!wide && qrow[qb] >= p.Lq) continue;
 #pragma unroll
     for (int dvb = 0; dvb < DVB; ++dvb) {
+      if (!mine(dvb)) continue;
       ex4 quad[4];
 #pragma unroll
       for (int g = 0; g < 4; ++g) {

@@ -14,6 +14,7 @@ struct Instance {
   uint32_t feat;
   int lds_fixed_bytes;  // LDS without the tile list (4 more bytes per key tile)
   int max_groups;  // groups of nw waves a workgroup can be launched with (1, 2 or 4), each with lds_fixed_bytes
+  int branches_lds_bytes;  // differential attention: LDS with a group of waves per softmax branch
   hipError_t (*launch)(const KParams&, int groups, int grid, int lds_bytes, hipStream_t);
 };
 
@@ -32,22 +33,41 @@ hipError_t launch_fwd(const KParams& kp, int grid, int lds_bytes, hipStream_t st
   return hipGetLastError();
 }
 
+template <int DQK, int DV, int RW, int BN, int NW, uint32_t FEAT, int NS>
+constexpr int branches_lds_bytes() {
+  if constexpr ((FEAT & F_DIFF) != 0) return FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, bf16_t, 2>::LDS_FIXED_BYTES;
+  return 0;
+}
+
 // Groups of waves the shape can be launched with (plan_few in api.hip): every instance compiled for them is that many kernels, so
 // only the default tiles have them.  Eight waves are two per SIMD, all the registers hold (four groups of four spill).
 constexpr int max_groups(int dqk, int dv, int rw, int bn, int nw, int ns, uint32_t feat) {
+  if (feat & F_DIFF) return feat & F_DUMP ? 1 : 2;
   if (dqk != dv || (dqk != 64 && dqk != 128) || rw != 32 || ns != 2 || (feat & ~(F_ALIBI | F_SOFTCAP | F_DOC))) return 1;
   if (nw == 2) return dqk == 64 ? 4 : 2;
   return nw == 4 && bn == (dqk == 128 && (feat & F_DOC) ? 32 : 64) ? 2 : 1;
 }
 
+// Differential attention with the branches one after the other: 32-key tiles (both results and two tiles of 64 keys have no room in the
+// registers), 128 rows; the dump of attended pairs has no other form.
+constexpr bool diff_sequential(int bn, int nw) { return bn == 32 && nw == 4; }
+
 template <int DQK, int DV, int RW, int BN, int NW, int NS, uint32_t FEAT, class E>
 hipError_t launch_fwd_groups(const KParams& kp, int groups, int grid, int lds_bytes, hipStream_t stream) {
+  if constexpr ((FEAT & F_DIFF) != 0) {
+    if constexpr (!(FEAT & F_DUMP))
+      if (groups == 2) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E, 2>>(kp, grid, lds_bytes, stream);
+    if constexpr (diff_sequential(BN, NW))
+      if (groups == 1) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E>>(kp, grid, lds_bytes, stream);
+    return hipErrorInvalidValue;
+  } else {
   constexpr int MAX = max_groups(DQK, DV, RW, BN, NW, NS, FEAT);
   if constexpr (MAX >= 4)
     if (groups == 4) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E, 4>>(kp, grid, lds_bytes, stream);
   if constexpr (MAX >= 2)
     if (groups == 2) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E, 2>>(kp, grid, lds_bytes, stream);
   return groups == 1 ? launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E>>(kp, grid, lds_bytes, stream) : hipErrorInvalidValue;
+  }
 }
 
 }  // namespace fl
@@ -67,6 +87,6 @@ hipError_t launch_fwd_groups(const KParams& kp, int groups, int grid, int lds_by
 #define FL_INSTANCE_DEF(NAME, SFX, ELEM, ...) FL_INSTANCE_DEF_(NAME, SFX, ELEM, __VA_ARGS__)
 #define FL_INSTANCE_ROW_(NAME, SFX, DT, DQK, DV, RW, BN, NW, NS, FEAT) \
   {#NAME, DT, DQK, DV, RW, BN, NW, NS, (FEAT), fl::FwdTraits<DQK, DV, RW, BN, NW, (FEAT), NS>::LDS_FIXED_BYTES, \
-   fl::max_groups(DQK, DV, RW, BN, NW, NS, (FEAT)), &fl::launch_##NAME##SFX},
+   fl::max_groups(DQK, DV, RW, BN, NW, NS, (FEAT)), fl::branches_lds_bytes<DQK, DV, RW, BN, NW, (FEAT), NS>(), &fl::launch_##NAME##SFX},
 #define FL_INSTANCE_ROW(NAME, ...) \
   FL_INSTANCE_ROW_(NAME, _bf16, 0, __VA_ARGS__) FL_INSTANCE_ROW_(NAME, _f16, 2, __VA_ARGS__)

@@ -209,7 +209,7 @@ int fl_attn_fwd_ungated(const fl_attn_params* p, void* ungated, void* stream);
  * dim 32, one dense bias shared by several batch entries, 256 / 320 / 384 keys: the Evoformer shape), 2 when it goes to the
  * shared-bias stripe kernel (such a bias at other lengths, in fp32 or with row statistics; out[1]=keys it covers).
  * out[7]=groups of waves per workgroup that share its rows and take a part of the key tiles each (calls of few workgroups;
- * out[2] and out[4] are one group's). */
+ * out[2] and out[4] are one group's) or, in differential attention, a softmax branch each (out[2] is one group's). */
 int fl_attn_plan(const fl_attn_params* p, int64_t out[8]);
 
 /* Backward of fl_attn_fwd.  No counterpart in the reference, which is forward-only (its FLOP helper models a
