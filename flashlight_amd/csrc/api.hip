@@ -1466,9 +1466,10 @@ static int launch_gradients(const fl_attn_bwd_params* b, bool planned, void* scr
     bp.role[r].by_splits = fl::Div::by(r ? plan.dkv : plan.dq);
     bp.role[r].by_tiles = fl::Div::by(tiles);
   }
-  hipError_t e = in->launch_delta(bp, stream);
-  if (e != hipSuccess) return fail((int)e, "backward: launch of the row-sum kernel failed: %s", hipGetErrorString(e));
+  hipError_t e;
   if (plan.both) {
+    e = in->launch_delta(bp, stream);
+    if (e != hipSuccess) return fail((int)e, "backward: launch of the row-sum kernel failed: %s", hipGetErrorString(e));
     e = in->launch_both(bp, stream);
     if (e != hipSuccess) return fail((int)e, "backward: launch of the gradient kernel failed: %s", hipGetErrorString(e));
     return 0;

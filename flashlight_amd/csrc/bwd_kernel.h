@@ -72,8 +72,24 @@ struct BParams {
   } role[2];
 };
 
+// dot product of eight 16-bit pairs, the same bits wherever it stands (left to itself the compiler forms two-element dot products of fp16
+// in one kernel and not in the other)
+template <class E8>
+__device__ __forceinline__ float dot8(const E8& a, const E8& b) {
+  float s = 0.f;
+  if constexpr (std::is_same<E8, f16x8>::value) {
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) s = dot2acc(f16x2{a[e], a[e + 1]}, f16x2{b[e], b[e + 1]}, s);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = __builtin_fmaf((float)a[e], (float)b[e], s);
+  }
+  return s;
+}
+
 // delta[b, h, q] = -sum_d dO[b, h, q, d] * O[b, h, q, d]; one row per group of DV / 8 lanes, delta_blocks workgroups per (batch, head):
-// bound by reading both (6.4 TB/s at 4 x 16 x 4096, head dim 128).
+// bound by reading both (6.4 TB/s at 4 x 16 x 4096, head dim 128).  For calls whose two roles share a launch; with a launch each, dQ's
+// workgroups, which hold dO's rows in any case, form the sums (row_sum in bwd_tile, the same bits).
 template <int DV, class E>
 __global__ __launch_bounds__(256) void bwd_delta_kernel(const BParams p) {
   fetch_params<BParams>();
@@ -85,8 +101,7 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const BParams p) {
   if (q < p.Lq) {
     const ex8 a = *reinterpret_cast<const ex8*>(p.dout + b * p.dos[0] + h * p.dos[1] + q * p.dos[2] + 8 * c);
     const ex8 o = *reinterpret_cast<const ex8*>(p.o + b * p.os[0] + h * p.os[1] + q * p.os[2] + 8 * c);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s += (float)a[e] * (float)o[e];
+    s = dot8(a, o);
   }
 #pragma unroll
   for (int d = 1; d < LPR; d *= 2) s += __shfl_xor(s, d);
@@ -98,6 +113,7 @@ template <int D_, int ROLE_, uint32_t FEAT_, class Elem_ = bf16_t, bool SHARED_ 
 struct BwdTraits {
   using Elem = Elem_;  // element type of q, k, v, o, dout and the gradients: bf16_t or f16_t
   static constexpr int D = D_, ROLE = ROLE_;
+  static constexpr bool SHARED = SHARED_;
   static constexpr uint32_t FEAT = FEAT_;
   static constexpr int OWN = 128;                          // owner positions per workgroup: 4 waves x 32
   // ROLE_DKV at D = 128 holds 128 accumulator registers per lane; to still run two waves per SIMD its workgroup has
@@ -293,7 +309,24 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     const int64_t row = ((int64_t)batch * p.Hq + ohead) * p.Lq + qr;
     lse_o = p.lse[row];
-    delta_o = p.delta[row];
+    if constexpr (T::SHARED) {
+      delta_o = p.delta[row];
+    } else {
+      // minus rowsum(dO o O), in the order of bwd_delta_kernel, left for the dK/dV launch that follows
+      const bf16_t* op = p.o + (int64_t)batch * p.os[0] + (int64_t)ohead * p.os[1] + (int64_t)qr * p.os[2];
+      float sum[KS];
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const ex8 o = *reinterpret_cast<const ex8*>(op + ks * 16 + 8 * h);
+        sum[ks] = xhalf_sum(dot8(o2f[ks], o));
+      }
+#pragma unroll
+      for (int d = 1; d < KS; d *= 2)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks += 2 * d) sum[ks] += sum[ks + d];
+      delta_o = -sum[0];
+      if (h == 0 && opos < p.Lq) p.delta[row] = delta_o;
+    }
   }
 
   // ---- global -> LDS transfers of a [rows][D] tile into its swizzled image ---------------------------------------------------
