@@ -108,88 +108,81 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const BParams p) {
   if (q < p.Lq && c == 0) p.delta[(int64_t)bh * p.Lq + q] = -s;  // stored negated: the consumers add it (or start dP's accumulators from it)
 }
 
-// SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size
+// LDS image of a [rows][D] tile that is read both ways: blocks of 16 rows x 64 bytes (1 KiB, a wave's transfer), block after block
+// along the row, then down the rows; a row's four 16-byte chunks are exchanged by XOR with row / 4 % 4.  Row-wise reads (16 rows at one
+// chunk) and transposing ones (4 rows x 64 bytes) touch every bank once, as with rows kept whole and swizzled over their 16 chunks, but the
+// chunk index reaches only two bits into the swizzle: all reads of a kind are at two addresses plus constants (six registers instead of 24 at
+// head dim 128).
+template <int D>
+struct QuadLayout {
+  static constexpr int BPR = D / 32;  // blocks along a row
+  // byte of 16-byte chunk `chunk` of row `row`
+  __host__ __device__ static constexpr unsigned at(int row, int chunk) {
+    return (unsigned)((row / 16 * BPR + chunk / 4) * 1024 + row % 16 * 64 + ((chunk % 4) ^ (row / 4 % 4)) * 16);
+  }
+  // the row and the chunk that 16-byte piece `id` of the image holds
+  __host__ __device__ static constexpr int row_of(int id) { return id / 64 / BPR * 16 + id % 64 / 4; }
+  __host__ __device__ static constexpr int chunk_of(int id) { return id / 64 % BPR * 4 + ((id % 4) ^ (id % 64 / 16)); }
+};
+static_assert([]() constexpr {
+  for (int id = 0; id < 1024; ++id)
+    if (QuadLayout<128>::at(QuadLayout<128>::row_of(id), QuadLayout<128>::chunk_of(id)) != 16u * id || QuadLayout<64>::at(QuadLayout<64>::row_of(id), QuadLayout<64>::chunk_of(id)) != 16u * id ||
+        QuadLayout<32>::at(QuadLayout<32>::row_of(id), QuadLayout<32>::chunk_of(id)) != 16u * id) return false;
+  return true;
+}(), "one place per chunk");
+
+// SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size.
 template <int D_, int ROLE_, uint32_t FEAT_, class Elem_ = bf16_t, bool SHARED_ = false>
 struct BwdTraits {
   using Elem = Elem_;  // element type of q, k, v, o, dout and the gradients: bf16_t or f16_t
   static constexpr int D = D_, ROLE = ROLE_;
   static constexpr bool SHARED = SHARED_;
   static constexpr uint32_t FEAT = FEAT_;
-  static constexpr int OWN = 128;                          // owner positions per workgroup: 4 waves x 32
+  static constexpr int OWN = 128;                          // owner positions per workgroup
+  static constexpr int OB = OWN / 32;                      // blocks of 32 of them, a wave each (two with QH == 2)
   // ROLE_DKV at D = 128 holds 128 accumulator registers per lane; to still run two waves per SIMD its workgroup has
   // 8 waves, two per owner block, which take the two halves of every streamed tile and add up their partial sums
   // through LDS at the end (one workgroup per CU, 128 KB of LDS).
   static constexpr int QH = ((ROLE == ROLE_DKV || SHARED_) && D_ > 64) ? 2 : 1;   // waves per owner block
-  static constexpr int NW = 4 * QH, NT = 64 * NW;
+  static constexpr int NW = OB * QH, NT = 64 * NW;
   static constexpr int TB = (D_ <= 64) ? 2 : 1;  // 32-position blocks per wave and step (register budget)
   static constexpr int BT = 32 * TB * QH;                  // streamed positions per step
   static constexpr int KS = D / 16, DB = D / 32;
   static constexpr int TBYTES = BT * D * 2;                // one streamed tile
   static constexpr int T_PER_T = TBYTES / (NT * 16);       // 16-byte transfers per thread per tile
   static_assert(TBYTES % (NT * 16) == 0, "streamed tile must divide evenly over the threads");
+  // The order of a step's LDS reads, products and vector work is written out (run_ordered).  Left to the compiler, also with
+  // sched_group_barrier, most products stood right behind the wait for their own LDS read, and exponentials in a row.  us, gradients, the
+  // compiler's order -> this: head dim 64, 4 x 16 x 4096 causal 502 -> 477, 3 x 16 over 4 of 1000 with a prefix 65.2 -> 58.9, 32 over 10 x 8 of 1139
+  // 431 -> 393, documents of 32 over 2 x 8 x 8037 1023 -> 1004, ALiBi and soft-cap 239 -> 230; head dim 128, 4 x 16 x 4096 causal 935 -> 922,
+  // documents, 16 over 4 x 4 of 3000, 273 -> 252, ALiBi and soft-cap, 32 over 2 x 4 of 2000, 366 -> 355.  How far the reads run ahead hardly
+  // matters (2 to 5 products); documents with ALiBi and a soft-cap spill.
+  static constexpr bool ORDERED = ((FEAT_ & ~F_DOC) == 0 || (FEAT_ & ~(F_ALIBI | F_SOFTCAP)) == 0) && D_ >= 64;
+  static constexpr int AHEAD = 3;
+  // ROLE_DKV: the owner's K and V rows as operands in registers, where there is room, instead of in LDS
+  static constexpr bool K_REGS = ROLE == ROLE_DKV && ORDERED && D <= 64, V_REGS = ROLE == ROLE_DQ || K_REGS;
   static constexpr int OBYTES = (ROLE == ROLE_DKV) ? OWN * D * 2 : 0;  // owner tile kept in LDS (ROLE_DKV: K and V)
   static constexpr int O_PER_T = OBYTES / (NT * 16);
   static_assert(OBYTES % (NT * 16) == 0, "owner tile must divide evenly over the threads");
   // ROLE_DKV also stages the streamed rows' statistics (LSE and Delta, fp32) with every tile: 1 KiB each per slot
   static constexpr int SBYTES = (ROLE == ROLE_DKV) ? 1024 : 0;
-  static constexpr int T1_OFF = 0, T2_OFF = 2 * TBYTES, O1_OFF = 4 * TBYTES, O2_OFF = O1_OFF + OBYTES,
-                       S1_OFF = O2_OFF + OBYTES, S2_OFF = S1_OFF + 2 * SBYTES;
+  static constexpr int T1_OFF = 0, T2_OFF = 2 * TBYTES, O1_OFF = 4 * TBYTES, O2_OFF = O1_OFF + (K_REGS ? 0 : OBYTES),
+                       S1_OFF = O2_OFF + (V_REGS ? 0 : OBYTES), S2_OFF = S1_OFF + 2 * SBYTES;
   // Document masks: the list of live tiles (up to LIST of them at a time, with one count per wave behind it) and, per slot, the ids
   // of the streamed positions
   static constexpr bool DOC = FEAT_ & F_DOC;
   static constexpr int LIST = 1024, LIST_OFF = S2_OFF + 2 * SBYTES, IDS_OFF = LIST_OFF + (DOC ? LIST * 4 + 64 : 0);
   static constexpr int LDS_BYTES = IDS_OFF + (DOC ? 2 * BT * 8 : 0);
   static_assert(QH == 1 || LDS_BYTES >= 4 * 64 * 64 * 4, "the partial sums of one accumulator set must fit in LDS");
-  // Calls without score modifications: the LDS addresses of the operand reads stay in registers (24 at head dim 128; worked out
-  // where they are used they were a third of the vector instructions), and the order of reads, products and vector work is
-  // prescribed (sched_scores, sched_gradients).  4 x 16 x 4096, unmasked / causal, us: head dim 128, dQ 744 / 398 -> 695 / 380, dK and
-  // dV 1187 / 644 -> 1095 / 630; head dim 64, dQ 435 / 235 -> 385 / 204; dK and dV there are the slower for it (581 / 311 -> 626 / 332:
-  // two blocks per step leave less room).
-  static constexpr bool TUNED = (FEAT_ == 0 && D_ > 64) || ((FEAT_ & ~F_DOC) == 0 && D_ == 64 && ROLE_ == ROLE_DQ);
   // ROLE_DQ: dP's accumulators start from a tile of -Delta that stays in registers, where there is room for it
-  static constexpr bool DELTA_TILE = ROLE_ == ROLE_DQ && (TUNED || (D_ <= 64 && !(FEAT_ & (F_BIAS | F_DROPOUT))));
+  static constexpr bool DELTA_TILE = ROLE_ == ROLE_DQ && (ORDERED || (D_ <= 64 && !(FEAT_ & (F_BIAS | F_DROPOUT))));
   // two steps per turn of the loop, see there (without addresses in registers the dK/dV kernel is 1 to 4 % slower with it; bias
   // operands have no registers for it)
-  static constexpr bool UNROLL2 = (ROLE == ROLE_DQ || TUNED) && !(FEAT_ & F_BIAS);
+  static constexpr bool UNROLL2 = (ROLE == ROLE_DQ || ORDERED) && !(FEAT_ & F_BIAS);
   static constexpr int WAVES_PER_EU = 2;
   static constexpr bool WIDE_X2 = D_ > 64;                      // dP's fp32 tile declared next to S's
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
 };
-
-// The order of a step's instructions (T::TUNED): N times M products, each followed by R LDS reads and V vector instructions.
-template <int N, int M, int R, int V>
-__device__ __forceinline__ void sched_run() {
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    __builtin_amdgcn_sched_group_barrier(SG_MFMA, M, 0);
-    if constexpr (R > 0) __builtin_amdgcn_sched_group_barrier(SG_DS_READ, R, 0);
-    if constexpr (V > 0) __builtin_amdgcn_sched_group_barrier(SG_VALU | SG_TRANS, V, 0);
-  }
-}
-// X1's products, their operands read two k-steps ahead (left to itself the compiler waits for the two reads in front of every one)
-template <int KS, int TB, bool DQ>
-__device__ __forceinline__ void sched_scores() {
-  constexpr int R = TB + (DQ ? 0 : 1), A = 2;
-  __builtin_amdgcn_sched_group_barrier(SG_DS_READ, A * R, 0);
-  sched_run<KS - A, TB, R, 0>();
-  sched_run<A, TB, 0, 0>();
-}
-// X2's products with the weights' vector work under them, then (ROLE_DKV) dV's with dS's, then those of dS
-template <int KS, int TB, int DB, bool DQ>
-__device__ __forceinline__ void sched_gradients() {
-  constexpr int R = TB + (DQ ? 0 : 1), A = 2, NA = 2 * TB * DB, PA = 2;
-  __builtin_amdgcn_sched_group_barrier(SG_DS_READ, (DQ ? 0 : 8 * TB) + A * R, 0);
-  sched_run<KS - A, TB, R, 32 * TB / KS>();
-  sched_run<A, TB, 2 * PA / A, 32 * TB / KS>();
-  if constexpr (DQ) {
-    __builtin_amdgcn_sched_group_barrier(SG_VALU, 24 * TB, 0);
-  } else {
-    __builtin_amdgcn_sched_group_barrier(SG_VALU, 8 * TB, 0);
-    sched_run<NA, 1, 2, 12 / DB>();
-  }
-  sched_run<NA - PA, 1, 2, 0>();
-  sched_run<PA, 1, 0, 0>();
-}
 
 // One workgroup's share of the work of a role: workgroup `block` of tiles * splits.  SPLIT: several workgroups per owner tile
 // (one at run time is fine), compiled apart: with the second epilogue in it the dK/dV kernel at head dim 128 is 4 %
@@ -205,15 +198,14 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   typedef E ex4 __attribute__((ext_vector_type(4)));
   constexpr bool kDrop = FEAT & F_DROPOUT;
   constexpr float kLog2e = 1.4426950408889634f;
-  using L = TileLayout<D>;
-  using Ops = TileOperands<D, E>;
+  using L = QuadLayout<D>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
   const int r = lane % 32, h = lane / 32;
-  const int ow = wave % 4;       // owner block of this wave
-  const int qh = wave / 4;       // which part of every streamed tile this wave takes (0 unless QH == 2)
+  const int ow = wave % T::OB;   // owner block of this wave
+  const int qh = wave / T::OB;   // which part of every streamed tile this wave takes (0 unless QH == 2)
 
   // workgroup -> (batch, owner head, owner tile).  All owner tiles of one head stream the same tensors, so they should
   // run at the same time on one XCD (its L2 then serves all but the first read): consecutive workgroup ids land on
@@ -294,7 +286,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // ---- owner operands ---------------------------------------------------------------------------------------------------
   // ROLE_DQ: Q and dO fragments of this lane's query row live in registers (B operands), with its LSE and Delta.
   // ROLE_DKV: the workgroup's K and V rows are staged in LDS once and read as B operands where they are used.
-  ex8 o1f[kDQ ? KS : 1], o2f[kDQ ? KS : 1];
+  ex8 o1f[kDQ || T::K_REGS ? KS : 1], o2f[T::V_REGS ? KS : 1];
   float lse_o = 0.f, delta_o = 0.f;  // delta_o: minus this row's rowsum(dO o O)
   const bf16_t* kptr = p.k + (int64_t)batch * p.ks[0] + (int64_t)kvh * p.ks[1];
   const bf16_t* vptr = p.v + (int64_t)batch * p.vs[0] + (int64_t)kvh * p.vs[1];
@@ -329,14 +321,25 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
   }
 
-  // ---- global -> LDS transfers of a [rows][D] tile into its swizzled image ---------------------------------------------------
-  // lane l of a 1 KiB transfer writes LDS bytes [16 l, 16 l + 16); it fetches the logical chunk that the swizzle maps
-  // there.  Rows past `valid` repeat the last valid row (their contributions are masked).
+  if constexpr (T::K_REGS) {
+    const bf16_t* kp = kptr + (int64_t)min(opos, p.Lk - 1) * p.ks[2];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) o1f[ks] = *reinterpret_cast<const ex8*>(kp + ks * 16 + 8 * h);
+  }
+  if constexpr (!kDQ && T::V_REGS) {
+    const bf16_t* vp = vptr + (int64_t)min(opos, p.Lk - 1) * p.vs[2];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) o2f[ks] = *reinterpret_cast<const ex8*>(vp + ks * 16 + 8 * h);
+  }
+
+  // ---- global -> LDS transfers of a [rows][D] tile into its image (QuadLayout) -------------------------------------------------------
+  // lane l of a 1 KiB transfer writes LDS bytes [16 l, 16 l + 16); it fetches the chunk that the layout has there.  Rows past `valid` repeat
+  // the last valid row (their contributions are masked).
   auto load_tile = [&](uint64_t base, int64_t stride, int valid, unsigned lds_off, int n_per_t) FL_INLINE {
     const unsigned lds0 = (unsigned)(uintptr_t)smem + lds_off + wave * 1024;
     for (int it = 0; it < n_per_t; ++it) {
-      const int id = it * NT + tid, row = id / L::CPR, pc = id % L::CPR;
-      const unsigned off = (unsigned)(min(row, valid - 1) * (int)stride + L::swz_kv(row, pc) * 8) * 2u;
+      const int id = it * NT + tid;
+      const unsigned off = (unsigned)(min(L::row_of(id), valid - 1) * (int)stride + L::chunk_of(id) * 8) * 2u;
       dma16(base, off, lds0 + it * NT * 16);
     }
   };
@@ -347,8 +350,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // 668; 16 over 3 x 4 of 1000 with a prefix 86.8 -> 84.9; 32 over 7 x 8 of 306, head dim 128, 104.9 -> 100.8.)  ROLE_DKV: the statistics of the streamed rows (LSE, Delta) ride the tile transfers into LDS, 4 bytes
   // per lane, so that the loop holds no ordinary global load: the wait such a load needs would also wait for the tile transfers that are
   // in flight for the next step.
-  constexpr int ROWS_PER_T = NT / L::CPR;
-  static_assert(NT % L::CPR == 0 && ROWS_PER_T % (L::RPW * (L::CPR >= 16 ? 16 : L::CPR >= 8 ? 8 : 4)) == 0, "one offset for all transfers of a thread");
+  constexpr int ROWS_PER_T = NT / (D / 8);
+  static_assert(NT % (D / 8) == 0 && ROWS_PER_T % 16 == 0, "one offset for all transfers of a thread");
   struct Operand {
     uint64_t base;       // of the batch entry's (or, ROLE_DQ, of the head's) first row
     int64_t head_bytes;  // ROLE_DKV: from one query head to the next
@@ -358,7 +361,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   auto operand = [&](const bf16_t* ptr, const int64_t (&st)[3]) FL_INLINE -> Operand {
     const uint32_t row_bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)st[2] * 2u));
     return {uniform_ptr(ptr), uniform_i64(st[1] * 2), row_bytes * BT, row_bytes,
-            (unsigned)(tid / L::CPR) * row_bytes + L::swz_kv(tid / L::CPR, tid % L::CPR) * 16u};
+            (unsigned)L::row_of(tid) * row_bytes + L::chunk_of(tid) * 16u};
   };
   const Operand s1 = operand(kDQ ? kptr : p.q + (int64_t)batch * p.qs[0], kDQ ? p.ks : p.qs);
   const Operand s2 = operand(kDQ ? vptr : p.dout + (int64_t)batch * p.dos[0], kDQ ? p.vs : p.dos);
@@ -407,49 +410,40 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   };
 
   // ---- LDS operand reads --------------------------------------------------------------------------------------------------
-  // The addresses of the k-steps (and of the column blocks) differ in swizzled bits, those of tiles, slots and blocks of rows by
-  // constants.  TUNED: held in registers (the empty asm keeps the compiler from working them out again at every read).
-  constexpr int RB = D * 2;  // bytes per row
-  unsigned a_row[KS], a_own[KS], a_tr[2][DB];
-  if constexpr (T::TUNED) {
+  // Two addresses per kind of read, held in registers (the empty asm keeps the compiler from working them out again at every read);
+  // everything else is a constant of the instruction.
+  unsigned a_row[2], a_own[2], a_tr[2];
+  {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
+    const int i16 = lane % 16;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      a_row[ks] = lds0 + (qh * TB * 32 + r) * RB + L::swz_kv(r, 2 * ks + h) * 16;
-      asm volatile("" : "+v"(a_row[ks]));
+    for (int j = 0; j < 2; ++j) {
+      a_row[j] = lds0 + L::at(qh * TB * 32 + r, 2 * j + h);
+      asm volatile("" : "+v"(a_row[j]));
       if constexpr (!kDQ) {
-        a_own[ks] = lds0 + T::O1_OFF + (ow * 32 + r) * RB + L::swz_kv(r, 2 * ks + h) * 16;
-        asm volatile("" : "+v"(a_own[ks]));
+        a_own[j] = lds0 + T::O1_OFF + L::at(ow * 32 + r, 2 * j + h);
+        asm volatile("" : "+v"(a_own[j]));
       }
+      a_tr[j] = lds0 + L::at(qh * TB * 32 + 8 * j + 4 * h + i16 / 4, (lane / 16) % 2 * 2 + i16 % 4 / 2) + i16 % 2 * 8;
+      asm volatile("" : "+v"(a_tr[j]));
     }
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const int i16 = lane % 16, row = 8 * j + 4 * h + i16 / 4, col = db * 32 + (lane / 16) % 2 * 16 + 4 * (i16 % 4);
-        a_tr[j][db] = lds0 + (qh * TB * 32 + row) * RB + L::swz_kv(row, col / 8) * 16 + (col % 8) * 2;
-        asm volatile("" : "+v"(a_tr[j][db]));
-      }
   }
   typedef __attribute__((address_space(3))) const ex8* lds_ex8_ptr;
   typedef s16x4 __attribute__((address_space(3))) * lds_s16x4_ptr;
   // row-wise: 8 consecutive elements [row][16 ks + 8 h, +8), row = 32 (qh TB + sb) + r of a streamed tile (A operand of X1/X2) or this
   // lane's row of an owner tile (B operand)
   auto frag_row = [&](unsigned tile_off, int sb, int ks) FL_INLINE -> ex8 {
-    if constexpr (T::TUNED) return *(lds_ex8_ptr)(a_row[ks] + tile_off + sb * 32 * RB);
-    return Ops::rows(smem + tile_off, (qh * TB + sb) * 32 + r, ks, h);
+    return *(lds_ex8_ptr)(a_row[ks % 2] + tile_off + L::at(32 * sb, 4 * (ks / 2)));
   };
   auto frag_own = [&](unsigned tile_off, int ks) FL_INLINE -> ex8 {
-    if constexpr (T::TUNED) return *(lds_ex8_ptr)(a_own[ks] + (tile_off - T::O1_OFF));
-    return Ops::rows(smem + tile_off, ow * 32 + r, ks, h);
+    return *(lds_ex8_ptr)(a_own[ks % 2] + (tile_off - T::O1_OFF) + L::at(0, 4 * (ks / 2)));
   };
   // transposing: A operand of the accumulating products for 16-position chunk c (of this wave's) and column block db
   auto frag_tr = [&](unsigned tile_off, int c, int db) FL_INLINE -> ex8 {
-    if constexpr (!T::TUNED) return Ops::columns(smem + tile_off, 2 * TB * qh + c, db, lane, h);
     ex8 f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j][db] + tile_off + c * 16 * RB)));
+      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j] + tile_off + L::at(16 * c, 4 * db))));
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
     }
@@ -479,8 +473,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   if (kDoc ? n_tiles > 0 : n_steps > s_first) {
     if constexpr (!kDQ) {
       const int valid = o1 - o0;
-      load_tile(uniform_ptr(kptr + (int64_t)o0 * p.ks[2]), p.ks[2], valid, T::O1_OFF, T::O_PER_T);
-      load_tile(uniform_ptr(vptr + (int64_t)o0 * p.vs[2]), p.vs[2], valid, T::O2_OFF, T::O_PER_T);
+      if constexpr (!T::K_REGS) load_tile(uniform_ptr(kptr + (int64_t)o0 * p.ks[2]), p.ks[2], valid, T::O1_OFF, T::O_PER_T);
+      if constexpr (!T::V_REGS) load_tile(uniform_ptr(vptr + (int64_t)o0 * p.vs[2]), p.vs[2], valid, T::O2_OFF, T::O_PER_T);
     }
   }
 
@@ -519,11 +513,164 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     return b;
   };
+  // element predicate as an interval of the register offset `off` (8 (i / 4) + i % 4): lo <= off <= hi
+  auto bounds = [&](int sbase, int& lo, int& hi) FL_INLINE {
+    if constexpr (kDQ) {
+      // streamed = key, owner = query: key < Lk && (dmin <= key - q <= dmax || key < pfx)
+      const int rel = sbase - opos;
+      hi = min(p.Lk - sbase - 1, max(p.dmax - rel, p.pfx - sbase - 1));
+      lo = p.dmin - rel;
+    } else {
+      // streamed = query, owner = key: q < Lq && (dmin <= key - q <= dmax || key < pfx), key = opos
+      const int rel = opos - sbase;  // key - q at off = 0; key - q = rel - off
+      hi = min(p.Lq - sbase - 1, opos < p.pfx ? (1 << 29) : rel - p.dmin);
+      lo = opos < p.pfx ? -(1 << 29) : rel - p.dmax;
+      if (opos >= p.Lk) hi = -(1 << 29);
+    }
+  };
+  auto attended = [&](int t0, int sbase, int slot, int off, int lo, int hi, bool doc_uniform) FL_INLINE -> bool {
+    bool ok = (off <= hi) & (off >= lo);
+    if constexpr (kDoc) {
+      if (!doc_uniform) ok = ok & (*reinterpret_cast<const int64_t*>(smem + T::IDS_OFF + slot * BT * 8 + (sbase - t0 + off) * 8) == odoc);
+    }
+    return ok;
+  };
   // ALiBi slope of the streamed head in log2 units, worked out where the head changes
   int slope_head = -1;
   float slope_l2 = 0.f;
+  // The blocks of 32 streamed positions of a step with their instructions in a prescribed order (T::ORDERED, see there).  Products: X1 of
+  // every block, X2 of every block, (ROLE_DKV) dV's, dS's.  In front of product m stand the LDS reads of product m + AHEAD, behind it its
+  // share of the vector work: weights(m) pairs of weights and gradients(m) pairs of score gradients are formed by then.
+  auto run_ordered = [&](auto tile, const int shead, const int slot, bool full, bool doc_uniform) FL_INLINE {  // (compiled only where it is called)
+    const int t0 = tile * BT;
+    const unsigned t1 = T::T1_OFF + slot * T::TBYTES, t2 = T::T2_OFF + slot * T::TBYTES;
+    constexpr int X2 = TB * KS, VP = 2 * X2, KP = VP + (kDQ ? 0 : 2 * TB * DB), M = KP + 2 * TB * DB;  // first of each kind, and their number
+    constexpr int AHEAD = T::AHEAD, RING = AHEAD + 1;
+    auto weights = [](int m) constexpr {
+      if (kDQ && TB == 2) return m < 5 ? 0 : m < 9 ? 2 * (m - 4) : m < 16 ? m : 16;
+      return m < KS ? 0 : m < KS + 8 * TB ? m - KS : 8 * TB;
+    };
+    auto gradients = [](int m) constexpr {
+      if (kDQ && TB == 2) return m < 13 ? 0 : m < 15 ? 3 * (m - 12) : m < 17 ? 8 : m < 20 ? 8 + 2 * (m - 16) : 16;
+      if (kDQ) return m < VP - 1 ? 0 : m < VP + 3 ? m - VP + 5 : 8;
+      if (TB == 2) return m < VP + 5 ? 0 : m < VP + 12 ? 2 * (m - VP - 4) : 16;
+      return m < VP ? 0 : m < VP + 8 ? m - VP : 8;
+    };
+    static_assert(TB == 1 ? KS == 8 && DB == 4 : KS == 4 && DB == 2, "the places of the vector work");
+    f32x16 x1[TB], x2[TB];
+    ex8 fa[RING], fb[T::V_REGS ? 1 : RING];  // operands in flight
+    f32x4 lse4[2];
+    ex8 pf[2 * TB], dsf[2 * TB];
+#pragma unroll
+    for (int sb = 0; sb < TB; ++sb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x1[sb][i] = 0.f;
+    // 4 consecutive streamed rows' values of a staged per-row fp32 array
+    auto rows4 = [&](unsigned staged_off, int sb, int g) FL_INLINE -> f32x4 {
+      return *reinterpret_cast<const f32x4*>(smem + staged_off + slot * T::SBYTES + (32 * (qh * TB + sb) + 4 * h + 8 * g) * 4);
+    };
+    auto read = [&](auto mt) FL_INLINE {
+      constexpr int m = decltype(mt)::value;
+      if constexpr (m < X2) {
+        fa[m % RING] = frag_row(t1, m / KS, m % KS);
+        if constexpr (!kDQ && !T::K_REGS) fb[m % RING] = frag_own(T::O1_OFF, m % KS);
+      } else if constexpr (m < VP) {
+        constexpr int sb = (m - X2) / KS, ks = (m - X2) % KS;
+        if constexpr (!kDQ && ks == 0) {  // dP starts from minus Delta
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x4 nd = rows4(T::S2_OFF, sb, g);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x2[sb][4 * g + e] = nd[e];
+          }
+        }
+        fa[m % RING] = frag_row(t2, sb, ks);
+        if constexpr (!kDQ && !T::V_REGS) fb[m % RING] = frag_own(T::O2_OFF, ks);
+      } else if constexpr (m < KP) {
+        fa[m % RING] = frag_tr(t2, (m - VP) / DB, (m - VP) % DB);
+      } else if constexpr (m < M) {
+        fa[m % RING] = frag_tr(t1, (m - KP) / DB, (m - KP) % DB);
+      }
+    };
+    if constexpr (kAlibi) {
+      if (shead != slope_head) {
+        slope_head = shead;
+        slope_l2 = p.alibi_heads > 0 ? exp2f(-8.0f * (float)(shead + 1) / (float)p.alibi_heads) * kLog2e : 0.f;
+      }
+    }
+    int lo[TB], hi[TB];     // the element mask's bounds, where it is asked
+    float alibi0[TB];       // the ALiBi term at register offset 0
+    static_while<0, AHEAD>([&](auto m) FL_INLINE { read(m); return true; });
+    static_while<0, M>([&](auto mt) FL_INLINE {
+      constexpr int m = decltype(mt)::value;
+      read(std::integral_constant<int, m + AHEAD>{});
+      if constexpr (!kDQ) {  // the LSE of four rows, two products ahead of their weights (the place is free: of the last but one)
+        constexpr int g = m - KS + 1;
+        if constexpr (g >= 0 && g % 2 == 0 && g / 2 < 4 * TB) lse4[g / 2 % 2] = rows4(T::S1_OFF, g / 8, g / 2 % 4);
+      }
+      if constexpr (m < X2) {
+        if constexpr (kDQ || T::K_REGS) x1[m / KS] = mfma32(fa[m % RING], o1f[m % KS], x1[m / KS]);
+        else x1[m / KS] = mfma32(fa[m % RING], fb[m % RING], x1[m / KS]);
+      } else if constexpr (m < VP) {
+        constexpr int sb = (m - X2) / KS, ks = (m - X2) % KS;
+        if constexpr (kDQ && ks == 0) x2[sb] = mfma32(fa[m % RING], o2f[0], delta_tile);
+        else if constexpr (kDQ || T::V_REGS) x2[sb] = mfma32(fa[m % RING], o2f[ks], x2[sb]);
+        else x2[sb] = mfma32(fa[m % RING], fb[m % RING], x2[sb]);
+      } else if constexpr (m < KP) {
+        acc2[(m - VP) % DB] = mfma32(fa[m % RING], pf[(m - VP) / DB], acc2[(m - VP) % DB]);
+      } else {
+        acc1[(m - KP) % DB] = mfma32(fa[m % RING], dsf[(m - KP) / DB], acc1[(m - KP) % DB]);
+      }
+#pragma unroll
+      for (int w = weights(m - 1); w < weights(m); ++w) {
+        const int sb = w / 8, sbase = t0 + 32 * (qh * TB + sb) + 4 * h;  // streamed position of register 0
+        if (w % 8 == 0) {
+          if constexpr (kAlibi) alibi0[sb] = slope_l2 * (float)(kDQ ? sbase - opos : opos - sbase);
+          if (!full) {  // uniform over the workgroup or the wave; the asm keeps it a branch
+            bounds(sbase, lo[sb], hi[sb]);
+            asm volatile("" : "+v"(lo[sb]), "+v"(hi[sb]));
+            if constexpr (!kSoftcap) {
+#pragma unroll
+              for (int i = 0; i < 16; ++i)
+                if (!attended(t0, sbase, slot, 8 * (i / 4) + i % 4, lo[sb], hi[sb], doc_uniform)) x1[sb][i] = -INFINITY;
+            }
+          }
+        }
+#pragma unroll
+        for (int e = w % 8 * 2; e < w % 8 * 2 + 2; ++e) {
+          const float x = x1[sb][e], lse = kDQ ? lse_o : lse4[w / 2 % 2][e % 4], c0 = kAlibi ? alibi0[sb] - lse : -lse;
+          const int off = 8 * (e / 4) + e % 4;
+          float s2, dfac = 1.0f;  // logit in log2 units minus the LSE; d(score) / d(qk * scale)
+          if constexpr (kSoftcap) {
+            const float th = __builtin_fmaf(fast_rcp(fast_exp2(x * cap_k1) + 1.0f), -2.0f, 1.0f);  // tanh(x * scale / cap)
+            s2 = cap_on ? __builtin_fmaf(th, cap_c, c0) : __builtin_fmaf(x, p.scale_log2, c0);
+            dfac = cap_on ? __builtin_fmaf(-th, th, 1.0f) : 1.0f;
+          } else {
+            s2 = __builtin_fmaf(x, p.scale_log2, c0);
+          }
+          if constexpr (kAlibi) s2 = __builtin_fmaf(kDQ ? slope_l2 : -slope_l2, (float)off, s2);
+          float pv = fast_exp2(s2);
+          if constexpr (kSoftcap) {  // (-inf would not do as a score)
+            if (!full) {
+              if (!attended(t0, sbase, slot, off, lo[sb], hi[sb], doc_uniform)) pv = 0.f;
+              asm volatile("" : "+v"(pv));
+            }
+          }
+          if constexpr (!kDQ) pf[2 * sb + e / 8][e % 8] = (E)pv;
+          x1[sb][e] = kSoftcap ? pv * dfac : pv;
+        }
+      }
+#pragma unroll
+      for (int w = gradients(m - 1); w < gradients(m); ++w)
+#pragma unroll
+        for (int e = w % 8 * 2; e < w % 8 * 2 + 2; ++e) dsf[w / 8 * 2 + e / 8][e % 8] = (E)(x1[w / 8][e] * x2[w / 8][e]);
+      __builtin_amdgcn_sched_barrier(0);
+      return true;
+    });
+  };
   // One step: the tile in ring slot `slot` against the owner operands.
   auto run_tile = [&](int tile, const int shead, int slot, bool full, bool doc_uniform) FL_INLINE {
+    if constexpr (T::ORDERED) return run_ordered(tile, shead, slot, full, doc_uniform);
     const int t0 = tile * BT;
     {
       const unsigned t1 = T::T1_OFF + slot * T::TBYTES, t2 = T::T2_OFF + slot * T::TBYTES;
@@ -540,32 +687,9 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       auto rows4 = [&](unsigned staged_off, int q4) FL_INLINE -> f32x4 {
         return *reinterpret_cast<const f32x4*>(smem + staged_off + slot * T::SBYTES + (q4 - t0) * 4);
       };
-      // element predicate as an interval of the register offset `off` (8 (i / 4) + i % 4): lo <= off <= hi
-      auto bounds = [&](int sbase, int& lo, int& hi) FL_INLINE {
-        if constexpr (kDQ) {
-          // streamed = key, owner = query: key < Lk && (dmin <= key - q <= dmax || key < pfx)
-          const int rel = sbase - opos;
-          hi = min(p.Lk - sbase - 1, max(p.dmax - rel, p.pfx - sbase - 1));
-          lo = p.dmin - rel;
-        } else {
-          // streamed = query, owner = key: q < Lq && (dmin <= key - q <= dmax || key < pfx), key = opos
-          const int rel = opos - sbase;  // key - q at off = 0; key - q = rel - off
-          hi = min(p.Lq - sbase - 1, opos < p.pfx ? (1 << 29) : rel - p.dmin);
-          lo = opos < p.pfx ? -(1 << 29) : rel - p.dmax;
-          if (opos >= p.Lk) hi = -(1 << 29);
-        }
-      };
-      auto attended = [&](int sbase, int off, int lo, int hi) FL_INLINE -> bool {
-        bool ok = (off <= hi) & (off >= lo);
-        if constexpr (kDoc) {
-          if (!doc_uniform) ok = ok & (*reinterpret_cast<const int64_t*>(smem + T::IDS_OFF + slot * BT * 8 + (sbase - t0 + off) * 8) == odoc);
-        }
-        return ok;
-      };
       // (document ids beside bias operands: the mask goes with each weight, sixteen ids in flight do not fit in the registers)
       constexpr bool kMaskApart = !(kDoc && kBias);
-      constexpr bool kMaskScores = FEAT == 0 || (FEAT == F_DOC && D <= 64);
-      constexpr bool kSched = T::TUNED;
+      constexpr bool kMaskScores = FEAT == 0 || FEAT == F_DOC;
       // X2 = T2 . O2^T (dP).  At D = 128 its fp32 tile is declared out here, next to X1's, and (ROLE_DQ) its MFMAs are issued
       // right after X1's, before the weights' vector work; at D = 64 it lives in the block that consumes it.  Both choices
       // are measured: the first is 15 % faster at D = 128 and 1-2 % slower at D = 64.
@@ -624,7 +748,6 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
           for (int sb = 0; sb < TB; ++sb)
             x1[sb] = mfma32(frag_row(t1, sb, ks), b1, x1[sb]);
         }
-        if constexpr (kSched) sched_scores<KS, TB, kDQ>();
         if constexpr (kMaskScores) {
           if (!full) {  // workgroup-uniform; here, so that everything from the weights on is one block to be ordered
 #pragma unroll
@@ -635,7 +758,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
               asm volatile("" : "+v"(lo), "+v"(hi));
 #pragma unroll
               for (int i = 0; i < 16; ++i) {
-                if (!attended(sbase, 8 * (i / 4) + i % 4, lo, hi)) x1[sb][i] = -INFINITY;
+                if (!attended(t0, sbase, slot, 8 * (i / 4) + i % 4, lo, hi, doc_uniform)) x1[sb][i] = -INFINITY;
               }
             }
           }
@@ -678,7 +801,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
                 s2 = __builtin_fmaf(bias_at(kDQ ? op : sp, kDQ ? sp : op, shead), kLog2e, s2);
               }
               pv[sb][i] = fast_exp2(s2);
-              if (!kMaskApart && !full && !attended(sbase, off, lo, hi)) pv[sb][i] = 0.f;
+              if (!kMaskApart && !full && !attended(t0, sbase, slot, off, lo, hi, doc_uniform)) pv[sb][i] = 0.f;
               pd[sb][i] = kSoftcap ? dfac : 1.0f;
             }
           }
@@ -699,7 +822,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
             asm volatile("" : "+v"(lo), "+v"(hi));
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-              if (!attended(sbase, 8 * (i / 4) + i % 4, lo, hi)) pv[sb][i] = 0.f;
+              if (!attended(t0, sbase, slot, 8 * (i / 4) + i % 4, lo, hi, doc_uniform)) pv[sb][i] = 0.f;
             }
           }
 #pragma unroll
@@ -789,7 +912,6 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
           acc1[db] = mfma32(frag_tr(t1, c, db), dsf[c], acc1[db]);
           if constexpr (!kDQ && !kMaskScores) acc2[db] = mfma32(frag_tr(t2, c, db), pf[c], acc2[db]);
         }
-      if constexpr (kSched) sched_gradients<KS, TB, DB, kDQ>();
     }
   };
   if constexpr (kDoc) {
