@@ -1368,6 +1368,19 @@ BwdPlan plan_bwd(const fl_attn_params* p) {
   x.bytes = x.dq_bytes + (x.dkv > 1 ? (uint64_t)x.dkv * k_tiles * 128 * D * 2 * sizeof(float) : 0);
   return x;
 }
+
+// dK and dV, a launch of their own at head dim 128 without score modifications: 256 keys per workgroup instead of 128, one workgroup of
+// eight waves per compute unit either way.  A round takes twice as long, so the last one must not be far from full (all of it under masks of
+// growing length, whose longest walk is twice the average), unless there are several; and few of the keys' places may be empty.
+// us, both roles, 128 -> 256 keys: causal, 16 heads of 4096 (256 tiles of 256 keys) 259 -> 303, 20 (320) 368 -> 432, 24 (384) 365 -> 365, 2 x 16 (512)
+// 473 -> 452, 4 x 16 922 -> 890, 16 x 32 of 512 (1024) 270 -> 253, 13 x 16 of 700 (624) 178 -> 180; unmasked, 16 of 4096 436 -> 420, 24 648 -> 679;
+// windows of 100, 8 x 16 of 4096, 515 -> 487; a prefix, 8 x 16 of 1500, 352 -> 325.
+bool wide_dkv(const fl_attn_params* p) {
+  const int64_t narrow = (p->Lk + 127) / 128, wide = (p->Lk + 255) / 256, tiles = (int64_t)p->B * p->Hkv * wide;
+  if (2 * wide > narrow && narrow < 16) return false;
+  if (tiles >= 1024) return true;
+  return tiles > (p->mask_kind == FL_MASK_NONE ? 224 : 480) && (tiles % 256 == 0 || tiles % 256 > 224);
+}
 }  // namespace
 
 uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p) {
@@ -1453,12 +1466,13 @@ static int launch_gradients(const fl_attn_bwd_params* b, bool planned, void* scr
   if (plan.dkv > 1) bp.part = bp.part_dq + plan.dq_bytes / sizeof(float);
   bp.splits_dq = plan.dq;
   bp.splits = plan.dkv;
+  bp.dkv_own = planned && !plan.both && in->d == 128 && in->feat == 0 && wide_dkv(p) ? 256 : 128;
   bp.head_group = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM || p->mask_kind == FL_MASK_DOCUMENT_CAUSAL ? 4 : 1;
   bp.by_head_group = fl::Div::by(bp.head_group);
   bp.by_group = fl::Div::by(bp.group);
   bp.by_Hq = fl::Div::by(p->Hq);
   for (int r = 0; r < 2; ++r) {
-    const uint32_t heads = r ? p->Hkv : p->Hq, tiles = ((r ? p->Lk : p->Lq) + 127) / 128, pairs = p->B * heads;
+    const uint32_t heads = r ? p->Hkv : p->Hq, own = r ? bp.dkv_own : 128, tiles = ((r ? p->Lk : p->Lq) + own - 1) / own, pairs = p->B * heads;
     const uint32_t rest = (pairs % 8 ? pairs : pairs / 8) % bp.head_group;
     bp.role[r].by_heads = fl::Div::by(bp.head_group * tiles);
     bp.role[r].by_rest = fl::Div::by(rest ? rest : 1);

@@ -85,6 +85,9 @@ hipError_t launch_delta(const BParams& bp, hipStream_t stream) {
     return launch_bwd_role<BwdTraits<D, ROLE_DQ, FEAT, ELEM>>(bp, bwd_q_tiles(bp), s);                              \
   }                                                                                                                 \
   hipError_t launch_bwd_dkv_##D##_##FEAT##SFX(const BParams& bp, hipStream_t s) {                                   \
+    if constexpr (D == 128 && FEAT == 0) {                                                                          \
+      if (bp.dkv_own == 256) return launch_bwd_role<BwdTraits<D, ROLE_DKV, FEAT, ELEM, false, true>>(bp, (int64_t)bp.B * bp.Hkv * ((bp.Lk + 255) / 256), s); \
+    }                                                                                                               \
     return launch_bwd_role<BwdTraits<D, ROLE_DKV, FEAT, ELEM>>(bp, bwd_k_tiles(bp), s);                             \
   }                                                                                                                 \
   hipError_t launch_bwd_both_##D##_##FEAT##SFX(const BParams& bp, hipStream_t s) { return launch_bwd_both<D, FEAT, ELEM>(bp, s); } \

@@ -64,6 +64,7 @@ struct BParams {
   // bwd_both_kernel: `part` and `splits` are the dK/dV role's, these the dQ role's
   float* part_dq;
   int32_t splits_dq;
+  int32_t dkv_own;  // owner positions per workgroup of the dK/dV launch
   // Divisors, per role (0: dQ, 1: dK/dV).  (batch, head) pairs are dealt head_group at a time
   int32_t head_group;
   Div by_head_group, by_group, by_Hq, by_delta_blocks;
@@ -131,19 +132,21 @@ static_assert([]() constexpr {
   return true;
 }(), "one place per chunk");
 
-// SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size.
-template <int D_, int ROLE_, uint32_t FEAT_, class Elem_ = bf16_t, bool SHARED_ = false>
+// SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size.  WIDE_: 256 owner positions per workgroup
+// (ROLE_DKV at head dim 128, wide_dkv in api.hip): eight waves own 32 keys each, so that a streamed tile comes in once for twice as many
+// keys, K stays in registers and nothing is added up at the end.
+template <int D_, int ROLE_, uint32_t FEAT_, class Elem_ = bf16_t, bool SHARED_ = false, bool WIDE_ = false>
 struct BwdTraits {
   using Elem = Elem_;  // element type of q, k, v, o, dout and the gradients: bf16_t or f16_t
   static constexpr int D = D_, ROLE = ROLE_;
-  static constexpr bool SHARED = SHARED_;
+  static constexpr bool SHARED = SHARED_, WIDE = WIDE_;
   static constexpr uint32_t FEAT = FEAT_;
-  static constexpr int OWN = 128;                          // owner positions per workgroup
+  static constexpr int OWN = WIDE ? 256 : 128;             // owner positions per workgroup
   static constexpr int OB = OWN / 32;                      // blocks of 32 of them, a wave each (two with QH == 2)
   // ROLE_DKV at D = 128 holds 128 accumulator registers per lane; to still run two waves per SIMD its workgroup has
   // 8 waves, two per owner block, which take the two halves of every streamed tile and add up their partial sums
   // through LDS at the end (one workgroup per CU, 128 KB of LDS).
-  static constexpr int QH = ((ROLE == ROLE_DKV || SHARED_) && D_ > 64) ? 2 : 1;   // waves per owner block
+  static constexpr int QH = ((ROLE == ROLE_DKV || SHARED_) && D_ > 64 && !WIDE) ? 2 : 1;   // waves per owner block
   static constexpr int NW = OB * QH, NT = 64 * NW;
   static constexpr int TB = (D_ <= 64) ? 2 : 1;  // 32-position blocks per wave and step (register budget)
   static constexpr int BT = 32 * TB * QH;                  // streamed positions per step
@@ -160,7 +163,7 @@ struct BwdTraits {
   static constexpr bool ORDERED = ((FEAT_ & ~F_DOC) == 0 || (FEAT_ & ~(F_ALIBI | F_SOFTCAP)) == 0) && D_ >= 64;
   static constexpr int AHEAD = 3;
   // ROLE_DKV: the owner's K and V rows as operands in registers, where there is room, instead of in LDS
-  static constexpr bool K_REGS = ROLE == ROLE_DKV && ORDERED && D <= 64, V_REGS = ROLE == ROLE_DQ || K_REGS;
+  static constexpr bool K_REGS = ROLE == ROLE_DKV && ORDERED && (WIDE || D <= 64), V_REGS = ROLE == ROLE_DQ || (K_REGS && D <= 64);
   static constexpr int OBYTES = (ROLE == ROLE_DKV) ? OWN * D * 2 : 0;  // owner tile kept in LDS (ROLE_DKV: K and V)
   static constexpr int O_PER_T = OBYTES / (NT * 16);
   static_assert(OBYTES % (NT * 16) == 0, "owner tile must divide evenly over the threads");
@@ -484,11 +487,13 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   auto classify_tile = [&](int tile, bool& full, bool& doc_uniform) FL_INLINE -> bool {
     const int t0 = tile * BT;
     const int s1 = min(t0 + BT, slen);
-    const int qa = kDQ ? o0 : t0, qb_ = kDQ ? o1 : s1, ka = kDQ ? t0 : o0, kb_ = kDQ ? s1 : o1;
+    const int w0 = T::WIDE ? o0 + 32 * ow : o0, w1 = T::WIDE ? min(w0 + 32, olen) : o1;  // (WIDE: this wave's own positions)
+    if (T::WIDE && w0 >= olen) return true;
+    const int qa = kDQ ? w0 : t0, qb_ = kDQ ? w1 : s1, ka = kDQ ? t0 : w0, kb_ = kDQ ? s1 : w1;
     const int cls = classify_positional(p.mask_kind, qa, qb_, ka, kb_, p.window, p.prefix);
     bool skip = cls == TILE_EMPTY;
     // every pair of the step attended: the positional mask holds everywhere and both ranges lie inside the sequences
-    full = cls == TILE_FULL && t0 + BT <= slen && o0 + T::OWN <= olen;
+    full = cls == TILE_FULL && t0 + BT <= slen && w0 + (T::WIDE ? 32 : T::OWN) <= olen;
     doc_uniform = false;
     if constexpr (kDoc) {
       int64_t mn, mx;
