@@ -43,31 +43,42 @@ static __global__ void doc_table_kernel(const int64_t* ids, int64_t ids_stride, 
 // FULL when both are the same single id and the positional part of the mask agrees, PARTIAL otherwise.  Valid for
 // arbitrary (unsorted, negative) ids.  The lists are the same for every head.  Output per workgroup: word 0 = number of
 // entries, then the entries in key order (bits 0-15 tile index, two class bits per wave from bit 16 on).
-// Three phases: a wave per key tile reads its ids with one coalesced load and leaves their (min, max) in LDS (every
-// load of a wave is in flight before the first is looked at: the kernel is a chain of round trips to memory with little
-// to do in between); a thread per key tile classifies it for every wave; one wave compacts the non-empty entries.
+// A wave per key tile reads its ids with one coalesced load and leaves their (min, max) in LDS (every load of a wave is in flight before
+// the first is looked at: the kernel is a chain of round trips to memory with little to do in between); the place of this query tile
+// in the order is found; a thread per key tile classifies it for every wave; the non-empty entries are compacted.
+//
+// The order: the query tiles of a batch row by falling length of their tile lists (ties by falling index), so that the workgroups still running
+// when the grid drains are short ones whatever the document layout.  Every workgroup works out the lengths of all query tiles, by a
+// binary search each where the ids are sorted, and writes its own place: a second launch for it was 5 of the 15 us of the pre-pass (16384
+// ids, 16 heads, us for the forward with its pre-pass: 139.9 -> 136.3).  The lengths count the key tiles whose range meets the whole query tile's; any order
+// gives the same results.  Unsorted ids are counted pair by pair, up to kOrderPairs, beyond that the order is that of the index.
+constexpr int kDocWaves = 4;  // waves of the forward that a query tile is classified for, at most
+constexpr int64_t kOrderPairs = 1 << 18;
 static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* ids, int64_t ids_stride, int L, int mask_kind,
                                                                 int bm, int rw, int bn, int n_qtiles, int nk, int list_stride,
-                                                                uint32_t* lists) {
+                                                                uint32_t* lists, int32_t* order) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
   int64_t* krange = reinterpret_cast<int64_t*>(lds_raw);                // [nk][2] = (min, max) id of a key tile
-  uint32_t* tl = reinterpret_cast<uint32_t*>(lds_raw + (size_t)nk * 16);  // [nk] uncompacted entries
-  __shared__ int64_t qrange[16];  // (min, max) id of the rows of each of up to 8 waves of the forward
+  uint32_t* tl = reinterpret_cast<uint32_t*>(lds_raw + (size_t)nk * 16);  // [nk] counts per query tile, then uncompacted entries
+  __shared__ int64_t qrange[2 * kDocWaves];  // (min, max) id of the rows of each wave of the forward
+  __shared__ uint32_t few[16];               // [0] ids are unsorted, [1] this tile's place; then entries per wave
   constexpr int kWaves = 16, kBatch = 16;
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int b = blockIdx.x / n_qtiles, qt = blockIdx.x % n_qtiles;
   const int nw = bm / rw, q0 = qt * bm;
   const int64_t* idb = ids + (int64_t)b * ids_stride;
+  const bool causal = mask_kind == MASK_DOC_CAUSAL;
   // rows past L repeat the last row (a wave without valid rows is EMPTY for every tile whatever its range)
   const int64_t qid = idb[min(q0 + min(wave, nw - 1) * rw + lane % rw, L - 1)];
   // key tiles some row may attend under the positional part of the mask: all of them, or those up to the diagonal
-  const int t_end = mask_kind == MASK_DOC_CAUSAL ? min(nk, (min(q0 + bm, L) - 1) / bn + 1) : nk;
+  const int t_end = causal ? min(nk, (min(q0 + bm, L) - 1) / bn + 1) : nk;
   const int nj = (bn + 63) / 64;  // loads per lane that cover one tile's ids
-  for (int t0 = wave; t0 < t_end || t0 == wave; t0 += kWaves * kBatch) {
+  if (tid < 16) few[tid] = 0;
+  for (int t0 = wave; t0 < nk || t0 == wave; t0 += kWaves * kBatch) {
     int64_t lo[kBatch], hi[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const int k0 = min(t0 + kWaves * u, t_end - 1) * bn;
+      const int k0 = min(t0 + kWaves * u, nk - 1) * bn;
       lo[u] = hi[u] = idb[min(k0 + lane % bn, L - 1)];
       for (int j = 1; j < nj; ++j) {
         const int64_t x = idb[min(k0 + j * 64 + lane, L - 1)];
@@ -86,7 +97,7 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
       const int t = t0 + kWaves * u;
-      if (t >= t_end) break;
+      if (t >= nk) break;
       int64_t kmn, kmx, unused;
       wave_id_range(lo[u], kmn, unused);
       if (nj > 1) wave_id_range(hi[u], unused, kmx); else kmx = unused;
@@ -97,7 +108,61 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
     }
   }
   __syncthreads();
-  for (int t = tid; t < t_end; t += 1024) {
+  // ---- this query tile's place
+  {
+    bool falls = false;
+    for (int t = tid; t + 1 < nk; t += 1024) falls = falls || krange[2 * t + 1] > krange[2 * t + 2];
+    if (__builtin_amdgcn_ballot_w64(falls) != 0 && lane == 0) few[0] = 1;
+    for (int j = tid; j < n_qtiles; j += 1024) tl[j] = 0;
+  }
+  __syncthreads();
+  const bool sorted = few[0] == 0, counted = !sorted && (int64_t)n_qtiles * nk <= kOrderPairs;
+  auto first_tile = [&](int j) FL_INLINE { return min(j * bm / bn, nk - 1); };  // key tiles that hold the rows of query tile j
+  auto last_tile = [&](int j) FL_INLINE { return min((min((j + 1) * bm, L) - 1) / bn, nk - 1); };
+  if (counted) {
+    for (int j0 = 0; j0 < n_qtiles; j0 += 64) {
+      const int j = min(j0 + lane, n_qtiles - 1), last = last_tile(j);
+      int64_t mn = krange[2 * first_tile(j)], mx = krange[2 * first_tile(j) + 1];
+      for (int t = first_tile(j) + 1; t <= last; ++t) {
+        mn = krange[2 * t] < mn ? krange[2 * t] : mn;
+        mx = krange[2 * t + 1] > mx ? krange[2 * t + 1] : mx;
+      }
+      uint32_t count = 0;
+      for (int t = wave; t < nk; t += kWaves) count += krange[2 * t + 1] >= mn && krange[2 * t] <= mx && (!causal || t <= last);
+      if (j0 + lane < n_qtiles) atomicAdd(&tl[j], count);
+    }
+    __syncthreads();
+  }
+  auto length = [&](int j) FL_INLINE -> int {
+    if (counted) return (int)tl[j];
+    if (!sorted) return 0;
+    // first tile whose range reaches the query tile's smallest id; last one whose range begins at or below its largest
+    const int64_t mn = krange[2 * first_tile(j)], mx = krange[2 * last_tile(j) + 1];
+    int lo = 0, hi = first_tile(j);
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if (krange[2 * mid + 1] >= mn) hi = mid; else lo = mid + 1;
+    }
+    int last = last_tile(j);
+    if (!causal) {
+      int end = nk - 1;
+      while (last < end) {
+        const int mid = (last + end + 1) / 2;
+        if (krange[2 * mid] <= mx) last = mid; else end = mid - 1;
+      }
+    }
+    return last - lo + 1;
+  };
+  const int mine = length(qt);
+  for (int j0 = wave * 64; j0 < n_qtiles; j0 += 1024) {
+    const int j = j0 + lane, len = length(min(j, n_qtiles - 1));
+    const uint64_t before = __builtin_amdgcn_ballot_w64(j < n_qtiles && (len > mine || (len == mine && j > qt)));
+    if (lane == 0 && before != 0) atomicAdd(&few[1], (uint32_t)__builtin_popcountll(before));
+  }
+  __syncthreads();
+  if (tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
+  // ---- the list
+  auto entry_of = [&](int t) FL_INLINE -> uint32_t {
     const int k0 = t * bn, k1 = min(k0 + bn, L);
     const int64_t kmn = krange[2 * t], kmx = krange[2 * t + 1];
     unsigned c = 0;
@@ -113,11 +178,30 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
       }
       c |= (unsigned)cw << (2 * w);
     }
-    tl[t] = (c << 16) | (unsigned)t;
+    return (c << 16) | (unsigned)t;
+  };
+  uint32_t* out = lists + (int64_t)blockIdx.x * list_stride;
+  if (t_end <= 1024) {  // an entry per thread
+    const uint32_t e = tid < t_end ? entry_of(tid) : 0u;
+    const bool keep = (e >> 16) != 0;
+    const uint64_t m = __builtin_amdgcn_ballot_w64(keep);
+    __syncthreads();  // (the tile's place has been read)
+    if (lane == 0) few[wave] = (uint32_t)__builtin_popcountll(m);
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const uint32_t n = few[w];
+      before += w < wave ? n : 0;
+      all += n;
+    }
+    if (keep) out[1 + before + __builtin_popcountll(m & ((1ull << lane) - 1))] = e;
+    if (tid == 0) out[0] = all;
+    return;
   }
+  for (int t = tid; t < t_end; t += 1024) tl[t] = entry_of(t);
   __syncthreads();
   if (wave == 0) {
-    uint32_t* out = lists + (int64_t)blockIdx.x * list_stride;
     int count = 0;
     for (int base = 0; base < t_end; base += 64) {
       const int t = base + lane;
@@ -129,23 +213,6 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
       count += __builtin_popcountll(m);
     }
     if (lane == 0) out[0] = (uint32_t)count;
-  }
-}
-
-// Second step of the forward pre-pass for document masks, one workgroup per batch row: the query tiles ordered by
-// falling length of their tile lists (ties by falling index), by counting for every tile how many come before it.
-static __global__ __launch_bounds__(1024) void doc_order_kernel(const uint32_t* lists, int list_stride, int n_qtiles,
-                                                               int32_t* order) {
-  extern __shared__ uint32_t cnt[];  // n_qtiles words
-  const int b = blockIdx.x;
-  const uint32_t* lb = lists + (int64_t)b * n_qtiles * list_stride;
-  for (int i = threadIdx.x; i < n_qtiles; i += 1024) cnt[i] = lb[(int64_t)i * list_stride];
-  __syncthreads();
-  for (int i = threadIdx.x; i < n_qtiles; i += 1024) {
-    const uint32_t mine = cnt[i];
-    int rank = 0;
-    for (int j = 0; j < n_qtiles; ++j) rank += (cnt[j] > mine) || (cnt[j] == mine && j > i);
-    order[(int64_t)b * n_qtiles + rank] = i;
   }
 }
 
@@ -1224,15 +1291,12 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
       static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fl::doc_lists_kernel),
                                                          hipFuncAttributeMaxDynamicSharedMemorySize, fl::kMaxLdsBytes - 128);
       if (attr != hipSuccess) return fail((int)attr, "doc_lists_kernel: %s", hipGetErrorString(attr));
+      if (in->nw > fl::kDocWaves) return fail(FL_ERR_UNSUPPORTED, "%s: more waves than the document lists have classes for", in->name);
       hipLaunchKernelGGL(fl::doc_lists_kernel, dim3(p->B * kp.n_qtiles), dim3(1024), (size_t)prepass_lds_bytes(kp.n_ktiles), stream,
                          p->doc_ids, p->doc_stride, p->Lk, p->mask_kind, bm, in->rw, in->bn, kp.n_qtiles, kp.n_ktiles,
-                         (int)d.list_stride, lists);
-      hipError_t e = hipGetLastError();
+                         (int)d.list_stride, lists, order);
+      const hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, "doc_lists_kernel launch failed: %s", hipGetErrorString(e));
-      hipLaunchKernelGGL(fl::doc_order_kernel, dim3(p->B), dim3(1024), (size_t)kp.n_qtiles * 4, stream, lists,
-                         (int)d.list_stride, kp.n_qtiles, order);
-      e = hipGetLastError();
-      if (e != hipSuccess) return fail((int)e, "doc_order_kernel launch failed: %s", hipGetErrorString(e));
     }
     kp.doc_lists = lists;
     kp.doc_list_stride = (int)d.list_stride;

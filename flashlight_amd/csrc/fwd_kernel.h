@@ -108,7 +108,7 @@ struct KParams {
   // entries in key order (bits 0-15 tile index, two class bits per wave from bit 16 on).
   uint32_t* doc_lists;
   int32_t doc_list_stride;  // words per (batch, query tile): a multiple of 4, at least n_ktiles + 1
-  // per batch row the query tiles ordered by falling list length (doc_order_kernel): workgroups are dealt in that order,
+  // per batch row the query tiles ordered by falling list length (doc_lists_kernel): workgroups are dealt in that order,
   // so that the ones still running when the grid drains are the short ones whatever the document layout
   int32_t* doc_order;
   // The lists have not been made by a launch of their own (at most kOwnListTiles key tiles): every workgroup lists its tiles itself, and

@@ -53,3 +53,26 @@ def test_prepared_workspaces_serve_calls_of_other_heads(D, S):
             out = _ffi.attn_fwd(q, k, v, mask_kind=_ffi.MASK_DOCUMENT_CAUSAL, doc_ids=ids, doc_workspace=ws)
             assert ready is None or ws.buffer is ready  # (not prepared anew)
             assert torch.equal(out, plain[H]), (first, then, H)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["sorted", "falling", "scattered"])
+@pytest.mark.parametrize("S", [8193, 20000, 66001])  # one entry per thread, counted pair by pair where unsorted, more of both
+def test_every_query_tile_has_a_place_in_the_order(S, kind):
+    """Documents of two positions: a row's result is its value, or the softmax of two logits over two values."""
+    H, D, pairs = 4, 64, (S + 1) // 2
+    g = torch.Generator().manual_seed(S)
+    q, k, v = (torch.randn(1, H, S, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(3))
+    number = torch.arange(S) // 2
+    ids = {"sorted": number, "falling": -number, "scattered": number * 7919 % pairs}[kind]
+    out = _ffi.attn_fwd(q, k, v, mask_kind=_ffi.MASK_DOCUMENT_CAUSAL, doc_ids=ids[None].to(DEV)).double()
+    qd, kd, vd = q.double(), k.double(), v.double()
+    even, odd = slice(0, None, 2), slice(1, None, 2)
+    assert torch.equal(out[:, :, even], vd[:, :, even])
+    n = S // 2
+    logits = torch.stack([(qd[:, :, odd] * kd[:, :, even][:, :, :n]).sum(-1), (qd[:, :, odd] * kd[:, :, odd]).sum(-1)], -1) * D ** -0.5
+    w = logits.softmax(-1)
+    want = w[..., :1] * vd[:, :, even][:, :, :n] + w[..., 1:] * vd[:, :, odd]
+    # weights rounded to 16 bits, numerator and row sum alike, and one rounding of the result
+    bound = 2.0 ** -8 * (w[..., :1] * vd[:, :, even][:, :, :n].abs() + w[..., 1:] * vd[:, :, odd].abs() + 2 * want.abs())
+    assert ((out[:, :, odd] - want).abs() <= bound).all()
