@@ -61,7 +61,8 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
   int64_t* krange = reinterpret_cast<int64_t*>(lds_raw);                // [nk][2] = (min, max) id of a key tile
   uint32_t* tl = reinterpret_cast<uint32_t*>(lds_raw + (size_t)nk * 16);  // [nk] counts per query tile, then uncompacted entries
   __shared__ int64_t qrange[2 * kDocWaves];  // (min, max) id of the rows of each wave of the forward
-  __shared__ uint32_t few[16];               // [0] ids are unsorted, [1] this tile's place; then entries per wave
+  __shared__ uint32_t few[2];                // [0] ids are unsorted, [1] this tile's place
+  __shared__ uint16_t kept[16];              // entries per wave (104 bytes of static LDS: the longest call, 8185 key tiles, leaves 128)
   constexpr int kWaves = 16, kBatch = 16;
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int b = blockIdx.x / n_qtiles, qt = blockIdx.x % n_qtiles;
@@ -73,12 +74,13 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
   // key tiles some row may attend under the positional part of the mask: all of them, or those up to the diagonal
   const int t_end = causal ? min(nk, (min(q0 + bm, L) - 1) / bn + 1) : nk;
   const int nj = (bn + 63) / 64;  // loads per lane that cover one tile's ids
-  if (tid < 16) few[tid] = 0;
+  if (tid < 2) few[tid] = 0;
+  const int turn = blockIdx.x / 8;  // (where a workgroup begins: all of an XCD's would ask for the same lines at the same time)
   for (int t0 = wave; t0 < nk || t0 == wave; t0 += kWaves * kBatch) {
     int64_t lo[kBatch], hi[kBatch];
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const int k0 = min(t0 + kWaves * u, nk - 1) * bn;
+      const int k0 = min(t0 + kWaves * ((u + turn) % kBatch), nk - 1) * bn;
       lo[u] = hi[u] = idb[min(k0 + lane % bn, L - 1)];
       for (int j = 1; j < nj; ++j) {
         const int64_t x = idb[min(k0 + j * 64 + lane, L - 1)];
@@ -94,17 +96,36 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
         qrange[2 * wave + 1] = mx;
       }
     }
+    // lane u keeps tile u's range: the first id where all are the same, the others are reduced one by one (reduced as they come, the
+    // sixteen were 3 us)
+    uint32_t mixed = 0;
+    int64_t mn = 0, mx = 0;
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const int t = t0 + kWaves * u;
-      if (t >= nk) break;
-      int64_t kmn, kmx, unused;
-      wave_id_range(lo[u], kmn, unused);
-      if (nj > 1) wave_id_range(hi[u], unused, kmx); else kmx = unused;
-      if (lane == 0) {
-        krange[2 * t] = kmn;
-        krange[2 * t + 1] = kmx;
+      const int64_t first = uniform_i64(lo[u]);
+      if (__builtin_amdgcn_ballot_w64(lo[u] != first || hi[u] != first) != 0) mixed |= 1u << u;
+      mn = lane == u ? first : mn;
+    }
+    mx = mn;
+#pragma unroll 1
+    for (; mixed != 0; mixed &= mixed - 1) {
+      const int which = (int)__builtin_ctz(mixed);
+      int64_t x = lo[0], y = hi[0];
+#pragma unroll
+      for (int u = 1; u < kBatch; ++u) {
+        x = which == u ? lo[u] : x;
+        y = which == u ? hi[u] : y;
       }
+      int64_t least, most, unused;
+      wave_id_range(x, least, most);
+      if (nj > 1) wave_id_range(y, unused, most);
+      mn = lane == which ? least : mn;
+      mx = lane == which ? most : mx;
+    }
+    const int t = t0 + kWaves * ((lane + turn) % kBatch);
+    if (lane < kBatch && t < nk) {
+      krange[2 * t] = mn;
+      krange[2 * t + 1] = mx;
     }
   }
   __syncthreads();
@@ -153,14 +174,12 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
     }
     return last - lo + 1;
   };
-  const int mine = length(qt);
-  for (int j0 = wave * 64; j0 < n_qtiles; j0 += 1024) {
-    const int j = j0 + lane, len = length(min(j, n_qtiles - 1));
+  // (the last waves first: the first ones have the entries)
+  for (int j0 = (kWaves - 1 - wave) * 64; j0 < n_qtiles; j0 += 1024) {
+    const int mine = length(qt), j = j0 + lane, len = length(min(j, n_qtiles - 1));
     const uint64_t before = __builtin_amdgcn_ballot_w64(j < n_qtiles && (len > mine || (len == mine && j > qt)));
     if (lane == 0 && before != 0) atomicAdd(&few[1], (uint32_t)__builtin_popcountll(before));
   }
-  __syncthreads();
-  if (tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
   // ---- the list
   auto entry_of = [&](int t) FL_INLINE -> uint32_t {
     const int k0 = t * bn, k1 = min(k0 + bn, L);
@@ -185,13 +204,13 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
     const uint32_t e = tid < t_end ? entry_of(tid) : 0u;
     const bool keep = (e >> 16) != 0;
     const uint64_t m = __builtin_amdgcn_ballot_w64(keep);
-    __syncthreads();  // (the tile's place has been read)
-    if (lane == 0) few[wave] = (uint32_t)__builtin_popcountll(m);
+    if (lane == 0) kept[wave] = (uint16_t)__builtin_popcountll(m);
     __syncthreads();
+    if (tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
     uint32_t before = 0, all = 0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      const uint32_t n = few[w];
+      const uint32_t n = kept[w];
       before += w < wave ? n : 0;
       all += n;
     }
@@ -199,6 +218,8 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
     if (tid == 0) out[0] = all;
     return;
   }
+  __syncthreads();  // (the counts in tl have been read)
+  if (tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
   for (int t = tid; t < t_end; t += 1024) tl[t] = entry_of(t);
   __syncthreads();
   if (wave == 0) {
@@ -508,7 +529,7 @@ int64_t lds_bytes_for(const fl::Instance* in, const fl_attn_params* p) {
   const DocScratch d = doc_scratch(p->B, p->Lk, (int64_t)in->rw * in->nw, in->bn);
   return in->lds_fixed_bytes + (d.list_stride * 4 + 1023) / 1024 * 1024;
 }
-// Dynamic LDS bytes of the document-mask pre-pass (doc_lists_kernel): 20 per key tile; it has 128 static bytes besides
+// Dynamic LDS bytes of the document-mask pre-pass (doc_lists_kernel): 20 per key tile; it has up to 128 static bytes besides
 int64_t prepass_lds_bytes(int64_t n_ktiles) { return n_ktiles * 20; }
 // Groups of waves a call is launched with, and the LDS of all of them
 int groups_for(const fl::Instance* in, const fl_attn_params* p) {
