@@ -1631,6 +1631,7 @@ int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* strea
   if (x.row >= 0) {
     pp.row = p->bias[x.row];
     pp.rowb = reinterpret_cast<float*>(ws + x.rowb);
+    pp.row_factor = 1.0f / p->scale;
     pp.row_batch = p->bias_strides[x.row][0];
     pp.row_key = (int)p->bias_strides[x.row][3];
     pp.row_div = p->bias_batch_div[x.row];
