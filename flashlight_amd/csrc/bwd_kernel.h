@@ -634,7 +634,11 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
           if (!full) {  // uniform over the workgroup or the wave; the asm keeps it a branch
             bounds(sbase, lo[sb], hi[sb]);
             asm volatile("" : "+v"(lo[sb]), "+v"(hi[sb]));
-            if constexpr (!kSoftcap) {
+            if constexpr (!kSoftcap && !kDoc) {
+              const unsigned out = outside_word(lo[sb], hi[sb]);
+#pragma unroll
+              for (int i = 0; i < 16; ++i) x1[sb][i] = minus_inf_outside(x1[sb][i], out, 8 * (i / 4) + i % 4);
+            } else if constexpr (!kSoftcap) {
 #pragma unroll
               for (int i = 0; i < 16; ++i)
                 if (!attended(t0, sbase, slot, 8 * (i / 4) + i % 4, lo[sb], hi[sb], doc_uniform)) x1[sb][i] = -INFINITY;
