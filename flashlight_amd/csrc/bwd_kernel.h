@@ -635,9 +635,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
             bounds(sbase, lo[sb], hi[sb]);
             asm volatile("" : "+v"(lo[sb]), "+v"(hi[sb]));
             if constexpr (!kSoftcap && !kDoc) {
-              const unsigned out = outside_word(lo[sb], hi[sb]);
-#pragma unroll
-              for (int i = 0; i < 16; ++i) x1[sb][i] = minus_inf_outside(x1[sb][i], out, 8 * (i / 4) + i % 4);
+              minus_inf_outside(x1[sb], outside_word(lo[sb], hi[sb]));
             } else if constexpr (!kSoftcap) {
 #pragma unroll
               for (int i = 0; i < 16; ++i)

@@ -429,14 +429,23 @@ __device__ __forceinline__ void sched_second_product() {
 // The positional mask of the 16 scores a lane holds of a block: bit `off` says that offset `off` (8 (i / 4) + i % 4 for register i, 27
 // at most, so that a shift by 31 reaches them all) lies outside lo <= off <= hi.  Two vector instructions per score, a bit spread over a
 // word and a bitwise choice, where two comparisons, the scalar product of their results and a select were needed; the first is written
-// as an instruction because the compiler makes a comparison of the bit again.  us, cold operands, head dim 128: forwards, window of 256,
-// 4 x 16 x 4096, 87.5 -> 86.0; differential causal 4 x 16 x 4096 229 -> 225.  Gradients, window of 300, 4 x 16 x 4096, 301 -> 296;
-// prefix of 200, 3 x 16 over 4 heads of 1000, head dim 64, 58.3 -> 54.7; causal 16 x 32 x 256, head dim 128, 97.7 -> 94.9.
+// as an instruction because the compiler makes a comparison of the bit again, four at a time because it puts a wait state behind each
+// such piece.  us, cold operands, head dim 128: forwards, window of 256, 4 x 16 x 4096, 87.5 -> 85.3; differential causal 4 x 16 x 4096
+// 229 -> 225.  Gradients, window of 300, 4 x 16 x 4096, 301 -> 290, head dim 64 150 -> 137; prefix of 200, 3 x 16 over 4 heads of 1000,
+// head dim 64, 58.3 -> 53.9; causal 16 x 32 x 256, head dim 128, 97.7 -> 95.0.
 __device__ __forceinline__ unsigned outside_word(int lo, int hi) { return (~0u << min(max(hi + 1, 0), 31)) | ~(~0u << min(max(lo, 0), 31)); }
-__device__ __forceinline__ float minus_inf_outside(float x, unsigned out, const int off) {
-  unsigned lost;
-  asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(lost) : "v"(out), "n"(off));
-  return __uint_as_float((lost & 0xff800000u) | (~lost & __float_as_uint(x)));
+__device__ __forceinline__ void minus_inf_outside(f32x16& x, unsigned out) {
+  unsigned low;
+  asm("s_mov_b32 %0, 0xff800000" : "=s"(low));  // (a constant in the choice below would make it two instructions)
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    unsigned lost[4];
+    asm("v_bfe_i32 %0, %4, %5, 1\n\tv_bfe_i32 %1, %4, %6, 1\n\tv_bfe_i32 %2, %4, %7, 1\n\tv_bfe_i32 %3, %4, %8, 1"
+        : "=&v"(lost[0]), "=&v"(lost[1]), "=&v"(lost[2]), "=v"(lost[3])
+        : "v"(out), "n"(8 * g), "n"(8 * g + 1), "n"(8 * g + 2), "n"(8 * g + 3));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[4 * g + e] = __uint_as_float((lost[e] & low) | (~lost[e] & __float_as_uint(x[4 * g + e])));
+  }
 }
 
 // Element types of q, k, v, biases (unless fp32), gate and the output: bf16 or fp16.  The two differ in the MFMA and dot
@@ -1118,9 +1127,7 @@ void fwd_kernel(const KParams p) {
           const int hi = min(t_len - 1, max(p.dmax - rel, t_pfx - 1));
           const int lo = p.dmin - rel;
           if constexpr (!kDoc) {
-            const unsigned out = outside_word(lo, hi);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) s[kb][qb][i] = minus_inf_outside(s[kb][qb][i], out, 8 * (i / 4) + (i % 4));
+            minus_inf_outside(s[kb][qb], outside_word(lo, hi));
             continue;
           }
 #pragma unroll
