@@ -533,7 +533,8 @@ int64_t lds_bytes_for(const fl::Instance* in, const fl_attn_params* p) {
 int64_t prepass_lds_bytes(int64_t n_ktiles) { return n_ktiles * 20; }
 // Groups of waves a call is launched with, and the LDS of all of them
 int groups_for(const fl::Instance* in, const fl_attn_params* p) {
-  if (p->diff) return std::min(plan_diff(p).groups, in->max_groups);
+  // (a tile that has no form with the branches one after the other takes a group for each, whatever the plan prefers: FL_TILE may force it)
+  if (p->diff) return fl::diff_sequential(in->bn, in->nw) ? std::min(plan_diff(p).groups, in->max_groups) : in->max_groups;
   const int groups = std::min(plan_few(p, wanted_features(p)).groups, in->max_groups);
   return lds_bytes_for(in, p) + (int64_t)(groups - 1) * in->lds_fixed_bytes <= fl::kMaxLdsBytes ? groups : 1;
 }

@@ -39,23 +39,24 @@ constexpr int branches_lds_bytes() {
   return 0;
 }
 
+// Differential attention with the branches one after the other: 32-key tiles (both results and two tiles of 64 keys have no room in the
+// registers), 128 rows; the dump of attended pairs has no other form.
+constexpr bool diff_sequential(int bn, int nw) { return bn == 32 && nw == 4; }
+
 // Groups of waves the shape can be launched with (plan_few in api.hip): every instance compiled for them is that many kernels, so
-// only the default tiles have them.  Eight waves are two per SIMD, all the registers hold (four groups of four spill).
+// only the default tiles have them.  Eight waves are two per SIMD, all the registers hold (four groups of four spill).  Differential
+// attention (plan_diff): a group per branch, at head dim 128 in 64-key tiles only.
 constexpr int max_groups(int dqk, int dv, int rw, int bn, int nw, int ns, uint32_t feat) {
-  if (feat & F_DIFF) return feat & F_DUMP ? 1 : 2;
+  if (feat & F_DIFF) return feat & F_DUMP || (dqk == 128 && diff_sequential(bn, nw)) ? 1 : 2;
   if (dqk != dv || (dqk != 64 && dqk != 128) || rw != 32 || ns != 2 || (feat & ~(F_ALIBI | F_SOFTCAP | F_DOC))) return 1;
   if (nw == 2) return dqk == 64 ? 4 : 2;
   return nw == 4 && bn == (dqk == 128 && (feat & F_DOC) ? 32 : 64) ? 2 : 1;
 }
 
-// Differential attention with the branches one after the other: 32-key tiles (both results and two tiles of 64 keys have no room in the
-// registers), 128 rows; the dump of attended pairs has no other form.
-constexpr bool diff_sequential(int bn, int nw) { return bn == 32 && nw == 4; }
-
 template <int DQK, int DV, int RW, int BN, int NW, int NS, uint32_t FEAT, class E>
 hipError_t launch_fwd_groups(const KParams& kp, int groups, int grid, int lds_bytes, hipStream_t stream) {
   if constexpr ((FEAT & F_DIFF) != 0) {
-    if constexpr (!(FEAT & F_DUMP))
+    if constexpr (max_groups(DQK, DV, RW, BN, NW, NS, FEAT) == 2)
       if (groups == 2) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E, 2>>(kp, grid, lds_bytes, stream);
     if constexpr (diff_sequential(BN, NW))
       if (groups == 1) return launch_fwd<FwdTraits<DQK, DV, RW, BN, NW, FEAT, NS, E>>(kp, grid, lds_bytes, stream);

@@ -1,6 +1,10 @@
 """Differential attention: a group of waves per softmax branch, in workgroups of 64 and 128 rows, or the branches one after the other
 (plan_diff in csrc/api.hip), against fp64 at the edges of the tiles."""
 import ctypes as C
+import os
+import subprocess
+import sys
+from pathlib import Path
 
 import pytest
 import torch
@@ -29,6 +33,22 @@ def test_which_calls_take_which_workgroups():
     assert _shape(16, 16, 200, 64, NONE) == (128, 32, 1) and _shape(16, 16, 200, 64, CAUSAL) == (64, 64, 2)
     assert _shape(4, 16, 4096, 64, SLIDING) == (64, 64, 2) and _shape(4, 16, 4096, 128, SLIDING) == (128, 32, 1)
     assert _shape(16, 16, 256, 128, CAUSAL) == (128, 32, 1) and _shape(2, 16, 1000, 128, CAUSAL) == (128, 64, 2)
+
+
+@pytest.mark.parametrize("tile,shapes", [
+    # tiles without a form for the branches one after the other take a group for each, also where the rule prefers one group ...
+    ("32x64x4x2", {(4, 16, 4096, 128, SLIDING): (128, 64, 2), (16, 16, 200, 64, NONE): (128, 64, 2)}),
+    ("32x64x2x2", {(16, 16, 200, 64, NONE): (64, 64, 2)}),
+    # ... and the 32-key tile of head dim 128 has no form with two
+    ("32x32x4x2", {(2, 16, 1000, 128, CAUSAL): (128, 32, 1), (16, 16, 200, 64, NONE): (128, 32, 1), (2, 16, 1000, 64, CAUSAL): (128, 32, 2)}),
+])
+def test_a_forced_tile_is_planned_with_groups_that_it_has(tile, shapes):
+    # (the knob is read once per process)
+    script = "from tests.test_differential_branches import _shape\nprint([_shape(*s) for s in %r])" % (list(shapes),)
+    env = dict(os.environ, FL_TILE=tile)
+    got = subprocess.run([sys.executable, "-c", script], env=env, cwd=Path(__file__).parent.parent, capture_output=True, text=True, timeout=300)
+    assert got.returncode == 0, got.stderr
+    assert got.stdout.splitlines()[-1] == str(list(shapes.values()))
 
 
 @pytest.mark.gpu
