@@ -48,12 +48,19 @@ static __global__ void doc_table_kernel(const int64_t* ids, int64_t ids_stride, 
 // in the order is found; a thread per key tile classifies it for every wave; the non-empty entries are compacted.
 //
 // The order: the query tiles of a batch row by falling length of their tile lists (ties by falling index), so that the workgroups still running
-// when the grid drains are short ones whatever the document layout.  Every workgroup works out the lengths of all query tiles, by a
-// binary search each where the ids are sorted, and writes its own place: a second launch for it was 5 of the 15 us of the pre-pass (16384
-// ids, 16 heads, us for the forward with its pre-pass: 139.9 -> 136.3).  The lengths count the key tiles whose range meets the whole query tile's; any order
-// gives the same results.  Unsorted ids are counted pair by pair, up to kOrderPairs, beyond that the order is that of the index.
+// when the grid drains are short ones whatever the document layout.  ORDERS: every workgroup works out the lengths of all query tiles, by a
+// binary search each where the ids are sorted and pair by pair where they are not, and writes its own place: a second launch for it was 5 of
+// the 15 us of the pre-pass (16384 ids, 16 heads, us for the forward with its pre-pass: 139.9 -> 136.3).  The lengths count the key tiles whose
+// range meets the whole query tile's; any order gives the same results.  Without ORDERS doc_order_kernel follows.
+//
+// ORDERS pays while all workgroups run at once (doc_orders): a compute unit holds one, and every one of them reads the ids of all key tiles, not
+// only those up to its diagonal, and looks at all pairs of tiles where the ids are unsorted.  us, two launches -> one, documents of 64 to 512 unless
+// said, head dim 64: 1 x 16 x 8192 64.3 -> 63.0, 1 x 16 x 16384 (to 2048) 108 -> 103, 1 x 8 x 32768 83.0 -> 76.3, unmasked 101 -> 94, ids
+// unsorted 770 -> 778; head dim 128, 1 x 8 x 32768 113 -> 106, unsorted 1034 -> 1055.  Beyond: 40000 (313 workgroups) 104 -> 116, 65536 119 -> 130,
+// unsorted 1538 -> 1657, 262144 656 -> 1063; 6 x 8 x 8192 97 -> 101.  Few query tiles per row, whose order is soon found: 8 x 16 x 2048, head dim
+// 128, 85.0 -> 86.6.
 constexpr int kDocWaves = 4;  // waves of the forward that a query tile is classified for, at most
-constexpr int64_t kOrderPairs = 1 << 18;
+template <bool ORDERS>
 static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* ids, int64_t ids_stride, int L, int mask_kind,
                                                                 int bm, int rw, int bn, int n_qtiles, int nk, int list_stride,
                                                                 uint32_t* lists, int32_t* order) {
@@ -75,12 +82,14 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
   const int t_end = causal ? min(nk, (min(q0 + bm, L) - 1) / bn + 1) : nk;
   const int nj = (bn + 63) / 64;  // loads per lane that cover one tile's ids
   if (tid < 2) few[tid] = 0;
-  const int turn = blockIdx.x / 8;  // (where a workgroup begins: all of an XCD's would ask for the same lines at the same time)
-  for (int t0 = wave; t0 < nk || t0 == wave; t0 += kWaves * kBatch) {
+  const int turn = ORDERS ? blockIdx.x / 8 : 0;  // (where a workgroup begins: all of an XCD's would ask for the same lines at the same time)
+  const int n_read = ORDERS ? nk : t_end;
+  for (int t0 = wave; t0 < n_read || t0 == wave; t0 += kWaves * kBatch) {
     int64_t lo[kBatch], hi[kBatch];
+    auto tile = [&](int u) FL_INLINE { return t0 + kWaves * ((u + turn) % kBatch); };
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const int k0 = min(t0 + kWaves * ((u + turn) % kBatch), nk - 1) * bn;
+      const int k0 = min(tile(u), n_read - 1) * bn;
       lo[u] = hi[u] = idb[min(k0 + lane % bn, L - 1)];
       for (int j = 1; j < nj; ++j) {
         const int64_t x = idb[min(k0 + j * 64 + lane, L - 1)];
@@ -96,89 +105,103 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
         qrange[2 * wave + 1] = mx;
       }
     }
-    // lane u keeps tile u's range: the first id where all are the same, the others are reduced one by one (reduced as they come, the
-    // sixteen were 3 us)
-    uint32_t mixed = 0;
-    int64_t mn = 0, mx = 0;
+    if constexpr (ORDERS) {
+      // lane u keeps tile u's range: the first id where all are the same, the others are reduced one by one (reduced as they come, the
+      // sixteen were 3 us)
+      uint32_t mixed = 0;
+      int64_t mn = 0, mx = 0;
 #pragma unroll
-    for (int u = 0; u < kBatch; ++u) {
-      const int64_t first = uniform_i64(lo[u]);
-      if (__builtin_amdgcn_ballot_w64(lo[u] != first || hi[u] != first) != 0) mixed |= 1u << u;
-      mn = lane == u ? first : mn;
-    }
-    mx = mn;
-#pragma unroll 1
-    for (; mixed != 0; mixed &= mixed - 1) {
-      const int which = (int)__builtin_ctz(mixed);
-      int64_t x = lo[0], y = hi[0];
-#pragma unroll
-      for (int u = 1; u < kBatch; ++u) {
-        x = which == u ? lo[u] : x;
-        y = which == u ? hi[u] : y;
+      for (int u = 0; u < kBatch; ++u) {
+        const int64_t first = uniform_i64(lo[u]);
+        if (__builtin_amdgcn_ballot_w64(lo[u] != first || hi[u] != first) != 0 && tile(u) < n_read) mixed |= 1u << u;
+        mn = lane == u ? first : mn;
       }
-      int64_t least, most, unused;
-      wave_id_range(x, least, most);
-      if (nj > 1) wave_id_range(y, unused, most);
-      mn = lane == which ? least : mn;
-      mx = lane == which ? most : mx;
-    }
-    const int t = t0 + kWaves * ((lane + turn) % kBatch);
-    if (lane < kBatch && t < nk) {
-      krange[2 * t] = mn;
-      krange[2 * t + 1] = mx;
+      mx = mn;
+#pragma unroll 1
+      for (; mixed != 0; mixed &= mixed - 1) {
+        const int which = (int)__builtin_ctz(mixed);
+        int64_t x = lo[0], y = hi[0];
+#pragma unroll
+        for (int u = 1; u < kBatch; ++u) {
+          x = which == u ? lo[u] : x;
+          y = which == u ? hi[u] : y;
+        }
+        int64_t least, most, unused;
+        wave_id_range(x, least, most);
+        if (nj > 1) wave_id_range(y, unused, most);
+        mn = lane == which ? least : mn;
+        mx = lane == which ? most : mx;
+      }
+      if (lane < kBatch && tile(lane) < n_read) {
+        krange[2 * tile(lane)] = mn;
+        krange[2 * tile(lane) + 1] = mx;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        if (tile(u) >= n_read) break;
+        int64_t mn, mx, unused;
+        wave_id_range(lo[u], mn, mx);
+        if (nj > 1) wave_id_range(hi[u], unused, mx);
+        if (lane == 0) {
+          krange[2 * tile(u)] = mn;
+          krange[2 * tile(u) + 1] = mx;
+        }
+      }
     }
   }
   __syncthreads();
   // ---- this query tile's place
-  {
-    bool falls = false;
-    for (int t = tid; t + 1 < nk; t += 1024) falls = falls || krange[2 * t + 1] > krange[2 * t + 2];
-    if (__builtin_amdgcn_ballot_w64(falls) != 0 && lane == 0) few[0] = 1;
-    for (int j = tid; j < n_qtiles; j += 1024) tl[j] = 0;
-  }
-  __syncthreads();
-  const bool sorted = few[0] == 0, counted = !sorted && (int64_t)n_qtiles * nk <= kOrderPairs;
-  auto first_tile = [&](int j) FL_INLINE { return min(j * bm / bn, nk - 1); };  // key tiles that hold the rows of query tile j
-  auto last_tile = [&](int j) FL_INLINE { return min((min((j + 1) * bm, L) - 1) / bn, nk - 1); };
-  if (counted) {
-    for (int j0 = 0; j0 < n_qtiles; j0 += 64) {
-      const int j = min(j0 + lane, n_qtiles - 1), last = last_tile(j);
-      int64_t mn = krange[2 * first_tile(j)], mx = krange[2 * first_tile(j) + 1];
-      for (int t = first_tile(j) + 1; t <= last; ++t) {
-        mn = krange[2 * t] < mn ? krange[2 * t] : mn;
-        mx = krange[2 * t + 1] > mx ? krange[2 * t + 1] : mx;
-      }
-      uint32_t count = 0;
-      for (int t = wave; t < nk; t += kWaves) count += krange[2 * t + 1] >= mn && krange[2 * t] <= mx && (!causal || t <= last);
-      if (j0 + lane < n_qtiles) atomicAdd(&tl[j], count);
+  if constexpr (ORDERS) {
+    {
+      bool falls = false;
+      for (int t = tid; t + 1 < nk; t += 1024) falls = falls || krange[2 * t + 1] > krange[2 * t + 2];
+      if (__builtin_amdgcn_ballot_w64(falls) != 0 && lane == 0) few[0] = 1;
+      for (int j = tid; j < n_qtiles; j += 1024) tl[j] = 0;
     }
     __syncthreads();
-  }
-  auto length = [&](int j) FL_INLINE -> int {
-    if (counted) return (int)tl[j];
-    if (!sorted) return 0;
-    // first tile whose range reaches the query tile's smallest id; last one whose range begins at or below its largest
-    const int64_t mn = krange[2 * first_tile(j)], mx = krange[2 * last_tile(j) + 1];
-    int lo = 0, hi = first_tile(j);
-    while (lo < hi) {
-      const int mid = (lo + hi) / 2;
-      if (krange[2 * mid + 1] >= mn) hi = mid; else lo = mid + 1;
-    }
-    int last = last_tile(j);
-    if (!causal) {
-      int end = nk - 1;
-      while (last < end) {
-        const int mid = (last + end + 1) / 2;
-        if (krange[2 * mid] <= mx) last = mid; else end = mid - 1;
+    const bool sorted = few[0] == 0;
+    auto first_tile = [&](int j) FL_INLINE { return min(j * bm / bn, nk - 1); };  // key tiles that hold the rows of query tile j
+    auto last_tile = [&](int j) FL_INLINE { return min((min((j + 1) * bm, L) - 1) / bn, nk - 1); };
+    if (!sorted) {
+      for (int j0 = 0; j0 < n_qtiles; j0 += 64) {
+        const int j = min(j0 + lane, n_qtiles - 1), last = last_tile(j);
+        int64_t mn = krange[2 * first_tile(j)], mx = krange[2 * first_tile(j) + 1];
+        for (int t = first_tile(j) + 1; t <= last; ++t) {
+          mn = krange[2 * t] < mn ? krange[2 * t] : mn;
+          mx = krange[2 * t + 1] > mx ? krange[2 * t + 1] : mx;
+        }
+        uint32_t count = 0;
+        for (int t = wave; t < nk; t += kWaves) count += krange[2 * t + 1] >= mn && krange[2 * t] <= mx && (!causal || t <= last);
+        if (j0 + lane < n_qtiles) atomicAdd(&tl[j], count);
       }
+      __syncthreads();
     }
-    return last - lo + 1;
-  };
-  // (the last waves first: the first ones have the entries)
-  for (int j0 = (kWaves - 1 - wave) * 64; j0 < n_qtiles; j0 += 1024) {
-    const int mine = length(qt), j = j0 + lane, len = length(min(j, n_qtiles - 1));
-    const uint64_t before = __builtin_amdgcn_ballot_w64(j < n_qtiles && (len > mine || (len == mine && j > qt)));
-    if (lane == 0 && before != 0) atomicAdd(&few[1], (uint32_t)__builtin_popcountll(before));
+    auto length = [&](int j) FL_INLINE -> int {
+      if (!sorted) return (int)tl[j];
+      // first tile whose range reaches the query tile's smallest id; last one whose range begins at or below its largest
+      const int64_t mn = krange[2 * first_tile(j)], mx = krange[2 * last_tile(j) + 1];
+      int lo = 0, hi = first_tile(j);
+      while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (krange[2 * mid + 1] >= mn) hi = mid; else lo = mid + 1;
+      }
+      int last = last_tile(j);
+      if (!causal) {
+        int end = nk - 1;
+        while (last < end) {
+          const int mid = (last + end + 1) / 2;
+          if (krange[2 * mid] <= mx) last = mid; else end = mid - 1;
+        }
+      }
+      return last - lo + 1;
+    };
+    // (the last waves first: the first ones have the entries)
+    for (int j0 = (kWaves - 1 - wave) * 64; j0 < n_qtiles; j0 += 1024) {
+      const int mine = length(qt), j = j0 + lane, len = length(min(j, n_qtiles - 1));
+      const uint64_t before = __builtin_amdgcn_ballot_w64(j < n_qtiles && (len > mine || (len == mine && j > qt)));
+      if (lane == 0 && before != 0) atomicAdd(&few[1], (uint32_t)__builtin_popcountll(before));
+    }
   }
   // ---- the list
   auto entry_of = [&](int t) FL_INLINE -> uint32_t {
@@ -200,13 +223,13 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
     return (c << 16) | (unsigned)t;
   };
   uint32_t* out = lists + (int64_t)blockIdx.x * list_stride;
-  if (t_end <= 1024) {  // an entry per thread
+  if (ORDERS || t_end <= 1024) {  // an entry per thread
     const uint32_t e = tid < t_end ? entry_of(tid) : 0u;
     const bool keep = (e >> 16) != 0;
     const uint64_t m = __builtin_amdgcn_ballot_w64(keep);
     if (lane == 0) kept[wave] = (uint16_t)__builtin_popcountll(m);
     __syncthreads();
-    if (tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
+    if (ORDERS && tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
     uint32_t before = 0, all = 0;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
@@ -218,8 +241,6 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
     if (tid == 0) out[0] = all;
     return;
   }
-  __syncthreads();  // (the counts in tl have been read)
-  if (tid == 0) order[(int64_t)b * n_qtiles + few[1]] = qt;
   for (int t = tid; t < t_end; t += 1024) tl[t] = entry_of(t);
   __syncthreads();
   if (wave == 0) {
@@ -234,6 +255,23 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
       count += __builtin_popcountll(m);
     }
     if (lane == 0) out[0] = (uint32_t)count;
+  }
+}
+
+// Whether the lists' launch finds the order too (see above).  It has a thread per entry, and room for a count per key tile.
+static bool doc_orders(int64_t B, int64_t n_qtiles, int64_t nk) { return n_qtiles >= 64 && B * n_qtiles <= 256 && nk <= 1024 && n_qtiles <= nk; }
+
+// The same order from the lengths of the lists, a workgroup per batch row: counts for every query tile how many come before it.
+static __global__ __launch_bounds__(1024) void doc_order_kernel(const uint32_t* lists, int list_stride, int n_qtiles, int32_t* order) {
+  extern __shared__ uint32_t lengths[];  // n_qtiles words
+  const uint32_t* of_row = lists + (int64_t)blockIdx.x * n_qtiles * list_stride;
+  for (int i = threadIdx.x; i < n_qtiles; i += 1024) lengths[i] = of_row[(int64_t)i * list_stride];
+  __syncthreads();
+  for (int i = threadIdx.x; i < n_qtiles; i += 1024) {
+    const uint32_t mine = lengths[i];
+    int place = 0;
+    for (int j = 0; j < n_qtiles; ++j) place += lengths[j] > mine || (lengths[j] == mine && j > i);
+    order[(int64_t)blockIdx.x * n_qtiles + place] = i;
   }
 }
 
@@ -1310,14 +1348,17 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
       kp.doc_own = 1;
       lds += fl::kOwnListBytes;
     } else if (!(p->flags & FL_FLAG_DOC_PREPARED)) {
-      static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fl::doc_lists_kernel),
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, fl::kMaxLdsBytes - 128);
-      if (attr != hipSuccess) return fail((int)attr, "doc_lists_kernel: %s", hipGetErrorString(attr));
       if (in->nw > fl::kDocWaves) return fail(FL_ERR_UNSUPPORTED, "%s: more waves than the document lists have classes for", in->name);
-      hipLaunchKernelGGL(fl::doc_lists_kernel, dim3(p->B * kp.n_qtiles), dim3(1024), (size_t)prepass_lds_bytes(kp.n_ktiles), stream,
+      const bool orders = fl::doc_orders(p->B, kp.n_qtiles, kp.n_ktiles);
+      const auto make_lists = orders ? &fl::doc_lists_kernel<true> : &fl::doc_lists_kernel<false>;
+      static const hipError_t attrs[2] = {
+          hipFuncSetAttribute(reinterpret_cast<const void*>(&fl::doc_lists_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, fl::kMaxLdsBytes - 128),
+          hipFuncSetAttribute(reinterpret_cast<const void*>(&fl::doc_lists_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, fl::kMaxLdsBytes - 128)};
+      if (attrs[orders] != hipSuccess) return fail((int)attrs[orders], "doc_lists_kernel: %s", hipGetErrorString(attrs[orders]));
+      hipLaunchKernelGGL(make_lists, dim3(p->B * kp.n_qtiles), dim3(1024), (size_t)prepass_lds_bytes(kp.n_ktiles), stream,
                          p->doc_ids, p->doc_stride, p->Lk, p->mask_kind, bm, in->rw, in->bn, kp.n_qtiles, kp.n_ktiles,
                          (int)d.list_stride, lists, order);
-      const hipError_t e = hipGetLastError();
+      hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, "doc_lists_kernel launch failed: %s", hipGetErrorString(e));
     }
     kp.doc_lists = lists;
