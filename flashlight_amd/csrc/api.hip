@@ -1360,6 +1360,11 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
                          (int)d.list_stride, lists, order);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return fail((int)e, "doc_lists_kernel launch failed: %s", hipGetErrorString(e));
+      if (!orders) {
+        hipLaunchKernelGGL(fl::doc_order_kernel, dim3(p->B), dim3(1024), (size_t)kp.n_qtiles * 4, stream, lists, (int)d.list_stride, kp.n_qtiles, order);
+        e = hipGetLastError();
+        if (e != hipSuccess) return fail((int)e, "doc_order_kernel launch failed: %s", hipGetErrorString(e));
+      }
     }
     kp.doc_lists = lists;
     kp.doc_list_stride = (int)d.list_stride;
