@@ -1502,22 +1502,47 @@ BwdPlan plan_bwd(const fl_attn_params* p) {
 }
 
 // dK and dV, a launch of their own at head dim 128 without score modifications: 256 keys per workgroup instead of 128, one workgroup of
-// eight waves per compute unit either way.  A round takes twice as long, so the last one must not be far from full (all of it under masks of
-// growing length, whose longest walk is twice the average), unless there are several; and few of the keys' places may be empty.
-// us, both roles, 128 -> 256 keys: causal, 16 heads of 4096 (256 tiles of 256 keys) 259 -> 303, 20 (320) 368 -> 432, 24 (384) 365 -> 365, 2 x 16 (512)
-// 473 -> 452, 4 x 16 922 -> 890, 16 x 32 of 512 (1024) 270 -> 253, 13 x 16 of 700 (624) 178 -> 180; unmasked, 16 of 4096 436 -> 420, 24 648 -> 679;
-// windows of 100, 8 x 16 of 4096, 515 -> 487; a prefix, 8 x 16 of 1500, 352 -> 325.
+// eight waves per compute unit either way, so a round takes twice as long and there are half as many.  us, both roles, 128 -> 256 keys:
+// A last round that is far from full costs more of them: no mask, 16 heads of 4096 (256 tiles of 256 keys) 428 -> 411, 24 (384) 648 -> 679 (below
+// 256 tiles both roles share a launch, of 128 keys); from 1024 tiles on there are rounds enough, 128 heads of 2048 890 -> 850, 129 968 -> 965, 96
+// of 3000 (1152) 1398 -> 1381, but 43 of 6000 (1032) 2400 -> 2530.  Windows of 100, 8 x 16 of 4096, 515 -> 487; of 256, 129 of 2048 320 -> 303; of
+// more than half the keys, 32 of 4096 424 -> 440, of all of them 492 -> 549, 129 of 2048 833 -> 859, 121 of 1000 240 -> 217.  Few of the keys'
+// places may be empty.
+// Masks of growing length, whose longest walk is twice the average, want more rounds.  Where the heads divide by the 8 XCDs, causal, 16 of 4096
+// 259 -> 303, 32 (512) 464 -> 443, 64 901 -> 863, 104 of 3000 897 -> 906, a prefix, 8 x 16 of 1500, 352 -> 325; with one tile per head full rounds
+// only, 1024 of 256 225 -> 213, 1088 233 -> 236.  Where they do not, and tiles go round the XCDs, causal, 121 of 1000 (484) 220 -> 199, but 81
+// of 1536 (486) 254 -> 261, 63 of 3000 (756) 620 -> 643; from 1000 tiles on 0.92 to 1.0 of the time at 1100 to 7000 keys (0.93 to 1.02 under a
+// prefix), but for tiles per head that are a multiple of 8: 129 of 2048 628 -> 735, 65 of 4096 1053 -> 1079, 43 of 6000 1386 -> 1468.
 bool wide_dkv(const fl_attn_params* p) {
-  const int64_t narrow = (p->Lk + 127) / 128, wide = (p->Lk + 255) / 256, tiles = (int64_t)p->B * p->Hkv * wide;
+  const int64_t narrow = (p->Lk + 127) / 128, wide = (p->Lk + 255) / 256, heads = (int64_t)p->B * p->Hkv, tiles = heads * wide, last = tiles % 256;
+  if (p->Dqk != 128 || p->alibi_heads > 0 || p->softcap > 0.f || p->bias[0] || p->bias[1] || is_doc(p->mask_kind) || p->dropout_threshold) return false;
   if (2 * wide > narrow && narrow < 16) return false;
-  if (tiles >= 1024) return true;
-  return tiles > (p->mask_kind == FL_MASK_NONE ? 224 : 480) && (tiles % 256 == 0 || tiles % 256 > 224);
+  const bool full = last == 0 || last > 224, window = p->mask_kind == FL_MASK_SLIDING;
+  if (p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM) {
+    if (heads % 8) return (tiles >= 1000 ? wide % 8 != 0 : p->Lk <= 1024) && (tiles >= 1024 || (tiles > 480 && full));
+    return (tiles >= 1024 && wide > 1) || (tiles > 480 && full);
+  }
+  if (window && 2 * (int64_t)p->window > p->Lk && p->Lk > 1536) return false;
+  if (tiles >= 1024) return window || p->Lk <= 4096 || full || last > 64;
+  return tiles > (window ? 480 : 0) && full;
 }
 }  // namespace
 
 uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p) {
   if (!p || p->B <= 0 || p->Hkv <= 0 || p->Hq < p->Hkv || p->Lq <= 0 || p->Lk <= 0 || p->Dqk <= 0) return 0;
   return plan_bwd(p).bytes;
+}
+
+int fl_attn_bwd_plan(const fl_attn_params* p, int64_t out[4]) {
+  if (!p || !out) return fail(FL_ERR_NULL, "%s is null", p ? "out" : "params");
+  if (p->B <= 0 || p->Hkv <= 0 || p->Hq < p->Hkv || p->Hq % p->Hkv || p->Lq <= 0 || p->Lk <= 0 || p->Dqk <= 0)
+    return fail(FL_ERR_SHAPE, "sizes must be positive, query heads a multiple of key/value heads");
+  const BwdPlan x = plan_bwd(p);
+  out[0] = x.both ? 1 : 2;
+  out[1] = x.dq;
+  out[2] = x.dkv;
+  out[3] = !x.both && wide_dkv(p) ? 256 : 128;
+  return 0;
 }
 
 // `planned`: sums may be taken in another order than one workgroup per tile and role takes them in, whatever else the call holds
@@ -1598,7 +1623,7 @@ static int launch_gradients(const fl_attn_bwd_params* b, bool planned, void* scr
   if (plan.dkv > 1) bp.part = bp.part_dq + plan.dq_bytes / sizeof(float);
   bp.splits_dq = plan.dq;
   bp.splits = plan.dkv;
-  bp.dkv_own = planned && !plan.both && in->d == 128 && in->feat == 0 && wide_dkv(p) ? 256 : 128;
+  bp.dkv_own = planned && !plan.both && wide_dkv(p) ? 256 : 128;
   bp.head_group = p->mask_kind == FL_MASK_CAUSAL || p->mask_kind == FL_MASK_PREFIX_LM || p->mask_kind == FL_MASK_DOCUMENT_CAUSAL ? 4 : 1;
   bp.by_head_group = fl::Div::by(bp.head_group);
   bp.by_group = fl::Div::by(bp.group);

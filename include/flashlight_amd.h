@@ -261,6 +261,10 @@ int fl_attn_bwd(const fl_attn_bwd_params* p, void* stream);
 int fl_attn_bwd_split(const fl_attn_bwd_params* p, void* scratch, uint64_t scratch_bytes, void* stream);
 /* Bytes of scratch fl_attn_bwd_split can use for the gradients of the forward call *p; 0: none.  Host only. */
 uint64_t fl_attn_bwd_split_bytes(const fl_attn_params* p);
+/* How fl_attn_bwd_split launches the gradients of the forward call *p, given that scratch: out[0]=1 when dQ, dK and dV are formed
+ * in one launch, 2 when dQ is formed ahead of dK and dV; out[1]=workgroups that share a tile of dQ, out[2]=of dK and dV;
+ * out[3]=keys per workgroup of dK and dV.  Host only; the pointers of *p need not be set, apart from which of the biases are. */
+int fl_attn_bwd_plan(const fl_attn_params* p, int64_t out[4]);
 
 /* fl_attn_bwd for callers that cannot allocate device memory (code under HIP graph capture, tight training loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments and results as fl_attn_bwd,
