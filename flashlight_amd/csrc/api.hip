@@ -466,12 +466,30 @@ DiffPlan plan_diff(const fl_attn_params* p) {
   const int64_t visited = window ? std::min<int64_t>(p->Lk, (int64_t)p->window + 128) : p->Lk;
   x.waves = 4;
   x.keys = 32;
-  // Short walks whose workgroups of 128 rows fill rounds of two per compute unit: one start and one store for both branches.  us, one after
-  // the other / a group each: head dim 64, unmasked, 16 x 16 of 160 14.7 / 17.2, of 256 22.4 / 23.5, of 450 61.0 / 65.7, of 512 65.0 / 65.7, but of
-  // 300 (768 tiles) 39.1 / 34.4; causal of 200 20.9 / 19.4; head dim 128, causal of 256 57.9 / 60.6, of 512 145 / 134, unmasked of 512 170 / 174.
+  // Short walks of calls that fill the compute units: one start and one store for both branches, and two workgroups of 128 rows per compute
+  // unit.  us, one after the other / a group each.
+  // Head dim 64 takes 64 rows with groups, which loses where the last 128 rows have none to save: unmasked, 16 x 16 of 160 14.7 / 17.2, of
+  // 450 61.0 / 65.7, of 512 65.0 / 65.7, 896 tiles of 200 1 : 1.13, but 16 x 16 of 300 39.1 / 34.4, 640 tiles of 256 1 : 0.86, of 512 1 : 0.79; full
+  // rounds of 600 and 850 1 : 1.02 to 1.04, of 1000 1 : 0.92 to 1.0; heads that do not divide by the 8 XCDs, whose two halves of 128 rows then read the keys on two of them, 651
+  // of 200 1 : 1.19, 325 of 512 1 : 1.19, 261 of 600 1 : 1.07, 101 of 1000 1 : 0.90; masks of growing length, 1 : 0.7 to 0.95 from 200 on.
+  // Head dim 128, of 200 1 : 1.06 to 1.3 under any mask, of 256 1 : 1.0 to 1.2; unmasked, of 384 1 : 1.07 to 1.16, of 600 1 : 1.04 to 1.12, of
+  // 850 1 : 1.02 to 1.05, but a start into a second round of two (512 to 768 tiles) 1 : 0.85 to 1.0, into a third, of 700, 1 : 0.93; causal, of 300
+  // 1 : 1.0 to 1.11, of 384 1 : 0.8 to 1.04, of 512 1 : 0.8 to 1.0; heads that do not divide by 8, of 450 1 : 0.97 to 1.15, 187 to 429 of 850
+  // 1 : 1.06 to 1.15.
   // Windows, 4 x 16 of 4096, head dim 128: of 256 150 / 171, of 1100 336 / 325 (at head dim 64 with 64 rows: of 256 123 / 96, of 1500 322 / 283).
-  const bool full_rounds = tiles > 256 && (tiles % 512 == 0 || tiles % 512 > 384);
-  if (window ? !narrow && visited <= 1024 : full_rounds && visited <= (!growing ? 512 : narrow ? 0 : 256)) return x;
+  const int64_t last = tiles % 512;  // of the last round of two per compute unit
+  const bool odd = (int64_t)p->B * p->Hq % 8 != 0, full = last == 0 || last > 384, no_rows_saved = p->Lq % 128 == 0 || p->Lq % 128 > 64;
+  bool sequential = false;
+  if (window) sequential = !narrow && visited <= 1024;
+  else if (tiles <= 256) sequential = false;
+  else if (narrow && !growing)
+    sequential = (full && visited <= (no_rows_saved ? 900 : 512)) ||
+                 (no_rows_saved && ((visited <= 256 && last > 256) || (odd && visited <= 640 && !(visited > 512 && last > 0 && last <= 136 && tiles <= 768))));
+  else if (!narrow && growing)
+    sequential = visited <= 256 || (visited <= 300 && tiles > 300) || (odd && ((visited > 384 && visited <= 450) || (visited > 768 && visited <= 896 && tiles >= 1300)));
+  else if (!narrow)
+    sequential = visited <= 256 || (visited <= 900 && !(last > 0 && last <= 256 && (tiles <= 768 || visited > 640)));
+  if (sequential) return x;
   x.groups = 2;
   // Up to 16 tiles of 128 rows keep 32 keys, the shape that the dump of attended pairs has and is compared in at every edge (2 heads of 256:
   // 18.3 -> 13.9, where 64 rows and keys take 8.5).

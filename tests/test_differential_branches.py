@@ -35,6 +35,20 @@ def test_which_calls_take_which_workgroups():
     assert _shape(16, 16, 256, 128, CAUSAL) == (128, 32, 1) and _shape(2, 16, 1000, 128, CAUSAL) == (128, 64, 2)
 
 
+def test_short_walks_of_many_workgroups():
+    """Where two workgroups of 128 rows per compute unit are ahead of a group per branch."""
+    turns = (128, 32, 1)  # one branch after the other
+    for mask in (NONE, CAUSAL, PREFIX):
+        assert _shape(33, 32, 130, 128, mask) == turns and _shape(50, 16, 200, 128, mask) == turns and _shape(5, 16, 200, 128, mask) == (128, 64, 2)
+        assert _shape(5, 16, 1500, 128, mask) == (128, 64, 2)
+    assert _shape(20, 16, 600, 128, NONE) == turns and _shape(8, 16, 600, 128, NONE) == (128, 64, 2) and _shape(20, 16, 600, 128, CAUSAL) == (128, 64, 2)
+    assert _shape(1, 75, 450, 128, CAUSAL) == turns and _shape(1, 72, 450, 128, CAUSAL) == (128, 64, 2)
+    assert _shape(1, 251, 850, 128, PREFIX) == turns and _shape(1, 101, 850, 128, PREFIX) == (128, 64, 2)
+    assert _shape(1, 651, 200, 64, NONE) == turns and _shape(1, 448, 200, 64, NONE) == turns and _shape(1, 320, 256, 64, NONE) == (64, 64, 2)
+    assert _shape(1, 325, 512, 64, NONE) == turns and _shape(1, 325, 420, 64, NONE) == (64, 64, 2) and _shape(1, 325, 512, 64, CAUSAL) == (64, 64, 2)
+    assert _shape(1, 103, 600, 64, NONE) == (64, 64, 2) and _shape(1, 96, 600, 64, NONE) == turns
+
+
 @pytest.mark.parametrize("tile,shapes", [
     # tiles without a form for the branches one after the other take a group for each, also where the rule prefers one group ...
     ("32x64x4x2", {(4, 16, 4096, 128, SLIDING): (128, 64, 2), (16, 16, 200, 64, NONE): (128, 64, 2)}),
