@@ -864,6 +864,10 @@ int64_t chunks_of_entries(int64_t heads_and_groups, int64_t tiles, int per_cu, i
   return best;
 }
 
+// Whether a bias row may be what the accumulators of a product start from (the shared-bias stripe forward and gradients): times 1 / scale it
+// has to stay an ordinary number.  (A scale that has not been set yet is no reason against it.)
+bool row_starts_products(const fl_attn_params* p) { return !(p->scale > 0.f) || (p->scale >= 0x1p-100f && p->scale <= 0x1p100f); }
+
 // Whether *p (already validated) is a call the shared-bias stripe forward (stripe_kernel.h) takes.  Fills the kernel's parameters,
 // its wave count, and the number of workgroups and their LDS bytes.
 bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, int* waves, int64_t (&launch)[2]) {
@@ -881,7 +885,7 @@ bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, 
     else if (st[1] == 0 && st[2] == 0 && st[3] <= 0x7fffffff && ri < 0) ri = i;
     else return false;
   }
-  if (pi < 0) return false;
+  if (pi < 0 || (ri >= 0 && !row_starts_products(p))) return false;
   if (p->B % p->bias_batch_div[pi] != 0) return false;  // (workgroups walk whole groups of entries; the general kernel divides per entry)
   // Where the general kernel has to read the bias two bytes at a time (odd lengths, fp32), this one is three to five times sooner
   // (bf16, us: 414 x 4 x 494 x 494, head dim 32: 806 -> 201; 34 x 4 x 235 x 235, head dim 64: 43 -> 17; 28 x 4 x 106 x 106: 14 -> 6).  Where
@@ -1093,7 +1097,7 @@ bool plan_shared_bias_bwd(const fl_attn_params* p, SBScratch* out) {
     else if ((st[1] != 0 || p->Hq == 1) && (st[2] != 0 || p->Lq == 1) && (st[3] == 1 || p->Lk == 1) && x.dense < 0) x.dense = i;
     else return false;
   }
-  if (x.dense < 0) return false;
+  if (x.dense < 0 || (x.row >= 0 && !row_starts_products(p))) return false;
   // per-lane byte offsets inside one (batch entry, head) are 32-bit
   for (const int64_t* st : {p->q_strides, p->k_strides, p->v_strides, p->o_strides})
     if (st[2] < 0 || st[2] >= (1 << 20)) return false;

@@ -165,3 +165,42 @@ def test_layouts_partial_gradients_and_repetition():
     dq, = torch.autograd.grad(out.float().sum(), [q], create_graph=True)
     with pytest.raises(RuntimeError, match="not differentiable a second time"):
         dq.float().sum().backward()
+
+
+def test_scales_that_a_bias_row_cannot_be_divided_by():
+    """Bias rows start the products' accumulators, divided by the scale: where that is no ordinary number, another kernel takes the call."""
+    lib = _ffi.load_library()
+    lib.fl_attn_shared_bias_bwd_bytes.restype = C.c_uint64
+    out = (C.c_int64 * 8)()
+    for scale, taken in ((1e-39, False), (1e-31, False), (1e-29, True), (0.0, True), (1e29, True), (1e31, False), (3e38, False)):
+        for row in (False, True):
+            p = good_params(B=12, Hq=4, Hkv=4, L=101, D=32)
+            p.scale = scale
+            p.bias[0], p.bias_batch_div[0] = 0x60000, 6
+            p.bias_strides[0][:] = (4 * 101 * 101, 101 * 101, 101, 1)
+            if row:
+                p.bias[1], p.bias_batch_div[1] = 0x70000, 1
+                p.bias_strides[1][:] = (101, 0, 0, 1)
+            assert (lib.fl_attn_shared_bias_bwd_bytes(C.byref(p)) > 0) == (taken or not row), (scale, row)
+            if scale:
+                assert lib.fl_attn_plan(C.byref(p), out) == 0 and (out[6] == 2) == (taken or not row), (scale, row)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [101, 256])
+def test_a_tiny_scale_beside_a_bias_row(S):
+    """The products vanish: what is left are the weights of the biases alone, and their gradients."""
+    N, H, D = 6, 2, 32
+    g = torch.Generator().manual_seed(S)
+    q, k, v, dout = (torch.randn(N, H, S, D, generator=g).to(torch.bfloat16).to(DEV) for _ in range(4))
+    pair = torch.randn(1, H, S, S, generator=g).to(torch.bfloat16).to(DEV)
+    row = torch.where(torch.rand(N, 1, 1, S, generator=g) < 0.2, float("-inf"), torch.randn(N, 1, 1, S, generator=g)).to(torch.bfloat16).to(DEV)
+    leaves = [t.requires_grad_(True) for t in (q, k, v, pair)]
+    out = ops.dispatch(q, k, v, scale=1e-39, biases=[(pair, N), (row, 1)])
+    grads = torch.autograd.grad(out, leaves, dout)
+    exact = [v.detach().double().requires_grad_(True), pair.detach().double().requires_grad_(True)]
+    want = torch.matmul(torch.softmax(exact[1] + row.double(), -1), exact[0])
+    wgrads = torch.autograd.grad(want, exact, dout.double())
+    for name, a, b in zip(("out", "dv", "dbias"), (out, *grads[2:]), (want, *wgrads)):
+        assert ((a.double() - b).norm() / b.norm()).item() < 1e-2, name  # (weights, score gradients and results rounded to bf16)
+    assert all((t.abs() < 1e-30).all() for t in grads[:2])
