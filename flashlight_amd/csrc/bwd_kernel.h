@@ -187,6 +187,46 @@ struct BwdTraits {
   static constexpr bool EARLY_X2 = ROLE == ROLE_DQ && WIDE_X2;  // and its MFMAs issued right after those of S
 };
 
+// The order of a step (run_ordered): products X1 of every block of 32 streamed positions, X2 of every block, dV's (unless DQ), dS's, of TB
+// blocks with KS products each and DB columns of 32.  Behind product m the first weights(m) pairs of weights and gradients(m) pairs of score
+// gradients have been formed, eight pairs per block.
+template <bool DQ, int TB, int KS, int DB>
+struct OrderedStep {
+  static constexpr int X2 = TB * KS, VP = 2 * X2, KP = VP + (DQ ? 0 : 2 * TB * DB), M = KP + 2 * TB * DB;  // first of each kind, and their number
+  static constexpr int weights(int m) {
+    if (DQ && TB == 2) return m < 5 ? 0 : m < 9 ? 2 * (m - 4) : m < 16 ? m : 16;
+    return m < KS ? 0 : m < KS + 8 * TB ? m - KS : 8 * TB;
+  }
+  static constexpr int gradients(int m) {
+    if (DQ && TB == 2) return m < 13 ? 0 : m < 15 ? 3 * (m - 12) : m < 17 ? 8 : m < 20 ? 8 + 2 * (m - 16) : 16;
+    if (DQ) return m < VP - 1 ? 0 : m < VP + 3 ? m - VP + 5 : 8;
+    if (TB == 2) return m < VP + 5 ? 0 : m < VP + 12 ? 2 * (m - VP - 4) : 16;
+    return m < VP ? 0 : m < VP + 8 ? m - VP : 8;
+  }
+  // (unless DQ) which four rows' LSE are read in front of product m, into one of two places, or -1
+  static constexpr int lse_quad(int m) {
+    const int g = m - KS + 1;
+    return !DQ && g >= 0 && g % 2 == 0 && g / 2 < 4 * TB ? g / 2 : -1;
+  }
+  // Every weight behind its block's X1, with its LSE in place; every gradient behind its weight and its block's X2; every product of 16 positions
+  // behind their eight pairs; nothing left out.
+  static constexpr bool holds() {
+    if (TB == 1 ? KS != 8 || DB != 4 : TB != 2 || KS != 4 || DB != 2) return false;  // (the shapes that the places are written for)
+    if (weights(-1) != 0 || gradients(-1) != 0 || weights(M - 1) != 8 * TB || gradients(M - 1) != 8 * TB) return false;
+    int lse[2] = {-1, -1};
+    for (int m = 0; m < M; ++m) {
+      if (m >= KP ? gradients(m - 1) < 4 * ((m - KP) / DB) + 4 : m >= VP && weights(m - 1) < 4 * ((m - VP) / DB) + 4) return false;
+      if (lse_quad(m) >= 0) lse[lse_quad(m) % 2] = lse_quad(m);
+      if (weights(m) < weights(m - 1) || gradients(m) < gradients(m - 1) || gradients(m) > weights(m)) return false;
+      for (int w = weights(m - 1); w < weights(m); ++w)
+        if (m < (w / 8 + 1) * KS - 1 || (!DQ && lse[w / 2 % 2] != w / 2)) return false;
+      for (int w = gradients(m - 1); w < gradients(m); ++w)
+        if (m < X2 + (w / 8 + 1) * KS - 1) return false;
+    }
+    return true;
+  }
+};
+
 // One workgroup's share of the work of a role: workgroup `block` of tiles * splits.  SPLIT: several workgroups per owner tile
 // (one at run time is fine), compiled apart: with the second epilogue in it the dK/dV kernel at head dim 128 is 4 %
 // slower (another register allocation throughout).
@@ -544,24 +584,15 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   int slope_head = -1;
   float slope_l2 = 0.f;
   // The blocks of 32 streamed positions of a step with their instructions in a prescribed order (T::ORDERED, see there).  Products: X1 of
-  // every block, X2 of every block, (ROLE_DKV) dV's, dS's.  In front of product m stand the LDS reads of product m + AHEAD, behind it its
-  // share of the vector work: weights(m) pairs of weights and gradients(m) pairs of score gradients are formed by then.
+  // every block, X2 of every block, (ROLE_DKV) dV's, dS's (OrderedStep).  In front of product m stand the LDS reads of product m + AHEAD,
+  // behind it its share of the vector work.
   auto run_ordered = [&](auto tile, const int shead, const int slot, bool full, bool doc_uniform) FL_INLINE {  // (compiled only where it is called)
     const int t0 = tile * BT;
     const unsigned t1 = T::T1_OFF + slot * T::TBYTES, t2 = T::T2_OFF + slot * T::TBYTES;
-    constexpr int X2 = TB * KS, VP = 2 * X2, KP = VP + (kDQ ? 0 : 2 * TB * DB), M = KP + 2 * TB * DB;  // first of each kind, and their number
+    using Step = OrderedStep<kDQ, TB, KS, DB>;
+    constexpr int X2 = Step::X2, VP = Step::VP, KP = Step::KP, M = Step::M;
     constexpr int AHEAD = T::AHEAD, RING = AHEAD + 1;
-    auto weights = [](int m) constexpr {
-      if (kDQ && TB == 2) return m < 5 ? 0 : m < 9 ? 2 * (m - 4) : m < 16 ? m : 16;
-      return m < KS ? 0 : m < KS + 8 * TB ? m - KS : 8 * TB;
-    };
-    auto gradients = [](int m) constexpr {
-      if (kDQ && TB == 2) return m < 13 ? 0 : m < 15 ? 3 * (m - 12) : m < 17 ? 8 : m < 20 ? 8 + 2 * (m - 16) : 16;
-      if (kDQ) return m < VP - 1 ? 0 : m < VP + 3 ? m - VP + 5 : 8;
-      if (TB == 2) return m < VP + 5 ? 0 : m < VP + 12 ? 2 * (m - VP - 4) : 16;
-      return m < VP ? 0 : m < VP + 8 ? m - VP : 8;
-    };
-    static_assert(TB == 1 ? KS == 8 && DB == 4 : KS == 4 && DB == 2, "the places of the vector work");
+    static_assert(Step::holds(), "everything formed behind its products and ahead of those that take it");
     f32x16 x1[TB], x2[TB];
     ex8 fa[RING], fb[T::V_REGS ? 1 : RING];  // operands in flight
     f32x4 lse4[2];
@@ -610,8 +641,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
       constexpr int m = decltype(mt)::value;
       read(std::integral_constant<int, m + AHEAD>{});
       if constexpr (!kDQ) {  // the LSE of four rows, two products ahead of their weights (the place is free: of the last but one)
-        constexpr int g = m - KS + 1;
-        if constexpr (g >= 0 && g % 2 == 0 && g / 2 < 4 * TB) lse4[g / 2 % 2] = rows4(T::S1_OFF, g / 8, g / 2 % 4);
+        constexpr int q = Step::lse_quad(m);
+        if constexpr (q >= 0) lse4[q % 2] = rows4(T::S1_OFF, q / 4, q % 4);
       }
       if constexpr (m < X2) {
         if constexpr (kDQ || T::K_REGS) x1[m / KS] = mfma32(fa[m % RING], o1f[m % KS], x1[m / KS]);
@@ -627,7 +658,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         acc1[(m - KP) % DB] = mfma32(fa[m % RING], dsf[(m - KP) / DB], acc1[(m - KP) % DB]);
       }
 #pragma unroll
-      for (int w = weights(m - 1); w < weights(m); ++w) {
+      for (int w = Step::weights(m - 1); w < Step::weights(m); ++w) {
         const int sb = w / 8, sbase = t0 + 32 * (qh * TB + sb) + 4 * h;  // streamed position of register 0
         if (w % 8 == 0) {
           if constexpr (kAlibi) alibi0[sb] = slope_l2 * (float)(kDQ ? sbase - opos : opos - sbase);
@@ -668,7 +699,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
         }
       }
 #pragma unroll
-      for (int w = gradients(m - 1); w < gradients(m); ++w)
+      for (int w = Step::gradients(m - 1); w < Step::gradients(m); ++w)
 #pragma unroll
         for (int e = w % 8 * 2; e < w % 8 * 2 + 2; ++e) dsf[w / 8 * 2 + e / 8][e % 8] = (E)(x1[w / 8][e] * x2[w / 8][e]);
       __builtin_amdgcn_sched_barrier(0);
