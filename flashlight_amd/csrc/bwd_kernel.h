@@ -132,6 +132,14 @@ static_assert([]() constexpr {
   return true;
 }(), "one place per chunk");
 
+// The image with rows kept whole (TileLayout's two-way swizzle), read through TileOperands: T::WHOLE_ROWS
+template <int D>
+struct RowLayout {
+  static constexpr int CPR = D / 8;
+  __device__ static __forceinline__ int row_of(int id) { return id / CPR; }
+  __device__ static __forceinline__ int chunk_of(int id) { return TileLayout<D>::swz_kv(id / CPR, id % CPR); }
+};
+
 // SHARED_: the role as part of bwd_both_kernel, whose two roles have workgroups of one size.  WIDE_: 256 owner positions per workgroup
 // (ROLE_DKV at head dim 128, wide_dkv in api.hip): eight waves own 32 keys each, so that a streamed tile comes in once for twice as many
 // keys, K stays in registers and nothing is added up at the end.
@@ -162,6 +170,13 @@ struct BwdTraits {
   // matters (2 to 5 products); documents with ALiBi and a soft-cap spill.
   static constexpr bool ORDERED = ((FEAT_ & ~F_DOC) == 0 || (FEAT_ & ~(F_ALIBI | F_SOFTCAP)) == 0) && D_ >= 64;
   static constexpr int AHEAD = 3;
+  // Bias operands without documents: rows kept whole.  The compiler orders those steps, and does it worse with all reads at two addresses.
+  // us, blocks of 16 rows -> this: head dim 64, a bias row, 2 x 16 of 300 37.7 -> 36.4, dense 47.4 -> 46.4, dense, 3 x 7 of 1200 266 -> 262, 4 x 16 of
+  // 2048 1427 -> 1415; with ALiBi 484 -> 470, with dropout 942 -> 927; head dim 128, dense, 2 x 16 over 4 of 1000 243 -> 239, a row, 4 x 16 of 2048
+  // 954 -> 933, with dropout 1158 -> 1134; head dim 32, 43.3 -> 42.7.  Beside ALiBi or the soft-cap the addresses spill at head dim 128 (3 x 7 of
+  // 1200: 169 against 183; head dim 32, 2048: 431 against 440), and documents lose (a row, 2 x 16 over 4 of 1000: head dim 64 134 against
+  // 142, 128 165 against 175).
+  static constexpr bool WHOLE_ROWS = (FEAT_ & F_BIAS) && !(FEAT_ & F_DOC) && (D_ == 64 || !(FEAT_ & (F_ALIBI | F_SOFTCAP)));
   // ROLE_DKV: the owner's K and V rows as operands in registers, where there is room, instead of in LDS
   static constexpr bool K_REGS = ROLE == ROLE_DKV && ORDERED && (WIDE || D <= 64), V_REGS = ROLE == ROLE_DQ || (K_REGS && D <= 64);
   static constexpr int OBYTES = (ROLE == ROLE_DKV) ? OWN * D * 2 : 0;  // owner tile kept in LDS (ROLE_DKV: K and V)
@@ -241,7 +256,9 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   typedef E ex4 __attribute__((ext_vector_type(4)));
   constexpr bool kDrop = FEAT & F_DROPOUT;
   constexpr float kLog2e = 1.4426950408889634f;
-  using L = QuadLayout<D>;
+  using L = typename std::conditional<T::WHOLE_ROWS, RowLayout<D>, QuadLayout<D>>::type;
+  using Quad = QuadLayout<D>;
+  using Ops = TileOperands<D, E>;
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
 
   const int tid = threadIdx.x;
@@ -375,7 +392,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     for (int ks = 0; ks < KS; ++ks) o2f[ks] = *reinterpret_cast<const ex8*>(vp + ks * 16 + 8 * h);
   }
 
-  // ---- global -> LDS transfers of a [rows][D] tile into its image (QuadLayout) -------------------------------------------------------
+  // ---- global -> LDS transfers of a [rows][D] tile into its image (QuadLayout or RowLayout) -----------------------------------------
   // lane l of a 1 KiB transfer writes LDS bytes [16 l, 16 l + 16); it fetches the chunk that the layout has there.  Rows past `valid` repeat
   // the last valid row (their contributions are masked).
   auto load_tile = [&](uint64_t base, int64_t stride, int valid, unsigned lds_off, int n_per_t) FL_INLINE {
@@ -453,21 +470,21 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   };
 
   // ---- LDS operand reads --------------------------------------------------------------------------------------------------
-  // Two addresses per kind of read, held in registers (the empty asm keeps the compiler from working them out again at every read);
-  // everything else is a constant of the instruction.
+  // QuadLayout: two addresses per kind of read, held in registers (the empty asm keeps the compiler from working them out again at every
+  // read); everything else is a constant of the instruction.
   unsigned a_row[2], a_own[2], a_tr[2];
-  {
+  if constexpr (!T::WHOLE_ROWS) {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
     const int i16 = lane % 16;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      a_row[j] = lds0 + L::at(qh * TB * 32 + r, 2 * j + h);
+      a_row[j] = lds0 + Quad::at(qh * TB * 32 + r, 2 * j + h);
       asm volatile("" : "+v"(a_row[j]));
       if constexpr (!kDQ) {
-        a_own[j] = lds0 + T::O1_OFF + L::at(ow * 32 + r, 2 * j + h);
+        a_own[j] = lds0 + T::O1_OFF + Quad::at(ow * 32 + r, 2 * j + h);
         asm volatile("" : "+v"(a_own[j]));
       }
-      a_tr[j] = lds0 + L::at(qh * TB * 32 + 8 * j + 4 * h + i16 / 4, (lane / 16) % 2 * 2 + i16 % 4 / 2) + i16 % 2 * 8;
+      a_tr[j] = lds0 + Quad::at(qh * TB * 32 + 8 * j + 4 * h + i16 / 4, (lane / 16) % 2 * 2 + i16 % 4 / 2) + i16 % 2 * 8;
       asm volatile("" : "+v"(a_tr[j]));
     }
   }
@@ -476,17 +493,20 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
   // row-wise: 8 consecutive elements [row][16 ks + 8 h, +8), row = 32 (qh TB + sb) + r of a streamed tile (A operand of X1/X2) or this
   // lane's row of an owner tile (B operand)
   auto frag_row = [&](unsigned tile_off, int sb, int ks) FL_INLINE -> ex8 {
-    return *(lds_ex8_ptr)(a_row[ks % 2] + tile_off + L::at(32 * sb, 4 * (ks / 2)));
+    if constexpr (T::WHOLE_ROWS) return Ops::rows(smem + tile_off, (qh * TB + sb) * 32 + r, ks, h);
+    return *(lds_ex8_ptr)(a_row[ks % 2] + tile_off + Quad::at(32 * sb, 4 * (ks / 2)));
   };
   auto frag_own = [&](unsigned tile_off, int ks) FL_INLINE -> ex8 {
-    return *(lds_ex8_ptr)(a_own[ks % 2] + (tile_off - T::O1_OFF) + L::at(0, 4 * (ks / 2)));
+    if constexpr (T::WHOLE_ROWS) return Ops::rows(smem + tile_off, ow * 32 + r, ks, h);
+    return *(lds_ex8_ptr)(a_own[ks % 2] + (tile_off - T::O1_OFF) + Quad::at(0, 4 * (ks / 2)));
   };
   // transposing: A operand of the accumulating products for 16-position chunk c (of this wave's) and column block db
   auto frag_tr = [&](unsigned tile_off, int c, int db) FL_INLINE -> ex8 {
+    if constexpr (T::WHOLE_ROWS) return Ops::columns(smem + tile_off, 2 * TB * qh + c, db, lane, h);
     ex8 f;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j] + tile_off + L::at(16 * c, 4 * db))));
+      const ex4 b4 = __builtin_bit_cast(ex4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a_tr[j] + tile_off + Quad::at(16 * c, 4 * db))));
 #pragma unroll
       for (int e = 0; e < 4; ++e) f[4 * j + e] = b4[e];
     }
