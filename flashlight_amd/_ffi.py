@@ -452,7 +452,8 @@ def attn_bwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, out: torch.Tenso
              grads: Optional[Sequence[torch.Tensor]] = None, biases: Sequence[tuple[torch.Tensor, int]] = (),
              dscores: Optional[torch.Tensor] = None, split: bool = False):
     """Gradients (dq, dk, dv) of `attn_fwd` called with the same arguments (dropout rate and seed included); `out` and `lse` are what that call
-    returned and filled, `dout` [B, Hq, Lq, Dv] the gradient of its result.  Three launches on the current stream.
+    returned and filled, `dout` [B, Hq, Lq, Dv] the gradient of its result.  Two or three launches on the current stream, one
+    more under a document mask.
     `grads` = (dq, dk, dv) receives the results when given.  `static_scratch` goes through `fl_attn_bwd_static`: nothing
     is allocated here beyond the results, the library's own static device array serves as scratch (calls that may
     overlap on one GPU must not both use it).

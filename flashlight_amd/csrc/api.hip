@@ -491,8 +491,8 @@ DiffPlan plan_diff(const fl_attn_params* p) {
     sequential = visited <= 256 || (visited <= 900 && !(last > 0 && last <= 256 && (tiles <= 768 || visited > 640)));
   if (sequential) return x;
   x.groups = 2;
-  // Up to 16 tiles of 128 rows keep 32 keys, the shape that the dump of attended pairs has and is compared in at every edge (2 heads of 256:
-  // 18.3 -> 13.9, where 64 rows and keys take 8.5).
+  // Up to 16 tiles of 128 rows keep the 128 rows and 32 keys that the dump of attended pairs is compared in at every edge, though not for
+  // speed (2 heads of 256, us: the branches one after the other 18.3, a group each 13.9, with 64 rows and keys 8.5).
   if (narrow && tiles <= 16) return x;
   x.keys = 64;
   // 64 rows per workgroup, two of which share a compute unit, where 128 would leave a round far from full or the walks are short (head

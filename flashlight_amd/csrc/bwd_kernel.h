@@ -7,8 +7,8 @@
 //
 // One kernel template, two roles, no atomics:
 //   ROLE_DQ   a workgroup owns 128 query rows of one head and streams the key tiles they attend;
-//   ROLE_DKV  a workgroup owns 128 keys of one key/value head and streams the query tiles (of every query head of the
-//             group) that attend them.
+//   ROLE_DKV  a workgroup owns 128 keys of one key/value head (256 in the wide form, BwdTraits) and streams the query tiles (of every
+//             query head of the group) that attend them.
 // In both roles a lane owns one *owner* position (the column of every accumulator it holds) and its registers run over
 // the streamed positions, because every product is issued with the streamed tile as the A operand:
 //   X1 = T1 . O1^T   (ROLE_DQ: K.Q^T = S^T;   ROLE_DKV: Q.K^T = S)       v_mfma_f32_32x32x16_bf16
@@ -345,7 +345,8 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
 
   // ---- owner operands ---------------------------------------------------------------------------------------------------
   // ROLE_DQ: Q and dO fragments of this lane's query row live in registers (B operands), with its LSE and Delta.
-  // ROLE_DKV: the workgroup's K and V rows are staged in LDS once and read as B operands where they are used.
+  // ROLE_DKV: so do this lane's K and V rows where the registers have room for them (T::K_REGS, T::V_REGS); otherwise the workgroup's are staged
+  // in LDS once and read as B operands where they are used.
   ex8 o1f[kDQ || T::K_REGS ? KS : 1], o2f[T::V_REGS ? KS : 1];
   float lse_o = 0.f, delta_o = 0.f;  // delta_o: minus this row's rowsum(dO o O)
   const bf16_t* kptr = p.k + (int64_t)batch * p.ks[0] + (int64_t)kvh * p.ks[1];

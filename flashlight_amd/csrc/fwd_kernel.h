@@ -1362,7 +1362,7 @@ void fwd_kernel(const KParams p) {
 
     // Documents of few key tiles, whose pre-pass was not launched (doc_own): the list is made here, by the steps of doc_lists_kernel.  A
     // wave per key tile leaves its ids' (min, max) in LDS; every wave then classifies all tiles, one per lane, for all waves, and writes
-    // the same list.  The two launches ahead of this one were 6 to 7 us; here it is a round trip to memory and some 150 instructions
+    // the same list.  The two launches ahead of this one (rows this short take an order of their own, doc_orders) are 6 to 7 us; here it is a round trip to memory and some 150 instructions
     // (8 heads of 837 ids, head dim 64: 21.5 -> 16.3 us; 16 x 16 of 100: 16.0 -> 11.5).
     if constexpr (kDoc) {
       if (__builtin_expect(p.doc_own, 0)) {

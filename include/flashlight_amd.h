@@ -251,7 +251,8 @@ uint64_t fl_bwd_params_sizeof(void);
 /* Host-only argument check of a backward call. */
 int fl_attn_bwd_validate(const fl_attn_bwd_params* p);
 
-/* Launches the backward kernels (row sums of dO o O; then dQ, dK and dV, in one launch or two) on `stream`. */
+/* Launches the backward kernels on `stream`: row sums of dO o O, then dQ, dK and dV in one launch; or dQ, whose workgroups form the row
+ * sums, then dK and dV. */
 int fl_attn_bwd(const fl_attn_bwd_params* p, void* stream);
 
 /* fl_attn_bwd for calls whose tiles alone would leave most of the GPU idle: sums may be taken in an order that depends on
