@@ -1270,6 +1270,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   kp.doc_stride = p->doc_stride;
   kp.alibi_heads = p->alibi_heads;
   kp.softcap = p->softcap;
+  if (p->softcap > 0.f) kp.near_cap = fl::NearCap::of(p->scale, p->softcap);
   if (p->score_fn != FL_SCORE_NONE) {
     // scale and log2(e) folded into the constants (in double): the kernel works on the raw q.k and in log2 units
     const double l2e = 1.4426950408889634, sc = p->scale;

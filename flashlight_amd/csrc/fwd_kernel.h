@@ -88,6 +88,39 @@ __device__ __forceinline__ void fetch_params() {
                "s"(x[10]), "s"(x[11]));
 }
 
+// The soft-cap cap * tanh(y), y = x * scale / cap, in log2 units for scores of |y| <= 1/4: an odd polynomial of the fifth degree (least largest
+// relative error, 4e-7, so that the capped score is off by 1e-7 cap at most; the exponential and the reciprocal leave 1.2e-7 cap).  With a
+// square completed it is  x * (u * u + b) * last,  u = x * x + a, and the last factor meets the addend of what follows: four
+// vector instructions per score, the ALiBi term included, where the exponential, the reciprocal and four more were needed.  Vector
+// issue bounds these kernels: an instruction per score is 3 to 4 %.  us, cap 50: ALiBi, causal, 2 x 32 over 8 x 8192, head dim 128, 1196 ->
+// 1076; cap alone, 4 x 16 x 2048, head dim 64, 106.6 -> 97.6; at head dim 256 122 -> 117.  With a seventh degree, which holds up to 1/2, the
+// first is 1128.  Scores four times as large, which take the exact form from the first tile on: 324 -> 322 (4096 long), 8 heads of 700 15.0 -> 15.2.
+struct NearCap {
+  static constexpr double K0 = 0.9999995827674866, K1 = -0.33321908116340637, K2 = 0.12841613590717316, R = 0.25;
+  float a, b, last, per_last;  // (per_last = 1 / last)
+  // u of the largest |x|, and of five sixths of it: the scores of 64 keys do not yet show the largest of a row.  (Numbers that nothing
+  // reaches where a float does not hold the powers of scale and cap.)
+  uint32_t least, least_first;
+  __host__ static NearCap of(float scale, float cap) {
+    NearCap c = {-1.0f, 0.f, 0.f, 0.f, ~0u, ~0u};
+    const double y = (double)scale / cap, z = 1.0 / (y * y);
+    if (!(y > 0x1p-24 && y < 0x1p24 && scale > 0x1p-20f && scale < 0x1p20f)) return c;
+    c.a = (float)(K1 / (2.0 * K2) * z);
+    c.b = (float)((K0 / K2 - K1 * K1 / (4.0 * K2 * K2)) * z * z);
+    c.last = (float)(K2 * 1.4426950408889634 * scale / (z * z));
+    c.per_last = 1.0f / c.last;
+    const float far[2] = {(float)((K1 / (2.0 * K2) + R * R) * z), (float)((K1 / (2.0 * K2) + 25.0 / 36.0 * R * R) * z)};
+    __builtin_memcpy(&c.least, &far[0], 4);
+    __builtin_memcpy(&c.least_first, &far[1], 4);
+    return c;
+  }
+  __device__ __forceinline__ float inner(float x) const { return __builtin_fmaf(x, x, a); }
+  __device__ __forceinline__ float outer(float u) const { return __builtin_fmaf(u, u, b); }
+  // of u as an unsigned number, or of the least of several: a is negative, so what lies further out, infinities and NaN are smaller numbers
+  __device__ __forceinline__ bool holds(uint32_t u) const { return u >= least; }
+  __device__ __forceinline__ bool holds_first(uint32_t u) const { return u >= least_first; }
+};
+
 struct KParams {
   const bf16_t* q;
   const bf16_t* k;
@@ -116,6 +149,7 @@ struct KParams {
   int32_t doc_own;
   int32_t alibi_heads;
   float softcap;
+  NearCap near_cap;
   const bf16_t* bias[2];
   int64_t bs[2][4];
   int32_t bdiv[2];
@@ -724,6 +758,17 @@ void fwd_kernel(const KParams p) {
   // kernels are relative to the reference of the moment; it can move only on the path that recomputes a tile's
   // weights, which accounts for the difference.
   constexpr bool kFoldRef = kSoftcap && !kDrop;  // (the dropout instances have no registers to spare for it)
+  // A wave whose scores are small beside the cap walks with the polynomial; from the first tile on that has others it takes the exact form.
+  constexpr bool kNear = kFoldRef;
+  const NearCap near_cap = p.near_cap;
+  bool near = kNear;  // (uniform over the wave)
+  float alibi_r[kNear && kAlibi ? 16 : 1];  // the ALiBi term at the registers' offsets, ahead of NearCap's last factor (scalar registers)
+  if constexpr (kNear && kAlibi) {
+    // (this order of the factors: with the offset last the compiler multiplies by it in the loop, and spills)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      alibi_r[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, slope_l2 * (float)(8 * (i / 4) + i % 4) * near_cap.per_last)));
+  }
 
   // Gate logits of this lane's output elements, fetched before the key loop when they fit the register budget so that
   // their latency is not paid in the epilogue.
@@ -954,8 +999,12 @@ void fwd_kernel(const KParams p) {
 
     // ---- score modifications of one tile; afterwards s * c2 is the logit in log2 units ---------------------------------
     // Register i of block (kb, qb) is key k0 + 32*kb + 8*(i/4) + 4*h + i%4 against query qrow[qb].
-    auto score_mods = [&](f32x16 (&s)[KB][QB], int t, int bslot) FL_INLINE {
+    // (near_tag: the soft-cap as a polynomial; `nearest` then says whether it holds)
+    uint32_t nearest = 0;
+    auto score_mods = [&](f32x16 (&s)[KB][QB], int t, int bslot, auto near_tag) FL_INLINE {
+      constexpr bool kPoly = decltype(near_tag)::value;
       const int k0 = t * BN;
+      if constexpr (kPoly) nearest = ~0u;
       if constexpr (kMod) {
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
@@ -970,7 +1019,7 @@ void fwd_kernel(const KParams p) {
             // ALiBi: slope * (rel0 + off) with off a per-register constant; slope * rel0 rides in the addend of the
             // multiply-add that precedes it, leaving one multiply-add with a literal per score
             const float alibi0 = kAlibi ? slope_l2 * rel0 : 0.f;
-            const float cap_shift = cap_c + alibi0 - (kFoldRef ? ref_now(qb) : 0.f);
+            const float cap_shift = (kPoly ? 0.f : cap_c) + alibi0 - (kFoldRef ? ref_now(qb) : 0.f);
             auto combine_as = [&](auto fn_tag) FL_INLINE {
               constexpr int kFn = decltype(fn_tag)::value;
 #pragma unroll
@@ -980,7 +1029,12 @@ void fwd_kernel(const KParams p) {
                 if constexpr (kNatural) {
                   tl2 = __builtin_fmaf(x, p.scale, bv[i]);  // natural units: one operation per score
                 } else {
-                  if constexpr (kSoftcap) {
+                  if constexpr (kPoly) {
+                    const float u = near_cap.inner(x);
+                    nearest = min(nearest, __float_as_uint(u));
+                    const float q = near_cap.outer(u);
+                    tl2 = __builtin_fmaf(kAlibi && i > 0 ? __builtin_fmaf(x, q, alibi_r[i]) : x * q, near_cap.last, cap_shift);
+                  } else if constexpr (kSoftcap) {
                     const float e = fast_exp2(x * cap_k1);
                     const float rc = fast_rcp(e + 1.0f);
                     tl2 = __builtin_fmaf(rc, -2.0f * cap_c, cap_shift);
@@ -993,7 +1047,7 @@ void fwd_kernel(const KParams p) {
                   } else {
                     tl2 = kAlibi ? __builtin_fmaf(x, p.scale_log2, alibi0) : x * p.scale_log2;
                   }
-                  if constexpr (kAlibi) tl2 = __builtin_fmaf(slope_l2, (float)(8 * (i / 4) + (i % 4)), tl2);
+                  if constexpr (kAlibi && !kPoly) tl2 = __builtin_fmaf(slope_l2, (float)(8 * (i / 4) + (i % 4)), tl2);
                   if constexpr (kBias) tl2 = __builtin_fmaf(bv[i], kLog2e, tl2);
                 }
                 s[kb][qb][i] = tl2;
@@ -1090,6 +1144,21 @@ void fwd_kernel(const KParams p) {
             }
           }
       }
+    };
+    // The scores of a wave's first tile, which nothing covers; they say which form the soft-cap starts with.
+    auto first_scores = [&](f32x16 (&s)[KB][QB], int t) FL_INLINE {
+      qk(s, 0);
+      if constexpr (kNear) {
+        uint32_t least = ~0u;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+          for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) least = min(least, __float_as_uint(near_cap.inner(s[kb][qb][i])));
+        near = near && __builtin_amdgcn_ballot_w64(!near_cap.holds_first(least)) == 0;
+      }
+      score_mods(s, t, 0, std::false_type{});
     };
     // Element mask of a tile that is not FULL for this wave: attend iff
     // key < Lk && ((dmin <= key - q <= dmax) || key < pfx) [&& same document]; with key = kbase + off and off a
@@ -1519,8 +1588,7 @@ void fwd_kernel(const KParams p) {
       live_run(a_live, b_live);
       f32x16 s_a[KB][QB], s_b[KB][QB];
       if (a_live == 0 && b_live > 0) {
-        qk(s_a, 0);
-        score_mods(s_a, entry_tile(ent[0]), 0);
+        first_scores(s_a, entry_tile(ent[0]));
       }
       __syncthreads();  // K slot 0 may be overwritten from here on
 
@@ -1549,7 +1617,7 @@ void fwd_kernel(const KParams p) {
       // slot j % NS, V likewise.  The body after `settle` is one straight-line block in which the scheduler
       // interleaves both MFMA groups with the exponentials.  The loop unrolls NS steps so that every slot index is a
       // constant and the two score buffers swap roles without copies.
-      auto step = [&](f32x16 (&sc)[KB][QB], f32x16 (&sn)[KB][QB], auto slot_tag) FL_INLINE {
+      auto step = [&](f32x16 (&sc)[KB][QB], f32x16 (&sn)[KB][QB], auto slot_tag, auto near_tag) FL_INLINE {
         constexpr int slot = decltype(slot_tag)::value;
         // K slot `slot` held this tile's K and V slot `slot - 1` the previous tile's V: both were last read before the
         // barrier that ended the previous step
@@ -1564,12 +1632,24 @@ void fwd_kernel(const KParams p) {
         ex8 vfirst[DVB];
         weights_checked(sc, pf, reference_free(ent[0]), std::true_type{}, vfirst, slot, entry_tile(ent[0]), std::true_type{});
         pv_mma(pf, slot, vfirst, std::true_type{});
-        score_mods(sn, entry_tile(ent[1]), (slot + 1) % NS);
+        score_mods(sn, entry_tile(ent[1]), (slot + 1) % NS, near_tag);
         {
           // the next tile's score modifications (if any) go under the second product's MFMAs
           constexpr int NB = 2 * KB * DVB * QB;
-          constexpr int mod_ops = (kSoftcap ? 4 : (kMod ? 1 : 0)) + (kAlibi ? 2 : 0) + (kBias ? 3 : 0);
+          constexpr int mod_ops = (decltype(near_tag)::value ? 5 : (kSoftcap ? 4 : (kMod ? 1 : 0)) + (kAlibi ? 2 : 0)) + (kBias ? 3 : 0);
           sched_second_product<NB, (16 * KB * QB * mod_ops + NB - 1) / NB>();
+        }
+        if constexpr (decltype(near_tag)::value) {
+          // (the asm keeps the polynomial under the products: the branch would take it along behind them)
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int qb = 0; qb < QB; ++qb) asm volatile("" : "+v"(sn[kb][qb]));
+          if (__builtin_amdgcn_ballot_w64(!near_cap.holds(nearest)) != 0) {
+            near = false;
+            qk(sn, (slot + 1) % NS);
+            score_mods(sn, entry_tile(ent[1]), (slot + 1) % NS, std::false_type{});
+          }
         }
         __builtin_amdgcn_s_setprio(0);
         end_step(steady);
@@ -1579,25 +1659,29 @@ void fwd_kernel(const KParams p) {
       while (pos < a_live && pos + 1 < n_list) {
         const bool steady = issue_loads(pos % NS);
         if (pos + 1 == a_live) {
-          qk(s_a, 0);
-          score_mods(s_a, entry_tile(ent[1]), 0);
+          first_scores(s_a, entry_tile(ent[1]));
         }
         end_step(steady);
       }
       if (pos >= a_live && pos < b_live) {
       int last_slot = 0;  // ring slot of the run's final tile; its scores are in s_a when the slot is even
       bool more = true;
-      while (more) {
+      auto steps = [&](auto near_tag) FL_INLINE {
         more = static_while<0, NS>([&](auto idx) FL_INLINE  {
           constexpr int slot = decltype(idx)::value;
           if (!(pos + 1 < b_live)) {
             last_slot = slot;
             return false;
           }
-          if constexpr (slot % 2 == 0) step(s_a, s_b, idx); else step(s_b, s_a, idx);
+          if constexpr (slot % 2 == 0) step(s_a, s_b, idx, near_tag); else step(s_b, s_a, idx, near_tag);
           return true;
         });
+      };
+      // (two loops: the two forms as branches of one step spill)
+      if constexpr (kNear) {
+        while (more && near) steps(std::true_type{});
       }
+      while (more) steps(std::false_type{});
       // the run's last tile: no scores of a next tile to form; the step's transfers and barrier only if the workgroup
       // has further steps
       const bool more_steps = pos + 1 < n_list;
