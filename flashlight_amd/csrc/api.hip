@@ -868,6 +868,13 @@ int64_t chunks_of_entries(int64_t heads_and_groups, int64_t tiles, int per_cu, i
 // has to stay an ordinary number.  (A scale that has not been set yet is no reason against it.)
 bool row_starts_products(const fl_attn_params* p) { return !(p->scale > 0.f) || (p->scale >= 0x1p-100f && p->scale <= 0x1p100f); }
 
+// Whether the heads of a chunk of entries share an XCD in the shared-bias kernels that walk over entries.  With operands as the Evoformer has them a
+// head's row is half of a cache line at head dim 32: heads on XCDs of their own bring every line into two L2s (forward and gradients, 128 x 8 x
+// 256 x 256: 67 instead of 134 MB read by each).  A head's bias is then read by every XCD, which short chunks do not pay for.  us, heads apart ->
+// together: gradients with their forward, 256 x 8 x 256 x 256, 268 -> 258, 512 entries 567 -> 502, 150 x 8 x 333 x 333, head dim 64, 755 -> 723; forwards, 512 x 8 x 160 x 160,
+// 121 -> 116; of 5 entries 7.4 -> 7.7, of 8 with a bias in fp32 7.7 -> 9.5.
+bool shared_bias_by_chunk(int chunk_len) { return chunk_len >= 4; }
+
 // Whether *p (already validated) is a call the shared-bias stripe forward (stripe_kernel.h) takes.  Fills the kernel's parameters,
 // its wave count, and the number of workgroups and their LDS bytes.
 bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, int* waves, int64_t (&launch)[2]) {
@@ -944,6 +951,7 @@ bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, 
   k.chunk_len = (int)((k.div + most - 1) / most);
   k.chunks = (k.div + k.chunk_len - 1) / k.chunk_len;
   if (units * k.chunks > (1 << 28)) return false;
+  k.by_chunk = shared_bias_by_chunk(k.chunk_len);
   *out = k;
   *waves = shape.waves;
   launch[0] = ((int64_t)k.groups * k.chunks * k.H + 7) / 8 * 8 * k.tiles;
@@ -1780,6 +1788,10 @@ int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* strea
   sp.chunks = x.chunks;
   sp.chunk_len = x.chunk_len;
   sp.tiles = (sp.S + 31) / 32;
+  sp.by_chunk = shared_bias_by_chunk(sp.chunk_len);
+  // (operands that stay in the 256 MB of cache behind the L2s from the kernels before arrive soon enough without: 67 MB, 128 x 4 x 256 x 256 of
+  // head dim 64, 128 -> 130 us)
+  sp.ahead = (int64_t)p->B * p->Hq * p->Lq * p->Dqk * 8 > (int64_t)80 << 20;
   sp.s_pad = (sp.S + 3) / 4 * 4;
   sp.scale = p->scale;
   sp.scale_log2 = p->scale * 1.4426950408889634f;

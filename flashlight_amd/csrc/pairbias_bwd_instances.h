@@ -17,7 +17,7 @@ constexpr SBShape pairbias_bwd_shape(int d, int s) {
   x.nb = blocks <= 4 ? 1 : blocks <= 8 ? (d == 32 ? 2 : 1) : 2;
   x.waves = (blocks + x.nb - 1) / x.nb;
   const int slot = x.waves * (x.nb * 128 * d + 512) + 128 * d + 512;
-  x.lds_bytes = (2 * slot <= 160 * 1024 ? 2 : 1) * slot;
+  x.lds_bytes = (2 * slot <= 160 * 1024 ? 2 : 1) * slot + 256;
   return x;
 }
 hipError_t launch_pairbias_bwd_bf16(int d, const SBShape& shape, const SBParams& p, hipStream_t stream);

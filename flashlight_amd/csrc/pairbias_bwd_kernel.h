@@ -42,6 +42,8 @@ struct SBParams {
   int32_t B, H, S;
   int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
   int32_t tiles;                   // 32-row stripes
+  int32_t by_chunk;                // see StripePlace
+  int32_t ahead;                   // rows are touched two entries ahead
   int32_t s_pad;                   // row length of the partial bias gradient (S rounded up to 4)
   float scale, scale_log2;
   float* dbias_part;               // [groups][chunks][H][S][s_pad], or null: no gradient of the bias wanted
@@ -65,7 +67,7 @@ struct SBTraits {
   static constexpr int SLOT_BYTES = NW * W_BYTES + S_OWN;  // one batch entry
   // tiles of batch entries resident in LDS
   static constexpr int SLOTS = 2 * SLOT_BYTES <= 160 * 1024 ? 2 : 1;
-  static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES;
+  static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES + 256;  // (and where touch() puts what nothing reads)
   // the partial sums go where the consumed tiles were: both sets at once when a wave's two tiles have room for them
   static constexpr bool ONE_PASS = DQ || 2 * T_BYTES >= 2 * PARK;
 };
@@ -221,7 +223,29 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
   constexpr int RPP = 256 / D, PIECES = 32 / RPP, PPW = (PIECES + NW - 1) / NW;
   const int pieces = (rows + RPP - 1) / RPP, my_pieces = (pieces - wave + NW - 1) / NW;
 
+  // The rows of the stripe's own places in both streamed operands, touched two entries ahead: the stripes of a head touch between them all rows
+  // that they will all ask for, a cache line per lane.  The stripes ask for the same rows at the same time, so that little is on its way
+  // from memory although every wave has an entry in flight: us, forward and gradients, 256 x 8 x 256 x 256, 274 -> 258; 512 entries 562 -> 502;
+  // 150 x 8 x 333 x 333, head dim 64, 799 -> 723.
+  const int ahead_end = __builtin_amdgcn_readfirstlane(wave == 0 && p.ahead ? n1 : 0);
+  uint64_t ahead_at = 0, ahead_step = 0;
+  {
+    const bool second = lane >= 32;
+    const bf16_t* base = kDQ ? (second ? p.v : p.k) : (second ? p.dout : p.q);
+    const int64_t b = kDQ ? (second ? p.vs[0] : p.ks[0]) : (second ? p.dos[0] : p.qs[0]);
+    const int64_t hd = kDQ ? (second ? p.vs[1] : p.ks[1]) : (second ? p.dos[1] : p.qs[1]);
+    const int64_t sq = kDQ ? (second ? p.vs[2] : p.ks[2]) : (second ? p.dos[2] : p.qs[2]);
+    ahead_at = (uint64_t)(base + (int64_t)(n0 + 1) * b + (int64_t)head * hd + (int64_t)min(own, S - 1) * sq);
+    ahead_step = (uint64_t)(b * 2);
+  }
+  auto touch_entry = [&](int n) FL_INLINE {  // n: n0 + 1, n0 + 2, ... in this order
+    if (n < ahead_end) {
+      touch(ahead_at, lds0 + T::SLOTS * slot_bytes);
+      ahead_at += ahead_step;
+    }
+  };
   if (n0 < n1) load_entry(0);
+  touch_entry(n0 + 1);
   for (int n = n0; n < n1; ++n) {
     const int slot = T::SLOTS == 2 ? (n - n0) & 1 : 0;
     // everything this wave has asked for has landed, except the stores that were issued since
@@ -229,6 +253,7 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
     else dma_wait<(kDQ ? 1 : 2) * PPW>();
     __syncthreads();  // the owned rows are visible; everyone is done with the other slot
     if (T::SLOTS == 2 && n + 1 < n1) load_entry(slot ^ 1);
+    touch_entry(n + 2);
 
     unsigned char* s0 = smem + slot * slot_bytes;
     unsigned char* mine = s0 + wave * T::W_BYTES;

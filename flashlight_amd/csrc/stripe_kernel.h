@@ -43,6 +43,7 @@ struct StripeParams {
   int32_t B, H, Lq, Lk;
   int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
   int32_t tiles;                       // stripes of 32 QB rows
+  int32_t by_chunk;                    // see StripePlace
   int32_t by_maximum;                  // weights are formed against the row's maximum from the start
   float scale, scale_log2;
 };

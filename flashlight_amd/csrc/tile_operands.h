@@ -42,15 +42,22 @@ struct TileOperands {
   __device__ static __forceinline__ int park_at(int row, int c) { return row * (D * 4) + ((c ^ row) & (D / 4 - 1)) * 16; }
 };
 
+// Brings the cache line at each lane's address into the L2, and four bytes of it into 256 bytes of LDS that nothing reads.
+__device__ __forceinline__ void touch(uint64_t lane_address, unsigned lds_base) {
+  const unsigned lds_base_uniform = (unsigned)__builtin_amdgcn_readfirstlane((int)lds_base);
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(lane_address), "s"(lds_base_uniform) : "m0");
+}
+
 // Workgroup -> (group of batch entries that share the bias, chunk of them, head, stripe): the stripes of one (chunk, head) read the
-// same tensors and stay on one XCD.  unit: (group, chunk, head) as one number; `none`: a workgroup past the last of them.
+// same tensors and stay on one XCD.  unit: (group, chunk, head) as one number; `none`: a workgroup past the last of them.  by_chunk: the heads of
+// a chunk on one XCD, otherwise (chunk, head) pairs in turn (shared_bias_by_chunk in api.hip).
 struct StripePlace {
   int tile, unit;
   template <class P, class Block>
   __device__ __forceinline__ StripePlace(const P& p, const Block block) {
-    const int x = block % 8, i = block / 8;
+    const int x = block % 8, i = block / 8, each = (p.groups * p.chunks * p.H + 7) / 8, of_x = i / p.tiles;
     tile = i % p.tiles;
-    unit = i / p.tiles * 8 + x;
+    unit = !p.by_chunk ? of_x * 8 + x : of_x < each ? x * each + of_x : 8 * each;
   }
   template <class P>
   __device__ __forceinline__ bool none(const P& p) const { return unit >= p.groups * p.chunks * p.H; }
