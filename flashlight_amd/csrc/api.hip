@@ -1452,6 +1452,8 @@ static int validate_bwd(const fl_attn_bwd_params* b, const fl::BwdInstance** out
     return fail(FL_ERR_SHAPE, "backward: too many workgroups");
   uint32_t want = 0;
   if (p->alibi_heads > 0 || p->softcap > 0.f) want = fl::F_ALIBI | fl::F_SOFTCAP;
+  // ALiBi alone: a kernel without the soft-cap where there is one (T::ORDERED, whose kernels with it take it as given)
+  if (want != 0 && !(p->softcap > 0.f) && p->Dqk >= 64 && !is_doc(p->mask_kind) && !has_bias && !p->dropout_threshold) want = fl::F_ALIBI;
   if (is_doc(p->mask_kind)) want |= fl::F_DOC;
   if (has_bias) want |= fl::F_BIAS;
   if (p->dropout_threshold) want |= fl::F_DROPOUT;  // (head dims 64 and 128)

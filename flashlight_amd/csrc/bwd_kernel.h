@@ -232,7 +232,8 @@ struct OrderedStep {
     for (int m = 0; m < M; ++m) {
       if (m >= KP ? gradients(m - 1) < 4 * ((m - KP) / DB) + 4 : m >= VP && weights(m - 1) < 4 * ((m - VP) / DB) + 4) return false;
       if (lse_quad(m) >= 0) lse[lse_quad(m) % 2] = lse_quad(m);
-      if (weights(m) < weights(m - 1) || gradients(m) < gradients(m - 1) || gradients(m) > weights(m)) return false;
+      // (by fours: under the soft-cap the mask follows each four pairs of weights)
+      if (weights(m) < weights(m - 1) || gradients(m) < gradients(m - 1) || gradients(m) > weights(m) / 4 * 4) return false;
       for (int w = weights(m - 1); w < weights(m); ++w)
         if (m < (w / 8 + 1) * KS - 1 || (!DQ && lse[w / 2 % 2] != w / 2)) return false;
       for (int w = gradients(m - 1); w < gradients(m); ++w)
@@ -657,6 +658,7 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
     }
     int lo[TB], hi[TB];     // the element mask's bounds, where it is asked
     float alibi0[TB];       // the ALiBi term at register offset 0
+    unsigned out[TB];       // (under the soft-cap) positions outside the mask
     static_while<0, AHEAD>([&](auto m) FL_INLINE { read(m); return true; });
     static_while<0, M>([&](auto mt) FL_INLINE {
       constexpr int m = decltype(mt)::value;
@@ -686,9 +688,11 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
           if (!full) {  // uniform over the workgroup or the wave; the asm keeps it a branch
             bounds(sbase, lo[sb], hi[sb]);
             asm volatile("" : "+v"(lo[sb]), "+v"(hi[sb]));
-            if constexpr (!kSoftcap && !kDoc) {
+            if constexpr (kSoftcap) {
+              out[sb] = outside_word(lo[sb], hi[sb]);
+            } else if constexpr (!kDoc) {
               minus_inf_outside(x1[sb], outside_word(lo[sb], hi[sb]));
-            } else if constexpr (!kSoftcap) {
+            } else {
 #pragma unroll
               for (int i = 0; i < 16; ++i)
                 if (!attended(t0, sbase, slot, 8 * (i / 4) + i % 4, lo[sb], hi[sb], doc_uniform)) x1[sb][i] = -INFINITY;
@@ -702,21 +706,39 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
           float s2, dfac = 1.0f;  // logit in log2 units minus the LSE; d(score) / d(qk * scale)
           if constexpr (kSoftcap) {
             const float th = __builtin_fmaf(fast_rcp(fast_exp2(x * cap_k1) + 1.0f), -2.0f, 1.0f);  // tanh(x * scale / cap)
-            s2 = cap_on ? __builtin_fmaf(th, cap_c, c0) : __builtin_fmaf(x, p.scale_log2, c0);
-            dfac = cap_on ? __builtin_fmaf(-th, th, 1.0f) : 1.0f;
+            s2 = __builtin_fmaf(th, cap_c, c0);
+            dfac = __builtin_fmaf(-th, th, 1.0f);
           } else {
             s2 = __builtin_fmaf(x, p.scale_log2, c0);
           }
           if constexpr (kAlibi) s2 = __builtin_fmaf(kDQ ? slope_l2 : -slope_l2, (float)off, s2);
           float pv = fast_exp2(s2);
-          if constexpr (kSoftcap) {  // (-inf would not do as a score)
-            if (!full) {
-              if (!attended(t0, sbase, slot, off, lo[sb], hi[sb], doc_uniform)) pv = 0.f;
-              asm volatile("" : "+v"(pv));
-            }
-          }
           if constexpr (!kDQ) pf[2 * sb + e / 8][e % 8] = (E)pv;
           x1[sb][e] = kSoftcap ? pv * dfac : pv;
+        }
+        // Under the soft-cap -inf would not do as a score: what is masked is taken out again, eight positions at a time.  (Asked at every score, and
+        // with the calls without a cap in the same kernel, a step was 64 branches with two or three vector instructions between them.  us, forward
+        // and gradients, causal, ALiBi and a soft-cap, with the branches -> this: 4 x 16 x 2048, head dim 128, 447 -> 426, scores far out 457 -> 436; over 4
+        // heads, head dim 64, 293 -> 277, 299 -> 286; 3 x 16 over 4 of 1000, fp16, 117 -> 101.  ALiBi alone, which has kernels without the cap
+        // now, 436 -> 364 and 276 -> 208.)
+        if constexpr (kSoftcap) {
+          if (w % 4 == 3 && !full) {
+            const int half = w % 8 / 4;
+            int lost[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const int i = 8 * half + e;
+              lost[e] = __builtin_amdgcn_sbfe((int)out[sb], 8 * (i / 4) + i % 4, 1);
+              x1[sb][i] = __uint_as_float(~(uint32_t)lost[e] & __float_as_uint(x1[sb][i]));
+            }
+            if constexpr (!kDQ) {
+              u32x4 two = __builtin_bit_cast(u32x4, pf[2 * sb + half]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) two[e] &= ~(((uint32_t)lost[2 * e] & 0xFFFFu) | ((uint32_t)lost[2 * e + 1] << 16));
+              pf[2 * sb + half] = __builtin_bit_cast(ex8, two);
+            }
+            asm volatile("" : "+v"(x1[sb][8 * half]));  // (a branch)
+          }
         }
       }
 #pragma unroll
