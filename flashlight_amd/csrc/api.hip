@@ -40,7 +40,7 @@ static __global__ void doc_table_kernel(const int64_t* ids, int64_t ids_stride, 
 // Forward pre-pass for document masks, one workgroup of 1024 threads per (batch, query tile of `bm` rows), straight from
 // the ids: lists the key tiles (of `bn` keys) that some row of the query tile attends, with the class of each for every
 // wave of the forward (`rw` rows per wave): EMPTY when the id ranges of the tile's keys and the wave's rows do not meet,
-// FULL when both are the same single id and the positional part of the mask agrees, PARTIAL otherwise.  Valid for
+// FULL when both are the same single id and the positional part of the mask agrees, ONE_DOC when they are and it does not, PARTIAL otherwise.  Valid for
 // arbitrary (unsorted, negative) ids.  The lists are the same for every head.  Output per workgroup: word 0 = number of
 // entries, then the entries in key order (bits 0-15 tile index, two class bits per wave from bit 16 on).
 // A wave per key tile reads its ids with one coalesced load and leaves their (min, max) in LDS (every load of a wave is in flight before
@@ -213,10 +213,8 @@ static __global__ __launch_bounds__(1024) void doc_lists_kernel(const int64_t* i
       const int64_t qmn = qrange[2 * w], qmx = qrange[2 * w + 1];
       int cw = TILE_EMPTY;
       if (a < e) {
-        cw = classify_positional(mask_kind, a, e, k0, k1, 0, 0);
-        if (kmx < qmn || kmn > qmx) cw = TILE_EMPTY;
-        else if (!(kmn == kmx && qmn == qmx && kmn == qmn) && cw == TILE_FULL) cw = TILE_PARTIAL;
-        if (cw == TILE_FULL && k0 + bn > L) cw = TILE_PARTIAL;  // ragged tail: keys >= L are masked
+        cw = kmx < qmn || kmn > qmx ? TILE_EMPTY
+                                    : classify_document(mask_kind, a, e, k0, k1, kmn == kmx && qmn == qmx && kmn == qmn, k0 + bn > L);
       }
       c |= (unsigned)cw << (2 * w);
     }

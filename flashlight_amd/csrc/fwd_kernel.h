@@ -43,7 +43,8 @@ enum : uint32_t {
 };
 
 enum : int { MASK_NONE = 0, MASK_CAUSAL = 1, MASK_SLIDING = 2, MASK_PREFIX = 3, MASK_DOC = 4, MASK_DOC_CAUSAL = 5 };
-enum : int { TILE_EMPTY = 0, TILE_PARTIAL = 1, TILE_FULL = 2 };
+// (TILE_ONE_DOC: under a document mask, keys and rows that all have one id, and a part that the positions mask)
+enum : int { TILE_EMPTY = 0, TILE_PARTIAL = 1, TILE_FULL = 2, TILE_ONE_DOC = 3 };
 
 // Key tiles are numbered in 16 bits inside the LDS tile list.
 constexpr int kMaxKeyTiles = 65535;
@@ -338,6 +339,11 @@ __device__ __forceinline__ int classify_positional(int kind, int q0, int q1, int
       return (k1 <= prefix || k1 - 1 <= q0) ? TILE_FULL : TILE_PARTIAL;
     default: return TILE_FULL;
   }
+}
+// ... and with the documents: one_id: keys and rows all have one id; ragged: the tile has places past the last key, which are masked
+__device__ __forceinline__ int classify_document(int kind, int q0, int q1, int k0, int k1, bool one_id, bool ragged) {
+  const int c = classify_positional(kind, q0, q1, k0, k1, 0, 0);
+  return c == TILE_EMPTY ? TILE_EMPTY : !one_id ? TILE_PARTIAL : c == TILE_FULL && !ragged ? TILE_FULL : TILE_ONE_DOC;
 }
 
 // (min, max) document id over positions [p0, p1) from the per-kDocBlock table.
@@ -969,11 +975,11 @@ void fwd_kernel(const KParams p) {
     auto entry_tile = [&](uint32_t e) FL_INLINE  { return (int)(__builtin_amdgcn_readfirstlane(e) & 0xffffu); };
     auto entry_class = [&](uint32_t e) FL_INLINE  { return (int)((__builtin_amdgcn_readfirstlane(e) >> (16 + 2 * wave)) & 3u); };
 
-    // whether some wave may apply the element mask to the entry's tile: not when it is FULL (class bits 10) for every
+    // whether some wave may look at the ids of the entry's tile: not when it is FULL or ONE_DOC (class bits 10 and 11) for every
     // wave.  (A tile that is EMPTY for a wave can still lie inside that wave's run, where it is computed and masked.)
     auto entry_masked = [&](uint32_t e) FL_INLINE {
-      constexpr uint32_t kAll = (1u << (2 * NW)) - 1u;
-      return ((__builtin_amdgcn_readfirstlane(e) >> 16) & kAll) != (0xAAAAu & kAll);
+      constexpr uint32_t kHigh = 0xAAAAu & ((1u << (2 * NW)) - 1u);
+      return ((__builtin_amdgcn_readfirstlane(e) >> 16) & kHigh) != kHigh;
     };
 
     // ---- S^T = K . Q^T for one tile: A = K fragment from LDS, B = Q fragment ---------------------------------------
@@ -1167,45 +1173,42 @@ void fwd_kernel(const KParams p) {
     // With off = key - kbase a compile-time constant per register, the positional predicate is lo <= off <= hi for
     // per-lane bounds: every mask is one interval of key - q cut at Lk; the prefix-LM mask is the union of two
     // intervals that both start at -inf, i.e. again one (dmin is far below any offset unless a window is set).
-    auto apply_mask = [&](f32x16 (&s)[KB][QB], int t, int vslot) FL_INLINE {
+    auto apply_mask = [&](f32x16 (&s)[KB][QB], int t, int vslot, int cls) FL_INLINE {
       const int k0 = t * BN;
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb) {
         const int kbase = k0 + 32 * kb + 4 * h;
         const int t_len = p.Lk - kbase;   // off < t_len   <=> key < Lk
         const int t_pfx = p.pfx - kbase;  // off < t_pfx   <=> key < pfx
-        // Under a document mask the ids of this lane's 16 keys come from the wave's LDS image of the tile's ids (it
-        // arrived with the V tile in ring slot `vslot`): four runs of four consecutive keys.
-        int64_t kdoc[16];
-        if constexpr (kDoc) {
-          typedef int64_t i64x2 __attribute__((ext_vector_type(2)));
-          const unsigned char* il = smem + T::I_OFF + vslot * T::IBYTES + wave * (BN * 8) + (32 * kb + 4 * h) * 8;
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int e2 = 0; e2 < 2; ++e2) {
-              const i64x2 two = *reinterpret_cast<const i64x2*>(il + (8 * g + 2 * e2) * 8);
-              kdoc[4 * g + 2 * e2] = two[0];
-              kdoc[4 * g + 2 * e2 + 1] = two[1];
-            }
-        }
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
           const int rel = kbase - qrow[qb];
           // off <= hi <=> key < Lk && (key - q <= dmax || key < pfx);  off >= lo <=> key - q >= dmin
           const int hi = min(t_len - 1, max(p.dmax - rel, t_pfx - 1));
           const int lo = p.dmin - rel;
-          if constexpr (!kDoc) {
-            minus_inf_outside(s[kb][qb], outside_word(lo, hi));
-            continue;
-          }
+          unsigned out = outside_word(lo, hi);
+          // Under a document mask the ids of this lane's 16 keys come from the wave's LDS image of the tile's ids (it
+          // arrived with the V tile in ring slot `vslot`): four runs of four consecutive keys.  Most masked tiles hold the diagonal of one
+          // document (ONE_DOC), where the positions alone decide and no ids are fetched.  (The ids' part is a branch around a word of bits, which the
+          // choice takes; as comparisons of ids and positions at every score: us, causal, 16 heads of 16384, head dim 64, 144.7 -> 137.8; 4 x 16 x
+          // 2048 47.4 -> 42.2; 4 x 16 x 4096, head dim 128, 153.3 -> 146.9.  The choice itself in both forms, behind a branch, was 155.6 in the
+          // first.)
+          if constexpr (kDoc) {
+            if (cls != TILE_ONE_DOC) {
+              typedef int64_t i64x2 __attribute__((ext_vector_type(2)));
+              const unsigned char* il = smem + T::I_OFF + vslot * T::IBYTES + wave * (BN * 8) + (32 * kb + 4 * h) * 8;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int off = 8 * (i / 4) + (i % 4);
-            bool ok = (off <= hi) & (off >= lo);
-            if constexpr (kDoc) ok = ok & (kdoc[i] == qdoc[qb]);
-            s[kb][qb][i] = ok ? s[kb][qb][i] : -INFINITY;
+              for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e2 = 0; e2 < 2; ++e2) {
+                  const i64x2 two = *reinterpret_cast<const i64x2*>(il + (8 * g + 2 * e2) * 8);
+#pragma unroll
+                  for (int e = 0; e < 2; ++e) out |= two[e] == qdoc[qb] ? 0u : 1u << (8 * g + 2 * e2 + e);
+                }
+              asm volatile("" : "+v"(out));  // (a branch)
+            }
           }
+          minus_inf_outside(s[kb][qb], out);
         }
       }
     };
@@ -1484,8 +1487,7 @@ void fwd_kernel(const KParams p) {
           const int64_t qmn = qrange[2 * w], qmx = qrange[2 * w + 1];
           int cw = TILE_EMPTY;
           if (a < e && !(kmx < qmn || kmn > qmx)) {
-            cw = classify_positional(p.mask_kind, a, e, k0, k1, 0, 0);
-            if (cw == TILE_FULL && (!(kmn == kmx && qmn == qmx && kmn == qmn) || k0 + BN > p.Lk)) cw = TILE_PARTIAL;
+            cw = classify_document(p.mask_kind, a, e, k0, k1, kmn == kmx && qmn == qmx && kmn == qmn, k0 + BN > p.Lk);
           }
           classes |= (uint32_t)cw << (2 * w);
         }
@@ -1517,12 +1519,12 @@ void fwd_kernel(const KParams p) {
     // rounding of 16-bit weights is least where the largest is 1: without it the error against fp64 of 3 x 8 heads of 967 causal rows
     // is that of the whole walk, 2.06e-3 of the result's norm, with it 2.01e-3; 0.1 us).
     auto settle = [&](f32x16 (&sc)[KB][QB], uint32_t e, int vslot, bool own_max) FL_INLINE {
-      const int t = entry_tile(e);
-      const bool full = entry_class(e) == TILE_FULL;
+      const int t = entry_tile(e), cls = entry_class(e);
+      const bool full = cls == TILE_FULL;
       if constexpr (kLazyMasked) {
-        if (!full) apply_mask(sc, t, vslot);
+        if (!full) apply_mask(sc, t, vslot, cls);
       } else if (!full || !kFastRef || own_max) {
-        if (!full) apply_mask(sc, t, vslot);
+        if (!full) apply_mask(sc, t, vslot, cls);
         float mx[QB];
         row_max(sc, mx);
         rescale_if_grown(mx, false);
