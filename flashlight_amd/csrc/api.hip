@@ -592,6 +592,19 @@ int groups_for(const fl::Instance* in, const fl_attn_params* p) {
   const int groups = std::min(plan_few(p, wanted_features(p)).groups, in->max_groups);
   return lds_bytes_for(in, p) + (int64_t)(groups - 1) * in->lds_fixed_bytes <= fl::kMaxLdsBytes ? groups : 1;
 }
+// Whether a call with a soft-cap runs the kernel that takes NearCap's polynomial where the scores allow.  That kernel saves up to 15 % where they
+// stay within five sixths of a quarter of the cap, costs 0 to 1 % (at most 3: 2 x 16 x 2048 with ALiBi at head dim 64, 4 x 16 x 2048 at 32) where they do not, and half a microsecond, whatever the call, where they
+// leave that range on the way: a second loop to be fetched, and a tile's scores formed twice where they jump past the range itself.  Short calls
+// therefore keep the exponential.  us, exponential -> polynomial, scores N(0,1) and a quarter of the cap at 9 / 4 / 2 of them.  Below the line: 4 x 16 x 300,
+// head dim 64, causal, 8.6 -> 8.2 / 9.2 / 8.6; 2 x 8 x 700 14.2 -> 13.1 / 15.0 / 14.3; 8 x 8 x 512 12.3 -> 11.6 / 13.0 / 12.4; head dim 32, 3 x 16 x 600, ALiBi,
+// 14.4 -> 12.7 / 15.3 / 14.7; 2 x 32 x 512, head dim 128, 16.8 -> 16.1 / 17.7 / 17.1.  Above: 8 x 2048, head dim 64, ALiBi, causal, 22.2 -> 20.2 / 22.7 / 22.5; 8 x 16 x 512
+// 20.2 -> 18.3 / 20.4 / 20.3; 4 x 16 x 700, head dim 128, 26.4 -> 24.5 / 26.7 / 26.8; 4 x 16 x 1024 42.9 -> 38.5 / 43.3 / 43.3; under a window of 256, 4 x 16 x 4096,
+// head dim 64, 55.2 -> 51.4 / 55.9 / 55.9; 4 x 16 over 4 x 2048, causal, 75.1 -> 63.6 / 75.5 / 74.8.
+bool near_cap_pays(const fl_attn_params* p, const fl::Instance* in, int groups, int64_t grid) {
+  // keys of a wave's longest walk, times the waves (of which two per SIMD run at once, and one alone takes as long as half a pair)
+  const int64_t walk = p->mask_kind == FL_MASK_SLIDING ? std::min<int64_t>(p->Lk, (int64_t)p->window + in->rw * in->nw) : p->Lk;
+  return walk / groups * std::max<int64_t>(1024, grid * in->nw * groups) >= (int64_t)1024 * 1024;
+}
 int64_t max_keys_for(const fl::Instance* in) {
   int64_t tiles = fl::kMaxKeyTiles;
   if (in->feat & fl::F_DOC) {
@@ -1276,7 +1289,6 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   kp.doc_stride = p->doc_stride;
   kp.alibi_heads = p->alibi_heads;
   kp.softcap = p->softcap;
-  if (p->softcap > 0.f) kp.near_cap = fl::NearCap::of(p->scale, p->softcap);
   if (p->score_fn != FL_SCORE_NONE) {
     // scale and log2(e) folded into the constants (in double): the kernel works on the raw q.k and in log2 units
     const double l2e = 1.4426950408889634, sc = p->scale;
@@ -1362,6 +1374,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
   const int grid = p->B * p->Hq * kp.n_qtiles;
 
   const int groups = groups_for(in, p);
+  if (p->softcap > 0.f && near_cap_pays(p, in, groups, grid)) kp.near_cap = fl::NearCap::of(p->scale, p->softcap);
   int lds = p->diff && groups == 2 ? in->branches_lds_bytes : (int)lds_bytes_for(in, p) + (groups - 1) * in->lds_fixed_bytes;
 
   if (is_doc(p->mask_kind)) {

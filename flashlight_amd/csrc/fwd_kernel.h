@@ -90,36 +90,34 @@ __device__ __forceinline__ void fetch_params() {
 }
 
 // The soft-cap cap * tanh(y), y = x * scale / cap, in log2 units for scores of |y| <= 1/4: an odd polynomial of the fifth degree (least largest
-// relative error, 4e-7, so that the capped score is off by 1e-7 cap at most; the exponential and the reciprocal leave 1.2e-7 cap).  With a
-// square completed it is  x * (u * u + b) * last,  u = x * x + a, and the last factor meets the addend of what follows: four
-// vector instructions per score, the ALiBi term included, where the exponential, the reciprocal and four more were needed.  Vector
+// relative error, 4.2e-7; evaluated in fp32 6e-7, or 1.35e-7 of the cap, where the exponential and the reciprocal leave 1.5e-7 of it with both
+// correctly rounded).  With a square completed it is  x * (u * u + b) * last,  u = x * x + a, and the last factor meets the addend of what
+// follows: four vector instructions per score, the ALiBi term included, where the exponential, the reciprocal and four more were needed.  Vector
 // issue bounds these kernels: an instruction per score is 3 to 4 %.  us, cap 50: ALiBi, causal, 2 x 32 over 8 x 8192, head dim 128, 1196 ->
 // 1076; cap alone, 4 x 16 x 2048, head dim 64, 106.6 -> 97.6; at head dim 256 122 -> 117.  With a seventh degree, which holds up to 1/2, the
-// first is 1128.  Scores four times as large, which take the exact form from the first tile on: 324 -> 322 (4096 long), 8 heads of 700 15.0 -> 15.2.
+// first is 1128.
 struct NearCap {
   static constexpr double K0 = 0.9999995827674866, K1 = -0.33321908116340637, K2 = 0.12841613590717316, R = 0.25;
-  float a, b, last, per_last;  // (per_last = 1 / last)
-  // u of the largest |x|, and of five sixths of it: the scores of 64 keys do not yet show the largest of a row.  (Numbers that nothing
-  // reaches where a float does not hold the powers of scale and cap.)
-  uint32_t least, least_first;
+  float a, b, last, per_last;  // (per_last = 1 / last; last = 0: the exact form throughout)
+  uint32_t least, least_well;  // u of the largest |x|, and of five sixths of it
   __host__ static NearCap of(float scale, float cap) {
-    NearCap c = {-1.0f, 0.f, 0.f, 0.f, ~0u, ~0u};
+    NearCap c = {0.f, 0.f, 0.f, 0.f, 0u, 0u};
     const double y = (double)scale / cap, z = 1.0 / (y * y);
-    if (!(y > 0x1p-24 && y < 0x1p24 && scale > 0x1p-20f && scale < 0x1p20f)) return c;
+    if (!(y > 0x1p-24 && y < 0x1p24 && scale > 0x1p-20f && scale < 0x1p20f)) return c;  // (a float does not hold the powers)
     c.a = (float)(K1 / (2.0 * K2) * z);
     c.b = (float)((K0 / K2 - K1 * K1 / (4.0 * K2 * K2)) * z * z);
     c.last = (float)(K2 * 1.4426950408889634 * scale / (z * z));
     c.per_last = 1.0f / c.last;
     const float far[2] = {(float)((K1 / (2.0 * K2) + R * R) * z), (float)((K1 / (2.0 * K2) + 25.0 / 36.0 * R * R) * z)};
     __builtin_memcpy(&c.least, &far[0], 4);
-    __builtin_memcpy(&c.least_first, &far[1], 4);
+    __builtin_memcpy(&c.least_well, &far[1], 4);
     return c;
   }
   __device__ __forceinline__ float inner(float x) const { return __builtin_fmaf(x, x, a); }
   __device__ __forceinline__ float outer(float u) const { return __builtin_fmaf(u, u, b); }
   // of u as an unsigned number, or of the least of several: a is negative, so what lies further out, infinities and NaN are smaller numbers
   __device__ __forceinline__ bool holds(uint32_t u) const { return u >= least; }
-  __device__ __forceinline__ bool holds_first(uint32_t u) const { return u >= least_first; }
+  __device__ __forceinline__ bool holds_well(uint32_t u) const { return u >= least_well; }
 };
 
 struct KParams {
@@ -564,7 +562,9 @@ struct FwdTraits {
 //
 // KG > 1, for calls of few workgroups: one wave per SIMD takes 0.8 us per tile and two take 1.35, so KG groups of waves with a ring each
 // walk consecutive parts of the list of tiles and the first adds up what they leave in LDS.  Registers allow two waves per SIMD.
-template <class T>
+//
+// NEAR: a kernel with a soft-cap whose waves take NearCap's polynomial as long as their scores allow.
+template <class T, bool NEAR = false>
 __global__ __launch_bounds__(T::KG * T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_EU, T::WAVES_PER_EU)))
 void fwd_kernel(const KParams p) {
   constexpr int DQK = T::DQK, DV = T::DV, RW = T::RW, BN = T::BN, NW = T::NW, NT = T::NT, BM = T::BM;
@@ -764,17 +764,9 @@ void fwd_kernel(const KParams p) {
   // kernels are relative to the reference of the moment; it can move only on the path that recomputes a tile's
   // weights, which accounts for the difference.
   constexpr bool kFoldRef = kSoftcap && !kDrop;  // (the dropout instances have no registers to spare for it)
-  // A wave whose scores are small beside the cap walks with the polynomial; from the first tile on that has others it takes the exact form.
-  constexpr bool kNear = kFoldRef;
-  const NearCap near_cap = p.near_cap;
-  bool near = kNear;  // (uniform over the wave)
-  float alibi_r[kNear && kAlibi ? 16 : 1];  // the ALiBi term at the registers' offsets, ahead of NearCap's last factor (scalar registers)
-  if constexpr (kNear && kAlibi) {
-    // (this order of the factors: with the offset last the compiler multiplies by it in the loop, and spills)
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-      alibi_r[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, slope_l2 * (float)(8 * (i / 4) + i % 4) * near_cap.per_last)));
-  }
+  static_assert(!NEAR || kFoldRef, "the polynomial's addend takes the reference");
+  bool near = false;  // (uniform over the wave) the wave's next tile takes the polynomial
+  float alibi_r[NEAR && kAlibi ? 16 : 1];  // the ALiBi term at the registers' offsets, ahead of NearCap's last factor (scalar registers)
 
   // Gate logits of this lane's output elements, fetched before the key loop when they fit the register budget so that
   // their latency is not paid in the epilogue.
@@ -1036,10 +1028,10 @@ void fwd_kernel(const KParams p) {
                   tl2 = __builtin_fmaf(x, p.scale, bv[i]);  // natural units: one operation per score
                 } else {
                   if constexpr (kPoly) {
-                    const float u = near_cap.inner(x);
+                    const float u = p.near_cap.inner(x);
                     nearest = min(nearest, __float_as_uint(u));
-                    const float q = near_cap.outer(u);
-                    tl2 = __builtin_fmaf(kAlibi && i > 0 ? __builtin_fmaf(x, q, alibi_r[i]) : x * q, near_cap.last, cap_shift);
+                    const float q = p.near_cap.outer(u);
+                    tl2 = __builtin_fmaf(kAlibi && i > 0 ? __builtin_fmaf(x, q, alibi_r[i]) : x * q, p.near_cap.last, cap_shift);
                   } else if constexpr (kSoftcap) {
                     const float e = fast_exp2(x * cap_k1);
                     const float rc = fast_rcp(e + 1.0f);
@@ -1151,18 +1143,18 @@ void fwd_kernel(const KParams p) {
           }
       }
     };
-    // The scores of a wave's first tile, which nothing covers; they say which form the soft-cap starts with.
+    // The scores of a wave's first tile, which nothing covers; they say which form the soft-cap goes on with.
     auto first_scores = [&](f32x16 (&s)[KB][QB], int t) FL_INLINE {
       qk(s, 0);
-      if constexpr (kNear) {
-        uint32_t least = ~0u;
+      if constexpr (NEAR) {
+        float far = 0.f;
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
           for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) least = min(least, __float_as_uint(near_cap.inner(s[kb][qb][i])));
-        near = near && __builtin_amdgcn_ballot_w64(!near_cap.holds_first(least)) == 0;
+            for (int i = 0; i < 16; ++i) far = __builtin_fmaxf(far, __builtin_fabsf(s[kb][qb][i]));
+        near = __builtin_amdgcn_ballot_w64(!p.near_cap.holds_well(__float_as_uint(p.near_cap.inner(far)))) == 0;
       }
       score_mods(s, t, 0, std::false_type{});
     };
@@ -1647,10 +1639,14 @@ void fwd_kernel(const KParams p) {
           for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int qb = 0; qb < QB; ++qb) asm volatile("" : "+v"(sn[kb][qb]));
-          if (__builtin_amdgcn_ballot_w64(!near_cap.holds(nearest)) != 0) {
+          // From the first tile on that has scores beyond five sixths of the range the wave takes the exact form; only scores beyond the range
+          // itself are formed again, with nothing to cover that.
+          if (__builtin_amdgcn_ballot_w64(!p.near_cap.holds_well(nearest)) != 0) {
             near = false;
-            qk(sn, (slot + 1) % NS);
-            score_mods(sn, entry_tile(ent[1]), (slot + 1) % NS, std::false_type{});
+            if (__builtin_amdgcn_ballot_w64(!p.near_cap.holds(nearest)) != 0) {
+              qk(sn, (slot + 1) % NS);
+              score_mods(sn, entry_tile(ent[1]), (slot + 1) % NS, std::false_type{});
+            }
           }
         }
         __builtin_amdgcn_s_setprio(0);
@@ -1679,9 +1675,18 @@ void fwd_kernel(const KParams p) {
           return true;
         });
       };
-      // (two loops: the two forms as branches of one step spill)
-      if constexpr (kNear) {
-        while (more && near) steps(std::true_type{});
+      // (two loops: the two forms as branches of one step spill, and so does an exact loop that begins in the middle of a turn)
+      if constexpr (NEAR) {
+        if (near) {
+          if constexpr (kAlibi) {
+            // (this order of the factors: with the offset last the compiler multiplies by it in the loop, and spills)
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+              alibi_r[i] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, slope_l2 * (float)(8 * (i / 4) + i % 4) * p.near_cap.per_last)));
+          }
+          do steps(std::true_type{});
+          while (more && near);
+        }
       }
       while (more) steps(std::false_type{});
       // the run's last tile: no scores of a next tile to form; the step's transfers and barrier only if the workgroup

@@ -24,12 +24,14 @@ extern const int kNumInstances;
 
 constexpr int kMaxLdsBytes = 160 * 1024;  // per workgroup on gfx950
 
-template <class T>
+template <class T, bool NEAR = false>
 hipError_t launch_fwd(const KParams& kp, int grid, int lds_bytes, hipStream_t stream) {
-  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<T>),
+  if constexpr (!NEAR && (T::FEAT & F_SOFTCAP) && !(T::FEAT & F_DROPOUT))
+    if (kp.near_cap.last > 0.f) return launch_fwd<T, true>(kp, grid, lds_bytes, stream);
+  static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<T, NEAR>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
   if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL(fwd_kernel<T>, dim3(grid), dim3(T::KG * T::NT), lds_bytes, stream, kp);
+  hipLaunchKernelGGL((fwd_kernel<T, NEAR>), dim3(grid), dim3(T::KG * T::NT), lds_bytes, stream, kp);
   return hipGetLastError();
 }
 
