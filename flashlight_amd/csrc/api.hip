@@ -886,6 +886,13 @@ bool row_starts_products(const fl_attn_params* p) { return !(p->scale > 0.f) || 
 // 121 -> 116; of 5 entries 7.4 -> 7.7, of 8 with a bias in fp32 7.7 -> 9.5.
 bool shared_bias_by_chunk(int chunk_len) { return chunk_len >= 4; }
 
+int64_t streamed_bytes(const fl_attn_params* p) { return (int64_t)p->B * p->Hq * p->Lq * p->Dqk * 8; }
+// Whether the gradients touch rows two entries ahead (pairbias_bwd_kernel.h): operands that stay in the 256 MB of cache behind the L2s from the kernels
+// before arrive soon enough without (67 MB, 128 x 4 x 256 x 256 of head dim 64, 128 -> 130 us), and up to four stripes of a head have few rows to share out (400 x 8
+// x 128 100.2 -> 102.4, 1000 x 8 x 64 109 -> 115).  256 x 8 x 256 181 -> 164, 512 x 8 x 160 208 -> 195, 96 x 8 x 450 301 -> 241, 128 x 8 x 320 202 -> 202; head dim 64,
+// 64 x 8 x 512 376 -> 265, 100 x 8 x 256 156 -> 147.
+bool gradient_ahead(const fl_attn_params* p) { return streamed_bytes(p) > (int64_t)80 << 20 && p->Lk > 128; }
+
 // Whether *p (already validated) is a call the shared-bias stripe forward (stripe_kernel.h) takes.  Fills the kernel's parameters,
 // its wave count, and the number of workgroups and their LDS bytes.
 bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, int* waves, int64_t (&launch)[2]) {
@@ -1802,15 +1809,12 @@ int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* strea
   sp.chunk_len = x.chunk_len;
   sp.tiles = (sp.S + 31) / 32;
   sp.by_chunk = shared_bias_by_chunk(sp.chunk_len);
-  // (operands that stay in the 256 MB of cache behind the L2s from the kernels before arrive soon enough without: 67 MB, 128 x 4 x 256 x 256 of
-  // head dim 64, 128 -> 130 us)
-  sp.ahead = (int64_t)p->B * p->Hq * p->Lq * p->Dqk * 8 > (int64_t)80 << 20;
   sp.s_pad = (sp.S + 3) / 4 * 4;
   sp.scale = p->scale;
   sp.scale_log2 = p->scale * 1.4426950408889634f;
   sp.dbias_part = b->dbias ? reinterpret_cast<float*>(ws + x.part) : nullptr;
   const fl::SBShape shape = fl::pairbias_bwd_shape(p->Dqk, sp.S);
-  e = (f16 ? fl::launch_pairbias_bwd_f16 : fl::launch_pairbias_bwd_bf16)(p->Dqk, shape, sp, stream);
+  e = (f16 ? fl::launch_pairbias_bwd_f16 : fl::launch_pairbias_bwd_bf16)(p->Dqk, shape, gradient_ahead(p), sp, stream);
   if (e != hipSuccess) return fail((int)e, "shared-bias backward: launch failed: %s", hipGetErrorString(e));
   if (b->dbias) {
     e = (f16 ? fl::launch_pairbias_bwd_reduce_f16 : fl::launch_pairbias_bwd_reduce_bf16)(f32, sp, b->dbias, stream);

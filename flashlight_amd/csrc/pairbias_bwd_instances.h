@@ -17,11 +17,11 @@ constexpr SBShape pairbias_bwd_shape(int d, int s) {
   x.nb = blocks <= 4 ? 1 : blocks <= 8 ? (d == 32 ? 2 : 1) : 2;
   x.waves = (blocks + x.nb - 1) / x.nb;
   const int slot = x.waves * (x.nb * 128 * d + 512) + 128 * d + 512;
-  x.lds_bytes = (2 * slot <= 160 * 1024 ? 2 : 1) * slot + 256;
+  x.lds_bytes = (2 * slot <= 160 * 1024 ? 2 : 1) * slot;
   return x;
 }
-hipError_t launch_pairbias_bwd_bf16(int d, const SBShape& shape, const SBParams& p, hipStream_t stream);
-hipError_t launch_pairbias_bwd_f16(int d, const SBShape& shape, const SBParams& p, hipStream_t stream);
+hipError_t launch_pairbias_bwd_bf16(int d, const SBShape& shape, bool ahead, const SBParams& p, hipStream_t stream);
+hipError_t launch_pairbias_bwd_f16(int d, const SBShape& shape, bool ahead, const SBParams& p, hipStream_t stream);
 hipError_t launch_pairbias_bwd_prep_bf16(int d, bool gate, const SBPrepParams& p, hipStream_t stream);
 hipError_t launch_pairbias_bwd_prep_f16(int d, bool gate, const SBPrepParams& p, hipStream_t stream);
 // bias_f32: the bias gradient's type, fp32 or the element type

@@ -43,14 +43,14 @@ struct SBParams {
   int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
   int32_t tiles;                   // 32-row stripes
   int32_t by_chunk;                // see StripePlace
-  int32_t ahead;                   // rows are touched two entries ahead
   int32_t s_pad;                   // row length of the partial bias gradient (S rounded up to 4)
   float scale, scale_log2;
   float* dbias_part;               // [groups][chunks][H][S][s_pad], or null: no gradient of the bias wanted
 };
 
 // rows of an operand that are not in the sequence repeat the last one; their weights are 0 (their bias is -inf)
-template <int D_, int ROLE_, int NB_, int NW_, bool ROWB_, class Elem_>
+// AHEAD: rows are touched two entries ahead of their use
+template <int D_, int ROLE_, int NB_, int NW_, bool ROWB_, class Elem_, bool AHEAD_ = false>
 struct SBTraits {
   using Elem = Elem_;
   static constexpr int D = D_, ROLE = ROLE_, NB = NB_, NW = NW_;
@@ -67,7 +67,8 @@ struct SBTraits {
   static constexpr int SLOT_BYTES = NW * W_BYTES + S_OWN;  // one batch entry
   // tiles of batch entries resident in LDS
   static constexpr int SLOTS = 2 * SLOT_BYTES <= 160 * 1024 ? 2 : 1;
-  static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES + 256;  // (and where touch() puts what nothing reads)
+  static constexpr bool AHEAD = AHEAD_;
+  static constexpr int LDS_BYTES = SLOTS * SLOT_BYTES + (AHEAD ? 256 : 0);  // (and where touch() puts what nothing reads)
   // the partial sums go where the consumed tiles were: both sets at once when a wave's two tiles have room for them
   static constexpr bool ONE_PASS = DQ || 2 * T_BYTES >= 2 * PARK;
 };
@@ -227,9 +228,10 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
   // that they will all ask for, a cache line per lane.  The stripes ask for the same rows at the same time, so that little is on its way
   // from memory although every wave has an entry in flight: us, forward and gradients, 256 x 8 x 256 x 256, 274 -> 258; 512 entries 562 -> 502;
   // 150 x 8 x 333 x 333, head dim 64, 799 -> 723.
-  const int ahead_end = __builtin_amdgcn_readfirstlane(wave == 0 && p.ahead ? n1 : 0);
+  // (A kernel of its own: the addresses alone were 2 to 4 % of a call of 30 us.)
+  const int ahead_end = T::AHEAD && wave == 0 ? n1 : 0;
   uint64_t ahead_at = 0, ahead_step = 0;
-  {
+  if constexpr (T::AHEAD) {
     const bool second = lane >= 32;
     const bf16_t* base = kDQ ? (second ? p.v : p.k) : (second ? p.dout : p.q);
     const int64_t b = kDQ ? (second ? p.vs[0] : p.ks[0]) : (second ? p.dos[0] : p.qs[0]);
@@ -238,8 +240,9 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
     ahead_at = (uint64_t)(base + (int64_t)(n0 + 1) * b + (int64_t)head * hd + (int64_t)min(own, S - 1) * sq);
     ahead_step = (uint64_t)(b * 2);
   }
-  auto touch_entry = [&](int n) FL_INLINE {  // n: n0 + 1, n0 + 2, ... in this order
-    if (n < ahead_end) {
+  // n: n0 + 1, n0 + 2, ... in this order.  (Only where entry n exists: the wait at the top of the walk's next entry, or of that after it, covers it.)
+  auto touch_entry = [&](int n) FL_INLINE {
+    if (T::AHEAD && n < ahead_end) {
       touch(ahead_at, lds0 + T::SLOTS * slot_bytes);
       ahead_at += ahead_step;
     }

@@ -4,11 +4,11 @@
 
 namespace fl {
 namespace {
-template <int D, int NB, int NW, bool ROWB, class E>
+template <int D, int NB, int NW, bool ROWB, class E, bool AHEAD>
 hipError_t launch_one(const SBParams& p, hipStream_t stream) {
-  using TQ = SBTraits<D, 0, NB, NW, ROWB, E>;
-  using TKV = SBTraits<D, 1, NB, NW, ROWB, E>;
-  static_assert(TQ::LDS_BYTES == pairbias_bwd_shape(D, 32 * NB * NW).lds_bytes, "one rule");
+  using TQ = SBTraits<D, 0, NB, NW, ROWB, E, AHEAD>;
+  using TKV = SBTraits<D, 1, NB, NW, ROWB, E, AHEAD>;
+  static_assert(TQ::SLOTS * TQ::SLOT_BYTES == pairbias_bwd_shape(D, 32 * NB * NW).lds_bytes, "one rule");
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pairbias_bwd_kernel<TQ, TKV>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, TQ::LDS_BYTES);
   if (attr != hipSuccess) return attr;
@@ -19,18 +19,19 @@ hipError_t launch_one(const SBParams& p, hipStream_t stream) {
 }
 // the shapes that pairbias_bwd_shape names
 template <int D, bool ROWB, class E, int BLOCKS = 16>
-hipError_t launch_shape(const SBShape& shape, const SBParams& p, hipStream_t stream) {
+hipError_t launch_shape(const SBShape& shape, bool ahead, const SBParams& p, hipStream_t stream) {
   if constexpr (BLOCKS > 0) {
     constexpr SBShape x = pairbias_bwd_shape(D, 32 * BLOCKS);
-    if (shape.nb == x.nb && shape.waves == x.waves) return launch_one<D, x.nb, x.waves, ROWB, E>(p, stream);
-    return launch_shape<D, ROWB, E, BLOCKS - 1>(shape, p, stream);
+    if (shape.nb == x.nb && shape.waves == x.waves)
+      return ahead ? launch_one<D, x.nb, x.waves, ROWB, E, true>(p, stream) : launch_one<D, x.nb, x.waves, ROWB, E, false>(p, stream);
+    return launch_shape<D, ROWB, E, BLOCKS - 1>(shape, ahead, p, stream);
   }
   return hipErrorInvalidValue;
 }
 template <class E>
-hipError_t launch_any(int d, const SBShape& shape, const SBParams& p, hipStream_t stream) {
-  if (d == 32) return p.rowb ? launch_shape<32, true, E>(shape, p, stream) : launch_shape<32, false, E>(shape, p, stream);
-  if (d == 64) return p.rowb ? launch_shape<64, true, E>(shape, p, stream) : launch_shape<64, false, E>(shape, p, stream);
+hipError_t launch_any(int d, const SBShape& shape, bool ahead, const SBParams& p, hipStream_t stream) {
+  if (d == 32) return p.rowb ? launch_shape<32, true, E>(shape, ahead, p, stream) : launch_shape<32, false, E>(shape, ahead, p, stream);
+  if (d == 64) return p.rowb ? launch_shape<64, true, E>(shape, ahead, p, stream) : launch_shape<64, false, E>(shape, ahead, p, stream);
   return hipErrorInvalidValue;
 }
 template <int D, bool GATE, class E>
@@ -61,8 +62,8 @@ typedef f16_t sb_elem;
 #define FL_SB_NAME(x) x##_bf16
 typedef bf16_t sb_elem;
 #endif
-hipError_t FL_SB_NAME(launch_pairbias_bwd)(int d, const SBShape& shape, const SBParams& p, hipStream_t stream) {
-  return launch_any<sb_elem>(d, shape, p, stream);
+hipError_t FL_SB_NAME(launch_pairbias_bwd)(int d, const SBShape& shape, bool ahead, const SBParams& p, hipStream_t stream) {
+  return launch_any<sb_elem>(d, shape, ahead, p, stream);
 }
 hipError_t FL_SB_NAME(launch_pairbias_bwd_prep)(int d, bool gate, const SBPrepParams& p, hipStream_t stream) {
   return launch_prep<sb_elem>(d, gate, p, stream);
