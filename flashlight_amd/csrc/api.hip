@@ -879,14 +879,18 @@ int64_t chunks_of_entries(int64_t heads_and_groups, int64_t tiles, int per_cu, i
 // has to stay an ordinary number.  (A scale that has not been set yet is no reason against it.)
 bool row_starts_products(const fl_attn_params* p) { return !(p->scale > 0.f) || (p->scale >= 0x1p-100f && p->scale <= 0x1p100f); }
 
-// Whether the heads of a chunk of entries share an XCD in the shared-bias kernels that walk over entries.  With operands as the Evoformer has them a
-// head's row is half of a cache line at head dim 32: heads on XCDs of their own bring every line into two L2s (forward and gradients, 128 x 8 x
-// 256 x 256: 67 instead of 134 MB read by each).  A head's bias is then read by every XCD, which short chunks do not pay for.  us, heads apart ->
-// together: gradients with their forward, 256 x 8 x 256 x 256, 268 -> 258, 512 entries 567 -> 502, 150 x 8 x 333 x 333, head dim 64, 755 -> 723; forwards, 512 x 8 x 160 x 160,
-// 121 -> 116; of 5 entries 7.4 -> 7.7, of 8 with a bias in fp32 7.7 -> 9.5.
-bool shared_bias_by_chunk(int chunk_len) { return chunk_len >= 4; }
-
+// Whether neighbours among the (chunk of entries, head) pairs share an XCD in the shared-bias kernels that walk over entries (StripePlace), and are not
+// dealt round the XCDs.  With operands as the Evoformer has them a head's row is half of a cache line at head dim 32, and dealt round every line comes into
+// two L2s (forward and gradients, 128 x 8 x 256 x 256: 134 MB read by each, 67 by neighbours: four pairs to an XCD there, half of a chunk's heads).  What
+// it costs is a bias read by more XCDs.  us, dealt round -> neighbours.
+// Forward, from chunks of 5 entries on: 400 x 4 x 100 (chunks of 5) 23.7 -> 23.3; 50 x 4 x 333, head dim 64 (5), 41.5 -> 40.7; 150 x 8 x 250 (10) 44.4 ->
+// 44.0; 512 x 8 x 160 105.6 -> 102.6; 150 x 8 x 333, head dim 64, 288 -> 244; even or 1 % at most: 96 x 8 x 256 (6), 96 x 8 x 450.  Chunks of 4: 64 x 8 x 256 20.5 -> 20.8.
+bool forward_neighbours(int chunk_len) { return chunk_len >= 5; }
+// Gradients, where q, k, v and dout are more than 24 MB: 96 x 7 x 160 (28 MB) 49.9 -> 48.1; 40 x 8 x 384 (31) 101 -> 91.7; 80 x 8 x 200 (33) 60.0 -> 58.0; 400 x 4 x
+// 100 (41) 52.2 -> 49.0; 72 x 8 x 190, head dim 64 (56), 94.8 -> 87.3; 128 x 8 x 256 (67) 101.4 -> 99.3; 256 x 8 x 130 (68) 108 -> 102; but 64 x 8 x 256 (34) 56.8 -> 57.7.
+// Below it the L2s hold both copies: 20 x 8 x 300 (12) 42.6 -> 43.3, 32 x 8 x 256 (17) 32.1 -> 33.9, 128 x 4 x 128 (17) 22.4 -> 22.8, 100 x 8 x 100 (20) 28.8 -> 29.3.
 int64_t streamed_bytes(const fl_attn_params* p) { return (int64_t)p->B * p->Hq * p->Lq * p->Dqk * 8; }
+bool gradient_neighbours(const fl_attn_params* p) { return streamed_bytes(p) > (int64_t)24 << 20; }
 // Whether the gradients touch rows two entries ahead (pairbias_bwd_kernel.h): operands that stay in the 256 MB of cache behind the L2s from the kernels
 // before arrive soon enough without (67 MB, 128 x 4 x 256 x 256 of head dim 64, 128 -> 130 us), and up to four stripes of a head have few rows to share out (400 x 8
 // x 128 100.2 -> 102.4, 1000 x 8 x 64 109 -> 115).  256 x 8 x 256 181 -> 164, 512 x 8 x 160 208 -> 195, 96 x 8 x 450 301 -> 241, 128 x 8 x 320 202 -> 202; head dim 64,
@@ -969,7 +973,6 @@ bool plan_stripe(const fl_attn_params* p, void* ungated, fl::StripeParams* out, 
   k.chunk_len = (int)((k.div + most - 1) / most);
   k.chunks = (k.div + k.chunk_len - 1) / k.chunk_len;
   if (units * k.chunks > (1 << 28)) return false;
-  k.by_chunk = shared_bias_by_chunk(k.chunk_len);
   *out = k;
   *waves = shape.waves;
   launch[0] = ((int64_t)k.groups * k.chunks * k.H + 7) / 8 * 8 * k.tiles;
@@ -1250,7 +1253,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
     int waves = 0;
     int64_t plan[2];
     if (plan_stripe(p, ungated, &sp, &waves, plan)) {
-      const hipError_t e = (p->dtype == FL_F16 ? fl::launch_stripe_f16 : fl::launch_stripe_bf16)(p->Dqk, waves, sp, stream);
+      const hipError_t e = (p->dtype == FL_F16 ? fl::launch_stripe_f16 : fl::launch_stripe_bf16)(p->Dqk, waves, forward_neighbours(sp.chunk_len), sp, stream);
       if (e != hipSuccess) return fail((int)e, "launch of the shared-bias stripe forward failed: %s", hipGetErrorString(e));
       return 0;
     }
@@ -1808,7 +1811,7 @@ int fl_attn_shared_bias_bwd(const fl_attn_shared_bias_bwd_params* b, void* strea
   sp.chunks = x.chunks;
   sp.chunk_len = x.chunk_len;
   sp.tiles = (sp.S + 31) / 32;
-  sp.by_chunk = shared_bias_by_chunk(sp.chunk_len);
+  sp.neighbours = gradient_neighbours(p);
   sp.s_pad = (sp.S + 3) / 4 * 4;
   sp.scale = p->scale;
   sp.scale_log2 = p->scale * 1.4426950408889634f;

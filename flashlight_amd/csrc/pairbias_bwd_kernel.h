@@ -42,7 +42,7 @@ struct SBParams {
   int32_t B, H, S;
   int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
   int32_t tiles;                   // 32-row stripes
-  int32_t by_chunk;                // see StripePlace
+  int32_t neighbours;              // see StripePlace
   int32_t s_pad;                   // row length of the partial bias gradient (S rounded up to 4)
   float scale, scale_log2;
   float* dbias_part;               // [groups][chunks][H][S][s_pad], or null: no gradient of the bias wanted
@@ -93,7 +93,7 @@ __device__ __forceinline__ void pairbias_bwd_stripe(const SBParams& p, const int
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r = lane % 32, h = lane / 32;
 
-  const StripePlace place(p, block);
+  const StripePlace place(p, block, p.neighbours != 0);
   if (place.none(p)) return;  // (before any barrier)
   const int tile = place.tile, head = place.unit % p.H, gc = place.unit / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
   const int n0 = group * p.div + chunk * p.chunk_len, n1 = min(group * p.div + p.div, n0 + p.chunk_len);

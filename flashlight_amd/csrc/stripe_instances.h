@@ -16,6 +16,6 @@ constexpr StripeShape stripe_shape(int d, int lk, bool row) {
   x.per_cu = 8 / x.waves < 160 * 1024 / x.lds_bytes ? 8 / x.waves : 160 * 1024 / x.lds_bytes;
   return x;
 }
-hipError_t launch_stripe_bf16(int d, int waves, const StripeParams& p, hipStream_t stream);
-hipError_t launch_stripe_f16(int d, int waves, const StripeParams& p, hipStream_t stream);
+hipError_t launch_stripe_bf16(int d, int waves, bool neighbours, const StripeParams& p, hipStream_t stream);
+hipError_t launch_stripe_f16(int d, int waves, bool neighbours, const StripeParams& p, hipStream_t stream);
 }  // namespace fl

@@ -17,8 +17,9 @@
 // products, exponentials, sums over the waves, stores: about 600 instructions per wave, 350 of them for its four blocks of
 // 32 x 32) with two waves per SIMD to cover it.  Two blocks of queries per wave share the K and V operands, and halve what is
 // exchanged per score against one (128 x 8 x 256 x 256, head dim 32, gate and row: 61 us with one; head dim 64 has no registers
-// for two).  Head dim 32 is at the limit of the 256 registers that two waves per SIMD leave: with three waves, or two and a bias row, one
-// value goes to scratch and comes back once per batch entry, with one wave and a row nine do; the other shapes fit.  Wave counts are compiled in: sums over a run-time count wait for one LDS read after the other (55 us against 39).
+// for two).  Head dim 32 is at the limit of the 256 registers that two waves per SIMD leave: with a bias row and up to three waves 12 to 72 bytes
+// of a lane go to scratch, without one and up to four waves 12 to 36 (one and two waves that take neighbours: 68 and 100); the other shapes
+// fit.  Wave counts are compiled in: sums over a run-time count wait for one LDS read after the other (55 us against 39).
 // bf16, general kernel -> here: 128 x 8 x 256 x 256, head dim 32, gate, row and statistics: 48 -> 39 us; 2 x 207 x 4 x 494 x 494, head
 // dim 32: 806 -> 201; 2 x 17 x 4 x 235 x 235, head dim 64, gate and row: 43 -> 17; 28 x 4 x 106 x 106, head dim 32, gate: 14 -> 6.
 #pragma once
@@ -43,16 +44,16 @@ struct StripeParams {
   int32_t B, H, Lq, Lk;
   int32_t div, groups, chunks, chunk_len;  // batch entries per bias; groups = B / div; entries are cut into chunks of chunk_len
   int32_t tiles;                       // stripes of 32 QB rows
-  int32_t by_chunk;                    // see StripePlace
   int32_t by_maximum;                  // weights are formed against the row's maximum from the start
   float scale, scale_log2;
 };
 
-template <int D_, int QB_, int NB_, int NW_, bool ROW_, class Elem_>
+// NEIGHBOURS: see StripePlace (compiled in: its arithmetic was 0.1 us of a call of 8)
+template <int D_, int QB_, int NB_, int NW_, bool ROW_, class Elem_, bool NEIGHBOURS_ = false>
 struct StripeTraits {
   using Elem = Elem_;
   static constexpr int D = D_, QB = QB_, NB = NB_, NW = NW_;
-  static constexpr bool ROW = ROW_;
+  static constexpr bool ROW = ROW_, NEIGHBOURS = NEIGHBOURS_;
   static constexpr int KS = D / 16, DB = D / 32;
   static constexpr int T_BYTES = NB * 32 * D * 2;  // K or V rows of one wave
   static constexpr int W_BYTES = 2 * T_BYTES;
@@ -96,7 +97,7 @@ void stripe_kernel(const StripeParams p) {
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
   const int r = lane % 32, h = lane / 32;
 
-  const StripePlace place(p, blockIdx.x);
+  const StripePlace place(p, blockIdx.x, T::NEIGHBOURS);
   if (place.none(p)) return;  // (before any barrier)
   const int tile = place.tile, head = place.unit % p.H, gc = place.unit / p.H, chunk = gc % p.chunks, group = gc / p.chunks;
   const int n0 = group * p.div + chunk * p.chunk_len, n1 = min(group * p.div + p.div, n0 + p.chunk_len);

@@ -4,9 +4,9 @@
 
 namespace fl {
 namespace {
-template <int D, int QB, int NW, bool ROW, class E>
+template <int D, int QB, int NW, bool ROW, class E, bool NEIGHBOURS>
 hipError_t launch_one(const StripeParams& p, hipStream_t stream) {
-  using T = StripeTraits<D, QB, 2, NW, ROW, E>;
+  using T = StripeTraits<D, QB, 2, NW, ROW, E, NEIGHBOURS>;
   static_assert(T::LDS_BYTES == stripe_shape(D, 64 * NW, ROW).lds_bytes && T::PER_CU == stripe_shape(D, 64 * NW, ROW).per_cu, "one rule");
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&stripe_kernel<T>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS_BYTES);
@@ -16,28 +16,28 @@ hipError_t launch_one(const StripeParams& p, hipStream_t stream) {
   return hipGetLastError();
 }
 template <int D, int QB, bool ROW, class E, int NW = 8>
-hipError_t launch_waves(int waves, const StripeParams& p, hipStream_t stream) {
+hipError_t launch_waves(int waves, bool neighbours, const StripeParams& p, hipStream_t stream) {
   if constexpr (NW > 0) {
-    if (waves == NW) return launch_one<D, QB, NW, ROW, E>(p, stream);
-    return launch_waves<D, QB, ROW, E, NW - 1>(waves, p, stream);
+    if (waves == NW) return neighbours ? launch_one<D, QB, NW, ROW, E, true>(p, stream) : launch_one<D, QB, NW, ROW, E, false>(p, stream);
+    return launch_waves<D, QB, ROW, E, NW - 1>(waves, neighbours, p, stream);
   }
   return hipErrorInvalidValue;
 }
 template <class E>
-hipError_t launch_any(int d, int waves, const StripeParams& p, hipStream_t stream) {
-  if (d == 32) return p.row ? launch_waves<32, 2, true, E>(waves, p, stream) : launch_waves<32, 2, false, E>(waves, p, stream);
-  if (d == 64) return p.row ? launch_waves<64, 1, true, E>(waves, p, stream) : launch_waves<64, 1, false, E>(waves, p, stream);
+hipError_t launch_any(int d, int waves, bool neighbours, const StripeParams& p, hipStream_t stream) {
+  if (d == 32) return p.row ? launch_waves<32, 2, true, E>(waves, neighbours, p, stream) : launch_waves<32, 2, false, E>(waves, neighbours, p, stream);
+  if (d == 64) return p.row ? launch_waves<64, 1, true, E>(waves, neighbours, p, stream) : launch_waves<64, 1, false, E>(waves, neighbours, p, stream);
   return hipErrorInvalidValue;
 }
 }  // namespace
 
 #if defined(FL_INST_F16) && FL_INST_F16
-hipError_t launch_stripe_f16(int d, int waves, const StripeParams& p, hipStream_t stream) {
-  return launch_any<f16_t>(d, waves, p, stream);
+hipError_t launch_stripe_f16(int d, int waves, bool neighbours, const StripeParams& p, hipStream_t stream) {
+  return launch_any<f16_t>(d, waves, neighbours, p, stream);
 }
 #else
-hipError_t launch_stripe_bf16(int d, int waves, const StripeParams& p, hipStream_t stream) {
-  return launch_any<bf16_t>(d, waves, p, stream);
+hipError_t launch_stripe_bf16(int d, int waves, bool neighbours, const StripeParams& p, hipStream_t stream) {
+  return launch_any<bf16_t>(d, waves, neighbours, p, stream);
 }
 #endif
 }  // namespace fl

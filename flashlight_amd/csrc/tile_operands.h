@@ -49,15 +49,15 @@ __device__ __forceinline__ void touch(uint64_t lane_address, unsigned lds_base) 
 }
 
 // Workgroup -> (group of batch entries that share the bias, chunk of them, head, stripe): the stripes of one (chunk, head) read the
-// same tensors and stay on one XCD.  unit: (group, chunk, head) as one number; `none`: a workgroup past the last of them.  by_chunk: the heads of
-// a chunk on one XCD, otherwise (chunk, head) pairs in turn (shared_bias_by_chunk in api.hip).
+// same tensors and stay on one XCD.  unit: (group, chunk, head) as one number; `none`: a workgroup past the last of them.  neighbours: an XCD takes
+// an eighth of the units that follow each other, otherwise every eighth unit (forward_neighbours and gradient_neighbours in api.hip).
 struct StripePlace {
   int tile, unit;
   template <class P, class Block>
-  __device__ __forceinline__ StripePlace(const P& p, const Block block) {
+  __device__ __forceinline__ StripePlace(const P& p, const Block block, const bool neighbours) {
     const int x = block % 8, i = block / 8, each = (p.groups * p.chunks * p.H + 7) / 8, of_x = i / p.tiles;
     tile = i % p.tiles;
-    unit = !p.by_chunk ? of_x * 8 + x : of_x < each ? x * each + of_x : 8 * each;
+    unit = !neighbours ? of_x * 8 + x : of_x < each ? x * each + of_x : 8 * each;
   }
   template <class P>
   __device__ __forceinline__ bool none(const P& p) const { return unit >= p.groups * p.chunks * p.H; }
