@@ -601,6 +601,7 @@ int groups_for(const fl::Instance* in, const fl_attn_params* p) {
 // 20.2 -> 18.3 / 20.4 / 20.3; 4 x 16 x 700, head dim 128, 26.4 -> 24.5 / 26.7 / 26.8; 4 x 16 x 1024 42.9 -> 38.5 / 43.3 / 43.3; under a window of 256, 4 x 16 x 4096,
 // head dim 64, 55.2 -> 51.4 / 55.9 / 55.9; 4 x 16 over 4 x 2048, causal, 75.1 -> 63.6 / 75.5 / 74.8.
 bool near_cap_pays(const fl_attn_params* p, const fl::Instance* in, int groups, int64_t grid) {
+  if (!fl::has_near(in->feat)) return false;
   // keys of a wave's longest walk, times the waves (of which two per SIMD run at once, and one alone takes as long as half a pair)
   const int64_t walk = p->mask_kind == FL_MASK_SLIDING ? std::min<int64_t>(p->Lk, (int64_t)p->window + in->rw * in->nw) : p->Lk;
   return walk / groups * std::max<int64_t>(1024, grid * in->nw * groups) >= (int64_t)1024 * 1024;

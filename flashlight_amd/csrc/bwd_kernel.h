@@ -698,7 +698,10 @@ __device__ __forceinline__ void bwd_tile(const BParams& p, const int block, cons
                 for (int g = 0; g < 4; ++g) {
 #pragma unroll
                   for (int off = 8 * g; off < 8 * g + 4; ++off) out[sb] |= *reinterpret_cast<const int64_t*>(ids + off * 8) == odoc ? 0u : 1u << off;
-                  asm volatile("" : "+v"(out[sb]));  // (a branch, and four ids at a time: sixteen spill)
+                  // (a branch, and four ids at a time, which leaves scratch of 8 bytes a lane where head dim 64 has both roles in one launch and of 20 in
+                  // dK and dV at 128.  Two leave none at 64 and the same 20 at 128, but gradients of documents take longer: 4 x 16 x 2048, head dim 64,
+                  // 112 -> 114, 16 over 4 x 8000 163 -> 169, 2 x 16 x 4096, head dim 128, 261 -> 268; in a loop 36 bytes; sixteen at once spill.)
+                  asm volatile("" : "+v"(out[sb]));
                 }
               }
             }

@@ -24,9 +24,14 @@ extern const int kNumInstances;
 
 constexpr int kMaxLdsBytes = 160 * 1024;  // per workgroup on gfx950
 
+// Whether a set of features has a kernel with NearCap's polynomial beside that with the exponential (near_cap_pays in api.hip).  With bias operands, whose
+// reads and additions are what the loop waits for, it is behind: 2 x 8 x 1024, dense bias and gate, head dim 128, 43.1 us -> 50.0 with the scores in its range
+// throughout, 45.9 where they leave it; head dim 64 37.1 -> 36.0 and 38.8.
+constexpr bool has_near(uint32_t feat) { return (feat & F_SOFTCAP) && !(feat & (F_DROPOUT | F_BIAS)); }
+
 template <class T, bool NEAR = false>
 hipError_t launch_fwd(const KParams& kp, int grid, int lds_bytes, hipStream_t stream) {
-  if constexpr (!NEAR && (T::FEAT & F_SOFTCAP) && !(T::FEAT & F_DROPOUT))
+  if constexpr (!NEAR && has_near(T::FEAT))
     if (kp.near_cap.last > 0.f) return launch_fwd<T, true>(kp, grid, lds_bytes, stream);
   static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_kernel<T, NEAR>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);

@@ -208,6 +208,7 @@ def _attended(kind, S):
     ("causal", 64, torch.bfloat16, True, False, 4200, 2), ("none", 128, torch.float16, False, False, 2150, 2),
     ("window", 64, torch.bfloat16, True, False, 1093, 1), ("window", 128, torch.float16, False, False, 1093, 1),
     ("documents", 64, torch.bfloat16, True, False, 1093, 1), ("documents", 128, torch.float16, True, False, 1093, 1),
+    # (bias operands: the exponential throughout)
     ("none", 64, torch.bfloat16, False, True, 1096, 3), ("none", 128, torch.float16, True, True, 1096, 3),
     ("causal", 64, torch.float16, False, True, 1093, 3), ("none", 32, torch.bfloat16, False, True, 1096, 3)])
 def test_waves_that_leave_the_polynomial_on_the_way(kind, D, dtype, alibi, bias, S, heads, far):
