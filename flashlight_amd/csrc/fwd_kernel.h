@@ -967,11 +967,13 @@ void fwd_kernel(const KParams p) {
     auto entry_tile = [&](uint32_t e) FL_INLINE  { return (int)(__builtin_amdgcn_readfirstlane(e) & 0xffffu); };
     auto entry_class = [&](uint32_t e) FL_INLINE  { return (int)((__builtin_amdgcn_readfirstlane(e) >> (16 + 2 * wave)) & 3u); };
 
-    // whether some wave may look at the ids of the entry's tile: not when it is FULL or ONE_DOC (class bits 10 and 11) for every
+    // Documents: the ids as bits of the mask's word (apply_mask), where the registers allow
+    constexpr bool kIdBits = kDoc && DQK <= 128;
+    // whether some wave may look at the ids of the entry's tile: not when it is FULL or, with ids as bits, ONE_DOC (class bits 10 and 11) for every
     // wave.  (A tile that is EMPTY for a wave can still lie inside that wave's run, where it is computed and masked.)
     auto entry_masked = [&](uint32_t e) FL_INLINE {
-      constexpr uint32_t kHigh = 0xAAAAu & ((1u << (2 * NW)) - 1u);
-      return ((__builtin_amdgcn_readfirstlane(e) >> 16) & kHigh) != kHigh;
+      constexpr uint32_t kAll = (1u << (2 * NW)) - 1u, kLook = kIdBits ? 0xAAAAu & kAll : kAll;
+      return ((__builtin_amdgcn_readfirstlane(e) >> 16) & kLook) != (0xAAAAu & kAll);
     };
 
     // ---- S^T = K . Q^T for one tile: A = K fragment from LDS, B = Q fragment ---------------------------------------
@@ -1172,28 +1174,45 @@ void fwd_kernel(const KParams p) {
         const int kbase = k0 + 32 * kb + 4 * h;
         const int t_len = p.Lk - kbase;   // off < t_len   <=> key < Lk
         const int t_pfx = p.pfx - kbase;  // off < t_pfx   <=> key < pfx
+        // Under a document mask the ids of this lane's 16 keys come from the wave's LDS image of the tile's ids (it
+        // arrived with the V tile in ring slot `vslot`): four runs of four consecutive keys.
+        typedef int64_t i64x2 __attribute__((ext_vector_type(2)));
+        auto two_ids = [&](int g, int e2) FL_INLINE -> i64x2 {
+          return *reinterpret_cast<const i64x2*>(smem + T::I_OFF + vslot * T::IBYTES + wave * (BN * 8) + (32 * kb + 4 * h + 8 * g + 2 * e2) * 8);
+        };
+        i64x2 ids[kDoc && !kIdBits ? 8 : 1];
+        if constexpr (kDoc && !kIdBits) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) ids[i] = two_ids(i / 2, i % 2);
+        }
 #pragma unroll
         for (int qb = 0; qb < QB; ++qb) {
           const int rel = kbase - qrow[qb];
           // off <= hi <=> key < Lk && (key - q <= dmax || key < pfx);  off >= lo <=> key - q >= dmin
           const int hi = min(t_len - 1, max(p.dmax - rel, t_pfx - 1));
           const int lo = p.dmin - rel;
+          if constexpr (kDoc && !kIdBits) {
+            // (head dims above 128 have no registers for the word and its branch: 2 x 8 x 1000, head dim 256, 27.8 -> 29.8, with ALiBi and a soft-cap 33.8 -> 36.6)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int off = 8 * (i / 4) + (i % 4);
+              const bool ok = (off <= hi) & (off >= lo) & (ids[i / 2][i % 2] == qdoc[qb]);
+              s[kb][qb][i] = ok ? s[kb][qb][i] : -INFINITY;
+            }
+            continue;
+          }
           unsigned out = outside_word(lo, hi);
-          // Under a document mask the ids of this lane's 16 keys come from the wave's LDS image of the tile's ids (it
-          // arrived with the V tile in ring slot `vslot`): four runs of four consecutive keys.  Most masked tiles hold the diagonal of one
-          // document (ONE_DOC), where the positions alone decide and no ids are fetched.  (The ids' part is a branch around a word of bits, which the
-          // choice takes; as comparisons of ids and positions at every score: us, causal, 16 heads of 16384, head dim 64, 144.7 -> 137.8; 4 x 16 x
+          // Most masked tiles hold the diagonal of one document (ONE_DOC), where the positions alone decide and no ids are fetched.  (The ids' part
+          // is a branch around a word of bits, which the choice takes; as comparisons of ids and positions at every score: us, causal, 16 heads of 16384, head dim 64, 144.7 -> 137.8; 4 x 16 x
           // 2048 47.4 -> 42.2; 4 x 16 x 4096, head dim 128, 153.3 -> 146.9.  The choice itself in both forms, behind a branch, was 155.6 in the
           // first.)
-          if constexpr (kDoc) {
+          if constexpr (kIdBits) {
             if (cls != TILE_ONE_DOC) {
-              typedef int64_t i64x2 __attribute__((ext_vector_type(2)));
-              const unsigned char* il = smem + T::I_OFF + vslot * T::IBYTES + wave * (BN * 8) + (32 * kb + 4 * h) * 8;
 #pragma unroll
               for (int g = 0; g < 4; ++g)
 #pragma unroll
                 for (int e2 = 0; e2 < 2; ++e2) {
-                  const i64x2 two = *reinterpret_cast<const i64x2*>(il + (8 * g + 2 * e2) * 8);
+                  const i64x2 two = two_ids(g, e2);
 #pragma unroll
                   for (int e = 0; e < 2; ++e) out |= two[e] == qdoc[qb] ? 0u : 1u << (8 * g + 2 * e2 + e);
                 }

@@ -53,3 +53,23 @@ def test_ids_that_alternate_and_come_back(D):
     for ids in (n % 2, n // 70 % 2, (n * 7919) % 5 - 2):  # every tile has several, in runs of every length
         for causal in (False, True):
             _check(ids, D, 2, causal)
+
+
+@pytest.mark.parametrize("D", [256, 512])
+@pytest.mark.parametrize("causal", [False, True])
+def test_head_dims_whose_masked_tiles_compare_ids_at_every_score(D, causal):
+    S, H = 229, 2
+    n = torch.arange(S)
+    for ids in (torch.full((S,), -5), n // 70, (n * 7919) % 3, (n >= 101).long() << 40):
+        g = torch.Generator().manual_seed(D)
+        q, k, v = (torch.randn(1, H, S, d, generator=g).to(torch.bfloat16) for d in (D, D, 128))
+        kw = dict(mask_kind=_ffi.MASK_DOCUMENT_CAUSAL if causal else _ffi.MASK_DOCUMENT, doc_ids=ids[None].to(DEV))
+        off = ids[:, None] != ids[None, :]
+        if causal:
+            off = off | torch.ones(S, S, dtype=torch.bool).triu(1)
+        for cap in (0.0, 9.0):
+            got = _ffi.attn_fwd(q.to(DEV), k.to(DEV), v.to(DEV), softcap=cap, **kw).double().cpu()
+            x = q.double() @ k.double().transpose(-1, -2) / math.sqrt(D)
+            want = torch.softmax((cap * torch.tanh(x / cap) if cap else x).masked_fill(off, -math.inf), -1) @ v.double()
+            # weights and results are each rounded by 2^-8 of themselves at most, 2^-8 / sqrt(3) in the norm (emulated in 64 bits: 2.17e-3 in all)
+            assert ((got - want).norm() / want.norm()).item() <= math.sqrt(2 / 3) * 2.0 ** -8, (D, causal, cap)
