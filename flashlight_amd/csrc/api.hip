@@ -885,8 +885,9 @@ bool row_starts_products(const fl_attn_params* p) { return !(p->scale > 0.f) || 
 // two L2s (forward and gradients, 128 x 8 x 256 x 256: 134 MB read by each, 67 by neighbours: four pairs to an XCD there, half of a chunk's heads).  What
 // it costs is a bias read by more XCDs.  us, dealt round -> neighbours.
 // Forward, from chunks of 5 entries on: 400 x 4 x 100 (chunks of 5) 23.7 -> 23.3; 50 x 4 x 333, head dim 64 (5), 41.5 -> 40.7; 150 x 8 x 250 (10) 44.4 ->
-// 44.0; 512 x 8 x 160 105.6 -> 102.6; 150 x 8 x 333, head dim 64, 288 -> 244; even or 1 % at most: 96 x 8 x 256 (6), 96 x 8 x 450.  Chunks of 4: 64 x 8 x 256 20.5 -> 20.8.
-bool forward_neighbours(int chunk_len) { return chunk_len >= 5; }
+// 44.0; 512 x 8 x 160 105.6 -> 102.6; 150 x 8 x 333, head dim 64, 288 -> 244; even: 96 x 8 x 256 (6).  Chunks of 4: 64 x 8 x 256 20.5 -> 20.8.  Nor from 320 keys on at head
+// dim 32: 256 x 8 x 384, 100 x 8 x 400, 64 x 8 x 512 even, 96 x 8 x 450 113.0 -> 114.5, with a bias row 135.3 -> 137.4.
+bool forward_neighbours(const fl::StripeParams& k, int d) { return k.chunk_len >= 5 && (d != 32 || k.Lk <= 320); }
 // Gradients, where q, k, v and dout are more than 24 MB: 96 x 7 x 160 (28 MB) 49.9 -> 48.1; 40 x 8 x 384 (31) 101 -> 91.7; 80 x 8 x 200 (33) 60.0 -> 58.0; 400 x 4 x
 // 100 (41) 52.2 -> 49.0; 72 x 8 x 190, head dim 64 (56), 94.8 -> 87.3; 128 x 8 x 256 (67) 101.4 -> 99.3; 256 x 8 x 130 (68) 108 -> 102; but 64 x 8 x 256 (34) 56.8 -> 57.7.
 // Below it the L2s hold both copies: 20 x 8 x 300 (12) 42.6 -> 43.3, 32 x 8 x 256 (17) 32.1 -> 33.9, 128 x 4 x 128 (17) 22.4 -> 22.8, 100 x 8 x 100 (20) 28.8 -> 29.3.
@@ -1254,7 +1255,7 @@ static int launch_forward(const fl_attn_params* p, void* ungated, void* stream_)
     int waves = 0;
     int64_t plan[2];
     if (plan_stripe(p, ungated, &sp, &waves, plan)) {
-      const hipError_t e = (p->dtype == FL_F16 ? fl::launch_stripe_f16 : fl::launch_stripe_bf16)(p->Dqk, waves, forward_neighbours(sp.chunk_len), sp, stream);
+      const hipError_t e = (p->dtype == FL_F16 ? fl::launch_stripe_f16 : fl::launch_stripe_bf16)(p->Dqk, waves, forward_neighbours(sp, p->Dqk), sp, stream);
       if (e != hipSuccess) return fail((int)e, "launch of the shared-bias stripe forward failed: %s", hipGetErrorString(e));
       return 0;
     }
