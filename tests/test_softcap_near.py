@@ -96,6 +96,39 @@ def test_infinite_scores_are_the_cap():
     _check(q, k, v, 5.0, False, False)
 
 
+@gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,B,S,heads", [(32, 2, 1030, 8), (64, 4, 708, 16), (128, 4, 700, 16), (256, 1, 1100, 4)])
+@pytest.mark.parametrize("alibi,causal", [(False, False), (True, True)])
+def test_scores_on_both_sides_of_the_range_in_calls_with_the_polynomial(D, B, S, heads, dtype, alibi, causal):
+    # standard deviation 1.5: the range ends at 4 and 4.5 of it, which some tiles of a wave's reach and others do not, and at 8, which none does
+    q, k, v = _operands(B, heads, S, D, dtype, 7, 1.5)
+    x = (q[:1].float() @ k[:1].float().transpose(-1, -2)).abs().cpu() / math.sqrt(D)
+    tiles = torch.nn.functional.pad(x, (0, -S % 64, 0, -S % 32)).unflatten(-1, (-1, 64)).unflatten(-3, (-1, 32)).amax((-1, -3))
+    for cap in (24.0, 27.0, 50.0):
+        outside = tiles > cap / 4
+        assert not outside.any() if cap == 50.0 else (outside.any(-1) & ~outside.all(-1)).any()
+        _check(q, k, v, cap, alibi, causal)
+
+
+@gpu
+@pytest.mark.parametrize("D,alibi", [(64, False), (64, True), (128, False), (128, True)])
+@pytest.mark.parametrize("far", [2.5, -2.5, 0.3])
+def test_one_score_far_out_in_any_place_of_a_tile_of_the_polynomial(D, alibi, far):
+    # as above, in a call that is long enough for it: head h has its pair in tile 1 + h % 10 at place 7 h of it
+    H, S, cap = 64, 64 * 11, 30.0
+    q, k, v = _operands(1, H, S, D, torch.bfloat16, 11)
+    q[..., 0] = 0.0
+    k[..., 0] = 0.0
+    for h in range(H):
+        q[0, h, 64 + 5 * h % 640, 0] = 16.0
+        k[0, h, 64 * (1 + h % 10) + 7 * h % 64, 0] = far * cap * math.sqrt(D) / 16.0
+    out, ref = _check(q, k, v, cap, alibi, False)
+    for h in range(H):
+        row = 64 + 5 * h % 640
+        assert ((out - ref)[0, h, row].norm() / ref[0, h, row].norm()).item() <= 2.0 ** -6
+
+
 def _near_caps(pairs, tmp_path):
     """NearCap::of(scale, cap) of the header, for each pair: (a, b, last, per_last, least, least_well)"""
     try:
